@@ -116,6 +116,7 @@ bool tinym_enabled() { return glm_option(GLM_OPT_TINYM) != 0; }
 
 int dispatch(int mode, const GemmParams& p, hipStream_t st) {
     if (p.R <= 0) return GLM_OK;
+    if (glm_midm_takes(mode, p)) return glm_launch_gemm_midm(mode, p, st);
     const int64_t avg = (p.R_hint > 0 ? p.R_hint : p.R) / (p.G > 0 ? p.G : 1);
     if (avg >= LARGEM_MIN_AVG_ROWS) return glm_launch_gemm_largem(mode, p, st);
     return glm_launch_gemm_smallm(mode, p, st);
@@ -163,6 +164,7 @@ extern "C" int glm_gemm_bf16_act(const void* x, int64_t ldx, const void* w, int6
         const int rc = glm_launch_gemm_tinym(GEMM_PLAIN, p, 1, glm_s(stream));
         if (rc != GLM_ERR_UNSUPPORTED) return rc;
     }
+    if (glm_midm_takes(GEMM_PLAIN, p)) return glm_launch_gemm_midm(GEMM_PLAIN, p, glm_s(stream));
     // (a few hundred rows on a few columns, a router's logits: the tiled kernel would be a handful of workgroups)
     if (M >= LARGEM_MIN_AVG_ROWS && !(N <= 256 && M < 1024)) return glm_launch_gemm_largem(GEMM_ACT, p, glm_s(stream));
     return glm_launch_gemm_smallm(GEMM_PLAIN, p, glm_s(stream));

@@ -149,6 +149,9 @@ int glm_launch_gemm_tinym_router_tail(const GemmParams& p, unsigned* ticket, flo
                                       void* scale, int32_t* pos, int with_shared, hipStream_t st);
 // same, weights stored as OCP fp8 e4m3 (1 byte/element, ldw/w_gstride in elements) + per-row scale
 int glm_launch_gemm_smallm_fp8w(int mode, const GemmParams& p, hipStream_t st);
+// some dozen to some hundred rows of one weight matrix (gemm_midm.hip); takes: the shape belongs there, by size and form
+bool glm_midm_takes(int mode, const GemmParams& p);
+int glm_launch_gemm_midm(int mode, const GemmParams& p, hipStream_t st);
 // LDS-tiled MFMA kernels for many rows per group (prefill); p.wscale != nullptr: per-weight-row fp32 scale applied to
 // the accumulator before the bf16 roundings (weights expanded from fp8, elementwise.hip)
 int glm_launch_gemm_largem(int mode, const GemmParams& p, hipStream_t st);

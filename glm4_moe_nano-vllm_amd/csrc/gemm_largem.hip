@@ -1837,6 +1837,7 @@ int glm_launch_gemm_largem_qkv(const GemmParams& p, hipStream_t st) {
     GemmParams q = p;
     q.y = p.qkv_q;  // never stored through; keeps the generic alignment checks meaningful
     q.ldy = p.N;
+    if (glm_midm_takes(GEMM_PLAIN, q)) return glm_launch_gemm_midm(GEMM_PLAIN, q, st);  // where glm_gemm_bf16 goes there, bit-identical to it
     return launch_largem<GEMM_PLAIN>(q, st);
 }
 #endif  // !GLM_DENSE_ONLY

@@ -26,6 +26,7 @@
 //     expert_offsets — no host sync, graph-capturable (the reference's per-expert Python loop with
 //     .any()/where host syncs is moe.py:135-151).
 #include "gemm_internal.h"
+#include "gemm_epilogue.h"
 #include <stdlib.h>
 #include <type_traits>
 
@@ -79,85 +80,6 @@ constexpr int SM_KS = GLM_SM_KS;   // k-steps (of 32) per chunk
 constexpr int SM_KC = 32 * SM_KS;  // 128 elements = 256 B per row per chunk
 constexpr int SM_XROWB = SM_KC * 2;  // bytes per activation row per chunk in LDS
 constexpr int SM_CPR = SM_KC / 8;    // 16-B chunks per row
-
-// epilogue shared by both variants: lane (c,g4) holds, per (rt, mt), columns n..n+3 of token
-// row 16*mt + c
-template <int MODE, int RT, int MT>
-__device__ __forceinline__ void smallm_epilogue(const GemmParams& p, f32x4_t (&acc)[RT][MT], int grp, int m0,
-                                                int mcnt, int ncol0, int c, int g4) {
-    if (MODE == GEMM_PLAIN && p.ypart != nullptr) {
-        // K-split: this workgroup's fp32 partial sums; bias and the bf16 rounding belong to the consumer
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int row = 16 * mt + c;
-            if (row >= mcnt) continue;
-            float* prow = p.ypart + (int64_t)(m0 + row) * p.N;
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const int n = ncol0 + 16 * rt + 4 * g4;
-                if (n < p.N) *reinterpret_cast<f32x4_t*>(prow + n) = acc[rt][mt];
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int row = 16 * mt + c;
-        if (row >= mcnt) continue;
-        bf16_t* yrow = p.y + (int64_t)(m0 + row) * p.ldy;
-        if (gemm_paired(MODE)) {
-            // row tiles [0, RT/2) are gate columns, [RT/2, RT) the matching up columns
-#pragma unroll
-            for (int j = 0; j < RT / 2; ++j) {
-                const int n = ncol0 + 16 * j + 4 * g4;
-                if (n < p.N) {  // N % 4 == 0 is checked on the host
-                    float o[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        o[r] = MODE == GEMM_GLU ? glm_glu_fast(p.act, acc[j][mt][r], acc[RT / 2 + j][mt][r])
-                                                : rbf(glm_silu(rbf(acc[j][mt][r]))) * rbf(acc[RT / 2 + j][mt][r]);
-                    u32x2_t v = {pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
-                    *reinterpret_cast<u32x2_t*>(yrow + n) = v;
-                }
-            }
-        } else {
-            float sc = 1.0f;
-            bool scaled = false;
-            if (MODE == GEMM_DOWN && grp < p.n_scaled) {
-                sc = bf2f(p.scale[m0 + row]);
-                scaled = true;
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const int n = ncol0 + 16 * rt + 4 * g4;
-                if (n >= p.N) continue;
-                float o[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float a = acc[rt][mt][r];
-                    if (MODE == GEMM_PLAIN && p.bias) a += bf2f(p.bias[n + r]);
-                    if (scaled) a = rbf(a) * sc;
-                    o[r] = a;
-                }
-                if (MODE == GEMM_PLAIN) {
-                    if (p.yf != nullptr) {
-                        f32x4_t v;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) v[r] = glm_act_precise(p.act, o[r], n + r);
-                        *reinterpret_cast<f32x4_t*>(p.yf + (int64_t)(m0 + row) * p.ldy + n) = v;
-                        continue;
-                    }
-                    if (p.act.kind != GLM_ACT_NONE) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) o[r] = glm_act_fast(p.act, o[r], n + r);
-                    }
-                }
-                u32x2_t v = {pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
-                *reinterpret_cast<u32x2_t*>(yrow + n) = v;
-            }
-        }
-    }
-}
 
 // One workgroup's work for a block of at most 16*MT rows of group `grp` (rows m0 .. m0+mcnt).
 // MT is a template parameter so that the chunk loop is straight-line code: every load is
@@ -362,7 +284,7 @@ __device__ __forceinline__ void smallm_body(const GemmParams& p, char* smem, int
                 for (int r = 0; r < 4; ++r) acc[rt][mt][r] *= sc[r];
         }
     }
-    smallm_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
+    gemm_row_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
 }
 
 template <int MODE, int NWAVES, int WS, int RT, int MTMAX, bool W8>
@@ -669,7 +591,7 @@ __device__ __forceinline__ void smallm_body_dma(const GemmParams& p, char* smem,
                     acc[rt][mt] += *reinterpret_cast<const f32x4_t*>(
                         red + ((((wr * (WS - 1) + (s - 1)) * RT + rt) * MT + mt) * 64 + lane) * 4);
     }
-    smallm_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
+    gemm_row_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
 }
 
 template <int MODE, int NWAVES, int WS, int RT, int MTMAX, int TPW>
@@ -880,7 +802,7 @@ __device__ __forceinline__ void smallm_body_sx(const GemmParams& p, char* smem, 
                 for (int r = 0; r < 4; ++r) acc[rt][mt][r] *= sc[r];
         }
     }
-    smallm_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
+    gemm_row_epilogue<MODE, RT, MT>(p, acc, grp, m0, mcnt, ncol0, c, g4);
 }
 
 #ifndef GLM_SM_SX_STAGES

@@ -1,0 +1,101 @@
+"""Projections of 33 to some hundred rows (csrc/gemm_midm.hip): both tiles, every epilogue, ragged rows and columns, waves without a chunk
+of K — against the operators in fp64 on the same bf16 operands.  A result is one rounding of an fp32 sum of K products: off by at most half
+a bf16 ulp plus the sum's error (K terms of the size of the result at most: 2e-6 of the row's absolute sum, far below an ulp), so by one ulp
+where that sum lies on a rounding boundary."""
+import pytest
+import torch
+
+from oracle import dafolorn_oracle as D
+from oracle import glm4_moe_oracle as O
+from oracle import napadra_oracle as N_
+from util import assert_close_bf16
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from nanovllm import hip_ops
+    hip_ops.load_library()
+    return hip_ops
+
+
+def rnd(*shape, seed, scale=1.0):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale).to(BF)
+
+
+def close(got, ref, what):
+    """ref fp64, one rounding away."""
+    assert_close_bf16(got.float().to(BF) if got.dtype == torch.float32 else got, ref.to(BF), 1, 0.05, atol=2 ** -9, what=what)
+
+
+# (rows, columns, K): one column of tiles and many, more than 256 small tiles (the 64-column one), K of one chunk (three waves without
+# work) up to several rounds of the ring, columns that end inside a tile, rows that end inside a block
+SIZES = [(33, 36, 64), (64, 100, 128), (65, 2048, 192), (97, 2052, 1088), (211, 2112, 2048), (256, 8200, 576), (33, 16420, 320), (128, 264, 4096),
+         (520, 1000, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_plain(ops, M, N, K):
+    x, w, b = rnd(M, K + 8, seed=1)[:, :K], rnd(N, K, seed=2, scale=K ** -0.5), rnd(N, seed=3)
+    wp = ops.padded_weight(N, K, dtype=BF, device="cuda")
+    wp.copy_(w)
+    xd = torch.empty(M, K + 8, dtype=BF, device="cuda")[:, :K]
+    xd.copy_(x)
+    ref = x.double() @ w.double().T
+    close(ops.gemm_bf16(xd, wp), ref, "plain")
+    close(ops.gemm_bf16(xd, wp, b.cuda()), ref + b.double(), "bias")
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_activations(ops, M, N, K):
+    """Act in the epilogue: per-column ones, xIELU, fp32 rows with and without a soft cap, rows into a wider buffer."""
+    if N % 8:
+        N += 4      # (fp32 rows and rows of a wider buffer are whole 16-byte pieces)
+    x, w = rnd(M, K, seed=4), rnd(N, K, seed=5, scale=K ** -0.5)
+    z = x.double() @ w.double().T
+    cut = N // 3 // 8 * 8
+    gate = torch.cat([z[:, :cut], torch.sigmoid(z[:, cut:])], 1)
+    relu = torch.cat([z[:, :cut].clamp(min=0) ** 2, z[:, cut: 2 * cut], torch.sigmoid(z[:, 2 * cut:])], 1)
+    p, q = torch.tensor(0.3).double(), torch.tensor(-0.4).double()
+    xielu = (ops.ACT_XIELU, float(D.softplus(p)), float(0.5 + D.softplus(q)))
+    xd, wd = x.cuda(), w.cuda()
+    out = torch.full((M, N + 16), 7.0, dtype=BF, device="cuda")
+    close(ops.linear_act(xd, wd, act=(ops.ACT_GATE, float(cut), 0.0), out=out[:, 8: 8 + N]), gate, "gate")
+    assert torch.all(out[:, :8] == 7) and torch.all(out[:, 8 + N:] == 7)
+    close(ops.linear_act(xd, wd, act=(ops.ACT_RELU2_GATE, float(cut), float(2 * cut))), relu, "relu^2 | pass | gate")
+    close(ops.linear_act(xd, wd, act=xielu), D.xielu(z, p, q), "xielu")
+    # fp32 rows: the sum's own error, K products of magnitude |x| |w|
+    bound = 2.0 ** -23 * (x.double().abs() @ w.double().abs().T) * 8
+    assert ((ops.linear_act(xd, wd, out_f32=True).cpu().double() - z).abs() <= bound + 1e-7).all()
+    capped = ops.linear_act(xd, wd, act=(ops.ACT_SOFTCAP, 3.0, 0.0), out_f32=True).cpu().double()
+    assert ((capped - N_.soft_cap(z, 3.0)).abs() <= bound + 2e-6).all()
+
+
+@pytest.mark.parametrize("M,I,K", [(33, 24, 64), (65, 1000, 192), (97, 1408, 1088), (211, 4104, 576), (300, 264, 1024)])
+def test_gated(ops, M, I, K):
+    x, w = rnd(M, K, seed=6), rnd(2 * I, K, seed=7, scale=K ** -0.5)
+    g, u = (x.double() @ w.double().T).chunk(2, 1)
+    close(ops.gated_glu(x.cuda(), w.cuda(), 2.0), N_.clamped_glu(g, u, 2.0), "clamped unit")
+    act = ops.grouped_gemm_gateup_silu(x.cuda(), w.cuda().unsqueeze(0), None, None, M)
+    assert_close_bf16(act, O.silu_and_mul(torch.cat([g, u], 1).to(BF)), 2, 0.06, atol=2 ** -8, what="silu")   # (its input's rounding on top)
+    d = rnd(K, I, seed=8, scale=I ** -0.5)
+    y = ops.grouped_gemm_down(act, d.cuda().unsqueeze(0), None, None, 0)
+    close(y, act.cpu().double() @ d.double().T, "down")
+
+
+@pytest.mark.parametrize("T,nh,nkv,K", [(97, 4, 1, 1024), (211, 6, 2, 640), (256, 2, 2, 512)])
+def test_qkv_epilogue(ops, T, nh, nkv, K):
+    """Split, rotation and cache rows in the projection's epilogue: the projection and the split kernel, bit for bit."""
+    x, w, b = rnd(T, K, seed=9).cuda(), rnd((nh + 2 * nkv) * 128, K, seed=10, scale=K ** -0.5).cuda(), rnd((nh + 2 * nkv) * 128, seed=11).cuda()
+    g = torch.Generator().manual_seed(12)
+    pos = torch.randint(0, 500, (T,), generator=g).cuda()
+    cs = O.build_cos_sin_cache(64, 512, 10000.0).reshape(512, 64).contiguous().cuda()
+    slots = torch.randperm(512, generator=g)[:T].to(torch.int32)
+    slots[::5] = -1
+    caches = [torch.full((2, 256, nkv, 128), 3.0, dtype=BF, device="cuda") for _ in range(4)]
+    q, k, v = ops.gemm_qkv_rope_store(x, w, b, nh, nkv, 128, pos, cs, 64, caches[0], caches[1], slots.cuda(), True)
+    q2, k2, v2 = ops.qkv_split_norm_rope_store(ops.gemm_bf16(x, w, b), nh, nkv, 128, pos, cs, 64, None, None, 1e-5, caches[2], caches[3], slots.cuda(), True)
+    assert torch.equal(q, q2) and torch.equal(k, k2) and torch.equal(v, v2)
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
