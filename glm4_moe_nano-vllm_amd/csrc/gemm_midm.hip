@@ -280,6 +280,9 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
 // 4096 x 12288 at 128 rows 57.5 / 41.0 (256 tiles), at 211 rows 48.5 / 61.6 (512 tiles), 14336 x 4096 at 64 rows 28.4 / 35.1
 template <int MODE>
 int launch_midm(const GemmParams& p, hipStream_t st) {
+    // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
+    // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
+    if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
     if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);   // (half a head; the sums are the same in both tiles)
     const int half = gemm_paired(MODE) ? 16 : 32;   // columns of the small tile
     const int64_t tiles = (int64_t)((p.N + half - 1) / half) * ((p.R + 63) / 64);
@@ -289,7 +292,17 @@ int launch_midm(const GemmParams& p, hipStream_t st) {
 }  // namespace
 
 bool glm_midm_takes(int mode, const GemmParams& p) {
-    if (p.offs != nullptr || p.src != nullptr || p.G > 1 || p.ksplit > 1 || p.wscale != nullptr || p.R <= 32 || p.K % 64 != 0) return false;
+    if (p.ksplit > 1 || p.wscale != nullptr || p.K % 64 != 0) return false;
+    if (p.offs != nullptr) {
+        // Experts with 24 to 95 rows on average: the weight-streaming kernel's blocks of 32 rows read an expert's weights once per block.
+        // gate|up, down of 1408 x 4096, us: 26 rows 298 / 160 there, 261 / 147 here; 55 rows 557 / 279 and 307 / 174; 18 rows 263 / 149 and
+        // 265 / 145; of 1024 x 2048: 20 rows 108 / 57 and 106 / 60, 38 rows 168 / 82 and 109 / 62.
+        const int64_t rows = p.R_hint > 0 ? p.R_hint : p.R;
+        if (mode != GEMM_GATEUP && mode != GEMM_DOWN) return false;
+        return rows >= 24 * (int64_t)p.G && rows < 96 * (int64_t)p.G && p.R * p.ldx * 2 < (1ll << 31) &&
+               (mode == GEMM_GATEUP ? 2 : 1) * (int64_t)p.N * p.ldw * 2 < (1ll << 31);
+    }
+    if (p.src != nullptr || p.G > 1 || p.R <= 32) return false;
     // (a loop of the tiled kernel that is asked for keeps its shapes)
     if (p.R >= 96 && (glm_option(GLM_OPT_LARGEM_VARIANT) >= 0 || glm_option(GLM_OPT_LARGEM_CFG) != 0)) return false;
     const bool paired = gemm_paired(mode);

@@ -85,6 +85,40 @@ def test_gated(ops, M, I, K):
     close(y, act.cpu().double() @ d.double().T, "down")
 
 
+@pytest.mark.parametrize("T,E,k,H,I,shared", [(33, 3, 2, 192, 100, True), (97, 5, 3, 576, 72, False), (211, 8, 2, 128, 264, True), (64, 1, 1, 64, 40, False)])
+def test_experts(ops, T, E, k, H, I, shared):
+    """Groups of 24 to 95 rows on average, ragged ones among them (an expert without rows, one with more than a block of 64)."""
+    G = E + int(shared)
+    g = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(max(E - 1, 1), generator=g)[: k] if t % 5 or E == 1 else torch.arange(k) for t in range(T)]).sort(-1).values
+    wt = (torch.rand(T, k, generator=g) + 0.1).to(BF)
+    offs, tok, scale, _ = ops.moe_align(idx.cuda(), wt.cuda(), E, shared)
+    R = T * k + (T if shared else 0)
+    assert 24 * G <= R < 96 * G
+    x, w13, w2 = rnd(T, H, seed=20), rnd(G, 2 * I, H, seed=21, scale=H ** -0.5), rnd(G, H, I, seed=22, scale=I ** -0.5)
+    I64 = I // 64 * 64 or 64
+    act_in, w2 = rnd(R, I64, seed=23), rnd(G, H, I64, seed=22, scale=I64 ** -0.5)
+    act = ops.grouped_gemm_gateup_silu(x.cuda(), w13.cuda(), offs, tok, R)
+    y = ops.grouped_gemm_down(act_in.cuda(), w2.cuda(), offs, scale, E)
+    o, s = offs.cpu().tolist(), scale.cpu()
+    for e in range(G):
+        if o[e + 1] > o[e]:
+            rows = slice(o[e], o[e + 1])
+            z = x[tok.cpu()[rows].long()].double() @ w13[e].double().T
+            assert_close_bf16(act[rows], O.silu_and_mul(z.to(BF)), 2, 0.06, atol=2 ** -8, what=f"act of expert {e}")
+            d = (act_in[rows].double() @ w2[e].double().T).to(BF)
+            assert_close_bf16(y[rows], (d.float() * s[rows, None].float()).to(BF) if e < E else d, 2, 0.06, atol=2 ** -8, what=f"y of expert {e}")
+
+
+@pytest.mark.parametrize("M,I", [(1, 1408), (1, 10944)])
+def test_one_row_feed_forward(ops, M, I):
+    H = 512
+    x, w, d = rnd(M, H, seed=30), rnd(2 * I, H, seed=31, scale=H ** -0.5), rnd(H, I, seed=32, scale=I ** -0.5)
+    act = ops.grouped_gemm_gateup_silu(x.cuda(), w.cuda().unsqueeze(0), None, None, M)
+    assert_close_bf16(act, O.silu_and_mul((x.double() @ w.double().T).to(BF)), 2, 0.06, atol=2 ** -8, what="silu")
+    close(ops.grouped_gemm_down(act, d.cuda().unsqueeze(0), None, None, 0), act.cpu().double() @ d.double().T, "down")
+
+
 @pytest.mark.parametrize("T,nh,nkv,K", [(97, 4, 1, 1024), (211, 6, 2, 640), (256, 2, 2, 512)])
 def test_qkv_epilogue(ops, T, nh, nkv, K):
     """Split, rotation and cache rows in the projection's epilogue: the projection and the split kernel, bit for bit."""
