@@ -1712,7 +1712,13 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int64_t avg_rows = (p.R_hint > 0 ? p.R_hint : p.R) / (p.G > 0 && MODE != GEMM_SLICES ? p.G : 1);
     // ... and a projection onto <= 128 columns (the router logits at prefill: N = E = 64) is one column tile however the rows
     // are cut, so its parallelism is its row-block count: 128-row blocks (75.8 -> 55.1 us at T = 16384)
-    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS) && p.offs == nullptr && p.N <= 128));
+    // ... and so is every single projection whose 128-row tiles are at most one round of the chip (with the band's rounding, as
+    // launch_largem_cfg counts): a K step costs two thirds (14336 x 4096 at 200 and 400 rows 83 / 60 and 86 / 59 us, 2048 x 2048 at 2000
+    // rows 42 / 28, 4096 x 12288 at 1200 rows 234 / 153; beyond a round 9728 x 2048 at 800 rows 48 / 60)
+    const int64_t cb = (p.R + 127) / 128, bd = cb < g_largem_band ? cb : (int64_t)g_largem_band;
+    const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
+                           (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
+    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS) && p.offs == nullptr && p.N <= 128));
     // the lean load phase addresses x and the group's weights through 32-bit buffer offsets and has no K tail path
     // default (tools/largem_ab.py, one process, T = 16384): the quadrant-phase loop with 4 x 2-tile quadrants and the
     // fragment reads of a load interval issued before its DMA, no priority flips (86531: +1 % over 86019), epilogue

@@ -11,7 +11,7 @@
 //   * 16-byte pieces are swizzled at the source, piece ^ ((row >> 1) & 7): the 16 rows of a fragment read cover all banks;
 //   * the fragments of a k-step are read under the MFMAs of the one before, a freed stage is refilled right after;
 //   * the partial tiles of the waves are summed through LDS in wave order, each wave finishes its share of the rows;
-//   * workgroups that share weight rows sit on one XCD (blockIdx.x & 7), next to one another.
+//   * workgroups that share weight rows sit on one XCD, next to one another, and every XCD has as many.
 #include "gemm_internal.h"
 #include "gemm_epilogue.h"
 
@@ -228,7 +228,7 @@ constexpr int midm_lds() {
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
-__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p_in, int mblocks) {
+__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p_in, int mblocks, int interleaved) {
     GemmParams p = p_in;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int COLS = gemm_paired(MODE) ? 8 * RT : 16 * RT;
@@ -250,10 +250,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p_i
         ntile = blockIdx.x;
         if (grp < 0) return;
     } else {
-        const int q = blockIdx.x >> 3;
-        m0 = q % mblocks * (16 * MT);
+        int m;
+        if (interleaved) {   // column tiles dealt to the XCDs (workgroups b, b + 8, ...) one by one, their row blocks behind one another
+            const int q = blockIdx.x >> 3;
+            m = q % mblocks;
+            ntile = q / mblocks * 8 + (blockIdx.x & 7);
+        } else {             // few column tiles: an XCD takes a run of all tiles
+            const int lin = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+            ntile = lin / mblocks;
+            m = lin % mblocks;
+        }
+        m0 = m * (16 * MT);
         mcnt = min(16 * MT, (int)p.R - m0);
-        ntile = q / mblocks * 8 + (blockIdx.x & 7);
     }
     if (ntile * COLS >= p.N) return;
     midm_body<MODE, MT, RT, NW, NST>(p, smem, grp, m0, mcnt, ntile * COLS);
@@ -266,27 +274,34 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
     static_assert(LDS <= 160 * 1024, "the rings of all waves must fit the CU's LDS");
     const int cols = gemm_paired(MODE) ? 8 * RT : 16 * RT, nt = (p.N + cols - 1) / cols;
     const int64_t mblocks = (p.R + 16 * MT - 1) / (16 * MT);
-    const int64_t gx = p.offs ? nt : (int64_t)(nt + 7) / 8 * 8 * mblocks, gy = p.offs ? p.R / (16 * MT) + p.G : 1;
+    const bool dealt = nt >= 64;
+    const int64_t gx = p.offs ? nt : dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8, gy = p.offs ? p.R / (16 * MT) + p.G : 1;
     GLM_CHECK_ARG(gx < (1 << 30) && gy <= 65535, GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
     auto kern = gemm_midm_kernel<MODE, MT, RT, NW, NST>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
-    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(NW * 64), LDS, st, p, (int)mblocks);
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt);
     GLM_CHECK_LAUNCH("gemm_midm");
     return GLM_OK;
 }
 
-// the 64-column tile reads 64 + 64 rows per 64 columns, the 32-column one 64 + 32 per 32: it is taken while the grid would not cover
-// the chip otherwise (one workgroup of either kind per CU).  Cold weights, 64x64 against 64x32, us: 2048 x 2048 at 128 rows 10.5 / 7.5,
-// 4096 x 12288 at 128 rows 57.5 / 41.0 (256 tiles), at 211 rows 48.5 / 61.6 (512 tiles), 14336 x 4096 at 64 rows 28.4 / 35.1
+// tiles of 64 rows and 32 columns
+int64_t small_tiles(int mode, const GemmParams& p) {
+    const int cols = gemm_paired(mode) ? 16 : 32;
+    return (int64_t)((p.N + cols - 1) / cols) * ((p.R + 63) / 64);
+}
+
+// Up to a workgroup per CU: 64 x 32 with four waves.  Beyond: workgroups of two waves, three to a CU, so that one's start and end lie under
+// the others' loops.  A long K pays those once per tile and the activation traffic always: 64 x 64.  Four waves 64 x 32, two waves 64 x 32,
+// four waves 64 x 64, us, cold operands: 2048 x 2048 at 128 rows (128 tiles) 8.2 / 10.7 / 15.8; 6144 x 2048 at 256 (768) 20.6 / 17.0 / 34.0;
+// 14336 x 4096 at 128 (896) 58.9 / 55.4 / 59.3; 4096 x 12288 at 128 (256) 42.7 / 53.4 / 66.2, at 256 (512) 74.2 / 79.5 / 66.1.
 template <int MODE>
 int launch_midm(const GemmParams& p, hipStream_t st) {
     // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
     // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
     if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
     if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);   // (half a head; the sums are the same in both tiles)
-    const int half = gemm_paired(MODE) ? 16 : 32;   // columns of the small tile
-    const int64_t tiles = (int64_t)((p.N + half - 1) / half) * ((p.R + 63) / 64);
-    return tiles <= 256 ? launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st) : launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);
+    if (small_tiles(MODE, p) <= 256) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
+    return p.K >= 8192 ? launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st) : launch_midm_cfg<MODE, 4, 2, 2, 2>(p, st);
 }
 
 }  // namespace
@@ -308,18 +323,19 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     const bool paired = gemm_paired(mode);
     const int64_t wrows = paired ? 2 * (int64_t)p.N : (int64_t)p.N;
     if (p.R * p.ldx * 2 >= (1ll << 31) || wrows * p.ldw * 2 >= (1ll << 31)) return false;   // 32-bit offsets
-    const int64_t cols = paired ? 32 : 64, tiles = (p.N + cols - 1) / cols * ((p.R + 63) / 64);
+    const int64_t tiles = small_tiles(mode, p);
     // Fewer rows than the tiled kernel takes: the weight-streaming kernel gets ahead where it has a wave of workgroups to spare (32768 x 2048
-    // at 64 rows 31 us, here 35; 18944 x 4096 50 / 50; 14336 x 4096 45 / 28; 2048 x 6144 62 / 23).
-    if (p.R < 96) return tiles <= 300;
-    // (A short reduction is a handful of steps of the tiled kernel's loop: K = 512, 128 rows: 2048 columns 11.5 / 4.8, 14336 (448 tiles)
-    // 13.6 / 12.0; 256 rows: 2048 16.9 / 4.9, 14336 (896) 18.7 / 20.8.  Beyond 256 rows nothing here has such a projection and few columns.)
-    if (p.K <= 512) return p.R <= 256 && tiles <= 450;
+    // at 64 rows, 1024 tiles, 31 us, here 35; 18944 x 4096, 592, 50 / 49; 14336 x 4096 45 / 37; 2048 x 6144 62 / 16).
+    // A gated projection runs there in blocks of 32 rows: 10944 gated columns x 4096 (684 tiles) 75 us, here 52.
+    if (p.R < 96) return tiles <= (paired ? 1100 : 600);
+    // (A short reduction is a handful of steps of the tiled kernel's loop: K = 512, 128 rows: 2048 columns 11.5 / 4.8, 14336 (896 tiles)
+    // 13.6 / 12.0; 256 rows: 2048 16.9 / 4.9, 14336 (1792) 18.7 / 20.8.  Beyond 256 rows nothing here has such a projection and few columns.)
+    if (p.K <= 512) return p.R <= 256 && tiles <= 900;
     // The tiled kernel's time is its K loop's as long as its tiles are one round of the chip; here it grows with the tiles (L2 -> LDS
-    // traffic, about 11 TB/s): 14336 x 4096 at 211 rows (896 tiles) 78 / 70 us, 18944 x 4096 at 211 rows (1184) 79 / 88, 14336 x 4096 at
-    // 384 rows (1344) 78 / 103, 6144 x 2048 at 384 rows (576) 43 / 32, 2048 x 6144 at 128 rows 89 / 21.
-    const int64_t big = (p.R + 255) / 256 * ((p.N + (paired ? 127 : 255)) / (paired ? 128 : 256));
-    return tiles <= 900 * ((big + 255) / 256);
+    // traffic, about 11 TB/s).  Tiled / here, us: 2048 x 6144 at 128 rows (128 tiles) 68 / 16, 6144 x 2048 at 256 (768) 28 / 17, 14336 x 4096
+    // at 128 (896) 66 / 55, 9728 x 2048 at 200 (1216) 33 / 33, 6144 x 2048 at 400 (1344) 28 / 29, 14336 x 4096 at 200 (1792) 60 / 77.
+    const int64_t big = (p.R + 127) / 128 * ((p.N + (paired ? 127 : 255)) / (paired ? 128 : 256));
+    return tiles <= 1100 * ((big + 255) / 256);
 }
 
 int glm_launch_gemm_midm(int mode, const GemmParams& p, hipStream_t st) {
