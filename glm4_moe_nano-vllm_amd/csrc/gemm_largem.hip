@@ -298,7 +298,7 @@ __device__ __forceinline__ void lm_locate_wave(const int32_t* __restrict__ offs,
 template <int MODE, class C, int VAR, bool WSCALE>
 __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND) {
     constexpr bool LEAN = (VAR & LM_LEAN) != 0;
-    constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES;  // may store fp32 rows (p.yf)
+    constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP;  // may store fp32 rows (p.yf)
     // DMA instructions of a K tile issued from the MFMA phase (the rest from the load phase)
     constexpr int S2 = !LEAN ? 0 : (VAR & LM_DMA4) ? C::DPW : (VAR & LM_DMA2) ? C::DPW / 2 : 0;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1556,9 +1556,10 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
                     } else {
                         float a = acc[t][mt][r];
                         if constexpr (WSCALE) a *= wsv[t][r];
-                        if ((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS) && p.bias) a += bf2f(p.bias[min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)]);
+                        if ((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP) && p.bias) a += bf2f(p.bias[min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)]);
                         if (scaled) a = rbf(a) * sc;
                         if (MODE == GEMM_XIELU) a = glm_xielu_fast(p.act.a, p.act.b, a);
+                        if (MODE == GEMM_CAP) a = p.act.a * tanhf(a / p.act.a);
                         if (MODE == GEMM_COLS) a = glm_act_cols(p.act, a, ncol_w + 16 * t + 4 * g4 + r);
                         if (MODE == GEMM_ACT) a = p.yf != nullptr ? glm_act_precise(p.act, a, ncol_w + 16 * t + 4 * g4 + r) : glm_act_fast(p.act, a, ncol_w + 16 * t + 4 * g4 + r);
                         o[r] = a;
@@ -1718,7 +1719,7 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int64_t cb = (p.R + 127) / 128, bd = cb < g_largem_band ? cb : (int64_t)g_largem_band;
     const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
                            (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
-    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS) && p.offs == nullptr && p.N <= 128));
+    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP) && p.offs == nullptr && p.N <= 128));
     // the lean load phase addresses x and the group's weights through 32-bit buffer offsets and has no K tail path
     // default (tools/largem_ab.py, one process, T = 16384): the quadrant-phase loop with 4 x 2-tile quadrants and the
     // fragment reads of a load interval issued before its DMA, no priority flips (86531: +1 % over 86019), epilogue
@@ -1860,6 +1861,8 @@ int glm_launch_gemm_largem(int mode, const GemmParams& p, hipStream_t st) {
 #endif  // GLM_EXPERTS
     if (mode == GEMM_ACT && p.yf == nullptr && p.act.kind >= GLM_ACT_GATE) return launch_largem<GEMM_COLS>(p, st);
     if (mode == GEMM_ACT && p.yf == nullptr && p.act.kind == GLM_ACT_XIELU) return launch_largem<GEMM_XIELU>(p, st);
+    if (mode == GEMM_ACT && p.yf != nullptr && p.act.kind == GLM_ACT_NONE) return launch_largem<GEMM_F32>(p, st);
+    if (mode == GEMM_ACT && p.yf != nullptr && p.act.kind == GLM_ACT_SOFTCAP) return launch_largem<GEMM_CAP>(p, st);
     if (mode == GEMM_SLICES) return launch_largem<GEMM_SLICES>(p, st);
     if (mode == GEMM_ACT) return launch_largem<GEMM_ACT>(p, st);
     if (mode == GEMM_GLU) return launch_largem<GEMM_GLU>(p, st);

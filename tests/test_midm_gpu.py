@@ -36,9 +36,11 @@ def close(got, ref, what):
 SILU = (4, 0.06, 2 ** -8)
 
 # (rows, columns, K): one column of tiles and many, more than 256 small tiles (the 64-column one), K of one chunk (three waves without
-# work) up to several rounds of the ring, columns that end inside a tile, rows that end inside a block, and the large tile of long reductions
+# work) up to several rounds of the ring, columns that end inside a tile, rows that end inside a block, the large tile of long reductions,
+# and one of the tiled kernel's (its epilogues)
 SIZES = [(33, 36, 64), (64, 100, 128), (65, 2048, 192), (97, 2052, 1088), (211, 2112, 2048), (256, 8200, 576), (33, 16420, 320), (128, 264, 4096),
-         (520, 1000, 1024), (130, 4128, 8256)]
+         (520, 1000, 1024), (130, 4128, 8256),
+         (1300, 2056, 128)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
