@@ -401,7 +401,10 @@ template <int TAPS, int NT>
 int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
     // decode: one row per workgroup; else runs of rows long enough to spread the halo and the register setup, short enough
     // to fill the chip
-    int tr = a.T <= 512 ? 1 : (int)((a.T + 511) / 512);
+    // four waves on every SIMD: a row is a chain of one load, two reductions and a store, with one row's loads in flight per workgroup (15074
+    // rows of 2048: with 512 workgroups of 256 threads 95 us, 1024 75, 2048 78)
+    constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
+    int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;
     hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT>), dim3((unsigned)((a.T + tr - 1) / tr)), dim3(NT), 0, st, a, tr);
     GLM_CHECK_LAUNCH("glm_seq_norm");
