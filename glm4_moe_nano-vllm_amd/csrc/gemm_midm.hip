@@ -2,16 +2,19 @@
 // prompts, the experts of a short prompt.  gfx950 only.
 //
 // What bounds it: the weights are still read once and dominate the HBM bytes, but an output tile must be small for the grid to cover
-// the chip, and every workgroup pulls its own activation rows through L2 -> LDS (about 11 TB/s over the chip, which binds from some 200 tiles
-// on): the tile (64 rows x 64 or 32 weight rows) is chosen for that traffic, and the LDS reads behind it are not allowed to exceed it.  So the waves of a workgroup split
-// K, not the tile: a wave computes the whole output tile over its own K chunks, every staged byte is read from LDS exactly once, and
-// there is no workgroup barrier in the loop — a wave waits for its own DMA only (counted vmcnt), as in the weight-streaming kernels.
+// the chip, and every workgroup pulls its own activation and weight rows through L2 -> LDS, some 32 bytes per clock and CU: the tile is
+// chosen for that traffic and for the number of workgroups (midm_tile_of), from 64 rows x 32 weight rows up to 128 x 128.
 //   * a stage = one 64-wide K chunk of the tile's activation and weight rows, a whole 128-byte line per row (with 32-wide chunks, half
 //     lines: 14336 x 4096 at 128 rows 53 instead of 45 us, 4096 x 12288 at 64 rows 60 instead of 45);
 //   * 16-byte pieces are swizzled at the source, piece ^ ((row >> 1) & 7): the 16 rows of a fragment read cover all banks;
-//   * the fragments of a k-step are read under the MFMAs of the one before, a freed stage is refilled right after;
-//   * the partial tiles of the waves are summed through LDS in wave order, each wave finishes its share of the rows;
+//   * the fragments of a k-step are read under the MFMAs of the one before;
 //   * workgroups that share weight rows sit on one XCD, next to one another, and every XCD has as many.
+// Two bodies.  Split (few tiles, a long K, experts): the waves split K, not the tile.  A wave computes the whole output tile over its own
+// chunks, every staged byte is read from LDS exactly once, and there is no workgroup barrier in the loop: a wave waits for its own DMA only
+// (counted vmcnt) and refills a stage once it is in registers; the partial tiles are summed through LDS in wave order, each wave finishes its
+// share of the rows.  Shared (more tiles): the waves split the tile over one ring of three or four stages with a barrier per stage; no ring per
+// wave, so the tile can be larger and a stage's bytes serve more MFMAs.  14336 x 4096 at 64 rows 37 -> 28 us, at 128 56 -> 38, at 211 61 -> 43,
+// 4096 x 4096 at 1000 rows 58 -> 43 (tiled), 10944 gated columns x 4096 at 64 rows 53 -> 43.
 #include "gemm_internal.h"
 #include "gemm_epilogue.h"
 
@@ -57,11 +60,26 @@ struct MmFrags {                       // one k-step of 32 columns
     }
 };
 
-// The QKV projection's epilogue (glm_gemm_qkv_rope_store) on a tile of 64 columns, one half of a head: bias, rounding of the packed value,
-// rotation of the first half's columns i and i + 32 (row tiles t and t + 2 in the same lane), rows of q / k / v and of the caches.  The
-// tiled kernel's arithmetic and rounding points, so the fused launch stays bit-identical to the projection and the split kernel.
-template <int MPW>
-__device__ __forceinline__ void midm_qkv_rows(const GemmParams& p, const f32x4_t (&acc)[4][MPW], int m0, int mcnt, int ncol0, int c, int g4) {
+template <int MT, int RT>
+struct MmShared : MmFrags<MT, RT> {    // the same out of a shared stage: the wave's weight rows and activation rows apart
+    template <int I>
+    __device__ __forceinline__ void read_rows(unsigned a) {
+        mm_lds_read<I * 2048>(this->x[I], a);
+        if constexpr (I + 1 < MT) read_rows<I + 1>(a);
+    }
+    __device__ __forceinline__ void read(unsigned aw, unsigned ax) {
+        this->template read_w<0>(aw);
+        read_rows<0>(ax);
+    }
+};
+
+// The QKV projection's epilogue (glm_gemm_qkv_rope_store) on T row tiles out of one half of a head, tile t's columns from ncol0 + sub +
+// 64 t / T: bias, rounding of the packed value, rotation of the first half's columns i and i + 32 (row tiles t and t + T / 2 in the same
+// lane), rows of q / k / v and of the caches.  The tiled kernel's arithmetic and rounding points, so the fused launch stays bit-identical to
+// the projection and the split kernel.
+template <int T, int MPW>
+__device__ __forceinline__ void midm_qkv_rows(const GemmParams& p, const f32x4_t (&acc)[T][MPW], int m0, int mcnt, int ncol0, int sub, int c, int g4) {
+    constexpr int TC = 64 / T;   // columns from tile to tile
     const int nh = p.qkv_nh, nkv = p.qkv_nkv, head = ncol0 >> 7, half = (ncol0 >> 6) & 1;
     const bool is_q = head < nh, is_k = !is_q && head < nh + nkv;
     const int kh = is_q ? head : is_k ? head - nh : head - nh - nkv;
@@ -73,31 +91,31 @@ __device__ __forceinline__ void midm_qkv_rows(const GemmParams& p, const f32x4_t
         const int row = 16 * j + c;
         if (row >= mcnt) continue;
         const int64_t m = m0 + row;
-        float o[4][4];
+        float o[T][4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int n = ncol0 + 16 * t + 4 * g4;
+        for (int t = 0; t < T; ++t) {
+            const int n = ncol0 + sub + TC * t + 4 * g4;
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[t][r] = rbf(acc[t][j][r] + (p.bias ? bf2f(p.bias[n + r]) : 0.0f));
         }
         if (half == 0 && (is_q || is_k)) {
-            const float* cs = p.qkv_cs + p.qkv_pos[m] * 64;
+            const float* cs = p.qkv_cs + p.qkv_pos[m] * 64 + sub;
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < T / 2; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float cv = cs[16 * t + 4 * g4 + r], sv = cs[32 + 16 * t + 4 * g4 + r], x1 = o[t][r], x2 = o[t + 2][r];
+                    const float cv = cs[TC * t + 4 * g4 + r], sv = cs[32 + TC * t + 4 * g4 + r], x1 = o[t][r], x2 = o[t + T / 2][r];
                     o[t][r] = x1 * cv - x2 * sv;
-                    o[t + 2][r] = x2 * cv + x1 * sv;
+                    o[t + T / 2][r] = x2 * cv + x1 * sv;
                 }
         }
         int64_t slot = -1;
         if (cache != nullptr && p.qkv_slots != nullptr) slot = p.qkv_slots[m];
         const bool to_cache = slot >= 0 && slot < p.qkv_nslots;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < T; ++t) {
             const u32x2_t v = {pack2bf(o[t][0], o[t][1]), pack2bf(o[t][2], o[t][3])};
-            const int col = kh * 128 + 64 * half + 16 * t + 4 * g4;
+            const int col = kh * 128 + 64 * half + sub + TC * t + 4 * g4;
             if (dense != nullptr) *reinterpret_cast<u32x2_t*>(dense + m * ldd + col) = v;
             if (to_cache) *reinterpret_cast<u32x2_t*>(cache + slot * nkv * 128 + col) = v;
         }
@@ -214,11 +232,24 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
     if (first >= mcnt) return;
     if constexpr (MODE == GEMM_PLAIN && RT == 4) {
         if (p.qkv_q != nullptr) {
-            midm_qkv_rows<MPW>(p, sum, m0 + first, mcnt - first, ncol0, c, g4);
+            midm_qkv_rows<4, MPW>(p, sum, m0 + first, mcnt - first, ncol0, 0, c, g4);
             return;
         }
     }
     gemm_row_epilogue<MODE, RT, MPW>(p, sum, grp, m0 + first, mcnt - first, ncol0, c, g4);
+}
+
+// row block and column tile of this workgroup
+__device__ __forceinline__ void midm_tile(int mblocks, int interleaved, int& m, int& ntile) {
+    if (interleaved) {   // column tiles dealt to the XCDs (workgroups b, b + 8, ...) one by one, their row blocks behind one another
+        const int q = blockIdx.x >> 3;
+        m = q % mblocks;
+        ntile = q / mblocks * 8 + (blockIdx.x & 7);
+    } else {             // few column tiles: an XCD takes a run of all tiles
+        const int lin = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+        ntile = lin / mblocks;
+        m = lin % mblocks;
+    }
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
@@ -228,17 +259,9 @@ constexpr int midm_lds() {
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
-__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p_in, int mblocks, int interleaved) {
-    GemmParams p = p_in;
+__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, int mblocks, int interleaved) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int COLS = gemm_paired(MODE) ? 8 * RT : 16 * RT;
-    if (MODE == GEMM_PLAIN && p_in.ksplit > 1) {   // K slice of this workgroup (whole pairs of chunks)
-        const int per = (p_in.K / 64 + p_in.ksplit - 1) / p_in.ksplit * 64, kb = blockIdx.z * per;
-        p.x = p_in.x + kb;
-        p.w = p_in.w + kb;
-        p.K = max(0, min(per, p_in.K - kb));
-        p.ypart = p_in.ypart + (int64_t)blockIdx.z * p_in.R * p_in.N;
-    }
     int grp = 0, m0, mcnt, ntile;
     if (p.offs) {
         int* sh = reinterpret_cast<int*>(smem + midm_lds<MODE, MT, RT, NW, NST>() - 16);
@@ -251,20 +274,119 @@ __global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p_i
         if (grp < 0) return;
     } else {
         int m;
-        if (interleaved) {   // column tiles dealt to the XCDs (workgroups b, b + 8, ...) one by one, their row blocks behind one another
-            const int q = blockIdx.x >> 3;
-            m = q % mblocks;
-            ntile = q / mblocks * 8 + (blockIdx.x & 7);
-        } else {             // few column tiles: an XCD takes a run of all tiles
-            const int lin = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-            ntile = lin / mblocks;
-            m = lin % mblocks;
-        }
+        midm_tile(mblocks, interleaved, m, ntile);
         m0 = m * (16 * MT);
         mcnt = min(16 * MT, (int)p.R - m0);
     }
     if (ntile * COLS >= p.N) return;
     midm_body<MODE, MT, RT, NW, NST>(p, smem, grp, m0, mcnt, ntile * COLS);
+}
+
+// rows m0 .. m0 + mcnt - 1, columns from ncol0, tile shared by the workgroup: WM x WN waves of MT x RT 16-row tiles each.  Every wave brings
+// its share of a stage (one 64-wide K chunk of all rows); the counted wait is for its own share, the barrier behind it for the others', and
+// it also says that every wave has the stage before in registers: its slot takes the chunk NST - 1 ahead.
+template <int MODE, int WM, int WN, int MT, int RT, int NST>
+__device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem, int m0, int mcnt, int ncol0, int slice) {
+    static_assert(RT == 2, "the QKV epilogue takes the two columns that turn together from one lane");
+    constexpr int NW = WM * WN, WR = 16 * RT * WN, XR = 16 * MT * WM;   // weight rows and activation rows of a stage
+    constexpr int STAGE = (WR + XR) * MM_ROWB, D = (WR + XR) / 8 / NW, DW = WR / 8 / NW;
+    constexpr int HALF = 8 * RT;               // paired modes: gate rows of a wave's columns, then as many up rows
+    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && NST >= 2, "whole DMA instructions per wave");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wid % WN, wm = wid / WN;
+    const int c = lane & 15, g4 = lane >> 4;
+    const unsigned ring = (unsigned)(uintptr_t)(const mm_lds_void*)smem;
+    const int r8 = lane >> 3, pc = lane & 7;
+    const int K = p.ksplit > 1 ? p.K / p.ksplit : p.K;   // (equal slices of whole chunks)
+    const __amdgpu_buffer_rsrc_t wrs = mm_rsrc(p.w + (int64_t)slice * K), xrs = mm_rsrc(p.x + (int64_t)slice * K);
+    const bool qkv = MODE == GEMM_PLAIN && p.qkv_q != nullptr;   // a wave's two row tiles are 32 columns apart
+    unsigned vo[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+        const bool isw = i < DW;
+        const int row = 8 * ((isw ? i : i - DW) * NW + wid) + r8;
+        int src;
+        if (!isw) src = m0 + min(row, mcnt - 1);    // rows past the end repeat the last one; they are never stored
+        else if (gemm_paired(MODE)) {
+            const int rr = row % (16 * RT), col = ncol0 + row / (16 * RT) * HALF + rr % HALF;
+            src = (rr < HALF ? 0 : p.N) + min(col, p.N - 1);
+        } else src = min(ncol0 + (qkv ? (row & ~63) + (row >> 5 & 1) * 16 + (row >> 4 & 1) * 32 + (row & 15) : row), p.N - 1);
+        vo[i] = ((unsigned)src * (unsigned)(isw ? p.ldw : p.ldx) + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
+    }
+    const int n = K / MM_KC;
+    auto issue = [&](int j, int slot) {
+        const int soff = j * MM_ROWB;
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            const bool isw = i < DW;
+            char* dst = smem + slot * STAGE + (isw ? 0 : WR * MM_ROWB) + ((isw ? i : i - DW) * NW + wid) * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? wrs : xrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 0);
+        }
+    };
+    f32x4_t acc[RT][MT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    unsigned rel_w[2], rel_x[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        const unsigned r = c * MM_ROWB + (((4 * ks + g4) ^ ((c >> 1) & 7)) << 4);
+        rel_w[ks] = r + wn * RT * 2048;
+        rel_x[ks] = r + WR * MM_ROWB + wm * MT * 2048;
+    }
+#pragma unroll
+    for (int j = 0; j < NST - 1; ++j)
+        if (j < n) issue(j, j);
+    int slot = 0;
+    for (int j = 0; j < n; ++j) {
+        if (j + NST - 1 <= n) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((NST - 2) * D) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        MmShared<MT, RT> f0, f1;
+        const unsigned st = ring + slot * STAGE;
+        f0.read(st + rel_w[0], st + rel_x[0]);
+        if (j + NST - 1 < n) issue(j + NST - 1, slot == 0 ? NST - 1 : slot - 1);
+        f0.settle();
+        f1.read(st + rel_w[1], st + rel_x[1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f0.w[rt]), __builtin_bit_cast(bf16x8_t, f0.x[mt]), acc[rt][mt], 0, 0, 0);
+        f1.settle();
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f1.w[rt]), __builtin_bit_cast(bf16x8_t, f1.x[mt]), acc[rt][mt], 0, 0, 0);
+        slot = slot + 1 == NST ? 0 : slot + 1;
+    }
+    const int first = 16 * MT * wm;
+    if (first >= mcnt) return;
+    if constexpr (MODE == GEMM_PLAIN) {
+        if (qkv) {
+            midm_qkv_rows<2, MT>(p, acc, m0 + first, mcnt - first, ncol0 + wn / 2 * 64, wn % 2 * 16, c, g4);
+            return;
+        }
+    }
+    // (slab s of the partial sums: rows s R ..)
+    gemm_row_epilogue<MODE, RT, MT>(p, acc, 0, slice * (int)p.R + m0 + first, mcnt - first, ncol0 + wn * (gemm_paired(MODE) ? HALF : 16 * RT), c, g4);
+}
+
+template <int WM, int WN, int MT, int RT, int NST>
+constexpr int midm_shared_lds() { return NST * (16 * RT * WN + 16 * MT * WM) * MM_ROWB; }
+
+template <int MODE, int WM, int WN, int MT, int RT, int NST>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_midm_shared_kernel(const GemmParams p, int mblocks, int interleaved) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    constexpr int COLS = (gemm_paired(MODE) ? 8 : 16) * RT * WN, ROWS = 16 * MT * WM;
+    int m, ntile;
+    midm_tile(mblocks, interleaved, m, ntile);
+    if (ntile * COLS >= p.N) return;
+    midm_shared_body<MODE, WM, WN, MT, RT, NST>(p, smem, m * ROWS, min(ROWS, (int)p.R - m * ROWS), ntile * COLS, blockIdx.z);
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
@@ -279,29 +401,63 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
     GLM_CHECK_ARG(gx < (1 << 30) && gy <= 65535, GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
     auto kern = gemm_midm_kernel<MODE, MT, RT, NW, NST>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
-    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt);
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt);
     GLM_CHECK_LAUNCH("gemm_midm");
     return GLM_OK;
 }
 
-// tiles of 64 rows and 32 columns
-int64_t small_tiles(int mode, const GemmParams& p) {
-    const int cols = gemm_paired(mode) ? 16 : 32;
-    return (int64_t)((p.N + cols - 1) / cols) * ((p.R + 63) / 64);
+template <int MODE, int WM, int WN, int MT, int RT, int NST>
+int launch_midm_shared(const GemmParams& p, hipStream_t st) {
+    constexpr int LDS = midm_shared_lds<WM, WN, MT, RT, NST>();
+    static_assert(LDS <= 160 * 1024, "the ring must fit the CU's LDS");
+    const int cols = (gemm_paired(MODE) ? 8 : 16) * RT * WN, nt = (p.N + cols - 1) / cols;
+    const int64_t mblocks = (p.R + 16 * MT * WM - 1) / (16 * MT * WM);
+    const bool dealt = nt >= 64;
+    const int64_t gx = dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8;
+    GLM_CHECK_ARG(gx < (1 << 30), GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
+    auto kern = gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST>;
+    if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx, 1, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(WM * WN * 64), LDS, st, p, (int)mblocks, (int)dealt);
+    GLM_CHECK_LAUNCH("gemm_midm");
+    return GLM_OK;
 }
 
-// Up to a workgroup per CU: 64 x 32 with four waves.  Beyond: workgroups of two waves, three to a CU, so that one's start and end lie under
-// the others' loops.  A long K pays those once per tile and the activation traffic always: 64 x 64.  Four waves 64 x 32, two waves 64 x 32,
-// four waves 64 x 64, us, cold operands: 2048 x 2048 at 128 rows (128 tiles) 8.2 / 10.7 / 15.8; 6144 x 2048 at 256 (768) 20.6 / 17.0 / 34.0;
-// 14336 x 4096 at 128 (896) 58.9 / 55.4 / 59.3; 4096 x 12288 at 128 (256) 42.7 / 53.4 / 66.2, at 256 (512) 74.2 / 79.5 / 66.1.
+// The tile of a dense projection: the first of these with a workgroup per CU at most.  More and smaller workgroups put more of the chip to
+// work and have more bytes on their way; a larger tile pulls fewer, and two rounds of one cost more than one round of the next.  Split, 64 x 64,
+// 128 x 64, 128 x 128 (64 rows: 64 x 128), us, cold operands, * the one taken: 4096 x 4096 at 64 rows 16.5* / 21.2 / - / 30, at 211 24.5 / 20.5* /
+// 30.0 / 36.2, at 512 47 / - / 31.8* / 40.2; 14336 x 4096 at 64 36.7 / 27.6* / - / 37.5, at 128 56 / 42.6 / 37.7* / 46.3, at 211 77 / 61.5 / 52 /
+// 43.0*; 2048 x 2048 at 1000 rows - / 16.9* / 17.2 / 19.8, at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
+// A long K favours split waves at 64 x 64 too, which read each staged byte once: 4096 x 12288 at 211 rows 50 (shared 58), K = 8192 36 (40).
+enum MidmTile { MM_NONE, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
+
+MidmTile midm_tile_of(int mode, const GemmParams& p) {
+    const int64_t n = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
+    auto fits = [&](int rows, int cols) { return (n + cols - 1) / cols * ((p.R + rows - 1) / rows) <= 256; };
+    // (K steps of a short reduction are few: what the tiled kernel adds up in order stays so there for more rows)
+    if (fits(64, 32) && (p.K > 512 || p.R <= 256)) return MM_SPLIT32;
+    if (fits(64, 64)) return p.K >= 8192 ? MM_SPLIT64 : MM_64;
+    if (p.R <= 64) return fits(64, 128) ? MM_64x128 : MM_NONE;
+    if (fits(128, 64)) return MM_128x64;
+    return fits(128, 128) ? MM_128 : MM_NONE;
+}
+
 template <int MODE>
 int launch_midm(const GemmParams& p, hipStream_t st) {
     // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
     // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
     if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
-    if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);   // (half a head; the sums are the same in both tiles)
-    if (small_tiles(MODE, p) <= 256) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
-    return p.K >= 8192 ? launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st) : launch_midm_cfg<MODE, 4, 2, 2, 2>(p, st);
+    switch (midm_tile_of(MODE, p)) {
+        case MM_SPLIT32:   // (half a head in the QKV epilogue; the sums are the same in both tiles)
+            if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
+            [[fallthrough]];
+        case MM_SPLIT64: return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);
+        case MM_64: return launch_midm_shared<MODE, 2, 2, 2, 2, 4>(p, st);
+        case MM_128x64: return launch_midm_shared<MODE, 2, 2, 4, 2, 3>(p, st);
+        case MM_64x128: return launch_midm_shared<MODE, 2, 4, 2, 2, 3>(p, st);
+        case MM_128: return launch_midm_shared<MODE, 2, 4, 4, 2, 4>(p, st);
+        default: break;
+    }
+    GLM_CHECK_ARG(false, GLM_ERR_UNSUPPORTED, "gemm_midm: no tile for %ld rows, N=%d", (long)p.R, p.N);
 }
 
 }  // namespace
@@ -320,22 +476,12 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     if (p.src != nullptr || p.G > 1 || p.R <= 32) return false;
     // (a loop of the tiled kernel that is asked for keeps its shapes)
     if (p.R >= 96 && (glm_option(GLM_OPT_LARGEM_VARIANT) >= 0 || glm_option(GLM_OPT_LARGEM_CFG) != 0)) return false;
-    const bool paired = gemm_paired(mode);
-    const int64_t wrows = paired ? 2 * (int64_t)p.N : (int64_t)p.N;
+    const int64_t wrows = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
     if (p.R * p.ldx * 2 >= (1ll << 31) || wrows * p.ldw * 2 >= (1ll << 31)) return false;   // 32-bit offsets
-    const int64_t tiles = small_tiles(mode, p);
-    // Fewer rows than the tiled kernel takes: the weight-streaming kernel gets ahead where it has a wave of workgroups to spare (32768 x 2048
-    // at 64 rows, 1024 tiles, 31 us, here 35; 18944 x 4096, 592, 50 / 49; 14336 x 4096 45 / 37; 2048 x 6144 62 / 16).
-    // A gated projection runs there in blocks of 32 rows: 10944 gated columns x 4096 (684 tiles) 75 us, here 52.
-    if (p.R < 96) return tiles <= (paired ? 1100 : 600);
-    // (A short reduction is a handful of steps of the tiled kernel's loop: K = 512, 128 rows: 2048 columns 11.5 / 4.8, 14336 (896 tiles)
-    // 13.6 / 12.0; 256 rows: 2048 16.9 / 4.9, 14336 (1792) 18.7 / 20.8.  Beyond 256 rows nothing here has such a projection and few columns.)
-    if (p.K <= 512) return p.R <= 256 && tiles <= 900;
-    // The tiled kernel's time is its K loop's as long as its tiles are one round of the chip; here it grows with the tiles (L2 -> LDS
-    // traffic, about 11 TB/s).  Tiled / here, us: 2048 x 6144 at 128 rows (128 tiles) 68 / 16, 6144 x 2048 at 256 (768) 28 / 17, 14336 x 4096
-    // at 128 (896) 66 / 55, 9728 x 2048 at 200 (1216) 33 / 33, 6144 x 2048 at 400 (1344) 28 / 29, 14336 x 4096 at 200 (1792) 60 / 77.
-    const int64_t big = (p.R + 127) / 128 * ((p.N + (paired ? 127 : 255)) / (paired ? 128 : 256));
-    return tiles <= 1100 * ((big + 255) / 256);
+    // Beyond one round of the largest tile the tiled kernel's 128 x 256 and 256 x 256 ones pull less (14336 x 4096 at 400 rows, 448 tiles: 60 us
+    // there, 76 here; 9728 x 2048 at 400, 304: 31 / 39; 6144 x 2048 at 1000, 384: 33 / 42), and 64 rows of more than 32768 columns stay with
+    // the weight-streaming kernel.
+    return midm_tile_of(mode, p) != MM_NONE;
 }
 
 int glm_launch_gemm_midm(int mode, const GemmParams& p, hipStream_t st) {

@@ -1,4 +1,4 @@
-"""Projections of 33 to some hundred rows (csrc/gemm_midm.hip): both tiles, every epilogue, ragged rows and columns, waves without a chunk
+"""Projections of 33 to some hundred rows (csrc/gemm_midm.hip): every tile, every epilogue, ragged rows and columns, waves without a chunk
 of K — against the operators in fp64 on the same bf16 operands.  A result is one rounding of an fp32 sum of K products: off by at most half
 a bf16 ulp plus the sum's error (K terms of the size of the result at most: 2e-6 of the row's absolute sum, far below an ulp), so by one ulp
 where that sum lies on a rounding boundary."""
@@ -35,12 +35,13 @@ def close(got, ref, what):
 # absolute one is 2^-8 of the factors (of the order of one).
 SILU = (4, 0.06, 2 ** -8)
 
-# (rows, columns, K): one column of tiles and many, more than 256 small tiles (the 64-column one), K of one chunk (three waves without
-# work) up to several rounds of the ring, columns that end inside a tile, rows that end inside a block, the large tile of long reductions,
-# and one of the tiled kernel's (its epilogues)
-SIZES = [(33, 36, 64), (64, 100, 128), (65, 2048, 192), (97, 2052, 1088), (211, 2112, 2048), (256, 8200, 576), (33, 16420, 320), (128, 264, 4096),
-         (520, 1000, 1024), (130, 4128, 8256),
-         (1300, 2056, 128)]
+# (rows, columns, K): split waves (K of one chunk, three waves without work, up to several rounds of the ring; the large tile of long
+# reductions), then every tile of the shared ring, fewer chunks than stages and many, columns that end inside a tile, rows that end inside a
+# block, and one of the tiled kernel's (its epilogues)
+SIZES = [(33, 36, 64), (64, 100, 128), (65, 2048, 192), (97, 2052, 1088), (128, 264, 4096), (130, 4128, 8256),
+         (211, 2112, 2048), (520, 1000, 1024), (300, 3000, 64), (130, 6404, 64), (129, 5700, 704), (33, 16420, 320), (64, 20000, 128), (256, 8200, 576),
+         (1300, 2056, 128),
+         (1300, 6152, 128)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
@@ -80,7 +81,8 @@ def test_activations(ops, M, N, K):
     assert ((capped - N_.soft_cap(z, 3.0)).abs() <= bound + 2e-6).all()
 
 
-@pytest.mark.parametrize("M,I,K", [(33, 24, 64), (65, 1000, 192), (97, 1408, 1088), (211, 4104, 576), (300, 264, 1024)])
+@pytest.mark.parametrize("M,I,K", [(33, 24, 64), (65, 1000, 192), (97, 1408, 1088), (211, 4104, 576), (300, 264, 1024), (100, 3000, 128), (130, 3016, 64),
+                                   (64, 9000, 192)])
 def test_gated(ops, M, I, K):
     x, w = rnd(M, K, seed=6), rnd(2 * I, K, seed=7, scale=K ** -0.5)
     g, u = (x.double() @ w.double().T).chunk(2, 1)
@@ -126,7 +128,7 @@ def test_one_row_feed_forward(ops, M, I):
     close(ops.grouped_gemm_down(act, d.cuda().unsqueeze(0), None, None, 0), act.cpu().double() @ d.double().T, "down")
 
 
-@pytest.mark.parametrize("T,nh,nkv,K", [(97, 4, 1, 1024), (211, 6, 2, 640), (256, 2, 2, 512)])
+@pytest.mark.parametrize("T,nh,nkv,K", [(97, 4, 1, 1024), (211, 6, 2, 640), (256, 2, 2, 512), (450, 6, 2, 576), (130, 40, 2, 128), (211, 96, 8, 320)])
 def test_qkv_epilogue(ops, T, nh, nkv, K):
     """Split, rotation and cache rows in the projection's epilogue: the projection and the split kernel, bit for bit."""
     x, w, b = rnd(T, K, seed=9).cuda(), rnd((nh + 2 * nkv) * 128, K, seed=10, scale=K ** -0.5).cuda(), rnd((nh + 2 * nkv) * 128, seed=11).cuda()
