@@ -282,6 +282,14 @@ extern "C" int glm_gemm_bf16_slices(int64_t M, int N, int K) {
     return best;
 }
 
+// ... and from 33 rows on: the tiles of gemm_midm.hip first, then those of the tiled kernel where K is long enough to pay for their sums (with
+// the norm that adds them up, us, one pass / slices: 4096 x 4096 at 400 rows 36 / 39, at 1000 50 / 54; 2048 x 6144 at 700 47 / 40, at 1000
+// 50 / 46; 4096 x 12288 at 400 95 / 62, at 1000 123 / 101)
+extern "C" int glm_gemm_bf16_row_slices(int64_t M, int N, int K) {
+    const int s = glm_midm_slices(M, N, K);
+    return s > 1 ? s : K >= 6144 ? glm_gemm_bf16_slices(M, N, K) : 1;
+}
+
 extern "C" int glm_gemm_bf16_partial(const void* x, int64_t ldx, const void* w, int64_t ldw, float* ypart,
                                      int64_t M, int N, int K, int nslices, glm_stream_t stream) {
     GLM_CHECK_ARG(x && w && ypart, GLM_ERR_INVALID, "glm_gemm_bf16_partial: null pointer");
@@ -293,13 +301,15 @@ extern "C" int glm_gemm_bf16_partial(const void* x, int64_t ldx, const void* w, 
     p.x = (const bf16_t*)x; p.ldx = ldx;
     p.w = (const bf16_t*)w; p.w_gstride = 0; p.ldw = ldw;
     p.R = M; p.N = N; p.K = K; p.G = 1;
+    p.ksplit = nslices; p.ypart = ypart;
+    if (glm_midm_takes_slices(p)) return glm_launch_gemm_midm_slices(p, glm_s(stream));
     if (M >= LARGEM_MIN_AVG_ROWS) {
+        p.ksplit = 0; p.ypart = nullptr;
         GLM_CHECK_ARG(K % (64 * nslices) == 0 && glm_aligned16(ypart) && N % 8 == 0, GLM_ERR_UNSUPPORTED, "glm_gemm_bf16_partial: K=%d in %d slices of whole tiles", K, nslices);
         p.K = K / nslices; p.G = nslices; p.w_gstride = p.K;
         p.yf = ypart; p.y = (bf16_t*)ypart; p.ldy = N;  // (y: alignment checks only)
         return glm_launch_gemm_largem(GEMM_SLICES, p, glm_s(stream));
     }
-    p.ksplit = nslices; p.ypart = ypart;
     return glm_launch_gemm_smallm_partial(p, glm_s(stream));
 }
 

@@ -157,6 +157,10 @@ int glm_launch_gemm_smallm_fp8w(int mode, const GemmParams& p, hipStream_t st);
 // some dozen to some hundred rows of one weight matrix (gemm_midm.hip); takes: the shape belongs there, by size and form
 bool glm_midm_takes(int mode, const GemmParams& p);
 int glm_launch_gemm_midm(int mode, const GemmParams& p, hipStream_t st);
+// fp32 partial sums of p.ksplit slices of K there (p.ypart), a slab of R rows each; slices: how many pay, 1 if none do
+int glm_midm_slices(int64_t M, int N, int K);
+bool glm_midm_takes_slices(const GemmParams& p);
+int glm_launch_gemm_midm_slices(const GemmParams& p, hipStream_t st);
 // LDS-tiled MFMA kernels for many rows per group (prefill); p.wscale != nullptr: per-weight-row fp32 scale applied to
 // the accumulator before the bf16 roundings (weights expanded from fp8, elementwise.hip)
 int glm_launch_gemm_largem(int mode, const GemmParams& p, hipStream_t st);

@@ -442,11 +442,8 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
 }
 
 template <int MODE>
-int launch_midm(const GemmParams& p, hipStream_t st) {
-    // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
-    // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
-    if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
-    switch (midm_tile_of(MODE, p)) {
+int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
+    switch (tile) {
         case MM_SPLIT32:   // (half a head in the QKV epilogue; the sums are the same in both tiles)
             if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
             [[fallthrough]];
@@ -458,6 +455,35 @@ int launch_midm(const GemmParams& p, hipStream_t st) {
         default: break;
     }
     GLM_CHECK_ARG(false, GLM_ERR_UNSUPPORTED, "gemm_midm: no tile for %ld rows, N=%d", (long)p.R, p.N);
+}
+
+template <int MODE>
+int launch_midm(const GemmParams& p, hipStream_t st) {
+    // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
+    // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
+    if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
+    return launch_midm_tile<MODE>(midm_tile_of(MODE, p), p, st);
+}
+
+// K slices of a projection whose tiles are a quarter of the chip at most, and the tile for them: as many as bring a workgroup to every CU.  A
+// smaller tile with at least four slices goes before a larger one with more (fewer partial sums for the same workgroups).  One pass / slices, us:
+// 4096 x 12288 at 64 rows 45 / 23 (4 of 64 x 64), at 128 43 / 31 (4 of 128 x 64; 8 of 128 x 128 27), at 211 56 / 37 (4 of 128 x 128; the tiled
+// kernel's 16 38); 2048 x 8192 at 64 26 / 10, at 128 25 / 13 (the tiled kernel's 16 19), at 400 41 / 25 (28).  K = 2048: 8.1 / 6.7, which the
+// consumer's wider reads take back.
+int midm_slices(int64_t M, int N, int K, MidmTile* tile) {
+    if (M <= 32 || K % 64 != 0 || K < 4096 || N % 4 != 0) return 1;
+    static const struct { MidmTile t; int rows, cols; } tiles[] = {{MM_64, 64, 64}, {MM_128x64, 128, 64}, {MM_128, 128, 128}};
+    for (const auto& c : tiles) {
+        if ((c.rows == 64) != (M <= 64)) continue;
+        const int64_t n = (M + c.rows - 1) / c.rows * ((N + c.cols - 1) / c.cols);
+        int best = 1;
+        for (int s = 2; s <= 8 && s * n <= 256 && K / s >= 512; ++s)
+            if (K % (64 * s) == 0) best = s;
+        if (best < 4) continue;
+        *tile = c.t;
+        return best;
+    }
+    return 1;
 }
 
 }  // namespace
@@ -482,6 +508,26 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     // there, 76 here; 9728 x 2048 at 400, 304: 31 / 39; 6144 x 2048 at 1000, 384: 33 / 42), and 64 rows of more than 32768 columns stay with
     // the weight-streaming kernel.
     return midm_tile_of(mode, p) != MM_NONE;
+}
+
+int glm_midm_slices(int64_t M, int N, int K) {
+    MidmTile tile;
+    return midm_slices(M, N, K, &tile);
+}
+
+bool glm_midm_takes_slices(const GemmParams& p) {
+    MidmTile tile;
+    if (p.R <= 32 || p.K % (64ll * p.ksplit) != 0 || p.R * p.ldx * 2 >= (1ll << 31) || (int64_t)p.N * p.ldw * 2 >= (1ll << 31)) return false;
+    // (up to 95 rows there is no other kernel for slices of another number)
+    return p.R < 96 || midm_slices(p.R, p.N, p.K, &tile) == p.ksplit;
+}
+
+int glm_launch_gemm_midm_slices(const GemmParams& p, hipStream_t st) {
+    GLM_CHECK_ARG(p.N % 4 == 0 && p.ldx % 8 == 0 && p.ldw % 8 == 0 && glm_aligned16(p.x) && glm_aligned16(p.w) && glm_aligned16(p.ypart), GLM_ERR_UNSUPPORTED,
+                  "gemm_midm(slices): needs N%%4==0, ldx/ldw%%8==0, 16B-aligned x/W/partial sums (N=%d)", p.N);
+    MidmTile tile = p.R <= 64 ? MM_64 : MM_128x64;
+    midm_slices(p.R, p.N, p.K, &tile);
+    return launch_midm_tile<GEMM_PLAIN>(tile, p, st);
 }
 
 int glm_launch_gemm_midm(int mode, const GemmParams& p, hipStream_t st) {

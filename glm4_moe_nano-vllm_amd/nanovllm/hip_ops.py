@@ -179,6 +179,7 @@ _SIGNATURES = {
     "glm_group_norm_store": (c_int, [c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_float,
         c_float, c_int, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "glm_gemm_bf16_slices": (c_int, [c_int64, c_int, c_int]),
+    "glm_gemm_bf16_row_slices": (c_int, [c_int64, c_int, c_int]),
     "glm_residual_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
         c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_int, c_float, c_void_p]),
     "glm_memory_recurrent": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p,
@@ -1220,7 +1221,7 @@ class PartialSum:
 
 
 def gemm_bf16_partial(x: torch.Tensor, w: torch.Tensor, want_slices: int = 8) -> PartialSum:
-    """K-slice partial sums of x @ w.T for decode batches: M <= 32, or gemm_slices of them; see glm_gemm_bf16_partial."""
+    """K-slice partial sums of x @ w.T: up to 32 rows, or row_slices / gemm_slices of them; see glm_gemm_bf16_partial."""
     _bf16(x, "x"); _bf16(w, "w")
     K = x.shape[-1]
     N = w.shape[0]
@@ -1237,6 +1238,11 @@ def gemm_bf16_partial(x: torch.Tensor, w: torch.Tensor, want_slices: int = 8) ->
 def gemm_slices(M: int, N: int, K: int) -> int:
     """K slices that spread a projection of some hundred rows over the chip (1: its output tiles do)."""
     return load_library().glm_gemm_bf16_slices(M, N, K)
+
+
+def row_slices(M: int, N: int, K: int) -> int:
+    """gemm_slices from 33 rows on, the tiles for fewer rows first."""
+    return load_library().glm_gemm_bf16_row_slices(M, N, K)
 
 
 def add_rmsnorm_partial(ps: PartialSum, residual: torch.Tensor, weight: torch.Tensor,

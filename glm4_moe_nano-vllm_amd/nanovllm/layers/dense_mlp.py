@@ -36,8 +36,13 @@ class DenseMLP(nn.Module):
         self.down.load([w["down"][:, lo: lo + self.ff]], device)
         self.act = xielu_constants(w["act"])
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
-        y = self.down(self.up(h, act=self.act))
+    def forward(self, h: torch.Tensor):
+        """[T, width], or its K-slice partial sums, which the norm behind it adds up (2048 x 6144 at 128 rows with that norm 19 -> 15 us)."""
+        u = self.up(h, act=self.act)
+        slices = hip_ops.row_slices(h.shape[0], self.down.N, self.down.K) if self.tp_size == 1 and u.dtype == torch.bfloat16 else 1
+        if slices > 1:
+            return hip_ops.gemm_bf16_partial(u, self.down.weight, slices)
+        y = self.down(u)
         if self.tp_size > 1:
             get_tp_group().all_reduce(y)
         return y

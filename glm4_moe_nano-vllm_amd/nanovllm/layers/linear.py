@@ -140,17 +140,22 @@ class RowParallelLinear(LinearBase):
     partial_min_k = 8192
     partial_slices = 8
 
-    @staticmethod
-    def _partial_rows(m: int) -> bool:
+    partial_max_rows = 1024   # (the norm and the router behind it are launches of their own from here on)
+
+    def _slices(self, m: int) -> int:
+        if m > 32:   # 4096 x 12288: 64 rows 45 -> 23 us, 211 rows 56 -> 37, 400 rows 108 -> 50
+            return hip_ops.row_slices(m, *self.weight.shape) if m < self.partial_max_rows else 1
         lo = 1 if hip_ops.opt("tinym") != 0 else 0  # one row: the GEMV body (glm_gemm_bf16 picks it)
-        return lo < m <= 32
+        return self.partial_slices if m > lo else 1
 
     def forward(self, x: torch.Tensor, defer_reduce: bool = False):
         # (not for a single row: the single-sequence GEMV body streams the whole reduction per row and needs no K split)
-        if (defer_reduce and self.tp_size == 1 and self.bias is None and x.dim() == 2 and self._partial_rows(x.shape[0])
+        if (defer_reduce and self.tp_size == 1 and self.bias is None and x.dim() == 2
                 and x.shape[1] >= self.partial_min_k and x.shape[1] >= 2 * self.weight.shape[0]
                 and x.shape[1] % 8 == 0 and x.stride(1) == 1):
-            return hip_ops.gemm_bf16_partial(x, self.weight.data, self.partial_slices)
+            slices = self._slices(x.shape[0])
+            if slices > 1:
+                return hip_ops.gemm_bf16_partial(x, self.weight.data, slices)
         y = self._gemm(x, with_bias=self.tp_rank == 0)
         if self.tp_size > 1:
             get_tp_group().all_reduce(y)

@@ -46,7 +46,7 @@ class ParallelBlock(nn.Module):
         """K slices of the output projection, summed up by the next norm (few rows, or few output tiles; not across ranks)."""
         if self.tp_size > 1 or T == 1 or self.out_proj.K < PARTIAL_MIN_K:
             return 1
-        return PARTIAL_SLICES if T <= PARTIAL_ROWS else hip_ops.gemm_slices(T, self.wp, self.out_proj.K)
+        return PARTIAL_SLICES if T <= PARTIAL_ROWS else hip_ops.row_slices(T, self.wp, self.out_proj.K)
 
     def forward(self, h: torch.Tensor, meta, run: int = 0, cs: torch.Tensor | None = None):
         """What the layer adds to the residual, [T, wp] (or its K-slice partial sums)."""

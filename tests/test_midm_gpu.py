@@ -142,3 +142,22 @@ def test_qkv_epilogue(ops, T, nh, nkv, K):
     q2, k2, v2 = ops.qkv_split_norm_rope_store(ops.gemm_bf16(x, w, b), nh, nkv, 128, pos, cs, 64, None, None, 1e-5, caches[2], caches[3], slots.cuda(), True)
     assert torch.equal(q, q2) and torch.equal(k, k2) and torch.equal(v, v2)
     assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 100, 4096), (64, 2052, 6144), (95, 1000, 4608), (130, 2048, 8192), (211, 4096, 4096), (500, 2048, 6144), (400, 4096, 8192)])
+def test_row_slices(ops, M, N, K):
+    """Partial sums of K slices, out of wider rows: every slab its own slice's fp32 sum (K products of magnitude |x| |w|)."""
+    xw, w = rnd(M, K + 16, seed=40), rnd(N, K, seed=41, scale=K ** -0.5)
+    x = xw[:, 8: 8 + K]
+    best = ops.row_slices(M, N, K)
+    assert best >= 4 and ops.row_slices(M, N, K + 8) == 1 and ops.row_slices(32, N, K) == 1
+    for ns in sorted({best, 2} if M < 96 else {best}):
+        part = ops.gemm_bf16_partial(xw.cuda()[:, 8: 8 + K], w.cuda(), ns).part.cpu().double()
+        assert part.shape == (ns, M, N)
+        k = K // ns
+        for s in range(ns):
+            a, b = x[:, s * k: (s + 1) * k].double(), w[:, s * k: (s + 1) * k].double()
+            assert ((part[s] - a @ b.T).abs() <= 2.0 ** -23 * 8 * (a.abs() @ b.abs().T) + 1e-7).all(), (ns, s)
+    if M < 96:
+        with pytest.raises(RuntimeError):
+            ops.gemm_bf16_partial(x.cuda(), w.cuda(), 7)
