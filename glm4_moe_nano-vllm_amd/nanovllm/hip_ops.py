@@ -642,11 +642,15 @@ def varlen_attn_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, scale
 # a [T, H] x [H, E] GEMM, and glm_router_select does R2..R7 from them; below, the token-per-workgroup kernel
 # (glm_router_topk / the fused add-RMSNorm + router + bucketing launch), which is built for decode latency: at T = 16384
 # it takes 1.2 ms per layer against 0.34 ms for norm + GEMM + select + bucketing (tools/prefill_router_probe.py).
+# That kernel reads all of Wg for every other token, so it also falls behind with tokens x experts.  One launch / four, us, hidden size 4096, in
+# parentheses from four K slices of o_proj: 64 experts at 128 tokens 16 / 22 (21 / 23), at 211 24.0 / 23.5 (37 / 25), at 700 58 / 35 (96 / 37);
+# 128 experts at 96 tokens 21 / 23 (29 / 25), at 128 25.0 / 24.6 (35 / 26).
 ROUTER_GEMM_MIN_ROWS = 1024
+ROUTER_GEMM_MIN_LOGITS = 12288
 
 
 def router_by_gemm(T: int, E: int) -> bool:
-    return T >= ROUTER_GEMM_MIN_ROWS and E % 8 == 0  # the GEMM kernels want 16-byte output rows
+    return (T >= ROUTER_GEMM_MIN_ROWS or T * E >= ROUTER_GEMM_MIN_LOGITS) and E % 8 == 0  # the GEMM kernels want 16-byte output rows
 
 
 def router_select(logits: torch.Tensor, bias: torch.Tensor, k: int, routed_scaling_factor: float):
@@ -712,9 +716,9 @@ def add_rmsnorm_router_topk(x, residual: torch.Tensor, norm_weight: torch.Tensor
     r2 = residual.reshape(-1, H).contiguous()
     T = r2.shape[0]
     E = gate_w.shape[0]
-    if router_by_gemm(T, E) and not isinstance(x, PartialSum):
+    if router_by_gemm(T, E):
         # prefill sizes: norm, logits GEMM + selection, bucketing as separate launches (see ROUTER_GEMM_MIN_ROWS)
-        yn, rn = add_rmsnorm(x.reshape(-1, H), r2, norm_weight, eps)
+        yn, rn = add_rmsnorm_partial(x, r2, norm_weight, eps) if isinstance(x, PartialSum) else add_rmsnorm(x.reshape(-1, H), r2, norm_weight, eps)
         idx, w = router_topk(yn, gate_w, bias, k, routed_scaling_factor)
         if align_with_shared is None:
             return yn.view(residual.shape), rn.view(residual.shape), idx, w

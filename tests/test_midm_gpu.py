@@ -161,3 +161,24 @@ def test_row_slices(ops, M, N, K):
     if M < 96:
         with pytest.raises(RuntimeError):
             ops.gemm_bf16_partial(x.cuda(), w.cuda(), 7)
+
+
+@pytest.mark.parametrize("T,E,slices", [(192, 64, 4), (191, 64, 4), (97, 128, 8), (300, 64, 0)])
+def test_norm_and_router_of_slices(ops, T, E, slices):
+    """The norm behind a projection (its partial sums or its rows), the router and the bucketing: as launches of their own, on either side of the
+    number of logits from which they are."""
+    H, k = 1024, 4
+    rows = rnd(T, H, seed=50).cuda()
+    parts = torch.randn(slices, T, H, generator=torch.Generator().manual_seed(51)).cuda() if slices else None
+    res, nw, gw = rnd(T, H, seed=52).cuda(), (1 + 0.1 * rnd(H, seed=53).float()).to(BF).cuda(), rnd(E, H, seed=54, scale=H ** -0.5).cuda()
+    bias = (torch.rand(E, generator=torch.Generator().manual_seed(55)) * 0.2 - 0.1).float().cuda()
+    x = ops.PartialSum(parts) if slices else rows
+    y, ro, idx, w, al = ops.add_rmsnorm_router_topk(x, res, nw, 1e-5, gw, bias, k, 1.0, align_with_shared=True)
+    y2, ro2 = ops.add_rmsnorm_partial(x, res, nw, 1e-5) if slices else ops.add_rmsnorm(x, res, nw, 1e-5)
+    idx2, w2 = ops.router_topk(y2, gw, bias, k, 1.0)
+    assert torch.equal(y, y2) and torch.equal(ro, ro2) and torch.equal(idx, idx2) and torch.equal(w, w2)
+    (offs, tok, scale, pos), flat = [t.cpu() for t in al], idx.cpu().flatten()
+    counts = torch.bincount(flat, minlength=E)
+    assert offs.tolist() == [0] + counts.cumsum(0).tolist() + [T * (k + 1)]
+    assert torch.equal(tok[pos.long()].long(), torch.arange(T).repeat_interleave(k)) and torch.equal(scale[pos.long()], w.cpu().flatten())
+    assert (pos >= offs[flat]).all() and (pos < offs[flat + 1]).all() and pos.unique().numel() == T * k   # (any order within an expert)
