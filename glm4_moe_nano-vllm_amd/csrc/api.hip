@@ -171,7 +171,7 @@ extern "C" int glm_gemm_bf16_act(const void* x, int64_t ldx, const void* w, int6
         if (rc != GLM_ERR_UNSUPPORTED) return rc;
     }
     if (glm_midm_takes(GEMM_PLAIN, p)) return glm_launch_gemm_midm(GEMM_PLAIN, p, glm_s(stream));
-    // (a few hundred rows on a few columns, a router's logits: the tiled kernel would be a handful of workgroups)
+    // (a few hundred rows on a few columns with K off the 64-wide chunks: the tiled kernel would be a handful of workgroups)
     if (M >= LARGEM_MIN_AVG_ROWS && !(N <= 256 && M < 1024)) return glm_launch_gemm_largem(GEMM_ACT, p, glm_s(stream));
     return glm_launch_gemm_smallm(GEMM_PLAIN, p, glm_s(stream));
 }

@@ -1714,8 +1714,8 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     // ... and a projection onto <= 128 columns (the router logits at prefill: N = E = 64) is one column tile however the rows
     // are cut, so its parallelism is its row-block count: 128-row blocks (75.8 -> 55.1 us at T = 16384)
     // ... and so is every single projection whose 128-row tiles are at most one round of the chip (with the band's rounding, as
-    // launch_largem_cfg counts): a K step costs two thirds (14336 x 4096 at 200 and 400 rows 83 / 60 and 86 / 59 us, 2048 x 2048 at 2000
-    // rows 42 / 28, 4096 x 12288 at 1200 rows 234 / 153; beyond a round 9728 x 2048 at 800 rows 48 / 60)
+    // launch_largem_cfg counts): a K step costs two thirds (14336 x 4096 at 400 rows 86 / 59 us, 4096 x 12288 at 1200 rows 234 / 153; beyond a
+    // round 9728 x 2048 at 800 rows 48 / 60; what is a round of 128 x 128 tiles does not come here, gemm_midm.hip)
     const int64_t cb = (p.R + 127) / 128, bd = cb < g_largem_band ? cb : (int64_t)g_largem_band;
     const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
                            (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;

@@ -461,7 +461,9 @@ template <int MODE>
 int launch_midm(const GemmParams& p, hipStream_t st) {
     // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
     // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
-    if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
+    if constexpr (MODE == GEMM_GATEUP || MODE == GEMM_DOWN) {
+        if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
+    }
     return launch_midm_tile<MODE>(midm_tile_of(MODE, p), p, st);
 }
 

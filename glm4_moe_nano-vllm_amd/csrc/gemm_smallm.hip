@@ -16,7 +16,8 @@
 //     double-buffered, one barrier per chunk.  Each weight register is refilled for the NEXT chunk right after its
 //     last MFMA, so one full chunk (8 x 1 KiB per wave) stays in flight across the barrier; the activation loads are
 //     issued before it in program order, so waiting for them never drains the stream.  Used for fp8 weights, for
-//     single-sequence decode, very short K and more than 32 rows per block.
+//     single-sequence decode, very short K and more than 32 rows per block (K off the 64-wide chunks of
+//     gemm_midm.hip, or more columns than it takes).
 //     (Measured alternatives that lost on the same box: B fragments straight from L2 without LDS and barriers,
 //     298 vs 267 us for the grouped gate|up; two-chunk-deep weight registers at half the resident waves, 281 us.)
 //
