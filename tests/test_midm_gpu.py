@@ -128,6 +128,16 @@ def test_one_row_feed_forward(ops, M, I):
     close(ops.grouped_gemm_down(act, d.cuda().unsqueeze(0), None, None, 0), act.cpu().double() @ d.double().T, "down")
 
 
+@pytest.mark.parametrize("R", [1, 2, 40, 130])
+def test_one_group_of_gathered_rows(ops, R):
+    """No offsets, rows of a longer x by number: one row (the last of x) and more, on either side of every row count that picks a kernel."""
+    T, H, I = 300, 192, 72
+    x, w = rnd(T, H, seed=33), rnd(2 * I, H, seed=34, scale=H ** -0.5)
+    tok = (T - 1 - 7 * torch.arange(R)) % T
+    act = ops.grouped_gemm_gateup_silu(x.cuda(), w.cuda().unsqueeze(0), None, tok.to(torch.int32).cuda(), R)
+    assert_close_bf16(act, O.silu_and_mul((x[tok].double() @ w.double().T).to(BF)), *SILU, what="silu")
+
+
 @pytest.mark.parametrize("T,nh,nkv,K", [(97, 4, 1, 1024), (211, 6, 2, 640), (256, 2, 2, 512), (450, 6, 2, 576), (130, 40, 2, 128), (211, 96, 8, 320)])
 def test_qkv_epilogue(ops, T, nh, nkv, K):
     """Split, rotation and cache rows in the projection's epilogue: the projection and the split kernel, bit for bit."""
