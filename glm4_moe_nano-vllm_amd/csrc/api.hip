@@ -118,7 +118,8 @@ int dispatch(int mode, const GemmParams& p, hipStream_t st) {
     if (p.R <= 0) return GLM_OK;
     // one row of one matrix (a dense feed-forward at single-sequence decode): the GEMV body, as for the experts.  21888 x 4096 gate|up
     // 33 -> 30 us, 4096 x 10944 down 65 -> 18.  A gathered row is not for it: it holds row 0 of x only.
-    if (p.R == 1 && p.offs == nullptr && p.src == nullptr && p.G == 1 && tinym_enabled() && (mode == GEMM_GATEUP || (mode == GEMM_DOWN && p.n_scaled == 0))) {
+    // N % 4: what the kernels for more rows refuse is refused for one.
+    if (p.R == 1 && p.N % 4 == 0 && p.offs == nullptr && p.src == nullptr && p.G == 1 && tinym_enabled() && (mode == GEMM_GATEUP || (mode == GEMM_DOWN && p.n_scaled == 0))) {
         const int rc = glm_launch_gemm_tinym(mode == GEMM_DOWN ? GEMM_PLAIN : mode, p, 1, st);   // (without scales down is a plain projection)
         if (rc != GLM_ERR_UNSUPPORTED) return rc;
     }

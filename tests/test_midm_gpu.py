@@ -128,6 +128,13 @@ def test_one_row_feed_forward(ops, M, I):
     close(ops.grouped_gemm_down(act, d.cuda().unsqueeze(0), None, None, 0), act.cpu().double() @ d.double().T, "down")
 
 
+@pytest.mark.parametrize("M", [1, 2])
+def test_feed_forward_refuses_columns_off_four(ops, M):
+    x, w = rnd(M, 64, seed=35).cuda(), rnd(12, 64, seed=36).cuda().unsqueeze(0)
+    with pytest.raises(RuntimeError, match="N%4"):
+        ops.grouped_gemm_gateup_silu(x, w, None, None, M)
+
+
 @pytest.mark.parametrize("R", [1, 2, 40, 130])
 def test_one_group_of_gathered_rows(ops, R):
     """No offsets, rows of a longer x by number: one row (the last of x) and more, on either side of every row count that picks a kernel."""
