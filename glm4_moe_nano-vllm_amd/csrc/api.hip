@@ -288,7 +288,7 @@ extern "C" int glm_gemm_bf16_slices(int64_t M, int N, int K) {
 // 50 / 46; 4096 x 12288 at 400 95 / 62, at 1000 123 / 101)
 extern "C" int glm_gemm_bf16_row_slices(int64_t M, int N, int K) {
     const int s = glm_midm_slices(M, N, K);
-    return s > 1 ? s : K >= 6144 ? glm_gemm_bf16_slices(M, N, K) : 1;
+    return s > 1 ? s : K >= 6144 && N % 8 == 0 ? glm_gemm_bf16_slices(M, N, K) : 1;   // (N % 8: what the tiled kernel's slabs need)
 }
 
 extern "C" int glm_gemm_bf16_partial(const void* x, int64_t ldx, const void* w, int64_t ldw, float* ypart,

@@ -474,6 +474,7 @@ int launch_midm(const GemmParams& p, hipStream_t st) {
 // consumer's wider reads take back.
 int midm_slices(int64_t M, int N, int K, MidmTile* tile) {
     if (M <= 32 || K % 64 != 0 || K < 4096 || N % 4 != 0) return 1;
+    if (M < 96 && (int64_t)N * K >= 1ll << 29) return 1;   // up to 95 rows slices have no other kernel, and this one's offsets (of padded rows) are 32-bit
     static const struct { MidmTile t; int rows, cols; } tiles[] = {{MM_64, 64, 64}, {MM_128x64, 128, 64}, {MM_128, 128, 128}};
     for (const auto& c : tiles) {
         if ((c.rows == 64) != (M <= 64)) continue;

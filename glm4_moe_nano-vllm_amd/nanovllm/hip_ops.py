@@ -1249,6 +1249,9 @@ def row_slices(M: int, N: int, K: int) -> int:
     return load_library().glm_gemm_bf16_row_slices(M, N, K)
 
 
+ADD_NORM_PARTIAL_MAX_H = 16384   # columns glm_add_rmsnorm_partial takes, whole 16-byte pieces of them
+
+
 def add_rmsnorm_partial(ps: PartialSum, residual: torch.Tensor, weight: torch.Tensor,
                         eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """add_rmsnorm whose x is bf16(sum of the K-slice partial sums)."""

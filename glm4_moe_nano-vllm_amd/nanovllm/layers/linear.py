@@ -142,9 +142,12 @@ class RowParallelLinear(LinearBase):
 
     partial_max_rows = 1024   # (one pass / slices with the norm at 1000 rows still 123 / 101 us; not measured beyond)
 
-    def _slices(self, m: int) -> int:
+    def _slices(self, x: torch.Tensor) -> int:
+        m, n = x.shape[0], self.weight.shape[0]
         if m > 32:   # 4096 x 12288: 64 rows 45 -> 23 us, 211 rows 56 -> 37, 400 rows 108 -> 50
-            return hip_ops.row_slices(m, *self.weight.shape) if m < self.partial_max_rows else 1
+            # (columns that the norm can add up; rows that 32-bit offsets reach)
+            ok = m < self.partial_max_rows and n % 8 == 0 and n <= hip_ops.ADD_NORM_PARTIAL_MAX_H and m * x.stride(0) < 1 << 30
+            return hip_ops.row_slices(m, *self.weight.shape) if ok else 1
         lo = 1 if hip_ops.opt("tinym") != 0 else 0  # one row: the GEMV body (glm_gemm_bf16 picks it)
         return self.partial_slices if m > lo else 1
 
@@ -153,7 +156,7 @@ class RowParallelLinear(LinearBase):
         if (defer_reduce and self.tp_size == 1 and self.bias is None and x.dim() == 2
                 and x.shape[1] >= self.partial_min_k and x.shape[1] >= 2 * self.weight.shape[0]
                 and x.shape[1] % 8 == 0 and x.stride(1) == 1):
-            slices = self._slices(x.shape[0])
+            slices = self._slices(x)
             if slices > 1:
                 return hip_ops.gemm_bf16_partial(x, self.weight.data, slices)
         y = self._gemm(x, with_bias=self.tp_rank == 0)

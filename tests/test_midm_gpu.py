@@ -180,6 +180,38 @@ def test_row_slices(ops, M, N, K):
             ops.gemm_bf16_partial(x.cuda(), w.cuda(), 7)
 
 
+def test_row_slices_only_where_they_are_taken(ops):
+    """No count that gemm_bf16_partial refuses: tiled slabs of columns off eight, weights beyond 32-bit offsets with no kernel to fall back on."""
+    assert ops.row_slices(700, 2056, 8192) > 1 and ops.row_slices(700, 2052, 8192) == 1
+    assert ops.row_slices(64, 4096, 65536) > 1 and ops.row_slices(64, 4096, 262144) == 1 and ops.row_slices(95, 2048, 262144) == 1
+
+
+@pytest.mark.parametrize("M,N", [(40, 100), (700, 2052), (200, 2052), (64, 2048)])
+def test_projection_and_norm_of_any_width(ops, M, N):
+    """RowParallelLinear hands slices to the norm only where the norm adds them up (whole 16-byte pieces), rows otherwise."""
+    from nanovllm.layers.layernorm import RMSNorm
+    from nanovllm.layers.linear import RowParallelLinear
+    K = 8192
+    old = torch.get_default_dtype()
+    torch.set_default_dtype(BF)
+    try:
+        with torch.device("cuda"):
+            lin, norm = RowParallelLinear(K, N), RMSNorm(N, 1e-5)
+    finally:
+        torch.set_default_dtype(old)
+    x, w, res = rnd(M, K, seed=60), rnd(N, K, seed=61, scale=K ** -0.5), rnd(M, N, seed=62)
+    lin.weight.data.copy_(w)
+    y = lin(x.cuda(), defer_reduce=True)
+    assert isinstance(y, ops.PartialSum) == (N % 8 == 0)
+    h, r = norm(y, res.cuda())
+    # the projection's rounding is off by one of its ulps beside a boundary, 2^-5 at most below 8, which is what a sum near zero then differs by;
+    # the norm divides by more than one and rounds twice more
+    assert x.shape[0] * N < 1 << 22     # (so many normal values stay below 8)
+    s = (x.double() @ w.double().T).to(BF).double() + res.double()
+    assert_close_bf16(r, s.to(BF), 1, 0.05, atol=2 ** -5, what="residual")
+    assert_close_bf16(h, (s * (s.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()).to(BF), 2, 0.35, atol=2 ** -5, what="norm")
+
+
 @pytest.mark.parametrize("T,E,slices", [(192, 64, 4), (191, 64, 4), (97, 128, 8), (300, 64, 0)])
 def test_norm_and_router_of_slices(ops, T, E, slices):
     """The norm behind a projection (its partial sums or its rows), the router and the bucketing: as launches of their own, on either side of the
