@@ -17,10 +17,12 @@
 // 4096 x 4096 at 1000 rows 58 -> 43 (tiled), 10944 gated columns x 4096 at 64 rows 53 -> 43.
 #include "gemm_internal.h"
 #include "gemm_epilogue.h"
+#include <type_traits>
 
 namespace {
 
 typedef __attribute__((address_space(3))) void mm_lds_void;
+typedef __attribute__((address_space(1))) const void mm_glb_void;
 
 constexpr int MM_KC = 64;     // K columns of a stage
 constexpr int MM_ROWB = 128;  // bytes of a staged row
@@ -122,9 +124,10 @@ __device__ __forceinline__ void midm_qkv_rows(const GemmParams& p, const f32x4_t
     }
 }
 
-// rows m0 .. m0 + mcnt - 1 of group grp, columns from ncol0; MT 16-row activation tiles, RT 16-row weight tiles
+// rows m0 .. m0 + mcnt - 1 of group grp, columns from ncol0; MT 16-row activation tiles, RT 16-row weight tiles; reach: rows of x whose bytes
+// 32-bit offsets address
 template <int MODE, int MT, int RT, int NW, int NST>
-__device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int grp, int m0, int mcnt, int ncol0) {
+__device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int grp, int m0, int mcnt, int ncol0, int reach) {
     constexpr int D = 2 * (MT + RT);           // DMA instructions of a stage
     constexpr int STAGE = D * 1024;
     constexpr int HALF = 8 * RT;               // paired modes: gate rows of the tile, then as many up rows
@@ -144,21 +147,34 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
         const int wr = gemm_paired(MODE) ? (row < HALF ? 0 : p.N) + min(ncol0 + (row < HALF ? row : row - HALF), p.N - 1) : min(ncol0 + row, p.N - 1);
         wvo[i] = ((unsigned)wr * (unsigned)p.ldw + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
     }
+    int last = 0;
+    auto source = [&](int i) {
+        const int m = m0 + min(8 * i + r8, mcnt - 1);   // rows past the end repeat the last one; they are never stored
+        return MODE == GEMM_GATEUP && p.src ? p.src[m] : m;
+    };
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) {
-        const int row = 8 * i + r8, m = m0 + min(row, mcnt - 1);   // rows past the end repeat the last one; they are never stored
-        const int src = p.src ? p.src[m] : m;
-        xvo[i] = ((unsigned)src * (unsigned)p.ldx + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
+        const int src = source(i);
+        xvo[i] = ((unsigned)src * (unsigned)p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8) * 2u;
+        last = max(last, src);
     }
     // ---- this wave's chunks: wid, wid + 4, ... of the K columns
     const int n = max(0, (p.K / MM_KC - wid + NW - 1) / NW);
-    auto issue = [&](int j, int slot) {
+    auto issue_w = [&](int j, int slot) {
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)(ringp + slot * STAGE + i * 1024), 16, wvo[i], (j * NW + wid) * MM_ROWB, 0, 0);
+    };
+    auto issue_x = [&](auto far_rows, int j, int slot) {
         const int soff = (j * NW + wid) * MM_ROWB;
-        char* st = ringp + slot * STAGE;
+        char* st = ringp + slot * STAGE + 2 * RT * 1024;
 #pragma unroll
-        for (int i = 0; i < 2 * RT; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)(st + i * 1024), 16, wvo[i], soff, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (mm_lds_void*)(st + (2 * RT + i) * 1024), 16, xvo[i], soff, 0, 0);
+        for (int i = 0; i < 2 * MT; ++i) {
+            if constexpr (decltype(far_rows)::value)
+                __builtin_amdgcn_global_load_lds((mm_glb_void*)(p.x + (int64_t)source(i) * p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8 + soff / 2),
+                                                 (mm_lds_void*)(st + i * 1024), 16, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (mm_lds_void*)(st + i * 1024), 16, xvo[i], soff, 0, 0);
+        }
     };
     // stage j has arrived, the younger ones stay in flight
     auto arrived = [&](int j) {
@@ -181,10 +197,13 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             for (int mt = 0; mt < MT; ++mt)
                 acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f.w[rt]), __builtin_bit_cast(bf16x8_t, f.x[mt]), acc[rt][mt], 0, 0, 0);
     };
-    if (n > 0) {
+    auto loop = [&](auto far_rows) {
 #pragma unroll
         for (int j = 0; j < NST; ++j)
-            if (j < n) issue(j, j);
+            if (j < n) {
+                if (j > 0) issue_w(j, j);
+                issue_x(far_rows, j, j);
+            }
         MmFrags<MT, RT> f0, f1;        // the two k-steps of a stage
         int slot = 0;
         arrived(0);
@@ -195,7 +214,10 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             __builtin_amdgcn_sched_barrier(0);
             mm(f0);
             f1.settle();               // the stage is in registers: its slot takes chunk j + NST
-            if (j + NST < n) issue(j + NST, slot);
+            if (j + NST < n) {
+                issue_w(j + NST, slot);
+                issue_x(far_rows, j + NST, slot);
+            }
             slot = slot + 1 == NST ? 0 : slot + 1;
             if (j + 1 < n) {
                 arrived(j + 1);
@@ -205,6 +227,14 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             mm(f1);
             if (j + 1 < n) f0.settle();
         }
+    };
+    if (n > 0) {
+        issue_w(0, 0);   // (ahead of the wait for the row numbers)
+        // gathered rows (of an x whose length nobody here knows) beyond what 32-bit offsets reach: the wave looks its rows up again at every stage
+        if constexpr (MODE == GEMM_GATEUP) {
+            if (__any(last >= reach)) loop(std::true_type{});
+            else loop(std::false_type{});
+        } else loop(std::false_type{});
     }
 
     // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / 4 ..
@@ -259,7 +289,7 @@ constexpr int midm_lds() {
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
-__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, int mblocks, int interleaved) {
+__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, int mblocks, int interleaved, int reach) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int COLS = gemm_paired(MODE) ? 8 * RT : 16 * RT;
     int grp = 0, m0, mcnt, ntile;
@@ -279,7 +309,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, 
         mcnt = min(16 * MT, (int)p.R - m0);
     }
     if (ntile * COLS >= p.N) return;
-    midm_body<MODE, MT, RT, NW, NST>(p, smem, grp, m0, mcnt, ntile * COLS);
+    midm_body<MODE, MT, RT, NW, NST>(p, smem, grp, m0, mcnt, ntile * COLS, reach);
 }
 
 // rows m0 .. m0 + mcnt - 1, columns from ncol0, tile shared by the workgroup: WM x WN waves of MT x RT 16-row tiles each.  Every wave brings
@@ -401,7 +431,8 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
     GLM_CHECK_ARG(gx < (1 << 30) && gy <= 65535, GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
     auto kern = gemm_midm_kernel<MODE, MT, RT, NW, NST>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
-    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt);
+    const int64_t reach = (1ll << 30) / p.ldx;
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt, (int)reach);
     GLM_CHECK_LAUNCH("gemm_midm");
     return GLM_OK;
 }

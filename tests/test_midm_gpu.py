@@ -119,6 +119,22 @@ def test_experts(ops, T, E, k, H, I, shared):
             assert_close_bf16(y[rows], (d.float() * s[rows, None].float()).to(BF) if e < E else d, 2, 0.06, atol=2 ** -8, what=f"y of expert {e}")
 
 
+def test_experts_of_rows_far_apart(ops):
+    """Gathered rows of an x longer than 32-bit byte offsets reach (rows 2 MiB apart: past 2 GiB from row 1024, past 4 GiB from row 2048): an
+    expert of near rows, one of far ones, one of both, with a partial last block of 64."""
+    H, I, T = 192, 72, 2100
+    x = torch.empty(T, 1 << 20, dtype=BF, device="cuda")[:, :H]
+    x.copy_(rnd(T, H, seed=63))
+    tok = torch.cat([torch.arange(30), torch.arange(1023, 1053), torch.arange(0, T, 31)]).to(torch.int32)
+    offs = [0, 30, 60, tok.numel()]
+    w = rnd(3, 2 * I, H, seed=64, scale=H ** -0.5)
+    act = ops.grouped_gemm_gateup_silu(x, w.cuda(), torch.tensor(offs, dtype=torch.int32).cuda(), tok.cuda(), tok.numel())
+    for e in range(3):
+        rows = slice(offs[e], offs[e + 1])
+        z = rnd(T, H, seed=63)[tok[rows].long()].double() @ w[e].double().T
+        assert_close_bf16(act[rows], O.silu_and_mul(z.to(BF)), *SILU, what=f"expert {e}")
+
+
 @pytest.mark.parametrize("M,I", [(1, 1408), (1, 10944)])
 def test_one_row_feed_forward(ops, M, I):
     H = 512
