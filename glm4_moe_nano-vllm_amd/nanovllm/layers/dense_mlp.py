@@ -36,10 +36,13 @@ class DenseMLP(nn.Module):
         self.down.load([w["down"][:, lo: lo + self.ff]], device)
         self.act = xielu_constants(w["act"])
 
-    def forward(self, h: torch.Tensor):
-        """[T, width], or its K-slice partial sums, which the norm behind it adds up (2048 x 6144 at 128 rows with that norm 19 -> 15 us)."""
+    def forward(self, h: torch.Tensor, defer_reduce: bool = False):
+        """[T, width].  defer_reduce: the caller hands the result to the norm behind it and takes the K-slice partial sums that the norm adds up
+        (both, us, one pass / slices: 2048 x 6144 at 128 rows 19 / 15)."""
         u = self.up(h, act=self.act)
-        slices = hip_ops.row_slices(h.shape[0], self.down.N, self.down.K) if self.tp_size == 1 and u.dtype == torch.bfloat16 else 1
+        slices = 1
+        if defer_reduce and self.tp_size == 1 and u.dtype == torch.bfloat16:
+            slices = hip_ops.row_slices(h.shape[0], self.down.N, self.down.K)
         if slices > 1:
             return hip_ops.gemm_bf16_partial(u, self.down.weight, slices)
         y = self.down(u)

@@ -145,7 +145,7 @@ class DafolornForCausalLM(nn.Module):
             y, g_post = layer.mixer(h, meta, r), layer.g_post1
             if layer.mlp is not None:
                 x, h = layer.entry2(x, y, g_post, meta, r, dt)
-                y, g_post = layer.mlp(h), layer.g_post2
+                y, g_post = layer.mlp(h, defer_reduce=True), layer.g_post2
         if residual_tap is not None:
             tap(hip_ops.seq_norm(x, cfg.hidden_size, eps, y=y, g_post=g_post, act_dtype=dt)[0])
         if meta.want.numel() == 0:

@@ -228,6 +228,18 @@ def test_projection_and_norm_of_any_width(ops, M, N):
     assert_close_bf16(h, (s * (s.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()).to(BF), 2, 0.35, atol=2 ** -5, what="norm")
 
 
+def test_feed_forward_gives_rows_unless_asked(ops):
+    """A module's own caller (and its hooks) get a tensor; partial sums only where they are asked for, the same to a rounding."""
+    from nanovllm.layers.dense_mlp import DenseMLP
+    T, W, ff = 128, 1024, 4096
+    m = DenseMLP(W, ff, BF)
+    m.load({"up": rnd(ff, W, seed=65, scale=W ** -0.5), "down": rnd(W, ff, seed=66, scale=ff ** -0.5), "act": torch.zeros(2)}, "cuda")
+    h = rnd(T, W, seed=67).cuda()
+    y, parts = m(h), m(h, defer_reduce=True)
+    assert isinstance(y, torch.Tensor) and y.shape == (T, W) and y.dtype == BF and isinstance(parts, ops.PartialSum)
+    close(y, parts.part.cpu().double().sum(0), "rows and slabs")
+
+
 @pytest.mark.parametrize("T,E,slices", [(192, 64, 4), (191, 64, 4), (97, 128, 8), (300, 64, 0)])
 def test_norm_and_router_of_slices(ops, T, E, slices):
     """The norm behind a projection (its partial sums or its rows), the router and the bucketing: as launches of their own, on either side of the
