@@ -116,10 +116,14 @@ bool tinym_enabled() { return glm_option(GLM_OPT_TINYM) != 0; }
 
 int dispatch(int mode, const GemmParams& p, hipStream_t st) {
     if (p.R <= 0) return GLM_OK;
-    // one row of one matrix (a dense feed-forward at single-sequence decode): the GEMV body, as for the experts.  21888 x 4096 gate|up
-    // 33 -> 30 us, 4096 x 10944 down 65 -> 18.  A gathered row is not for it: it holds row 0 of x only.
-    // N % 4: what the kernels for more rows refuse is refused for one.
-    if (p.R == 1 && p.N % 4 == 0 && p.offs == nullptr && p.src == nullptr && p.G == 1 && tinym_enabled() && (mode == GEMM_GATEUP || (mode == GEMM_DOWN && p.n_scaled == 0))) {
+    // one row of one matrix (a dense feed-forward at single-sequence decode): the GEMV body, as for the experts.  A gathered row is not for it: it
+    // holds row 0 of x only.  N % 4: what the kernels for more rows refuse is refused for one.  It reads 4 KiB of a weight row at a time whatever
+    // K is, so a short K stays with the streaming kernel, longer with more columns.  Streaming / GEMV, us: gate|up 1024 x 256 3.9 / 4.6, x 384
+    // 5.3 / 4.7; 4096 x 640 7.2 / 8.6, x 768 8.9 / 8.8; 8192 x 1024 12.9 / 14.0, x 1280 16.5 / 15.2; 10944 x 1536 18.7 / 19.3, x 2048 22.8 / 21.1,
+    // x 4096 43 / 32; down 1024 x 384 3.6 / 3.8, x 448 4.5 / 3.8; 4096 x 512 4.9 / 4.3; 8192 x 512 5.2 / 6.2, x 640 6.5 / 6.4; 16384 x 768
+    // 9.5 / 10.4, x 1024 11.2 / 10.9; 4096 x 10944 56 / 20
+    const bool gemv = mode == GEMM_GATEUP ? p.K >= 256 + p.N / 8 : mode == GEMM_DOWN && p.n_scaled == 0 && p.K >= 384 + p.N / 32;
+    if (p.R == 1 && gemv && p.N % 4 == 0 && p.offs == nullptr && p.src == nullptr && p.G == 1 && tinym_enabled()) {
         const int rc = glm_launch_gemm_tinym(mode == GEMM_DOWN ? GEMM_PLAIN : mode, p, 1, st);   // (without scales down is a plain projection)
         if (rc != GLM_ERR_UNSUPPORTED) return rc;
     }

@@ -135,9 +135,9 @@ def test_experts_of_rows_far_apart(ops):
         assert_close_bf16(act[rows], O.silu_and_mul(z.to(BF)), *SILU, what=f"expert {e}")
 
 
-@pytest.mark.parametrize("M,I", [(1, 1408), (1, 10944)])
-def test_one_row_feed_forward(ops, M, I):
-    H = 512
+@pytest.mark.parametrize("M,I,H", [(1, 1408, 512), (1, 10944, 512), (1, 10944, 1624), (1, 1024, 384), (1, 1024, 376), (1, 40, 64), (1, 416, 1024), (1, 408, 1024)])
+def test_one_row_feed_forward(ops, M, I, H):
+    """Either side of the K from which the GEMV body takes it (gate|up 256 + I / 8, down 384 + H / 32)."""
     x, w, d = rnd(M, H, seed=30), rnd(2 * I, H, seed=31, scale=H ** -0.5), rnd(H, I, seed=32, scale=I ** -0.5)
     act = ops.grouped_gemm_gateup_silu(x.cuda(), w.cuda().unsqueeze(0), None, None, M)
     assert_close_bf16(act, O.silu_and_mul((x.double() @ w.double().T).to(BF)), *SILU, what="silu")
