@@ -536,6 +536,23 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     if (p.src != nullptr || p.G > 1 || p.R <= 32) return false;
     // (a loop of the tiled kernel that is asked for keeps its shapes)
     if (p.R >= 96 && (glm_option(GLM_OPT_LARGEM_VARIANT) >= 0 || glm_option(GLM_OPT_LARGEM_CFG) != 0)) return false;
+    // Feed-forwards below 96 rows: the streaming kernel has configurations for them with a workgroup per 16 act columns or 32 columns and block of
+    // 32 rows, which cover the chip where these tiles of 64 rows leave half of it idle, or where K is a few chunks.  Streaming / here, us, cold
+    // operands: gate|up (K x columns of at least 4M) 1024 x 4096 at 48 rows 12.8 / 14.1, 2048 x 4096 at 64 13.7 / 16.8, 768 x 12288 at 64
+    // 32 / 41, but 768 x 4096 at 64 13.0 / 11.3, 2304 x 4096 at 64 23 / 18, 2048 x 8192 at 33 32 / 26; short ones 1536 x 512 at 48 4.4 / 4.8, 1024 x 1024 at 33 5.5 / 5.7,
+    // but 512 x 512 4.3 / 4.0, 2304 x 512 at 64 5.8 / 5.0.  Down (split over its waves from K = 4096 on) 1024 x 4096 at 48 8.3 / 10.5, 2048 x 6144
+    // at 64 12.8 / 23.1, 2048 x 12288 at 33 24.8 / 34.8, but 3072 x 4096 at 48 14.9 / 15.2, 2048 x 3072 at 64 17.2 / 9.7, 2048 x 4096 at 65
+    // 14.2 / 12.9; 2048 x 256 at 64 3.3 / 3.7, 4096 x 384 at 33 4.3 / 4.8, 2048 x 448 at 95 4.2 / 4.4, but 2048 x 512 5.3 / 4.7, 6144 x 384 at 64
+    // 5.4 / 5.0.
+    if (p.R < 96 && mode != GEMM_PLAIN) {
+        const int64_t n = (p.R + 31) / 32 * p.N;
+        if (mode == GEMM_DOWN) {
+            if (p.K < 512 ? n <= 8192 : p.K >= 4096 && p.R <= 64 && p.N <= 2560 && p.R * p.N <= 131072) return false;
+        } else {
+            if (p.K > 320 && p.K <= 1024 && p.N >= 1024 && n <= 4096) return false;
+            if (p.R <= 64 && p.N <= 2048 && (int64_t)p.N * p.K >= 4 << 20 && (p.R > 40 || p.K < 8192)) return false;
+        }
+    }
     const int64_t wrows = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
     if (p.R * p.ldx * 2 >= (1ll << 31) || wrows * p.ldw * 2 >= (1ll << 31)) return false;   // 32-bit offsets
     // Beyond one round of the largest tile the tiled kernel's 128 x 256 and 256 x 256 ones pull less (14336 x 4096 at 400 rows, 448 tiles: 60 us

@@ -82,7 +82,8 @@ def test_activations(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M,I,K", [(33, 24, 64), (65, 1000, 192), (97, 1408, 1088), (211, 4104, 576), (300, 264, 1024), (100, 3000, 128), (130, 3016, 64),
-                                   (64, 9000, 192)])
+                                   (64, 9000, 192), (48, 1024, 1024), (64, 1032, 512), (95, 1368, 512), (64, 2048, 2048), (64, 2056, 2048), (64, 4096, 1024), (65, 4096, 64),
+                                   (33, 384, 4096), (95, 448, 2688), (95, 448, 2736)])
 def test_gated(ops, M, I, K):
     x, w = rnd(M, K, seed=6), rnd(2 * I, K, seed=7, scale=K ** -0.5)
     g, u = (x.double() @ w.double().T).chunk(2, 1)
