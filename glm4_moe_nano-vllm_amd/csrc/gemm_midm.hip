@@ -525,9 +525,12 @@ int midm_slices(int64_t M, int N, int K, MidmTile* tile) {
 bool glm_midm_takes(int mode, const GemmParams& p) {
     if (p.ksplit > 1 || p.wscale != nullptr || p.K % 64 != 0) return false;
     if (p.offs != nullptr) {
-        // Experts with 24 to 95 rows on average: the weight-streaming kernel's blocks of 32 rows read an expert's weights once per block.
-        // gate|up, down of 1408 x 4096, us: 26 rows 298 / 160 there, 261 / 147 here; 55 rows 557 / 279 and 307 / 174; 18 rows 263 / 149 and
-        // 265 / 145; of 1024 x 2048: 20 rows 108 / 57 and 106 / 60, 38 rows 168 / 82 and 109 / 62.
+        // Experts with 24 to 95 rows on average: the weight-streaming kernel's blocks of 32 rows read an expert's weights once per block.  gate|up,
+        // down, us, rows dealt at random: 65 of 1408 x 4096 at 24 rows 292 / 159 there, 278 / 151 here, at 30 330 / 184 and 274 / 153, at 55
+        // 557 / 279 and 307 / 174; 64 of 1024 x 2048 at 20 108 / 57 and 106 / 60, at 24 109 / 61 and 104 / 59, at 38 168 / 82 and 109 / 62.  Rows
+        // dealt evenly up to 32 are read once there too, and with few experts it hangs on how they fall: 8 of 2048 x 4096 at 24 rows 50 / 27
+        // there, 53 / 31 here, at 25 64 / 35 and 54 / 31, at 26 51 / 28 and 54 / 31, at 27 63 / 37 and 54 / 31; 16 of 1408 x 4096 gate|up at 25 74 / 83,
+        // at 28 82 / 78; 32 of 1024 x 1024 down at 25 17 / 20, at 28 22 / 20; 128 of 512 x 1024 down at 24 39 / 41, at 32 45 / 42.
         const int64_t rows = p.R_hint > 0 ? p.R_hint : p.R;
         if (mode != GEMM_GATEUP && mode != GEMM_DOWN) return false;
         return rows >= 24 * (int64_t)p.G && rows < 96 * (int64_t)p.G && p.R * p.ldx * 2 < (1ll << 31) &&
