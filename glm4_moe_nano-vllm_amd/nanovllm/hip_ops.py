@@ -642,15 +642,31 @@ def varlen_attn_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, scale
 # a [T, H] x [H, E] GEMM, and glm_router_select does R2..R7 from them; below, the token-per-workgroup kernel
 # (glm_router_topk / the fused add-RMSNorm + router + bucketing launch), which is built for decode latency: at T = 16384
 # it takes 1.2 ms per layer against 0.34 ms for norm + GEMM + select + bucketing (tools/prefill_router_probe.py).
-# That kernel reads all of Wg for every other token, so it also falls behind with tokens x experts.  One launch / four, us, hidden size 4096, in
-# parentheses from four K slices of o_proj: 64 experts at 128 tokens 16 / 22 (21 / 23), at 211 24.0 / 23.5 (37 / 25), at 700 58 / 35 (96 / 37);
-# 128 experts at 96 tokens 21 / 23 (29 / 25), at 128 25.0 / 24.6 (35 / 26).
+# That kernel is one workgroup a token: beyond 256 tokens it is a second round of the chip, and with many experts a token's pass over Wg is long.
+# One launch / GEMM and selection, us, hidden size 2048 and 4096: 64 experts at 256 tokens 8.9 / 11.3 and 12.3 / 14.4, at 257 14.6 / 11.3 and
+# 20.2 / 14.7; 96 at 256 12.4 / 13.5 and 17.2 / 16.6; 128 at 128 13.6 / 13.6 and 19.3 / 16.8; 192 at 96 17.3 / 13.9 and 24.3 / 17.2; 16 at 768
+# 17.1 / 11.0 and 20.5 / 14.2.  With the norm, in the one launch or ahead of the two: 64 at 256 10.0 / 14.7 and 14.1 / 19.3, at 257 16.8 / 14.8 and
+# 23.0 / 20.1; 128 at 128 15.0 / 16.6 and 21.0 / 21.1; 160 at 96 16.1 / 16.7 and 22.1 / 21.1; 192 at 96 18.2 / 16.9 and 25.7 / 21.4.  (With the bucketing,
+# from rows, the launches around a GEMM lose a little below 16384 logits: 128 at 96, 4096 wide, 20.0 / 22.9.)
 ROUTER_GEMM_MIN_ROWS = 1024
-ROUTER_GEMM_MIN_LOGITS = 12288
+ROUTER_GEMM_MIN_LOGITS = 12288     # (T x E; nothing below was measured to gain)
+ROUTER_ROUND_TOKENS = 256
+ROUTER_GEMM_MIN_EXPERTS, ROUTER_GEMM_MIN_GATE = 128, 160 * 2048   # within the first round: experts, E x H
+# The bucketing in the same launch spreads a token's experts over workgroups, each of which repeats the norm and reads the K slices: the norm, the
+# router and the bucketing as launches of their own are ahead from T x E logits on, whichever way those are computed.  One / three or four, us,
+# H = 2048 and 4096: 64 at 192 18.0 / 17.9 and 20.1 / 22.3, at 256 20.3 / 18.7 and 23.8 / 23.4, at 700 43 / 25 and 52 / 33; 128 at 96 17.3 / 18.8 and
+# 20.0 / 22.9, at 128 20.3 / 19.3 and 23.6 / 24.2; 256 at 64 20.6 / 19.7 and 24.0 / 23.9; from four slabs 64 at 192 22.7 / 18.5 and 27.1 / 24.6, at
+# 700 75 / 28 and 93 / 36, 128 at 96 23.2 / 19.3 and 27.5 / 24.0, 256 at 48 24.1 / 19.7 and 28.4 / 24.4.
+ROUTER_SPLIT_LOGITS, ROUTER_SPLIT_LOGITS_SLABS = 16384, 12288
 
 
-def router_by_gemm(T: int, E: int) -> bool:
-    return (T >= ROUTER_GEMM_MIN_ROWS or T * E >= ROUTER_GEMM_MIN_LOGITS) and E % 8 == 0  # the GEMM kernels want 16-byte output rows
+def router_by_gemm(T: int, E: int, H: int = 0) -> bool:
+    """The logits come from a GEMM: by the sizes alone, so that every entry point rounds a step's logits alike."""
+    if E % 8:      # the GEMM kernels want 16-byte output rows
+        return False
+    if T > ROUTER_ROUND_TOKENS:
+        return T >= ROUTER_GEMM_MIN_ROWS or T * E >= ROUTER_GEMM_MIN_LOGITS
+    return E >= ROUTER_GEMM_MIN_EXPERTS and E * H >= ROUTER_GEMM_MIN_GATE and T * E >= ROUTER_GEMM_MIN_LOGITS
 
 
 def router_select(logits: torch.Tensor, bias: torch.Tensor, k: int, routed_scaling_factor: float):
@@ -672,7 +688,7 @@ def router_topk(x: torch.Tensor, gate_w: torch.Tensor, bias: torch.Tensor, k: in
     T, H = x.shape
     E = gate_w.shape[0]
     x = x.contiguous()
-    if router_by_gemm(T, E):
+    if router_by_gemm(T, E, H):
         logits = gemm_bf16(x, gate_w, None)
         idx, w = router_select(logits, bias, k, routed_scaling_factor)
         return (idx, w, logits) if return_logits else (idx, w)
@@ -716,8 +732,9 @@ def add_rmsnorm_router_topk(x, residual: torch.Tensor, norm_weight: torch.Tensor
     r2 = residual.reshape(-1, H).contiguous()
     T = r2.shape[0]
     E = gate_w.shape[0]
-    if router_by_gemm(T, E):
-        # prefill sizes: norm, logits GEMM + selection, bucketing as separate launches (see ROUTER_GEMM_MIN_ROWS)
+    split = ROUTER_SPLIT_LOGITS_SLABS if isinstance(x, PartialSum) else ROUTER_SPLIT_LOGITS
+    if router_by_gemm(T, E, H) or (align_with_shared is not None and E % 8 == 0 and T * E >= split):
+        # norm, router and bucketing as separate launches
         yn, rn = add_rmsnorm_partial(x, r2, norm_weight, eps) if isinstance(x, PartialSum) else add_rmsnorm(x.reshape(-1, H), r2, norm_weight, eps)
         idx, w = router_topk(yn, gate_w, bias, k, routed_scaling_factor)
         if align_with_shared is None:

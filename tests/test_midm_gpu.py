@@ -241,22 +241,45 @@ def test_feed_forward_gives_rows_unless_asked(ops):
     close(y, parts.part.cpu().double().sum(0), "rows and slabs")
 
 
-@pytest.mark.parametrize("T,E,slices", [(192, 64, 4), (191, 64, 4), (97, 128, 8), (300, 64, 0)])
-def test_norm_and_router_of_slices(ops, T, E, slices):
-    """The norm behind a projection (its partial sums or its rows), the router and the bucketing: as launches of their own, on either side of the
-    number of logits from which they are."""
-    H, k = 1024, 4
-    rows = rnd(T, H, seed=50).cuda()
-    parts = torch.randn(slices, T, H, generator=torch.Generator().manual_seed(51)).cuda() if slices else None
-    res, nw, gw = rnd(T, H, seed=52).cuda(), (1 + 0.1 * rnd(H, seed=53).float()).to(BF).cuda(), rnd(E, H, seed=54, scale=H ** -0.5).cuda()
-    bias = (torch.rand(E, generator=torch.Generator().manual_seed(55)) * 0.2 - 0.1).float().cuda()
-    x = ops.PartialSum(parts) if slices else rows
-    y, ro, idx, w, al = ops.add_rmsnorm_router_topk(x, res, nw, 1e-5, gw, bias, k, 1.0, align_with_shared=True)
-    y2, ro2 = ops.add_rmsnorm_partial(x, res, nw, 1e-5) if slices else ops.add_rmsnorm(x, res, nw, 1e-5)
-    idx2, w2 = ops.router_topk(y2, gw, bias, k, 1.0)
-    assert torch.equal(y, y2) and torch.equal(ro, ro2) and torch.equal(idx, idx2) and torch.equal(w, w2)
-    (offs, tok, scale, pos), flat = [t.cpu() for t in al], idx.cpu().flatten()
-    counts = torch.bincount(flat, minlength=E)
-    assert offs.tolist() == [0] + counts.cumsum(0).tolist() + [T * (k + 1)]
-    assert torch.equal(tok[pos.long()].long(), torch.arange(T).repeat_interleave(k)) and torch.equal(scale[pos.long()], w.cpu().flatten())
-    assert (pos >= offs[flat]).all() and (pos < offs[flat + 1]).all() and pos.unique().numel() == T * k   # (any order within an expert)
+@pytest.mark.parametrize("T,E,H,slices,gemm,split", [
+    (191, 64, 1024, 4, False, False), (192, 64, 1024, 4, False, True), (255, 64, 512, 0, False, False), (256, 64, 512, 0, False, True), (257, 64, 512, 0, True, True),
+    (300, 64, 1024, 3, True, True), (257, 40, 512, 4, False, False), (95, 128, 4096, 0, False, False), (96, 128, 4096, 0, True, True), (95, 128, 4096, 4, False, False),
+    (128, 128, 2048, 0, False, True), (48, 256, 2048, 4, True, True), (103, 152, 2048, 4, False, True), (700, 16, 512, 0, False, False), (1024, 16, 512, 0, True, True), (400, 60, 512, 4, False, False)])
+def test_norm_router_and_bucketing_by_size(ops, monkeypatch, T, E, H, slices, gemm, split):
+    """The norm behind a projection (its rows or its K slices), the router and the bucketing, on either side of every line between one launch and
+    several and between the launch's own logits and a GEMM: norm and routing against the oracle, the bucketing as moe_align's contract, and all
+    entry points alike — with the one launch too, wherever the logits are its own."""
+    from test_hip_kernels import _check_align, _check_router
+    k = 4
+    assert ops.router_by_gemm(T, E, H) == gemm
+    rows = rnd(T, H, seed=50)
+    parts = torch.randn(max(slices, 1), T, H, generator=torch.Generator().manual_seed(51))
+    res, nw, gw = rnd(T, H, seed=52), (1 + 0.1 * rnd(H, seed=53).float()).to(BF), rnd(E, H, seed=54, scale=H ** -0.5)
+    bias = (torch.rand(E, generator=torch.Generator().manual_seed(55)) * 0.2 - 0.1).float()
+    x = ops.PartialSum(parts.cuda()) if slices else rows.cuda()
+    calls = []
+    for name in ("add_rmsnorm", "add_rmsnorm_partial"):
+        f = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *a, f=f: (calls.append(1), f(*a))[1])
+    args = (x, res.cuda(), nw.cuda(), 1e-5, gw.cuda(), bias.cuda(), k, 1.0)
+    y, ro, idx, w, al = ops.add_rmsnorm_router_topk(*args, align_with_shared=True)
+    assert bool(calls) == split
+    # the sum's rounding: one ulp of a value below 8 beside a boundary (2^-5), which is what a residual near zero then differs by; the norm
+    # divides by the root of a mean square above one and rounds twice more
+    s = ((parts.double().sum(0).to(BF) if slices else rows).double() + res.double())
+    assert s.abs().max() < 16 and s.pow(2).mean(-1).min() > 1
+    assert_close_bf16(ro, s.to(BF), 1, 0.05, atol=2 ** -5, what="residual")
+    ref = (s * (s.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()).to(BF).double() * nw.double()
+    assert_close_bf16(y, ref.to(BF), 2, 0.35, atol=2 ** -5, what="norm")
+    _check_router(ops, y.cpu(), gw, bias, k, 1.0, f"{T} x {E}", allow_flip_rows=0.05)
+    _check_align(*al, idx.cpu(), w.cpu(), E, True)
+    idx2, w2 = ops.router_topk(y, gw.cuda(), bias.cuda(), k, 1.0)
+    y3, ro3, idx3, w3 = ops.add_rmsnorm_router_topk(*args)
+    assert torch.equal(idx, idx2) and torch.equal(w, w2) and all(torch.equal(a, b) for a, b in zip((y, ro, idx, w), (y3, ro3, idx3, w3)))
+    if not gemm:
+        for name in ("ROUTER_SPLIT_LOGITS", "ROUTER_SPLIT_LOGITS_SLABS"):
+            monkeypatch.setattr(ops, name, 1 << 40)
+        del calls[:]
+        y4, ro4, idx4, w4, al4 = ops.add_rmsnorm_router_topk(*args, align_with_shared=True)
+        assert not calls and all(torch.equal(a, b) for a, b in zip((y, ro, idx, w), (y4, ro4, idx4, w4)))
+        _check_align(*al4, idx4.cpu(), w4.cpu(), E, True)
