@@ -464,8 +464,11 @@ enum MidmTile { MM_NONE, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM
 MidmTile midm_tile_of(int mode, const GemmParams& p) {
     const int64_t n = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
     auto fits = [&](int rows, int cols) { return (n + cols - 1) / cols * ((p.R + rows - 1) / rows) <= 256; };
-    // (K steps of a short reduction are few: what the tiled kernel adds up in order stays so there for more rows)
-    if (fits(64, 32) && (p.K > 512 || p.R <= 256)) return MM_SPLIT32;
+    // A short reduction is mostly the two ends, a ring filled once and the sum of the waves: the shared tile's are shorter with gate and up rows in
+    // it, and with a hundred row blocks and more.  Shared 64 x 64 / split 64 x 32, us: 1024 x 256 at 300 rows 4.3 / 3.8, 264 x 512 at 700 5.7 / 4.7,
+    // 512 x 384 at 1000 4.7 / 4.1, fp32 rows 6.2 / 4.8, 64 x 512 at 3000 5.2 / 4.6, at 8000 6.1 / 6.4; gated columns 512 x 128 at 96 rows 3.0 / 3.4,
+    // 1024 x 320 at 128 4.1 / 4.2, 256 x 512 at 300 4.4 / 3.9, 132 x 512 at 700 4.6 / 4.4, at 1500 4.9 / 5.5.
+    if (fits(64, 32) && (gemm_paired(mode) ? p.K >= (p.R <= 1000 ? 384 : 576) : p.K > 512 || p.R <= 4096)) return MM_SPLIT32;
     if (fits(64, 64)) return p.K >= 8192 ? MM_SPLIT64 : MM_64;
     if (p.R <= 64) return fits(64, 128) ? MM_64x128 : MM_NONE;
     if (fits(128, 64)) return MM_128x64;
