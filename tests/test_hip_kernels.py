@@ -852,9 +852,14 @@ def test_error_reporting(ops):
 
 # ------------------------------------------------------------------------------------------
 # prefill regime: LDS-tiled MFMA GEMM (avg rows/group >= 96) and varlen causal attention
+@pytest.mark.parametrize("cfg", [0, 1, 2])
 @pytest.mark.parametrize("M,N,K,bias", [(96, 64, 64, False), (128, 200, 4096, True), (200, 4096, 1408, False),
-                                        (1000, 384, 352, True), (130, 14336 // 4, 512, True)])
-def test_gemm_bf16_large_m(ops, M, N, K, bias):
+                                        (1000, 384, 352, True), (130, 14336 // 4, 512, True),
+                                        # by size on the tiled kernel: one round of 128-row blocks, 256-row blocks, both ragged
+                                        (391, 14336, 128, True), (777, 14328, 64, False), (1300, 11000, 128, True)])
+def test_gemm_bf16_large_m(ops, opt_guard, M, N, K, bias, cfg):
+    """cfg: 0 by size (gemm_midm where its tiles are a round), 1 and 2 the tiled kernel's 128- and 256-row blocks."""
+    opt_guard("largem_cfg", cfg)
     x = rnd(M, K, seed=81)
     w = rnd(N, K, seed=82, scale=K ** -0.5)
     b = rnd(N, seed=83) if bias else None
@@ -905,13 +910,21 @@ def test_gemm_large_m_quadrant_loop_equals_plain_loop(ops, K):
     assert_close_bf16(got[2], O.linear(xp, wp, bias), 1, 0.05, atol=2 ** -9, what=f"plain K={K}")
 
 
-@pytest.mark.parametrize("T,nh,nkv,K,with_cache,need_kv", [(1024, 12, 2, 512, True, True), (300, 4, 1, 256, True, False),
-                                                          (777, 6, 2, 192, False, True), (4096, 96, 8, 4096, True, True)])
-def test_qkv_gemm_with_rope_store_epilogue(ops, T, nh, nkv, K, with_cache, need_kv):
+@pytest.mark.parametrize("T,nh,nkv,K,with_cache,need_kv,cfg", [
+    (1024, 12, 2, 512, True, True, 0), (300, 4, 1, 256, True, False, 0), (777, 6, 2, 192, False, True, 0), (4096, 96, 8, 4096, True, True, 0),
+    # the tiled kernel's epilogue: ragged row blocks of 256 and of 128, asked for and by size (one round of 128-row blocks up to 512 rows here,
+    # 256-row blocks beyond)
+    (1024, 12, 2, 512, True, True, 2), (300, 4, 1, 256, True, False, 2), (777, 6, 2, 192, False, True, 2),
+    (1024, 12, 2, 512, True, True, 1), (300, 4, 1, 256, True, False, 1), (777, 6, 2, 192, False, True, 1),
+    (300, 96, 8, 128, True, True, 0), (400, 96, 8, 192, True, False, 0), (512, 96, 8, 64, False, True, 0), (391, 96, 8, 128, False, False, 0),
+    (777, 96, 8, 128, True, True, 0), (1000, 96, 8, 128, True, False, 0)])
+def test_qkv_gemm_with_rope_store_epilogue(ops, opt_guard, T, nh, nkv, K, with_cache, need_kv, cfg):
     """r04: glm_gemm_qkv_rope_store (QKV projection whose epilogue splits, rotates q / k and scatters K / V into the paged
     cache) == glm_gemm_bf16 followed by glm_qkv_split_norm_rope_store, bit for bit — q, k, v and every cache row, rows with
     slot -1 untouched — and both against the oracle (linear.py:74-75, rotary_embedding.py:39-55, attention.py:10-42).  The
-    last case is the Air shape (H = 4096, 96 / 8 heads); ragged T exercises partial row blocks."""
+    4096-row case is the Air shape (H = 4096, 96 / 8 heads); ragged T exercises partial row blocks, cfg the tiled kernel where the row count alone
+    goes to gemm_midm."""
+    opt_guard("largem_cfg", cfg)
     hd, rd = 128, 64
     N = (nh + 2 * nkv) * hd
     x = rnd(T, K, seed=901)

@@ -37,11 +37,11 @@ SILU = (4, 0.06, 2 ** -8)
 
 # (rows, columns, K): split waves (K of one chunk, three waves without work, up to several rounds of the ring; the large tile of long
 # reductions), then every tile of the shared ring, fewer chunks than stages and many, columns that end inside a tile, rows that end inside a
-# block, and one of the tiled kernel's (its epilogues)
+# block, and the tiled kernel's epilogues on 256-row blocks and on 128-row blocks
 SIZES = [(33, 36, 64), (64, 100, 128), (65, 2048, 192), (97, 2052, 1088), (128, 264, 4096), (130, 4128, 8256),
          (211, 2112, 2048), (520, 1000, 1024), (300, 3000, 64), (130, 6404, 64), (129, 5700, 704), (33, 16420, 320), (64, 20000, 128), (256, 8200, 576),
          (1300, 2056, 128), (700, 264, 512), (4096, 64, 192), (4100, 60, 192),
-         (1300, 6152, 128)]
+         (1300, 6152, 128), (391, 14344, 64)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
@@ -84,7 +84,7 @@ def test_activations(ops, M, N, K):
 @pytest.mark.parametrize("M,I,K", [(33, 24, 64), (65, 1000, 192), (97, 1408, 1088), (211, 4104, 576), (300, 264, 1024), (100, 3000, 128), (130, 3016, 64),
                                    (64, 9000, 192), (48, 1024, 1024), (64, 1032, 512), (95, 1368, 512), (64, 2048, 2048), (64, 2056, 2048), (64, 4096, 1024), (65, 4096, 64),
                                    (33, 384, 4096), (95, 448, 2688), (95, 448, 2736),
-                                   (97, 40, 320), (97, 40, 384), (1000, 40, 512), (1001, 40, 512), (1001, 40, 576)])
+                                   (97, 40, 320), (97, 40, 384), (1000, 40, 512), (1001, 40, 512), (1001, 40, 576), (391, 7176, 128), (1300, 7176, 64)])
 def test_gated(ops, M, I, K):
     x, w = rnd(M, K, seed=6), rnd(2 * I, K, seed=7, scale=K ** -0.5)
     g, u = (x.double() @ w.double().T).chunk(2, 1)
