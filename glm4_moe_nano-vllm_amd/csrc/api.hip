@@ -287,12 +287,17 @@ extern "C" int glm_gemm_bf16_slices(int64_t M, int N, int K) {
     return best;
 }
 
-// ... and from 33 rows on: the tiles of gemm_midm.hip first, then those of the tiled kernel where K is long enough to pay for their sums (with
-// the norm that adds them up, us, one pass / slices: 4096 x 4096 at 400 rows 36 / 39, at 1000 50 / 54; 2048 x 6144 at 700 47 / 40, at 1000
-// 50 / 46; 4096 x 12288 at 400 95 / 62, at 1000 123 / 101)
+// ... and from 33 rows on: the tiles of gemm_midm.hip first, then those of the tiled kernel where K is long enough to pay for their sums, which is
+// sooner where one pass is more than half a round of gemm_midm's 128 x 128 tiles, and soonest where it is beyond the round.  With the norm that adds
+// them up, us, one pass / slices: 2048 x 6144 at 700 rows 47 / 40, at 1000 50 / 46, 4096 x 12288 at 400 95 / 62, at 1000 123 / 101; less than half a
+// round 2048 x 5632 at 1000 50 / 63, 4096 x 5120 at 512 48 / 53; 2048 x 4608 at 1500 59 / 57, x 5120 66 / 62, x 5632 69 / 62, 3072 x 4608 at 1000 62 / 60,
+// x 5120 69 / 63, 4096 x 5120 at 1000 70 / 71; 3072 x 4096 at 1500 74 / 69, x 4608 82 / 69, 2048 x 4096 at 3000 73 / 70, x 5120 88 / 80, 4096 x 4096
+// at 2000 82 / 85, x 5120 99 / 97
 extern "C" int glm_gemm_bf16_row_slices(int64_t M, int N, int K) {
     const int s = glm_midm_slices(M, N, K);
-    return s > 1 ? s : K >= 6144 && N % 8 == 0 ? glm_gemm_bf16_slices(M, N, K) : 1;   // (N % 8: what the tiled kernel's slabs need)
+    if (s > 1 || N % 8 != 0) return s;   // (N % 8: what the tiled kernel's slabs need)
+    const int64_t tiles = (M + 127) / 128 * ((N + 127) / 128);
+    return K >= (tiles > 256 ? 4096 : tiles >= 144 ? 5120 : 6144) ? glm_gemm_bf16_slices(M, N, K) : 1;
 }
 
 extern "C" int glm_gemm_bf16_partial(const void* x, int64_t ldx, const void* w, int64_t ldw, float* ypart,

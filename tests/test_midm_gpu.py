@@ -199,8 +199,10 @@ def test_row_slices(ops, M, N, K):
 
 
 def test_row_slices_only_where_they_are_taken(ops):
-    """No count that gemm_bf16_partial refuses: tiled slabs of columns off eight, weights beyond 32-bit offsets with no kernel to fall back on."""
+    """Where they pay (fewer K for more tiles); no count that gemm_bf16_partial refuses: tiled slabs of columns off eight, weights beyond 32-bit offsets with no kernel to fall back on."""
     assert ops.row_slices(700, 2056, 8192) > 1 and ops.row_slices(700, 2052, 8192) == 1
+    assert ops.row_slices(1000, 2048, 5632) == 1 < ops.row_slices(1000, 2048, 6144) and ops.row_slices(1500, 2048, 4608) == 1 < ops.row_slices(1500, 2048, 5120)
+    assert ops.row_slices(3000, 2048, 4096) > 1 and ops.row_slices(3000, 2048, 4032) == 1 and ops.row_slices(16384, 2048, 8192) == 1
     assert ops.row_slices(64, 4096, 65536) > 1 and ops.row_slices(64, 4096, 262144) == 1 and ops.row_slices(95, 2048, 262144) == 1
 
 
