@@ -643,20 +643,20 @@ def varlen_attn_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, scale
 # (glm_router_topk / the fused add-RMSNorm + router + bucketing launch), which is built for decode latency: at T = 16384
 # it takes 1.2 ms per layer against 0.34 ms for norm + GEMM + select + bucketing (tools/prefill_router_probe.py).
 # That kernel is one workgroup a token: beyond 256 tokens it is a second round of the chip, and with many experts a token's pass over Wg is long.
-# One launch / GEMM and selection, us, hidden size 2048 and 4096: 64 experts at 256 tokens 8.9 / 11.3 and 12.3 / 14.4, at 257 14.6 / 11.3 and
-# 20.2 / 14.7; 96 at 256 12.4 / 13.5 and 17.2 / 16.6; 128 at 128 13.6 / 13.6 and 19.3 / 16.8; 192 at 96 17.3 / 13.9 and 24.3 / 17.2; 16 at 768
-# 17.1 / 11.0 and 20.5 / 14.2.  With the norm, in the one launch or ahead of the two: 64 at 256 10.0 / 14.7 and 14.1 / 19.3, at 257 16.8 / 14.8 and
-# 23.0 / 20.1; 128 at 128 15.0 / 16.6 and 21.0 / 21.1; 160 at 96 16.1 / 16.7 and 22.1 / 21.1; 192 at 96 18.2 / 16.9 and 25.7 / 21.4.  (With the bucketing,
-# from rows, the launches around a GEMM lose a little below 16384 logits: 128 at 96, 4096 wide, 20.0 / 22.9.)
+# One launch / GEMM and selection, us, hidden size 2048 and 4096, Wg not in the caches: 64 experts at 256 tokens 10 / 13 and 14 / 18, at 257 16 / 13 and
+# 21 / 17; 96 at 256 13 / 15 and 18 / 20; 128 at 160 15 / 15 and 21 / 20; 160 at 128 16 / 16 and 23 / 21; 256 at 48 22 / 16 and 34 / 21.  With the
+# norm, in the one launch or ahead of the two: 64 at 256 11 / 17 and 15 / 23, at 257 18 / 16 and 25 / 22; 128 at 128 16 / 19 and 23 / 25, at 160 16 / 18 and
+# 23 / 24; 160 at 96 17 / 18 and 24 / 24; 256 at 48 23 / 19 and 35 / 25.
 ROUTER_GEMM_MIN_ROWS = 1024
 ROUTER_GEMM_MIN_LOGITS = 12288     # (T x E; nothing below was measured to gain)
 ROUTER_ROUND_TOKENS = 256
 ROUTER_GEMM_MIN_EXPERTS, ROUTER_GEMM_MIN_GATE = 128, 160 * 2048   # within the first round: experts, E x H
+ROUTER_MANY_EXPERTS, ROUTER_SPLIT_LOGITS_MANY = 192, 20480
 # The bucketing in the same launch spreads a token's experts over workgroups, each of which repeats the norm and reads the K slices: the norm, the
-# router and the bucketing as launches of their own are ahead from T x E logits on, whichever way those are computed.  One / three or four, us,
-# H = 2048 and 4096: 64 at 192 18.0 / 17.9 and 20.1 / 22.3, at 256 20.3 / 18.7 and 23.8 / 23.4, at 700 43 / 25 and 52 / 33; 128 at 96 17.3 / 18.8 and
-# 20.0 / 22.9, at 128 20.3 / 19.3 and 23.6 / 24.2; 256 at 64 20.6 / 19.7 and 24.0 / 23.9; from four slabs 64 at 192 22.7 / 18.5 and 27.1 / 24.6, at
-# 700 75 / 28 and 93 / 36, 128 at 96 23.2 / 19.3 and 27.5 / 24.0, 256 at 48 24.1 / 19.7 and 28.4 / 24.4.
+# router and the bucketing as launches of their own are ahead from T x E logits on, whichever way those are computed.  One / three or four, us:
+# 64 at 256 20 / 17 and 25 / 21, at 512 32 / 24 and 40 / 31; 96 at 192 23 / 19 and 28 / 24; 128 at 128 19 / 21 and 24 / 27, at 160 23 / 21 and
+# 28 / 27; 160 at 128 23 / 22 and 28 / 28; 256 at 64 19 / 22 and 24 / 29, at 96 24 / 22 and 31 / 27 (its logits are a GEMM already).  From four slabs 64 at
+# 192 23 / 17 and 28 / 21, at 512 53 / 25 and 72 / 33, 128 at 96 24 / 21 and 29 / 28, at 128 29 / 21 and 37 / 29, 256 at 48 24 / 23 and 30 / 29.
 ROUTER_SPLIT_LOGITS, ROUTER_SPLIT_LOGITS_SLABS = 16384, 12288
 
 
@@ -666,7 +666,8 @@ def router_by_gemm(T: int, E: int, H: int = 0) -> bool:
         return False
     if T > ROUTER_ROUND_TOKENS:
         return T >= ROUTER_GEMM_MIN_ROWS or T * E >= ROUTER_GEMM_MIN_LOGITS
-    return E >= ROUTER_GEMM_MIN_EXPERTS and E * H >= ROUTER_GEMM_MIN_GATE and T * E >= ROUTER_GEMM_MIN_LOGITS
+    return (E >= ROUTER_GEMM_MIN_EXPERTS and E * H >= ROUTER_GEMM_MIN_GATE
+            and T * E >= (ROUTER_GEMM_MIN_LOGITS if E >= ROUTER_MANY_EXPERTS else ROUTER_SPLIT_LOGITS_MANY))
 
 
 def router_select(logits: torch.Tensor, bias: torch.Tensor, k: int, routed_scaling_factor: float):
@@ -732,7 +733,7 @@ def add_rmsnorm_router_topk(x, residual: torch.Tensor, norm_weight: torch.Tensor
     r2 = residual.reshape(-1, H).contiguous()
     T = r2.shape[0]
     E = gate_w.shape[0]
-    split = ROUTER_SPLIT_LOGITS_SLABS if isinstance(x, PartialSum) else ROUTER_SPLIT_LOGITS
+    split = ROUTER_SPLIT_LOGITS_SLABS if isinstance(x, PartialSum) else ROUTER_SPLIT_LOGITS if E < ROUTER_GEMM_MIN_EXPERTS else ROUTER_SPLIT_LOGITS_MANY
     if router_by_gemm(T, E, H) or (align_with_shared is not None and E % 8 == 0 and T * E >= split):
         # norm, router and bucketing as separate launches
         yn, rn = add_rmsnorm_partial(x, r2, norm_weight, eps) if isinstance(x, PartialSum) else add_rmsnorm(x.reshape(-1, H), r2, norm_weight, eps)

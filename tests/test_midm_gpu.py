@@ -246,8 +246,10 @@ def test_feed_forward_gives_rows_unless_asked(ops):
 
 @pytest.mark.parametrize("T,E,H,slices,gemm,split", [
     (191, 64, 1024, 4, False, False), (192, 64, 1024, 4, False, True), (255, 64, 512, 0, False, False), (256, 64, 512, 0, False, True), (257, 64, 512, 0, True, True),
-    (300, 64, 1024, 3, True, True), (257, 40, 512, 4, False, False), (95, 128, 4096, 0, False, False), (96, 128, 4096, 0, True, True), (95, 128, 4096, 4, False, False),
-    (128, 128, 2048, 0, False, True), (48, 256, 2048, 4, True, True), (103, 152, 2048, 4, False, True), (700, 16, 512, 0, False, False), (1024, 16, 512, 0, True, True), (400, 60, 512, 4, False, False)])
+    (300, 64, 1024, 3, True, True), (257, 40, 512, 4, False, False), (159, 128, 4096, 0, False, False), (160, 128, 4096, 0, True, True),
+    (95, 128, 4096, 4, False, False), (96, 128, 4096, 4, False, True), (160, 128, 2048, 0, False, True), (48, 256, 2048, 4, True, True),
+    (103, 152, 2048, 4, False, True), (128, 160, 2048, 0, True, True), (127, 160, 2048, 0, False, False), (700, 16, 512, 0, False, False),
+    (1024, 16, 512, 0, True, True), (400, 60, 512, 4, False, False)])
 def test_norm_router_and_bucketing_by_size(ops, monkeypatch, T, E, H, slices, gemm, split):
     """The norm behind a projection (its rows or its K slices), the router and the bucketing, on either side of every line between one launch and
     several and between the launch's own logits and a GEMM: norm and routing against the oracle, the bucketing as moe_align's contract, and all
@@ -280,7 +282,7 @@ def test_norm_router_and_bucketing_by_size(ops, monkeypatch, T, E, H, slices, ge
     y3, ro3, idx3, w3 = ops.add_rmsnorm_router_topk(*args)
     assert torch.equal(idx, idx2) and torch.equal(w, w2) and all(torch.equal(a, b) for a, b in zip((y, ro, idx, w), (y3, ro3, idx3, w3)))
     if not gemm:
-        for name in ("ROUTER_SPLIT_LOGITS", "ROUTER_SPLIT_LOGITS_SLABS"):
+        for name in ("ROUTER_SPLIT_LOGITS", "ROUTER_SPLIT_LOGITS_SLABS", "ROUTER_SPLIT_LOGITS_MANY"):
             monkeypatch.setattr(ops, name, 1 << 40)
         del calls[:]
         y4, ro4, idx4, w4, al4 = ops.add_rmsnorm_router_topk(*args, align_with_shared=True)
