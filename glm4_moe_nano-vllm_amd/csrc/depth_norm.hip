@@ -383,7 +383,8 @@ constexpr int64_t DN_SPLIT_ROWS = 512;   // rows from which norm and convolution
 
 template <int TAPS>
 int launch_depth_conv(const DepthArgs& a, const float* xs, hipStream_t st) {
-    // 16 rows per workgroup: four workgroups to a CU (15074 rows of 2048: 57 -> 40 us; 32 rows left two, 8 read too many rows twice: 43)
+    // 16 rows per workgroup: four workgroups to a CU (15074 rows of 2048: 57 -> 40 us; 32 rows left two, 8 read too many rows twice: 43).  With the
+    // norm ahead of it, 32 / 16 rows, us: 1000 rows of 1024 32 / 21, of 4096 44 / 31; 4096 rows of 2048 52 / 40, 15074 rows of 4096 206 / 209
     const int tr = 16;
     hipLaunchKernelGGL(depth_conv_kernel<TAPS>, dim3((unsigned)((a.T + tr - 1) / tr), (unsigned)((a.wp + 2047) / 2048)), dim3(256), 0, st, a, xs, tr);
     GLM_CHECK_LAUNCH("glm_depth_norm(convolution)");

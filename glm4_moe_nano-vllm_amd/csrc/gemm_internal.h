@@ -23,7 +23,7 @@ enum GemmMode : int {
     GEMM_COLS = 6,   // per-column activation (glm_act_cols), bf16 rows
     // Fp32 rows with nothing behind the bias (a loop's entry, logits), and logits through a soft cap: every activation inlined per element
     // and chosen at run time made GEMM_ACT's epilogue as long as its loop.  2048 x 4096 at 15074 rows 293 -> 212 us (bf16 rows 200); on these
-    // tiles 32768 x 2048 at 128 rows 85 -> 43, with the cap 93 -> 50 (since then a round of gemm_midm.hip's, 38).
+    // tiles 32768 x 2048 at 128 rows 85 -> 43, with the cap 93 -> 50 (since then a round of gemm_midm.hip's: 43 and 48, weights not in the caches).
     GEMM_F32 = 8,
     GEMM_CAP = 9,
     GEMM_SLICES = 7, // G slices of K side by side, K the length of one: fp32 partial sums, slab s of R rows at yf + s R ldy

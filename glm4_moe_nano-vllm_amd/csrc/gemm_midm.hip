@@ -137,7 +137,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
     const unsigned ring = (unsigned)(uintptr_t)(const mm_lds_void*)smem + wid * NST * STAGE;
     char* ringp = smem + wid * NST * STAGE;
 
-    // ---- sources: instruction i brings rows 16 i + (lane >> 2), piece lane & 3 of the LDS row
+    // ---- sources: instruction i brings rows 8 i + (lane >> 3), piece lane & 7 of the LDS row
     const int r8 = lane >> 3, pc = lane & 7;
     const __amdgpu_buffer_rsrc_t wrs = mm_rsrc(p.w + (int64_t)grp * p.w_gstride), xrs = mm_rsrc(p.x);
     unsigned wvo[2 * RT], xvo[2 * MT];
@@ -158,7 +158,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
         xvo[i] = ((unsigned)src * (unsigned)p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8) * 2u;
         last = max(last, src);
     }
-    // ---- this wave's chunks: wid, wid + 4, ... of the K columns
+    // ---- this wave's chunks: wid, wid + NW, ... of the K columns
     const int n = max(0, (p.K / MM_KC - wid + NW - 1) / NW);
     auto issue_w = [&](int j, int slot) {
 #pragma unroll
@@ -237,7 +237,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
         } else loop(std::false_type{});
     }
 
-    // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / 4 ..
+    // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / NW ..
     constexpr int MPW = MT / NW;
     __syncthreads();
     float* red = reinterpret_cast<float*>(smem);
@@ -457,7 +457,7 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
 // work and have more bytes on their way; a larger tile pulls fewer, and two rounds of one cost more than one round of the next.  Split, 64 x 64,
 // 128 x 64, 128 x 128 (64 rows: 64 x 128), us, cold operands, * the one taken: 4096 x 4096 at 64 rows 16.5* / 21.2 / - / 30, at 211 24.5 / 20.5* /
 // 30.0 / 36.2, at 512 47 / - / 31.8* / 40.2; 14336 x 4096 at 64 36.7 / 27.6* / - / 37.5, at 128 56 / 42.6 / 37.7* / 46.3, at 211 77 / 61.5 / 52 /
-// 43.0*; 2048 x 2048 at 1000 rows - / 16.9* / 17.2 / 19.8, at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
+// 43.0*; 2048 x 2048 at 1000 rows - / 16.9 / 17.2* / 19.8 (512 tiles of 64 x 64), at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
 // A long K favours split waves at 64 x 64 too, which read each staged byte once: 4096 x 12288 at 211 rows 50 (shared 58), K = 8192 36 (40).
 enum MidmTile { MM_NONE, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
 

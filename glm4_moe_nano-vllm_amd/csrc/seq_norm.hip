@@ -400,9 +400,11 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
 template <int TAPS, int NT>
 int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
     // decode: one row per workgroup; else runs of rows long enough to spread the halo and the register setup, short enough
-    // to fill the chip
-    // four waves on every SIMD: a row is a chain of one load, two reductions and a store, with one row's loads in flight per workgroup (15074
-    // rows of 2048: with 512 workgroups of 256 threads 95 us, 1024 75, 2048 78)
+    // to fill the chip: a row is a chain of one load, two reductions and a store, with one row's loads in flight per workgroup, so some hundred rows
+    // stay one to a workgroup, re-reading the halo, as long as those are no more than four waves a SIMD (2048 workgroups of 64 threads: two), and
+    // longer runs are cut for as many.  Four taps, us, runs of eight rows and more for 512 workgroups / this: 1024 columns at 800 rows 19.4 / 10.4, at 2048 20.6 / 15.9, at 8000
+    // 46 / 33; 2048 at 600 rows 21.5 / 12.5, at 1024 21.9 / 16.0 (1025: 21.8, runs of eight), at 6000 45 / 40, at 15074 108 / 98 (without taps
+    // 95 / 83; 2048 workgroups 78 where 1024 took 75).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;

@@ -140,11 +140,11 @@ class RowParallelLinear(LinearBase):
     partial_min_k = 8192
     partial_slices = 8
 
-    partial_max_rows = 1024   # (one pass / slices with the norm at 1000 rows still 123 / 101 us; not measured beyond)
+    partial_max_rows = 1024   # (4096 x 12288, one pass / slices with the norm behind it, at 1000 rows 123 / 101 us)
 
     def _slices(self, x: torch.Tensor) -> int:
         m, n = x.shape[0], self.weight.shape[0]
-        if m > 32:   # 4096 x 12288: 64 rows 45 -> 23 us, 211 rows 56 -> 37, 400 rows 108 -> 50
+        if m > 32:   # 4096 x 12288, one pass / slices with the norm behind it, us: 64 rows 49 / 31, 211 rows 54 / 45, 400 rows 95 / 62
             # (columns that the norm can add up; rows that 32-bit offsets reach)
             ok = m < self.partial_max_rows and n % 8 == 0 and n <= hip_ops.ADD_NORM_PARTIAL_MAX_H and m * x.stride(0) < 1 << 30
             return hip_ops.row_slices(m, *self.weight.shape) if ok else 1
