@@ -360,7 +360,8 @@ int glm_gemm_bf16_partial_slices(int K, int want);
 /* From 33 rows on glm_gemm_bf16_partial takes equal slices of whole 64-wide K tiles (K % (64 nslices) == 0); for 96 rows and more
  *     glm_gemm_bf16_slices returns how many bring a launch of the tiled kernel's few output tiles to a workgroup per CU (1: no split). */
 int glm_gemm_bf16_slices(int64_t M, int N, int K);
-/* ... from 33 rows on, with the smaller tiles of some dozen to some hundred rows where those have four slices at least       */
+/* ... from 33 rows on, with the smaller tiles of some dozen to some hundred rows where those have four slices at least; the
+ *     number is one that glm_gemm_bf16_partial takes (rows of x and of W behind 32-bit byte offsets up to 95 rows).          */
 int glm_gemm_bf16_row_slices(int64_t M, int N, int K);
 int glm_gemm_bf16_partial(const void* x, int64_t ldx, const void* w, int64_t ldw, float* ypart,
                           int64_t M, int N, int K, int nslices, glm_stream_t stream);
