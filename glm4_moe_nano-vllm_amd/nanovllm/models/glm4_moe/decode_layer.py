@@ -98,7 +98,7 @@ class Glm4MoeDecoderLayer(nn.Module):
                 return hidden_states, residual
             hidden_states = op(o, defer_reduce=True)  # shape outside the fused launch's window: two launches
         else:
-            # o_proj may hand over K-slice partial sums; the add-RMSNorm right below reduces them (decode batches)
+            # o_proj may hand over K-slice partial sums; the add-RMSNorm right below reduces them (up to 1023 rows)
             hidden_states = self.self_attn(hidden_states, positions, defer_o_reduce=True, qkv=qkv)
         if self.fuse_norm_router and gate is not None and residual.shape[-1] <= 8192:
             # post-attention add-RMSNorm and the router of the same token in one launch

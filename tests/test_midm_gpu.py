@@ -288,3 +288,38 @@ def test_norm_router_and_bucketing_by_size(ops, monkeypatch, T, E, H, slices, ge
         y4, ro4, idx4, w4, al4 = ops.add_rmsnorm_router_topk(*args, align_with_shared=True)
         assert not calls and all(torch.equal(a, b) for a, b in zip((y, ro, idx, w), (y4, ro4, idx4, w4)))
         _check_align(*al4, idx4.cpu(), w4.cpu(), E, True)
+
+
+@pytest.mark.parametrize("T", [64, 211, 300])
+def test_layer_half_replayed(ops, T):
+    """K slices, norm, router, bucketing and experts of a step in a HIP graph: every replay, on new rows and between eager work, is the eager result."""
+    H, E, k, I, K = 1024, 64, 8, 192, 8192
+    wo, gw, nw = rnd(H, K, seed=70, scale=K ** -0.5).cuda(), rnd(E, H, seed=71, scale=H ** -0.5).cuda(), (1 + 0.1 * rnd(H, seed=72).float()).to(BF).cuda()
+    bias = (torch.rand(E, generator=torch.Generator().manual_seed(73)) * 0.2 - 0.1).cuda()
+    w13, w2 = rnd(E + 1, 2 * I, H, seed=74, scale=H ** -0.5).cuda(), rnd(E + 1, H, I, seed=75, scale=I ** -0.5).cuda()
+    x, res = torch.empty(T, K, dtype=BF, device="cuda"), torch.empty(T, H, dtype=BF, device="cuda")
+    slices = ops.row_slices(T, H, K)
+    assert slices > 1
+
+    def step():
+        y, ro, idx, w, (offs, tok, scale, pos) = ops.add_rmsnorm_router_topk(ops.gemm_bf16_partial(x, wo, slices), res, nw, 1e-5, gw, bias, k, 1.0, align_with_shared=True)
+        rows = ops.grouped_gemm_down(ops.grouped_gemm_gateup_silu(y, w13, offs, tok, T * (k + 1)), w2, offs, scale, E)
+        return y, ro, idx, w, ops.moe_combine(rows, pos, T, k, T * k)
+
+    def fill(seed):
+        x.copy_(rnd(T, K, seed=seed))
+        res.copy_(rnd(T, H, seed=seed + 1))
+
+    fill(80)
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for i in range(4):
+        fill(90 + 2 * i)
+        want = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want)), i
