@@ -124,10 +124,9 @@ __device__ __forceinline__ void midm_qkv_rows(const GemmParams& p, const f32x4_t
     }
 }
 
-// rows m0 .. m0 + mcnt - 1 of group grp, columns from ncol0; MT 16-row activation tiles, RT 16-row weight tiles; reach: rows of x whose bytes
-// 32-bit offsets address
+// rows m0 .. m0 + mcnt - 1, columns from ncol0; MT 16-row activation tiles, RT 16-row weight tiles
 template <int MODE, int MT, int RT, int NW, int NST>
-__device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int grp, int m0, int mcnt, int ncol0, int reach) {
+__device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int m0, int mcnt, int ncol0) {
     constexpr int D = 2 * (MT + RT);           // DMA instructions of a stage
     constexpr int STAGE = D * 1024;
     constexpr int HALF = 8 * RT;               // paired modes: gate rows of the tile, then as many up rows
@@ -139,7 +138,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
 
     // ---- sources: instruction i brings rows 8 i + (lane >> 3), piece lane & 7 of the LDS row
     const int r8 = lane >> 3, pc = lane & 7;
-    const __amdgpu_buffer_rsrc_t wrs = mm_rsrc(p.w + (int64_t)grp * p.w_gstride), xrs = mm_rsrc(p.x);
+    const __amdgpu_buffer_rsrc_t wrs = mm_rsrc(p.w), xrs = mm_rsrc(p.x);
     unsigned wvo[2 * RT], xvo[2 * MT];
 #pragma unroll
     for (int i = 0; i < 2 * RT; ++i) {
@@ -147,34 +146,20 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
         const int wr = gemm_paired(MODE) ? (row < HALF ? 0 : p.N) + min(ncol0 + (row < HALF ? row : row - HALF), p.N - 1) : min(ncol0 + row, p.N - 1);
         wvo[i] = ((unsigned)wr * (unsigned)p.ldw + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
     }
-    int last = 0;
-    auto source = [&](int i) {
-        const int m = m0 + min(8 * i + r8, mcnt - 1);   // rows past the end repeat the last one; they are never stored
-        return MODE == GEMM_GATEUP && p.src ? p.src[m] : m;
-    };
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) {
-        const int src = source(i);
-        xvo[i] = ((unsigned)src * (unsigned)p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8) * 2u;
-        last = max(last, src);
+        const int row = m0 + min(8 * i + r8, mcnt - 1);   // rows past the end repeat the last one; they are never stored
+        xvo[i] = ((unsigned)row * (unsigned)p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8) * 2u;
     }
     // ---- this wave's chunks: wid, wid + NW, ... of the K columns
     const int n = max(0, (p.K / MM_KC - wid + NW - 1) / NW);
-    auto issue_w = [&](int j, int slot) {
-#pragma unroll
-        for (int i = 0; i < 2 * RT; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)(ringp + slot * STAGE + i * 1024), 16, wvo[i], (j * NW + wid) * MM_ROWB, 0, 0);
-    };
-    auto issue_x = [&](auto far_rows, int j, int slot) {
+    auto issue = [&](int j, int slot) {
+        char* st = ringp + slot * STAGE;
         const int soff = (j * NW + wid) * MM_ROWB;
-        char* st = ringp + slot * STAGE + 2 * RT * 1024;
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) {
-            if constexpr (decltype(far_rows)::value)
-                __builtin_amdgcn_global_load_lds((mm_glb_void*)(p.x + (int64_t)source(i) * p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8 + soff / 2),
-                                                 (mm_lds_void*)(st + i * 1024), 16, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (mm_lds_void*)(st + i * 1024), 16, xvo[i], soff, 0, 0);
-        }
+        for (int i = 0; i < 2 * RT; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)(st + i * 1024), 16, wvo[i], soff, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (mm_lds_void*)(st + (2 * RT + i) * 1024), 16, xvo[i], soff, 0, 0);
     };
     // stage j has arrived, the younger ones stay in flight
     auto arrived = [&](int j) {
@@ -197,13 +182,10 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             for (int mt = 0; mt < MT; ++mt)
                 acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f.w[rt]), __builtin_bit_cast(bf16x8_t, f.x[mt]), acc[rt][mt], 0, 0, 0);
     };
-    auto loop = [&](auto far_rows) {
+    if (n > 0) {
 #pragma unroll
         for (int j = 0; j < NST; ++j)
-            if (j < n) {
-                if (j > 0) issue_w(j, j);
-                issue_x(far_rows, j, j);
-            }
+            if (j < n) issue(j, j);
         MmFrags<MT, RT> f0, f1;        // the two k-steps of a stage
         int slot = 0;
         arrived(0);
@@ -214,10 +196,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             __builtin_amdgcn_sched_barrier(0);
             mm(f0);
             f1.settle();               // the stage is in registers: its slot takes chunk j + NST
-            if (j + NST < n) {
-                issue_w(j + NST, slot);
-                issue_x(far_rows, j + NST, slot);
-            }
+            if (j + NST < n) issue(j + NST, slot);
             slot = slot + 1 == NST ? 0 : slot + 1;
             if (j + 1 < n) {
                 arrived(j + 1);
@@ -227,14 +206,6 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             mm(f1);
             if (j + 1 < n) f0.settle();
         }
-    };
-    if (n > 0) {
-        issue_w(0, 0);   // (ahead of the wait for the row numbers)
-        // gathered rows (of an x whose length nobody here knows) beyond what 32-bit offsets reach: the wave looks its rows up again at every stage
-        if constexpr (MODE == GEMM_GATEUP) {
-            if (__any(last >= reach)) loop(std::true_type{});
-            else loop(std::false_type{});
-        } else loop(std::false_type{});
     }
 
     // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / NW ..
@@ -266,7 +237,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int g
             return;
         }
     }
-    gemm_row_epilogue<MODE, RT, MPW>(p, sum, grp, m0 + first, mcnt - first, ncol0, c, g4);
+    gemm_row_epilogue<MODE, RT, MPW>(p, sum, 0, m0 + first, mcnt - first, ncol0, c, g4);
 }
 
 // row block and column tile of this workgroup
@@ -285,32 +256,219 @@ __device__ __forceinline__ void midm_tile(int mblocks, int interleaved, int& m, 
 template <int MODE, int MT, int RT, int NW, int NST>
 constexpr int midm_lds() {
     constexpr int ring = NW * NST * (MT + RT) * 2048, red = NW * MT * RT * 1024;
-    return (ring > red ? ring : red) + 16;
+    return ring > red ? ring : red;
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
-__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, int mblocks, int interleaved, int reach) {
+__global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, int mblocks, int interleaved) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int COLS = gemm_paired(MODE) ? 8 * RT : 16 * RT;
-    int grp = 0, m0, mcnt, ntile;
-    if (p.offs) {
-        int* sh = reinterpret_cast<int*>(smem + midm_lds<MODE, MT, RT, NW, NST>() - 16);
-        glm_locate_block(p.offs, p.G, p.R, 16 * MT, blockIdx.y, sh);
-        __syncthreads();
-        grp = __builtin_amdgcn_readfirstlane(sh[0]);
-        m0 = __builtin_amdgcn_readfirstlane(sh[1]);
-        mcnt = __builtin_amdgcn_readfirstlane(sh[2]);
-        ntile = blockIdx.x;
-        if (grp < 0) return;
-    } else {
-        int m;
-        midm_tile(mblocks, interleaved, m, ntile);
-        m0 = m * (16 * MT);
-        mcnt = min(16 * MT, (int)p.R - m0);
-    }
+    int m, ntile;
+    midm_tile(mblocks, interleaved, m, ntile);
+    const int m0 = m * (16 * MT);
     if (ntile * COLS >= p.N) return;
-    midm_body<MODE, MT, RT, NW, NST>(p, smem, grp, m0, mcnt, ntile * COLS, reach);
+    midm_body<MODE, MT, RT, NW, NST>(p, smem, m0, min(16 * MT, (int)p.R - m0), ntile * COLS);
 }
+
+#if GLM_EXPERTS
+// The split body for experts: rows m0 .. m0 + mcnt - 1 of group grp, 64 weight rows, two waves and two workgroups per CU, so that one is at work
+// while the other starts or sums up.  MT: 16-row activation tiles, two where the rows are no more (the chip then moves half as many activation
+// bytes as weight bytes, not as many).  once: no other row block reads these weights, which then leave the caches to the activations (nt; with
+// several blocks it costs a tenth).  A wave sends the other one the half of its partial tile that it does not finish, and everything that the
+// end needs is loaded before the stream.  65 experts of 1408 x 4096, gate|up / down, us: 211 tokens 270 / 155 (without all this) -> 247 / 142, 350
+// 294 / 165 -> 277 / 161, 600 477 / 236 -> 465 / 220; 64 of 1024 x 2048 at 300 tokens 109 / 63 -> 106 / 60.  Not taken: 32 weight rows (278 / 154 at
+// 211 tokens) or 128 (248 / 147), a third stage (equal), one wave (264 / 151), two or four column tiles as one stream (253 / 149, 300 / 168).
+template <int MODE, int MT>
+__device__ __forceinline__ void midm_expert_body(const GemmParams& p, char* smem, int grp, int m0, int mcnt, int ncol0, bool once, int reach) {
+    constexpr int RT = 4, NW = 2, NST = 2, D = 2 * (MT + RT), STAGE = D * 1024, MPW = MT / NW;
+    constexpr int HALF = 8 * RT;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g4 = lane >> 4;
+    const unsigned ring = (unsigned)(uintptr_t)(const mm_lds_void*)smem + wid * NST * STAGE;
+    char* ringp = smem + wid * NST * STAGE;
+    const int r8 = lane >> 3, pc = lane & 7;
+    const __amdgpu_buffer_rsrc_t wrs = mm_rsrc(p.w + (int64_t)grp * p.w_gstride), xrs = mm_rsrc(p.x);
+    unsigned wvo[2 * RT], xvo[2 * MT];
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) {
+        const int row = 8 * i + r8;
+        const int wr = gemm_paired(MODE) ? (row < HALF ? 0 : p.N) + min(ncol0 + (row < HALF ? row : row - HALF), p.N - 1) : min(ncol0 + row, p.N - 1);
+        wvo[i] = ((unsigned)wr * (unsigned)p.ldw + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
+    }
+    const int n = max(0, (p.K / MM_KC - wid + NW - 1) / NW);   // this wave's chunks: wid, wid + NW, ...
+    auto issue_w = [&](auto ntc, int j, int slot) {
+        const int soff = (j * NW + wid) * MM_ROWB;
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)(ringp + slot * STAGE + i * 1024), 16, wvo[i], soff, 0, decltype(ntc)::value ? 2 : 0);
+    };
+    int last = 0;
+    auto source = [&](int i) {
+        const int m = m0 + min(8 * i + r8, mcnt - 1);   // rows past the end repeat the last one; they are never stored
+        return MODE == GEMM_GATEUP && p.src ? p.src[m] : m;
+    };
+    auto issue_x = [&](auto far_rows, int j, int slot) {
+        const int soff = (j * NW + wid) * MM_ROWB;
+        char* st = ringp + slot * STAGE + 2 * RT * 1024;
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) {
+            if constexpr (decltype(far_rows)::value)
+                __builtin_amdgcn_global_load_lds((mm_glb_void*)(p.x + (int64_t)source(i) * p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8 + soff / 2),
+                                                 (mm_lds_void*)(st + i * 1024), 16, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (mm_lds_void*)(st + i * 1024), 16, xvo[i], soff, 0, 0);
+        }
+    };
+    if (n > 0) {   // (ahead of the wait for the row numbers)
+        if (once) issue_w(std::true_type{}, 0, 0);
+        else issue_w(std::false_type{}, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) {
+        const int src = source(i);
+        xvo[i] = ((unsigned)src * (unsigned)p.ldx + (pc ^ (((8 * i + r8) >> 1) & 7)) * 8) * 2u;
+        last = max(last, src);
+    }
+    float sc[MPW];   // of this wave's rows; a load inside the stream would wait behind every DMA in flight
+    const bool scaled = MODE == GEMM_DOWN && grp < p.n_scaled;
+#pragma unroll
+    for (int j = 0; j < MPW; ++j) {
+        const int row = 16 * (MPW * wid + j) + c;
+        sc[j] = scaled && row < mcnt ? bf2f(p.scale[m0 + row]) : 1.0f;
+        asm volatile("" : "+v"(sc[j]));
+    }
+    unsigned rel[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) rel[ks] = c * MM_ROWB + (((4 * ks + g4) ^ ((c >> 1) & 7)) << 4);
+    f32x4_t acc[RT][MT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto mm = [&](const MmFrags<MT, RT>& f) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f.w[rt]), __builtin_bit_cast(bf16x8_t, f.x[mt]), acc[rt][mt], 0, 0, 0);
+    };
+    auto stream = [&](auto far_rows, auto ntc) {
+        auto arrived = [&](int j) {    // stage j has, the younger ones stay in flight
+            if (j + NST <= n) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((NST - 1) * D) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        };
+#pragma unroll
+        for (int j = 0; j < NST; ++j)
+            if (j < n) {
+                if (j > 0) issue_w(ntc, j, j);
+                issue_x(far_rows, j, j);
+            }
+        MmFrags<MT, RT> f0, f1;        // the two k-steps of a stage
+        int slot = 0;
+        arrived(0);
+        f0.read(ring + rel[0]);
+        f0.settle();
+        for (int j = 0; j < n; ++j) {
+            f1.read(ring + slot * STAGE + rel[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(f0);
+            f1.settle();               // the stage is in registers: its slot takes chunk j + NST
+            if (j + NST < n) {
+                issue_w(ntc, j + NST, slot);
+                issue_x(far_rows, j + NST, slot);
+            }
+            slot = slot + 1 == NST ? 0 : slot + 1;
+            if (j + 1 < n) {
+                arrived(j + 1);
+                f0.read(ring + slot * STAGE + rel[0]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            mm(f1);
+            if (j + 1 < n) f0.settle();
+        }
+    };
+    if (n > 0) {
+        // gathered rows (of an x whose length nobody here knows) beyond what 32-bit offsets reach: the wave looks its rows up again at every stage
+        if (MODE == GEMM_GATEUP && __any(last >= reach)) {
+            if constexpr (MODE == GEMM_GATEUP) stream(std::true_type{}, std::false_type{});
+        } else if (once) stream(std::false_type{}, std::true_type{});
+        else stream(std::false_type{}, std::false_type{});
+    }
+
+    // ---- sum of the waves' tiles, in wave order: wave w finishes row tiles w MPW ..
+    __syncthreads();               // the rings are read
+    f32x4_t* red = reinterpret_cast<f32x4_t*>(smem);
+#pragma unroll
+    for (int j = 0; j < MPW; ++j)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const f32x4_t a = wid == 0 ? acc[rt][MPW + j] : acc[rt][j];
+            red[((wid * MPW + j) * RT + rt) * 64 + lane] = a;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MPW; ++j) {
+        f32x4_t sum[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const f32x4_t other = red[(((1 - wid) * MPW + j) * RT + rt) * 64 + lane];
+            sum[rt] = wid == 0 ? acc[rt][j] + other : other + acc[rt][MPW + j];
+        }
+        const int row = 16 * (MPW * wid + j) + c;
+        if (row >= mcnt) continue;
+        bf16_t* yrow = p.y + (int64_t)(m0 + row) * p.ldy + ncol0 + 4 * g4;
+        const int left = p.N - ncol0 - 4 * g4;   // N % 4 == 0 is checked on the host
+        if constexpr (gemm_paired(MODE)) {
+#pragma unroll
+            for (int h = 0; h < RT / 2; ++h) {
+                float o[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = rbf(glm_silu(rbf(sum[h][r]))) * rbf(sum[RT / 2 + h][r]);
+                if (16 * h < left) *reinterpret_cast<u32x2_t*>(yrow + 16 * h) = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+            }
+        } else {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                float o[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = scaled ? rbf(sum[rt][r]) * sc[j] : sum[rt][r];
+                if (16 * rt < left) *reinterpret_cast<u32x2_t*>(yrow + 16 * rt) = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+            }
+        }
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(128) void gemm_midm_experts_kernel(const GemmParams p, int reach) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    int* sh = reinterpret_cast<int*>(smem);
+    glm_locate_block(p.offs, p.G, p.R, 64, blockIdx.y, sh);
+    __syncthreads();
+    const int grp = __builtin_amdgcn_readfirstlane(sh[0]);
+    const int m0 = __builtin_amdgcn_readfirstlane(sh[1]);
+    const int mcnt = __builtin_amdgcn_readfirstlane(sh[2]);
+    __syncthreads();   // everyone has read sh before the first DMA lands on it
+    if (grp < 0) return;
+    const int ncol0 = blockIdx.x * (gemm_paired(MODE) ? 32 : 64);
+    const bool once = p.offs[grp + 1] - p.offs[grp] <= 64;
+    if (mcnt <= 32) midm_expert_body<MODE, 2>(p, smem, grp, m0, mcnt, ncol0, once, reach);
+    else midm_expert_body<MODE, 4>(p, smem, grp, m0, mcnt, ncol0, once, reach);
+}
+
+template <int MODE>
+int launch_midm_experts(const GemmParams& p, hipStream_t st) {
+    constexpr int LDS = 2 * 2 * (4 + 4) * 2048;   // two waves, two stages
+    const int cols = gemm_paired(MODE) ? 32 : 64;
+    const int64_t gy = p.R / 64 + p.G;
+    GLM_CHECK_ARG(gy <= 65535, GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
+    auto kern = gemm_midm_experts_kernel<MODE>;
+    const int64_t reach = (1ll << 30) / p.ldx;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((p.N + cols - 1) / cols), (unsigned)gy), dim3(128), LDS, st, p, (int)reach);
+    GLM_CHECK_LAUNCH("gemm_midm");
+    return GLM_OK;
+}
+
+#endif  // GLM_EXPERTS
 
 // rows m0 .. m0 + mcnt - 1, columns from ncol0, tile shared by the workgroup: WM x WN waves of MT x RT 16-row tiles each.  Every wave brings
 // its share of a stage (one 64-wide K chunk of all rows); the counted wait is for its own share, the barrier behind it for the others', and
@@ -427,12 +585,11 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
     const int cols = gemm_paired(MODE) ? 8 * RT : 16 * RT, nt = (p.N + cols - 1) / cols;
     const int64_t mblocks = (p.R + 16 * MT - 1) / (16 * MT);
     const bool dealt = nt >= 64;
-    const int64_t gx = p.offs ? nt : dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8, gy = p.offs ? p.R / (16 * MT) + p.G : 1;
-    GLM_CHECK_ARG(gx < (1 << 30) && gy <= 65535, GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
+    const int64_t gx = dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8;
+    GLM_CHECK_ARG(gx < (1 << 30), GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
     auto kern = gemm_midm_kernel<MODE, MT, RT, NW, NST>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
-    const int64_t reach = (1ll << 30) / p.ldx;
-    hipLaunchKernelGGL(kern, dim3((unsigned)gx, (unsigned)gy), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt, (int)reach);
+    hipLaunchKernelGGL(kern, dim3((unsigned)gx), dim3(NW * 64), LDS, st, p, (int)mblocks, (int)dealt);
     GLM_CHECK_LAUNCH("gemm_midm");
     return GLM_OK;
 }
@@ -493,11 +650,11 @@ int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
 
 template <int MODE>
 int launch_midm(const GemmParams& p, hipStream_t st) {
-    // experts: two waves, two workgroups per CU, so that one is at work while the other starts or sums up (short K, many tiles; four waves: 211
-    // tokens on 65 experts of 1408 x 4096 291 / 186 us instead of 274 / 154)
+#if GLM_EXPERTS
     if constexpr (MODE == GEMM_GATEUP || MODE == GEMM_DOWN) {
-        if (p.offs != nullptr) return launch_midm_cfg<MODE, 4, 4, 2, 2>(p, st);
+        if (p.offs != nullptr) return launch_midm_experts<MODE>(p, st);
     }
+#endif
     return launch_midm_tile<MODE>(midm_tile_of(MODE, p), p, st);
 }
 
@@ -529,15 +686,18 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     if (p.ksplit > 1 || p.wscale != nullptr || p.K % 64 != 0) return false;
     if (p.offs != nullptr) {
         // Experts with 24 to 95 rows on average: the weight-streaming kernel's blocks of 32 rows read an expert's weights once per block.  gate|up,
-        // down, us, rows dealt at random: 65 of 1408 x 4096 at 24 rows 292 / 159 there, 278 / 151 here, at 30 330 / 184 and 274 / 153, at 55
-        // 557 / 279 and 307 / 174; 64 of 1024 x 2048 at 20 108 / 57 and 106 / 60, at 24 109 / 61 and 104 / 59, at 38 168 / 82 and 109 / 62.  Rows
-        // dealt evenly up to 32 are read once there too, and with few experts it hangs on how they fall: 8 of 2048 x 4096 at 24 rows 50 / 27
-        // there, 53 / 31 here, at 25 64 / 35 and 54 / 31, at 26 51 / 28 and 54 / 31, at 27 63 / 37 and 54 / 31; 16 of 1408 x 4096 gate|up at 25 74 / 83,
-        // at 28 82 / 78; 32 of 1024 x 1024 down at 25 17 / 20, at 28 22 / 20; 128 of 512 x 1024 down at 24 39 / 41, at 32 45 / 42.
+        // down, us, rows dealt at random: 65 of 1408 x 4096 at 28 rows 330 / 184 there, 247 / 142 here, at 55 557 / 279 and 277 / 161.
+        // With fewer rows, where there are column tiles for several rounds of the chip: there every 32 weight rows move as many activation
+        // bytes.  There / here: gate|up 65 of 1408 x 4096 at 9 rows 232 / 236, at 13 240 / 236, at 18 251 / 239, at 22 264 / 241, 64 of 1024 x 2048
+        // at 11 95.9 / 97.7, at 15 99.6 / 99.0, at 20 107 / 101, 129 of 512 x 1024 at 18 63 / 57, of 768 x 2048 at 7 133 / 137; one round: 17 of
+        // 1408 x 4096 at 18 74 / 79, 65 of 352 x 4096 at 14 68 / 75.  Down 65 of 1408 x 4096 at 7 129 / 120, at 9 133 / 122, at 18 145 / 131, 129 of
+        // 768 x 2048 at 7 80 / 77, at 4 68 / 73, 17 of 1408 x 4096 at 18 44 / 40, 64 of 1024 x 2048 at 11 54.7 / 54.6; 33 of 1024 x 1024 at 15 19.6 / 21.0,
+        // 9 of 2048 x 4096 at 13 31 / 40.
         const int64_t rows = p.R_hint > 0 ? p.R_hint : p.R;
         if (mode != GEMM_GATEUP && mode != GEMM_DOWN) return false;
-        return rows >= 24 * (int64_t)p.G && rows < 96 * (int64_t)p.G && p.R * p.ldx * 2 < (1ll << 31) &&
-               (mode == GEMM_GATEUP ? 2 : 1) * (int64_t)p.N * p.ldw * 2 < (1ll << 31);
+        const int64_t G = p.G, tiles = (p.N + (mode == GEMM_GATEUP ? 31 : 63)) / (mode == GEMM_GATEUP ? 32 : 64) * G;
+        const bool enough = rows >= 24 * G || (mode == GEMM_GATEUP ? rows >= 13 * G && tiles >= 2048 : rows > 6 * G && tiles >= 1024);
+        return enough && rows < 96 * G && p.R * p.ldx * 2 < (1ll << 31) && (mode == GEMM_GATEUP ? 2 : 1) * (int64_t)p.N * p.ldw * 2 < (1ll << 31);
     }
     if (p.src != nullptr || p.G > 1 || p.R <= 32) return false;
     // (a loop of the tiled kernel that is asked for keeps its shapes)

@@ -121,6 +121,28 @@ def test_experts(ops, T, E, k, H, I, shared):
             assert_close_bf16(y[rows], (d.float() * s[rows, None].float()).to(BF) if e < E else d, 2, 0.06, atol=2 ** -8, what=f"y of expert {e}")
 
 
+@pytest.mark.parametrize("T,E,k,H,I", [(300, 128, 6, 192, 512), (250, 80, 3, 4096, 832), (260, 128, 7, 448, 544)])
+def test_many_experts_of_few_rows(ops, T, E, k, H, I):
+    """Groups of 7 to 23 rows on average with column tiles for several rounds of the chip, one of them with more than a block of 64."""
+    g = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(E - 1, generator=g)[: k] if t % 3 else torch.arange(k) for t in range(T)]).sort(-1).values
+    wt = (torch.rand(T, k, generator=g) + 0.1).to(BF)
+    offs, tok, scale, _ = ops.moe_align(idx.cuda(), wt.cuda(), E, False)
+    R, K2 = T * k, 64 * (I // 64)
+    x, w13 = rnd(T, H, seed=20), rnd(E, 2 * I, H, seed=21, scale=H ** -0.5)
+    act_in, w2 = rnd(R, K2, seed=23), rnd(E, H, K2, seed=22, scale=K2 ** -0.5)
+    act = ops.grouped_gemm_gateup_silu(x.cuda(), w13.cuda(), offs, tok, R)
+    y = ops.grouped_gemm_down(act_in.cuda(), w2.cuda(), offs, scale, E)
+    o, s = offs.cpu().tolist(), scale.cpu()
+    for e in (0, k - 1, k, E // 2, E - 2, E - 1):
+        if o[e + 1] > o[e]:
+            rows = slice(o[e], o[e + 1])
+            z = x[tok.cpu()[rows].long()].double() @ w13[e].double().T
+            assert_close_bf16(act[rows], O.silu_and_mul(z.to(BF)), *SILU, what=f"act of expert {e}")
+            d = (act_in[rows].double() @ w2[e].double().T).to(BF)
+            assert_close_bf16(y[rows], (d.float() * s[rows, None].float()).to(BF), 2, 0.06, atol=2 ** -8, what=f"y of expert {e}")
+
+
 def test_experts_of_rows_far_apart(ops):
     """Gathered rows of an x longer than 32-bit byte offsets reach (rows 2 MiB apart: past 2 GiB from row 1024, past 4 GiB from row 2048): an
     expert of near rows, one of far ones, one of both, with a partial last block of 64."""
