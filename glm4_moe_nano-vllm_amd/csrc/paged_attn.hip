@@ -22,6 +22,7 @@
 //     across kv-splits by a small second kernel when num_splits > 1.
 #include "common.h"
 #include <string.h>
+#include <type_traits>
 
 namespace {
 
@@ -124,30 +125,57 @@ struct PaFuse {
     const bf16_t* bias;    // [qkv_stride] or nullptr
 };
 
-// 8 consecutive elements of row b of the packed QKV matrix, starting at column col (a multiple of 8)
-__device__ __forceinline__ u32x4_t pa_qkv8(const PaFuse& fu, int64_t b, int64_t col) {
-    if (fu.part == nullptr) return *reinterpret_cast<const u32x4_t*>(fu.qkv + b * fu.qkv_stride + col);
-    const float* pp = fu.part + b * fu.qkv_stride + col;
-    f32x4_t lo = *reinterpret_cast<const f32x4_t*>(pp), hi = *reinterpret_cast<const f32x4_t*>(pp + 4);
-    for (int sl = 1; sl < fu.nslices; ++sl) {
-        lo += *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride);
-        hi += *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride + 4);
+// 8 consecutive elements of row b of the packed QKV matrix, starting at column col (a multiple of 8): the loads, and the bf16 values out of
+// them.  NS: 0 bf16 rows, 2 two slices of partial sums (the usual count, so that all loads go out at once), -1 any number of them.
+template <int NS>
+struct PaRow8 {
+    f32x4_t f[NS > 0 ? 2 * NS : 2];
+    u32x4_t h;
+    __device__ __forceinline__ void load(const PaFuse& fu, int64_t b, int64_t col) {
+        if constexpr (NS == 0) {
+            h = *reinterpret_cast<const u32x4_t*>(fu.qkv + b * fu.qkv_stride + col);
+        } else {
+            const float* pp = fu.part + b * fu.qkv_stride + col;
+#pragma unroll
+            for (int sl = 0; sl < (NS > 0 ? NS : 1); ++sl) {
+                f[2 * sl] = *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride);
+                f[2 * sl + 1] = *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride + 4);
+            }
+            // (no bias: any 16 bytes, unused; a branch per load made the compiler wait for the loads so far)
+            h = *reinterpret_cast<const u32x4_t*>(fu.bias != nullptr ? reinterpret_cast<const float*>(fu.bias + col) : pp);
+        }
     }
-    if (fu.bias != nullptr) {
-        const u32x4_t bv = *reinterpret_cast<const u32x4_t*>(fu.bias + col);
-        lo[0] += bflo(bv[0]); lo[1] += bfhi(bv[0]); lo[2] += bflo(bv[1]); lo[3] += bfhi(bv[1]);
-        hi[0] += bflo(bv[2]); hi[1] += bfhi(bv[2]); hi[2] += bflo(bv[3]); hi[3] += bfhi(bv[3]);
+    __device__ __forceinline__ u32x4_t value(const PaFuse& fu, int64_t b, int64_t col) {
+        if constexpr (NS == 0) return h;
+        f32x4_t lo = f[0], hi = f[1];
+        if constexpr (NS > 0) {
+#pragma unroll
+            for (int sl = 1; sl < NS; ++sl) {
+                lo += f[2 * sl];
+                hi += f[2 * sl + 1];
+            }
+        } else {
+            const float* pp = fu.part + b * fu.qkv_stride + col;
+            for (int sl = 1; sl < fu.nslices; ++sl) {
+                lo += *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride);
+                hi += *reinterpret_cast<const f32x4_t*>(pp + sl * fu.slice_stride + 4);
+            }
+        }
+        if (fu.bias != nullptr) {
+            lo[0] += bflo(h[0]); lo[1] += bfhi(h[0]); lo[2] += bflo(h[1]); lo[3] += bfhi(h[1]);
+            hi[0] += bflo(h[2]); hi[1] += bfhi(h[2]); hi[2] += bflo(h[3]); hi[3] += bfhi(h[3]);
+        }
+        return u32x4_t{pack2bf(lo[0], lo[1]), pack2bf(lo[2], lo[3]), pack2bf(hi[0], hi[1]), pack2bf(hi[2], hi[3])};
     }
-    return u32x4_t{pack2bf(lo[0], lo[1]), pack2bf(lo[2], lo[3]), pack2bf(hi[0], hi[1]), pack2bf(hi[2], hi[3])};
-}
+};
 
-// NeoX rotation of 8 packed bf16 pairs: y1 = a*cos - b*sin, y2 = b*cos + a*sin (rope8, elementwise.hip)
-__device__ __forceinline__ void pa_rope8(const u32x4_t a, const u32x4_t b, const float* cosp, const float* sinp,
+// NeoX rotation of 8 packed bf16 pairs: y1 = a*cos - b*sin, y2 = b*cos + a*sin (rope8, elementwise.hip); cs: cos and sin, 8 of each
+__device__ __forceinline__ void pa_rope8(const u32x4_t a, const u32x4_t b, const f32x4_t (&cs)[4],
                                          u32x4_t& y1, u32x4_t& y2) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float c0 = cosp[2 * j], c1 = cosp[2 * j + 1];
-        const float s0 = sinp[2 * j], s1 = sinp[2 * j + 1];
+        const float c0 = cs[j >> 1][2 * (j & 1)], c1 = cs[j >> 1][2 * (j & 1) + 1];
+        const float s0 = cs[2 + (j >> 1)][2 * (j & 1)], s1 = cs[2 + (j >> 1)][2 * (j & 1) + 1];
         const float a0 = bflo(a[j]), a1 = bfhi(a[j]);
         const float b0 = bflo(b[j]), b1 = bfhi(b[j]);
         y1[j] = pack2bf(a0 * c0 - b0 * s0, a1 * c1 - b1 * s1);
@@ -155,43 +183,89 @@ __device__ __forceinline__ void pa_rope8(const u32x4_t a, const u32x4_t b, const
     }
 }
 
+// FUSED: 0 rotated q and an up-to-date cache, 1 packed bf16 rows, 2 two slices of partial sums, 3 any number of slices
 template <int FUSED>
 __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ context_lens, const int32_t* __restrict__ block_tables,
     int64_t bt_stride, bf16_t* __restrict__ out, float* part_o,
     float* part_ml, unsigned* tickets, int nh, int nkv, int block_size, float scale_log2e,
-    int num_splits, const PaFuse fu) {
+    int num_splits, int by_length, const PaFuse fu) {
+    constexpr int NS = FUSED == 2 ? 2 : FUSED == 3 ? -1 : 0;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int split = blockIdx.x, kvh = blockIdx.y;
-    const int64_t b = blockIdx.z;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int gq = nh / nkv;  // query heads per kv head (<= 16)
-    const int len = context_lens[b];
+    char* ring = smem + wid * PA_RING;
+    int* bt_lds = reinterpret_cast<int*>(smem + PA_WAVES * PA_RING);
+    int64_t b = blockIdx.z;
+    // ---- prologue, ordered so that the K/V stream starts as early as possible ----
+    // Only the block table gates the K/V DMAs; everything else is requested in front of them and used behind: (1) length and block table, at
+    // once where a row of it is short (up to 256 entries: all of them, which lie in front of the next row's first; not the last row), raw Q chunks, position, slot, the new token's raw K/V row; (2) cos/sin of the
+    // position.  Vector-memory results come in issue order, so what is requested behind a DMA waits for it.  The new token's row never has to
+    // come back from the cache: wave 0 rotates it, leaves it in LDS (PA_NEWROW) and fires the cache store without waiting for it; the wave that
+    // reaches the last key group overwrites that row (and the clamped copies of it behind it) in its landed stage before it reads fragments.
+    // 32 sequences of 4096, two slices: first DMA after 7.0 us with a loop over the slices in front of it.
+    bool whole_table = false;
+    int bt_entry = 0;
+    auto read_table = [&]() {
+        whole_table = bt_stride <= 256 && b + 1 < gridDim.z;
+        if (whole_table && tid < bt_stride) bt_entry = block_tables[b * bt_stride + tid];
+    };
+    read_table();
+    int len;
+    if (by_length) {
+        // More workgroups than CUs: the ones of the longest sequences first, so that the last to start are the shortest (64 sequences of 6.1k
+        // to 8.2k keys, two workgroups per CU one after the other: 298 -> 286 us).  Up to 64 sequences, one per lane, each wave for itself; where the
+        // lengths are short or alike the block table is on its way already.
+        const int nb = gridDim.z, mine = lane < nb ? context_lens[lane] : -1;
+        int hi = mine, lo = lane < nb ? mine : 0x7fffffff;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            hi = max(hi, __shfl_xor(hi, o, 64));
+            lo = min(lo, __shfl_xor(lo, o, 64));
+        }
+        if (hi >= 2048 && hi - lo > hi / 16) {  // (uniform)
+            int rank = 0;
+            for (int i = 0; i < nb; ++i) {
+                const int v = __builtin_amdgcn_readlane(mine, i);
+                rank += v > mine || (v == mine && i < lane) ? 1 : 0;
+            }
+            b = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(lane < nb && rank == (int)blockIdx.z)) - 1);
+            read_table();
+        }
+        len = __builtin_amdgcn_readlane(mine, (int)b);
+    } else len = context_lens[b];
+    int64_t ps = 0;
+    if (FUSED) ps = fu.pos[b];
+
+    // raw Q^T chunks (B operand: lane (c,g), k-step ks holds Q[head c][32ks + 8g .. +8)); FUSED: out of the packed row
+    const bool hv = c < gq;
+    const int64_t qcol = ((int64_t)kvh * gq + (hv ? c : 0)) * PA_HD + 8 * g;
+    PaRow8<NS> qr[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        if (FUSED) qr[ks].load(fu, b, qcol + 32 * ks);
+        else qr[ks].h = *reinterpret_cast<const u32x4_t*>(q + b * nh * PA_HD + qcol + 32 * ks);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the loads above are in flight before anything waits
+
     const int ngroups = (len + PA_GK - 1) / PA_GK;
     const int gps = (ngroups + num_splits - 1) / num_splits;
     const int G0 = split * gps;
     const int G1 = min(ngroups, G0 + gps);
-
-    char* ring = smem + wid * PA_RING;
-    int* bt_lds = reinterpret_cast<int*>(smem + PA_WAVES * PA_RING);
-
     // block-table slice of this workgroup → LDS (so the loop has no VMEM loads besides the DMA)
     const int gpb = block_size / PA_GK;  // groups per block
-    const int blk0 = G0 < G1 ? G0 / gpb : 0;
-    const int blk1 = G0 < G1 ? (G1 - 1) / gpb + 1 : 0;
-    for (int i = tid; i < blk1 - blk0; i += 256) bt_lds[i] = block_tables[b * bt_stride + blk0 + i];
-
-    // ---- prologue, ordered so that the K/V stream starts as early as possible ----
-    // One memory round trip per line: (1) block table, raw Q chunks, position, slot, the new token's raw K/V row; (2)
-    // cos/sin of the position.  Only the block table gates the K/V DMAs.  The new token's row never has to come back from
-    // the cache: wave 0 rotates it, leaves it in LDS (PA_NEWROW) and fires the cache store without waiting for it; the
-    // wave that reaches the last key group overwrites that row (and the clamped copies of it behind it) in its landed
-    // stage before it reads fragments.  Before r02 the row was stored, acknowledged and barriered in front of the first
-    // DMA: ~4 round trips of prologue (in-graph 88.6 us at C3 against 85.8 us for the plain kernel).
+    const int blk0 = G0 < G1 && !whole_table ? G0 / gpb : 0;
+    if (whole_table) {
+        if (tid < bt_stride) bt_lds[tid] = bt_entry;
+    } else {
+        const int blk1 = G0 < G1 ? (G1 - 1) / gpb + 1 : 0;
+        for (int i = tid; i < blk1 - blk0; i += 256) bt_lds[i] = block_tables[b * bt_stride + blk0 + i];
+    }
     const int nmine = (G1 - G0 - wid + PA_WAVES - 1) / PA_WAVES;  // groups G0+wid, +4, ...
     auto issue = [&](int it) {
         const int gi = G0 + wid + it * PA_WAVES;
@@ -204,57 +278,63 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(
     const bool owner = FUSED && len > 0 && glast >= G0 && glast < G1;  // this workgroup reads the new token's key
     char* newrow = smem + PA_WAVES * PA_RING + PA_MAX_BT * 4;
 
-    // (1) raw loads: Q^T chunks (B operand: lane (c,g), k-step ks holds Q[head c][32ks + 8g .. +8)), position, new row
-    const bool hv = c < gq;
-    u32x4_t v[4];
-    {
-        const int64_t qcol = ((int64_t)kvh * gq + (hv ? c : 0)) * PA_HD;  // FUSED: column of the head in the packed row
-        const bf16_t* qrow = q + (b * nh + (int64_t)kvh * gq + (hv ? c : 0)) * PA_HD;
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            v[ks] = u32x4_t{0, 0, 0, 0};
-            if (hv) v[ks] = FUSED ? pa_qkv8(fu, b, qcol + 32 * ks + 8 * g) : *reinterpret_cast<const u32x4_t*>(qrow + 32 * ks + 8 * g);
-        }
-    }
-    int64_t ps = 0;
-    if (FUSED) ps = min(max(fu.pos[b], (int64_t)0), fu.n_pos - 1);
+    // (2) cos / sin, the new row
     const bool row_lane = owner && wid == 0 && lane < 32;  // lanes 0-15 rotate and store the K row, 16-31 copy the V row
     const int sub = lane & 15;
     const bool is_k = lane < 16;
-    u32x4_t xv = {0, 0, 0, 0}, pv = {0, 0, 0, 0};
+    const bool turns = is_k && sub < 8;
+    const int64_t rcol = ((int64_t)nh + (is_k ? 0 : nkv) + kvh) * PA_HD + sub * 8, pcol = rcol + (sub < 4 ? 32 : -32);
+    PaRow8<NS> xr, pr;
     int64_t slot = -1;
-    if (FUSED && row_lane) {
-        const int64_t rcol = ((int64_t)nh + (is_k ? 0 : nkv) + kvh) * PA_HD;
-        xv = pa_qkv8(fu, b, rcol + sub * 8);
-        if (is_k && sub < 8) pv = pa_qkv8(fu, b, rcol + (sub < 4 ? sub + 4 : sub - 4) * 8);
-        slot = fu.slots[b];
+    f32x4_t cs[4], cs_row[4];
+    if (FUSED) {
+        ps = min(max(ps, (int64_t)0), fu.n_pos - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4_t*>(fu.cos_sin + ps * 64 + 8 * g + 32 * (i >> 1) + 4 * (i & 1));
+        if (row_lane) {
+            xr.load(fu, b, rcol);
+            slot = fu.slots[b];
+            if (turns) {
+                pr.load(fu, b, pcol);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) cs_row[i] = *reinterpret_cast<const f32x4_t*>(fu.cos_sin + ps * 64 + 8 * (sub & 3) + 32 * (i >> 1) + 4 * (i & 1));
+            }
+        }
     }
-    __syncthreads();  // block table visible
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // block table visible
     if (nmine > 0) issue(0);
     if (nmine > 1) issue(1);
-    // (2) rotary (rotary_dim 64: chunk g of the first half pairs with chunk g of the second half)
+    __builtin_amdgcn_sched_barrier(0);
+    // (3) rotary (rotary_dim 64: chunk g of the first half pairs with chunk g of the second half)
     bf16x8_t qf[4];
     {
+        u32x4_t v[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            v[ks] = FUSED ? qr[ks].value(fu, b, qcol + 32 * ks) : qr[ks].h;
+            if (!hv) v[ks] = u32x4_t{0, 0, 0, 0};
+        }
         if (FUSED) {
-            const float* cosp = fu.cos_sin + ps * 64 + 8 * g;
             u32x4_t y1, y2;
-            pa_rope8(v[0], v[1], cosp, cosp + 32, y1, y2);
+            pa_rope8(v[0], v[1], cs, y1, y2);
             v[0] = y1;
             v[1] = y2;
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) qf[ks] = __builtin_bit_cast(bf16x8_t, v[ks]);
     }
-    // (3) the new token's K/V row into the cache
+    // (4) the new token's K/V row into the cache
     if (FUSED && row_lane) {
-        if (is_k && sub < 8) {
-            const float* cosp = fu.cos_sin + ps * 64 + 8 * (sub & 3);
+        u32x4_t xv = xr.value(fu, b, rcol);
+        if (turns) {
+            const u32x4_t pv = pr.value(fu, b, pcol);
             u32x4_t y1, y2;
             if (sub < 4) {
-                pa_rope8(xv, pv, cosp, cosp + 32, y1, y2);
+                pa_rope8(xv, pv, cs_row, y1, y2);
                 xv = y1;
             } else {
-                pa_rope8(pv, xv, cosp, cosp + 32, y1, y2);
+                pa_rope8(pv, xv, cs_row, y1, y2);
                 xv = y2;
             }
         }
@@ -468,32 +548,49 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(
     __syncthreads();
     if (!flag[0]) return;
     {
-        // same arithmetic and summation order as paged_attn_reduce_kernel: thread (head h, 8 dims at d0)
+        // same arithmetic and summation order as paged_attn_reduce_kernel: thread (head h, 8 dims at d0).  Every partial was stored
+        // write-through and drained before its split's ticket: sc1 loads, no acquire; those of eight splits at a time go out together (one
+        // after the other they took 4.1 us of a 13 us launch, 8 splits).
         const int h = tid >> 4, d0 = (tid & 15) * 8;
         if (h < gq) {
             const int64_t bh = b * nh + (int64_t)kvh * gq + h;
-            // every partial was stored write-through and drained before its split's ticket: sc1 loads, no acquire
+            auto max_sum = [&](int sp) {
+                return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(part_ml + (bh * num_splits + sp) * 2), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+            };
             float M = -INFINITY;
-            for (int sp = 0; sp < num_splits; ++sp) {
-                const unsigned long long ml = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(part_ml + (bh * num_splits + sp) * 2),
-                                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                M = fmaxf(M, __uint_as_float((unsigned)ml));
+            for (int sp = 0; sp < num_splits; sp += 8) {
+                unsigned long long ml[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ml[i] = max_sum(min(sp + i, num_splits - 1));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) M = fmaxf(M, __uint_as_float((unsigned)ml[i]));
             }
             float L = 0.f, o[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) o[i] = 0.f;
-            for (int sp = 0; sp < num_splits; ++sp) {
-                const unsigned long long ml = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(part_ml + (bh * num_splits + sp) * 2),
-                                                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const float m = __uint_as_float((unsigned)ml);
-                const float f = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - M);
-                L += f * __uint_as_float((unsigned)(ml >> 32));
-                const int64_t po = (bh * num_splits + sp) * PA_HD + d0;
-                const f32x4_t a = load16_sc1(part_o, po), c4 = load16_sc1(part_o, po + 4);
+            for (int sp = 0; sp < num_splits; sp += 8) {
+                unsigned long long ml[8];
+                f32x4_t a[8], a4[8];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    o[i] += f * a[i];
-                    o[4 + i] += f * c4[i];
+                for (int i = 0; i < 8; ++i) {
+                    const int s1 = min(sp + i, num_splits - 1);
+                    const int64_t po = (bh * num_splits + s1) * PA_HD + d0;
+                    ml[i] = max_sum(s1);
+                    a[i] = load16_sc1(part_o, po);
+                    a4[i] = load16_sc1(part_o, po + 4);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float m = __uint_as_float((unsigned)ml[i]);
+                    if (sp + i >= num_splits) continue;
+                    const float f = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - M);
+                    L += f * __uint_as_float((unsigned)(ml[i] >> 32));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        o[r] += f * a[i][r];
+                        o[4 + r] += f * a4[i][r];
+                    }
                 }
             }
             u32x4_t ov;
@@ -587,24 +684,25 @@ static int pa_launch(const void* q, const void* k_cache, const void* v_cache, co
         // in-kernel merge by the last-arriving split when the counters fit; else the separate reduce launch
         if ((size_t)B * nkv * sizeof(unsigned) <= PA_TICKET_BYTES) tickets = (unsigned*)workspace;
     }
-    const int fz = fuse != nullptr;
-    if (fz) GLM_SET_MAX_LDS(paged_attn_decode_kernel<1>, PA_LDS, name);
-    else GLM_SET_MAX_LDS(paged_attn_decode_kernel<0>, PA_LDS, name);
     hipStream_t st = glm_s(stream);
     const float scale_log2e = scale * 1.4426950408889634f;
     const dim3 grid((unsigned)splits, (unsigned)nkv, (unsigned)B);
+    const int by_length = splits == 1 && B * nkv > 256 && B <= 64 && (max_context_len > 0 ? max_context_len : bt_stride * block_size) >= 6144;
     PaFuse fu;
     memset(&fu, 0, sizeof(fu));
-    if (fz) {
-        fu = *fuse;
-        hipLaunchKernelGGL((paged_attn_decode_kernel<1>), grid, dim3(256), PA_LDS, st, (const bf16_t*)nullptr,
-                           (const bf16_t*)k_cache, (const bf16_t*)v_cache, context_lens, block_tables, bt_stride,
-                           (bf16_t*)out, part_o, part_ml, tickets, nh, nkv, block_size, scale_log2e, splits, fu);
-    } else {
-        hipLaunchKernelGGL((paged_attn_decode_kernel<0>), grid, dim3(256), PA_LDS, st, (const bf16_t*)q,
-                           (const bf16_t*)k_cache, (const bf16_t*)v_cache, context_lens, block_tables, bt_stride,
-                           (bf16_t*)out, part_o, part_ml, tickets, nh, nkv, block_size, scale_log2e, splits, fu);
-    }
+    if (fuse != nullptr) fu = *fuse;
+    auto run = [&](auto fusedc) -> int {
+        auto kern = paged_attn_decode_kernel<decltype(fusedc)::value>;
+        GLM_SET_MAX_LDS(kern, PA_LDS, name);
+        hipLaunchKernelGGL(kern, grid, dim3(256), PA_LDS, st, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, context_lens,
+                           block_tables, bt_stride, (bf16_t*)out, part_o, part_ml, tickets, nh, nkv, block_size, scale_log2e, splits, by_length, fu);
+        return GLM_OK;
+    };
+    const int rc = fuse == nullptr       ? run(std::integral_constant<int, 0>{})
+                   : fu.part == nullptr  ? run(std::integral_constant<int, 1>{})
+                   : fu.nslices == 2     ? run(std::integral_constant<int, 2>{})
+                                         : run(std::integral_constant<int, 3>{});
+    if (rc != GLM_OK) return rc;
     GLM_CHECK_LAUNCH(name);
     if (splits > 1 && tickets == nullptr) {
         hipLaunchKernelGGL(paged_attn_reduce_kernel, dim3((unsigned)(B * nh)), dim3(128), 0, st, part_o,

@@ -282,6 +282,24 @@ def test_qkv_projection_as_partial_sums_matches_one_pass(ops):
     assert_close_bf16(red, one, 1, 0.05, atol=2 ** -9, what="QKV partial sums vs one pass")
 
 
+@pytest.mark.parametrize("B,nh,nkv,width", [(33, 8, 8, 24), (64, 24, 8, 24), (40, 16, 16, 300), (64, 8, 8, 257), (64, 16, 8, 256)])
+def test_paged_attn_decode_longest_first(ops, B, nh, nkv, width):
+    """More workgroups than CUs and room for long contexts: sequences start by length (equal lengths, empty rows and the last table row among
+    them).  An order and nothing more: the same launch with a promise of short contexts, which keeps the order of the rows, gives the same bits."""
+    g = torch.Generator().manual_seed(B + width)
+    lens = torch.randint(1, 500, (B,), generator=g).tolist()
+    lens[3] = lens[B - 1] = 2500
+    lens[5], lens[7], lens[B - 2] = 0, 2049, 0
+    q, kc, vc, cl, bt = _paged_case(lens, nh, nkv, seed=B * 3 + nkv)
+    wide = torch.full((B, width), -1, dtype=torch.int32)
+    wide[:, : bt.shape[1]] = bt
+    scale = 128 ** -0.5
+    args = dev(q), dev(kc), dev(vc), dev(cl), dev(wide), scale
+    got = ops.paged_attn_decode(*args)
+    assert torch.equal(got, ops.paged_attn_decode(*args, max_context_len=4096))
+    assert_mixed(got, O.attn_decode_paged(q, kc, vc, cl, bt, scale), 1.6e-2, 4e-3, f"longest first B={B} nkv={nkv}")
+
+
 def test_paged_attn_decode_spiky_scores(ops):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
     q, kc, vc, cl, bt = _paged_case([777], 12, 1, seed=99)
