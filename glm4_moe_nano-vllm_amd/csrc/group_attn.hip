@@ -347,6 +347,113 @@ struct Slab {
             }
         });
     }
+    // ---- the same in units of one slab and one tile, for a caller that keeps the fragments itself (heads up to 128 + 128: VEARLY)
+    // scores of tile T: start from the distance bias where there is one
+    template <int T>
+    __device__ __forceinline__ void scores(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int j0, int g, bool biased) const {
+        auto add = [&](int kt, int i, const f32x4_t& to) {
+            s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][SPLIT ? T * KQ + i : i]), __builtin_bit_cast(bf16x8_t, qf[T][i]), to, 0, 0, 0);
+        };
+        if (F == GA_SOFTMAX && biased) {
+            const float b0 = slope[T] * (float)(j0 + 4 * g - rp[T]);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                f32x4_t bias4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bias4[r] = fmaf(slope[T], (float)(16 * kt + r), b0);
+                add(kt, 0, bias4);
+            }
+        } else {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) add(kt, 0, f32x4_t{0.f, 0.f, 0.f, 0.f});
+        }
+#pragma unroll
+        for (int i = 1; i < KQ; ++i)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) add(kt, i, s[kt]);
+    }
+    // largest of the eight scores (inline asm: hipcc would quiet every operand of a maximum first)
+    __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
+        float m;
+        asm("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\tv_max_f32 %0, %0, %8"
+            : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
+        return m;
+    }
+    // weights of tile T; fac: sigmoid form, factors of the lane's keys times scale and log2 e, negative; EDGE: some keys may be hidden
+    template <int T, bool EDGE>
+    __device__ __forceinline__ bf16x8_t weights(f32x4_t (&s)[2], int j0, int g, float sc, const u32x4_t (&fac)[2]) {
+        bf16x8_t pf;
+        if constexpr (F == GA_SIGMOID_KV) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const f32x4_t f = __builtin_bit_cast(f32x4_t, fac[kt]) * -sc;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(s[kt][r], f[r], -slope[T]);
+            }
+        }
+        if constexpr (F == GA_TWO_MAPS) {
+            float big = 0.f;
+            asm("v_max3_f32 %0, abs(%1), abs(%2), abs(%3)\n\tv_max3_f32 %0, %0, abs(%4), abs(%5)\n\tv_max3_f32 %0, %0, abs(%6), abs(%7)\n\tv_max_f32 %0, %0, abs(%8)"
+                : "=&v"(big) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
+            if (__any(!(big <= cap_lim))) {
+                cap_exact(s);
+            } else {
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float u = s[kt][r] * s[kt][r];
+                        s[kt][r] *= fmaf(fmaf(fmaf(ca3, u, ca2), u, ca1), u, ca0);
+                    }
+            }
+        }
+        if (F == GA_TWO_MAPS_ANY && cap_out > 0.f) cap_exact(s);
+        if (EDGE && (j0 < full_lo[T] || j0 + 31 > full_hi[T])) {
+            const int jl = j0 + 4 * g;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = jl + 16 * kt + r;
+                    if (j > rp[T] || j < rlo[T]) s[kt][r] = F == GA_SIGMOID_KV ? INFINITY : -INFINITY;
+                }
+        }
+        float m_use = 0.f;
+        if constexpr (F == GA_SOFTMAX || F == GA_TWO_MAPS_ANY) {
+            float mx = largest(s) * sc;
+            if (__any(mx > m_run[T] + 8.0f || (m_run[T] == -INFINITY && mx > -INFINITY))) {
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                const float m_new = fmaxf(m_run[T], mx);
+                const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[T] - m_new);
+                l_run[T] *= alpha;
+#pragma unroll
+                for (int d = 0; d < VT; ++d) acc[T][d] *= alpha;
+                m_run[T] = m_new;
+            }
+            m_use = m_run[T] == -INFINITY ? 0.f : m_run[T];
+        }
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float p;
+                if constexpr (F == GA_SIGMOID_KV) p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r]));
+                else if constexpr (F == GA_TWO_MAPS) p = __builtin_amdgcn_exp2f(s[kt][r]);
+                else p = __builtin_amdgcn_exp2f(fmaf(s[kt][r], sc, -m_use));
+                if constexpr (F != GA_SIGMOID_KV) l_run[T] += p;
+                pf[4 * kt + r] = (__bf16)p;
+            }
+        return pf;
+    }
+    template <int T>
+    __device__ __forceinline__ void values(const bf16x8_t pf, const u32x2_t (&vf)[VT][2]) {
+#pragma unroll
+        for (int d = 0; d < VT; ++d) {
+            const u32x4_t vv = {vf[d][0][0], vf[d][0][1], vf[d][1][0], vf[d][1][1]};
+            acc[T][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf, acc[T][d], 0, 0, 0);
+        }
+    }
     __device__ __forceinline__ void set_cap(const GroupArgs& a) {
         if constexpr (!ga_two(F)) return;
         cap_in = a.cap > 0.f ? 2.f * GA_LOG2E * a.scale / a.cap : 0.f;
@@ -429,40 +536,58 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
 #pragma unroll
         for (int i = 0; i < KQ; ++i) asm volatile("" : "+v"(S.qf[t][i]));
     const unsigned base = lds_addr(smem);
-    // per-lane source offsets of the DMA pieces: constant over the tiles
-    unsigned koff[KDMA], voff[VDMA + 1];
-    int krow[KDMA], vrow[VDMA + 1];
-    bool kpad[KDMA], vpad[VDMA + 1];
+    // Sources of the DMA pieces: piece i of a wave holds 64 / CPR rows from row0 + i 64 / CPR on, and the chunk permutation repeats after eight
+    // rows: offsets of the pieces of eight rows and whole strides between them.  Tiles whose rows are all there, without padding
+    // columns, take them as they are; the others choose per lane between a row and zeros.
+    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KPER = KRP < 8 ? 8 / KRP : 1, VPER = VRP < 8 ? 8 / VRP : 1;
+    unsigned koff[KPER], voff[VPER];
+    auto k_piece = [&](int i, int& row, int& ch) {
+        row = (w * KDMA + i) * KRP + lane / KCPR;
+        ch = (lane % KCPR) ^ attn_swz(row);
+    };
+    auto v_piece = [&](int i, int& row, int& ch) {
+        row = (w * VDMA + i) * VRP + lane / VCPR;
+        ch = (lane % VCPR) ^ attn_swz(row);
+    };
 #pragma unroll
-    for (int i = 0; i < KDMA; ++i) {
-        const int q = (w * KDMA + i) * 64 + lane, row = q / KCPR, ch = (q % KCPR) ^ attn_swz(row);
-        krow[i] = row;
-        kpad[i] = (ch % MAPC) * 8 >= dm;
-        koff[i] = (unsigned)(row * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8);
+    for (int i = 0; i < KPER; ++i) {
+        int row, ch;
+        k_piece(i, row, ch);
+        koff[i] = (unsigned)(row * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2u;
     }
 #pragma unroll
-    for (int i = 0; i < VDMA; ++i) {
-        const int q = (w * VDMA + i) * 64 + lane, row = q / VCPR, ch = (q % VCPR) ^ attn_swz(row);
-        vrow[i] = row;
-        vpad[i] = ch * 8 >= a.dv;
-        voff[i] = (unsigned)(row * a.dv + ch * 8);
+    for (int i = 0; i < VPER; ++i) {
+        int row, ch;
+        v_piece(i, row, ch);
+        voff[i] = (unsigned)(row * a.dv + ch * 8) * 2u;
     }
+    const bool padded = dm != MAPC * 8 || (!KV && a.dv != DV);
     // tiles from the last keys to the first: under a distance bias the maximum is found early and stays
     auto issue = [&](int it, int blk) {
         const int j0 = jlo + (n - 1 - it) * 64, left = ga_ok(a, blk) ? plast - j0 + 1 : 0;
         const int64_t row = ga_row(a, blk, j0, kvh);
-        const bf16_t* kb = reinterpret_cast<const bf16_t*>(a.kc) + row * a.dk;
-        const bf16_t* vb = reinterpret_cast<const bf16_t*>(a.vc) + row * a.dv;
+        const char* kb = reinterpret_cast<const char*>(a.kc) + row * a.dk * 2;
+        const char* vb = reinterpret_cast<const char*>(a.vc) + row * a.dv * 2;
         char* st = smem + (it & 1) * STAGE;
+        if (left >= 64 && !padded) {
 #pragma unroll
-        for (int i = 0; i < KDMA; ++i) {
-            const void* s = (kpad[i] || krow[i] >= left) ? (const void*)ga_zero_page : (const void*)(kb + koff[i]);
-            lds_dma16(s, st + (w * KDMA + i) * 1024);
-        }
+            for (int i = 0; i < KDMA; ++i) lds_dma16(kb + (i / KPER) * (KPER * KRP * 2) * a.dk + koff[i % KPER], st + (w * KDMA + i) * 1024);
 #pragma unroll
-        for (int i = 0; i < VDMA; ++i) {
-            const void* s = (vpad[i] || vrow[i] >= left) ? (const void*)ga_zero_page : (const void*)(vb + voff[i]);
-            lds_dma16(s, st + KTILE + (w * VDMA + i) * 1024);
+            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (i / VPER) * (VPER * VRP * 2) * a.dv + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < KDMA; ++i) {
+                int r, ch;
+                k_piece(i, r, ch);
+                const bool none = (ch % MAPC) * 8 >= dm || r >= left;
+                lds_dma16(none ? (const void*)ga_zero_page : (const void*)(kb + (int64_t)(r * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2), st + (w * KDMA + i) * 1024);
+            }
+#pragma unroll
+            for (int i = 0; i < VDMA; ++i) {
+                int r, ch;
+                v_piece(i, r, ch);
+                lds_dma16(ch * 8 >= a.dv || r >= left ? (const void*)ga_zero_page : (const void*)(vb + (int64_t)(r * a.dv + ch * 8) * 2), st + KTILE + (w * VDMA + i) * 1024);
+            }
         }
         if constexpr (KV) {
             if (w == 0) lds_dma4(a.kscale + (int64_t)(ga_ok(a, blk) ? blk : 0) * a.bs + (j0 - ga_block(a, j0) * a.bs) + lane, st + KTILE);
@@ -470,18 +595,151 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
     };
     const float sc = TWO && a.cap > 0.f ? 1.f : a.scale * GA_LOG2E;  // (capped scores are in log2 units)
     auto block_of = [&](int it) { return bt[ga_block(a, jlo + max(n - 1 - it, 0) * 64)]; };  // 64-key tiles lie in one block
-    int blk = block_of(1);
-    issue(0, ga_uniform(block_of(0)));
-    for (int it = 0; it < n; ++it) {
-        wait_vm<0>();
-        __builtin_amdgcn_s_barrier();
-        if (it + 1 < n) {
-            issue(it + 1, ga_uniform(blk));
-            blk = block_of(it + 2);
-        }
-        const unsigned kst = base + (it & 1) * STAGE, vst = kst + (KV ? 0 : KTILE);
+    if constexpr (SL::VEARLY) {
+        // ---- units (slab, tile): the scores of the next unit are started in front of the weights of this one, and the fragments they need are
+        // requested a unit ahead, so that neither LDS nor the matrix pipe's latency stands between a unit's parts.  Per tile of 64 keys (slabs 1, 0):
+        //   (1, t0)  scores (1, t1); V of slab 1, K of slab 0 requested; weights, values
+        //   (1, t1)  scores (0, t0); weights, values
+        //   (0, t0)  scores (0, t1); V of slab 0 requested; weights; the next tile has arrived, the one after it is requested into this
+        //            tile's buffer, whose last fragments are in (barrier), K of the next tile's slab 1 requested; values
+        //   (0, t1)  scores of the next tile's (1, t0); weights, values
+        // 15074 tokens of 4 prompts, 16 heads of 128 + 128, slabs one after the other / units, us: softmax 348 / 316, two maps of 64 under a cap
+        // 617 / 584, sigmoid weights 323 / 314.  What is left: LDS reads (every wave reads all keys and values for 32 rows, 2300 of some 5000 clocks a
+        // tile with the staging), exponentials and products beside one another, some 8 us of start and end per workgroup.
+        constexpr int KS = SL::KS, FR = KV ? 2 : 0;
+        u32x4_t kf[2][KS], fac[2][2];   // K fragments; factors of the keys of slab 1 and 0 (sigmoid)
+        u32x2_t vf[VT][2];
+        f32x4_t sa[2], sb[2];
+        const bool biased = F == GA_SOFTMAX && a.slope != nullptr;
+        auto read_k = [&](unsigned st, auto slabc) {
+            constexpr int sl = decltype(slabc)::value;
+            const unsigned kst = st + sl * 32 * KB;
+            static_for<KS>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                lds_read_b128<(i >> 1) * 128>(kf[0][i], kst + S.k_rel[i & 1]);
+                lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i], kst + S.k_rel[i & 1]);
+            });
+            if constexpr (KV) {
+                const unsigned fst = st + KTILE + sl * 128 + 16 * g;
+                lds_read_b128<0>(fac[1 - sl][0], fst);
+                lds_read_b128<64>(fac[1 - sl][1], fst);
+            }
+        };
+        auto read_v = [&](unsigned st, auto slabc) {
+            const unsigned vst = st + (KV ? 0 : KTILE) + decltype(slabc)::value * 32 * VB;
+            static_for<VT>([&](auto I) {
+                constexpr int d = decltype(I)::value;
+                lds_read_tr16_b64<(d >> 2) * 128>(vf[d][0], vst + S.v_rel[d & 3]);
+                lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[d][1], vst + S.v_rel[d & 3]);
+            });
+        };
+        // the registers pass through: no use moves above the wait
+        auto k_here = [&]() {
+            wait_lds();
 #pragma unroll
-        for (int s = 1; s >= 0; --s) S.run(kst + s * 32 * KB, vst + s * 32 * VB, jlo + (n - 1 - it) * 64 + s * 32, g, sc, kst + KTILE + s * 128);
+            for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
+            if constexpr (KV) asm volatile("" : "+v"(fac[0][0]), "+v"(fac[0][1]), "+v"(fac[1][0]), "+v"(fac[1][1]));
+        };
+        auto v_here = [&]() {
+#pragma unroll
+            for (int d = 0; d < VT; ++d) asm volatile("" : "+v"(vf[d][0]), "+v"(vf[d][1]));
+        };
+        auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        auto seen = [&](int j, int t) { return j <= S.any_hi[t] && j + 31 >= S.any_lo[t]; };   // by some row of the tile
+        int blk = ga_uniform(block_of(0));
+        const int blk1 = ga_uniform(block_of(1));
+        issue(0, blk);
+        if (n > 1) {
+            issue(1, blk1);
+            wait_vm<KDMA + VDMA>();   // (the wave that brings factors waits for one piece more)
+        } else {
+            wait_vm<0>();
+        }
+        blk = block_of(2);
+        __builtin_amdgcn_s_barrier();
+        read_k(base, I1{});
+        if constexpr (KV) asm volatile("" : "=v"(fac[1][0]), "=v"(fac[1][1]));
+        k_here();
+        S.template scores<0>(sa, kf, jlo + (n - 1) * 64 + 32, g, biased);
+        auto tile = [&](auto edgec, int it) {
+            constexpr bool EDGE = decltype(edgec)::value;
+            const unsigned st = base + (it & 1) * STAGE;
+            const int j0 = jlo + (n - 1 - it) * 64, j1 = j0 + 32;
+            const bool more = it + 1 < n;
+            // (1, t0)
+            S.template scores<1>(sb, kf, j1, g, biased);
+            fence();
+            read_v(st, I1{});
+            read_k(st, I0{});
+            const bool s10 = !EDGE || seen(j1, 0), s11 = !EDGE || seen(j1, 1), s00 = !EDGE || seen(j0, 0), s01 = !EDGE || seen(j0, 1);
+            bf16x8_t pf;
+            if (s10) pf = S.template weights<0, EDGE>(sa, j1, g, sc, fac[0]);
+            asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * KS + FR) : "memory");  // (the K fragments may still be on their way)
+            v_here();
+            if (s10) S.template values<0>(pf, vf);
+            fence();
+            // (1, t1)
+            k_here();
+            S.template scores<0>(sa, kf, j0, g, biased);
+            fence();
+            if (s11) {
+                pf = S.template weights<1, EDGE>(sb, j1, g, sc, fac[0]);
+                S.template values<1>(pf, vf);
+            }
+            fence();
+            // (0, t0)
+            S.template scores<1>(sb, kf, j0, g, biased);
+            fence();
+            read_v(st, I0{});
+            if (s00) pf = S.template weights<0, EDGE>(sa, j0, g, sc, fac[1]);
+            wait_lds();
+            v_here();
+            if (more) {
+                wait_vm<0>();
+                __builtin_amdgcn_s_barrier();
+                if (it + 2 < n) {
+                    issue(it + 2, ga_uniform(blk));
+                    blk = block_of(it + 3);
+                }
+            }
+            // (behind the last tile: whatever the other buffer holds, for scores that nobody uses; a branch would part the reads from their wait)
+            read_k(base + ((it + 1) & 1) * STAGE, I1{});
+            if (s00) S.template values<0>(pf, vf);
+            fence();
+            // (0, t1)
+            k_here();
+            S.template scores<0>(sa, kf, j0 - 32, g, biased);
+            fence();
+            if (s01) {
+                pf = S.template weights<1, EDGE>(sb, j0, g, sc, fac[1]);
+                S.template values<1>(pf, vf);
+            }
+            fence();
+        };
+        // tiles of which every row sees every key, and the others
+        const int in_lo = max(S.full_lo[0], S.full_lo[1]), in_hi = min(S.full_hi[0], S.full_hi[1]);
+        auto inside = [&](int it) { const int j0 = jlo + (n - 1 - it) * 64; return j0 >= in_lo && j0 + 63 <= in_hi; };
+        int it = 0;
+        while (it < n) {
+            while (it < n && inside(it)) tile(std::false_type{}, it++);
+            while (it < n && !inside(it)) tile(std::true_type{}, it++);
+        }
+    } else {
+        int blk = block_of(1);
+        issue(0, ga_uniform(block_of(0)));
+        for (int it = 0; it < n; ++it) {
+            wait_vm<0>();
+            __builtin_amdgcn_s_barrier();
+            if (it + 1 < n) {
+                issue(it + 1, ga_uniform(blk));
+                blk = block_of(it + 2);
+            }
+            const unsigned kst = base + (it & 1) * STAGE, vst = kst + (KV ? 0 : KTILE);
+    #pragma unroll
+            for (int s = 1; s >= 0; --s) S.run(kst + s * 32 * KB, vst + s * 32 * VB, jlo + (n - 1 - it) * 64 + s * 32, g, sc, kst + KTILE + s * 128);
+        }
     }
     if constexpr (TWO) {
         // both maps of a row are in the same lane: their difference and its norm over the head's columns (padding columns are zeros)
