@@ -26,10 +26,10 @@
 // a score exceeds it by more than 2^8 (the sums stay exact: the reference point cancels).
 #include "common.h"
 #include "attn_lds.h"
+#include "attn_units.h"
 
 namespace {
 
-constexpr float GA_LOG2E = 1.4426950408889634f;
 __device__ const u32x4_t ga_zero_page[4] = {};
 
 struct GroupArgs {
@@ -85,12 +85,6 @@ __device__ __forceinline__ f32x4_t ga_gate(const GroupArgs& a, int64_t row, int 
     const u32x2_t u = *reinterpret_cast<const u32x2_t*>(g + (int64_t)h * a.dv + d);
     return f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
 }
-// forms of the tiled kernels
-// (GA_TWO_MAPS: the scores have a soft cap that 2^score fits under as it is; GA_TWO_MAPS_ANY: any cap, or none)
-enum : int { GA_SOFTMAX = 0, GA_TWO_MAPS = 1, GA_SIGMOID_KV = 2, GA_TWO_MAPS_ANY = 3 };
-constexpr float GA_CAP_FITS = 55.f;  // cap log2(e) <= 80: the sums of 2^score stay far inside fp32 whatever their number
-__host__ __device__ constexpr bool ga_two(int form) { return form == GA_TWO_MAPS || form == GA_TWO_MAPS_ANY; }
-
 // ---------------------------------------------------------------------------------------------------------------------------
 struct StoreArgs {
     const char* src;      // row r at r*ld bytes; keys at k_off, values at v_off (bytes)
@@ -115,367 +109,6 @@ __global__ __launch_bounds__(256) void group_kv_store_kernel(const StoreArgs a) 
     char* dst = val ? a.vc : a.kc;
     *reinterpret_cast<u32x4_t*>(dst + (((slot / a.bs * a.G + g) * a.bs + slot % a.bs) * w + c) * 16) = x;
 }
-
-// ---------------------------------------------------------------------------------------------------------------------------
-// the two products of a 32-key slab and the softmax between them, for NT tiles of 16 query rows (lane c holds row c of each)
-// (two maps: of two tiles, tile t holds map t's rows of the queries and meets the keys' half t; in one tile a row's queries are
-// zeros in the other map's half)
-template <int DK, int DV, int NT, int F>
-struct Slab {
-    static constexpr bool SPLIT = ga_two(F) && NT == 2;
-    static constexpr int KS = DK / 32, KQ = SPLIT ? KS / 2 : KS, VT = DV / 16, KB = DK * 2, VB = DV * 2;
-    static constexpr bool VEARLY = DK + DV <= 256;                    // V fragments requested in front of the score products
-    static constexpr int KG = KS < 4 ? KS : 4, VG = VEARLY ? VT : 4;  // fragments per request group
-    u32x4_t qf[NT][KQ];
-    f32x4_t acc[NT][VT];
-    float m_run[NT], l_run[NT], slope[NT];                // slope: per key, in units of the unscaled score; sigmoid: the bias in log2 units
-    float cap_in, cap_out;                                // soft cap: exponent per unit of score, cap in log2 units (0: none)
-    float cap_lim, ca0, ca1, ca2, ca3;                    // scores up to cap_lim: odd polynomial
-    int rp[NT], rlo[NT];                                  // position of the lane's row and the first one it sees; rp < 0: no row
-    int any_lo[NT], any_hi[NT], full_lo[NT], full_hi[NT]; // keys that some row / every row of the tile sees
-    unsigned k_rel[2], v_rel[4];
-
-    __device__ __forceinline__ void init(int lane) {
-        const int c = lane & 15, g = lane >> 4;
-        // K row c, chunk 4 i + g (its low three bits depend on the parity of i only); V row 4 g + qq
-#pragma unroll
-        for (int e = 0; e < 2; ++e) k_rel[e] = c * KB + (((4 * e + g) ^ attn_swz(c)) << 4);
-        const int qq = (lane >> 2) & 3, pp = lane & 3, vr = 4 * g + qq;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v_rel[e] = vr * VB + (((2 * e + (pp >> 1)) ^ attn_swz(vr)) << 4) + ((pp & 1) << 3);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            m_run[t] = -INFINITY;
-            l_run[t] = 0.f;
-#pragma unroll
-            for (int d = 0; d < VT; ++d) acc[t][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    // cap tanh(s / cap) in log2 units, by tanh y = 1 - 2 / (1 + e^(2 y))
-    __device__ __forceinline__ void cap_exact(f32x4_t (&s)[2]) const {
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(-2.f * cap_out, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r] * cap_in)), cap_out);
-    }
-    // all tiles: up to a fifth of the cap tanh is its odd polynomial of degree 7 (the next term is below 2e-8 of the cap)
-    __device__ __forceinline__ void cap_scores(f32x4_t (&s)[NT][2]) const {
-        float big = 0.f;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) big = fmaxf(big, fabsf(s[t][kt][r]));
-        if (__any(big > cap_lim)) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) cap_exact(s[t]);
-            return;
-        }
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float u = s[t][kt][r] * s[t][kt][r];
-                    s[t][kt][r] *= fmaf(fmaf(fmaf(ca3, u, ca2), u, ca1), u, ca0);
-                }
-    }
-    // kst, vst: LDS addresses of the slab's first key row and value row; j0: position of its first key
-    // kst, vst, fst: ... and of the keys' factors (sigmoid form)
-    __device__ __forceinline__ void run(unsigned kst, unsigned vst, int j0, int g, float sc, unsigned fst) {
-        bool live[NT], some = false;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            live[t] = j0 <= any_hi[t] && j0 + 31 >= any_lo[t];
-            some = some || live[t];
-        }
-        if (!some) return;
-        u32x2_t vf[VG][2];
-        auto read_v = [&](auto D0) {
-            static_for<VG>([&](auto I) {
-                constexpr int i = decltype(I)::value, d = decltype(D0)::value + i;
-                lds_read_tr16_b64<(d >> 2) * 128>(vf[i][0], vst + v_rel[d & 3]);
-                lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[i][1], vst + v_rel[d & 3]);
-            });
-        };
-        f32x4_t s[NT][2];  // starts from the distance bias: the products are added to it
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const float b0 = F == GA_SOFTMAX ? slope[t] * (float)(j0 + 4 * g - rp[t]) : 0.f;
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) s[t][kt][r] = F == GA_SOFTMAX ? fmaf(slope[t], (float)(16 * kt + r), b0) : 0.f;
-        }
-        u32x4_t ks[2];
-        if constexpr (F == GA_SIGMOID_KV) {  // (in front of the K fragments: in when they are)
-            lds_read_b128<0>(ks[0], fst + 16 * g);
-            lds_read_b128<64>(ks[1], fst + 16 * g);
-        }
-        static_for<(KS + KG - 1) / KG>([&](auto GI) {
-            constexpr int k0 = decltype(GI)::value * KG, kn = KS - k0 < KG ? KS - k0 : KG;
-            constexpr bool last = k0 + KG >= KS;
-            u32x4_t kf[2][KG];
-            static_for<kn>([&](auto I) {
-                constexpr int i = k0 + decltype(I)::value;
-                lds_read_b128<(i >> 1) * 128>(kf[0][i - k0], kst + k_rel[i & 1]);
-                lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i - k0], kst + k_rel[i & 1]);
-            });
-            if constexpr (last && VEARLY) {
-                read_v(std::integral_constant<int, 0>{});
-                // the K fragments are in; the V fragments (issued last) may still be on their way
-                asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * VG <= 15 ? 2 * VG : 15) : "memory");
-            } else {
-                wait_lds();
-            }
-#pragma unroll
-            for (int i = 0; i < kn; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
-#pragma unroll
-            for (int i = 0; i < kn; ++i)
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        if (SPLIT && (k0 + i) / KQ != t) continue;
-                        s[t][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][i]), __builtin_bit_cast(bf16x8_t, qf[t][(k0 + i) % KQ]), s[t][kt], 0, 0, 0);
-                    }
-        });
-        if constexpr (F == GA_SIGMOID_KV) asm volatile("" : "+v"(ks[0]), "+v"(ks[1]));
-        bf16x8_t pf[NT];
-        if constexpr (F == GA_TWO_MAPS || F == GA_SIGMOID_KV) {  // no maximum: all tiles go through every step together
-            if constexpr (F == GA_TWO_MAPS) cap_scores(s);
-            if constexpr (F == GA_SIGMOID_KV) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-#pragma unroll
-                    for (int kt = 0; kt < 2; ++kt) {
-                        const f32x4_t f = __builtin_bit_cast(f32x4_t, ks[kt]);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) s[t][kt][r] = fmaf(s[t][kt][r] * sc, f[r], slope[t]);
-                    }
-            }
-            bool edge = false;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) edge = edge || j0 < full_lo[t] || j0 + 31 > full_hi[t];
-            if (edge) {
-                const int jl = j0 + 4 * g;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            const int j = jl + 16 * kt + r, row = F == GA_TWO_MAPS ? 0 : t;  // (two maps: the same tokens)
-                            if (j > rp[row] || j < rlo[row]) s[t][kt][r] = -INFINITY;
-                        }
-            }
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float p;
-                        if constexpr (F == GA_SIGMOID_KV) {
-                            p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-s[t][kt][r]));
-                        } else {
-                            p = __builtin_amdgcn_exp2f(s[t][kt][r]);
-                            l_run[t] += p;
-                        }
-                        pf[t][4 * kt + r] = (__bf16)p;
-                    }
-        } else {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                if (!live[t]) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)0.f;
-                    continue;
-                }
-                if (F == GA_TWO_MAPS_ANY && cap_out > 0.f) cap_exact(s[t]);
-                if (j0 < full_lo[t] || j0 + 31 > full_hi[t]) {
-                    const int jl = j0 + 4 * g;
-#pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int j = jl + 16 * kt + r;
-                            if (j > rp[t] || j < rlo[t]) s[t][kt][r] = -INFINITY;
-                        }
-                }
-                float mx = -INFINITY;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[t][kt][r]);
-                mx *= sc;
-                if (__any(mx > m_run[t] + 8.0f || (m_run[t] == -INFINITY && mx > -INFINITY))) {
-                    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                    const float m_new = fmaxf(m_run[t], mx);
-                    const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[t] - m_new);
-                    l_run[t] *= alpha;
-#pragma unroll
-                    for (int d = 0; d < VT; ++d) acc[t][d] *= alpha;
-                    m_run[t] = m_new;
-                }
-                const float m_use = m_run[t] == -INFINITY ? 0.f : m_run[t];
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float p = __builtin_amdgcn_exp2f(fmaf(s[t][kt][r], sc, -m_use));
-                        l_run[t] += p;
-                        pf[t][4 * kt + r] = (__bf16)p;
-                    }
-            }
-        }
-        static_for<VT / VG>([&](auto GI) {
-            constexpr int d0 = decltype(GI)::value * VG;
-            if constexpr (!VEARLY) read_v(std::integral_constant<int, d0>{});
-            wait_lds();
-#pragma unroll
-            for (int i = 0; i < VG; ++i) asm volatile("" : "+v"(vf[i][0]), "+v"(vf[i][1]));
-#pragma unroll
-            for (int i = 0; i < VG; ++i) {
-                const u32x4_t vv = {vf[i][0][0], vf[i][0][1], vf[i][1][0], vf[i][1][1]};
-#pragma unroll
-                for (int t = 0; t < NT; ++t)
-                    acc[t][d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf[t], acc[t][d0 + i], 0, 0, 0);
-            }
-        });
-    }
-    // ---- the same in units of one slab and one tile, for a caller that keeps the fragments itself (heads up to 128 + 128: VEARLY)
-    // scores of tile T: start from the distance bias where there is one
-    template <int T>
-    __device__ __forceinline__ void scores(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int j0, int g, bool biased) const {
-        auto add = [&](int kt, int i, const f32x4_t& to) {
-            s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][SPLIT ? T * KQ + i : i]), __builtin_bit_cast(bf16x8_t, qf[T][i]), to, 0, 0, 0);
-        };
-        if (F == GA_SOFTMAX && biased) {
-            const float b0 = slope[T] * (float)(j0 + 4 * g - rp[T]);
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                f32x4_t bias4;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) bias4[r] = fmaf(slope[T], (float)(16 * kt + r), b0);
-                add(kt, 0, bias4);
-            }
-        } else {
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) add(kt, 0, f32x4_t{0.f, 0.f, 0.f, 0.f});
-        }
-#pragma unroll
-        for (int i = 1; i < KQ; ++i)
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) add(kt, i, s[kt]);
-    }
-    // largest of the eight scores (inline asm: hipcc would quiet every operand of a maximum first)
-    __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
-        float m;
-        asm("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\tv_max_f32 %0, %0, %8"
-            : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
-        return m;
-    }
-    // weights of tile T; fac: sigmoid form, factors of the lane's keys times scale and log2 e, negative; EDGE: some keys may be hidden
-    template <int T, bool EDGE>
-    __device__ __forceinline__ bf16x8_t weights(f32x4_t (&s)[2], int j0, int g, float sc, const u32x4_t (&fac)[2]) {
-        bf16x8_t pf;
-        if constexpr (F == GA_SIGMOID_KV) {
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                const f32x4_t f = __builtin_bit_cast(f32x4_t, fac[kt]) * -sc;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(s[kt][r], f[r], -slope[T]);
-            }
-        }
-        if constexpr (F == GA_TWO_MAPS) {
-            float big = 0.f;
-            asm("v_max3_f32 %0, abs(%1), abs(%2), abs(%3)\n\tv_max3_f32 %0, %0, abs(%4), abs(%5)\n\tv_max3_f32 %0, %0, abs(%6), abs(%7)\n\tv_max_f32 %0, %0, abs(%8)"
-                : "=&v"(big) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
-            if (__any(!(big <= cap_lim))) {
-                cap_exact(s);
-            } else {
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float u = s[kt][r] * s[kt][r];
-                        s[kt][r] *= fmaf(fmaf(fmaf(ca3, u, ca2), u, ca1), u, ca0);
-                    }
-            }
-        }
-        if (F == GA_TWO_MAPS_ANY && cap_out > 0.f) cap_exact(s);
-        if (EDGE && (j0 < full_lo[T] || j0 + 31 > full_hi[T])) {
-            const int jl = j0 + 4 * g;
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int j = jl + 16 * kt + r;
-                    if (j > rp[T] || j < rlo[T]) s[kt][r] = F == GA_SIGMOID_KV ? INFINITY : -INFINITY;
-                }
-        }
-        float m_use = 0.f;
-        if constexpr (F == GA_SOFTMAX || F == GA_TWO_MAPS_ANY) {
-            float mx = largest(s) * sc;
-            if (__any(mx > m_run[T] + 8.0f || (m_run[T] == -INFINITY && mx > -INFINITY))) {
-                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                const float m_new = fmaxf(m_run[T], mx);
-                const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[T] - m_new);
-                l_run[T] *= alpha;
-#pragma unroll
-                for (int d = 0; d < VT; ++d) acc[T][d] *= alpha;
-                m_run[T] = m_new;
-            }
-            m_use = m_run[T] == -INFINITY ? 0.f : m_run[T];
-        }
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float p;
-                if constexpr (F == GA_SIGMOID_KV) p = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r]));
-                else if constexpr (F == GA_TWO_MAPS) p = __builtin_amdgcn_exp2f(s[kt][r]);
-                else p = __builtin_amdgcn_exp2f(fmaf(s[kt][r], sc, -m_use));
-                if constexpr (F != GA_SIGMOID_KV) l_run[T] += p;
-                pf[4 * kt + r] = (__bf16)p;
-            }
-        return pf;
-    }
-    template <int T>
-    __device__ __forceinline__ void values(const bf16x8_t pf, const u32x2_t (&vf)[VT][2]) {
-#pragma unroll
-        for (int d = 0; d < VT; ++d) {
-            const u32x4_t vv = {vf[d][0][0], vf[d][0][1], vf[d][1][0], vf[d][1][1]};
-            acc[T][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf, acc[T][d], 0, 0, 0);
-        }
-    }
-    __device__ __forceinline__ void set_cap(const GroupArgs& a) {
-        if constexpr (!ga_two(F)) return;
-        cap_in = a.cap > 0.f ? 2.f * GA_LOG2E * a.scale / a.cap : 0.f;
-        cap_out = a.cap * GA_LOG2E;
-        const float k = a.cap > 0.f ? a.scale / a.cap : 0.f, kk = k * k;
-        cap_lim = k > 0.f ? 0.2f / k : 0.f;
-        ca0 = cap_out * k;
-        ca1 = ca0 * kk * (-1.f / 3.f);
-        ca2 = ca0 * kk * kk * (2.f / 15.f);
-        ca3 = ca0 * kk * kk * kk * (-17.f / 315.f);
-        if constexpr (F == GA_TWO_MAPS) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) m_run[t] = 0.f;
-        }
-    }
-    __device__ __forceinline__ float mass(int t) const {
-        float l = l_run[t];
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
-        return l;
-    }
-};
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // DK, DV: multiples of 64
@@ -506,7 +139,7 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
     const int dm = TWO ? a.dk / 2 : a.dk;
     SL S;
     S.init(lane);
-    S.set_cap(a);
+    S.set_cap(a.cap, a.scale);
     // this wave's rows: tile t holds rows qo + 64 t + 16 w + c of the head (the two half-dead tiles of the causal edge cost all waves the
     // same) or, of a pair, rows qo + 16 w + c of its head t, or of its map t
     const int trow = a.pair ? 0 : 64;
@@ -541,24 +174,24 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
     // columns, take them as they are; the others choose per lane between a row and zeros.
     constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KPER = KRP < 8 ? 8 / KRP : 1, VPER = VRP < 8 ? 8 / VRP : 1;
     unsigned koff[KPER], voff[VPER];
-    auto k_piece = [&](int i, int& row, int& ch) {
+    auto k_piece = [&](int lane, int i, int& row, int& ch) {
         row = (w * KDMA + i) * KRP + lane / KCPR;
         ch = (lane % KCPR) ^ attn_swz(row);
     };
-    auto v_piece = [&](int i, int& row, int& ch) {
+    auto v_piece = [&](int lane, int i, int& row, int& ch) {
         row = (w * VDMA + i) * VRP + lane / VCPR;
         ch = (lane % VCPR) ^ attn_swz(row);
     };
 #pragma unroll
     for (int i = 0; i < KPER; ++i) {
         int row, ch;
-        k_piece(i, row, ch);
+        k_piece(lane, i, row, ch);
         koff[i] = (unsigned)(row * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2u;
     }
 #pragma unroll
     for (int i = 0; i < VPER; ++i) {
         int row, ch;
-        v_piece(i, row, ch);
+        v_piece(lane, i, row, ch);
         voff[i] = (unsigned)(row * a.dv + ch * 8) * 2u;
     }
     const bool padded = dm != MAPC * 8 || (!KV && a.dv != DV);
@@ -575,17 +208,19 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
 #pragma unroll
             for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (i / VPER) * (VPER * VRP * 2) * a.dv + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
         } else {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // (worked out here and now: kept over the tiles, these offsets cost the loop its registers)
 #pragma unroll
             for (int i = 0; i < KDMA; ++i) {
                 int r, ch;
-                k_piece(i, r, ch);
+                k_piece(ln, i, r, ch);
                 const bool none = (ch % MAPC) * 8 >= dm || r >= left;
                 lds_dma16(none ? (const void*)ga_zero_page : (const void*)(kb + (int64_t)(r * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2), st + (w * KDMA + i) * 1024);
             }
 #pragma unroll
             for (int i = 0; i < VDMA; ++i) {
                 int r, ch;
-                v_piece(i, r, ch);
+                v_piece(ln, i, r, ch);
                 lds_dma16(ch * 8 >= a.dv || r >= left ? (const void*)ga_zero_page : (const void*)(vb + (int64_t)(r * a.dv + ch * 8) * 2), st + KTILE + (w * VDMA + i) * 1024);
             }
         }
@@ -595,152 +230,16 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
     };
     const float sc = TWO && a.cap > 0.f ? 1.f : a.scale * GA_LOG2E;  // (capped scores are in log2 units)
     auto block_of = [&](int it) { return bt[ga_block(a, jlo + max(n - 1 - it, 0) * 64)]; };  // 64-key tiles lie in one block
-    if constexpr (SL::VEARLY) {
-        // ---- units (slab, tile): the scores of the next unit are started in front of the weights of this one, and the fragments they need are
-        // requested a unit ahead, so that neither LDS nor the matrix pipe's latency stands between a unit's parts.  Per tile of 64 keys (slabs 1, 0):
-        //   (1, t0)  scores (1, t1); V of slab 1, K of slab 0 requested; weights, values
-        //   (1, t1)  scores (0, t0); weights, values
-        //   (0, t0)  scores (0, t1); V of slab 0 requested; weights; the next tile has arrived, the one after it is requested into this
-        //            tile's buffer, whose last fragments are in (barrier), K of the next tile's slab 1 requested; values
-        //   (0, t1)  scores of the next tile's (1, t0); weights, values
-        // 15074 tokens of 4 prompts, 16 heads of 128 + 128, slabs one after the other / units, us: softmax 348 / 316, two maps of 64 under a cap
-        // 617 / 584, sigmoid weights 323 / 314.  What is left: LDS reads (every wave reads all keys and values for 32 rows, 2300 of some 5000 clocks a
-        // tile with the staging), exponentials and products beside one another, some 8 us of start and end per workgroup.
-        constexpr int KS = SL::KS, FR = KV ? 2 : 0;
-        u32x4_t kf[2][KS], fac[2][2];   // K fragments; factors of the keys of slab 1 and 0 (sigmoid)
-        u32x2_t vf[VT][2];
-        f32x4_t sa[2], sb[2];
-        const bool biased = F == GA_SOFTMAX && a.slope != nullptr;
-        auto read_k = [&](unsigned st, auto slabc) {
-            constexpr int sl = decltype(slabc)::value;
-            const unsigned kst = st + sl * 32 * KB;
-            static_for<KS>([&](auto I) {
-                constexpr int i = decltype(I)::value;
-                lds_read_b128<(i >> 1) * 128>(kf[0][i], kst + S.k_rel[i & 1]);
-                lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i], kst + S.k_rel[i & 1]);
-            });
-            if constexpr (KV) {
-                const unsigned fst = st + KTILE + sl * 128 + 16 * g;
-                lds_read_b128<0>(fac[1 - sl][0], fst);
-                lds_read_b128<64>(fac[1 - sl][1], fst);
-            }
-        };
-        auto read_v = [&](unsigned st, auto slabc) {
-            const unsigned vst = st + (KV ? 0 : KTILE) + decltype(slabc)::value * 32 * VB;
-            static_for<VT>([&](auto I) {
-                constexpr int d = decltype(I)::value;
-                lds_read_tr16_b64<(d >> 2) * 128>(vf[d][0], vst + S.v_rel[d & 3]);
-                lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[d][1], vst + S.v_rel[d & 3]);
-            });
-        };
-        // the registers pass through: no use moves above the wait
-        auto k_here = [&]() {
-            wait_lds();
-#pragma unroll
-            for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
-            if constexpr (KV) asm volatile("" : "+v"(fac[0][0]), "+v"(fac[0][1]), "+v"(fac[1][0]), "+v"(fac[1][1]));
-        };
-        auto v_here = [&]() {
-#pragma unroll
-            for (int d = 0; d < VT; ++d) asm volatile("" : "+v"(vf[d][0]), "+v"(vf[d][1]));
-        };
-        auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        auto seen = [&](int j, int t) { return j <= S.any_hi[t] && j + 31 >= S.any_lo[t]; };   // by some row of the tile
-        int blk = ga_uniform(block_of(0));
-        const int blk1 = ga_uniform(block_of(1));
-        issue(0, blk);
-        if (n > 1) {
-            issue(1, blk1);
-            wait_vm<KDMA + VDMA>();   // (the wave that brings factors waits for one piece more)
-        } else {
-            wait_vm<0>();
-        }
-        blk = block_of(2);
-        __builtin_amdgcn_s_barrier();
-        read_k(base, I1{});
-        if constexpr (KV) asm volatile("" : "=v"(fac[1][0]), "=v"(fac[1][1]));
-        k_here();
-        S.template scores<0>(sa, kf, jlo + (n - 1) * 64 + 32, g, biased);
-        auto tile = [&](auto edgec, int it) {
-            constexpr bool EDGE = decltype(edgec)::value;
-            const unsigned st = base + (it & 1) * STAGE;
-            const int j0 = jlo + (n - 1 - it) * 64, j1 = j0 + 32;
-            const bool more = it + 1 < n;
-            // (1, t0)
-            S.template scores<1>(sb, kf, j1, g, biased);
-            fence();
-            read_v(st, I1{});
-            read_k(st, I0{});
-            const bool s10 = !EDGE || seen(j1, 0), s11 = !EDGE || seen(j1, 1), s00 = !EDGE || seen(j0, 0), s01 = !EDGE || seen(j0, 1);
-            bf16x8_t pf;
-            if (s10) pf = S.template weights<0, EDGE>(sa, j1, g, sc, fac[0]);
-            asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * KS + FR) : "memory");  // (the K fragments may still be on their way)
-            v_here();
-            if (s10) S.template values<0>(pf, vf);
-            fence();
-            // (1, t1)
-            k_here();
-            S.template scores<0>(sa, kf, j0, g, biased);
-            fence();
-            if (s11) {
-                pf = S.template weights<1, EDGE>(sb, j1, g, sc, fac[0]);
-                S.template values<1>(pf, vf);
-            }
-            fence();
-            // (0, t0)
-            S.template scores<1>(sb, kf, j0, g, biased);
-            fence();
-            read_v(st, I0{});
-            if (s00) pf = S.template weights<0, EDGE>(sa, j0, g, sc, fac[1]);
-            wait_lds();
-            v_here();
-            if (more) {
-                wait_vm<0>();
-                __builtin_amdgcn_s_barrier();
-                if (it + 2 < n) {
-                    issue(it + 2, ga_uniform(blk));
-                    blk = block_of(it + 3);
-                }
-            }
-            // (behind the last tile: whatever the other buffer holds, for scores that nobody uses; a branch would part the reads from their wait)
-            read_k(base + ((it + 1) & 1) * STAGE, I1{});
-            if (s00) S.template values<0>(pf, vf);
-            fence();
-            // (0, t1)
-            k_here();
-            S.template scores<0>(sa, kf, j0 - 32, g, biased);
-            fence();
-            if (s01) {
-                pf = S.template weights<1, EDGE>(sb, j0, g, sc, fac[1]);
-                S.template values<1>(pf, vf);
-            }
-            fence();
-        };
-        // tiles of which every row sees every key, and the others
-        const int in_lo = max(S.full_lo[0], S.full_lo[1]), in_hi = min(S.full_hi[0], S.full_hi[1]);
-        auto inside = [&](int it) { const int j0 = jlo + (n - 1 - it) * 64; return j0 >= in_lo && j0 + 63 <= in_hi; };
-        int it = 0;
-        while (it < n) {
-            while (it < n && inside(it)) tile(std::false_type{}, it++);
-            while (it < n && !inside(it)) tile(std::true_type{}, it++);
-        }
-    } else {
-        int blk = block_of(1);
-        issue(0, ga_uniform(block_of(0)));
-        for (int it = 0; it < n; ++it) {
-            wait_vm<0>();
-            __builtin_amdgcn_s_barrier();
-            if (it + 1 < n) {
-                issue(it + 1, ga_uniform(blk));
-                blk = block_of(it + 2);
-            }
-            const unsigned kst = base + (it & 1) * STAGE, vst = kst + (KV ? 0 : KTILE);
-    #pragma unroll
-            for (int s = 1; s >= 0; --s) S.run(kst + s * 32 * KB, vst + s * 32 * VB, jlo + (n - 1 - it) * 64 + s * 32, g, sc, kst + KTILE + s * 128);
-        }
-    }
+    // (the blocks of the first two tiles are looked up in front of their DMA, the others behind the DMA of the tile before, for which the walk waits
+    // before it asks again)
+    const int blk0 = ga_uniform(block_of(0)), blk1 = ga_uniform(block_of(1));
+    int blk = -1;
+    attn_tiles<DK, DV, F, KDMA + VDMA>(S, base, n, jlo, g, sc, F == GA_SOFTMAX && a.slope != nullptr, [&](int it, auto startc) {
+        if constexpr (decltype(startc)::value == 0) issue(0, blk0);
+        else if constexpr (decltype(startc)::value == 1) issue(1, blk1);
+        else issue(it, ga_uniform(blk));
+        if constexpr (decltype(startc)::value != 0) blk = block_of(it + 1);
+    });
     if constexpr (TWO) {
         // both maps of a row are in the same lane: their difference and its norm over the head's columns (padding columns are zeros)
         const float i0 = 1.0f / S.mass(0), i1 = a.lam / S.mass(1);
@@ -822,7 +321,7 @@ __global__ __launch_bounds__(NW * 64, 1) void group_attn_decode_kernel(const Gro
     const int dm = TWO ? a.dk / 2 : a.dk;
     SL S;
     S.init(lane);
-    S.set_cap(a);
+    S.set_cap(a.cap, a.scale);
     S.rp[0] = row_ok && pA >= 0 ? pA + tok : -1;
     S.rlo[0] = S.rp[0] >= 0 ? ga_first(a, S.rp[0]) : 0;
     if constexpr (KV) S.slope[0] = a.bias && row_ok ? a.bias[h] * GA_LOG2E : 0.f;
@@ -921,7 +420,7 @@ __global__ __launch_bounds__(NW * 64, 1) void group_attn_decode_kernel(const Gro
             wait_vm<0>();
         }
         const unsigned kst = base + (k & 1) * STAGE;
-        S.run(kst, kst + (KV ? 0 : KSLAB), key0(k), g, sc, kst + KSLAB);
+        S.run(kst, kst + (KV ? 0 : KSLAB), key0(k), g, sc, kst + KSLAB, F == GA_SOFTMAX && a.slope != nullptr);
     }
     // ---- the waves' sums through LDS (over the stages: every wave is past its last read) ----
     const float l = S.mass(0);

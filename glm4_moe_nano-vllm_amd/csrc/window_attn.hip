@@ -4,16 +4,14 @@
 //
 // Roofline: MFMA.  A workgroup owns 128 query rows of one (sequence, head); each of its 4 waves two 16-row query tiles, so
 // that every K / V fragment read from LDS feeds two tiles.  64-key tiles are staged by LDS-DMA, double-buffered, one barrier per
-// tile, only over the keys the rows can see: [first row - window + 1, last row].  S^T = K . Q^T, fp32 online softmax per lane
-// column in log2 units, O^T += V^T . P^T straight from registers.  Tiles that all rows of a wave see in full take a path
-// without masks; the running maximum is raised only when a score exceeds it by more than 2^8 (the sums stay exact:
-// the reference point cancels).  The sink joins the denominator once, at the end.
+// tile, only over the keys the rows can see: [first row - window + 1, last row], and walked as in attn_units.h.  The sink joins the
+// denominator once, at the end.
 #include "common.h"
 #include "attn_lds.h"
+#include "attn_units.h"
 
 namespace {
 
-constexpr float WA_LOG2E = 1.4426950408889634f;
 __device__ const u32x4_t wa_zero_page[4] = {};
 
 struct WinArgs {
@@ -40,10 +38,8 @@ struct WinArgs {
 // DK, DV: multiples of 64
 template <int DK, int DV>
 __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_kernel(const WinArgs a) {
-    constexpr int KS = DK / 32, VT = DV / 16;
-    constexpr bool VEARLY = DK + DV <= 256;                      // V fragments requested in front of the score products
-    constexpr int KG = KS < 4 ? KS : 4, VG = VEARLY ? VT : 4;    // fragments per request group
-    constexpr int KB = DK * 2, VB = DV * 2, KTILE = 64 * KB, VTILE = 64 * VB, STAGE = KTILE + VTILE;
+    using SL = Slab<DK, DV, 2, GA_SOFTMAX>;
+    constexpr int KS = SL::KS, VT = SL::VT, KTILE = 64 * SL::KB, STAGE = KTILE + 64 * SL::VB;
     constexpr int KCPR = DK / 8, VCPR = DV / 8, KDMA = DK / 32, VDMA = DV / 32;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -63,24 +59,31 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
     const int jlo = max(0, hist + qo - a.window + 1), jhi = hist + qlast;
     const int n = (jhi - jlo + 64) >> 6;
     // this wave's rows: tile t holds rows qo + 64 t + 16 w + c (the two half-dead tiles of the causal edge cost all waves the same)
-    int rq[2];   // key index of the row itself; -1: no row
-    u32x4_t qf[2][KS];
+    SL S;
+    S.init(lane);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int r = qo + 64 * t + 16 * w + c;
-        rq[t] = r < nq ? hist + r : -1;
+        const int r0 = qo + 64 * t + 16 * w, r = r0 + c;
+        const bool some = r0 < nq;
+        const int a0 = hist + r0, a1 = hist + min(r0 + 15, nq - 1);
+        S.rp[t] = r < nq ? hist + r : -1;      // key index of the row itself
+        S.rlo[t] = S.rp[t] - a.window + 1;
+        S.any_lo[t] = some ? a0 - a.window + 1 : 1 << 30;
+        S.any_hi[t] = some ? a1 : -1;
+        S.full_lo[t] = some ? a1 - a.window + 1 : 1 << 30;
+        S.full_hi[t] = some ? a0 : -1;
         const bf16_t* qp = a.q + (int64_t)(qs + min(r, nq - 1)) * a.ldq + (int64_t)h * a.dk;
 #pragma unroll
         for (int i = 0; i < KS; ++i) {
             const int k = 32 * i + 8 * g;
-            qf[t][i] = u32x4_t{0, 0, 0, 0};
-            if (k < a.dk) qf[t][i] = *reinterpret_cast<const u32x4_t*>(qp + k);
+            S.qf[t][i] = u32x4_t{0, 0, 0, 0};
+            if (k < a.dk) S.qf[t][i] = *reinterpret_cast<const u32x4_t*>(qp + k);
             if (k >= a.dkn && k < a.dk) {  // rotated here: a lane holds whole pairs
                 const float* cs = a.cs + (int64_t)(qs + min(r, nq - 1)) * (a.dk - a.dkn) + (k - a.dkn);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float u = bflo(qf[t][i][j]), v = bfhi(qf[t][i][j]), co = cs[2 * j], si = cs[2 * j + 1];
-                    qf[t][i][j] = pack2bf(u * co - v * si, v * co + u * si);
+                    const float u = bflo(S.qf[t][i][j]), v = bfhi(S.qf[t][i][j]), co = cs[2 * j], si = cs[2 * j + 1];
+                    S.qf[t][i][j] = pack2bf(u * co - v * si, v * co + u * si);
                 }
             }
         }
@@ -88,195 +91,84 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[t][i]));
+        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(S.qf[t][i]));
     const unsigned base = lds_addr(smem);
     const bf16_t* kbase = a.k + (int64_t)(ks0 + jlo) * a.ldkv + (int64_t)h * a.dkn;
     const bf16_t* rbase = a.kr ? a.kr + (int64_t)(ks0 + jlo) * a.ldr : kbase;
     const bf16_t* vbase = a.v + (int64_t)(ks0 + jlo) * a.ldkv + (int64_t)h * a.dv;
     const int nkeys = jhi - jlo + 1;
-    // per-lane source offsets of the DMA pieces: constant over the tiles
-    unsigned koff[KDMA], voff[VDMA];
-    int krow[KDMA], vrow_[VDMA];
-    bool kpad[KDMA], krot[KDMA], vpad[VDMA];
+    // Sources of the DMA pieces: as in group_attn.hip, with the last dk - dkn key columns from rows of their own.  Which pieces of a tile's keys a lane
+    // takes from there repeats with the chunk permutation.
+    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KEVEN = 64 % KCPR == 0, KPER = KEVEN ? (KRP < 8 ? 8 / KRP : 1) : KDMA, VEVEN = 64 % VCPR == 0, VPER = VEVEN ? (VRP < 8 ? 8 / VRP : 1) : VDMA;
+    auto k_piece = [&](int lane, int i, int& row, int& ch) {
+        const int q = (w * KDMA + i) * 64 + lane;
+        row = q / KCPR;
+        ch = (q % KCPR) ^ attn_swz(row);
+    };
+    auto v_piece = [&](int lane, int i, int& row, int& ch) {
+        const int q = (w * VDMA + i) * 64 + lane;
+        row = q / VCPR;
+        ch = (q % VCPR) ^ attn_swz(row);
+    };
+    unsigned koff[KPER], voff[VPER];   // bytes
+    unsigned krot = 0;                 // bit i: piece i of a period is of the other rows
 #pragma unroll
-    for (int i = 0; i < KDMA; ++i) {
-        const int q = (w * KDMA + i) * 64 + lane, row = q / KCPR, ch = (q % KCPR) ^ attn_swz(row);
-        krow[i] = row;
-        kpad[i] = ch * 8 >= a.dk;
-        krot[i] = ch * 8 >= a.dkn;
-        koff[i] = (unsigned)(krot[i] ? row * (int)a.ldr + ch * 8 - a.dkn : row * (int)a.ldkv + ch * 8);
+    for (int i = 0; i < KPER; ++i) {
+        int row, ch;
+        k_piece(lane, i, row, ch);
+        const bool rot = ch * 8 >= a.dkn;
+        krot |= rot ? 1u << i : 0u;
+        koff[i] = (unsigned)(rot ? row * (int)a.ldr + ch * 8 - a.dkn : row * (int)a.ldkv + ch * 8) * 2u;
     }
 #pragma unroll
-    for (int i = 0; i < VDMA; ++i) {
-        const int q = (w * VDMA + i) * 64 + lane, row = q / VCPR, ch = (q % VCPR) ^ attn_swz(row);
-        vrow_[i] = row;
-        vpad[i] = ch * 8 >= a.dv;
-        voff[i] = (unsigned)(row * (int)a.ldkv + ch * 8);
+    for (int i = 0; i < VPER; ++i) {
+        int row, ch;
+        v_piece(lane, i, row, ch);
+        voff[i] = (unsigned)(row * (int)a.ldkv + ch * 8) * 2u;
     }
-    auto issue = [&](int it) {
-        const int64_t adv = (int64_t)it * 64 * a.ldkv, advr = (int64_t)it * 64 * a.ldr;
-        const int left = nkeys - it * 64;
+    const bool padded = a.dk != DK || a.dv != DV, rotated = a.dkn != a.dk;
+    auto issue = [&](int it, auto) {
+        const int first = (n - 1 - it) * 64, left = nkeys - first;
+        const char* kb = reinterpret_cast<const char*>(kbase + (int64_t)first * a.ldkv);
+        const char* rb = reinterpret_cast<const char*>(rbase + (int64_t)first * a.ldr);
+        const char* vb = reinterpret_cast<const char*>(vbase + (int64_t)first * a.ldkv);
         char* st = smem + (it & 1) * STAGE;
+        if (left >= 64 && !padded) {
 #pragma unroll
-        for (int i = 0; i < KDMA; ++i) {
-            const void* s = (kpad[i] || krow[i] >= left) ? (const void*)wa_zero_page : (const void*)((krot[i] ? rbase + advr : kbase + adv) + koff[i]);
-            lds_dma16(s, st + (w * KDMA + i) * 1024);
-        }
+            for (int i = 0; i < KDMA; ++i) {
+                const int64_t kstep = (int64_t)(i / KPER) * (KPER * KRP) * a.ldkv * 2, rstep = (int64_t)(i / KPER) * (KPER * KRP) * a.ldr * 2;
+                const char* s = kb + kstep + koff[i % KPER];
+                if (rotated) s = krot >> (i % KPER) & 1 ? rb + rstep + koff[i % KPER] : s;
+                lds_dma16(s, st + (w * KDMA + i) * 1024);
+            }
 #pragma unroll
-        for (int i = 0; i < VDMA; ++i) {
-            const void* s = (vpad[i] || vrow_[i] >= left) ? (const void*)wa_zero_page : (const void*)(vbase + adv + voff[i]);
-            lds_dma16(s, st + KTILE + (w * VDMA + i) * 1024);
+            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (int64_t)(i / VPER) * (VPER * VRP) * a.ldkv * 2 + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
+        } else {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // (worked out here and now: kept over the tiles, these offsets cost the loop its registers)
+#pragma unroll
+            for (int i = 0; i < KDMA; ++i) {
+                int r, ch;
+                k_piece(ln, i, r, ch);
+                const char* s = ch * 8 >= a.dkn ? rb + ((int64_t)r * a.ldr + ch * 8 - a.dkn) * 2 : kb + ((int64_t)r * a.ldkv + ch * 8) * 2;
+                lds_dma16(ch * 8 >= a.dk || r >= left ? (const void*)wa_zero_page : (const void*)s, st + (w * KDMA + i) * 1024);
+            }
+#pragma unroll
+            for (int i = 0; i < VDMA; ++i) {
+                int r, ch;
+                v_piece(ln, i, r, ch);
+                lds_dma16(ch * 8 >= a.dv || r >= left ? (const void*)wa_zero_page : (const void*)(vb + ((int64_t)r * a.ldkv + ch * 8) * 2), st + KTILE + (w * VDMA + i) * 1024);
+            }
         }
     };
-    f32x4_t acc[2][VT];
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int d = 0; d < VT; ++d) acc[t][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // fragment offsets: K row 16 kt + c, chunk 4 i + g (its low three bits depend on the parity of i only); V row 4 g + qq
-    unsigned k_rel[2], v_rel[4];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) k_rel[e] = c * KB + (((4 * e + g) ^ attn_swz(c)) << 4);
-    const int qq = (lane >> 2) & 3, pp = lane & 3, vr = 4 * g + qq;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v_rel[e] = vr * VB + (((2 * e + (pp >> 1)) ^ attn_swz(vr)) << 4) + ((pp & 1) << 3);
-    const float sc = a.scale * WA_LOG2E;
-    // key range every row of the wave's tile t sees in full / at all
-    int full_lo[2], full_hi[2], any_lo[2], any_hi[2];
+    attn_tiles<DK, DV, GA_SOFTMAX, KDMA + VDMA>(S, base, n, jlo, g, a.scale * GA_LOG2E, false, issue);
+    const float sk = a.sink[h] * GA_LOG2E;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int r0 = qo + 64 * t + 16 * w;
-        const bool some = r0 < nq;
-        const int a0 = hist + r0, a1 = hist + min(r0 + 15, nq - 1);
-        any_lo[t] = some ? a0 - a.window + 1 : 1 << 30;
-        any_hi[t] = some ? a1 : -1;
-        full_lo[t] = some ? a1 - a.window + 1 : 1 << 30;
-        full_hi[t] = some ? a0 : -1;
-    }
-    issue(0);
-    for (int it = 0; it < n; ++it) {
-        wait_vm<0>();
-        __builtin_amdgcn_s_barrier();
-        if (it + 1 < n) issue(it + 1);
-        const unsigned kst = base + (it & 1) * STAGE, vst = kst + KTILE;
-#pragma unroll
-        for (int sl = 0; sl < 2; ++sl) {  // 32-key slabs
-            const int j0 = jlo + it * 64 + sl * 32;
-            const bool live0 = j0 <= any_hi[0] && j0 + 31 >= any_lo[0], live1 = j0 <= any_hi[1] && j0 + 31 >= any_lo[1];
-            if (!live0 && !live1) continue;
-            u32x2_t vf[VG][2];
-            auto read_v = [&](auto D0) {
-                static_for<VG>([&](auto I) {
-                    constexpr int i = decltype(I)::value, d = decltype(D0)::value + i;
-                    lds_read_tr16_b64<(d >> 2) * 128>(vf[i][0], vst + sl * 32 * VB + v_rel[d & 3]);
-                    lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[i][1], vst + sl * 32 * VB + v_rel[d & 3]);
-                });
-            };
-            f32x4_t s[2][2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt) s[t][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            static_for<(KS + KG - 1) / KG>([&](auto G) {
-                constexpr int k0 = decltype(G)::value * KG, kn = KS - k0 < KG ? KS - k0 : KG;
-                constexpr bool last = k0 + KG >= KS;
-                u32x4_t kf[2][KG];
-                static_for<kn>([&](auto I) {
-                    constexpr int i = k0 + decltype(I)::value;
-                    lds_read_b128<(i >> 1) * 128>(kf[0][i - k0], kst + sl * 32 * KB + k_rel[i & 1]);
-                    lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i - k0], kst + sl * 32 * KB + k_rel[i & 1]);
-                });
-                if constexpr (last && VEARLY) {
-                    read_v(std::integral_constant<int, 0>{});
-                    // the K fragments are in; the V fragments (issued last) may still be on their way
-                    asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * VG <= 15 ? 2 * VG : 15) : "memory");
-                } else {
-                    wait_lds();
-                }
-#pragma unroll
-                for (int i = 0; i < kn; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
-#pragma unroll
-                for (int i = 0; i < kn; ++i)
-#pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int t = 0; t < 2; ++t)
-                            s[t][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][i]), __builtin_bit_cast(bf16x8_t, qf[t][k0 + i]), s[t][kt], 0, 0, 0);
-            });
-            bf16x8_t pf[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                if (!(t == 0 ? live0 : live1)) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)0.f;
-                    continue;
-                }
-                float mx = -INFINITY;
-                if (j0 >= full_lo[t] && j0 + 31 <= full_hi[t]) {
-#pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            s[t][kt][r] *= sc;
-                            mx = fmaxf(mx, s[t][kt][r]);
-                        }
-                } else {
-                    const int d0 = rq[t] - (j0 + 4 * g);
-#pragma unroll
-                    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int d = d0 - 16 * kt - r;
-                            s[t][kt][r] = (rq[t] >= 0 && d >= 0 && d < a.window) ? s[t][kt][r] * sc : -INFINITY;
-                            mx = fmaxf(mx, s[t][kt][r]);
-                        }
-                }
-                if (__any(mx > m_run[t] + 8.0f || (m_run[t] == -INFINITY && mx > -INFINITY))) {
-                    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                    const float m_new = fmaxf(m_run[t], mx);
-                    const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[t] - m_new);
-                    l_run[t] *= alpha;
-#pragma unroll
-                    for (int d = 0; d < VT; ++d) acc[t][d] *= alpha;
-                    m_run[t] = m_new;
-                }
-                const float m_use = m_run[t] == -INFINITY ? 0.f : m_run[t];
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float p = __builtin_amdgcn_exp2f(s[t][kt][r] - m_use);
-                        l_run[t] += p;
-                        pf[t][4 * kt + r] = (__bf16)p;
-                    }
-            }
-            static_for<VT / VG>([&](auto G) {
-                constexpr int d0 = decltype(G)::value * VG;
-                if constexpr (!VEARLY) read_v(std::integral_constant<int, d0>{});
-                wait_lds();
-#pragma unroll
-                for (int i = 0; i < VG; ++i) asm volatile("" : "+v"(vf[i][0]), "+v"(vf[i][1]));
-#pragma unroll
-                for (int i = 0; i < VG; ++i) {
-                    const u32x4_t vv = {vf[i][0][0], vf[i][0][1], vf[i][1][0], vf[i][1][1]};
-#pragma unroll
-                    for (int t = 0; t < 2; ++t)
-                        acc[t][d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf[t], acc[t][d0 + i], 0, 0, 0);
-                }
-            });
-        }
-    }
-    const float sk = a.sink[h] * WA_LOG2E;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        float l = l_run[t];
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+        const float l = S.mass(t);
         const int r = qo + 64 * t + 16 * w + c;
         if (r >= nq) continue;
-        const float M = fmaxf(m_run[t], sk), f = __builtin_amdgcn_exp2f(m_run[t] - M);
+        const float M = fmaxf(S.m_run[t], sk), f = __builtin_amdgcn_exp2f(S.m_run[t] - M);
         const float inv = f / (l * f + __builtin_amdgcn_exp2f(sk - M));
         bf16_t* o = a.out + (int64_t)(qs + r) * a.ldo + (int64_t)h * a.dv;
 #pragma unroll
@@ -284,9 +176,9 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
             const int dim = 16 * d + 4 * g;
             if (a.gate && dim < a.dv) {
                 const u32x2_t gt = *reinterpret_cast<const u32x2_t*>(a.gate + (int64_t)(qs + r) * a.ldg + (int64_t)h * a.dv + dim);
-                acc[t][d] *= f32x4_t{bflo(gt[0]), bfhi(gt[0]), bflo(gt[1]), bfhi(gt[1])};
+                S.acc[t][d] *= f32x4_t{bflo(gt[0]), bfhi(gt[0]), bflo(gt[1]), bfhi(gt[1])};
             }
-            if (dim < a.dv) *reinterpret_cast<u32x2_t*>(o + dim) = u32x2_t{pack2bf(acc[t][d][0] * inv, acc[t][d][1] * inv), pack2bf(acc[t][d][2] * inv, acc[t][d][3] * inv)};
+            if (dim < a.dv) *reinterpret_cast<u32x2_t*>(o + dim) = u32x2_t{pack2bf(S.acc[t][d][0] * inv, S.acc[t][d][1] * inv), pack2bf(S.acc[t][d][2] * inv, S.acc[t][d][3] * inv)};
         }
     }
 }
