@@ -8,7 +8,7 @@
 //
 //   latent_prepare   one launch: latent norm + cache store of the step's tokens, and q' = W_uk^T q of the absorbed rows
 //   latent_attn      split-KV flash loop over the pages; rows are (token, head) pairs; fp32 scores and softmax
-//   latent_up        out = W_uv ctx, times an output gate if there is one
+//   latent_up        out = W_uv ctx, times an output gate if there is one; latent_up_merge: ctx from the splits
 //
 // With a rotated key part that all heads share (rotp columns behind the latent's rp in a cache row), queries that go through a latent of
 // their own and positions, latent_prepare is two launches: latent_rows (both latents' norms, the rotated key, cache store) in front of
@@ -557,6 +557,286 @@ __global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs
     }
 }
 
+// Up to 32 query rows and more than a few keys: the waves divide the keys, 16 at a time, and nothing passes between them before the end.  A wave
+// has its own ring of NST stages of 16 keys (counted vmcnt, no barrier), forms the scores of all rows over the whole latent, keeps the weights in
+// the registers they come out in (a 16 x 16 result is the operand of the K = 16 product) and adds up all value columns; the waves' sums meet in
+// LDS.  latent_attn_kernel's tile is a chain of two barriers, weights through LDS and fragment reads that its next tile's bytes wait for; here
+// what bounds a long range is HBM (5.5 TB/s where 200 of 256 CUs have work), a short one the loads in front of the first key and the ends.
+// Together with the launch behind it, us, there / here: 128 sequences of 1024 keys, 16 heads over 256 columns, two splits 28.0 / 24.3; 100 of
+// 2250 to 3000 keys, 16 heads over 576, 512 of them values, two splits 75.4 / 66.6, one split 118 / 86, 33 of these 39.2 / 39.4; two 64-key tiles
+// per split, 8 sequences, 25.2 / 27.5.
+template <int NCT, int VCT, int MT>
+struct LkCfg {
+    static constexpr int STAGEB = 16 * NCT * 128;
+    static constexpr int NST = 144 * 1024 / (4 * STAGEB) < 4 ? 144 * 1024 / (4 * STAGEB) : 4;
+    static constexpr int WAVEB = NST * STAGEB, LDS = 4 * WAVEB + 4 * MT * 128;
+    static_assert(NST >= 2 && VCT * 4096 <= WAVEB && LDS <= 160 * 1024, "two stages, and a wave's sums of 16 rows in their place");
+};
+
+template <int NCT, int VCT, int MT>
+__global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
+    using C = LkCfg<NCT, VCT, MT>;
+    constexpr int RPAD = NCT * 64, ROWB = RPAD * 2, CPR = RPAD / 8, KS = 2 * NCT, P = 2 * NCT, ND = 4 * VCT, NST = C::NST;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    int id = blockIdx.x;
+    const int split = id % a.nsplit;
+    id /= a.nsplit;
+    const int hg = id % a.n_hg, tile = id / a.n_hg;
+    const int h0 = hg * a.hb, hb = min(a.hb, a.H - h0);
+    // (decoding, tile i is row i: its position and sequence are requested beside the tile, and again where it is another row)
+    const int guess = (int)min((int64_t)tile, a.Ta - 1);
+    const int tok0 = a.tile_tok[tile];
+    const int ntok = min(a.tile_n[tile], a.tq);
+    int p0 = a.pos[guess], seq = a.seq_of[guess];
+    if (tok0 < 0 || tok0 >= a.Ta || ntok <= 0) return;
+    if (tok0 != guess) {
+        p0 = a.pos[tok0];
+        seq = a.seq_of[tok0];
+    }
+    const int p1 = p0 + ntok - 1;
+    const int nrows = ntok * hb;
+    const int first = max(0, p0 - a.window + 1), lo = first & ~63;
+    const int ntile = p0 < 0 ? 0 : (p1 - lo + 64) >> 6;  // 64-key tiles of the whole range
+    const int per = (ntile + a.nsplit - 1) / a.nsplit;
+    const int t0 = split * per, t1 = min(t0 + per, ntile), n = t1 - t0;
+    if (n <= 0) {  // an empty split (or an unused row): no mass
+        for (int r = threadIdx.x; r < nrows; r += 256) {
+            const int64_t gr = (int64_t)(tok0 + r / hb) * a.H + h0 + r % hb;
+            if (a.nsplit > 1) {
+                a.part_ml[(gr * a.nsplit + split) * 2] = -INFINITY;
+                a.part_ml[(gr * a.nsplit + split) * 2 + 1] = 0.f;
+            } else {
+                for (int d = 0; d < a.vp; ++d) a.ctx[gr * a.vp + d] = 0;
+            }
+        }
+        return;
+    }
+    const int bmask = (1 << a.bs_shift) - 1;
+    const int klo = lo + t0 * 64, khi = min(p1, lo + t1 * 64 - 1);  // keys of this split
+    const int blk0 = klo >> a.bs_shift, nblk = (khi >> a.bs_shift) - blk0 + 1;
+    // the query rows, requested beside the block table
+    u32x4_t qf[MT][KS];
+    int rpos[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int r = 16 * m + c;
+        const bool own = r < nrows;
+        rpos[m] = own ? p0 + r / hb : -1;
+        const bf16_t* q = reinterpret_cast<const bf16_t*>(a.qa) + ((int64_t)(tok0 + (own ? r / hb : 0)) * a.H + h0 + (own ? r % hb : 0)) * a.rp;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int k = 32 * i + 8 * g;
+            qf[m][i] = u32x4_t{0, 0, 0, 0};
+            if (own && k < a.rp) qf[m][i] = *reinterpret_cast<const u32x4_t*>(q + k);
+        }
+    }
+    // 64 entries of the block table, one per lane (entries in front of the window may have been given back, -1: no key of theirs is fetched)
+    int bt0 = 0, bt_v;
+    auto load_bt = [&](int b0) {
+        bt0 = b0;
+        const int b = a.bt[(int64_t)seq * a.bt_stride + blk0 + min(b0 + lane, nblk - 1)];
+        bt_v = (int)min(max((int64_t)b, (int64_t)0), a.n_blocks - 1);
+    };
+    load_bt(0);
+    // per-lane source offsets (bytes) of a stage's pieces
+    unsigned off[P];
+    int orow[P];
+    const bool padded = RPAD != a.rp;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int q = i * 64 + lane, row = q / CPR, ch = (q % CPR) ^ attn_swz(row);
+        orow[i] = (padded && ch * 8 >= a.rp) ? 1 << 30 : row;
+        off[i] = (unsigned)(row * a.rp + ch * 8) * 2u;
+    }
+    char* const ring = smem + w * C::WAVEB;
+    auto issue = [&](int it, int slot) {  // the wave's keys of tile `it`
+        const int k0 = klo + it * 64 + w * 16;
+        const int b = min((k0 >> a.bs_shift) - blk0, nblk - 1);
+        if (b >= bt0 + 64) load_bt(b);
+        const int blk = __builtin_amdgcn_readlane(bt_v, b - bt0);
+        const char* src = reinterpret_cast<const char*>(a.cache) + (((int64_t)blk << a.bs_shift) + (k0 & bmask)) * a.rp * 2;
+        char* st = ring + slot * C::STAGEB;
+        const int left = khi - k0, skip = first - k0;
+        if (left >= 15 && skip <= 0 && !padded) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) lds_dma16<2>(src + off[i], st + i * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < P; ++i) lds_dma16<2>(orow[i] <= left && orow[i] >= skip ? (const void*)(src + off[i]) : (const void*)la_zero_page, st + i * 1024);
+        }
+    };
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[m][i]));  // landed before the stages are counted
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+        if (s < n) issue(s, s);
+    f32x4_t acc[MT][ND];
+    float m_run[MT], l_run[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        m_run[m] = -INFINITY;
+        l_run[m] = 0.f;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) acc[m][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    const unsigned base = lds_addr(ring);
+    unsigned k_rel[2], v_rel[4];  // K row c, chunk 4 i + g; V row 4 g + qq, column tile d (parts of either depend on the parity of i / d & 3 only)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) k_rel[e] = base + c * ROWB + (((4 * e + g) ^ attn_swz(c)) << 4);
+    const int qq = (lane >> 2) & 3, pp = lane & 3, vrow = 4 * g + qq;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v_rel[e] = base + vrow * ROWB + (((2 * e + (pp >> 1)) ^ attn_swz(vrow)) << 4) + ((pp & 1) << 3);
+    const float sc = a.scale * LOG2E;
+    int slot = 0;
+    for (int it = 0; it < n; ++it) {
+        const int behind = min(n - 1 - it, NST - 1);  // stages that may still be on their way
+        if (behind == 3) wait_vm<(NST > 3 ? 3 : 0) * P>();
+        else if (behind == 2) wait_vm<(NST > 2 ? 2 : 0) * P>();
+        else if (behind == 1) wait_vm<P>();
+        else wait_vm<0>();
+        const int key0 = klo + it * 64 + w * 16;
+        const unsigned so = slot * C::STAGEB;
+        if (key0 <= p1 && key0 + 15 >= first) {
+            // ---- scores, two accumulation chains per row tile ----
+            f32x4_t s2[MT][2];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) s2[m][0] = s2[m][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            constexpr int FG = 8;
+            static_for<(KS + FG - 1) / FG>([&](auto G) {
+                constexpr int i0 = decltype(G)::value * FG, ni = KS - i0 < FG ? KS - i0 : FG;
+                u32x4_t kf[FG];
+                static_for<ni>([&](auto I) { constexpr int i = i0 + decltype(I)::value; lds_read_b128<(i >> 1) * 128>(kf[i - i0], k_rel[i & 1] + so); });
+                wait_lds();
+#pragma unroll
+                for (int i = 0; i < ni; ++i) asm volatile("" : "+v"(kf[i]));
+#pragma unroll
+                for (int i = 0; i < ni; ++i)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+                        s2[m][i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[i]), __builtin_bit_cast(bf16x8_t, qf[m][i0 + i]), s2[m][i & 1], 0, 0, 0);
+            });
+            // ---- weights of row c: this lane holds keys 4 g + r.  The reference point is raised only when a score exceeds it by more than 2^8 ----
+            typedef short s16x4_t __attribute__((ext_vector_type(4)));
+            s16x4_t pf[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                float x[4], mx;
+                if (key0 > p1 - a.window && key0 + 15 <= p0) {  // every row sees every key
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = (s2[m][0][r] + s2[m][1][r]) * sc;
+                } else {
+                    const int d0 = rpos[m] - (key0 + 4 * g);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[r] = (rpos[m] >= 0 && d0 - r >= 0 && d0 - r < a.window) ? (s2[m][0][r] + s2[m][1][r]) * sc : -INFINITY;
+                }
+                mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+                if (__any(mx > m_run[m] + 8.0f || (m_run[m] == -INFINITY && mx > -INFINITY))) {
+                    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                    const float m_new = fmaxf(m_run[m], mx);
+                    const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[m] - m_new);
+                    l_run[m] *= alpha;
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) acc[m][d] *= alpha;
+                    m_run[m] = m_new;
+                }
+                const float m_use = m_run[m] == -INFINITY ? 0.f : m_run[m];
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(x[r] - m_use);
+                l_run[m] += (p[0] + p[1]) + (p[2] + p[3]);
+                pf[m] = __builtin_bit_cast(s16x4_t, u32x2_t{pack2bf(p[0], p[1]), pack2bf(p[2], p[3])});
+            }
+            // ---- O^T += C^T . P^T ----
+            constexpr int VG = 8;
+            static_for<(ND + VG - 1) / VG>([&](auto G) {
+                constexpr int d0 = decltype(G)::value * VG, nd = ND - d0 < VG ? ND - d0 : VG;
+                u32x2_t vf[VG];
+                static_for<nd>([&](auto I) { constexpr int d = d0 + decltype(I)::value; lds_read_tr16_b64<(d >> 2) * 128>(vf[d - d0], v_rel[d & 3] + so); });
+                wait_lds();
+#pragma unroll
+                for (int d = 0; d < nd; ++d) asm volatile("" : "+v"(vf[d]));
+#pragma unroll
+                for (int d = 0; d < nd; ++d)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) acc[m][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4_t, vf[d]), pf[m], acc[m][d0 + d], 0, 0, 0);
+            });
+        }
+        if (it + NST < n) issue(it + NST, slot);  // (the stage's last fragments are in registers)
+        slot = slot + 1 == NST ? 0 : slot + 1;
+    }
+    // ---- the waves' maxima, masses and sums meet in LDS, 16 rows at a time; wave w finishes column tiles w, w + 4, ... ----
+    float* ml = reinterpret_cast<float*>(smem + 4 * C::WAVEB);  // [4][MT][16][2]
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        l_run[m] += __shfl_xor(l_run[m], 16, 64);
+        l_run[m] += __shfl_xor(l_run[m], 32, 64);
+        if (g == 0) *reinterpret_cast<u32x2_t*>(ml + ((w * MT + m) * 16 + c) * 2) = u32x2_t{__builtin_bit_cast(unsigned, m_run[m]), __builtin_bit_cast(unsigned, l_run[m])};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        float M = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[((u * MT + m) * 16 + c) * 2]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float mu = ml[((u * MT + m) * 16 + c) * 2];
+            l += mu == -INFINITY ? 0.f : ml[((u * MT + m) * 16 + c) * 2 + 1] * __builtin_amdgcn_exp2f(mu - M);
+        }
+        const float f = m_run[m] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[m] - M);
+        if (m > 0) __syncthreads();  // the sums of the rows before have been read
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            acc[m][d] *= f;
+            if ((d & 3) != w) *reinterpret_cast<f32x4_t*>(ring + d * 1024 + lane * 16) = acc[m][d];
+        }
+        __syncthreads();
+        const int r = 16 * m + c;
+        const int hd = h0 + r % hb;
+        const int64_t gr = (int64_t)(tok0 + r / hb) * a.H + hd;
+        float inv = 1.0f;
+        if (a.nsplit == 1 && r < nrows) {
+            const float sk = a.sink[hd] * LOG2E, Ms = fmaxf(M, sk), fs = __builtin_amdgcn_exp2f(M - Ms);
+            inv = fs / (l * fs + __builtin_amdgcn_exp2f(sk - Ms));
+        }
+        static_for<ND>([&](auto D) {
+            constexpr int d = decltype(D)::value;
+            if ((d & 3) == w && r < nrows) {
+                f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) o += u == (d & 3) ? acc[m][d] : *reinterpret_cast<const f32x4_t*>(smem + u * C::WAVEB + d * 1024 + lane * 16);
+                const int dim = 16 * d + 4 * g;
+                if (dim < a.vp) {
+                    if (a.nsplit == 1) *reinterpret_cast<u32x2_t*>(a.ctx + gr * a.vp + dim) = u32x2_t{pack2bf(o[0] * inv, o[1] * inv), pack2bf(o[2] * inv, o[3] * inv)};
+                    else *reinterpret_cast<f32x4_t*>(a.part_o + (gr * a.nsplit + split) * a.vp + dim) = o;
+                }
+            }
+        });
+        if (a.nsplit > 1 && w == 0 && g == 0 && r < nrows) {
+            a.part_ml[(gr * a.nsplit + split) * 2] = M;
+            a.part_ml[(gr * a.nsplit + split) * 2 + 1] = l;
+        }
+    }
+}
+
+template <int NCT, int VCT, int MT>
+int launch_latent_keys(const AttnArgs& a, hipStream_t st) {
+    using C = LkCfg<NCT, VCT, MT>;
+    auto kern = latent_keys_kernel<NCT, VCT, MT>;
+    GLM_SET_MAX_LDS(kern, C::LDS, "glm_latent_attn");
+    const int64_t grid = (int64_t)a.n_tiles * a.n_hg * a.nsplit;
+    GLM_CHECK_ARG(grid < (1ll << 31), GLM_ERR_UNSUPPORTED, "glm_latent_attn: grid too large");
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), C::LDS, st, a);
+    GLM_CHECK_LAUNCH("glm_latent_attn");
+    return GLM_OK;
+}
+
 template <int NCT, int MT>
 int launch_latent_attn(const AttnArgs& a, hipStream_t st) {
     using C = LaCfg<NCT, MT>;
@@ -573,9 +853,16 @@ int launch_latent_attn(const AttnArgs& a, hipStream_t st) {
 constexpr int la_max_rows(int nct) { return nct > 9 ? 16 : nct > 4 ? 32 : 64; }
 
 template <int NCT>
-int launch_latent_attn_mt(const AttnArgs& a, int mt, hipStream_t st) {
+int launch_latent_attn_mt(const AttnArgs& a, int mt, bool many_keys, hipStream_t st) {
     if constexpr (la_max_rows(NCT) >= 64) {
         if (mt > 2) return launch_latent_attn<NCT, 4>(a, st);
+    }
+    if constexpr (NCT <= 9) {  // (a wave's sums and queries of all rows in its registers: 32 rows up to 256 columns)
+        constexpr int VCT = NCT < 8 ? NCT : 8;
+        if (many_keys && mt == 1 && a.vp <= 64 * VCT) return launch_latent_keys<NCT, VCT, 1>(a, st);
+        if constexpr (NCT <= 4) {
+            if (many_keys && mt == 2) return launch_latent_keys<NCT, VCT, 2>(a, st);
+        }
     }
     if constexpr (la_max_rows(NCT) >= 32) {
         if (mt > 1) return launch_latent_attn<NCT, 2>(a, st);
@@ -693,6 +980,101 @@ __global__ __launch_bounds__(256) void latent_up_kernel(const UpArgs a) {
     }
     if (t < a.Ta && v < a.vdimp)
         *reinterpret_cast<u32x2_t*>(a.out + t * a.ldo + (int64_t)h * a.vdimp + v) = u32x2_t{pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3])};
+}
+
+// The same behind splits of the keys (2 to 8: 128 tokens of 16 heads over 256 columns, two splits, 4.0 us instead of 4.8 for each of two launches): a workgroup forms the context of 16 tokens of one head from the splits' sums (their order and
+// roundings are attn_merge_kernel's), leaves it in LDS in bf16, and its waves multiply 16 value rows each, whose weights were requested first.
+// NK: 256-column blocks of the latent.
+struct UpMergeArgs {
+    UpArgs u;                       // ctx unused
+    const float *part_o, *part_ml;  // [Ta * H, nsplit, rp], [Ta * H, nsplit, 2]
+    const float* sink;              // [H]
+    int nsplit, nvb;                // nvb: blocks of 128 value rows
+};
+
+template <int NK>
+__global__ __launch_bounds__(512) void latent_up_merge_kernel(const UpMergeArgs m) {
+    const UpArgs& a = m.u;
+    constexpr int PITCH = NK * 512 + 16;
+    __shared__ __attribute__((aligned(16))) char ctx[16 * PITCH];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x / m.nvb, v0 = (blockIdx.x % m.nvb) * 128 + wid * 16;
+    const int64_t t0 = (int64_t)blockIdx.y * 16;
+    const bf16_t* wr = a.wuv + ((int64_t)h * a.vdimp + min(v0 + c, a.vdimp - 1)) * a.rp;
+    u32x4_t av[8 * NK];
+#pragma unroll
+    for (int i = 0; i < 8 * NK; ++i) {
+        const int k = 32 * i + 8 * g;
+        av[i] = *reinterpret_cast<const u32x4_t*>(wr + (k < a.rp ? k : 0));
+        if (k >= a.rp) av[i] = u32x4_t{0, 0, 0, 0};
+    }
+    {
+        const int r = threadIdx.x >> 5, l32 = threadIdx.x & 31;  // 32 lanes per token
+        const int64_t row = min(t0 + r, a.Ta - 1) * a.H + h;
+        float ms = -INFINITY, ls = 0.f;
+        if (l32 < m.nsplit) {
+            ms = m.part_ml[(row * m.nsplit + l32) * 2];
+            ls = m.part_ml[(row * m.nsplit + l32) * 2 + 1];
+        }
+        const float sk = m.sink[h] * LOG2E;
+        float M = ms;
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+        M = fmaxf(M, sk);
+        const float e = ls > 0.f ? __builtin_amdgcn_exp2f(ms - M) : 0.f;
+        float mass = ls * e;
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) mass += __shfl_xor(mass, o, 64);
+        mass += __builtin_amdgcn_exp2f(sk - M);
+        const float f = mass > 0.f ? e / mass : 0.f;  // 0: an empty split, its sums were never written
+        const float* p = m.part_o + row * m.nsplit * a.rp;
+#pragma unroll
+        for (int j0 = 0; j0 < 2 * NK; j0 += 2) {
+            f32x4_t o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int s0 = 0; s0 < m.nsplit; s0 += 4) {
+                f32x4_t x[4][2];
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const int k = (j0 + j) * 128 + 4 * l32;
+                        x[s][j] = *reinterpret_cast<const f32x4_t*>(p + (int64_t)min(s0 + s, m.nsplit - 1) * a.rp + (k < a.rp ? k : 0));
+                    }
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const float fs = s0 + s < m.nsplit ? __shfl(f, (lane & 32) + s0 + s, 64) : 0.f;
+                    if (fs != 0.f) {
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) o[j][i] += fs * x[s][j][i];
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int k = (j0 + j) * 128 + 4 * l32;
+                const bool on = k < a.rp;
+                *reinterpret_cast<u32x2_t*>(ctx + r * PITCH + k * 2) = u32x2_t{on ? pack2bf(o[j][0], o[j][1]) : 0u, on ? pack2bf(o[j][2], o[j][3]) : 0u};
+            }
+        }
+    }
+    __syncthreads();
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8 * NK; ++i) {
+        const u32x4_t bv = *reinterpret_cast<const u32x4_t*>(ctx + c * PITCH + (32 * i + 8 * g) * 2);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[i]), __builtin_bit_cast(bf16x8_t, bv), acc, 0, 0, 0);
+    }
+    const int v = v0 + 4 * g;
+    const int64_t t = t0 + c;
+    if (t >= a.Ta || v >= a.vdimp) return;
+    if (a.gate) {
+        const u32x2_t gt = *reinterpret_cast<const u32x2_t*>(a.gate + t * a.ldg + (int64_t)h * a.vdimp + v);
+        acc *= f32x4_t{bflo(gt[0]), bfhi(gt[0]), bflo(gt[1]), bfhi(gt[1])};
+    }
+    *reinterpret_cast<u32x2_t*>(a.out + t * a.ldo + (int64_t)h * a.vdimp + v) = u32x2_t{pack2bf(acc[0], acc[1]), pack2bf(acc[2], acc[3])};
 }
 
 int pick_nct(int rp) {
@@ -819,15 +1201,16 @@ extern "C" int glm_latent_attn(const void* qa, const void* cache, int64_t n_bloc
     const int64_t range = ((int64_t)bt_stride * block_size < (int64_t)window + tokens_per_tile ? (int64_t)bt_stride * block_size : (int64_t)window + tokens_per_tile);
     GLM_CHECK_ARG((range / nsplit + 128) / block_size + 2 <= LA_BT, GLM_ERR_UNSUPPORTED, "glm_latent_attn: %ld keys per split exceed the block-table slice", (long)(range / nsplit));
     const int rows = tokens_per_tile * a.hb, mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+    const bool many_keys = range / nsplit >= 256;  // four 64-key tiles per split, on both sides of which the two kernels are level
     switch (nct) {
-        case 1: return launch_latent_attn_mt<1>(a, mt, st);
-        case 2: return launch_latent_attn_mt<2>(a, mt, st);
-        case 3: return launch_latent_attn_mt<3>(a, mt, st);
-        case 4: return launch_latent_attn_mt<4>(a, mt, st);
-        case 6: return launch_latent_attn_mt<6>(a, mt, st);
-        case 8: return launch_latent_attn_mt<8>(a, mt, st);
-        case 9: return launch_latent_attn_mt<9>(a, mt, st);
-        default: return launch_latent_attn_mt<16>(a, mt, st);
+        case 1: return launch_latent_attn_mt<1>(a, mt, many_keys, st);
+        case 2: return launch_latent_attn_mt<2>(a, mt, many_keys, st);
+        case 3: return launch_latent_attn_mt<3>(a, mt, many_keys, st);
+        case 4: return launch_latent_attn_mt<4>(a, mt, many_keys, st);
+        case 6: return launch_latent_attn_mt<6>(a, mt, many_keys, st);
+        case 8: return launch_latent_attn_mt<8>(a, mt, many_keys, st);
+        case 9: return launch_latent_attn_mt<9>(a, mt, many_keys, st);
+        default: return launch_latent_attn_mt<16>(a, mt, many_keys, st);
     }
 }
 
@@ -841,5 +1224,23 @@ extern "C" int glm_latent_up(const void* ctx, const void* wuv, void* out, const 
     const int items = H * ((vdimp + 15) / 16);
     hipLaunchKernelGGL(latent_up_kernel, dim3((unsigned)((items + 3) / 4), (unsigned)((Ta + 15) / 16)), dim3(256), 0, glm_s(stream), a);
     GLM_CHECK_LAUNCH("glm_latent_up");
+    return GLM_OK;
+}
+
+extern "C" int glm_latent_up_merge(const float* part_o, const float* part_ml, const float* sink, int nsplit, const void* wuv, void* out, const void* gate, int64_t ldg, int64_t ldo,
+                                   int64_t Ta, int H, int vdimp, int rp, glm_stream_t stream) {
+    GLM_CHECK_ARG((!gate || (ldg >= (int64_t)H * vdimp && ldg % 4 == 0)), GLM_ERR_INVALID, "glm_latent_up_merge: bad gate (ldg=%ld)", (long)ldg);
+    GLM_CHECK_ARG(part_o && part_ml && sink && nsplit >= 1 && nsplit <= 32 && wuv && out && Ta >= 0 && H > 0 && vdimp > 0 && vdimp % 8 == 0 && rp > 0 && rp % 8 == 0 &&
+                      ldo >= (int64_t)H * vdimp && ldo % 4 == 0 && glm_aligned16(part_o) && glm_aligned16(wuv), GLM_ERR_INVALID,
+                  "glm_latent_up_merge: bad shape Ta=%ld H=%d vdimp=%d splits=%d", (long)Ta, H, vdimp, nsplit);
+    const int nvb = (vdimp + 127) / 128;
+    GLM_CHECK_ARG((Ta + 15) / 16 <= 65535 && rp <= 1024, GLM_ERR_UNSUPPORTED, "glm_latent_up_merge: too many rows, or a latent of %d columns", rp);
+    if (Ta == 0) return GLM_OK;
+    const UpMergeArgs a = {{nullptr, (const bf16_t*)wuv, (bf16_t*)out, (const bf16_t*)gate, ldg, ldo, Ta, H, vdimp, rp}, part_o, part_ml, sink, nsplit, nvb};
+    const dim3 grid((unsigned)(H * nvb), (unsigned)((Ta + 15) / 16));
+    if (rp <= 256) hipLaunchKernelGGL(latent_up_merge_kernel<1>, grid, dim3(512), 0, glm_s(stream), a);
+    else if (rp <= 512) hipLaunchKernelGGL(latent_up_merge_kernel<2>, grid, dim3(512), 0, glm_s(stream), a);
+    else hipLaunchKernelGGL(latent_up_merge_kernel<4>, grid, dim3(512), 0, glm_s(stream), a);
+    GLM_CHECK_LAUNCH("glm_latent_up_merge");
     return GLM_OK;
 }

@@ -156,6 +156,7 @@ _SIGNATURES = {
         c_int64, c_int64, c_int, c_int, c_int, c_int, c_float, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
     "glm_attn_merge": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int64, c_int, c_int, c_void_p, c_void_p]),
     "glm_latent_up": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
+    "glm_latent_up_merge": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_void_p]),
     "glm_window_attn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p, c_void_p,
         c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int, c_int, c_int, c_int,
         c_float, c_void_p, c_void_p]),
@@ -1535,7 +1536,8 @@ def latent_attn(qa: torch.Tensor, cache: torch.Tensor, tile_tok: torch.Tensor, t
         keys = min(window + tokens_per_tile, block_tables.shape[1] * bs)
         # (and no more keys per split than a workgroup's slice of the block table covers)
         ns = num_splits or max(1, min(64, 256 // max(1, wgs), -(-keys // 128)), -(-keys // (900 * bs)))
-    ctx = torch.empty((Ta, H, vp), dtype=qa.dtype, device=qa.device)
+    joint = 1 < ns <= 8     # the splits summed up in front of W_uv, in its launch (more of them: one after the other there, side by side in glm_attn_merge)
+    ctx = None if joint else torch.empty((Ta, H, vp), dtype=qa.dtype, device=qa.device)
     if ns > 1:
         part_o = torch.empty((Ta * H, ns, vp), dtype=torch.float32, device=qa.device)
         part_ml = torch.empty((Ta * H, ns, 2), dtype=torch.float32, device=qa.device)
@@ -1547,10 +1549,13 @@ def latent_attn(qa: torch.Tensor, cache: torch.Tensor, tile_tok: torch.Tensor, t
         if gate is not None:
             mul_f32(out[:Ta], gate[:Ta])
         return
+    ldg = gate.stride(0) if gate is not None else 0
+    if joint:
+        _check(lib.glm_latent_up_merge(_p(part_o), _p(part_ml), _p(sink), ns, _p(wuv), _p(out), _p(gate), ldg, out.stride(0), Ta, H, vdimp, vp, _stream()), "glm_latent_up_merge")
+        return
     if ns > 1:
         _check(lib.glm_attn_merge(_p(part_o), _p(part_ml), _p(sink), ns, _p(ctx), H * vp, Ta, H, vp, None, _stream()), "glm_attn_merge")
-    _check(lib.glm_latent_up(_p(ctx), _p(wuv), _p(out), _p(gate), gate.stride(0) if gate is not None else 0, out.stride(0), Ta, H, vdimp, vp, _stream()),
-           "glm_latent_up")
+    _check(lib.glm_latent_up(_p(ctx), _p(wuv), _p(out), _p(gate), ldg, out.stride(0), Ta, H, vdimp, vp, _stream()), "glm_latent_up")
 
 
 WINDOW_ATTN_MAX_DIM = 256  # head sizes of glm_window_attn_prefill

@@ -703,6 +703,9 @@ int glm_attn_merge(const float* part_o, const float* part_ml, const float* sink,
                    int cols, const glm_group_form* form, glm_stream_t stream);
 int glm_latent_up(const void* ctx, const void* wuv, void* out, const void* gate, int64_t ldg, int64_t ldo, int64_t Ta, int H, int vdimp, int rp,
                   glm_stream_t stream);
+/* the same from the splits of glm_latent_attn (up to 32, vp up to 1024): glm_attn_merge's sums, rounded to bf16, then W_uv; rp: its columns, vp of glm_latent_attn */
+int glm_latent_up_merge(const float* part_o, const float* part_ml, const float* sink, int nsplit, const void* wuv, void* out, const void* gate,
+                        int64_t ldg, int64_t ldo, int64_t Ta, int H, int vdimp, int rp, glm_stream_t stream);
 /* Prompts and long portions, bf16: q rows [q_start[s], q_start[s+1]) against expanded k / v rows [k_start[s], k_start[s+1]) — the
  * portion's own tokens last, in front of them the history the window still reaches.  Head h at h*dk (q, k) / h*dv (v, out).
  * Tiles of 128 query rows: (sequence, first row inside the portion).  dk, dv <= 256, multiples of 8.  rotp > 0: the last rotp of

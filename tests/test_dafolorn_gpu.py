@@ -180,6 +180,56 @@ def test_latent_attn(dtype, H, rank, vdim, window, bs, n_q, splits):
             assert err < tol, (s, h, float(err))
 
 
+@pytest.mark.parametrize("H,rank,vdim,window,bs,n_q,splits", [
+    (16, 256, 128, 1024, 64, 1, 2), (16, 256, 136, 1024, 64, 1, 0), (5, 40, 24, 300, 64, 1, 1), (2, 64, 16, 2400, 32, 1, 1), (32, 256, 16, 600, 64, 1, 1),
+    (4, 100, 16, 700, 64, 7, 2), (16, 384, 8, 2000, 128, 1, 7), (16, 512, 24, 1100, 64, 1, 3)])
+@pytest.mark.parametrize("extra", [0, 64])
+def test_latent_attn_long_ranges(H, rank, vdim, window, bs, n_q, splits, extra):
+    """Ranges of 256 keys per split and more, where the waves divide the keys: rings that go round, the block table's slice more than once,
+    windows that start inside a stage, sequences shorter than a split, two row tiles; extra columns that make scores only."""
+    from nanovllm import hip_ops
+    vp, S = hip_ops.round8(rank), 4
+    rp = vp + extra
+    lens = [n_q, window + n_q + 77, window // 3 + n_q, window + n_q]
+    c = [torch.zeros(n, rp) for n in lens]
+    q = torch.zeros(S, n_q, H, rp)
+    keep = [*range(rank), *range(vp, rp)]
+    for s, n in enumerate(lens):
+        c[s][:, keep] = torch.randn(n, len(keep), generator=g(s))
+    q[..., keep] = torch.randn(S, n_q, H, len(keep), generator=g(9)) * 0.5
+    for s, n in enumerate(lens):
+        p = n - 1
+        for h, j in ((0, p - window + 1), (H - 1, p - window), (H // 2, max(0, p - 100))):
+            if 0 <= j < n and (h == 0 or H > 2):
+                _standout(q[s], c[s], n_q - 1, h, j)
+    bf = torch.bfloat16
+    q, c = q.to(bf), [x.to(bf) for x in c]
+    wuv = (torch.randn(H, vdim, vp, generator=g(5)) * rank ** -0.5).to(bf)
+    wuv[..., rank:] = 0
+    sink = torch.randn(H, generator=g(6)) * 2
+    cache, bt = _paged([x.float() for x in c], bs, sum(-(-n // bs) for n in lens) + 3, 7)
+    pos = torch.cat([torch.arange(n - n_q, n) for n in lens])
+    seq_of = torch.arange(S).repeat_interleave(n_q)
+    tpt = min(hip_ops.latent_tokens_per_tile(rp, H), n_q)
+    tok = [s * n_q + k for s in range(S) for k in range(0, n_q, tpt)]
+    cnt = [min(tpt, n_q - k) for s in range(S) for k in range(0, n_q, tpt)]
+    out = torch.full((S * n_q, H * vdim), float("nan"), dtype=bf, device="cuda")
+    gate = torch.randn(S * n_q, H * vdim, generator=g(8)).to(bf)
+    hip_ops.latent_attn(dev(q.reshape(S * n_q, H, rp)), dev(cache, bf), i32(tok), i32(cnt), tpt, i32(pos), i32(seq_of), i32(bt), window, 1.0,
+                        dev(sink), dev(wuv), out, num_splits=splits, gate=dev(gate) if extra else None)
+    got = out.cpu().double().view(S, n_q, H, vdim)
+    for s, n in enumerate(lens):
+        vis = O.window_mask(n, window)[n - n_q:]
+        for h in range(0, H, max(1, H // 5)):
+            a = O.sink_softmax(q[s, :, h].double() @ c[s].double().T, vis, sink[h].double())
+            ref = a @ c[s][:, :vp].double() @ wuv[h].double().T
+            if extra:
+                ref = ref * gate.view(S, n_q, H, vdim)[s, :, h].double()
+            # roundings of the weights, the context and the result to bf16: 2 ** -9 each, summed up over what one row holds
+            err = (got[s, :, h] - ref).abs().max() / max(1.0, float(ref.abs().max()))
+            assert err < 2e-2, (s, h, float(err))
+
+
 @pytest.mark.parametrize("H,dk,dv,window", [(3, 24, 40, 50), (2, 128, 128, 200), (1, 136, 200, 1), (4, 64, 256, 64), (2, 200, 64, 1000), (2, 256, 256, 129)])
 def test_window_attn_prefill(H, dk, dv, window):
     from nanovllm import hip_ops
