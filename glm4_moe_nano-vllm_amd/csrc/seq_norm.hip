@@ -397,15 +397,171 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
     }
 }
 
+// ---- some hundred rows and fewer, a row per workgroup: nothing but latency, so whatever does not depend on something else is requested first
+// (the row with its slabs, four of them at a time, gains and taps; then seq_of -> q_start -> state), and only then come the sums.  The rows in
+// front of it in its portion are formed as well, the arithmetic is the stream kernel's.  128 decoded rows of 2048 columns,
+// half of these launches behind slabs: there 7.1 us with four taps and 6.4 without (a slab's load waited for the one before, the state's for
+// both sums), here 6.7 and 5.3. ----
+template <int TAPS, int NT>
+__global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
+    constexpr int HALO = TAPS - 1, NW = NT / 64;
+    __shared__ float s_red[2][NW];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int c = tid * 8;
+    const bool on = c < a.wp;
+    const int64_t r0 = blockIdx.x;
+    const float inv_w = 1.0f / (float)a.width;
+    const Row8 zero = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto load_row = [&](int64_t r, Row8& x, Row8& y) {
+        x = y = zero;
+        if (!on) return;
+        const int64_t row = a.row_index ? a.row_index[r] : r;
+        x = sn_ld8f(a.x_in + row * a.ldx + c);
+        if (!a.y) return;
+        if (!a.y_f32) {
+            const u32x4_t u = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const bf16_t*>(a.y) + row * a.ldy + c);
+            y.a = f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
+            y.b = f32x4_t{bflo(u[2]), bfhi(u[2]), bflo(u[3]), bfhi(u[3])};
+            return;
+        }
+        const float* p = reinterpret_cast<const float*>(a.y) + row * a.ldy + c;
+        y = sn_ld8f(p);
+        for (int s0 = 1; s0 < a.n_slabs; s0 += 4) {  // (added up in their order)
+            Row8 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = sn_ld8f(p + (int64_t)min(s0 + i, a.n_slabs - 1) * a.slab_stride);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (s0 + i < a.n_slabs) {
+                    y.a += v[i].a;
+                    y.b += v[i].b;
+                }
+        }
+    };
+    int par = 0;
+    auto reduce = [&](float u) {
+        u = sn_wave_sum(u);
+        if (lane == 63) s_red[par][wid] = u;
+        __syncthreads();
+        float su = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) su += s_red[par][i];
+        par ^= 1;
+        return su;
+    };
+    Row8 x, y, gq = zero, gp = zero;
+    load_row(r0, x, y);
+    u32x4_t w[TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) w[j] = u32x4_t{0, 0, 0, 0};
+    if (on) {
+        if (a.y) gq = sn_ld8f(a.g_post + c);
+        if (a.g_pre) gp = sn_ld8f(a.g_pre + c);
+        if constexpr (TAPS > 1) {
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) w[j] = *reinterpret_cast<const u32x4_t*>(a.conv_w + (int64_t)j * a.wp + c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto residual = [&](Row8& x, const Row8& y) {  // x_out
+        if (!a.y) return;
+        const float ry = 1.0f / sqrtf(reduce(sn_sumsq8(y)) * inv_w + a.eps);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x.a[i] = x.a[i] + y.a[i] * ry * gq.a[i];
+            x.b[i] = x.b[i] + y.b[i] * ry * gq.b[i];
+        }
+    };
+    auto normed = [&](const Row8& x) {
+        const float rx = 1.0f / sqrtf(reduce(sn_sumsq8(x)) * inv_w + a.eps);
+        Row8 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h.a[i] = x.a[i] * rx * gp.a[i];
+            h.b[i] = x.b[i] * rx * gp.b[i];
+        }
+        return h;
+    };
+    Row8 hist[TAPS], up[TAPS];  // hist[k - 1]: h of k tokens ago; up: state rows that move up behind a portion shorter than the history
+    int n = 0, e = 0;           // tokens of the portion, and of them behind this row
+    int64_t so = -1;
+    bool keep = false;
+    if constexpr (TAPS > 1) {
+        const int s = a.seq_of[r0], p = a.pos[r0], qs = a.q_start[s], qe = a.q_start[s + 1], d = (int)min(r0 - qs, (int64_t)HALO);
+        const int64_t sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
+        so = a.state_out[s];
+        n = qe - qs;
+        e = qe - 1 - (int)r0;
+        keep = e < HALO && on && so >= 0 && so < a.n_state && p >= 0;
+        const float* st = a.state + sin * HALO * a.wp + c;
+#pragma unroll
+        for (int k = 1; k < TAPS; ++k) {
+            hist[k - 1] = up[k - 1] = zero;
+            if (on && a.g_pre && k > d && p - k >= 0) hist[k - 1] = sn_ld8f(st + (int64_t)(HALO - k + d) * a.wp);
+            if (keep && a.g_pre && e == 0 && k + n <= HALO) up[k - 1] = sn_ld8f(st + (int64_t)(k - 1 + n) * a.wp);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (a.g_pre)
+            for (int64_t q = r0 - d; q < r0; ++q) {
+                Row8 xq, yq;
+                load_row(q, xq, yq);
+                residual(xq, yq);
+                const Row8 h = normed(xq);
+#pragma unroll
+                for (int k = 1; k < TAPS; ++k)
+                    if (r0 - q == k) hist[k - 1] = h;
+            }
+    }
+    residual(x, y);
+    if (on) {
+        if (a.x_out) sn_st8f(a.x_out + r0 * a.ldx + c, x);
+        if (a.x_cast) sn_st8(a.x_cast, r0 * a.ldc + c, a.act_f32, x);
+    }
+    if (!a.g_pre) return;
+    const Row8 h = normed(x);
+    Row8 o = h;
+    if constexpr (TAPS > 1) {
+        auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
+        Row8 acc = zero;
+#pragma unroll
+        for (int k = HALO; k >= 1; --k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * hist[k - 1].a[i];
+                acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * hist[k - 1].b[i];
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
+            o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
+        }
+        if (keep) {
+            float* to = a.state + so * HALO * a.wp + c;
+            sn_st8f(to + (int64_t)(HALO - 1 - e) * a.wp, h);
+#pragma unroll
+            for (int k = 1; k < TAPS; ++k)
+                if (e == 0 && k + n <= HALO) sn_st8f(to + (int64_t)(k - 1) * a.wp, up[k - 1]);
+        }
+    }
+    if (on) sn_st8(a.h, r0 * a.ldh + c, a.act_f32, o);
+}
+
 template <int TAPS, int NT>
 int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
-    // decode: one row per workgroup; else runs of rows long enough to spread the halo and the register setup, short enough
+    // decode: seq_norm_row_kernel; else runs of rows long enough to spread the halo and the register setup, short enough
     // to fill the chip: a row is a chain of one load, two reductions and a store, with one row's loads in flight per workgroup, so some hundred rows
     // stay one to a workgroup, re-reading the halo, as long as those are no more than four waves a SIMD (2048 workgroups of 64 threads: two), and
     // longer runs are cut for as many.  Four taps, us, runs of eight rows and more for 512 workgroups / this: 1024 columns at 800 rows 19.4 / 10.4, at 2048 20.6 / 15.9, at 8000
     // 46 / 33; 2048 at 600 rows 21.5 / 12.5, at 1024 21.9 / 16.0 (1025: 21.8, runs of eight), at 6000 45 / 40, at 15074 108 / 98 (without taps
     // 95 / 83; 2048 workgroups 78 where 1024 took 75).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
+    if constexpr (NT < 1024 || TAPS == 1) {  // (1024 threads do not have the registers for rows, taps and history at once)
+        if (a.T <= 512) {
+            hipLaunchKernelGGL((seq_norm_row_kernel<TAPS, NT>), dim3((unsigned)a.T), dim3(NT), 0, st, a);
+            GLM_CHECK_LAUNCH("glm_seq_norm");
+            return GLM_OK;
+        }
+    }
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;
     hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT>), dim3((unsigned)((a.T + tr - 1) / tr)), dim3(NT), 0, st, a, tr);

@@ -118,6 +118,20 @@ def test_seq_norm(width, taps, y_kind):
             assert torch.allclose(o[s], outs[0][s][: o[s].shape[0]], rtol=1e-6, atol=2e-6)
 
 
+@pytest.mark.parametrize("n", [1, 3, 5, 6, 9, 16])
+@pytest.mark.parametrize("T,width", [(1, 64), (7, 2048), (512, 520), (513, 520)])
+def test_seq_norm_adds_slabs_in_their_order(n, T, width):
+    from nanovllm import hip_ops
+    x, g1 = dev(torch.randn(T, width, generator=g(1))), dev(1 + 0.2 * torch.randn(width, generator=g(2)))
+    slabs = torch.randn(n, T, width, generator=g(3))
+    total = slabs[0].clone()
+    for s in slabs[1:]:
+        total += s
+    run = lambda y: hip_ops.seq_norm(x, width, 1e-5, y=y, g_post=g1, g_pre=g1, act_dtype=torch.float32)  # noqa: E731
+    (xa, ha), (xb, hb) = run(hip_ops.PartialSum(dev(slabs))), run(dev(total))
+    assert torch.equal(xa, xb) and torch.equal(ha, hb)
+
+
 def _paged(rows, bs, n_blocks, seed):
     """Latent rows of several sequences scattered over pages; unused memory is NaN."""
     perm = torch.randperm(n_blocks, generator=g(seed)).tolist()
