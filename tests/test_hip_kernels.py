@@ -1195,6 +1195,17 @@ def test_padded_weight_pitch(ops):
     assert torch.equal(a1, a2)
 
 
+@pytest.mark.parametrize("K,pad", [(2048, 64), (4104, 0), (6144, 64), (8192, 320), (16384, 320)])
+@pytest.mark.parametrize("M", [1, 3, 40, 130])
+def test_padded_weight_pitch_by_row_length(ops, K, pad, M):
+    N = 264
+    x, w = dev(rnd(M, K, seed=107)), dev(rnd(N, K, seed=108, scale=K ** -0.5))
+    wp = ops.padded_weight(N, K, dtype=BF, device="cuda")
+    assert wp.shape == (N, K) and wp.stride() == (K + pad, 1)
+    wp.copy_(w)
+    assert torch.equal(ops.gemm_bf16(x, wp, None), ops.gemm_bf16(x, w, None))
+
+
 # ------------------------------------------------------------------------------------------
 # N4: fp8 (OCP e4m3) weight-only quantised experts
 @pytest.mark.parametrize("T,E,k,H,I", [(32, 8, 2, 512, 128), (5, 4, 2, 4096, 192), (70, 4, 2, 256, 352),
