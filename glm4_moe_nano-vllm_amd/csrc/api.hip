@@ -181,6 +181,24 @@ extern "C" int glm_gemm_bf16_act(const void* x, int64_t ldx, const void* w, int6
     return glm_launch_gemm_smallm(GEMM_PLAIN, p, glm_s(stream));
 }
 
+extern "C" int glm_gemm_bf16_residual_norm(const float* x_in, const int32_t* rows, const void* add, int64_t ld_add, const void* table, int64_t ldt, int64_t vocab, const int64_t* ids,
+                                           float* x_out, const float* g, int width, int K, float eps, const void* w, int64_t ldw, void* y, int64_t ldy, int N, int out_f32, int act,
+                                           float act_a, float act_b, glm_stream_t stream) {
+    GLM_CHECK_ARG((x_in || table) && g && w && y && (!table || ids) && x_out != x_in, GLM_ERR_INVALID, "glm_gemm_bf16_residual_norm: null pointer, or the residual in its own place");
+    GLM_CHECK_ARG(N > 0 && K > 0 && width > 0 && width <= K && ldw >= K && ldy >= N && (!add || ld_add >= K) && (!table || (ldt >= K && vocab > 0)), GLM_ERR_INVALID,
+                  "glm_gemm_bf16_residual_norm: bad shape N=%d K=%d width=%d", N, K, width);
+    GLM_CHECK_ARG(act >= GLM_ACT_NONE && act <= GLM_ACT_RELU2_GATE && act != GLM_ACT_GLU_CLAMP, GLM_ERR_INVALID, "glm_gemm_bf16_residual_norm: unknown activation %d", act);
+    GLM_CHECK_ARG(!out_f32 || (glm_aligned16(y) && ldy % 4 == 0), GLM_ERR_UNSUPPORTED, "glm_gemm_bf16_residual_norm: fp32 rows need 16-byte alignment");
+    GemmParams p;
+    memset(&p, 0, sizeof(p));
+    p.w = (const bf16_t*)w; p.ldw = ldw;
+    p.y = (bf16_t*)y; p.ldy = ldy;
+    if (out_f32) p.yf = (float*)y;
+    p.R = 1; p.N = N; p.K = K; p.G = 1;
+    p.act = GlmAct{act, act_a, act_b};
+    return glm_launch_gemm_tinym_residual(p, x_in, rows, add, ld_add, table, ldt, vocab, ids, x_out, g, width, eps, glm_s(stream));
+}
+
 extern "C" int glm_gemm_bf16_glu(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int N, int K,
                                  float limit, float slope, glm_stream_t stream) {
     GLM_CHECK_ARG(x && w && y, GLM_ERR_INVALID, "glm_gemm_bf16_glu: null pointer");

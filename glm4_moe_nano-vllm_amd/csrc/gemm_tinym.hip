@@ -13,7 +13,9 @@
 //     wave-instruction is one whole KiB of one row) with TWO units in registers: the loads of unit i+1 are issued before
 //     the FMAs of unit i, across tile boundaries, so 16-32 KiB per wave stay in flight from the first to the last byte;
 //   * the token rows live in LDS for the whole kernel (fragment read = one conflict-free ds_read_b128 per segment).
-// Optional prologue (PRO_COMBINE): the activation row is not loaded but COMPUTED by every workgroup — MoE combine of the
+// Optional prologues.  TM_RESIDUAL: the row is the norm of a 32-bit residual and what it takes up (residual_norm.hip's arithmetic, bit for bit),
+// requested in front of the first weights and formed by every workgroup while they arrive; workgroup 0 stores the residual.  The
+// launch it replaces was 4.5 us in which no weights moved.  TM_COMBINE: the activation row is not loaded but COMPUTED by every workgroup — MoE combine of the
 // previous layer + the input add-RMSNorm (decode_layer.py:47-49 of the next layer) — behind the workgroup's first weight
 // loads, which removes the combine + norm launch of a one-token decode layer.  Bit-identical to that launch: same code
 // (fused_rows.h), same 512-thread mapping.
@@ -61,10 +63,12 @@ __device__ const u32x4_t g_tm_zero_page[4] = {};
 __device__ unsigned long long g_tm_stamps[512][3];
 #endif
 
+enum : int { TM_ROW = 0, TM_COMBINE = 1, TM_RESIDUAL = 2 };   // where the activation row comes from
+
 struct TinyParams {
     GemmParams g;
     int n_tokens;             // grouped gate|up: rows of x (= tokens) kept in LDS
-    // PRO_COMBINE: the activation rows are bf16(add_rmsnorm(moe_combine(y_prev), residual)) computed in the kernel
+    // TM_COMBINE: the activation rows are bf16(add_rmsnorm(moe_combine(y_prev), residual)) computed in the kernel
     const bf16_t* pc_y;       // rows of the previous layer's grouped down projection
     int64_t pc_ldy;
     const int32_t* pc_pos;    // pair_pos [T, k]
@@ -75,6 +79,18 @@ struct TinyParams {
     bf16_t* pc_res_out;       // [T, H]  (written by workgroup 0)
     bf16_t* pc_x_out;         // [T, H] or nullptr: the normalised rows, for callers that want them (workgroup 0)
     float pc_eps;
+    // TM_RESIDUAL: the row is bf16(norm(x_in + y + a row of the table) g)
+    const float* rn_x_in;     // or nullptr
+    const int32_t* rn_rows;   // one entry: the row of x_in, y and ids, or nullptr: 0
+    const bf16_t* rn_y;       // or nullptr
+    int64_t rn_ldy;
+    const bf16_t* rn_table;   // or nullptr
+    int64_t rn_ldt, rn_vocab;
+    const int64_t* rn_ids;
+    float* rn_x_out;          // [K] (written by workgroup 0) or nullptr
+    const float* rn_g;        // [K]
+    int rn_width;
+    float rn_eps;
     // TAIL_ROUTER (one token): the projection's output row is the attention's o_proj; the workgroup that finishes LAST
     // continues with the post-attention add-RMSNorm, the router (R1..R7) and glm_moe_align's structure for that token
     unsigned* tr_ticket;       // TWO zeroed uint32 (projection workgroups done, designated workgroups done); left zero
@@ -291,7 +307,7 @@ __device__ __forceinline__ void tinym_router_tail(const TinyParams& tp, char* sm
 }
 
 // MODE as gemm_smallm; M = token rows per group block (1 or 2); SEGS = 1-KiB segments of a weight row per unit
-template <int MODE, int M, int SEGS, bool PRO, bool TAIL = false, int RPW = TM_RPW>
+template <int MODE, int M, int SEGS, int PRO, bool TAIL = false, int RPW = TM_RPW>
 __global__ __launch_bounds__(TM_NT) void gemm_tinym_kernel(const TinyParams tp) {
     static_assert(RPW == 1 || RPW == 2 || RPW == 4, "1, 2 or 4 weight rows per tile");
     static_assert(!gemm_paired(MODE) || RPW >= 2, "gate|up: a tile is gate rows + the matching up rows");
@@ -301,7 +317,7 @@ __global__ __launch_bounds__(TM_NT) void gemm_tinym_kernel(const TinyParams tp) 
     __shared__ int sh_grp[TM_MAXG];   // non-empty groups
     __shared__ int sh_nact;
     __shared__ int sh_next;           // next tile of this workgroup
-    __shared__ float sh_red[TM_NW];
+    __shared__ float sh_red[PRO == TM_RESIDUAL ? 2 * TM_NW : TM_NW];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -374,6 +390,29 @@ __global__ __launch_bounds__(TM_NT) void gemm_tinym_kernel(const TinyParams tp) 
         }
     };
 
+    // TM_RESIDUAL: thread t holds columns 4 t .. and 4 (t + 512) .. of what the row is made of, requested in front of the weights
+    f32x4_t rv[2], rg[2], rt[2];
+    u32x2_t ry[2];
+    if constexpr (PRO == TM_RESIDUAL) {
+        const int64_t src = tp.rn_rows ? tp.rn_rows[0] : 0;
+        const int64_t id = tp.rn_table ? min(max(tp.rn_ids[src], (int64_t)0), tp.rn_vocab - 1) : 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int c = (tid + j * TM_NT) * 4;
+            rv[j] = rg[j] = rt[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            ry[j] = u32x2_t{0u, 0u};
+            if (c >= K) continue;
+            if (tp.rn_x_in) rv[j] = *reinterpret_cast<const f32x4_t*>(tp.rn_x_in + src * K + c);
+            if (tp.rn_y) ry[j] = *reinterpret_cast<const u32x2_t*>(tp.rn_y + src * tp.rn_ldy + c);
+            rg[j] = *reinterpret_cast<const f32x4_t*>(tp.rn_g + c);
+            if (tp.rn_table) {
+                const u32x2_t u = *reinterpret_cast<const u32x2_t*>(tp.rn_table + id * tp.rn_ldt + c);
+                rt[j] = f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
     // issue state runs one unit ahead of the compute state
     Tile it, ct;
     int i_tile = wid, i_u = 0;
@@ -399,11 +438,41 @@ __global__ __launch_bounds__(TM_NT) void gemm_tinym_kernel(const TinyParams tp) 
         }
     };
 
+    // behind a prologue of loads and sums the first tile's second unit is requested in front of it, too
+    bool ahead = PRO == TM_RESIDUAL && i_live && nunits > 1;
+    if (PRO == TM_RESIDUAL && ahead) {
+        i_u = 1;
+        issue(std::integral_constant<int, 1>{}, it, 1);
+    }
+
     // ---- activation rows into LDS: [rows][Kp] bf16, pad zeroed ----
     //   PLAIN: rows 0..M-1 = x rows;  GATEUP: row t = token t (T = p.R / ... tokens, all of x);  DOWN: row r = act row r
     const int xrows = MODE == GEMM_PLAIN ? M : (gemm_paired(MODE) ? tp.n_tokens : (int)p.R);
     bf16_t* xs = reinterpret_cast<bf16_t*>(smem);
-    if (PRO) {
+    if constexpr (PRO == TM_RESIDUAL) {
+        float q[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int c = (tid + j * TM_NT) * 4;
+            if (tp.rn_y) rv[j] += f32x4_t{bflo(ry[j][0]), bfhi(ry[j][0]), bflo(ry[j][1]), bfhi(ry[j][1])};
+            if (tp.rn_table) rv[j] += rt[j];
+            q[j] = c < K ? rv[j][0] * rv[j][0] + rv[j][1] * rv[j][1] + rv[j][2] * rv[j][2] + rv[j][3] * rv[j][3] : 0.f;
+            if (blockIdx.x == 0 && tp.rn_x_out && c < K) *reinterpret_cast<f32x4_t*>(tp.rn_x_out + c) = rv[j];
+            q[j] = wave_sum(q[j]);
+            if (lane == 0) sh_red[j * TM_NW + wid] = q[j];   // (the sixteen waves of the launch that this replaces)
+        }
+        __syncthreads();
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2 * TM_NW; ++i) sum += sh_red[i];
+        const float rinv = 1.0f / sqrtf(sum / (float)tp.rn_width + tp.rn_eps);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int c = (tid + j * TM_NT) * 4;
+            const f32x4_t o = rv[j] * rinv * rg[j];
+            if (c < Kp) *reinterpret_cast<u32x2_t*>(xs + c) = c < K ? u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])} : u32x2_t{0u, 0u};
+        }
+    } else if constexpr (PRO == TM_COMBINE) {
         // combine of the previous MoE block + input add-RMSNorm, token by token, exactly the stand-alone launch's code;
         // the first unit's weight loads are already in flight
         for (int t = 0; t < M; ++t) {
@@ -531,8 +600,11 @@ __global__ __launch_bounds__(TM_NT) void gemm_tinym_kernel(const TinyParams tp) 
     }
     while (c_live) {
         // buffer 0 holds (c_tile, c_u)
-        advance_issue();
-        if (i_live) issue(std::integral_constant<int, 1>{}, it, i_u);
+        if (PRO != TM_RESIDUAL || !ahead) {
+            advance_issue();
+            if (i_live) issue(std::integral_constant<int, 1>{}, it, i_u);
+        }
+        ahead = false;
         compute(std::integral_constant<int, 0>{}, ct, c_u, xr);
 #if GLM_TM_STAMP
         if (!stamped_first) {
@@ -596,7 +668,7 @@ int n_cus() {
     return n;
 }
 
-template <int MODE, int M, int SEGS, bool PRO, bool TAIL = false, int RPW = TM_RPW>
+template <int MODE, int M, int SEGS, int PRO, bool TAIL = false, int RPW = TM_RPW>
 int launch_tiny(const TinyParams& tp, int xrows, hipStream_t st) {
     const GemmParams& p = tp.g;
     constexpr int KU = SEGS * 512;
@@ -649,8 +721,8 @@ int glm_launch_gemm_tinym(int mode, const GemmParams& p, int n_tokens, hipStream
     const int M = mode == GEMM_PLAIN ? (int)p.R : n_tokens;
     GLM_CHECK_ARG(M == 1, GLM_ERR_UNSUPPORTED, "gemm_tinym: %d rows per block", M);
     // units: 4 rows x 4 KiB for long rows; a short K (expert down projection, 1408) as ONE unit of 3-KiB rows
-    if (mode == GEMM_PLAIN) return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, false, false, GLM_TM_RPW_PLAIN>(tp, 1, st);
-    if (mode == GEMM_GLU) return launch_tiny<GEMM_GLU, 1, 8, false, false, 2>(tp, 1, st);
+    if (mode == GEMM_PLAIN) return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, TM_ROW, false, GLM_TM_RPW_PLAIN>(tp, 1, st);
+    if (mode == GEMM_GLU) return launch_tiny<GEMM_GLU, 1, 8, TM_ROW, false, 2>(tp, 1, st);
 #if GLM_EXPERTS
     // grouped launches: rows per tile chosen for the TAIL of the launch — a workgroup's waves pull tiles from a counter, and
     // the launch ends when the slowest wave has finished its last tile; at Air dims one token gives 24.75 tiles of 4 rows per
@@ -661,12 +733,31 @@ int glm_launch_gemm_tinym(int mode, const GemmParams& p, int n_tokens, hipStream
 #ifndef GLM_TM_RPW_DOWN
 #define GLM_TM_RPW_DOWN 4
 #endif
-    if (mode == GEMM_GATEUP) return launch_tiny<GEMM_GATEUP, 1, (GLM_TM_RPW_GATEUP == 2 ? 8 : 4), false, false, GLM_TM_RPW_GATEUP>(tp, n_tokens, st);
-    if (p.K <= 1536) return launch_tiny<GEMM_DOWN, 1, 3, false, false, GLM_TM_RPW_DOWN>(tp, (int)p.R, st);
-    return launch_tiny<GEMM_DOWN, 1, 4, false, false, GLM_TM_RPW_DOWN>(tp, (int)p.R, st);
+    if (mode == GEMM_GATEUP) return launch_tiny<GEMM_GATEUP, 1, (GLM_TM_RPW_GATEUP == 2 ? 8 : 4), TM_ROW, false, GLM_TM_RPW_GATEUP>(tp, n_tokens, st);
+    if (p.K <= 1536) return launch_tiny<GEMM_DOWN, 1, 3, TM_ROW, false, GLM_TM_RPW_DOWN>(tp, (int)p.R, st);
+    return launch_tiny<GEMM_DOWN, 1, 4, TM_ROW, false, GLM_TM_RPW_DOWN>(tp, (int)p.R, st);
 #else
     return GLM_ERR_UNSUPPORTED;
 #endif
+}
+
+// One row whose activations are the norm of a residual and what it takes up (glm_residual_norm), 1024 < K <= 4096 columns.  p.x is ignored.
+int glm_launch_gemm_tinym_residual(const GemmParams& p, const float* x_in, const int32_t* rows, const void* y, int64_t ldy, const void* table, int64_t ldt, int64_t vocab,
+                                   const int64_t* ids, float* x_out, const float* g, int width, float eps, hipStream_t st) {
+    GemmParams q = p;
+    q.x = (const bf16_t*)g;  // any aligned pointer: the shape check wants one
+    q.ldx = p.K;
+    if (!tiny_shape_ok(GEMM_PLAIN, q) || p.R != 1 || p.K <= 1024 || p.K > 4096 || ldy % 8 != 0 || ldt % 8 != 0 || (x_in && !glm_aligned16(x_in)) || (y && !glm_aligned16(y)) ||
+        (table && !glm_aligned16(table)) || (x_out && !glm_aligned16(x_out)) || !glm_aligned16(g)) {
+        glm_set_error("gemm_tinym(residual norm): shape not covered (K=%d N=%d)", p.K, p.N);
+        return GLM_ERR_UNSUPPORTED;
+    }
+    TinyParams tp;
+    memset(&tp, 0, sizeof(tp));
+    tp.g = q;
+    tp.rn_x_in = x_in; tp.rn_rows = rows; tp.rn_y = (const bf16_t*)y; tp.rn_ldy = ldy; tp.rn_table = (const bf16_t*)table; tp.rn_ldt = ldt; tp.rn_vocab = vocab;
+    tp.rn_ids = ids; tp.rn_x_out = x_out; tp.rn_g = g; tp.rn_width = width; tp.rn_eps = eps;
+    return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, TM_RESIDUAL, false, GLM_TM_RPW_PLAIN>(tp, 1, st);
 }
 
 #if !GLM_DENSE_ONLY
@@ -690,7 +781,7 @@ int glm_launch_gemm_tinym_combine_norm(const GemmParams& p, const void* y_prev, 
     tp.pc_y = (const bf16_t*)y_prev; tp.pc_ldy = ld_yprev; tp.pc_pos = pair_pos; tp.pc_k = k; tp.pc_shared_base = shared_base;
     tp.pc_res_in = (const bf16_t*)residual_in; tp.pc_norm_w = (const bf16_t*)norm_w; tp.pc_res_out = (bf16_t*)residual_out;
     tp.pc_x_out = (bf16_t*)x_out; tp.pc_eps = eps;
-    return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, true, false, GLM_TM_RPW_PLAIN>(tp, 1, st);
+    return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, TM_COMBINE, false, GLM_TM_RPW_PLAIN>(tp, 1, st);
 }
 
 // o_proj of ONE token row continued, in the last workgroup to finish, by the post-attention add-RMSNorm + router +
@@ -716,7 +807,7 @@ int glm_launch_gemm_tinym_router_tail(const GemmParams& p, unsigned* ticket, flo
     tp.tr_y = (bf16_t*)y_norm; tp.tr_res_out = (bf16_t*)residual_out; tp.tr_gate_w = (const bf16_t*)gate_w; tp.tr_bias = bias;
     tp.tr_E = E; tp.tr_k = k; tp.tr_rsf = rsf; tp.tr_idx = topk_idx; tp.tr_w = (bf16_t*)topk_w;
     tp.tr_offs = offs; tp.tr_tok = tok; tp.tr_scale = (bf16_t*)scale; tp.tr_pos = pos; tp.tr_shared = with_shared;
-    return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, false, true, GLM_TM_RPW_PLAIN>(tp, 1, st);
+    return launch_tiny<GEMM_PLAIN, 1, GLM_TM_SEGS_PLAIN, TM_ROW, true, GLM_TM_RPW_PLAIN>(tp, 1, st);
 }
 #endif  // !GLM_DENSE_ONLY
 

@@ -148,6 +148,8 @@ _SIGNATURES = {
         c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_int, c_float, c_void_p]),
     "glm_embed_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,
         c_int64, c_int, c_int, c_float, c_void_p]),
+    "glm_gemm_bf16_residual_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float,
+        c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_float, c_float, c_void_p]),
     "glm_latent_prepare": (c_int, [c_void_p, c_int64, c_int, c_int64, c_int64, c_int, c_int, c_int, c_int, c_void_p,
         c_float, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_void_p]),
     "glm_latent_gather": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p]),
@@ -1830,6 +1832,49 @@ def residual_norm(x: torch.Tensor | None, width: int, wp: int, eps: float, y=Non
                                             table.shape[0] if table is not None else 0, _p(ids), _p(x_out), _p(g), _p(h), wp, _is_f32(act_dtype), T, width, wp, eps, _stream()),
            "glm_residual_norm")
     return x_out, h
+
+
+class NormedRow:
+    """The h of residual_norm for ONE row, formed inside the projection that reads it (glm_gemm_bf16_residual_norm): `linear` instead of linear_act.  x: the
+    residual, there once the projection has run."""
+    shape, dtype = None, torch.bfloat16
+
+    def __init__(self, x, width: int, wp: int, eps: float, y, embed, g, rows, keep_x: bool):
+        self.device = g.device
+        self.shape = torch.Size((1, wp))
+        self.x = torch.empty((1, wp), dtype=torch.float32, device=self.device) if keep_x else None
+        self.args = (x, width, eps, y, embed, g, rows)
+
+    def linear(self, w: torch.Tensor, act=NO_ACT, out_f32: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
+        x, width, eps, add, embed, g, rows = self.args
+        ids, table = embed or (None, None)
+        wp, N = self.shape[1], w.shape[0]
+        dt = torch.float32 if out_f32 else self.dtype
+        out = torch.empty((1, N), dtype=dt, device=self.device) if out is None else out
+        assert w.shape[1] == wp and w.dtype == self.dtype and w.stride(1) == 1 and out.shape == (1, N) and out.dtype == dt and out.stride(1) == 1
+        _check(load_library().glm_gemm_bf16_residual_norm(
+            _p(x), _p(rows), _p(add), wp, _p(table), table.stride(0) if table is not None else wp, table.shape[0] if table is not None else 0, _p(ids), _p(self.x), _p(g),
+            width, wp, eps, _p(w), w.stride(0), _p(out), out.stride(0), N, int(out_f32), *act, _stream()), "glm_gemm_bf16_residual_norm")
+        return out
+
+
+def normed_row(x, width: int, wp: int, eps: float, w: torch.Tensor, y=None, embed: tuple | None = None, g: torch.Tensor | None = None, rows: torch.Tensor | None = None,
+               keep_x: bool = True) -> NormedRow | None:
+    """NormedRow of residual_norm's arguments for a projection by w, or None: more than one row, other types, sizes that kernel does not take."""
+    T = rows.numel() if rows is not None else (x.shape[0] if x is not None else embed[0].numel())
+    if T != 1 or g is None or not 1024 < wp <= 4096 or w.dtype != torch.bfloat16 or w.shape[1] != wp or w.shape[0] % 4 or w.stride(0) % 8 or w.stride(1) != 1 or not opt("tinym"):
+        return None
+    if y is not None and (not isinstance(y, torch.Tensor) or y.dtype != torch.bfloat16 or not y.is_contiguous() or y.shape[-1] != wp):
+        return None
+    if embed is not None:
+        ids, table = embed
+        if table.dtype != torch.bfloat16 or table.stride(0) % 8 or table.stride(1) != 1 or table.shape[1] < wp or ids.dtype != torch.int64:
+            return None
+    if any(t is not None and t.data_ptr() % 16 for t in (x, y, embed[1] if embed else None, g, w)):
+        return None
+    assert x is None or (x.dtype == torch.float32 and x.is_contiguous() and x.shape[1] == wp)
+    assert (rows is None or rows.dtype == torch.int32) and g.dtype == torch.float32 and g.numel() == wp
+    return NormedRow(x, width, wp, eps, y, embed, g, rows, keep_x)
 
 
 MEMORY_CHUNK_MAX_DIM = 256   # key size of glm_memory_chunkwise

@@ -49,10 +49,13 @@ class ParallelBlock(nn.Module):
         return PARTIAL_SLICES if T <= PARTIAL_ROWS else hip_ops.row_slices(T, self.wp, self.out_proj.K)
 
     def forward(self, h: torch.Tensor, meta, run: int = 0, cs: torch.Tensor | None = None):
-        """What the layer adds to the residual, [T, wp] (or its K-slice partial sums)."""
+        """What the layer adds to the residual, [T, wp] (or its K-slice partial sums).  h: rows, or a hip_ops.NormedRow."""
         T, n = h.shape[0], self.attp + self.ffp
         rows = torch.empty((T, self.attp + self.in_proj.N), dtype=h.dtype, device=h.device)   # mixer's output | unit | queries, keys, values, gates
-        self.in_proj(h, act=self.act, out=rows[:, self.attp:])
+        if isinstance(h, hip_ops.NormedRow):
+            h.linear(self.in_proj.weight, self.act, out=rows[:, self.attp:])
+        else:
+            self.in_proj(h, act=self.act, out=rows[:, self.attp:])
         self.mixer.attend(rows[:, n:], rows[:, : self.attp], meta, run=run, cs=cs)
         slices = self.slices(T) if h.dtype == torch.bfloat16 else 1
         if slices > 1:

@@ -113,6 +113,11 @@ class LoselixForCausalLM(nn.Module):
             layer.mixer.allocate_cache(num_blocks, block_size, device)
 
     # ------------------------------------------------------------------ step
+    def one_row(self, x, y, w: torch.Tensor, **kw):
+        """The norm in front of a projection of one row, to be formed inside it, or None."""
+        cfg = self.config
+        return hip_ops.normed_row(x, cfg.hidden_size, cfg.padded_width, cfg.rms_norm_eps, w, y=y, **kw) if self.dtype == torch.bfloat16 else None
+
     def forward(self, meta, residual_tap: list | None = None) -> torch.Tensor:
         """fp32 logits [meta.want_rows, vocab] of the wanted rows of a step.  residual_tap (a list) receives the residual stream [T, width]
         after every layer run."""
@@ -125,11 +130,17 @@ class LoselixForCausalLM(nn.Module):
         x = y = None
         for (i, first_of_pass), r in zip(self.runs, self.run_index):
             layer, rot = self.layers[i], self.layers[i].mixer.rot
-            x, h = norm(x, y, g=layer.g, embed=(meta.ids, self.embed) if x is None or first_of_pass else None)
+            kw = dict(g=layer.g, embed=(meta.ids, self.embed) if x is None or first_of_pass else None)
+            h = self.one_row(x, y, layer.block.in_proj.weight, **kw)
+            x, h = (h.x, h) if h is not None else norm(x, y, **kw)
             y = layer.block(h, meta, r, rot.shared_table(meta.pos, tables) if rot is not None else None)
             if residual_tap is not None:
                 residual_tap.append(norm(x, y)[0][:, : cfg.hidden_size])
         if meta.want.numel() == 0:
             return torch.empty((0, cfg.vocab_size), dtype=torch.float32, device=x.device)
-        _, h = norm(x, y, g=self.g_final, rows=meta.want, keep_x=False)
+        kw = dict(g=self.g_final, rows=meta.want, keep_x=False)
+        h = self.one_row(x, y, self.head, **kw)
+        if h is not None:
+            return h.linear(self.head, out_f32=True)[:, : cfg.vocab_size]
+        _, h = norm(x, y, **kw)
         return hip_ops.linear_act(h, self.head, out_f32=True)[:, : cfg.vocab_size]

@@ -607,6 +607,11 @@ int glm_group_norm_store(void* x, int64_t ld, int q_off, int nq, int q_n, int k_
 int glm_residual_norm(const float* x_in, const int32_t* rows, const void* y, int64_t ldy, int y_f32, int n_slabs, int64_t slab_stride,
                       const void* table, int64_t ldt, int64_t vocab, const int64_t* ids, float* x_out, const float* g, void* h,
                       int64_t ldh, int act_f32, int64_t T, int width, int wp, float eps, glm_stream_t stream);
+/* glm_residual_norm of ONE row (bf16 `add`; rows: one entry or NULL) and act(h @ w^T) in one launch, 1024 < K <= 4096: the row's residual [K] to x_out (or
+ * NULL; not x_in), the projection to y [N] (bf16, or fp32: out_f32).  The same bits as the two calls.                                        */
+int glm_gemm_bf16_residual_norm(const float* x_in, const int32_t* rows, const void* add, int64_t ld_add, const void* table, int64_t ldt,
+                                int64_t vocab, const int64_t* ids, float* x_out, const float* g, int width, int K, float eps, const void* w,
+                                int64_t ldw, void* y, int64_t ldy, int N, int out_f32, int act, float act_a, float act_b, glm_stream_t stream);
 
 /* Gated matrix memory (mLSTM; the recurrence is written out in csrc/matrix_memory.hip).  Projection rows x hold q at h*dimp, k at
  * k_off + h*dimp, v at v_off + h*vdimp and the output gate at g_off + h*vdimp.  State rows S [n_state][H][dimp][vdimp], n

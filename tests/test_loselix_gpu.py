@@ -78,6 +78,31 @@ def test_residual_norm(dtype, width):
                         assert none is None and torch.equal(hr, h[dev(rows)])
 
 
+@pytest.mark.parametrize("width,N", [(1032, 8), (1500, 1028), (2048, 4100), (4090, 264), (4096, 12288)])
+def test_norm_of_one_row_in_its_projection(width, N):
+    """The same bits as the two launches, whatever the residual takes up; calls that it does not take get None."""
+    from nanovllm import hip_ops
+    bf, wp, eps = torch.bfloat16, hip_ops.round8(width), 1e-3
+    pad = lambda t: torch.nn.functional.pad(t, (0, wp - width))  # noqa: E731
+    x, y, gain = dev(pad(torch.randn(3, width, generator=g(1)))), dev(pad(torch.randn(3, width, generator=g(2))), bf), dev(pad(1 + 0.2 * torch.randn(width, generator=g(3))))
+    table, ids = dev(pad(torch.randn(30, width, generator=g(4))), bf), torch.randint(0, 30, (3,), generator=g(5)).cuda()
+    w = hip_ops.padded_weight(N, wp, dtype=bf, device="cuda")
+    w.copy_(torch.randn(N, wp, generator=g(6)) * wp ** -0.5)
+    acts = [(hip_ops.NO_ACT, False), (hip_ops.NO_ACT, True), ((hip_ops.ACT_RELU2_GATE, float(N // 2 // 4 * 4), float(N // 4 * 3 // 4 * 4)), False)]
+    for xx, yy, ee, rows in [(x, y, True, i32([2])), (x, None, True, i32([0])), (x, y, False, i32([1])), (x[:1], y[:1], True, None), (None, None, True, None), (None, y[:1], True, None)]:
+        emb = ((ids if rows is not None else ids[:1]), table) if ee else None
+        for act, f32 in acts:
+            xo, h = hip_ops.residual_norm(xx, width, wp, eps, y=yy, embed=emb, g=gain, rows=rows)
+            want = hip_ops.linear_act(h, w, act=act, out_f32=f32)
+            row = hip_ops.normed_row(xx, width, wp, eps, w, y=yy, embed=emb, g=gain, rows=rows)
+            wide = torch.full((1, N + 16), 7.0, dtype=torch.float32 if f32 else bf, device="cuda")
+            row.linear(w, act, f32, wide[:, 8: 8 + N])
+            assert torch.equal(wide[:, 8: 8 + N], want) and torch.equal(row.x, xo) and torch.all(wide[:, :8] == 7) and torch.all(wide[:, 8 + N:] == 7)
+    none = [hip_ops.normed_row(x, width, wp, eps, w, y=y, g=gain), hip_ops.normed_row(x[:1], width, wp, eps, w, y=y[:1].float(), g=gain),
+            hip_ops.normed_row(x[:1], width, wp, eps, w), hip_ops.normed_row(x[:1], width, wp, eps, w.float(), g=gain)]
+    assert none == [None] * 4
+
+
 def test_residual_norm_many_rows():
     """The form for long prompts (the residual past the caches) gives what the one for few rows does."""
     from nanovllm import hip_ops
