@@ -15,8 +15,8 @@
 // the query projection and latent_absorb (q' and the rotated query part behind it) after it; the scores then run over rp + rotp
 // columns, the values over the first rp.
 //
-// Roofline of latent_attn at decode: HBM — window * rank * 2 bytes per sequence, read once.  Four waves per 16 query rows share
-// every 64-key tile, double-buffered by LDS-DMA.  One LDS image serves both products: chunk ^ swz(key) with
+// Roofline of latent_attn at decode: HBM — window * rank * 2 bytes per sequence, read once.  Few rows and many keys: every wave takes keys of its
+// own (latent_keys_kernel); else four waves per 16 query rows share every 64-key tile, double-buffered by LDS-DMA.  One LDS image serves both products: chunk ^ swz(key) with
 // swz(key) = (key & 3) << 1 | (key >> 2) & 1 is conflict-free for the ds_read_b128 row reads and for the transposed
 // ds_read_b64_tr_b16 reads.  Keys outside the sequence's range and padding columns are fetched from a page of zeros, never
 // from unused cache memory (whatever lies there would turn a zero weight into a NaN).
