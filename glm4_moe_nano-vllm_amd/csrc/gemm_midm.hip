@@ -208,8 +208,8 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int m
         }
     }
 
-    // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / NW ..
-    constexpr int MPW = MT / NW;
+    // ---- sum of the waves' tiles, in wave order; wave w finishes row tiles w MT / NW .. (more waves than tiles: the first MT waves one each)
+    constexpr int MPW = MT < NW ? 1 : MT / NW;
     __syncthreads();
     float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
@@ -218,6 +218,7 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int m
         for (int rt = 0; rt < RT; ++rt)
             *reinterpret_cast<f32x4_t*>(red + (((wid * MT + mt) * RT + rt) * 64 + lane) * 4) = acc[rt][mt];
     __syncthreads();
+    if (MT < NW && wid >= MT) return;
     f32x4_t sum[RT][MPW];
 #pragma unroll
     for (int j = 0; j < MPW; ++j)
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_midm_shared_kernel(const Ge
 
 template <int MODE, int MT, int RT, int NW, int NST>
 int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
-    static_assert(MT % NW == 0, "row tiles split over the waves");
+    static_assert(MT % NW == 0 || NW % MT == 0, "row tiles split over the waves");
     constexpr int LDS = midm_lds<MODE, MT, RT, NW, NST>();
     static_assert(LDS <= 160 * 1024, "the rings of all waves must fit the CU's LDS");
     const int cols = gemm_paired(MODE) ? 8 * RT : 16 * RT, nt = (p.N + cols - 1) / cols;
@@ -616,7 +617,7 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
 // 30.0 / 36.2, at 512 47 / - / 31.8* / 40.2; 14336 x 4096 at 64 36.7 / 27.6* / - / 37.5, at 128 56 / 42.6 / 37.7* / 46.3, at 211 77 / 61.5 / 52 /
 // 43.0*; 2048 x 2048 at 1000 rows - / 16.9 / 17.2* / 19.8 (512 tiles of 64 x 64), at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
 // A long K favours split waves at 64 x 64 too, which read each staged byte once: 4096 x 12288 at 211 rows 50 (shared 58), K = 8192 36 (40).
-enum MidmTile { MM_NONE, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
+enum MidmTile { MM_NONE, MM_SPLIT16, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
 
 MidmTile midm_tile_of(int mode, const GemmParams& p) {
     const int64_t n = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
@@ -625,6 +626,11 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
     // it, and with a hundred row blocks and more.  Shared 64 x 64 / split 64 x 32, us: 1024 x 256 at 300 rows 4.3 / 3.8, 264 x 512 at 700 5.7 / 4.7,
     // 512 x 384 at 1000 4.7 / 4.1, fp32 rows 6.2 / 4.8, 64 x 512 at 3000 5.2 / 4.6, at 8000 6.1 / 6.4; gated columns 512 x 128 at 96 rows 3.0 / 3.4,
     // 1024 x 320 at 128 4.1 / 4.2, 256 x 512 at 300 4.4 / 3.9, 132 x 512 at 700 4.6 / 4.4, at 1500 4.9 / 5.5.
+    // Few columns (routers, gates, small latents): a workgroup takes in some 50 GB/s whatever it does, so 32 rows x 16 columns split over eight waves
+    // come before the larger tiles.  64 x 32 over four waves / this, us: 100 rows of 64 x 2048 6.6 / 4.1, x 256 3.5 / 2.9, 211 of 64 x 4096 11.1 /
+    // 6.8, 2000 of 64 x 2048 7.4 / 5.6, 300 of 376 x 2048 7.5 / 5.0, 33 of 376 x 8192 16.3 / 9.5, 8000 of 16 x 512 4.7 / 3.2.  From 384 columns
+    // on a projection may be queries, keys and values, whose fused form sums over four waves: there both keep that order.
+    if (!gemm_paired(mode) && p.N < 384 && p.K >= 256 && fits(32, 16)) return MM_SPLIT16;
     if (fits(64, 32) && (gemm_paired(mode) ? p.K >= (p.R <= 1000 ? 384 : 576) : p.K > 512 || p.R <= 4096)) return MM_SPLIT32;
     if (fits(64, 64)) return p.K >= 8192 ? MM_SPLIT64 : MM_64;
     if (p.R <= 64) return fits(64, 128) ? MM_64x128 : MM_NONE;
@@ -635,6 +641,9 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
 template <int MODE>
 int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
     switch (tile) {
+        case MM_SPLIT16:
+            if constexpr (!gemm_paired(MODE)) return launch_midm_cfg<MODE, 2, 1, 8, 2>(p, st);
+            break;
         case MM_SPLIT32:   // (half a head in the QKV epilogue; the sums are the same in both tiles)
             if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
             [[fallthrough]];

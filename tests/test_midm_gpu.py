@@ -345,3 +345,17 @@ def test_layer_half_replayed(ops, T):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(out, want)), i
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 4, 256), (64, 16, 320), (97, 64, 2048), (100, 132, 4096), (320, 380, 448), (2048, 64, 512), (8192, 12, 256), (341, 380, 256)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_few_columns(M, N, K, f32):
+    """32 rows x 16 columns over eight waves: ends of rows and columns, fewer chunks than waves, the largest grid of that tile and the next."""
+    from nanovllm import hip_ops
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16), (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    out = torch.full((M, N + 8), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda")
+    hip_ops.linear_act(x.cuda(), w.cuda(), out_f32=f32, out=out[:, :N])
+    want = x.double() @ w.double().T
+    err = (out[:, :N].cpu().double() - want).abs().max() / want.abs().max()
+    assert err < (K * 2.0 ** -24 if f32 else 2.0 ** -8) and torch.all(out[:, N:] == 7)   # sums in fp32; the result's rounding
