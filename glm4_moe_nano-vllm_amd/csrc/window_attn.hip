@@ -58,6 +58,9 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
     const int qlast = min(qo + 127, nq - 1);
     const int jlo = max(0, hist + qo - a.window + 1), jhi = hist + qlast;
     const int n = (jhi - jlo + 64) >> 6;
+    // The walk hides keys and takes maxima in front of the scale, which has to be positive there: the queries take its sign, and are zeros where it is zero.
+    const unsigned sign = a.scale < 0.f ? 0x80008000u : 0u, keep = a.scale == 0.f ? 0u : ~0u;
+    const float scale = a.scale == 0.f ? 1.f : fabsf(a.scale);
     // this wave's rows: tile t holds rows qo + 64 t + 16 w + c (the two half-dead tiles of the causal edge cost all waves the same)
     SL S;
     S.init(lane);
@@ -91,7 +94,11 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(S.qf[t][i]));
+        for (int i = 0; i < KS; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) S.qf[t][i][j] = (S.qf[t][i][j] & keep) ^ sign;
+            asm volatile("" : "+v"(S.qf[t][i]));
+        }
     const unsigned base = lds_addr(smem);
     const bf16_t* kbase = a.k + (int64_t)(ks0 + jlo) * a.ldkv + (int64_t)h * a.dkn;
     const bf16_t* rbase = a.kr ? a.kr + (int64_t)(ks0 + jlo) * a.ldr : kbase;
@@ -161,7 +168,7 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
             }
         }
     };
-    attn_tiles<DK, DV, GA_SOFTMAX, KDMA + VDMA>(S, base, n, jlo, g, a.scale * GA_LOG2E, false, issue);
+    attn_tiles<DK, DV, GA_SOFTMAX, KDMA + VDMA>(S, base, n, jlo, g, scale * GA_LOG2E, false, issue);
     const float sk = a.sink[h] * GA_LOG2E;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {

@@ -277,6 +277,32 @@ def test_window_attn_prefill(H, dk, dv, window):
             assert (got[qs[s]: qs[s + 1], h] - ref).abs().max() < 4e-2, (s, h)
 
 
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 128), (3, 24, 40), (2, 192, 128), (1, 256, 256)])
+@pytest.mark.parametrize("scale", [-0.3, 0.0, -0.0, -1e-40, 1e-40])
+def test_window_attn_prefill_any_scale(H, dk, dv, scale):
+    """A scale below zero turns the scores round, with zero (or what is as good as zero) every visible key weighs the same: hidden keys stay hidden."""
+    from nanovllm import hip_ops
+    n, window, rotp = 300, 90, 8
+    q, k, v = torch.randn(n, H, dk, generator=g(1)).bfloat16(), torch.randn(n, H, dk, generator=g(2)).bfloat16(), torch.randn(n, H, dv, generator=g(3)).bfloat16()
+    sink, vis = torch.randn(H, generator=g(4)), O.window_mask(n, window)
+    tiles = ([0, 0, 0], [0, 128, 256])
+    for kr in (False, True):
+        rot = {}
+        if kr:      # the last columns of the keys in rows of their own (one head's for all), not turned
+            k[:, :, dk - rotp:] = k[:, :1, dk - rotp:]
+            rot = dict(kr=dev(k[:, 0, dk - rotp:].contiguous()), cs=torch.tensor([1.0, 0.0], device="cuda").repeat(n * rotp // 2).view(n, rotp))
+        kk = k[:, :, : dk - rotp] if kr else k
+        kv = torch.cat([kk.reshape(n, -1), v.reshape(n, -1)], 1).cuda()
+        out = torch.full((n, H * dv), float("nan"), dtype=torch.bfloat16, device="cuda")
+        hip_ops.window_attn_prefill(dev(q.reshape(n, -1)), kv[:, : kk.shape[1] * kk.shape[2]], kv[:, kk.shape[1] * kk.shape[2]:], out, i32([0, n]), i32([0, n]),
+                                    i32(tiles[0]), i32(tiles[1]), H, dk, dv, window, scale, dev(sink), **rot)
+        got = out.cpu().double().view(n, H, dv)
+        for h in range(H):
+            ref = O.sink_softmax(scale * (q[:, h].double() @ k[:, h].double().T), vis, sink[h].double()) @ v[:, h].double()
+            # weights and result in bf16, 2 ** -9 each, of values around 1
+            assert (got[:, h] - ref).abs().max() < 2e-2, (kr, h)
+
+
 # ---- the model through the engine -------------------------------------------------------------------------------------------
 @pytest.fixture(scope="module", params=list(CONFIGS))
 def model(request, tmp_path_factory):
