@@ -1806,26 +1806,34 @@ def group_norm_store(x: torch.Tensor, q_off: int, k_off: int, gain: torch.Tensor
                                                *temperature, _p(pos), _p(slots), T, _p(cache), _p(kscale), n * bs, bs, _stream()), "glm_group_norm_store")
 
 
+def _check_residual(x, wp: int, y, embed, g, rows, act_dtype) -> None:
+    """Operands of residual_norm: rows and types that the kernels rely on."""
+    assert x is None or (x.dtype == torch.float32 and x.is_contiguous() and x.shape[1] == wp)
+    if y is not None:
+        t = y.part if isinstance(y, PartialSum) else y
+        assert t.shape[-1] == wp and t.is_contiguous() and (x is None or t.shape[-2] == x.shape[0])
+    if embed is not None:
+        ids, table = embed
+        assert ids.dtype == torch.int64 and ids.is_contiguous() and table.stride(1) == 1 and table.shape[1] >= wp and table.dtype == act_dtype
+        assert x is None or ids.numel() == x.shape[0]
+    assert rows is None or rows.dtype == torch.int32
+    assert g is None or (g.dtype == torch.float32 and g.numel() == wp)
+
+
 def residual_norm(x: torch.Tensor | None, width: int, wp: int, eps: float, y=None, embed: tuple | None = None, g: torch.Tensor | None = None, rows: torch.Tensor | None = None,
                   act_dtype=torch.bfloat16, keep_x: bool = True):
     """Between two layers (glm_residual_norm): returns (x_out, h) with x_out = x + y + rows of an embedding table and h its norm with gain g (None: no
     h).  y: [T, wp] in bf16, fp32 or a PartialSum; embed: (ids, table); rows: gather of rows."""
     T = rows.numel() if rows is not None else (x.shape[0] if x is not None else embed[0].numel())
     dev = embed[1].device if x is None else x.device
-    assert x is None or (x.dtype == torch.float32 and x.is_contiguous() and x.shape[1] == wp)
+    _check_residual(x, wp, y, embed, g, rows, act_dtype)
     yp, ldy, y_f32, ns, sstride = None, wp, 0, 1, 0
     if y is not None:
         t = y.part if isinstance(y, PartialSum) else y
-        assert t.shape[-1] == wp and t.is_contiguous() and (x is None or t.shape[-2] == x.shape[0])
         yp, y_f32 = _p(t), _is_f32(t.dtype)
         if isinstance(y, PartialSum):
             ns, sstride = t.shape[0], t.shape[1] * t.shape[2]
     ids, table = embed or (None, None)
-    if embed is not None:
-        assert ids.dtype == torch.int64 and ids.is_contiguous() and table.stride(1) == 1 and table.shape[1] >= wp and table.dtype == act_dtype
-        assert x is None or ids.numel() == x.shape[0]
-    assert rows is None or rows.dtype == torch.int32
-    assert g is None or (g.dtype == torch.float32 and g.numel() == wp)
     x_out = torch.empty((T, wp), dtype=torch.float32, device=dev) if keep_x else None
     h = torch.empty((T, wp), dtype=act_dtype, device=dev) if g is not None else None
     _check(load_library().glm_residual_norm(_p(x), _p(rows), yp, ldy, y_f32, ns, sstride, _p(table), table.stride(0) if table is not None else wp,
@@ -1835,15 +1843,21 @@ def residual_norm(x: torch.Tensor | None, width: int, wp: int, eps: float, y=Non
 
 
 class NormedRow:
-    """The h of residual_norm for ONE row, formed inside the projection that reads it (glm_gemm_bf16_residual_norm): `linear` instead of linear_act.  x: the
-    residual, there once the projection has run."""
+    """The h of residual_norm for ONE row, formed inside the projection that reads it (glm_gemm_bf16_residual_norm): `linear` instead of linear_act."""
     shape, dtype = None, torch.bfloat16
 
     def __init__(self, x, width: int, wp: int, eps: float, y, embed, g, rows, keep_x: bool):
         self.device = g.device
         self.shape = torch.Size((1, wp))
-        self.x = torch.empty((1, wp), dtype=torch.float32, device=self.device) if keep_x else None
+        self.x_out = torch.empty((1, wp), dtype=torch.float32, device=self.device) if keep_x else None
+        self.formed = False
         self.args = (x, width, eps, y, embed, g, rows)
+
+    @property
+    def x(self) -> torch.Tensor | None:
+        """The residual, which the projection leaves (None: not kept)."""
+        assert self.formed or self.x_out is None, "the residual of a NormedRow is there once its projection has been called"
+        return self.x_out
 
     def linear(self, w: torch.Tensor, act=NO_ACT, out_f32: bool = False, out: torch.Tensor | None = None) -> torch.Tensor:
         x, width, eps, add, embed, g, rows = self.args
@@ -1853,8 +1867,9 @@ class NormedRow:
         out = torch.empty((1, N), dtype=dt, device=self.device) if out is None else out
         assert w.shape[1] == wp and w.dtype == self.dtype and w.stride(1) == 1 and out.shape == (1, N) and out.dtype == dt and out.stride(1) == 1
         _check(load_library().glm_gemm_bf16_residual_norm(
-            _p(x), _p(rows), _p(add), wp, _p(table), table.stride(0) if table is not None else wp, table.shape[0] if table is not None else 0, _p(ids), _p(self.x), _p(g),
+            _p(x), _p(rows), _p(add), wp, _p(table), table.stride(0) if table is not None else wp, table.shape[0] if table is not None else 0, _p(ids), _p(self.x_out), _p(g),
             width, wp, eps, _p(w), w.stride(0), _p(out), out.stride(0), N, int(out_f32), *act, _stream()), "glm_gemm_bf16_residual_norm")
+        self.formed = True
         return out
 
 
@@ -1862,18 +1877,15 @@ def normed_row(x, width: int, wp: int, eps: float, w: torch.Tensor, y=None, embe
                keep_x: bool = True) -> NormedRow | None:
     """NormedRow of residual_norm's arguments for a projection by w, or None: more than one row, other types, sizes that kernel does not take."""
     T = rows.numel() if rows is not None else (x.shape[0] if x is not None else embed[0].numel())
+    _check_residual(x, wp, y, embed, g, rows, w.dtype)
     if T != 1 or g is None or not 1024 < wp <= 4096 or w.dtype != torch.bfloat16 or w.shape[1] != wp or w.shape[0] % 4 or w.stride(0) % 8 or w.stride(1) != 1 or not opt("tinym"):
         return None
-    if y is not None and (not isinstance(y, torch.Tensor) or y.dtype != torch.bfloat16 or not y.is_contiguous() or y.shape[-1] != wp):
+    if y is not None and (not isinstance(y, torch.Tensor) or y.dtype != torch.bfloat16):
         return None
-    if embed is not None:
-        ids, table = embed
-        if table.dtype != torch.bfloat16 or table.stride(0) % 8 or table.stride(1) != 1 or table.shape[1] < wp or ids.dtype != torch.int64:
-            return None
+    if embed is not None and embed[1].stride(0) % 8:
+        return None
     if any(t is not None and t.data_ptr() % 16 for t in (x, y, embed[1] if embed else None, g, w)):
         return None
-    assert x is None or (x.dtype == torch.float32 and x.is_contiguous() and x.shape[1] == wp)
-    assert (rows is None or rows.dtype == torch.int32) and g.dtype == torch.float32 and g.numel() == wp
     return NormedRow(x, width, wp, eps, y, embed, g, rows, keep_x)
 
 

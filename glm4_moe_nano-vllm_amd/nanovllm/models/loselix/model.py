@@ -131,9 +131,12 @@ class LoselixForCausalLM(nn.Module):
         for (i, first_of_pass), r in zip(self.runs, self.run_index):
             layer, rot = self.layers[i], self.layers[i].mixer.rot
             kw = dict(g=layer.g, embed=(meta.ids, self.embed) if x is None or first_of_pass else None)
-            h = self.one_row(x, y, layer.block.in_proj.weight, **kw)
-            x, h = (h.x, h) if h is not None else norm(x, y, **kw)
-            y = layer.block(h, meta, r, rot.shared_table(meta.pos, tables) if rot is not None else None)
+            row = self.one_row(x, y, layer.block.in_proj.weight, **kw)
+            if row is None:
+                x, h = norm(x, y, **kw)
+            y = layer.block(h if row is None else row, meta, r, rot.shared_table(meta.pos, tables) if rot is not None else None)
+            if row is not None:
+                x = row.x
             if residual_tap is not None:
                 residual_tap.append(norm(x, y)[0][:, : cfg.hidden_size])
         if meta.want.numel() == 0:

@@ -240,3 +240,32 @@ def test_parts_that_do_not_go_together():
         with pytest.raises(ValueError, match="go together"):
             GroupAttention(32, 4, 2, 8, 8, 0.3, torch.bfloat16, joint=True, **bad)
     assert not GroupAttention(32, 4, 2, 8, 8, 0.3, torch.bfloat16, joint=True, cap=3.0).tiled and GroupAttention(32, 4, 2, 8, 8, 0.3, torch.bfloat16, joint=True, cap=3.0, diff=0.2).tiled
+
+
+# ---- what the launch between two layers checks ----------------------------------------------------------------------------------
+def test_operands_of_a_norm_in_its_projection():
+    """hip_ops.normed_row refuses what residual_norm refuses, and hands the residual out only once it has been formed."""
+    from nanovllm import hip_ops
+    T, wp, N = 5, 2048, 64
+    bf = torch.bfloat16
+    x, y, gain, w = torch.zeros(T, wp), torch.zeros(T, wp, dtype=bf), torch.ones(wp), torch.zeros(N, wp, dtype=bf)
+    ids, table, last = torch.arange(T), torch.zeros(7, wp, dtype=bf), torch.tensor([T - 1], dtype=torch.int32)
+    good = dict(y=y, embed=(ids, table), g=gain, rows=last)
+    bad = [dict(y=y[: T - 1]), dict(embed=(ids[: T - 1], table)), dict(embed=(torch.arange(2 * T)[::2], table)), dict(g=torch.ones(wp + 8)), dict(g=torch.ones(wp, dtype=D)),
+           dict(rows=torch.tensor([T - 1]))]
+    for change in bad:
+        args = dict(good, **change)
+        with pytest.raises(AssertionError):
+            hip_ops.residual_norm(x, wp, wp, 1e-5, **args)
+        with pytest.raises(AssertionError):
+            hip_ops.normed_row(x, wp, wp, 1e-5, w, **args)
+    for bad_x in (x.to(D), torch.zeros(T, wp + 8), torch.zeros(T, 2 * wp)[:, ::2]):
+        with pytest.raises(AssertionError):
+            hip_ops.normed_row(bad_x, wp, wp, 1e-5, w, **good)
+    row = hip_ops.normed_row(x, wp, wp, 1e-5, w, **good)
+    assert row.shape == (1, wp) and row.dtype == bf
+    with pytest.raises(AssertionError):
+        row.x
+    assert hip_ops.normed_row(x, wp, wp, 1e-5, w, keep_x=False, **good).x is None
+    f32 = dict(good, y=y.float(), embed=(ids, table.float()))
+    assert hip_ops.normed_row(x, wp, wp, 1e-5, w.float(), **f32) is None
