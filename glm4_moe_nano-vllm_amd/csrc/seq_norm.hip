@@ -15,6 +15,7 @@
 // the previous portion's.  Everything is fp32 up to the store of h, and a token's h is the same arithmetic whether it was
 // computed in this step or kept from an earlier one: cutting a sequence differently gives the same bits here.
 #include "common.h"
+#include <type_traits>
 
 namespace {
 
@@ -398,21 +399,21 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
 }
 
 // ---- some hundred rows and fewer, a row per workgroup: nothing but latency, so whatever does not depend on something else is requested first
-// (the row with its slabs, four of them at a time, gains and taps; then seq_of -> q_start -> state), and only then come the sums.  The rows in
-// front of it in its portion are formed as well, the arithmetic is the stream kernel's.  128 decoded rows of 2048 columns,
-// half of these launches behind slabs: there 7.1 us with four taps and 6.4 without (a slab's load waited for the one before, the state's for
-// both sums), here 6.7 and 5.3. ----
+// (the row with its slabs, four of them at a time, gains and taps; then seq_of -> q_start -> state), and only then come the sums.  Rows with
+// others of their portion in front of them form those as well, as the stream kernel does: the next row is requested in front of this one's sums, and the sum over
+// this x_out^2 and the one over the next y^2 share a barrier.  The arithmetic is the stream kernel's. ----
 template <int TAPS, int NT>
-__global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
+__global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm_row_kernel(const SeqNormArgs a) {
     constexpr int HALO = TAPS - 1, NW = NT / 64;
-    __shared__ float s_red[2][NW];
+    __shared__ float s_red[2][2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int c = tid * 8;
     const bool on = c < a.wp;
     const int64_t r0 = blockIdx.x;
     const float inv_w = 1.0f / (float)a.width;
     const Row8 zero = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    auto load_row = [&](int64_t r, Row8& x, Row8& y) {
+    auto load_row = [&](int64_t r, Row8& x, Row8& y, auto in_flight) {
+        constexpr int SF = decltype(in_flight)::value;  // slabs requested at a time
         x = y = zero;
         if (!on) return;
         const int64_t row = a.row_index ? a.row_index[r] : r;
@@ -426,12 +427,12 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
         }
         const float* p = reinterpret_cast<const float*>(a.y) + row * a.ldy + c;
         y = sn_ld8f(p);
-        for (int s0 = 1; s0 < a.n_slabs; s0 += 4) {  // (added up in their order)
-            Row8 v[4];
+        for (int s0 = 1; s0 < a.n_slabs; s0 += SF) {  // (added up in their order)
+            Row8 v[SF];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = sn_ld8f(p + (int64_t)min(s0 + i, a.n_slabs - 1) * a.slab_stride);
+            for (int i = 0; i < SF; ++i) v[i] = sn_ld8f(p + (int64_t)min(s0 + i, a.n_slabs - 1) * a.slab_stride);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < SF; ++i)
                 if (s0 + i < a.n_slabs) {
                     y.a += v[i].a;
                     y.b += v[i].b;
@@ -441,16 +442,26 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
     int par = 0;
     auto reduce = [&](float u) {
         u = sn_wave_sum(u);
-        if (lane == 63) s_red[par][wid] = u;
+        if (lane == 63) s_red[par][0][wid] = u;
         __syncthreads();
         float su = 0.f;
 #pragma unroll
-        for (int i = 0; i < NW; ++i) su += s_red[par][i];
+        for (int i = 0; i < NW; ++i) su += s_red[par][0][i];
         par ^= 1;
         return su;
     };
+    auto reduce2 = [&](float u, float v, float& sv) {
+        v = sn_wave_sum(v);
+        if (lane == 63) s_red[par][1][wid] = v;
+        const int at = par;
+        const float su = reduce(u);
+        sv = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) sv += s_red[at][1][i];
+        return su;
+    };
     Row8 x, y, gq = zero, gp = zero;
-    load_row(r0, x, y);
+    load_row(r0, x, y, std::integral_constant<int, 4>{});
     u32x4_t w[TAPS];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) w[j] = u32x4_t{0, 0, 0, 0};
@@ -463,17 +474,16 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    auto residual = [&](Row8& x, const Row8& y) {  // x_out
+    auto residual = [&](Row8& x, const Row8& y, float ry) {  // x_out
         if (!a.y) return;
-        const float ry = 1.0f / sqrtf(reduce(sn_sumsq8(y)) * inv_w + a.eps);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             x.a[i] = x.a[i] + y.a[i] * ry * gq.a[i];
             x.b[i] = x.b[i] + y.b[i] * ry * gq.b[i];
         }
     };
-    auto normed = [&](const Row8& x) {
-        const float rx = 1.0f / sqrtf(reduce(sn_sumsq8(x)) * inv_w + a.eps);
+    auto rms = [&](float su) { return 1.0f / sqrtf(su * inv_w + a.eps); };
+    auto normed = [&](const Row8& x, float rx) {
         Row8 h;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -482,12 +492,15 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
         }
         return h;
     };
-    Row8 hist[TAPS], up[TAPS];  // hist[k - 1]: h of k tokens ago; up: state rows that move up behind a portion shorter than the history
-    int n = 0, e = 0;           // tokens of the portion, and of them behind this row
+    Row8 hist[TAPS];       // hist[k - 1]: h of k tokens ago, in front of the portion as the state has it
+    int n = 0, e = 0, d = 0, p = 0;  // tokens of the portion, of them behind this row and (as far as the taps reach) in front of it; the row's position
     int64_t so = -1;
     bool keep = false;
+    float ry = 0.f;
     if constexpr (TAPS > 1) {
-        const int s = a.seq_of[r0], p = a.pos[r0], qs = a.q_start[s], qe = a.q_start[s + 1], d = (int)min(r0 - qs, (int64_t)HALO);
+        const int s = a.seq_of[r0], qs = a.q_start[s], qe = a.q_start[s + 1];
+        p = a.pos[r0];
+        d = (int)min(r0 - qs, (int64_t)HALO);
         const int64_t sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
         so = a.state_out[s];
         n = qe - qs;
@@ -496,40 +509,48 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
         const float* st = a.state + sin * HALO * a.wp + c;
 #pragma unroll
         for (int k = 1; k < TAPS; ++k) {
-            hist[k - 1] = up[k - 1] = zero;
-            if (on && a.g_pre && k > d && p - k >= 0) hist[k - 1] = sn_ld8f(st + (int64_t)(HALO - k + d) * a.wp);
-            if (keep && a.g_pre && e == 0 && k + n <= HALO) up[k - 1] = sn_ld8f(st + (int64_t)(k - 1 + n) * a.wp);
+            hist[k - 1] = zero;
+            if (on && r0 - d == qs) hist[k - 1] = sn_ld8f(st + (int64_t)(HALO - k) * a.wp);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (a.g_pre)
+        if (d > 0) {  // (uniform; this row comes again, out of the cache)
+            Row8 xn, yn;
+            float sv;
+            load_row(r0 - d, x, y, std::integral_constant<int, 2>{});
+            if (a.y) ry = rms(reduce(sn_sumsq8(y)));
             for (int64_t q = r0 - d; q < r0; ++q) {
-                Row8 xq, yq;
-                load_row(q, xq, yq);
-                residual(xq, yq);
-                const Row8 h = normed(xq);
+                load_row(q + 1, xn, yn, std::integral_constant<int, 2>{});
+                residual(x, y, ry);
+                const float rx = rms(reduce2(sn_sumsq8(x), sn_sumsq8(yn), sv));
 #pragma unroll
-                for (int k = 1; k < TAPS; ++k)
-                    if (r0 - q == k) hist[k - 1] = h;
+                for (int k = HALO; k >= 2; --k) hist[k - 1] = hist[k - 2];
+                hist[0] = normed(x, rx);
+                ry = rms(sv);
+                x = xn;
+                y = yn;
             }
+        }
     }
-    residual(x, y);
+    if (a.y && d == 0) ry = rms(reduce(sn_sumsq8(y)));
+    residual(x, y, ry);
     if (on) {
         if (a.x_out) sn_st8f(a.x_out + r0 * a.ldx + c, x);
         if (a.x_cast) sn_st8(a.x_cast, r0 * a.ldc + c, a.act_f32, x);
     }
     if (!a.g_pre) return;
-    const Row8 h = normed(x);
+    const Row8 h = normed(x, rms(reduce(sn_sumsq8(x))));
     Row8 o = h;
     if constexpr (TAPS > 1) {
         auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
         Row8 acc = zero;
 #pragma unroll
-        for (int k = HALO; k >= 1; --k)
+        for (int k = HALO; k >= 1; --k) {
+            const bool there = k <= d || p - k >= 0;  // (in front of the sequence the state holds nothing)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * hist[k - 1].a[i];
-                acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * hist[k - 1].b[i];
+                acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * (there ? hist[k - 1].a[i] : 0.f);
+                acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * (there ? hist[k - 1].b[i] : 0.f);
             }
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
@@ -538,16 +559,17 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
         if (keep) {
             float* to = a.state + so * HALO * a.wp + c;
             sn_st8f(to + (int64_t)(HALO - 1 - e) * a.wp, h);
+            // a portion shorter than the history, whose rows are n = d + 1 with the last one: the older inputs move up
 #pragma unroll
-            for (int k = 1; k < TAPS; ++k)
-                if (e == 0 && k + n <= HALO) sn_st8f(to + (int64_t)(k - 1) * a.wp, up[k - 1]);
+            for (int k = 1; k < HALO; ++k)
+                if (e == 0 && k + n <= HALO) sn_st8f(to + (int64_t)(k - 1) * a.wp, hist[HALO - k - 1]);
         }
     }
     if (on) sn_st8(a.h, r0 * a.ldh + c, a.act_f32, o);
 }
 
 template <int TAPS, int NT>
-int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
+int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) {
     // decode: seq_norm_row_kernel; else runs of rows long enough to spread the halo and the register setup, short enough
     // to fill the chip: a row is a chain of one load, two reductions and a store, with one row's loads in flight per workgroup, so some hundred rows
     // stay one to a workgroup, re-reading the halo, as long as those are no more than four waves a SIMD (2048 workgroups of 64 threads: two), and
@@ -556,7 +578,12 @@ int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
     // 95 / 83; 2048 workgroups 78 where 1024 took 75).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
     if constexpr (NT < 1024 || TAPS == 1) {  // (1024 threads do not have the registers for rows, taps and history at once)
-        if (a.T <= 512) {
+        // With taps: portions of one row, up to three quarters of the CUs.  Longer ones take the stream kernel, which knows where a portion begins before it
+        // asks for a row; with a row per CU and more there is less to hide.  Stream / row kernel, four taps, us: two slabs of 2048 columns, 1 row 4.87 /
+        // 4.68, 32 5.23 / 5.05, 128 6.26 / 6.27, 200 7.10 / 7.08, 256 7.52 / 7.62, four slabs 1 5.36 / 4.78, 128 7.25 / 6.96; two of 4096, 1 5.88 / 5.17, 128 8.56 /
+        // 7.91, 256 10.63 / 10.40; prompts of 64, 211 and 512 tokens, two slabs of 2048, 8.8 / 9.3, 9.9 / 10.3, 14.6 / 15.5, without the pipeline of the rows in
+        // front 10.3, 11.0, 15.2.  No taps: 2048 columns, 1 row 3.74 / 3.54, 512 6.79 / 6.32.
+        if (TAPS == 1 ? a.T <= 512 : a.T <= 192 && (n_seq <= 0 || n_seq >= a.T)) {
             hipLaunchKernelGGL((seq_norm_row_kernel<TAPS, NT>), dim3((unsigned)a.T), dim3(NT), 0, st, a);
             GLM_CHECK_LAUNCH("glm_seq_norm");
             return GLM_OK;
@@ -570,13 +597,13 @@ int launch_seq_norm_stream(const SeqNormArgs& a, hipStream_t st) {
 }
 
 template <int TAPS>
-int launch_seq_norm(const SeqNormArgs& a, hipStream_t st) {
+int launch_seq_norm(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) {
     if constexpr (TAPS <= 8) {
-        if (a.wp <= 512) return launch_seq_norm_stream<TAPS, 64>(a, st);
-        if (a.wp <= 1024) return launch_seq_norm_stream<TAPS, 128>(a, st);
-        if (a.wp <= 2048) return launch_seq_norm_stream<TAPS, 256>(a, st);
-        if (a.wp <= 4096) return launch_seq_norm_stream<TAPS, 512>(a, st);
-        if (TAPS <= 4 && a.wp <= 8192) return launch_seq_norm_stream<TAPS, (TAPS <= 4 ? 1024 : 512)>(a, st);
+        if (a.wp <= 512) return launch_seq_norm_stream<TAPS, 64>(a, n_seq, st);
+        if (a.wp <= 1024) return launch_seq_norm_stream<TAPS, 128>(a, n_seq, st);
+        if (a.wp <= 2048) return launch_seq_norm_stream<TAPS, 256>(a, n_seq, st);
+        if (a.wp <= 4096) return launch_seq_norm_stream<TAPS, 512>(a, n_seq, st);
+        if (TAPS <= 4 && a.wp <= 8192) return launch_seq_norm_stream<TAPS, (TAPS <= 4 ? 1024 : 512)>(a, n_seq, st);
     }
     // few rows (decode): one row per workgroup; many: 16 rows share a halo
     if (a.T <= 512) hipLaunchKernelGGL((seq_norm_kernel<TAPS, 1>), dim3((unsigned)a.T), dim3(SN_NT), 0, st, a);
@@ -633,11 +660,12 @@ extern "C" int glm_seq_norm_taps(int taps) {
     return -1;
 }
 
-extern "C" int glm_seq_norm(const float* x_in, const int32_t* row_index, int64_t ldx, float* x_out, void* x_cast, int64_t ldc,
+extern "C" int glm_seq_norm_step(const float* x_in, const int32_t* row_index, int64_t ldx, float* x_out, void* x_cast, int64_t ldc,
                             const void* y, int64_t ldy, int y_f32, int n_slabs, int64_t slab_stride, const float* g_post,
                             const float* g_pre, const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos,
                             const int32_t* seq_of, const int32_t* q_start, const int32_t* state_in, const int32_t* state_out,
-                            void* h, int64_t ldh, int act_f32, int64_t T, int width, int wp, float eps, glm_stream_t stream) {
+                            void* h, int64_t ldh, int act_f32, int64_t T, int64_t n_seq, int width, int wp, float eps,
+                                 glm_stream_t stream) {
     GLM_CHECK_ARG(x_in && T >= 0 && width > 0 && wp >= width && wp % 8 == 0 && ldx >= wp && ldx % 4 == 0, GLM_ERR_INVALID,
                   "glm_seq_norm: bad shape T=%ld width=%d wp=%d ldx=%ld", (long)T, width, wp, (long)ldx);
     GLM_CHECK_ARG(!y || (g_post && ldy >= wp && ldy % 4 == 0 && n_slabs >= 1 && (y_f32 || n_slabs == 1)), GLM_ERR_INVALID,
@@ -653,15 +681,24 @@ extern "C" int glm_seq_norm(const float* x_in, const int32_t* row_index, int64_t
                      pos, seq_of, q_start, state_in, state_out, n_state, h, ldh, act_f32, T, width, wp, eps};
     hipStream_t st = glm_s(stream);
     switch (taps) {
-        case 1: return launch_seq_norm<1>(a, st);
-        case 2: return launch_seq_norm<2>(a, st);
-        case 3: return launch_seq_norm<3>(a, st);
-        case 4: return launch_seq_norm<4>(a, st);
-        case 6: return launch_seq_norm<6>(a, st);
-        case 8: return launch_seq_norm<8>(a, st);
-        case 16: return launch_seq_norm<16>(a, st);
-        default: return launch_seq_norm<32>(a, st);
+        case 1: return launch_seq_norm<1>(a, n_seq, st);
+        case 2: return launch_seq_norm<2>(a, n_seq, st);
+        case 3: return launch_seq_norm<3>(a, n_seq, st);
+        case 4: return launch_seq_norm<4>(a, n_seq, st);
+        case 6: return launch_seq_norm<6>(a, n_seq, st);
+        case 8: return launch_seq_norm<8>(a, n_seq, st);
+        case 16: return launch_seq_norm<16>(a, n_seq, st);
+        default: return launch_seq_norm<32>(a, n_seq, st);
     }
+}
+
+extern "C" int glm_seq_norm(const float* x_in, const int32_t* row_index, int64_t ldx, float* x_out, void* x_cast, int64_t ldc,
+                            const void* y, int64_t ldy, int y_f32, int n_slabs, int64_t slab_stride, const float* g_post,
+                            const float* g_pre, const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos,
+                            const int32_t* seq_of, const int32_t* q_start, const int32_t* state_in, const int32_t* state_out,
+                            void* h, int64_t ldh, int act_f32, int64_t T, int width, int wp, float eps, glm_stream_t stream) {
+    return glm_seq_norm_step(x_in, row_index, ldx, x_out, x_cast, ldc, y, ldy, y_f32, n_slabs, slab_stride, g_post, g_pre, conv_w, taps, state, n_state, pos, seq_of, q_start, state_in,
+                             state_out, h, ldh, act_f32, T, 0, width, wp, eps, stream);
 }
 
 extern "C" int glm_embed_rows(const int64_t* ids, const void* table, int64_t ldw, int64_t vocab, const int32_t* pos, const double* freq,

@@ -146,6 +146,9 @@ _SIGNATURES = {
     "glm_seq_norm": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int,
         c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
         c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_int, c_float, c_void_p]),
+    "glm_seq_norm_step": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int, c_int,
+        c_int64, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
+        c_void_p, c_void_p, c_int64, c_int, c_int64, c_int64, c_int, c_int, c_float, c_void_p]),
     "glm_embed_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,
         c_int64, c_int, c_int, c_float, c_void_p]),
     "glm_gemm_bf16_residual_norm": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float,
@@ -1420,11 +1423,11 @@ def seq_norm(x: torch.Tensor, width: int, eps: float, y=None, g_post: torch.Tens
     for g in (g_post, g_pre):
         assert g is None or (g.dtype == torch.float32 and g.is_contiguous() and g.numel() == wp)
     assert x_cast is None or (x_cast.dtype == act_dtype and x_cast.stride(1) == 1 and x_cast.shape[0] == T)
-    _check(load_library().glm_seq_norm(
+    _check(load_library().glm_seq_norm_step(
         _p(x), _p(rows), wp, _p(x_out), _p(x_cast), x_cast.stride(0) if x_cast is not None else wp, yp, ldy, y_f32, ns, sstride,
         _p(g_post) if y is not None else None, _p(g_pre), _p(w) if taps > 1 else None, taps, _p(st) if taps > 1 else None, n_state,
-        _p(pos), _p(seq_of), _p(q_start), _p(s_in), _p(s_out), _p(h), wp, _is_f32(act_dtype), T, width, wp, eps, _stream()),
-        "glm_seq_norm")
+        _p(pos), _p(seq_of), _p(q_start), _p(s_in), _p(s_out), _p(h), wp, _is_f32(act_dtype), T, q_start.numel() - 1 if taps > 1 else 0,
+        width, wp, eps, _stream()), "glm_seq_norm_step")
     return (x if x_out is None else x_out), h
 
 

@@ -533,6 +533,12 @@ int glm_seq_norm(const float* x_in, const int32_t* row_index, int64_t ldx, float
                  const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of,
                  const int32_t* q_start, const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32,
                  int64_t T, int width, int wp, float eps, glm_stream_t stream);
+/* the same with the number of sequences (entries of q_start less one; 0: not known): as many as rows, and every portion is one row */
+int glm_seq_norm_step(const float* x_in, const int32_t* row_index, int64_t ldx, float* x_out, void* x_cast, int64_t ldc, const void* y,
+                 int64_t ldy, int y_f32, int n_slabs, int64_t slab_stride, const float* g_post, const float* g_pre,
+                 const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of,
+                 const int32_t* q_start, const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32,
+                 int64_t T, int64_t n_seq, int width, int wp, float eps, glm_stream_t stream);
 /* embedding rows as the fp32 residual and, optionally, in the activation dtype; columns [width, wp) are zeros.  freq [width / 2 rounded
  * up] (double, or NULL) with pos [T]: sin(pos freq[i]) is added at column 2i, cos(pos freq[i]) at column 2i + 1; the table's rows are
  * multiplied by scale                                                                                                       */

@@ -118,6 +118,38 @@ def test_seq_norm(width, taps, y_kind):
             assert torch.allclose(o[s], outs[0][s][: o[s].shape[0]], rtol=1e-6, atol=2e-6)
 
 
+@pytest.mark.parametrize("width,taps", [(72, 2), (520, 3), (1032, 4), (2056, 6), (4096, 8), (4104, 4)])
+@pytest.mark.parametrize("lens", [[1] * 192, [1] * 193, [3, 1, 2, 5, 8, 1], [130, 1, 2, 59], [2, 0, 1]])
+def test_seq_norm_is_one_launch_whatever_the_portions(width, taps, lens, monkeypatch):
+    """The launch is chosen by what is known of the portions: rows, stream and state of all of them have the same bits."""
+    from nanovllm import hip_ops
+    wp, T, S = hip_ops.round8(width), sum(lens), len(lens)
+    lib = hip_ops.load_library()
+    start = [0, 1, 2, 40]   # (portions at the sequence's start need less of the state)
+    pos = i32([start[s % 4] + p for s, n in enumerate(lens) for p in range(n)])
+    meta = types.SimpleNamespace(pos=pos, seq_of=i32([s for s, n in enumerate(lens) for _ in range(n)]), q_start=i32([sum(lens[:s]) for s in range(S + 1)]),
+                                 state_in=i32(list(range(S))), state_out=i32([S + s if s % 5 != 4 else -1 for s in range(S)]))
+    x, gain, conv = torch.randn(T, wp, device="cuda"), torch.randn(wp, device="cuda"), torch.randn(taps, wp, device="cuda").bfloat16()
+    state = torch.randn(2 * S, taps - 1, wp, device="cuda")
+    for y in (hip_ops.PartialSum(torch.randn(2, T, wp, device="cuda")), torch.randn(T, wp, device="cuda").bfloat16(), hip_ops.PartialSum(torch.randn(7, T, wp, device="cuda"))):
+        got = []
+        for n_seq in (None, 0, max(1, T - 1)):
+
+            class Library:
+                def __getattr__(self, name):
+                    return getattr(lib, name)
+
+                def glm_seq_norm_step(self, *a):
+                    return lib.glm_seq_norm_step(*a[:26], n_seq if n_seq is not None else a[26], *a[27:])
+
+            monkeypatch.setattr(hip_ops, "load_library", Library)
+            kept = state.clone()
+            got.append(hip_ops.seq_norm(x, width, 1e-5, y=y, g_post=gain, g_pre=gain, conv=(conv, kept), meta=meta) + (kept,))
+            monkeypatch.undo()
+        for other in got[1:]:
+            assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+
+
 @pytest.mark.parametrize("n", [1, 3, 5, 6, 9, 16])
 @pytest.mark.parametrize("T,width", [(1, 64), (7, 2048), (512, 520), (513, 520)])
 def test_seq_norm_adds_slabs_in_their_order(n, T, width):
