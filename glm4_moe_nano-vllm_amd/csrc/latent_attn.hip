@@ -280,6 +280,57 @@ struct AttnArgs {
     float* part_ml;           // [Ta * H, nsplit, 2] running maximum (log2 units), mass
 };
 
+// The query rows and the keys of a workgroup.
+struct LaWork {
+    int split, h0, hb, tok0, p0, p1, seq, nrows;  // split of the keys, heads, first token; positions of the first and the last row, their sequence, rows
+    int first, lo, t0, t1, n;                     // first visible key; 64-key tiles t0 .. t1 - 1 from position lo, n of them
+};
+
+// false: nothing to do (an empty split or an unused row has left its marks)
+template <int NT>
+__device__ __forceinline__ bool la_work(const AttnArgs& a, LaWork& k) {
+    const int tid = threadIdx.x;
+    int id = blockIdx.x;
+    k.split = id % a.nsplit;
+    id /= a.nsplit;
+    const int hg = id % a.n_hg, tile = id / a.n_hg;
+    k.h0 = hg * a.hb;
+    k.hb = min(a.hb, a.H - k.h0);
+    // (decoding, tile i is row i: its position and sequence are requested beside the tile, and again where it is another row)
+    const int guess = (int)min((int64_t)tile, a.Ta - 1);
+    k.tok0 = a.tile_tok[tile];
+    const int ntok = min(a.tile_n[tile], a.tq);
+    k.p0 = a.pos[guess];
+    k.seq = a.seq_of[guess];
+    if (k.tok0 < 0 || k.tok0 >= a.Ta || ntok <= 0) return false;
+    if (k.tok0 != guess) {
+        k.p0 = a.pos[k.tok0];
+        k.seq = a.seq_of[k.tok0];
+    }
+    k.p1 = k.p0 + ntok - 1;
+    k.nrows = ntok * k.hb;
+    // tiles start at multiples of 64: a tile lies in one cache block (its halves in one each, with blocks of 32); what is in front
+    // of the first visible key or behind the last row's comes from the zero page
+    k.first = max(0, k.p0 - a.window + 1);
+    k.lo = k.first & ~63;
+    const int ntile = k.p0 < 0 ? 0 : (k.p1 - k.lo + 64) >> 6;  // 64-key tiles of the whole range
+    const int per = (ntile + a.nsplit - 1) / a.nsplit;
+    k.t0 = k.split * per;
+    k.t1 = min(k.t0 + per, ntile);
+    k.n = k.t1 - k.t0;
+    if (k.n > 0) return true;
+    for (int r = tid; r < k.nrows; r += NT) {  // no mass
+        const int64_t gr = (int64_t)(k.tok0 + r / k.hb) * a.H + k.h0 + r % k.hb;
+        if (a.nsplit > 1) {
+            a.part_ml[(gr * a.nsplit + k.split) * 2] = -INFINITY;
+            a.part_ml[(gr * a.nsplit + k.split) * 2 + 1] = 0.f;
+        } else {
+            for (int d = 0; d < a.vp; ++d) a.ctx[gr * a.vp + d] = 0;
+        }
+    }
+    return false;
+}
+
 // One wave per (16-row query tile, 16-key quarter of a 64-key tile): it computes those scores over the whole latent, their
 // weights, and hands them over through LDS; then the waves divide the latent's columns among themselves for O^T += C^T . P^T.
 template <int NCT, int MT>
@@ -294,43 +345,16 @@ struct LaCfg {
 };
 
 template <int NCT, int MT>
-__global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs a) {
+__device__ __forceinline__ void latent_tiles(const AttnArgs& a, const LaWork& k, char* smem) {
     using C = LaCfg<NCT, MT>;
     constexpr int RPAD = NCT * 64, ROWB = RPAD * 2, TILEB = C::TILEB, CPR = RPAD / 8, NST = C::NST, NW = C::NW, DPW = C::DPW, NT = C::NT;
     constexpr int KS = 2 * NCT, NDMA = 8 * NCT, DMAW = (NDMA + NW - 1) / NW;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int kt = w & 3, mw = w >> 2;  // key quarter and row tile of this wave's scores
-    int id = blockIdx.x;
-    const int split = id % a.nsplit;
-    id /= a.nsplit;
-    const int hg = id % a.n_hg, tile = id / a.n_hg;
-    const int h0 = hg * a.hb, hb = min(a.hb, a.H - h0);
-    const int tok0 = a.tile_tok[tile];
-    const int ntok = min(a.tile_n[tile], a.tq);
-    if (tok0 < 0 || tok0 >= a.Ta || ntok <= 0) return;
-    const int p0 = a.pos[tok0], p1 = p0 + ntok - 1, seq = a.seq_of[tok0];
-    const int nrows = ntok * hb;
-    // tiles start at multiples of 64: a tile lies in one cache block (its halves in one each, with blocks of 32); what is in front
-    // of the first visible key or behind the last row's comes from the zero page
-    const int first = max(0, p0 - a.window + 1), lo = first & ~63;
-    const int ntile = p0 < 0 ? 0 : (p1 - lo + 64) >> 6;  // 64-key tiles of the whole range
-    const int per = (ntile + a.nsplit - 1) / a.nsplit;
-    const int t0 = split * per, t1 = min(t0 + per, ntile), n = t1 - t0;
-    if (n <= 0) {  // an empty split (or an unused row): no mass
-        for (int r = tid; r < nrows; r += NT) {
-            const int64_t gr = (int64_t)(tok0 + r / hb) * a.H + h0 + r % hb;
-            if (a.nsplit > 1) {
-                a.part_ml[(gr * a.nsplit + split) * 2] = -INFINITY;
-                a.part_ml[(gr * a.nsplit + split) * 2 + 1] = 0.f;
-            } else {
-                for (int d = 0; d < a.vp; ++d) a.ctx[gr * a.vp + d] = 0;
-            }
-        }
-        return;
-    }
+    const int split = k.split, h0 = k.h0, hb = k.hb, tok0 = k.tok0, p0 = k.p0, p1 = k.p1, seq = k.seq, nrows = k.nrows;
+    const int first = k.first, lo = k.lo, t0 = k.t0, t1 = k.t1, n = k.n;
     const int bmask = (1 << a.bs_shift) - 1;
     const int klo = lo + t0 * 64;                 // first key of this split
     const int khi = min(p1, lo + t1 * 64 - 1);    // last key of this split
@@ -410,11 +434,20 @@ __global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs
     const float sc = a.scale * LOG2E;
 #pragma unroll
     for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[i]));  // landed before the DMAs are counted
-    issue(0);
-    for (int it = 0; it < n; ++it) {
-        wait_vm<0>();
-        __builtin_amdgcn_s_barrier();
-        if (NST == 2 && it + 1 < n) issue(it + 1);
+    // (one place where tiles are requested: latent_keys_kernel holds two bodies, 40 to 60 KB of code)
+    for (int it = NST == 2 ? -1 : 0; it < n; ++it) {
+        if (NST == 1) {
+            if (it > 0) __builtin_amdgcn_s_barrier();
+            issue(it);
+        }
+        if (it >= 0) {
+            wait_vm<0>();
+            __builtin_amdgcn_s_barrier();
+        }
+        if (NST == 2) {
+            if (it + 1 < n) issue(it + 1);
+            if (it < 0) continue;
+        }
         if (tid == 0) asm volatile("ds_write_b32 %0, %1" ::"v"(f_addr + ((it + 1) & 1) * 4), "v"(0) : "memory");
         const unsigned st = base + (NST == 2 ? (it & 1) * TILEB : 0);
         // ---- scores of 16 keys x 16 rows over the whole latent, two accumulation chains ----
@@ -520,10 +553,6 @@ __global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs
                 }
             });
         }
-        if (NST == 1 && it + 1 < n) {
-            __builtin_amdgcn_s_barrier();
-            issue(it + 1);
-        }
     }
     // ---- masses of the four key quarters meet in LDS ----
     l_own += __shfl_xor(l_own, 16, 64);
@@ -567,81 +596,54 @@ __global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs
     }
 }
 
-// Up to 32 query rows and more than a few keys: the waves divide the keys, 16 at a time, and nothing passes between them before the end.  A wave
+template <int NCT, int MT>
+__global__ __launch_bounds__(64 * 4 * MT) void latent_attn_kernel(const AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LaWork k;
+    if (la_work<64 * 4 * MT>(a, k)) latent_tiles<NCT, MT>(a, k, smem);
+}
+
+// Up to 16 query rows and more than a few keys: the waves divide the keys, 16 at a time, and nothing passes between them before the end.  A wave
 // has its own ring of NST stages of 16 keys (counted vmcnt, no barrier), forms the scores of all rows over the whole latent, keeps the weights in
 // the registers they come out in (a 16 x 16 result is the operand of the K = 16 product) and adds up all value columns; the waves' sums meet in
-// LDS.  latent_attn_kernel's tile is a chain of two barriers, weights through LDS and fragment reads that its next tile's bytes wait for; here
-// what bounds a long range is HBM (5.5 TB/s where 200 of 256 CUs have work), a short one the loads in front of the first key and the ends.
-// Together with the launch behind it, us, there / here: 128 sequences of 1024 keys, 16 heads over 256 columns, two splits 28.0 / 24.3; 100 of
-// 2250 to 3000 keys, 16 heads over 576, 512 of them values, two splits 75.4 / 66.6, one split 118 / 86, 33 of these 39.2 / 39.4; two 64-key tiles
-// per split, 8 sequences, 25.2 / 27.5.
-template <int NCT, int VCT, int MT>
+// LDS.  latent_tiles' step is a chain of two barriers, weights through LDS and fragment reads that its next tile's bytes wait for; here
+// what bounds a long range is HBM (5.5 TB/s where 200 of 256 CUs have work), a short one the loads in front of the first key and the ends.  Tiles / keys, us, 16
+// heads: 33 sequences, 576 columns, 512 of them values, one split of 128 keys 13.3 / 14.4, 256 17.8 / 18.2, 384 22.2 / 21.1, 1024 43.6 / 35.5, 4096 147 / 102; 64
+// sequences, 512 columns, two splits, 256 keys 13.4 / 14.2, 512 18.0 / 17.6, 1024 26.1 / 23.1, 4096 75.9 / 55.9; 128 sequences, 256 columns, one split, 256
+// 12.3 / 12.4, 512 17.8 / 15.6, 1024 28.5 / 22.3, two splits (a workgroup on every CU) 512 13.0 / 14.0, 768 16.2 / 16.6, 1024 19.1 / 18.0.  32 rows (two row tiles, 32
+// heads over 256 columns): behind everywhere, 64 sequences of 4096 86 / 90, of 1024 28 / 31.
+constexpr int LK_TILES = 6;   // 64-key tiles of a range from which the waves divide the keys
+
+template <int NCT, int VCT>
 struct LkCfg {
     static constexpr int STAGEB = 16 * NCT * 128;
     static constexpr int NST = 144 * 1024 / (4 * STAGEB) < 4 ? 144 * 1024 / (4 * STAGEB) : 4;
-    static constexpr int WAVEB = NST * STAGEB, LDS = 4 * WAVEB + 4 * MT * 128;
+    static constexpr int WAVEB = NST * STAGEB, OWN = 4 * WAVEB + 4 * 128, LDS = OWN > LaCfg<NCT, 1>::LDS ? OWN : LaCfg<NCT, 1>::LDS;
     static_assert(NST >= 2 && VCT * 4096 <= WAVEB && LDS <= 160 * 1024, "two stages, and a wave's sums of 16 rows in their place");
 };
 
-template <int NCT, int VCT, int MT>
-__global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
-    using C = LkCfg<NCT, VCT, MT>;
+template <int NCT, int VCT>
+__device__ __forceinline__ void latent_keys(const AttnArgs& a, const LaWork& k, char* smem) {
+    using C = LkCfg<NCT, VCT>;
     constexpr int RPAD = NCT * 64, ROWB = RPAD * 2, CPR = RPAD / 8, KS = 2 * NCT, P = 2 * NCT, ND = 4 * VCT, NST = C::NST;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    int id = blockIdx.x;
-    const int split = id % a.nsplit;
-    id /= a.nsplit;
-    const int hg = id % a.n_hg, tile = id / a.n_hg;
-    const int h0 = hg * a.hb, hb = min(a.hb, a.H - h0);
-    // (decoding, tile i is row i: its position and sequence are requested beside the tile, and again where it is another row)
-    const int guess = (int)min((int64_t)tile, a.Ta - 1);
-    const int tok0 = a.tile_tok[tile];
-    const int ntok = min(a.tile_n[tile], a.tq);
-    int p0 = a.pos[guess], seq = a.seq_of[guess];
-    if (tok0 < 0 || tok0 >= a.Ta || ntok <= 0) return;
-    if (tok0 != guess) {
-        p0 = a.pos[tok0];
-        seq = a.seq_of[tok0];
-    }
-    const int p1 = p0 + ntok - 1;
-    const int nrows = ntok * hb;
-    const int first = max(0, p0 - a.window + 1), lo = first & ~63;
-    const int ntile = p0 < 0 ? 0 : (p1 - lo + 64) >> 6;  // 64-key tiles of the whole range
-    const int per = (ntile + a.nsplit - 1) / a.nsplit;
-    const int t0 = split * per, t1 = min(t0 + per, ntile), n = t1 - t0;
-    if (n <= 0) {  // an empty split (or an unused row): no mass
-        for (int r = threadIdx.x; r < nrows; r += 256) {
-            const int64_t gr = (int64_t)(tok0 + r / hb) * a.H + h0 + r % hb;
-            if (a.nsplit > 1) {
-                a.part_ml[(gr * a.nsplit + split) * 2] = -INFINITY;
-                a.part_ml[(gr * a.nsplit + split) * 2 + 1] = 0.f;
-            } else {
-                for (int d = 0; d < a.vp; ++d) a.ctx[gr * a.vp + d] = 0;
-            }
-        }
-        return;
-    }
+    const int split = k.split, h0 = k.h0, hb = k.hb, tok0 = k.tok0, p0 = k.p0, p1 = k.p1, seq = k.seq, nrows = k.nrows;
+    const int first = k.first, lo = k.lo, t0 = k.t0, t1 = k.t1, n = k.n;
     const int bmask = (1 << a.bs_shift) - 1;
     const int klo = lo + t0 * 64, khi = min(p1, lo + t1 * 64 - 1);  // keys of this split
     const int blk0 = klo >> a.bs_shift, nblk = (khi >> a.bs_shift) - blk0 + 1;
     // the query rows, requested beside the block table
-    u32x4_t qf[MT][KS];
-    int rpos[MT];
+    const bool own = c < nrows;
+    const int rpos = own ? p0 + c / hb : -1;
+    const int64_t gr = (int64_t)(tok0 + (own ? c / hb : 0)) * a.H + h0 + (own ? c % hb : 0);
+    u32x4_t qf[KS];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int r = 16 * m + c;
-        const bool own = r < nrows;
-        rpos[m] = own ? p0 + r / hb : -1;
-        const bf16_t* q = reinterpret_cast<const bf16_t*>(a.qa) + ((int64_t)(tok0 + (own ? r / hb : 0)) * a.H + h0 + (own ? r % hb : 0)) * a.rp;
-#pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            const int k = 32 * i + 8 * g;
-            qf[m][i] = u32x4_t{0, 0, 0, 0};
-            if (own && k < a.rp) qf[m][i] = *reinterpret_cast<const u32x4_t*>(q + k);
-        }
+    for (int i = 0; i < KS; ++i) {
+        const int col = 32 * i + 8 * g;
+        qf[i] = u32x4_t{0, 0, 0, 0};
+        if (own && col < a.rp) qf[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const bf16_t*>(a.qa) + gr * a.rp + col);
     }
     // 64 entries of the block table, one per lane (entries in front of the window may have been given back, -1: no key of theirs is fetched)
     int bt0 = 0, bt_v;
@@ -653,12 +655,16 @@ __global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
     load_bt(0);
     // per-lane source offsets (bytes) of a stage's pieces
     unsigned off[P];
-    int orow[P];
     const bool padded = RPAD != a.rp;
+    auto piece_of = [&](int lane, int i, int& row, int& ch) {
+        const int q = i * 64 + lane;
+        row = q / CPR;
+        ch = (q % CPR) ^ attn_swz(row);
+    };
 #pragma unroll
     for (int i = 0; i < P; ++i) {
-        const int q = i * 64 + lane, row = q / CPR, ch = (q % CPR) ^ attn_swz(row);
-        orow[i] = (padded && ch * 8 >= a.rp) ? 1 << 30 : row;
+        int row, ch;
+        piece_of(lane, i, row, ch);
         off[i] = (unsigned)(row * a.rp + ch * 8) * 2u;
     }
     char* const ring = smem + w * C::WAVEB;
@@ -674,26 +680,22 @@ __global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
 #pragma unroll
             for (int i = 0; i < P; ++i) lds_dma16<2>(src + off[i], st + i * 1024);
         } else {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // (rows and columns worked out here and now: kept over the stages, they cost the loop its registers)
 #pragma unroll
-            for (int i = 0; i < P; ++i) lds_dma16<2>(orow[i] <= left && orow[i] >= skip ? (const void*)(src + off[i]) : (const void*)la_zero_page, st + i * 1024);
+            for (int i = 0; i < P; ++i) {
+                int row, ch;
+                piece_of(ln, i, row, ch);
+                lds_dma16<2>(ch * 8 < a.rp && row <= left && row >= skip ? (const void*)(src + off[i]) : (const void*)la_zero_page, st + i * 1024);
+            }
         }
     };
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[i]));  // landed before the stages are counted
+    f32x4_t acc[ND];
+    float m_run = -INFINITY, l_run = 0.f;
 #pragma unroll
-        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qf[m][i]));  // landed before the stages are counted
-#pragma unroll
-    for (int s = 0; s < NST; ++s)
-        if (s < n) issue(s, s);
-    f32x4_t acc[MT][ND];
-    float m_run[MT], l_run[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        m_run[m] = -INFINITY;
-        l_run[m] = 0.f;
-#pragma unroll
-        for (int d = 0; d < ND; ++d) acc[m][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int d = 0; d < ND; ++d) acc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const unsigned base = lds_addr(ring);
     unsigned k_rel[2], v_rel[4];  // K row c, chunk 4 i + g; V row 4 g + qq, column tile d (parts of either depend on the parity of i / d & 3 only)
 #pragma unroll
@@ -703,142 +705,137 @@ __global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
     for (int e = 0; e < 4; ++e) v_rel[e] = base + vrow * ROWB + (((2 * e + (pp >> 1)) ^ attn_swz(vrow)) << 4) + ((pp & 1) << 3);
     const float sc = a.scale * LOG2E;
     int slot = 0;
-    for (int it = 0; it < n; ++it) {
-        const int behind = min(n - 1 - it, NST - 1);  // stages that may still be on their way
-        if (behind == 3) wait_vm<(NST > 3 ? 3 : 0) * P>();
-        else if (behind == 2) wait_vm<(NST > 2 ? 2 : 0) * P>();
-        else if (behind == 1) wait_vm<P>();
-        else wait_vm<0>();
-        const int key0 = klo + it * 64 + w * 16;
-        const unsigned so = slot * C::STAGEB;
-        if (key0 <= p1 && key0 + 15 >= first) {
-            // ---- scores, two accumulation chains per row tile ----
-            f32x4_t s2[MT][2];
+    for (int it = -NST; it < n; ++it) {  // (one place where stages are requested, as in latent_tiles)
+        if (it >= 0) {
+            const int behind = min(n - 1 - it, NST - 1);  // stages that may still be on their way
+            if (behind == 3) wait_vm<(NST > 3 ? 3 : 0) * P>();
+            else if (behind == 2) wait_vm<(NST > 2 ? 2 : 0) * P>();
+            else if (behind == 1) wait_vm<P>();
+            else wait_vm<0>();
+            const int key0 = klo + it * 64 + w * 16;
+            const unsigned so = slot * C::STAGEB;
+            if (key0 <= p1 && key0 + 15 >= first) {
+                // ---- scores, two accumulation chains ----
+                f32x4_t s2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                constexpr int FG = 8;
+                static_for<(KS + FG - 1) / FG>([&](auto G) {
+                    constexpr int i0 = decltype(G)::value * FG, ni = KS - i0 < FG ? KS - i0 : FG;
+                    u32x4_t kf[FG];
+                    static_for<ni>([&](auto I) { constexpr int i = i0 + decltype(I)::value; lds_read_b128<(i >> 1) * 128>(kf[i - i0], k_rel[i & 1] + so); });
+                    wait_lds();
 #pragma unroll
-            for (int m = 0; m < MT; ++m) s2[m][0] = s2[m][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            constexpr int FG = 8;
-            static_for<(KS + FG - 1) / FG>([&](auto G) {
-                constexpr int i0 = decltype(G)::value * FG, ni = KS - i0 < FG ? KS - i0 : FG;
-                u32x4_t kf[FG];
-                static_for<ni>([&](auto I) { constexpr int i = i0 + decltype(I)::value; lds_read_b128<(i >> 1) * 128>(kf[i - i0], k_rel[i & 1] + so); });
-                wait_lds();
+                    for (int i = 0; i < ni; ++i) asm volatile("" : "+v"(kf[i]));
 #pragma unroll
-                for (int i = 0; i < ni; ++i) asm volatile("" : "+v"(kf[i]));
-#pragma unroll
-                for (int i = 0; i < ni; ++i)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m)
-                        s2[m][i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[i]), __builtin_bit_cast(bf16x8_t, qf[m][i0 + i]), s2[m][i & 1], 0, 0, 0);
-            });
-            // ---- weights of row c: this lane holds keys 4 g + r.  The reference point is raised only when a score exceeds it by more than 2^8 ----
-            typedef short s16x4_t __attribute__((ext_vector_type(4)));
-            s16x4_t pf[MT];
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
+                    for (int i = 0; i < ni; ++i)
+                        s2[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[i]), __builtin_bit_cast(bf16x8_t, qf[i0 + i]), s2[i & 1], 0, 0, 0);
+                });
+                // ---- weights of row c: this lane holds keys 4 g + r.  The reference point is raised only when a score exceeds it by more than 2^8 ----
+                typedef short s16x4_t __attribute__((ext_vector_type(4)));
                 float x[4], mx;
                 if (key0 > p1 - a.window && key0 + 15 <= p0) {  // every row sees every key
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = (s2[m][0][r] + s2[m][1][r]) * sc;
+                    for (int r = 0; r < 4; ++r) x[r] = (s2[0][r] + s2[1][r]) * sc;
                 } else {
-                    const int d0 = rpos[m] - (key0 + 4 * g);
+                    const int d0 = rpos - (key0 + 4 * g);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = (rpos[m] >= 0 && d0 - r >= 0 && d0 - r < a.window) ? (s2[m][0][r] + s2[m][1][r]) * sc : -INFINITY;
+                    for (int r = 0; r < 4; ++r) x[r] = (rpos >= 0 && d0 - r >= 0 && d0 - r < a.window) ? (s2[0][r] + s2[1][r]) * sc : -INFINITY;
                 }
                 mx = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-                if (__any(mx > m_run[m] + 8.0f || (m_run[m] == -INFINITY && mx > -INFINITY))) {
+                if (__any(mx > m_run + 8.0f || (m_run == -INFINITY && mx > -INFINITY))) {
                     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
                     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                    const float m_new = fmaxf(m_run[m], mx);
-                    const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run[m] - m_new);
-                    l_run[m] *= alpha;
+                    const float m_new = fmaxf(m_run, mx);
+                    const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+                    l_run *= alpha;
 #pragma unroll
-                    for (int d = 0; d < ND; ++d) acc[m][d] *= alpha;
-                    m_run[m] = m_new;
+                    for (int d = 0; d < ND; ++d) acc[d] *= alpha;
+                    m_run = m_new;
                 }
-                const float m_use = m_run[m] == -INFINITY ? 0.f : m_run[m];
+                const float m_use = m_run == -INFINITY ? 0.f : m_run;
                 float p[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(x[r] - m_use);
-                l_run[m] += (p[0] + p[1]) + (p[2] + p[3]);
-                pf[m] = __builtin_bit_cast(s16x4_t, u32x2_t{pack2bf(p[0], p[1]), pack2bf(p[2], p[3])});
+                l_run += (p[0] + p[1]) + (p[2] + p[3]);
+                const s16x4_t pf = __builtin_bit_cast(s16x4_t, u32x2_t{pack2bf(p[0], p[1]), pack2bf(p[2], p[3])});
+                // ---- O^T += C^T . P^T ----
+                constexpr int VG = 8;
+                static_for<(ND + VG - 1) / VG>([&](auto G) {
+                    constexpr int d0 = decltype(G)::value * VG, nd = ND - d0 < VG ? ND - d0 : VG;
+                    u32x2_t vf[VG];
+                    static_for<nd>([&](auto I) { constexpr int d = d0 + decltype(I)::value; lds_read_tr16_b64<(d >> 2) * 128>(vf[d - d0], v_rel[d & 3] + so); });
+                    wait_lds();
+#pragma unroll
+                    for (int d = 0; d < nd; ++d) asm volatile("" : "+v"(vf[d]));
+#pragma unroll
+                    for (int d = 0; d < nd; ++d) acc[d0 + d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4_t, vf[d]), pf, acc[d0 + d], 0, 0, 0);
+                });
             }
-            // ---- O^T += C^T . P^T ----
-            constexpr int VG = 8;
-            static_for<(ND + VG - 1) / VG>([&](auto G) {
-                constexpr int d0 = decltype(G)::value * VG, nd = ND - d0 < VG ? ND - d0 : VG;
-                u32x2_t vf[VG];
-                static_for<nd>([&](auto I) { constexpr int d = d0 + decltype(I)::value; lds_read_tr16_b64<(d >> 2) * 128>(vf[d - d0], v_rel[d & 3] + so); });
-                wait_lds();
-#pragma unroll
-                for (int d = 0; d < nd; ++d) asm volatile("" : "+v"(vf[d]));
-#pragma unroll
-                for (int d = 0; d < nd; ++d)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) acc[m][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4_t, vf[d]), pf[m], acc[m][d0 + d], 0, 0, 0);
-            });
         }
         if (it + NST < n) issue(it + NST, slot);  // (the stage's last fragments are in registers)
         slot = slot + 1 == NST ? 0 : slot + 1;
     }
-    // ---- the waves' maxima, masses and sums meet in LDS, 16 rows at a time; wave w finishes column tiles w, w + 4, ... ----
-    float* ml = reinterpret_cast<float*>(smem + 4 * C::WAVEB);  // [4][MT][16][2]
+    // ---- the waves' maxima, masses and sums meet in LDS; wave w finishes column tiles w, w + 4, ... ----
+    float* ml = reinterpret_cast<float*>(smem + 4 * C::WAVEB);  // [4][16][2]
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    if (g == 0) *reinterpret_cast<u32x2_t*>(ml + (w * 16 + c) * 2) = u32x2_t{__builtin_bit_cast(unsigned, m_run), __builtin_bit_cast(unsigned, l_run)};
+    __syncthreads();
+    float M = -INFINITY, l = 0.f;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        l_run[m] += __shfl_xor(l_run[m], 16, 64);
-        l_run[m] += __shfl_xor(l_run[m], 32, 64);
-        if (g == 0) *reinterpret_cast<u32x2_t*>(ml + ((w * MT + m) * 16 + c) * 2) = u32x2_t{__builtin_bit_cast(unsigned, m_run[m]), __builtin_bit_cast(unsigned, l_run[m])};
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(u * 16 + c) * 2]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float mu = ml[(u * 16 + c) * 2];
+        l += mu == -INFINITY ? 0.f : ml[(u * 16 + c) * 2 + 1] * __builtin_amdgcn_exp2f(mu - M);
+    }
+    const float f = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - M);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        acc[d] *= f;
+        if ((d & 3) != w) *reinterpret_cast<f32x4_t*>(ring + d * 1024 + lane * 16) = acc[d];
     }
     __syncthreads();
+    float inv = 1.0f;
+    if (a.nsplit == 1 && own) {
+        const float sk = a.sink[h0 + c % hb] * LOG2E, Ms = fmaxf(M, sk), fs = __builtin_amdgcn_exp2f(M - Ms);
+        inv = fs / (l * fs + __builtin_amdgcn_exp2f(sk - Ms));
+    }
+    static_for<ND>([&](auto D) {
+        constexpr int d = decltype(D)::value;
+        if ((d & 3) == w && own) {
+            f32x4_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        float M = -INFINITY, l = 0.f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[((u * MT + m) * 16 + c) * 2]);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const float mu = ml[((u * MT + m) * 16 + c) * 2];
-            l += mu == -INFINITY ? 0.f : ml[((u * MT + m) * 16 + c) * 2 + 1] * __builtin_amdgcn_exp2f(mu - M);
-        }
-        const float f = m_run[m] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[m] - M);
-        if (m > 0) __syncthreads();  // the sums of the rows before have been read
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            acc[m][d] *= f;
-            if ((d & 3) != w) *reinterpret_cast<f32x4_t*>(ring + d * 1024 + lane * 16) = acc[m][d];
-        }
-        __syncthreads();
-        const int r = 16 * m + c;
-        const int hd = h0 + r % hb;
-        const int64_t gr = (int64_t)(tok0 + r / hb) * a.H + hd;
-        float inv = 1.0f;
-        if (a.nsplit == 1 && r < nrows) {
-            const float sk = a.sink[hd] * LOG2E, Ms = fmaxf(M, sk), fs = __builtin_amdgcn_exp2f(M - Ms);
-            inv = fs / (l * fs + __builtin_amdgcn_exp2f(sk - Ms));
-        }
-        static_for<ND>([&](auto D) {
-            constexpr int d = decltype(D)::value;
-            if ((d & 3) == w && r < nrows) {
-                f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) o += u == (d & 3) ? acc[m][d] : *reinterpret_cast<const f32x4_t*>(smem + u * C::WAVEB + d * 1024 + lane * 16);
-                const int dim = 16 * d + 4 * g;
-                if (dim < a.vp) {
-                    if (a.nsplit == 1) *reinterpret_cast<u32x2_t*>(a.ctx + gr * a.vp + dim) = u32x2_t{pack2bf(o[0] * inv, o[1] * inv), pack2bf(o[2] * inv, o[3] * inv)};
-                    else *reinterpret_cast<f32x4_t*>(a.part_o + (gr * a.nsplit + split) * a.vp + dim) = o;
-                }
+            for (int u = 0; u < 4; ++u) o += u == (d & 3) ? acc[d] : *reinterpret_cast<const f32x4_t*>(smem + u * C::WAVEB + d * 1024 + lane * 16);
+            const int dim = 16 * d + 4 * g;
+            if (dim < a.vp) {
+                if (a.nsplit == 1) *reinterpret_cast<u32x2_t*>(a.ctx + gr * a.vp + dim) = u32x2_t{pack2bf(o[0] * inv, o[1] * inv), pack2bf(o[2] * inv, o[3] * inv)};
+                else *reinterpret_cast<f32x4_t*>(a.part_o + (gr * a.nsplit + split) * a.vp + dim) = o;
             }
-        });
-        if (a.nsplit > 1 && w == 0 && g == 0 && r < nrows) {
-            a.part_ml[(gr * a.nsplit + split) * 2] = M;
-            a.part_ml[(gr * a.nsplit + split) * 2 + 1] = l;
         }
+    });
+    if (a.nsplit > 1 && w == 0 && g == 0 && own) {
+        a.part_ml[(gr * a.nsplit + split) * 2] = M;
+        a.part_ml[(gr * a.nsplit + split) * 2 + 1] = l;
     }
 }
 
-template <int NCT, int VCT, int MT>
+// The length of a workgroup's range decides, not the room in the block table, which is as wide as the longest sequence that may come.  Both bodies in one
+// kernel cost the short ranges some 2 %, 576 columns some 0.3 us of 11.
+template <int NCT, int VCT>
+__global__ __launch_bounds__(256, 1) void latent_keys_kernel(const AttnArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LaWork k;
+    if (!la_work<256>(a, k)) return;
+    // (read where they are used: the arguments as they are passed stay in registers over both bodies, and 30 to 50 of them are spilled)
+    const AttnArgs& b = *reinterpret_cast<const AttnArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+    if (k.n >= LK_TILES) latent_keys<NCT, VCT>(b, k, smem);
+    else latent_tiles<NCT, 1>(b, k, smem);
+}
+
+template <int NCT, int VCT>
 int launch_latent_keys(const AttnArgs& a, hipStream_t st) {
-    using C = LkCfg<NCT, VCT, MT>;
-    auto kern = latent_keys_kernel<NCT, VCT, MT>;
+    using C = LkCfg<NCT, VCT>;
+    auto kern = latent_keys_kernel<NCT, VCT>;
     GLM_SET_MAX_LDS(kern, C::LDS, "glm_latent_attn");
     const int64_t grid = (int64_t)a.n_tiles * a.n_hg * a.nsplit;
     GLM_CHECK_ARG(grid < (1ll << 31), GLM_ERR_UNSUPPORTED, "glm_latent_attn: grid too large");
@@ -863,16 +860,15 @@ int launch_latent_attn(const AttnArgs& a, hipStream_t st) {
 constexpr int la_max_rows(int nct) { return nct > 9 ? 16 : nct > 4 ? 32 : 64; }
 
 template <int NCT>
-int launch_latent_attn_mt(const AttnArgs& a, int mt, bool many_keys, hipStream_t st) {
+int launch_latent_attn_mt(const AttnArgs& a, int mt, int64_t most_keys, hipStream_t st) {
     if constexpr (la_max_rows(NCT) >= 64) {
         if (mt > 2) return launch_latent_attn<NCT, 4>(a, st);
     }
-    if constexpr (NCT <= 9) {  // (a wave's sums and queries of all rows in its registers: 32 rows up to 256 columns)
+    if constexpr (NCT <= 9) {  // (a wave's sums and queries of all rows in its registers)
         constexpr int VCT = NCT < 8 ? NCT : 8;
-        if (many_keys && mt == 1 && a.vp <= 64 * VCT) return launch_latent_keys<NCT, VCT, 1>(a, st);
-        if constexpr (NCT <= 4) {
-            if (many_keys && mt == 2) return launch_latent_keys<NCT, VCT, 2>(a, st);
-        }
+        // (up to 256 columns latent_tiles fits a CU twice, and is ahead with more workgroups than CUs: 128 sequences in four splits, 1024 keys 17.1 us, here 25.4)
+        const bool once = NCT > 4 || (int64_t)a.n_tiles * a.n_hg * a.nsplit <= 256;
+        if (mt == 1 && a.vp <= 64 * VCT && once && most_keys > 64 * (LK_TILES - 1)) return launch_latent_keys<NCT, VCT>(a, st);
     }
     if constexpr (la_max_rows(NCT) >= 32) {
         if (mt > 1) return launch_latent_attn<NCT, 2>(a, st);
@@ -1211,16 +1207,16 @@ extern "C" int glm_latent_attn(const void* qa, const void* cache, int64_t n_bloc
     const int64_t range = ((int64_t)bt_stride * block_size < (int64_t)window + tokens_per_tile ? (int64_t)bt_stride * block_size : (int64_t)window + tokens_per_tile);
     GLM_CHECK_ARG((range / nsplit + 128) / block_size + 2 <= LA_BT, GLM_ERR_UNSUPPORTED, "glm_latent_attn: %ld keys per split exceed the block-table slice", (long)(range / nsplit));
     const int rows = tokens_per_tile * a.hb, mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
-    const bool many_keys = range / nsplit >= 256;  // four 64-key tiles per split, on both sides of which the two kernels are level
+    const int64_t most_keys = ((range + 127) / 64 + nsplit - 1) / nsplit * 64;   // of a split: the range begins inside a tile
     switch (nct) {
-        case 1: return launch_latent_attn_mt<1>(a, mt, many_keys, st);
-        case 2: return launch_latent_attn_mt<2>(a, mt, many_keys, st);
-        case 3: return launch_latent_attn_mt<3>(a, mt, many_keys, st);
-        case 4: return launch_latent_attn_mt<4>(a, mt, many_keys, st);
-        case 6: return launch_latent_attn_mt<6>(a, mt, many_keys, st);
-        case 8: return launch_latent_attn_mt<8>(a, mt, many_keys, st);
-        case 9: return launch_latent_attn_mt<9>(a, mt, many_keys, st);
-        default: return launch_latent_attn_mt<16>(a, mt, many_keys, st);
+        case 1: return launch_latent_attn_mt<1>(a, mt, most_keys, st);
+        case 2: return launch_latent_attn_mt<2>(a, mt, most_keys, st);
+        case 3: return launch_latent_attn_mt<3>(a, mt, most_keys, st);
+        case 4: return launch_latent_attn_mt<4>(a, mt, most_keys, st);
+        case 6: return launch_latent_attn_mt<6>(a, mt, most_keys, st);
+        case 8: return launch_latent_attn_mt<8>(a, mt, most_keys, st);
+        case 9: return launch_latent_attn_mt<9>(a, mt, most_keys, st);
+        default: return launch_latent_attn_mt<16>(a, mt, most_keys, st);
     }
 }
 

@@ -231,8 +231,8 @@ def test_latent_attn(dtype, H, rank, vdim, window, bs, n_q, splits):
     (4, 100, 16, 700, 64, 7, 2), (16, 384, 8, 2000, 128, 1, 7), (16, 512, 24, 1100, 64, 1, 3)])
 @pytest.mark.parametrize("extra", [0, 64])
 def test_latent_attn_long_ranges(H, rank, vdim, window, bs, n_q, splits, extra):
-    """Ranges of 256 keys per split and more, where the waves divide the keys: rings that go round, the block table's slice more than once,
-    windows that start inside a stage, sequences shorter than a split, two row tiles; extra columns that make scores only."""
+    """Ranges of six tiles per split and more, where the waves divide the keys: rings that go round, the block table's slice more than once,
+    windows that start inside a stage, sequences shorter than a split, two row tiles (which do not); extra columns that make scores only."""
     from nanovllm import hip_ops
     vp, S = hip_ops.round8(rank), 4
     rp = vp + extra
@@ -274,6 +274,37 @@ def test_latent_attn_long_ranges(H, rank, vdim, window, bs, n_q, splits, extra):
             # roundings of the weights, the context and the result to bf16: 2 ** -9 each, summed up over what one row holds
             err = (got[s, :, h] - ref).abs().max() / max(1.0, float(ref.abs().max()))
             assert err < 2e-2, (s, h, float(err))
+
+
+@pytest.mark.parametrize("H,vp,rp", [(16, 256, 256), (16, 512, 576), (5, 40, 48), (16, 384, 384), (16, 512, 512)])
+@pytest.mark.parametrize("window,splits", [(1 << 30, 1), (1 << 30, 2), (290, 1), (1 << 30, 7)])
+def test_latent_attn_by_the_length_of_a_range(H, vp, rp, window, splits):
+    """Ranges around the tiles from which the waves divide the keys, in a block table for far longer ones: right, and the same bits as each sequence
+    by itself in a table of its own length."""
+    from nanovllm import hip_ops
+    bf, vdim, lens = torch.bfloat16, 16, [1, 64, 257, 320, 321, 383, 384, 641, 645, 1300]
+    S = len(lens)
+    c = [torch.randn(n, rp, generator=g(s)).to(bf) for s, n in enumerate(lens)]
+    q = (torch.randn(S, H, rp, generator=g(99)) * 0.3).to(bf)
+    wuv, sink = (torch.randn(H, vdim, vp, generator=g(5)) * vp ** -0.5).to(bf), torch.randn(H, generator=g(6))
+    cache, bt = _paged([x.float() for x in c], 64, 80, 7)
+    wide = torch.full((S, 64), -1, dtype=torch.int32)
+    wide[:, : bt.shape[1]] = bt
+
+    def attend(rows, table):
+        n = len(rows)
+        out = torch.full((n, H * vdim), float("nan"), dtype=bf, device="cuda")
+        hip_ops.latent_attn(dev(q[rows]), dev(cache, bf), i32(list(range(n))), i32([1] * n), 1, i32([lens[s] - 1 for s in rows]), i32(list(range(n))), i32(table), window, 1.0,
+                            dev(sink), dev(wuv), out, num_splits=splits)
+        return out.cpu()
+    got = attend(list(range(S)), wide)
+    for s, n in enumerate(lens):
+        assert torch.equal(got[s], attend([s], bt[s: s + 1, : -(-n // 64)])[0]), n
+        vis = O.window_mask(n, window)[n - 1:]
+        for h in range(0, H, 4):
+            ref = O.sink_softmax(q[s, h].double()[None] @ c[s].double().T, vis, sink[h].double()) @ c[s][:, :vp].double() @ wuv[h].double().T
+            # roundings of the weights, the context and the result to bf16, as above
+            assert (got[s].view(H, vdim)[h].double() - ref).abs().max() < 2e-2 * max(1.0, float(ref.abs().max())), (n, h)
 
 
 @pytest.mark.parametrize("H,dk,dv,window", [(3, 24, 40, 50), (2, 128, 128, 200), (1, 136, 200, 1), (4, 64, 256, 64), (2, 200, 64, 1000), (2, 256, 256, 129)])
