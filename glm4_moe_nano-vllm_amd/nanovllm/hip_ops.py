@@ -1546,7 +1546,11 @@ def latent_attn(qa: torch.Tensor, cache: torch.Tensor, tile_tok: torch.Tensor, t
         keys = min(window + tokens_per_tile, block_tables.shape[1] * bs)
         # (and no more keys per split than a workgroup's slice of the block table covers)
         ns = num_splits or max(1, min(64, 256 // max(1, wgs), -(-keys // 128)), -(-keys // (900 * bs)))
-    joint = 1 < ns <= 8     # the splits summed up in front of W_uv, in its launch (more of them: one after the other there, side by side in glm_attn_merge)
+    # The splits summed up in front of W_uv, in its launch: a workgroup takes in the sums of 16 tokens of a head, which has to be few bytes or beside many others (more
+    # splits: one after the other there, side by side in glm_attn_merge).  Two launches / one, us, 16 heads: 256 columns of 8 tokens, two and eight splits 5.7 /
+    # 4.1, 6.2 / 5.4, of 128 6.8 / 4.7, 9.7 / 7.8; 512 columns of 8 7.8 / 7.2, 7.1 / 8.8, of 32 7.7 / 6.3, 10.0 / 10.4, of 64 9.5 / 7.1, 11.4 / 10.7; 1024
+    # columns of 8 10.2 / 12.9, 11.9 / 17.8, of 64 14.5 / 14.5, 17.1 / 19.1, of 128 15.4 / 15.0, 24.0 / 21.6.
+    joint = 1 < ns <= 8 and (vp <= 256 or vp <= 512 and (ns <= 4 or Ta > 32))
     ctx = None if joint else torch.empty((Ta, H, vp), dtype=qa.dtype, device=qa.device)
     if ns > 1:
         part_o = torch.empty((Ta * H, ns, vp), dtype=torch.float32, device=qa.device)
