@@ -17,6 +17,14 @@ template <int AUX = 0>
 __device__ __forceinline__ void lds_dma16(const void* gsrc, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((attn_glb_void*)gsrc, (attn_lds_void*)lds_wave_base, 16, 0, AUX);
 }
+// The same from 32-bit offsets into a buffer of whole rows (both wave-uniform): a lane beyond its end brings zeros.  ATTN_BEYOND is beyond any of them.
+constexpr unsigned ATTN_BEYOND = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t attn_rows(const void* base, int rows, int row_bytes) {   // up to 64 rows, 2 GiB
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)((unsigned)min(max(rows, 0), 64) * (unsigned)row_bytes), 0x00020000);
+}
+__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rows, unsigned offset, void* lds_wave_base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (attn_lds_void*)lds_wave_base, 16, offset, 0, 0, 0);
+}
 // 64 lanes x 4 bytes: 256 bytes of LDS
 __device__ __forceinline__ void lds_dma4(const void* gsrc, void* lds_wave_base) {
     __builtin_amdgcn_global_load_lds((attn_glb_void*)gsrc, (attn_lds_void*)lds_wave_base, 4, 0, 0);

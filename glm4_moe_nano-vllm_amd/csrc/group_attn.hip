@@ -111,8 +111,8 @@ __global__ __launch_bounds__(256) void group_kv_store_kernel(const StoreArgs a) 
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// DK, DV: multiples of 64
-template <int DK, int DV, int F>
+// DK, DV: multiples of 64; PAD: heads are narrower
+template <int DK, int DV, int F, bool PAD>
 __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_prefill_kernel(const GroupArgs a) {
     using SL = Slab<DK, DV, 2, F>;
     constexpr bool TWO = ga_two(F), KV = F == GA_SIGMOID_KV;
@@ -169,60 +169,42 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
 #pragma unroll
         for (int i = 0; i < KQ; ++i) asm volatile("" : "+v"(S.qf[t][i]));
     const unsigned base = lds_addr(smem);
-    // Sources of the DMA pieces: piece i of a wave holds 64 / CPR rows from row0 + i 64 / CPR on, and the chunk permutation repeats after eight
-    // rows: offsets of the pieces of eight rows and whole strides between them.  Tiles whose rows are all there, without padding
-    // columns, take them as they are; the others choose per lane between a row and zeros.
-    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KPER = KRP < 8 ? 8 / KRP : 1, VPER = VRP < 8 ? 8 / VRP : 1;
+    // Sources of the DMA pieces: piece i of a wave holds 64 / CPR rows from 16 w + i 64 / CPR on, and the chunk permutation repeats after eight
+    // rows: offsets of the pieces of eight rows, from two bases.  Tiles whose rows are all there, without padding columns, take addresses (a few per cent
+    // ahead); of the others the rows behind the last one lie beyond a buffer's end, and so do, by their offset, padding columns: such lanes bring zeros.
+    // (Lanes that worked out a row or a page of zeros for themselves, for every tile / this, us: 4096 and 3707 tokens, 16 heads over 4, 200 columns
+    // 620 / 591, two maps of 96 with 128 value columns 826 / 686, 96 217 / 198, 72 + 40 191 / 170; windowed, 200 + 136 629 / 494, 72 + 40 212 / 166.)
+    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KPER = 8 / KRP, VPER = 8 / VRP;
     unsigned koff[KPER], voff[VPER];
-    auto k_piece = [&](int lane, int i, int& row, int& ch) {
-        row = (w * KDMA + i) * KRP + lane / KCPR;
-        ch = (lane % KCPR) ^ attn_swz(row);
-    };
-    auto v_piece = [&](int lane, int i, int& row, int& ch) {
-        row = (w * VDMA + i) * VRP + lane / VCPR;
-        ch = (lane % VCPR) ^ attn_swz(row);
-    };
 #pragma unroll
     for (int i = 0; i < KPER; ++i) {
-        int row, ch;
-        k_piece(lane, i, row, ch);
-        koff[i] = (unsigned)(row * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2u;
+        const int row = w * 16 + i * KRP + lane / KCPR, ch = (lane % KCPR) ^ attn_swz(row);
+        koff[i] = !PAD || (ch % MAPC) * 8 < dm ? (unsigned)(row * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2u : ATTN_BEYOND;
     }
 #pragma unroll
     for (int i = 0; i < VPER; ++i) {
-        int row, ch;
-        v_piece(lane, i, row, ch);
-        voff[i] = (unsigned)(row * a.dv + ch * 8) * 2u;
+        const int row = w * 16 + i * VRP + lane / VCPR, ch = (lane % VCPR) ^ attn_swz(row);
+        voff[i] = !PAD || ch * 8 < a.dv ? (unsigned)(row * a.dv + ch * 8) * 2u : ATTN_BEYOND;
     }
-    const bool padded = dm != MAPC * 8 || (!KV && a.dv != DV);
     // tiles from the last keys to the first: under a distance bias the maximum is found early and stays
-    auto issue = [&](int it, int blk) {
+    auto issue = [&](int it, int blk) __attribute__((always_inline)) {
         const int j0 = jlo + (n - 1 - it) * 64, left = ga_ok(a, blk) ? plast - j0 + 1 : 0;
         const int64_t row = ga_row(a, blk, j0, kvh);
         const char* kb = reinterpret_cast<const char*>(a.kc) + row * a.dk * 2;
         const char* vb = reinterpret_cast<const char*>(a.vc) + row * a.dv * 2;
         char* st = smem + (it & 1) * STAGE;
-        if (left >= 64 && !padded) {
+        if (!PAD && left >= 64) {
 #pragma unroll
-            for (int i = 0; i < KDMA; ++i) lds_dma16(kb + (i / KPER) * (KPER * KRP * 2) * a.dk + koff[i % KPER], st + (w * KDMA + i) * 1024);
+            for (int i = 0; i < KDMA; ++i) lds_dma16(kb + (i / KPER) * 16 * a.dk + koff[i % KPER], st + (w * KDMA + i) * 1024);
 #pragma unroll
-            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (i / VPER) * (VPER * VRP * 2) * a.dv + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
+            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (i / VPER) * 16 * a.dv + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
         } else {
-            int ln = lane;
-            asm volatile("" : "+v"(ln));   // (worked out here and now: kept over the tiles, these offsets cost the loop its registers)
 #pragma unroll
-            for (int i = 0; i < KDMA; ++i) {
-                int r, ch;
-                k_piece(ln, i, r, ch);
-                const bool none = (ch % MAPC) * 8 >= dm || r >= left;
-                lds_dma16(none ? (const void*)ga_zero_page : (const void*)(kb + (int64_t)(r * a.dk + (ch / MAPC) * dm + (ch % MAPC) * 8) * 2), st + (w * KDMA + i) * 1024);
-            }
+            for (int i = 0; i < KDMA; ++i)
+                lds_dma16(attn_rows(kb + (i / KPER) * 16 * a.dk, left - 8 * (i / KPER), a.dk * 2), koff[i % KPER], st + (w * KDMA + i) * 1024);
 #pragma unroll
-            for (int i = 0; i < VDMA; ++i) {
-                int r, ch;
-                v_piece(ln, i, r, ch);
-                lds_dma16(ch * 8 >= a.dv || r >= left ? (const void*)ga_zero_page : (const void*)(vb + (int64_t)(r * a.dv + ch * 8) * 2), st + KTILE + (w * VDMA + i) * 1024);
-            }
+            for (int i = 0; i < VDMA; ++i)
+                lds_dma16(attn_rows(vb + (i / VPER) * 16 * a.dv, left - 8 * (i / VPER), a.dv * 2), voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
         }
         if constexpr (KV) {
             if (w == 0) lds_dma4(a.kscale + (int64_t)(ga_ok(a, blk) ? blk : 0) * a.bs + (j0 - ga_block(a, j0) * a.bs) + lane, st + KTILE);
@@ -596,7 +578,8 @@ template <int DK, int DV, int F>
 int launch_prefill(const GroupArgs& a, hipStream_t st) {
     constexpr int LDS = 2 * 64 * (DK + (F == GA_SIGMOID_KV ? 2 : DV)) * 2;
     static_assert(LDS <= 160 * 1024, "LDS of a CU");
-    auto kern = group_attn_prefill_kernel<DK, DV, F>;
+    const bool pad = (ga_two(F) ? a.dk / 2 != DK / 2 : a.dk != DK) || (F != GA_SIGMOID_KV && a.dv != DV);
+    auto kern = pad ? group_attn_prefill_kernel<DK, DV, F, true> : group_attn_prefill_kernel<DK, DV, F, false>;
     GLM_SET_MAX_LDS(kern, LDS, "glm_group_attn_prefill");
     const int64_t per = ((int64_t)a.n_tiles * (a.H >> (ga_two(F) ? 0 : a.pair)) + 7) / 8;
     GLM_CHECK_ARG(per * 8 < (1ll << 31), GLM_ERR_UNSUPPORTED, "glm_group_attn_prefill: grid too large");

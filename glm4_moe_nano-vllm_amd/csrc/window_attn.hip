@@ -35,8 +35,10 @@ struct WinArgs {
     float scale;
 };
 
+enum : int { WA_PLAIN = 0, WA_PADDED = 1, WA_ROTATED = 2 };   // heads as wide as the tiles, narrower ones, or (of any width) with key columns in rows of their own
+
 // DK, DV: multiples of 64
-template <int DK, int DV>
+template <int DK, int DV, int FORM>
 __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_kernel(const WinArgs a) {
     using SL = Slab<DK, DV, 2, GA_SOFTMAX>;
     constexpr int KS = SL::KS, VT = SL::VT, KTILE = 64 * SL::KB, STAGE = KTILE + 64 * SL::VB;
@@ -104,18 +106,13 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
     const bf16_t* rbase = a.kr ? a.kr + (int64_t)(ks0 + jlo) * a.ldr : kbase;
     const bf16_t* vbase = a.v + (int64_t)(ks0 + jlo) * a.ldkv + (int64_t)h * a.dv;
     const int nkeys = jhi - jlo + 1;
-    // Sources of the DMA pieces: as in group_attn.hip, with the last dk - dkn key columns from rows of their own.  Which pieces of a tile's keys a lane
-    // takes from there repeats with the chunk permutation.
-    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KEVEN = 64 % KCPR == 0, KPER = KEVEN ? (KRP < 8 ? 8 / KRP : 1) : KDMA, VEVEN = 64 % VCPR == 0, VPER = VEVEN ? (VRP < 8 ? 8 / VRP : 1) : VDMA;
+    // Sources of the DMA pieces: as in group_attn.hip (chunks that do not divide a piece evenly: offsets of all pieces, one base).  With the last dk - dkn key
+    // columns in rows of their own a piece has two sources and takes addresses, per lane a row of either or zeros.
+    constexpr int KRP = 64 / KCPR, VRP = 64 / VCPR, KEVEN = 64 % KCPR == 0, KPER = KEVEN ? 8 / KRP : KDMA, VEVEN = 64 % VCPR == 0, VPER = VEVEN ? 8 / VRP : VDMA;
     auto k_piece = [&](int lane, int i, int& row, int& ch) {
         const int q = (w * KDMA + i) * 64 + lane;
         row = q / KCPR;
         ch = (q % KCPR) ^ attn_swz(row);
-    };
-    auto v_piece = [&](int lane, int i, int& row, int& ch) {
-        const int q = (w * VDMA + i) * 64 + lane;
-        row = q / VCPR;
-        ch = (q % VCPR) ^ attn_swz(row);
     };
     unsigned koff[KPER], voff[VPER];   // bytes
     unsigned krot = 0;                 // bit i: piece i of a period is of the other rows
@@ -125,47 +122,56 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
         k_piece(lane, i, row, ch);
         const bool rot = ch * 8 >= a.dkn;
         krot |= rot ? 1u << i : 0u;
-        koff[i] = (unsigned)(rot ? row * (int)a.ldr + ch * 8 - a.dkn : row * (int)a.ldkv + ch * 8) * 2u;
+        koff[i] = ch * 8 < a.dk ? (unsigned)(rot ? row * (int)a.ldr + ch * 8 - a.dkn : row * (int)a.ldkv + ch * 8) * 2u : ATTN_BEYOND;
     }
 #pragma unroll
     for (int i = 0; i < VPER; ++i) {
-        int row, ch;
-        v_piece(lane, i, row, ch);
-        voff[i] = (unsigned)(row * (int)a.ldkv + ch * 8) * 2u;
+        const int q = (w * VDMA + i) * 64 + lane, row = q / VCPR, ch = (q % VCPR) ^ attn_swz(row);
+        voff[i] = ch * 8 < a.dv ? (unsigned)(row * (int)a.ldkv + ch * 8) * 2u : ATTN_BEYOND;
     }
-    const bool padded = a.dk != DK || a.dv != DV, rotated = a.dkn != a.dk;
-    auto issue = [&](int it, auto) {
+    const int kvb = (int)a.ldkv * 2;   // bytes of a row
+    const bool padded = FORM == WA_PADDED || (FORM == WA_ROTATED && (a.dk != DK || a.dv != DV));
+    auto issue = [&](int it, auto) __attribute__((always_inline)) {
         const int first = (n - 1 - it) * 64, left = nkeys - first;
         const char* kb = reinterpret_cast<const char*>(kbase + (int64_t)first * a.ldkv);
-        const char* rb = reinterpret_cast<const char*>(rbase + (int64_t)first * a.ldr);
         const char* vb = reinterpret_cast<const char*>(vbase + (int64_t)first * a.ldkv);
         char* st = smem + (it & 1) * STAGE;
-        if (left >= 64 && !padded) {
+        const bool whole = !padded && left >= 64;
+        if constexpr (FORM == WA_ROTATED) {
+            const char* rb = reinterpret_cast<const char*>(rbase + (int64_t)first * a.ldr);
+            if (whole) {
 #pragma unroll
-            for (int i = 0; i < KDMA; ++i) {
-                const int64_t kstep = (int64_t)(i / KPER) * (KPER * KRP) * a.ldkv * 2, rstep = (int64_t)(i / KPER) * (KPER * KRP) * a.ldr * 2;
-                const char* s = kb + kstep + koff[i % KPER];
-                if (rotated) s = krot >> (i % KPER) & 1 ? rb + rstep + koff[i % KPER] : s;
-                lds_dma16(s, st + (w * KDMA + i) * 1024);
+                for (int i = 0; i < KDMA; ++i) {
+                    const int64_t step = (int64_t)(i / KPER) * 8;
+                    lds_dma16(krot >> (i % KPER) & 1 ? rb + step * a.ldr * 2 + koff[i % KPER] : kb + step * kvb + koff[i % KPER], st + (w * KDMA + i) * 1024);
+                }
+            } else {
+                int ln = lane;
+                asm volatile("" : "+v"(ln));   // (rows worked out here and now: kept over the tiles they cost the loop its registers)
+#pragma unroll
+                for (int i = 0; i < KDMA; ++i) {
+                    int row, ch;
+                    k_piece(ln, i, row, ch);
+                    const int64_t step = (int64_t)(i / KPER) * 8;
+                    const char* s = krot >> (i % KPER) & 1 ? rb + step * a.ldr * 2 + koff[i % KPER] : kb + step * kvb + koff[i % KPER];
+                    lds_dma16(koff[i % KPER] == ATTN_BEYOND || row >= left ? (const void*)wa_zero_page : (const void*)s, st + (w * KDMA + i) * 1024);
+                }
             }
+        } else if (whole) {
 #pragma unroll
-            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (int64_t)(i / VPER) * (VPER * VRP) * a.ldkv * 2 + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
+            for (int i = 0; i < KDMA; ++i) lds_dma16(kb + (int64_t)(i / KPER) * 8 * kvb + koff[i % KPER], st + (w * KDMA + i) * 1024);
         } else {
-            int ln = lane;
-            asm volatile("" : "+v"(ln));   // (worked out here and now: kept over the tiles, these offsets cost the loop its registers)
 #pragma unroll
-            for (int i = 0; i < KDMA; ++i) {
-                int r, ch;
-                k_piece(ln, i, r, ch);
-                const char* s = ch * 8 >= a.dkn ? rb + ((int64_t)r * a.ldr + ch * 8 - a.dkn) * 2 : kb + ((int64_t)r * a.ldkv + ch * 8) * 2;
-                lds_dma16(ch * 8 >= a.dk || r >= left ? (const void*)wa_zero_page : (const void*)s, st + (w * KDMA + i) * 1024);
-            }
+            for (int i = 0; i < KDMA; ++i)
+                lds_dma16(attn_rows(kb + (int64_t)(i / KPER) * 8 * kvb, left - 8 * (i / KPER), kvb), koff[i % KPER], st + (w * KDMA + i) * 1024);
+        }
+        if (whole) {
 #pragma unroll
-            for (int i = 0; i < VDMA; ++i) {
-                int r, ch;
-                v_piece(ln, i, r, ch);
-                lds_dma16(ch * 8 >= a.dv || r >= left ? (const void*)wa_zero_page : (const void*)(vb + ((int64_t)r * a.ldkv + ch * 8) * 2), st + KTILE + (w * VDMA + i) * 1024);
-            }
+            for (int i = 0; i < VDMA; ++i) lds_dma16(vb + (int64_t)(i / VPER) * 8 * kvb + voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < VDMA; ++i)
+                lds_dma16(attn_rows(vb + (int64_t)(i / VPER) * 8 * kvb, left - 8 * (i / VPER), kvb), voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
         }
     };
     attn_tiles<DK, DV, GA_SOFTMAX, KDMA + VDMA>(S, base, n, jlo, g, scale * GA_LOG2E, false, issue);
@@ -194,7 +200,7 @@ template <int DK, int DV>
 int launch_window(const WinArgs& a, hipStream_t st) {
     constexpr int LDS = 2 * 64 * (DK + DV) * 2;
     static_assert(LDS <= 160 * 1024, "LDS of a CU");
-    auto kern = window_attn_kernel<DK, DV>;
+    auto kern = a.dkn != a.dk ? window_attn_kernel<DK, DV, WA_ROTATED> : a.dk != DK || a.dv != DV ? window_attn_kernel<DK, DV, WA_PADDED> : window_attn_kernel<DK, DV, WA_PLAIN>;
     GLM_SET_MAX_LDS(kern, LDS, "glm_window_attn_prefill");
     const int64_t per = ((int64_t)a.n_tiles * a.H + 7) / 8;
     GLM_CHECK_ARG(per * 8 < (1ll << 31), GLM_ERR_UNSUPPORTED, "glm_window_attn_prefill: grid too large");

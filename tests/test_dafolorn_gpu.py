@@ -366,6 +366,35 @@ def test_window_attn_prefill_any_scale(H, dk, dv, scale):
             assert (got[:, h] - ref).abs().max() < 2e-2, (kr, h)
 
 
+@pytest.mark.parametrize("H,dk,dv,rotp", [(3, 24, 40, 0), (2, 72, 40, 0), (2, 72, 40, 8), (2, 136, 200, 0), (1, 200, 136, 8), (2, 192, 128, 64)])
+def test_window_attn_prefill_padding_is_zero(H, dk, dv, rotp):
+    """What a head lacks of its tile's columns, and the keys behind the last one, count as zeros whatever the kernel before left in the shared memory: here not-a-numbers."""
+    from nanovllm import hip_ops
+    def run(q, kk, v, heads, dk, dv, n, **rot):
+        kv = torch.cat([kk.reshape(n, -1), v.reshape(n, -1)], 1).cuda()
+        out = torch.full((n, heads * dv), float("nan"), dtype=torch.bfloat16, device="cuda")
+        tiles = list(range(0, n, 128))
+        hip_ops.window_attn_prefill(dev(q.reshape(n, -1)), kv[:, : heads * (dk - rot_cols(rot))], kv[:, heads * (dk - rot_cols(rot)):], out, i32([0, n]), i32([0, n]),
+                                    i32([0] * len(tiles)), i32(tiles), heads, dk, dv, 4096, 0.5 * dk ** -0.5, dev(torch.zeros(heads)), **rot)
+        return out.cpu().double().view(n, heads, dv)
+    rot_cols = lambda rot: rot["kr"].shape[1] if rot else 0  # noqa: E731
+    n = 171
+    q, k, v = (torch.randn(n, H, d, generator=g(i)).bfloat16() for i, d in ((1, dk), (2, dk), (3, dv)))
+    rot = {}
+    if rotp:
+        k[:, :, dk - rotp:] = k[:, :1, dk - rotp:]
+        rot = dict(kr=dev(k[:, 0, dk - rotp:].contiguous()), cs=torch.tensor([1.0, 0.0], device="cuda").repeat(n * rotp // 2).view(n, rotp))
+    up = lambda d: next(t for t in (64, 128, 192, 256) if d <= t)  # noqa: E731
+    for wk, wv in ((up(dk), up(dv)), (256, 256)):
+        bad = torch.full((768, 64, wk), float("nan")).bfloat16()
+        assert run(bad, bad, bad[:, :, :1].expand(-1, -1, wv), 64, wk, wv, 768).isnan().all()
+        got = run(q, k[:, :, : dk - rotp] if rotp else k, v, H, dk, dv, n, **rot)
+        for h in range(H):
+            ref = O.sink_softmax(0.5 * dk ** -0.5 * (q[:, h].double() @ k[:, h].double().T), O.window_mask(n, 4096), torch.tensor(0.0).double()) @ v[:, h].double()
+            # weights and result in bf16, 2 ** -9 each, of values up to about 4
+            assert (got[:, h] - ref).abs().max() < 2e-2, (wk, wv, h)
+
+
 # ---- the model through the engine -------------------------------------------------------------------------------------------
 @pytest.fixture(scope="module", params=list(CONFIGS))
 def model(request, tmp_path_factory):

@@ -325,6 +325,51 @@ def test_group_attention_forms(form, H, G, dim, dv, bs, kind):
                 assert err < (5e-5 if dtype == "float32" else 3e-2), (gate, s, h, err)
 
 
+@pytest.mark.parametrize("form,G,dim,dv", [("softmax", 2, 40, 24), ("softmax", 2, 136, 200), ("softmax", 1, 72, 256), ("sigmoid", 2, 72, 72), ("sigmoid", 2, 24, 24), ("two_maps", 2, 40, 72),
+                                           ("two_maps", 1, 72, 40)])
+def test_group_attn_prefill_padding_is_zero(form, G, dim, dv):
+    """What a head lacks of its tile's columns, and the keys behind the last one, count as zeros whatever the kernel before left in the shared memory: here not-a-numbers."""
+    from nanovllm import hip_ops
+    maps, n, bs = 2 if form == "two_maps" else 1, 171, 64
+
+    def run(q, kc, vc, bt, n, H, **form):
+        out = torch.full((n, H * vc.shape[3]), float("nan"), dtype=torch.bfloat16, device="cuda")
+        tiles = list(range(0, n, hip_ops.group_attn_tile_rows(H, kc.shape[1], maps)))
+        parts = hip_ops.GroupParts(maps=maps, **form)
+        hip_ops.group_attn_prefill(q, kc, vc, i32(bt), 0, i32([0, n]), i32(torch.arange(n)), i32([0] * len(tiles)), i32(tiles), H, 0, 0, 0.5 * dim ** -0.5, None, None, out, parts=parts)
+        return out.cpu().double().view(n, H, -1)
+    k, v, q = (torch.randn(n, G, m, d, generator=g(i)).bfloat16() for i, m, d in ((1, maps, dim), (2, 1, dv), (3, maps, dim)))
+    scales = torch.ones(8, bs, device="cuda")
+    more = dict(sigmoid=True, bias=torch.zeros(G, device="cuda"), kscale=scales) if form == "sigmoid" else dict(cap=20.0, lam=0.4, post=0.6, eps=1e-3, vn=dv) if maps == 2 else {}
+    if form == "sigmoid":
+        v = k
+    perm = torch.randperm(8, generator=g(7)).tolist()
+    kc, bt = _paged([k.reshape(n, G, -1).float()], G, bs, 8, perm)
+    vc, _ = _paged([v[:, :, 0].float()], G, bs, 8, perm)
+    kc = dev(kc, torch.bfloat16)
+    vc = kc if form == "sigmoid" else dev(vc, torch.bfloat16)
+    up = lambda d: next(t for t in (64, 128, 192, 256) if d <= t)  # noqa: E731
+    for wk, wv in ((up(dim), up(dv)), (256 // maps, 256)):
+        bad = torch.full((12, 64, bs, wk * maps), float("nan"), dtype=torch.bfloat16, device="cuda")
+        badv = bad if form == "sigmoid" else torch.full((12, 64, bs, wv), float("nan"), dtype=torch.bfloat16, device="cuda")
+        poison = {**more, **(dict(bias=torch.zeros(64, device="cuda"), kscale=torch.ones(12, bs, device="cuda")) if form == "sigmoid" else dict(vn=wv) if maps == 2 else {})}
+        assert run(torch.ones(768, 64 * wk * maps, dtype=torch.bfloat16, device="cuda"), bad, badv, torch.arange(12)[None], 768, 64, **poison).isnan().all()
+        got = run(dev(q.reshape(n, -1)), kc, vc, bt, n, G, **more)
+        for h in range(G):
+            o = []
+            for m in range(maps):
+                s = 0.5 * dim ** -0.5 * (q[:, h, m].double() @ k[:, h, m].double().T)
+                s = 20.0 * torch.tanh(s / 20.0) if maps == 2 else s
+                s = s.masked_fill(~torch.ones(n, n).tril().bool(), -math.inf)
+                o.append((torch.sigmoid(s) if form == "sigmoid" else torch.softmax(s, -1)) @ v[:, h, 0].double())
+            ref = o[0]
+            if maps == 2:
+                d = o[0] - 0.4 * o[1]
+                ref = 0.6 * d / (d.square().mean(-1, keepdim=True) + 1e-3).sqrt()
+            # weights and result in bf16, 2 ** -9 each, of values up to about 4; sigmoids are not normalised: sums of up to n / 2 such values
+            assert (got[:, h] - ref).abs().max() < (2e-2 if form != "sigmoid" else 2 ** -8 * float(ref.abs().max()) + 2e-2), (wk, wv, h)
+
+
 # ---- the model through the engine -------------------------------------------------------------------------------------------
 @pytest.fixture(scope="module", params=list(CONFIGS))
 def model(request, tmp_path_factory):
