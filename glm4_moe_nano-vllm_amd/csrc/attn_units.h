@@ -53,9 +53,29 @@ struct Slab {
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(-2.f * cap_out, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r] * cap_in)), cap_out);
     }
-    // One 32-key slab, its parts one after the other: decoding, and head sizes whose fragments of two slabs do not fit the registers.  kst, vst,
-    // fst: LDS addresses of its first key row, value row and (sigmoid form) the keys' factors; j0: position of its first key.  All K fragments and the
-    // first V fragments are requested at once, the other V fragments a group ahead of their products.
+    // largest magnitude of the eight scores
+    __device__ __forceinline__ static float size(const f32x4_t (&s)[2]) {
+        float m;
+        asm("v_max3_f32 %0, abs(%1), abs(%2), abs(%3)\n\tv_max3_f32 %0, %0, abs(%4), abs(%5)\n\tv_max3_f32 %0, %0, abs(%6), abs(%7)\n\tv_max_f32 %0, %0, abs(%8)"
+            : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
+        return m;
+    }
+    // up to a fifth of the cap tanh is its odd polynomial of degree 7 (the next term is below 2e-8 of the cap)
+    __device__ __forceinline__ void cap_small(f32x4_t (&s)[2]) const {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float u = s[kt][r] * s[kt][r];
+                s[kt][r] *= fmaf(fmaf(fmaf(ca3, u, ca2), u, ca1), u, ca0);
+            }
+    }
+    // One 32-key slab, its parts one after the other: decoding, a tile or two, and head sizes whose fragments of two slabs do not fit the registers.  kst,
+    // vst, fst: LDS addresses of its first key row, value row and (sigmoid form) the keys' factors; j0: position of its first key.  K fragments in groups of four, the
+    // first V fragments beside the last of them, the others a group ahead of their products.  4096 and 3707 tokens, 16 heads, all K fragments at once / this, us: heads
+    // of 256 over 4 key heads, softmax 552 / 516, two maps 793 / 767, sigmoid weights 401 / 382; 256 + 128 442 / 409, two maps under a
+    // cap 686 / 640 (one after the other under it: 657); every head by itself with a sink 544 / 488, 192 + 128 249 / 232; 64 + 256 and 128 + 256, which have no more than four,
+    // 418 / 418 and 449 / 455.
     __device__ __forceinline__ void run(unsigned kst, unsigned vst, int j0, int g, float sc, unsigned fst, bool biased) {
         bool live[NT], some = false;
 #pragma unroll
@@ -65,37 +85,69 @@ struct Slab {
         }
         if (!some) return;
         constexpr int VG = VEARLY ? VT : 4, VN = VT / VG;   // V fragments per request group
+        constexpr int KG = KS <= 4 ? KS : 4, KN = (KS + KG - 1) / KG;   // K fragments per request group
         u32x4_t kf[2][KS], ks[2];
-        u32x2_t vf[VN > 1 ? 2 : 1][VG][2];
+        constexpr int VB2 = VN > 1 ? 2 : 1;                             // V groups in registers
+        u32x2_t vf[VB2][VG][2];
         auto read_v = [&](auto GI) {
             static_for<VG>([&](auto I) {
                 constexpr int gi = decltype(GI)::value, i = decltype(I)::value, d = gi * VG + i;
-                lds_read_tr16_b64<(d >> 2) * 128>(vf[gi & 1][i][0], vst + v_rel[d & 3]);
-                lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[gi & 1][i][1], vst + v_rel[d & 3]);
+                lds_read_tr16_b64<(d >> 2) * 128>(vf[gi % VB2][i][0], vst + v_rel[d & 3]);
+                lds_read_tr16_b64<(d >> 2) * 128 + 16 * VB>(vf[gi % VB2][i][1], vst + v_rel[d & 3]);
             });
         };
         if constexpr (F == GA_SIGMOID_KV) {  // (in front of the K fragments: in when they are)
             lds_read_b128<0>(ks[0], fst + 16 * g);
             lds_read_b128<64>(ks[1], fst + 16 * g);
         }
-        static_for<KS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            lds_read_b128<(i >> 1) * 128>(kf[0][i], kst + k_rel[i & 1]);
-            lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i], kst + k_rel[i & 1]);
-        });
-        read_v(std::integral_constant<int, 0>{});
-        // the K fragments are in; the V fragments (issued last) may still be on their way
-        asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * VG <= 15 ? 2 * VG : 15) : "memory");
-#pragma unroll
-        for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
-        if constexpr (F == GA_SIGMOID_KV) asm volatile("" : "+v"(ks[0]), "+v"(ks[1]));
         f32x4_t s[NT][2];
-        static_for<NT>([&](auto T) { scores<decltype(T)::value>(s[decltype(T)::value], kf, j0, g, biased); });
+        static_for<KN>([&](auto GI) {
+            constexpr int k0 = decltype(GI)::value * KG, kn = KS - k0 < KG ? KS - k0 : KG;
+            static_for<kn>([&](auto I) {
+                constexpr int i = k0 + decltype(I)::value;
+                lds_read_b128<(i >> 1) * 128>(kf[0][i], kst + k_rel[i & 1]);
+                lds_read_b128<(i >> 1) * 128 + 16 * KB>(kf[1][i], kst + k_rel[i & 1]);
+            });
+            if constexpr (k0 + KG >= KS) {
+                read_v(std::integral_constant<int, 0>{});
+                // the K fragments are in; the V fragments (issued last) may still be on their way
+                asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(2 * VG <= 15 ? 2 * VG : 15) : "memory");
+                if constexpr (F == GA_SIGMOID_KV) asm volatile("" : "+v"(ks[0]), "+v"(ks[1]));
+            } else {
+                wait_lds();
+            }
+#pragma unroll
+            for (int i = k0; i < k0 + kn; ++i) asm volatile("" : "+v"(kf[0][i]), "+v"(kf[1][i]));
+            static_for<kn>([&](auto I) {   // (the tiles' chains side by side: little else covers their latency where a CU holds one workgroup)
+                constexpr int i = k0 + decltype(I)::value;
+                static_for<NT>([&](auto T) {
+                    constexpr int t = decltype(T)::value;
+                    if constexpr (!SPLIT || i / KQ == t) {
+                        if constexpr (i % KQ == 0) {
+                            first_scores<t>(s[t], kf, j0, g, biased);
+                        } else {
+#pragma unroll
+                            for (int kt = 0; kt < 2; ++kt) add_score<t>(s[t], kf, kt, i % KQ, s[t][kt]);
+                        }
+                    }
+                });
+            });
+        });
+        constexpr bool JOINT = F == GA_TWO_MAPS && NT > 1 && DK > 64;   // both maps under the cap at once
+        if constexpr (JOINT) {
+            if (__any(!(fmaxf(size(s[0]), size(s[1])) <= cap_lim))) {
+                cap_exact(s[0]);
+                cap_exact(s[1]);
+            } else {
+                cap_small(s[0]);
+                cap_small(s[1]);
+            }
+        }
         bf16x8_t pf[NT];
         static_for<NT>([&](auto T) {
             constexpr int t = decltype(T)::value;
             if (live[t]) {
-                pf[t] = weights<t, true>(s[t], j0, g, sc, ks);
+                pf[t] = weights<t, true, JOINT>(s[t], j0, g, sc, ks);
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) pf[t][i] = (__bf16)0.f;
@@ -104,14 +156,14 @@ struct Slab {
         static_for<VN>([&](auto GI) {
             constexpr int gi = decltype(GI)::value;
             wait_lds();
-            vpin(vf[gi & 1]);
+            vpin(vf[gi % VB2]);
             if constexpr (gi + 1 < VN) {
                 read_v(std::integral_constant<int, gi + 1>{});
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int i = 0; i < VG; ++i) {
-                const u32x4_t vv = {vf[gi & 1][i][0][0], vf[gi & 1][i][0][1], vf[gi & 1][i][1][0], vf[gi & 1][i][1][1]};
+                const u32x4_t vv = {vf[gi % VB2][i][0][0], vf[gi % VB2][i][0][1], vf[gi % VB2][i][1][0], vf[gi % VB2][i][1][1]};
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
                     acc[t][gi * VG + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vv), pf[t], acc[t][gi * VG + i], 0, 0, 0);
@@ -125,10 +177,11 @@ struct Slab {
     }
     // scores of tile T: start from the distance bias where there is one
     template <int T>
-    __device__ __forceinline__ void scores(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int j0, int g, bool biased) const {
-        auto add = [&](int kt, int i, const f32x4_t& to) {
-            s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][SPLIT ? T * KQ + i : i]), __builtin_bit_cast(bf16x8_t, qf[T][i]), to, 0, 0, 0);
-        };
+    __device__ __forceinline__ void add_score(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int kt, int i, const f32x4_t& to) const {
+        s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[kt][SPLIT ? T * KQ + i : i]), __builtin_bit_cast(bf16x8_t, qf[T][i]), to, 0, 0, 0);
+    }
+    template <int T>
+    __device__ __forceinline__ void first_scores(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int j0, int g, bool biased) const {
         if (F == GA_SOFTMAX && biased) {
             const float b0 = slope[T] * (float)(j0 + 4 * g - rp[T]);
 #pragma unroll
@@ -136,16 +189,20 @@ struct Slab {
                 f32x4_t bias4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) bias4[r] = fmaf(slope[T], (float)(16 * kt + r), b0);
-                add(kt, 0, bias4);
+                add_score<T>(s, kf, kt, 0, bias4);
             }
         } else {
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt) add(kt, 0, f32x4_t{0.f, 0.f, 0.f, 0.f});
+            for (int kt = 0; kt < 2; ++kt) add_score<T>(s, kf, kt, 0, f32x4_t{0.f, 0.f, 0.f, 0.f});
         }
+    }
+    template <int T>
+    __device__ __forceinline__ void scores(f32x4_t (&s)[2], const u32x4_t (&kf)[2][KS], int j0, int g, bool biased) const {
+        first_scores<T>(s, kf, j0, g, biased);
 #pragma unroll
         for (int i = 1; i < KQ; ++i)
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt) add(kt, i, s[kt]);
+            for (int kt = 0; kt < 2; ++kt) add_score<T>(s, kf, kt, i, s[kt]);
     }
     // largest of the eight scores (inline asm: hipcc would quiet every operand of a maximum first)
     __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
@@ -154,8 +211,8 @@ struct Slab {
             : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
         return m;
     }
-    // weights of tile T; fac: sigmoid form, factors of the lane's keys times scale and log2 e, negative; EDGE: some keys may be hidden
-    template <int T, bool EDGE>
+    // weights of tile T; fac: sigmoid form, factors of the lane's keys times scale and log2 e, negative; EDGE: some keys may be hidden; CAPPED: the scores
+    template <int T, bool EDGE, bool CAPPED = false>
     __device__ __forceinline__ bf16x8_t weights(f32x4_t (&s)[2], int j0, int g, float sc, const u32x4_t (&fac)[2]) {
         bf16x8_t pf;
         if constexpr (F == GA_SIGMOID_KV) {
@@ -166,21 +223,9 @@ struct Slab {
                 for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(s[kt][r], f[r], -slope[T]);
             }
         }
-        if constexpr (F == GA_TWO_MAPS) {
-            float big = 0.f;
-            asm("v_max3_f32 %0, abs(%1), abs(%2), abs(%3)\n\tv_max3_f32 %0, %0, abs(%4), abs(%5)\n\tv_max3_f32 %0, %0, abs(%6), abs(%7)\n\tv_max_f32 %0, %0, abs(%8)"
-                : "=&v"(big) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
-            if (__any(!(big <= cap_lim))) {
-                cap_exact(s);
-            } else {
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float u = s[kt][r] * s[kt][r];
-                        s[kt][r] *= fmaf(fmaf(fmaf(ca3, u, ca2), u, ca1), u, ca0);
-                    }
-            }
+        if constexpr (F == GA_TWO_MAPS && !CAPPED) {
+            if (__any(!(size(s) <= cap_lim))) cap_exact(s);
+            else cap_small(s);
         }
         if (F == GA_TWO_MAPS_ANY && cap_out > 0.f) cap_exact(s);
         if (EDGE && (j0 < full_lo[T] || j0 + 31 > full_hi[T])) {
@@ -263,6 +308,19 @@ __device__ __forceinline__ void attn_tiles(Slab<DK, DV, 2, F>& S, unsigned base,
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
+    auto slabs = [&]() __attribute__((always_inline)) {
+        issue(0, I0{});
+        for (int it = 0; it < n; ++it) {
+            wait_vm<0>();
+            __builtin_amdgcn_s_barrier();
+            if (it == 0 && n > 1) issue(1, I1{});
+            else if (it + 1 < n) issue(it + 1, I2{});
+            const unsigned st = base + (it & 1) * STAGE;
+#pragma unroll
+            for (int s = 1; s >= 0; --s)
+                S.run(st + s * 32 * KB, st + (KV ? 0 : KTILE) + s * 32 * VB, jlo + (n - 1 - it) * 64 + s * 32, g, sc, st + KTILE + s * 128, biased);
+        }
+    };
     if constexpr (SL::VEARLY) {
         // ---- units (slab, tile): the scores of the next unit are started in front of the weights of this one, and the fragments they need are
         // requested a unit ahead, so that neither LDS nor the matrix pipe's latency stands between a unit's parts.  Per tile of 64 keys (slabs 1, 0):
@@ -271,6 +329,7 @@ __device__ __forceinline__ void attn_tiles(Slab<DK, DV, 2, F>& S, unsigned base,
         //   (0, t0)  scores (0, t1); V of slab 0 requested; weights; the next tile has arrived, the one after it is requested into this
         //            tile's buffer, whose last fragments are in (barrier), K of the next tile's slab 1 requested; values
         //   (0, t1)  scores of the next tile's (1, t0); weights, values
+        // One tile or two go by slabs, which pass by what no row sees: 40 tokens, 15 heads over 3 of 128 7.6 (before units), 8.0 (units), 7.9.
         // 15074 tokens of 4 prompts, 16 heads of 128 + 128, slabs one after the other / units, us: softmax 348 / 316, two maps of 64 under a cap
         // 617 / 584, sigmoid weights 323 / 314, windows of 1024 193 / 181.  What is left: LDS reads (every wave reads all keys and values for 32
         // rows, 2300 of some 5000 clocks a tile with the staging), exponentials and products beside one another, some 8 us of start and end per
@@ -314,6 +373,7 @@ __device__ __forceinline__ void attn_tiles(Slab<DK, DV, 2, F>& S, unsigned base,
         };
         auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
         auto seen = [&](int j, int t) { return j <= S.any_hi[t] && j + 31 >= S.any_lo[t]; };   // by some row of the tile
+        if (n <= 2) return slabs();
         issue(0, I0{});
         if (n > 1) {
             issue(1, I1{});
@@ -387,17 +447,7 @@ __device__ __forceinline__ void attn_tiles(Slab<DK, DV, 2, F>& S, unsigned base,
             while (it < n && !inside(it)) tile(std::true_type{}, it++);
         }
     } else {
-        issue(0, I0{});
-        for (int it = 0; it < n; ++it) {
-            wait_vm<0>();
-            __builtin_amdgcn_s_barrier();
-            if (it == 0 && n > 1) issue(1, I1{});
-            else if (it + 1 < n) issue(it + 1, I2{});
-            const unsigned st = base + (it & 1) * STAGE;
-#pragma unroll
-            for (int s = 1; s >= 0; --s)
-                S.run(st + s * 32 * KB, st + (KV ? 0 : KTILE) + s * 32 * VB, jlo + (n - 1 - it) * 64 + s * 32, g, sc, st + KTILE + s * 128, biased);
-        }
+        slabs();
     }
 }
 
