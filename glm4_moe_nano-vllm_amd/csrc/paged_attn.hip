@@ -218,22 +218,19 @@ __global__ __launch_bounds__(256, 2) void paged_attn_decode_kernel(
     read_table();
     int len;
     if (by_length) {
-        // More workgroups than CUs: the ones of the longest sequences first, so that the last to start are the shortest (64 sequences of 6.1k
-        // to 8.2k keys, two workgroups per CU one after the other: 298 -> 286 us).  Up to 64 sequences, one per lane, each wave for itself; where the
-        // lengths are short or alike the block table is on its way already.
+        // More workgroups than CUs: the ones of the longest sequences first, so that the last to start are the shortest.  Up to 64 sequences, one per
+        // lane, each wave for itself.  Alike is measured against the first one's length: in whole sequences' order / this, us, 96 heads over 8: 64 sequences of
+        // 3/4 to all of 8192 keys 298 / 286, of 4096 158 / 149, of none to all of 8192 212 / 173, of 4096 109 / 91, of 2048 58 / 51; with 3/4 to all of 3500 and 2048, where
+        // ordering gained nothing, 135 / 135 and 81 / 81 (no order).  Few that start second pay for the order: 40 of none to all of 4096 69.6 / 70.0, 20 of them over 16
+        // 68.8 / 70.2, but a seventh of 4096 among 512 64 / 57.  Below 2048 keys the look at the lengths is 0.2 us (27.0 / 27.2 at 512).
         const int nb = gridDim.z, mine = lane < nb ? context_lens[lane] : -1;
-        int hi = mine, lo = lane < nb ? mine : 0x7fffffff;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            hi = max(hi, __shfl_xor(hi, o, 64));
-            lo = min(lo, __shfl_xor(lo, o, 64));
-        }
-        if (hi >= 2048 && hi - lo > hi / 16) {  // (uniform)
+        const int ref = __builtin_amdgcn_readfirstlane(mine), apart = __ballot(mine >= 4096) ? ref / 16 : ref / 2;
+        if (__ballot(mine >= 2048) && __ballot(lane < nb && abs(mine - ref) > apart)) {  // (uniform)
+            const int key = lane < nb ? min(mine, (1 << 25) - 1) * 64 + 63 - lane : -1;  // no two alike
             int rank = 0;
-            for (int i = 0; i < nb; ++i) {
-                const int v = __builtin_amdgcn_readlane(mine, i);
-                rank += v > mine || (v == mine && i < lane) ? 1 : 0;
-            }
+            for (int i = 0; i < nb; i += 8)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) rank += __builtin_amdgcn_readlane(key, i + j) > key ? 1 : 0;
             b = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(lane < nb && rank == (int)blockIdx.z)) - 1);
             read_table();
         }
@@ -687,6 +684,8 @@ static int pa_launch(const void* q, const void* k_cache, const void* v_cache, co
     hipStream_t st = glm_s(stream);
     const float scale_log2e = scale * 1.4426950408889634f;
     const dim3 grid((unsigned)splits, (unsigned)nkv, (unsigned)B);
+    // The order of paged_attn_decode_kernel pays for itself by what sequences of 2048 keys and more differ in; the host knows no more than their bound.  (Under bounds
+    // from 2048 to 6143 they keep their own order, though longer differences gain there too: 64 of none to all of 4096, 109 / 91 us.)
     const int by_length = splits == 1 && B * nkv > 256 && B <= 64 && (max_context_len > 0 ? max_context_len : bt_stride * block_size) >= 6144;
     PaFuse fu;
     memset(&fu, 0, sizeof(fu));

@@ -300,6 +300,53 @@ def test_paged_attn_decode_longest_first(ops, B, nh, nkv, width):
     assert_mixed(got, O.attn_decode_paged(q, kc, vc, cl, bt, scale), 1.6e-2, 4e-3, f"longest first B={B} nkv={nkv}")
 
 
+@pytest.mark.parametrize("B,nh,nkv,width", [(33, 8, 8, 24), (64, 24, 8, 256), (40, 16, 16, 300), (57, 10, 5, 257)])
+@pytest.mark.parametrize("ns", [0, 2, 3])
+@pytest.mark.parametrize("spread", ["all", "first", "alike", "near"])
+def test_paged_attn_decode_from_qkv_longest_first(ops, B, nh, nkv, width, ns, spread):
+    """Sequences that start by length, straight from bf16 rows and from two and three K slices: every one's row, bias sum, position, slot and cache rows stay its own.
+    Outputs and caches are bit for bit those in the order of the rows."""
+    g = torch.Generator().manual_seed(B + width + ns)
+    if spread == "alike":
+        lens = [2100] * B
+    elif spread == "near":      # within 1/16 of the first one, but one just beyond
+        lens = [4096 + int(x) for x in torch.randint(-256, 257, (B,), generator=g)]
+        lens[0], lens[B - 1] = 4096, 4096 + 257
+    else:
+        lens = torch.randint(1, 500, (B,), generator=g).tolist()
+        lens[3] = lens[B - 1] = 2500
+        lens[5], lens[7], lens[B - 2] = 1, 2049, 2048
+        if spread == "first":
+            lens[0] = 3000
+    hd, bs, rd = 128, 256, 64
+    W, scale = (nh + 2 * nkv) * hd, hd ** -0.5
+    need = [-(-n // bs) for n in lens]
+    cl = torch.tensor(lens, dtype=torch.int32)
+    bt = torch.full((B, width), -1, dtype=torch.int32)
+    blocks = torch.randperm(sum(need), generator=g).to(torch.int32)
+    for b, n in enumerate(need):
+        bt[b, :n] = blocks[sum(need[:b]): sum(need[: b + 1])]
+    kc, vc = (torch.randn(sum(need), bs, nkv, hd, device="cuda", generator=torch.Generator("cuda").manual_seed(i)).to(BF) for i in (1, 2))
+    pos = (cl - 1).to(torch.int64)
+    slots = torch.tensor([int(bt[b, (n - 1) // bs]) * bs + (n - 1) % bs for b, n in enumerate(lens)], dtype=torch.int32)
+    fr = torch.outer(torch.arange(4608, dtype=torch.float), 1.0 / (1e6 ** (torch.arange(0, rd, 2, dtype=torch.float) / rd)))
+    cs = torch.cat((fr.cos(), fr.sin()), -1).unsqueeze(1).contiguous()
+    part = torch.randn(max(ns, 1), B, W, generator=g)
+    qkv = ops.PartialSum(dev(part)) if ns else dev(part[0].to(BF))
+    bias = dev((torch.randn(W, generator=g) * 0.1).to(BF)) if ns else None
+    res = []
+    for bound in (0, 4096 + 512 if spread == "near" else 4096):     # bounds below the ones that the order is for
+        k, v = kc.clone(), vc.clone()
+        out = ops.paged_attn_decode_qkv(qkv, nh, nkv, hd, dev(pos), dev(cs), rd, dev(slots), k, v, dev(cl), dev(bt), scale, num_splits=1, max_context_len=bound, qkv_bias=bias)
+        res.append((out, k, v))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    # the rows in the caches are the sequences' own ones: values as they come, keys turned to their position
+    x = (part.sum(0) if ns < 3 else part[0] + part[1] + part[2]) + (bias.cpu().float() if ns else 0)
+    at = dev(slots).long()
+    assert torch.equal(res[0][2].view(-1, nkv, hd)[at].cpu().view(B, -1), x[:, (nh + nkv) * hd:].to(BF))
+    assert torch.equal(res[0][1].view(-1, nkv, hd)[at].cpu()[:, :, rd:], x[:, nh * hd: (nh + nkv) * hd].to(BF).view(B, nkv, hd)[:, :, rd:])
+
+
 def test_paged_attn_decode_spiky_scores(ops):
     """Force the online-softmax rescale: one key far above the rest late in the sequence."""
     q, kc, vc, cl, bt = _paged_case([777], 12, 1, seed=99)
