@@ -279,6 +279,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_midm_kernel(const GemmParams p, 
 // end needs is loaded before the stream.  65 experts of 1408 x 4096, gate|up / down, us: 211 tokens 270 / 155 (without all this) -> 247 / 142, 350
 // 294 / 165 -> 277 / 161, 600 477 / 236 -> 465 / 220; 64 of 1024 x 2048 at 300 tokens 109 / 63 -> 106 / 60.  Not taken: 32 weight rows (278 / 154 at
 // 211 tokens) or 128 (248 / 147), a third stage (equal), one wave (264 / 151), two or four column tiles as one stream (253 / 149, 300 / 168).
+// Registers are held to what lets two waves share a SIMD: with all that one wave may have the compiler took 260, accumulators moved in and out of the
+// far half of them in the loop.  Without / with that bound, gate|up, rows alike: 40 per expert of 64 of 1024 x 2048 122 / 110, of 9 of 2048 x 4096
+// 85 / 72, 28 of 257 of 512 x 2048 220 / 193, of 65 of 1408 x 4096 280 / 261; down 40 of 64 of 1024 x 2048 61.2 / 59.8.
 template <int MODE, int MT>
 __device__ __forceinline__ void midm_expert_body(const GemmParams& p, char* smem, int grp, int m0, int mcnt, int ncol0, bool once, int reach) {
     constexpr int RT = 4, NW = 2, NST = 2, D = 2 * (MT + RT), STAGE = D * 1024, MPW = MT / NW;
@@ -440,7 +443,7 @@ __device__ __forceinline__ void midm_expert_body(const GemmParams& p, char* smem
 }
 
 template <int MODE>
-__global__ __launch_bounds__(128) void gemm_midm_experts_kernel(const GemmParams p, int reach) {
+__global__ __launch_bounds__(128, 2) void gemm_midm_experts_kernel(const GemmParams p, int reach) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     int* sh = reinterpret_cast<int*>(smem);
     glm_locate_block(p.offs, p.G, p.R, 64, blockIdx.y, sh);
