@@ -704,11 +704,15 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
         // at 11 95.9 / 97.7, at 15 99.6 / 99.0, at 20 107 / 101, 129 of 512 x 1024 at 18 63 / 57, of 768 x 2048 at 7 133 / 137; one round: 17 of
         // 1408 x 4096 at 18 74 / 79, 65 of 352 x 4096 at 14 68 / 75.  Down 65 of 1408 x 4096 at 7 129 / 120, at 9 133 / 122, at 18 145 / 131, 129 of
         // 768 x 2048 at 7 80 / 77, at 4 68 / 73, 17 of 1408 x 4096 at 18 44 / 40, 64 of 1024 x 2048 at 11 54.7 / 54.6; 33 of 1024 x 1024 at 15 19.6 / 21.0,
-        // 9 of 2048 x 4096 at 13 31 / 40.
+        // 9 of 2048 x 4096 at 13 31 / 40.  Down with K of 256, 512 or 1024 is ahead later than with lengths
+        // between: 129 of 512 x 1024 at 7 33.0 / 34.3, at 12 34.6 / 35.0, at 20 38.1 / 35.6, 64 of
+        // 1024 x 2048 at 7 47.3 / 48.7, at 12 50.4 / 49.8, 160 of 256 x 2048 at 7 50.2 / 51.7, at 14 56 / 54, but 64 of 768 x 2048 at 9 39.9 / 38.9, 65 of
+        // 704 x 4096 at 7 77 / 72.
         const int64_t rows = p.R_hint > 0 ? p.R_hint : p.R;
         if (mode != GEMM_GATEUP && mode != GEMM_DOWN) return false;
         const int64_t G = p.G, tiles = (p.N + (mode == GEMM_GATEUP ? 31 : 63)) / (mode == GEMM_GATEUP ? 32 : 64) * G;
-        const bool enough = rows >= 24 * G || (mode == GEMM_GATEUP ? rows >= 13 * G && tiles >= 2048 : rows > 6 * G && tiles >= 1024);
+        const int few = p.K <= 1024 && (p.K & (p.K - 1)) == 0 ? 12 : 6;
+        const bool enough = rows >= 24 * G || (mode == GEMM_GATEUP ? rows >= 13 * G && tiles >= 2048 : rows > few * G && tiles >= 1024);
         return enough && rows < 96 * G && p.R * p.ldx * 2 < (1ll << 31) && (mode == GEMM_GATEUP ? 2 : 1) * (int64_t)p.N * p.ldw * 2 < (1ll << 31);
     }
     if (p.src != nullptr || p.G > 1 || p.R <= 32) return false;
