@@ -66,16 +66,18 @@ void glm_set_error(const char* fmt, ...);
 #define GLM_MAX_DEVICES 16
 #define GLM_SET_MAX_LDS(kern, bytes, name)                                                                   \
     do {                                                                                                     \
-        static bool lds_set__[GLM_MAX_DEVICES] = {};                                                         \
-        int dev__ = -1;                                                                                      \
-        if (hipGetDevice(&dev__) != hipSuccess) dev__ = -1;                                                  \
-        if (dev__ < 0 || dev__ >= GLM_MAX_DEVICES || !lds_set__[dev__]) {                                    \
-            hipError_t e__ = hipFuncSetAttribute((const void*)(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (bytes)); \
+        static const void* lds_set__[GLM_MAX_DEVICES][4] = {};  /* a call may choose among as many kernels */ \
+        const void* kern__ = (const void*)(kern);                                                            \
+        int dev__ = -1, at__ = 0;                                                                            \
+        if (hipGetDevice(&dev__) != hipSuccess || dev__ < 0 || dev__ >= GLM_MAX_DEVICES) at__ = 4;           \
+        while (at__ < 4 && lds_set__[dev__][at__] != nullptr && lds_set__[dev__][at__] != kern__) ++at__;    \
+        if (at__ == 4 || lds_set__[dev__][at__] == nullptr) {                                                \
+            hipError_t e__ = hipFuncSetAttribute(kern__, hipFuncAttributeMaxDynamicSharedMemorySize, (bytes)); \
             if (e__ != hipSuccess) {                                                                         \
                 glm_set_error("%s: hipFuncSetAttribute(%d B LDS): %s", name, (int)(bytes), hipGetErrorString(e__)); \
                 return GLM_ERR_LAUNCH;                                                                       \
             }                                                                                                \
-            if (dev__ >= 0 && dev__ < GLM_MAX_DEVICES) lds_set__[dev__] = true;                              \
+            if (at__ < 4) lds_set__[dev__][at__] = kern__;                                                   \
         }                                                                                                    \
     } while (0)
 
