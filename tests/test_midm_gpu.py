@@ -359,3 +359,22 @@ def test_few_columns(M, N, K, f32):
     want = x.double() @ w.double().T
     err = (out[:, :N].cpu().double() - want).abs().max() / want.abs().max()
     assert err < (K * 2.0 ** -24 if f32 else 2.0 ** -8) and torch.all(out[:, N:] == 7)   # sums in fp32; the result's rounding
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 17, 256), (512, 208, 320), (900, 108, 4096), (1150, 100, 512), (1000, 128, 256), (4090, 20, 320), (2700, 36, 1088)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_few_columns_row_block_by_row_block(M, N, K, f32):
+    """Many rows of few columns: the order of the tiles is another one and nothing more, ends of the grid, rows and columns included."""
+    from nanovllm import hip_ops
+    N = N - N % 4
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    out = torch.full((M + 40, N + 8), 7.0, dtype=torch.float32 if f32 else torch.bfloat16, device="cuda")
+    hip_ops.linear_act(x, w, out_f32=f32, out=out[:M, :N])
+    assert torch.all(out[:, N:] == 7) and torch.all(out[M:] == 7)
+    for r in range(0, M, 480):      # so many rows go column tile by column tile
+        n = min(480, M - r)
+        if n > 32:
+            assert torch.equal(out[r: r + n, :N], hip_ops.linear_act(x[r: r + n], w, out_f32=f32)), r
+    want = x.cpu().double() @ w.cpu().double().T
+    assert (out[:M, :N].cpu().double() - want).abs().max() / want.abs().max() < (K * 2.0 ** -24 if f32 else 2.0 ** -8)
