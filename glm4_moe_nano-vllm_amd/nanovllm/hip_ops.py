@@ -496,9 +496,10 @@ def padded_weight(rows: int, cols: int, *lead: int, dtype=None, device=None) -> 
     multiple of 16 KiB get 320: with 64, sixteen and more neighbours still share what 4 KiB select.
     64 / 320, us: 4096 x 16384 at 1 row 33.9 / 25.2, at 64 73 / 56, at 128 70 / 52, at 1000 153 / 147, at
     2 to 32 and from 4096 on equal; 4096 x 8192 at 1 15.2 / 14.1, at 32 22.8 / 21.0, at 128 29.3 / 28.3; 4096 x
-    32768 at 1 48.6 / 47.9, x 24576 equal; 4096 columns have no such rows (equal)."""
+    32768 at 1 48.6 / 47.9, x 24576 equal; 4096 columns have no such rows (equal).  They keep 64 where 320 would
+    put the last rows beyond the 32-bit offsets of the GEMM kernels (a vocabulary of 128256 x 8192)."""
     pitch = cols * 2
-    pad = 320 if pitch % 16384 == 0 else 64 if pitch % 4096 == 0 else 0
+    pad = 320 if pitch % 16384 == 0 and rows * (pitch + 640) < 1 << 31 else 64 if pitch % 4096 == 0 else 0
     t = torch.empty((*lead, rows, cols + pad), dtype=dtype, device=device)
     return t[..., :cols] if pad else t
 

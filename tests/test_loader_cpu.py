@@ -32,3 +32,13 @@ def test_prefix_matches_whole_components_and_uses_the_shard_index(tmp_path):
     assert loader.load_one(d, "model.norm.weight") is not None
     assert loader.load_one(d, f"{p}.1.gate_proj.weight") is None  # not in the map: the map is authoritative
     loader._key_index.cache_clear()
+
+
+def test_row_padding_stays_within_32_bit_offsets():
+    """The wider padding of rows of 16 KiB goes where all rows stay below 2 GiB with it; elsewhere the narrow one, as for other rows of 4 KiB."""
+    from nanovllm import hip_ops
+    pad = lambda rows, cols, *lead: hip_ops.padded_weight(rows, cols, *lead, dtype=torch.bfloat16, device="meta").stride(-2) - cols  # noqa: E731
+    assert pad(128256, 8192) == 64 and pad(126140, 8192) == 320 and pad(126150, 8192) == 64
+    assert pad(4096, 8192) == 320 and pad(4096, 16384, 64) == 320 and pad(4096, 2048) == 64 and pad(4096, 2056) == 0
+    for rows, cols in ((126140, 8192), (128256, 8192)):
+        assert rows * (cols + pad(rows, cols)) * 2 < 1 << 31
