@@ -650,21 +650,28 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         //        B2(kt-1) >= other group's B1(kt-1); every wave finished reading kt-1 before its own
         //        B1(kt-1).
         if (wid >= 4) __builtin_amdgcn_s_barrier();   // the stagger
-        int slot = 0;  // ring slot of tile kt
+        int so = 0;  // ring slot of tile kt, its offset
         for (int kt = 0; kt < nk; ++kt) {
             // ---------------- phase 1 ----------------
             u32x4_t f[C::NF];
             u32x2_t fr[C::W8 ? C::KS * 4 : 1];
-            if (kt + C::DIST < nk) stage(slot == 0 ? C::NSTAGE - 1 : slot - 1, kt + C::DIST);  // the slot of tile kt-1
+            if (kt + C::DIST < nk) {  // into the slot of tile kt-1
+                const int no = so == 0 ? (C::NSTAGE - 1) * C::STAGE : so - C::STAGE;
+                stage_w(no, kt + C::DIST);
+                stage_x(no + C::WT, kt + C::DIST);
+            }
             if constexpr (LEAN) {
-                read_frags(f, fr, slot * C::STAGE);
+                read_frags(f, fr, so);
             } else {
-                const unsigned sb = base + slot * C::STAGE;
+                const unsigned sb = base + so;
 #pragma unroll
                 for (int i = 0; i < C::NF; ++i) lds_read_b128(f[i], sb + rel[i]);
             }
             // this wave's share of tile kt+1: leave only the tiles newer than kt+1 in flight
-            dma_wait_leave<C::DPW>(min(kt + C::DIST, nk - 1) - (kt + 1));
+            if constexpr (C::DIST == 2) {
+                if (kt + C::DIST < nk) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(C::DPW) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else dma_wait_leave<C::DPW>(min(kt + C::DIST, nk - 1) - (kt + 1));
             lds_wait(f);
             frags_cvt(f, fr);
             __builtin_amdgcn_sched_barrier(0);
@@ -683,7 +690,7 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
             if constexpr (!LEAN) __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_barrier();  // B2
-            slot = slot == C::NSTAGE - 1 ? 0 : slot + 1;
+            so = so == (C::NSTAGE - 1) * C::STAGE ? 0 : so + C::STAGE;
         }
         if (wid < 4) __builtin_amdgcn_s_barrier();  // match the other group's extra barrier
         }
