@@ -26,7 +26,7 @@ struct OptDesc {
 const OptDesc k_opts[GLM_OPT_COUNT] = {
     {"tinym", "GLM4MOE_TINYM", 1},                 // 0: one token row keeps the small-M MFMA kernels (A/B, bit-identity tests)
     {"fp8w_native", "GLM4MOE_FP8W_NATIVE", 1},     // 0: fp8 experts at prefill row counts take the expansion path
-    {"largem_variant", "GLM_LARGEM_VARIANT", -1},  // >= 0: loop variant bits of the tiled GEMM (0 = the plain loop)
+    {"largem_variant", "GLM_LARGEM_VARIANT", -1},  // tiled GEMM: 0 (any but -1 and 86787) = the plain form everywhere
     {"largem_cfg", "GLM_LARGEM_CFG", 0},           // 0 = by shape, 1 = 128-row blocks (A), 2 = 256-row blocks (B)
     {"fa_mfma32", "GLM_FA_MFMA32", -1},            // -1 = the build's default, 0 = 16x16x32 kernel, 1 = 32x32x16 kernel
     {"fa_rows64", "GLM_FA_ROWS64", 0},             // 1 = prefill attention with 64 query rows per wave (prefill_attn64.hip)

@@ -144,11 +144,12 @@ int glm_tinym_max_rows();
 int glm_launch_gemm_tinym(int mode, const GemmParams& p, int n_tokens, hipStream_t st);
 // ... with the activation rows COMPUTED in the kernel: moe_combine(y_prev) + add-RMSNorm (the previous MoE block's combine
 // and this layer's input norm), p.x ignored; residual_out / x_out (optional) written by one workgroup
-int glm_launch_gemm_tinym_residual(const GemmParams& p, const float* x_in, const int32_t* rows, const void* y, int64_t ldy, const void* table, int64_t ldt, int64_t vocab,
-                                   const int64_t* ids, float* x_out, const float* g, int width, float eps, hipStream_t st);
 int glm_launch_gemm_tinym_combine_norm(const GemmParams& p, const void* y_prev, int64_t ld_yprev, const int32_t* pair_pos,
                                        int k, int64_t shared_base, const void* residual_in, const void* norm_w,
                                        void* residual_out, void* x_out, float eps, hipStream_t st);
+// ... or the norm of one row of an fp32 residual and of what it takes up (glm_residual_norm)
+int glm_launch_gemm_tinym_residual(const GemmParams& p, const float* x_in, const int32_t* rows, const void* y, int64_t ldy, const void* table, int64_t ldt, int64_t vocab,
+                                   const int64_t* ids, float* x_out, const float* g, int width, float eps, hipStream_t st);
 // ... and, for ONE row, continued by the post-attention add-RMSNorm + router + bucketing in the last workgroup to finish
 int glm_launch_gemm_tinym_router_tail(const GemmParams& p, unsigned* ticket, float* logits_scratch, const void* residual_in, const void* norm_w,
                                       float eps, void* y_norm, void* residual_out, const void* gate_w, const float* bias, int E,
