@@ -53,12 +53,15 @@ struct Slab {
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(-2.f * cap_out, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r] * cap_in)), cap_out);
     }
-    // largest magnitude of the eight scores
+    // Largest of the eight scores, largest magnitude.  Not fmaxf: hipcc quiets every operand of one first.  Not inline asm: the compiler does not know how
+    // long an MFMA's result takes to get there for such a reader, and does not wait (with both maps' scores beside it, the choice between tanh's two forms
+    // changed from run to run).  A not-a-number comes out of these, for a row that is one anyway.
+    __device__ __forceinline__ static float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
+    __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
+        return __builtin_elementwise_maximum(max3(max3(max3(s[0][0], s[0][1], s[0][2]), s[0][3], s[1][0]), s[1][1], s[1][2]), s[1][3]);
+    }
     __device__ __forceinline__ static float size(const f32x4_t (&s)[2]) {
-        float m;
-        asm("v_max3_f32 %0, abs(%1), abs(%2), abs(%3)\n\tv_max3_f32 %0, %0, abs(%4), abs(%5)\n\tv_max3_f32 %0, %0, abs(%6), abs(%7)\n\tv_max_f32 %0, %0, abs(%8)"
-            : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
-        return m;
+        return __builtin_elementwise_maximum(max3(max3(max3(fabsf(s[0][0]), fabsf(s[0][1]), fabsf(s[0][2])), fabsf(s[0][3]), fabsf(s[1][0])), fabsf(s[1][1]), fabsf(s[1][2])), fabsf(s[1][3]));
     }
     // up to a fifth of the cap tanh is its odd polynomial of degree 7 (the next term is below 2e-8 of the cap)
     __device__ __forceinline__ void cap_small(f32x4_t (&s)[2]) const {
@@ -203,13 +206,6 @@ struct Slab {
         for (int i = 1; i < KQ; ++i)
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt) add_score<T>(s, kf, kt, i, s[kt]);
-    }
-    // largest of the eight scores (inline asm: hipcc would quiet every operand of a maximum first)
-    __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
-        float m;
-        asm("v_max3_f32 %0, %1, %2, %3\n\tv_max3_f32 %0, %0, %4, %5\n\tv_max3_f32 %0, %0, %6, %7\n\tv_max_f32 %0, %0, %8"
-            : "=&v"(m) : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]), "v"(s[1][3]));
-        return m;
     }
     // weights of tile T; fac: sigmoid form, factors of the lane's keys times scale and log2 e, negative; EDGE: some keys may be hidden; CAPPED: the scores
     template <int T, bool EDGE, bool CAPPED = false>

@@ -370,6 +370,37 @@ def test_group_attn_prefill_padding_is_zero(form, G, dim, dv):
             assert (got[:, h] - ref).abs().max() < (2e-2 if form != "sigmoid" else 2 ** -8 * float(ref.abs().max()) + 2e-2), (wk, wv, h)
 
 
+@pytest.mark.parametrize("form", ["softmax", "two_maps", "two_maps_any"])
+@pytest.mark.parametrize("dim,dv", [(32, 64), (32, 128), (64, 64), (64, 128), (128, 128)])
+def test_group_attn_prefill_repeats_itself(form, dim, dv):
+    """The same bits every time, whatever ran before: prompts of one, two and more key tiles, scores on both sides of a fifth of the cap, where the cap's two forms part."""
+    from nanovllm import hip_ops
+    maps, bs, G, H = 1 if form == "softmax" else 2, 64, 4, 16
+    lens = [64, 40, 128, 100, 64, 300, 17, 63]
+    qs = [0]
+    for n in lens:
+        qs.append(qs[-1] + n)
+    nb = [-(-n // bs) for n in lens]
+    bt = torch.full((len(lens), max(nb)), -1, dtype=torch.int32)
+    for s, n in enumerate(nb):
+        bt[s, :n] = torch.arange(sum(nb[:s]), sum(nb[: s + 1]))
+    q = torch.randn(qs[-1], H * maps * dim, generator=g(1)) * (1 + 7 * (torch.arange(qs[-1]) % 3 == 0)[:, None])
+    kc, vc = torch.randn(sum(nb), G, bs, maps * dim, generator=g(2)), torch.randn(sum(nb), G, bs, dv, generator=g(3))
+    parts = hip_ops.GroupParts() if maps == 1 else hip_ops.GroupParts(maps=2, cap=20.0 if form == "two_maps" else 70.0, lam=0.4, post=0.6, eps=1e-3, vn=dv)
+    tiles = [(s, o) for s, n in enumerate(lens) for o in range(0, n, hip_ops.group_attn_tile_rows(H, G, maps))]
+    qd, kd, vd = (dev(t, torch.bfloat16) for t in (q, kc, vc))
+    args = (i32(bt), 0, i32(qs), i32(torch.cat([torch.arange(n) for n in lens])), i32([t[0] for t in tiles]), i32([t[1] for t in tiles]), H, 0, 0, 0.5 * dim ** -0.5, None, None)
+
+    def run(q):
+        out = torch.empty(qs[-1], H * dv, dtype=torch.bfloat16, device="cuda")
+        hip_ops.group_attn_prefill(q, kd, vd, *args, out, parts=parts)
+        return out
+    first = run(qd)
+    for i in range(12):
+        run(qd * (0.01 if i % 2 else 30.0))     # small scores and large ones leave other values behind
+        assert torch.equal(run(qd), first), i
+
+
 # ---- the model through the engine -------------------------------------------------------------------------------------------
 @pytest.fixture(scope="module", params=list(CONFIGS))
 def model(request, tmp_path_factory):
