@@ -53,15 +53,12 @@ struct Slab {
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(-2.f * cap_out, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[kt][r] * cap_in)), cap_out);
     }
-    // Largest of the eight scores, largest magnitude.  Not fmaxf: hipcc quiets every operand of one first.  Not inline asm: the compiler does not know how
-    // long an MFMA's result takes to get there for such a reader, and does not wait (with both maps' scores beside it, the choice between tanh's two forms
-    // changed from run to run).  A not-a-number comes out of these, for a row that is one anyway.
-    __device__ __forceinline__ static float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
-    __device__ __forceinline__ static float largest(const f32x4_t (&s)[2]) {
-        return __builtin_elementwise_maximum(max3(max3(max3(s[0][0], s[0][1], s[0][2]), s[0][3], s[1][0]), s[1][1], s[1][2]), s[1][3]);
-    }
+    // Largest magnitude of the eight scores, as glm_largest8.  (Inline asm right behind the products: the choice between tanh's two forms changed from run to run.)
     __device__ __forceinline__ static float size(const f32x4_t (&s)[2]) {
-        return __builtin_elementwise_maximum(max3(max3(max3(fabsf(s[0][0]), fabsf(s[0][1]), fabsf(s[0][2])), fabsf(s[0][3]), fabsf(s[1][0])), fabsf(s[1][1]), fabsf(s[1][2])), fabsf(s[1][3]));
+        f32x4_t m[2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m[i >> 2][i & 3] = fabsf(s[i >> 2][i & 3]);
+        return glm_largest8(m);
     }
     // up to a fifth of the cap tanh is its odd polynomial of degree 7 (the next term is below 2e-8 of the cap)
     __device__ __forceinline__ void cap_small(f32x4_t (&s)[2]) const {
@@ -236,7 +233,7 @@ struct Slab {
         }
         float m_use = 0.f;
         if constexpr (F == GA_SOFTMAX || F == GA_TWO_MAPS_ANY) {
-            float mx = largest(s) * sc;
+            float mx = glm_largest8(s) * sc;
             if (__any(mx > m_run[T] + 8.0f || (m_run[T] == -INFINITY && mx > -INFINITY))) {
                 mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
                 mx = fmaxf(mx, __shfl_xor(mx, 32, 64));

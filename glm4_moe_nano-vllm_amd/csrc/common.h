@@ -81,5 +81,12 @@ void glm_set_error(const char* fmt, ...);
         }                                                                                                    \
     } while (0)
 
+// Largest of the eight scores of two MFMA results.  Not fmaxf: hipcc quiets every operand of one first.  Not inline asm: the compiler does not know how
+// long an MFMA's result takes to get there for such a reader, and does not wait.  A not-a-number comes out, for a row that is one anyway.
+__device__ __forceinline__ float glm_max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
+__device__ __forceinline__ float glm_largest8(const f32x4_t (&s)[2]) {
+    return __builtin_elementwise_maximum(glm_max3(glm_max3(glm_max3(s[0][0], s[0][1], s[0][2]), s[0][3], s[1][0]), s[1][1], s[1][2]), s[1][3]);
+}
+
 static inline bool glm_aligned16(const void* p) { return (((uintptr_t)p) & 15) == 0; }
 static inline hipStream_t glm_s(glm_stream_t s) { return (hipStream_t)s; }

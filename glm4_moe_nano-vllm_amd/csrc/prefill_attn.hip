@@ -425,27 +425,11 @@ __global__ __launch_bounds__(FA_NT, (FA_QT >= 4 ? 1 : 2)) void prefill_attn_kern
         // Slow path: exact row maximum over the four 16-lane groups that share a query column (VALU lane swaps, one
         // asm block: hipcc pads every separate asm VALU op with an s_nop), new reference point, rescale.
         auto maxchain = [&]() -> float {
-            float mloc;
 #if GLM_FA_CINIT
-            asm("v_max3_f32 %0, %1, %2, %3\n\t"
-                "v_max3_f32 %0, %0, %4, %5\n\t"
-                "v_max3_f32 %0, %0, %6, %7\n\t"
-                "v_max_f32 %0, %0, %8"
-                : "=&v"(mloc)
-                : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]),
-                  "v"(s[1][3]));
+            return glm_largest8(s);
 #else
-            // (the scale multiply sits inside the block: hipcc pads the boundary of an asm VALU block with an s_nop)
-            asm("v_max3_f32 %0, %1, %2, %3\n\t"
-                "v_max3_f32 %0, %0, %4, %5\n\t"
-                "v_max3_f32 %0, %0, %6, %7\n\t"
-                "v_max_f32 %0, %0, %8\n\t"
-                "v_mul_f32 %0, %9, %0"
-                : "=&v"(mloc)
-                : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]),
-                  "v"(s[1][3]), "s"(scale_log2e));
+            return scale_log2e * glm_largest8(s);
 #endif
-            return mloc;
         };
 #if GLM_FA_CINIT
         // S' = c*s - m_cur, m_cur = the reference point the accumulators started from (m_run, or 0 before the first unit)

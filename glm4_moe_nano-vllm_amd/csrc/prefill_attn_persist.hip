@@ -330,18 +330,7 @@ __global__ __launch_bounds__(P_NT, 2) void prefill_attn_persist_kernel(
                     if (j > jmax[qt] || j >= lk) s[tt][r] = -INFINITY;
                 }
         }
-        auto maxchain = [&]() -> float {
-            float mloc;
-            asm("v_max3_f32 %0, %1, %2, %3\n\t"
-                "v_max3_f32 %0, %0, %4, %5\n\t"
-                "v_max3_f32 %0, %0, %6, %7\n\t"
-                "v_max_f32 %0, %0, %8\n\t"
-                "v_mul_f32 %0, %9, %0"
-                : "=&v"(mloc)
-                : "v"(s[0][0]), "v"(s[0][1]), "v"(s[0][2]), "v"(s[0][3]), "v"(s[1][0]), "v"(s[1][1]), "v"(s[1][2]),
-                  "v"(s[1][3]), "s"(scale_log2e));
-            return mloc;
-        };
+        auto maxchain = [&]() -> float { return scale_log2e * glm_largest8(s); };
         float ms = 0.f;
         float m_use = m_run[qt];
         const bool first_unit = TK == 2 ? false : kbase == 0;

@@ -125,6 +125,15 @@ def test_one_token_fusions_refuse_two_rows():
     assert not hip_ops.can_gemm_router_tail(torch.zeros(2, 512, dtype=torch.bfloat16), 4096, 64)
 
 
+def test_no_asm_takes_maxima_of_mfma_results():
+    """The compiler does not count the wait states between an MFMA and an inline-asm reader of its result: maxima of scores are its own instructions (common.h,
+    glm_largest8).  prefill_attn64.hip issues its MFMAs from asm as well, with the waits in it (next test)."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "glm4_moe_nano-vllm_amd", "csrc")
+    for f in sorted(os.listdir(csrc)):
+        if f != "prefill_attn64.hip":
+            assert "v_max3_f32" not in open(os.path.join(csrc, f)).read(), f
+
+
 def test_asm_mfma_statements_have_no_compiler_placed_hazards():
     """csrc/prefill_attn64.hip issues its MFMAs from inline asm, which the compiler's hazard recogniser cannot see: a register
     copy it places right in front of one (VALU write of SrcC) or right behind one (VALU read of the result) silently corrupts
