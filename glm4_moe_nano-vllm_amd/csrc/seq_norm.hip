@@ -403,7 +403,7 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
 // others of their portion in front of them form those as well, as the stream kernel does: the next row is requested in front of this one's sums, and the sum over
 // this x_out^2 and the one over the next y^2 share a barrier.  The arithmetic is the stream kernel's. ----
 template <int TAPS, int NT>
-__global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm_row_kernel(const SeqNormArgs a) {
+__global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
     constexpr int HALO = TAPS - 1, NW = NT / 64;
     __shared__ float s_red[2][2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -496,7 +496,44 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
     int n = 0, e = 0, d = 0, p = 0;  // tokens of the portion, of them behind this row and (as far as the taps reach) in front of it; the row's position
     int64_t so = -1;
     bool keep = false;
-    float ry = 0.f;
+    // the row itself: y with its scale, the h of the tokens in front of it
+    auto finish = [&](Row8& x, const Row8& y, float ry, const Row8 (&hist)[TAPS]) __attribute__((always_inline)) {
+        residual(x, y, ry);
+        if (on) {
+            if (a.x_out) sn_st8f(a.x_out + r0 * a.ldx + c, x);
+            if (a.x_cast) sn_st8(a.x_cast, r0 * a.ldc + c, a.act_f32, x);
+        }
+        if (!a.g_pre) return;
+        const Row8 h = normed(x, rms(reduce(sn_sumsq8(x))));
+        Row8 o = h;
+        if constexpr (TAPS > 1) {
+            auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
+            Row8 acc = zero;
+#pragma unroll
+            for (int k = HALO; k >= 1; --k) {
+                const bool there = k <= d || p - k >= 0;  // (in front of the sequence the state holds nothing)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * (there ? hist[k - 1].a[i] : 0.f);
+                    acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * (there ? hist[k - 1].b[i] : 0.f);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
+                o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
+            }
+            if (keep) {
+                float* to = a.state + so * HALO * a.wp + c;
+                sn_st8f(to + (int64_t)(HALO - 1 - e) * a.wp, h);
+                // a portion shorter than the history, whose rows are n = d + 1 with the last one: the older inputs move up
+#pragma unroll
+                for (int k = 1; k < HALO; ++k)
+                    if (e == 0 && k + n <= HALO) sn_st8f(to + (int64_t)(k - 1) * a.wp, hist[HALO - k - 1]);
+            }
+        }
+        if (on) sn_st8(a.h, r0 * a.ldh + c, a.act_f32, o);
+    };
     if constexpr (TAPS > 1) {
         const int s = a.seq_of[r0], qs = a.q_start[s], qe = a.q_start[s + 1];
         p = a.pos[r0];
@@ -512,9 +549,10 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
             hist[k - 1] = zero;
             if (on && r0 - d == qs) hist[k - 1] = sn_ld8f(st + (int64_t)(HALO - k) * a.wp);
         }
-        if (d > 0) {  // (uniform; this row comes again, out of the cache)
+        // (uniform; this row comes again, out of the cache.  It ends here by itself: joining the others would make them wait for what is on its way)
+        if (d > 0) {
             Row8 xn, yn;
-            float sv;
+            float sv, ry = 0.f;
             load_row(r0 - d, x, y, std::integral_constant<int, 2>{});
             if (a.y) ry = rms(reduce(sn_sumsq8(y)));
             for (int64_t q = r0 - d; q < r0; ++q) {
@@ -528,44 +566,11 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
                 x = xn;
                 y = yn;
             }
+            finish(x, y, ry, hist);
+            return;
         }
     }
-    if (a.y && d == 0) ry = rms(reduce(sn_sumsq8(y)));
-    residual(x, y, ry);
-    if (on) {
-        if (a.x_out) sn_st8f(a.x_out + r0 * a.ldx + c, x);
-        if (a.x_cast) sn_st8(a.x_cast, r0 * a.ldc + c, a.act_f32, x);
-    }
-    if (!a.g_pre) return;
-    const Row8 h = normed(x, rms(reduce(sn_sumsq8(x))));
-    Row8 o = h;
-    if constexpr (TAPS > 1) {
-        auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
-        Row8 acc = zero;
-#pragma unroll
-        for (int k = HALO; k >= 1; --k) {
-            const bool there = k <= d || p - k >= 0;  // (in front of the sequence the state holds nothing)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * (there ? hist[k - 1].a[i] : 0.f);
-                acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * (there ? hist[k - 1].b[i] : 0.f);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
-            o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
-        }
-        if (keep) {
-            float* to = a.state + so * HALO * a.wp + c;
-            sn_st8f(to + (int64_t)(HALO - 1 - e) * a.wp, h);
-            // a portion shorter than the history, whose rows are n = d + 1 with the last one: the older inputs move up
-#pragma unroll
-            for (int k = 1; k < HALO; ++k)
-                if (e == 0 && k + n <= HALO) sn_st8f(to + (int64_t)(k - 1) * a.wp, hist[HALO - k - 1]);
-        }
-    }
-    if (on) sn_st8(a.h, r0 * a.ldh + c, a.act_f32, o);
+    finish(x, y, a.y ? rms(reduce(sn_sumsq8(y))) : 0.f, hist);
 }
 
 template <int TAPS, int NT>
