@@ -584,9 +584,9 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
     if constexpr (NT < 1024 || TAPS == 1) {  // (1024 threads do not have the registers for rows, taps and history at once)
         // With taps: portions of one row, up to three quarters of the CUs.  Longer ones take the stream kernel, which knows where a portion begins before it
-        // asks for a row; with a row per CU and more there is less to hide.  Stream / row kernel, four taps, us: two slabs of 2048 columns, 1 row 4.87 /
-        // 4.68, 32 5.23 / 5.05, 128 6.26 / 6.27, 200 7.10 / 7.08, 256 7.52 / 7.62, four slabs 1 5.36 / 4.78, 128 7.25 / 6.96; two of 4096, 1 5.88 / 5.17, 128 8.56 /
-        // 7.91, 256 10.63 / 10.40; prompts of 64, 211 and 512 tokens, two slabs of 2048, 8.8 / 9.3, 9.9 / 10.3, 14.6 / 15.5, without the pipeline of the rows in
+        // asks for a row; with a row per CU and more there is less to hide.  Stream / row kernel, four taps, us: two slabs of 2048 columns, 1 row 4.96 /
+        // 4.70, 32 5.24 / 5.01, 128 6.20 / 6.02 (6.27 with one end for both branches), 200 7.10 / 7.08, 256 7.52 / 7.62, four slabs 1 5.40 / 4.84, 128 7.22 / 6.82; two of
+        // 4096, 1 5.96 / 5.16, 128 8.67 / 8.04, 256 10.63 / 10.40; prompts of 64, 211 and 512 tokens, two slabs of 2048, 8.8 / 9.3, 9.9 / 10.3, 14.6 / 15.5, without the pipeline of the rows in
         // front 10.3, 11.0, 15.2.  No taps: 2048 columns, 1 row 3.74 / 3.54, 512 6.79 / 6.32.
         if (TAPS == 1 ? a.T <= 512 : a.T <= 192 && (n_seq <= 0 || n_seq >= a.T)) {
             hipLaunchKernelGGL((seq_norm_row_kernel<TAPS, NT>), dim3((unsigned)a.T), dim3(NT), 0, st, a);
