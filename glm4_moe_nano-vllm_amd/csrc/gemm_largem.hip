@@ -215,6 +215,7 @@ __device__ __forceinline__ void lm_locate_lanes(const int32_t* __restrict__ offs
 template <int MODE, class C, bool LEAN, bool WSCALE>
 __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND) {
     constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP;  // may store fp32 rows (p.yf)
+    constexpr bool BIAS = MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP;
     static_assert(LEAN || (!C::RING && !C::W8 && !C::A8), "the plain form has the plain ring");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -447,9 +448,8 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         });
     };
 
-    // Store instructions a wave issues behind the ring fill of the next tile, where their number is known exactly (all rows and
-    // columns of the tile exist): the waits that open a tile leave that many in flight (vmcnt counts in issue order).  -1: not
-    // known, wait for everything.
+    // Store instructions a wave issues behind the ring fill of the next tile, where their number is known: the waits that open a tile
+    // leave that many in flight (vmcnt counts in issue order).  -1: not known, wait for everything.
     constexpr int LM_NOUT = gemm_paired(MODE) ? 2 : 4;
     constexpr int STORES = C::MT * LM_NOUT / 2, STORES_F32 = C::MT * 4;
     int pending_stores = 0;
@@ -472,7 +472,6 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < C::MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        float sc_pre[C::MT];  // per-row scales of this tile (down projection), loaded before its epilogue
         using I0 = std::integral_constant<int, 0>;
         using I4 = std::integral_constant<int, 4>;
 
@@ -695,17 +694,36 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         if (wid < 4) __builtin_amdgcn_s_barrier();  // match the other group's extra barrier
         }
 
-        // per-row scales of the finished tile: requested before the ring fill (waiting for a load issued after the fill
-        // would drain the fill first)
-        if constexpr (LEAN && MODE == GEMM_DOWN) {
-            const bool sc_on = grp_c < p.n_scaled;
+        // What the epilogue reads of the finished tile's rows and columns: requested in front of the ring fill (waiting for a load issued behind the
+        // fill would drain the fill first).
+        float e_row[C::MT], e_col[4][4];
+        unsigned e_bias[4][2];
+        if constexpr (LEAN) {
+            if constexpr (MODE == GEMM_DOWN) {
+                const bool sc_on = grp_c < p.n_scaled;
 #pragma unroll
-            for (int mt = 0; mt < C::MT; ++mt) {
-                const int row = wm * (C::BM / 2) + 16 * mt + c;
-                sc_pre[mt] = (sc_on && row < mcnt_c) ? bf2f(p.scale[m0_c + row]) : 1.0f;
+                for (int mt = 0; mt < C::MT; ++mt) {
+                    const int row = wm * (C::BM / 2) + 16 * mt + c;
+                    e_row[mt] = (sc_on && row < mcnt_c) ? bf2f(p.scale[m0_c + row]) : 1.0f;
+                }
             }
+            // column of the wave's first output column, or gate column, of tile t
+            auto col = [&](int t, int r) { return gemm_paired(MODE) ? ntile_c * 128 + wn * 32 + 16 * (t & 1) + 4 * g4 + r : ntile_c * LM_BN + wn * 64 + 16 * t + 4 * g4 + r; };
+            if constexpr (WSCALE && !(C::A8 && gemm_paired(MODE))) {
 #pragma unroll
-            for (int mt = 0; mt < C::MT; ++mt) asm volatile("" : "+v"(sc_pre[mt]));  // the loads stay above the fill
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        e_col[t][r] = p.wscale[(int64_t)grp_c * p.wscale_gstride + (gemm_paired(MODE) && t > 1 ? p.N : 0) + min(col(t, r), p.N - 1)];
+            }
+            if constexpr (BIAS) {
+                if (p.bias != nullptr && (MODE != GEMM_PLAIN || p.qkv_q == nullptr)) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; r += 2) e_bias[t][r >> 1] = p.bias[min(col(t, r), p.N - 1)] | (unsigned)p.bias[min(col(t, r + 1), p.N - 1)] << 16;
+                }
+            }
         }
         // ---- next tile: every wave is past its last LDS read, so the ring can be refilled right away ----
         const bool more = find_tile();
@@ -714,11 +732,26 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         // There the next tile's fill is issued once the first 16-row block of the epilogue has its loads back, i.e. behind them and
         // in front of the bulk of the stores.  (The scale vectors as LDS-DMA pieces of the ring fill: no gain.)
         constexpr bool LATE_FILL = C::A8;
-        if (more) setup_sources();   // (its own loads — the gathered source rows — go out here, in front of the epilogue's)
+        if (more) setup_sources();   // (its own loads — the gathered source rows — go out here, behind the epilogue's)
+        if constexpr (LEAN && MODE == GEMM_DOWN) {
+#pragma unroll
+            for (int mt = 0; mt < C::MT; ++mt) asm volatile("" : "+v"(e_row[mt]));  // the loads stay above the fill
+        }
+        if constexpr (LEAN && WSCALE && !(C::A8 && gemm_paired(MODE))) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(e_col[i >> 2][i & 3]));
+        }
+        if constexpr (LEAN && BIAS) {
+            if (p.bias != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(e_bias[i >> 1][i & 1]));
+            }
+        }
         auto start_next = [&]() {
             if (more) fill_ring();
         };
         if constexpr (!LATE_FILL) start_next();
+        __builtin_amdgcn_sched_barrier(0);   // (pending_stores counts on the order)
 
         // ---- epilogue of the finished tile ----
         int stored = -1;  // (pending_stores)
@@ -855,29 +888,98 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
                 if (row_ok && g4 == 0) p.ybscale[m * 64 + wn * 16 + ntile_c] = (unsigned char)sb;
                 if (mt == 0) start_next();
             }
+        } else if constexpr (LEAN) {
+            // Decisions (bias, scale, kind of column) once per wave and not per element, and stores through a buffer of the tile's own rows and columns: what lies
+            // behind them is dropped by the bounds check, so every store is issued and its address is one addition.  Between a tile's loops the matrix pipe
+            // stands still: the instructions here are what counts.  15074 rows, us, with a test and a 64-bit address per element or row / this: 6144 x
+            // 2048 with a bias 329 / 285, xIELU 314 / 298, 4096 x 2048 half of them gates 207 / 188, 8192 x 2048 of SiLU and gates 411 / 377, 10240 x
+            // 2048 of three kinds 507 / 467, plain 6144 x 2048 283 / 281; down of 8 of 64 experts, 4096 x 1408, 1258 / 1238.
+            constexpr unsigned BEYOND = 0x80000000u;
+            const bool f32 = F32ROWS && (MODE != GEMM_ACT || p.yf != nullptr);   // (the others have no bf16 form here)
+            const unsigned es = f32 ? 4u : 2u, pitch = (unsigned)p.ldy * es;   // (256 rows are below 2 GiB: launch_largem)
+            const int64_t first = ((MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0) + m0_c) * p.ldy + ncol_w;
+            char* ybase = f32 ? reinterpret_cast<char*>(p.yf + first) : reinterpret_cast<char*>(p.y + first);
+            const unsigned bytes = ncol_w < p.N ? (unsigned)(mcnt_c - 1) * pitch + (unsigned)(p.N - ncol_w) * es : 0u;
+            const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(ybase, 0, bytes, 0x00020000);
+            const unsigned lrow = (unsigned)(wm * (C::BM / 2) + c) * pitch;
+            // stores f of every element
+            auto finish = [&](auto&& f) __attribute__((always_inline)) {
+                if constexpr (LATE_FILL) start_next();   // (its loads of scales are back: pinned above)
+                if constexpr (F32ROWS) {
+                    if (f32) {   // four columns per store
+#pragma unroll
+                        for (int mt = 0; mt < C::MT; ++mt) {
+#pragma unroll
+                            for (int t = 0; t < NOUT; ++t) {
+                                const int n = 16 * t + 4 * g4;
+                                f32x4_t o;
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) o[r] = f(t, mt, r);
+                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, (ncol_w + n < p.N ? lrow + n * 4 : BEYOND) + 16 * mt * pitch, 0, 0);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        return;
+                    }
+                }
+                // tiles (t, t+1): after the swaps lane row g4 holds 8 consecutive columns of tile t + (g4 & 1),
+                // starting at column 8 * (g4 >> 1)
+#pragma unroll
+                for (int mt = 0; mt < C::MT; ++mt) {
+#pragma unroll
+                    for (int t = 0; t < NOUT; t += 2) {
+                        const int n = 16 * (t + (g4 & 1)) + 8 * (g4 >> 1);
+                        const u32x2_t a = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 0), f(t, mt, 1)), pack2bf(f(t + 1, mt, 0), f(t + 1, mt, 1)), false, false);
+                        const u32x2_t b = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 2), f(t, mt, 3)), pack2bf(f(t + 1, mt, 2), f(t + 1, mt, 3)), false, false);
+                        __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{a[0], b[0], a[1], b[1]}, yrs, (ncol_w + n < p.N ? lrow + n * 2 : BEYOND) + 16 * mt * pitch, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);   // (the other rows' values would take registers that are not there)
+                }
+            };
+            auto sum = [&](int t, int mt, int r) { return WSCALE ? acc[t][mt][r] * e_col[t][r] : acc[t][mt][r]; };
+            if constexpr (gemm_paired(MODE)) {
+                finish([&](int t, int mt, int r) {
+                    const float g = sum(t, mt, r), u = sum(t + 2, mt, r);
+                    return MODE == GEMM_GLU ? glm_glu_fast(p.act, g, u) : rbf(glm_silu(rbf(g))) * rbf(u);
+                });
+            } else if constexpr (MODE == GEMM_DOWN) {
+                if (scaled) finish([&](int t, int mt, int r) { return rbf(sum(t, mt, r)) * e_row[mt]; });
+                else finish(sum);
+            } else {
+                auto act = [&](float a, int t, int r) {
+                    const int n = ncol_w + 16 * t + 4 * g4 + r;
+                    if constexpr (MODE == GEMM_XIELU) return glm_xielu_fast(p.act.a, p.act.b, a);
+                    else if constexpr (MODE == GEMM_CAP) return p.act.a * tanhf(a / p.act.a);
+                    else if constexpr (MODE == GEMM_COLS) return glm_act_cols(p.act, a, n);
+                    else if constexpr (MODE == GEMM_ACT) return f32 ? glm_act_precise(p.act, a, n) : glm_act_fast(p.act, a, n);
+                    else return a;
+                };
+                bool plain = !BIAS || p.bias == nullptr;
+                if (plain) {
+                    if constexpr (MODE == GEMM_COLS) {   // (a wave's 64 columns are of one kind nearly always)
+                        const int n1 = ncol_w + 64, ca = (int)p.act.a, cb = (int)p.act.b;
+                        const bool relu2 = p.act.kind == GLM_ACT_RELU2_GATE, silu = p.act.kind == GLM_ACT_SILU_GATE;
+                        auto sigmoid = [&](float a) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * a)); };
+                        if (relu2 && n1 <= ca && n1 <= cb) finish([&](int t, int mt, int r) { return fmaxf(acc[t][mt][r], 0.f) * fmaxf(acc[t][mt][r], 0.f); });
+                        else if (relu2 ? ncol_w >= ca && n1 <= cb : !silu && n1 <= ca) finish(sum);
+                        else if (ncol_w >= (relu2 ? cb : ca)) finish([&](int t, int mt, int r) { return sigmoid(acc[t][mt][r]); });
+                        else if (silu && n1 <= ca) finish([&](int t, int mt, int r) { return acc[t][mt][r] * sigmoid(acc[t][mt][r]); });
+                        else finish([&](int t, int mt, int r) { return act(acc[t][mt][r], t, r); });
+                    } else {
+                        finish([&](int t, int mt, int r) { return act(acc[t][mt][r], t, r); });
+                    }
+                } else if constexpr (BIAS) {
+                    finish([&](int t, int mt, int r) { return act(acc[t][mt][r] + (r & 1 ? bfhi(e_bias[t][r >> 1]) : bflo(e_bias[t][r >> 1])), t, r); });
+                }
+            }
+            if (!LATE_FILL) stored = f32 ? STORES_F32 : STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
         } else {
-        // weight-row scales of this wave's output columns: loaded ONCE, in front of the row blocks (and, for the fp8 x fp8
-        // kernels, in front of the next tile's ring fill)
-        float wsv[WSCALE && MODE != GEMM_GATEUP ? 4 : 1][4];
-        if constexpr (WSCALE && MODE != GEMM_GATEUP) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    wsv[t][r] = p.wscale[(int64_t)grp_c * p.wscale_gstride + min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)];
-        }
 #pragma unroll
         for (int mt = 0; mt < C::MT; ++mt) {
-            if constexpr (LATE_FILL) {
-                if (mt == 1) start_next();
-            }
             const int row = wm * (C::BM / 2) + 16 * mt + c;
             const bool row_ok = row < mcnt_c;
             bf16_t* yrow = p.y + (int64_t)(m0_c + (row_ok ? row : 0)) * p.ldy;
-            float sc;
-            if constexpr (LEAN && MODE == GEMM_DOWN) sc = sc_pre[mt];
-            else sc = (scaled && row_ok) ? bf2f(p.scale[m0_c + row]) : 1.0f;
-            u32x2_t v[NOUT];  // packed columns 4*g4 .. 4*g4+3 of output tile t
+            const float sc = (scaled && row_ok) ? bf2f(p.scale[m0_c + row]) : 1.0f;
 #pragma unroll
             for (int t = 0; t < NOUT; ++t) {
                 float o[4];
@@ -885,7 +987,7 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
                 for (int r = 0; r < 4; ++r) {
                     if (gemm_paired(MODE)) {
                         float ga = acc[t][mt][r], ua = acc[t + 2][mt][r];
-                        if constexpr (WSCALE) {  // weights expanded from fp8: per-row scale on the fp32 accumulators (uniform branch)
+                        if constexpr (WSCALE) {  // weights expanded from fp8: per-row scale on the fp32 accumulators
                             const float* ws = p.wscale + (int64_t)grp_c * p.wscale_gstride;
                             const int n1 = min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1);
                             ga *= ws[n1];
@@ -894,8 +996,8 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
                         o[r] = MODE == GEMM_GLU ? glm_glu_fast(p.act, ga, ua) : rbf(glm_silu(rbf(ga))) * rbf(ua);
                     } else {
                         float a = acc[t][mt][r];
-                        if constexpr (WSCALE) a *= wsv[t][r];
-                        if ((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP) && p.bias) a += bf2f(p.bias[min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)]);
+                        if constexpr (WSCALE) a *= p.wscale[(int64_t)grp_c * p.wscale_gstride + min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)];
+                        if (BIAS && p.bias) a += bf2f(p.bias[min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)]);
                         if (scaled) a = rbf(a) * sc;
                         if (MODE == GEMM_XIELU) a = glm_xielu_fast(p.act.a, p.act.b, a);
                         if (MODE == GEMM_CAP) a = p.act.a * tanhf(a / p.act.a);
@@ -904,37 +1006,16 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
                         o[r] = a;
                     }
                 }
+                const int n = ncol_w + 16 * t + 4 * g4;
                 if (F32ROWS && p.yf != nullptr) {  // fp32 rows: four columns per store
-                    const int n = ncol_w + 16 * t + 4 * g4;
                     const int64_t slab = MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0;
                     if (row_ok && n < p.N) *reinterpret_cast<f32x4_t*>(p.yf + (slab + m0_c + row) * p.ldy + n) = f32x4_t{o[0], o[1], o[2], o[3]};
                     continue;
                 }
-                v[t] = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
-            }
-            if (F32ROWS && p.yf != nullptr) continue;
-            if constexpr (LEAN) {
-                // tiles (t, t+1): after the swaps lane row g4 holds 8 consecutive columns of tile t + (g4 & 1),
-                // starting at column 8 * (g4 >> 1)
-#pragma unroll
-                for (int t = 0; t < NOUT; t += 2) {
-                    const u32x2_t a = __builtin_amdgcn_permlane16_swap(v[t][0], v[t + 1][0], false, false);
-                    const u32x2_t b = __builtin_amdgcn_permlane16_swap(v[t][1], v[t + 1][1], false, false);
-                    const int n = ncol_w + 16 * (t + (g4 & 1)) + 8 * (g4 >> 1);
-                    if (row_ok && n < p.N) *reinterpret_cast<u32x4_t*>(yrow + n) = u32x4_t{a[0], b[0], a[1], b[1]};
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < NOUT; ++t) {
-                    const int n = ncol_w + 16 * t + 4 * g4;
-                    if (row_ok && n < p.N) *reinterpret_cast<u32x2_t*>(yrow + n) = v[t];
-                }
+                if (row_ok && n < p.N) *reinterpret_cast<u32x2_t*>(yrow + n) = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
             }
         }
         }
-        // (the K tail form and the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
-        if (LEAN && !LATE_FILL && !qkv_epi && mcnt_c == C::BM && ncol_w + (gemm_paired(MODE) ? 32 : 64) <= p.N)
-            stored = F32ROWS && p.yf != nullptr ? STORES_F32 : STORES;
         pending_stores = stored;
         if (!more) break;
     }
@@ -999,11 +1080,11 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
                            (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
     const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP) && p.offs == nullptr && p.N <= 128));
-    // the lean form addresses x and the group's weights through 32-bit buffer offsets and has no K tail path
+    // the lean form addresses x, the group's weights and a tile's rows of y through 32-bit buffer offsets and has no K tail path
     const int var = glm_option(GLM_OPT_LARGEM_VARIANT);
     const int64_t wrows = gemm_paired(MODE) ? 2 * (int64_t)p.N : (int64_t)p.N;
     const bool lean_ok = p.K % 64 == 0 && p.R * p.ldx * 2 < (1ll << 31) && wrows * p.ldw * 2 < (1ll << 31) &&
-                         p.N % 8 == 0 && p.ldy % 8 == 0 && glm_aligned16(p.y);
+                         p.N % 8 == 0 && p.ldy % 8 == 0 && p.ldy < (1 << 21) && glm_aligned16(p.y);
     if (p.w_fp8) {
         // fp8 weight operand: the lean form only;
         // what they do not cover (a K tail, offsets past 2^31) goes back to the caller, which expands the stack instead
@@ -1041,7 +1122,7 @@ int glm_launch_gemm_largem_a8(int mode, const GemmParams& p, hipStream_t st) {
                     p.R * p.ldx < (1ll << 31) && wrows * p.ldw < (1ll << 31) && glm_aligned16(p.x) && glm_aligned16(p.w) &&
                     (mode == GEMM_GATEUP ? (p.xscale != nullptr && p.ybscale != nullptr && p.ldy % 4 == 0 && (((uintptr_t)p.y) & 3) == 0 &&
                                             p.N % 32 == 0 && p.N <= 2048)
-                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && glm_aligned16(p.y)));
+                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && p.ldy < (1 << 21) && glm_aligned16(p.y)));
     if (!ok) {
         glm_set_error("gemm_largem(fp8 x fp8): shape not covered (mode %d R=%ld G=%d N=%d K=%d)", mode, (long)p.R, p.G, p.N, p.K);
         return GLM_ERR_UNSUPPORTED;

@@ -1096,6 +1096,28 @@ def test_gemm_large_m_several_tiles_per_workgroup(ops, K, counts):
     assert_close_bf16(got[0][rows].cpu(), a_ref, 3, 0.06, atol=1e-3, what=f"act K={K} group {e}")
 
 
+@pytest.mark.parametrize("cfg", [1, 2])
+@pytest.mark.parametrize("M,N,K", [(600, 328, 128), (385, 64, 192), (1030, 1096, 64)])
+def test_gemm_large_m_epilogues(ops, M, N, K, cfg):
+    """Every epilogue of a dense projection against the plain form (a test and an address per element), bit for bit: kinds of columns that change
+    inside a wave's 64 and at their edges, columns and rows that end inside a tile, bf16 and fp32 rows in the middle of a buffer that stays as it was."""
+    x, w, b = dev(rnd(M, K, seed=K)), dev(rnd(N, K, seed=K + 1, scale=K ** -0.5)), dev(rnd(N, seed=K + 2))
+    acts = [ops.NO_ACT, (ops.ACT_XIELU, 0.8, 0.7), (ops.ACT_SOFTCAP, 3.0, 0.0)]
+    for c in (0, 40, 64, N):
+        acts += [(ops.ACT_GATE, float(c), 0.0), (ops.ACT_SILU_GATE, float(c), 0.0), (ops.ACT_RELU2_GATE, float(c), float(min(N, c + 128)))]
+    for act in acts:
+        for bias in (None, b):
+            for f32 in (False, True):
+                got = []
+                for v in (0, -1):
+                    buf = torch.full((M + 2, N), 7.0, device="cuda", dtype=torch.float32 if f32 else BF)
+                    with largem_variant(v), ops.option("largem_cfg", cfg):
+                        ops.linear_act(x, w, bias, act, out_f32=f32, out=buf[1: M + 1])
+                    got.append(buf)
+                assert torch.equal(*got), f"{act} bias={bias is not None} f32={f32}"
+                assert bool((got[1][0] == 7).all()) and bool((got[1][-1] == 7).all())
+
+
 @pytest.mark.parametrize("seed", range(6))
 def test_gemm_large_m_quadrant_loop_random_shapes(ops, seed):
     """Random ragged groupings (empty groups, single-row groups, partial row blocks and column tiles), random K in whole
