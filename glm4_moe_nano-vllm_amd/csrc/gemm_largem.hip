@@ -216,6 +216,7 @@ template <int MODE, class C, bool LEAN, bool WSCALE>
 __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND) {
     constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP;  // may store fp32 rows (p.yf)
     constexpr bool BIAS = MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP;
+    constexpr bool GROUPED = MODE == GEMM_GATEUP || MODE == GEMM_DOWN;
     static_assert(LEAN || (!C::RING && !C::W8 && !C::A8), "the plain form has the plain ring");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -592,48 +593,57 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         };
         unsigned ow = 0, ox = C::RING ? LM_SLOT : 0, of = 4 * LM_SLOT;  // ring: slots of W(kt) and X(kt), and the free one
         auto next2 = [](unsigned o) { return o >= 3 * LM_SLOT ? o - 3 * LM_SLOT : o + 2 * LM_SLOT; };
+        // rows_a, rows_b: this wave has rows in the phase; where it has none its MFMA interval is a barrier
+        auto k_tiles = [&](auto rows_a, auto rows_b) __attribute__((always_inline)) {
 #pragma unroll 1
-        for (int kt = 0; kt < nk; ++kt) {
-            const bool has1 = kt + 1 < nk, has2 = kt + 2 < nk;
-            if constexpr (C::A8) {
-                ow = ox = (kt & 1) * C::STAGE;
-                ksh = (kt & 3) * 8;
+            for (int kt = 0; kt < nk; ++kt) {
+                const bool has1 = kt + 1 < nk, has2 = kt + 2 < nk;
+                if constexpr (C::A8) {
+                    ow = ox = (kt & 1) * C::STAGE;
+                    ksh = (kt & 3) * 8;
+                }
+                // ---- phase A
+                rd_w(ow);
+                rd_x(ox, I0{});
+                rd_s(kt);
+                __builtin_amdgcn_sched_barrier(0);  // the reads are issued before the DMA, which then runs under their round trip
+                if constexpr (C::RING) {
+                    if (has2) stage_w(of, kt + 2);
+                } else {
+                    if (has1) stage_x((ow ^ C::STAGE) + C::WT, kt + 1);
+                }
+                reads_done(true);
+                close_load();
+                if (rows_a) mfmas(I0{});
+                __builtin_amdgcn_s_barrier();
+                // ---- phase B
+                rd_x(ox, I4{});
+                __builtin_amdgcn_sched_barrier(0);
+                if (has2) {
+                    if constexpr (C::RING) stage_x(ow, kt + 2);
+                    else stage_w(ow, kt + 2);
+                }
+                reads_done(false);
+                constexpr int YOUNGER = C::RING ? C::DPW : C::W_DMA;
+                if (!has2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                else if (C::RING && kt == 0) wait_behind_stores(std::integral_constant<int, YOUNGER>{});  // (K tile 1 was issued in front of them)
+                else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(YOUNGER) : "memory");
+                close_load();
+                if (rows_b) mfmas(I4{});
+                __builtin_amdgcn_s_barrier();
+                if constexpr (C::RING) {
+                    of = ox;
+                    ow = next2(ow);
+                    ox = next2(ox);
+                }
             }
-            // ---- phase A
-            rd_w(ow);
-            rd_x(ox, I0{});
-            rd_s(kt);
-            __builtin_amdgcn_sched_barrier(0);  // the reads are issued before the DMA, which then runs under their round trip
-            if constexpr (C::RING) {
-                if (has2) stage_w(of, kt + 2);
-            } else {
-                if (has1) stage_x((ow ^ C::STAGE) + C::WT, kt + 1);
-            }
-            reads_done(true);
-            close_load();
-            mfmas(I0{});
-            __builtin_amdgcn_s_barrier();
-            // ---- phase B
-            rd_x(ox, I4{});
-            __builtin_amdgcn_sched_barrier(0);
-            if (has2) {
-                if constexpr (C::RING) stage_x(ow, kt + 2);
-                else stage_w(ow, kt + 2);
-            }
-            reads_done(false);
-            constexpr int YOUNGER = C::RING ? C::DPW : C::W_DMA;
-            if (!has2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            else if (C::RING && kt == 0) wait_behind_stores(std::integral_constant<int, YOUNGER>{});  // (K tile 1 was issued in front of them)
-            else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(YOUNGER) : "memory");
-            close_load();
-            mfmas(I4{});
-            __builtin_amdgcn_s_barrier();
-            if constexpr (C::RING) {
-                of = ox;
-                ow = next2(ow);
-                ox = next2(ox);
-            }
-        }
+        };
+        // A group's last rows go through a loop of their own: with the tests in the one loop whole tiles were 1 to 2 % slower.  Without / with, us:
+        // gate|up, down of 64 experts, 6 of 1024 x 2048 at 6000 tokens 337 / 308, 200 / 186, 8 of 1408 x 4096 at 4096 800 / 774, 445 / 431, at 15074
+        // 2181 / 2184, 1258 / 1222.  (The rows dealt anew to both waves along m: 10 to 40 registers spilled, whole tiles 2 to 5 % slower.)
+        // A projection without groups has one such block per column tile: there the second loop costs more than it gives (0.3 to 1 %).
+        if (!GROUPED || mcnt_c > 192) k_tiles(std::true_type{}, std::true_type{});
+        else if constexpr (GROUPED) k_tiles(mcnt_c > wm * 128, mcnt_c > wm * 128 + 64);
         if (wid < 4) __builtin_amdgcn_s_barrier();  // match the other group's extra barrier
         } else {
         // ---- main loop: two phases per K tile, waves 4-7 run ONE BARRIER BEHIND waves 0-3 ----

@@ -1096,6 +1096,24 @@ def test_gemm_large_m_several_tiles_per_workgroup(ops, K, counts):
     assert_close_bf16(got[0][rows].cpu(), a_ref, 3, 0.06, atol=1e-3, what=f"act K={K} group {e}")
 
 
+@pytest.mark.parametrize("last", [1, 63, 64, 65, 128, 129, 192, 193])
+def test_gemm_large_m_last_rows_of_a_group(ops, last):
+    """Row blocks of 256 of which 64, 128 or 192 rows exist, or one more or less: waves without rows leave their products out.  Bit for bit against
+    the plain form, with experts that are one such block and experts that end in one."""
+    K, I, N2, counts = 192, 136, 264, [256 + last, last, 512 + last, 1024]
+    E, R, T = len(counts), sum(counts), 500
+    offs = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32)
+    tok = torch.randint(0, T, (R,), generator=torch.Generator().manual_seed(last), dtype=torch.int32)
+    x, act = dev(rnd(T, K, seed=1)), dev(rnd(R, K, seed=2))
+    w13, w2 = dev(rnd(E, 2 * I, K, seed=3, scale=K ** -0.5)), dev(rnd(E, N2, K, seed=4, scale=K ** -0.5))
+    scale = dev((torch.rand(R) + 0.1).to(BF))
+    got = []
+    for v in (0, -1):
+        with largem_variant(v), ops.option("largem_cfg", 2):
+            got.append((ops.grouped_gemm_gateup_silu(x, w13, dev(offs), dev(tok), R), ops.grouped_gemm_down(act, w2, dev(offs), scale, E - 1)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("cfg", [1, 2])
 @pytest.mark.parametrize("M,N,K", [(600, 328, 128), (385, 64, 192), (1030, 1096, 64)])
 def test_gemm_large_m_epilogues(ops, M, N, K, cfg):
