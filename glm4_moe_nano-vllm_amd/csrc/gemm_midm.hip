@@ -3,7 +3,7 @@
 //
 // What bounds it: the weights are still read once and dominate the HBM bytes, but an output tile must be small for the grid to cover
 // the chip, and every workgroup pulls its own activation and weight rows through L2 -> LDS, some 32 bytes per clock and CU: the tile is
-// chosen for that traffic and for the number of workgroups (midm_tile_of), from 64 rows x 32 weight rows up to 128 x 128.
+// chosen for that traffic and for the number of workgroups (midm_tile_of), from 32 rows x 16 weight rows up to 128 x 128.
 //   * a stage = one 64-wide K chunk of the tile's activation and weight rows, a whole 128-byte line per row (with 32-wide chunks, half
 //     lines: 14336 x 4096 at 128 rows 53 instead of 45 us, 4096 x 12288 at 64 rows 60 instead of 45);
 //   * 16-byte pieces are swizzled at the source, piece ^ ((row >> 1) & 7): the 16 rows of a fragment read cover all banks;
@@ -630,7 +630,7 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
 // 30.0 / 36.2, at 512 47 / - / 31.8* / 40.2; 14336 x 4096 at 64 36.7 / 27.6* / - / 37.5, at 128 56 / 42.6 / 37.7* / 46.3, at 211 77 / 61.5 / 52 /
 // 43.0*; 2048 x 2048 at 1000 rows - / 16.9 / 17.2* / 19.8 (512 tiles of 64 x 64), at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
 // A long K favours split waves at 64 x 64 too, which read each staged byte once: 4096 x 12288 at 211 rows 50 (shared 58), K = 8192 36 (40).
-enum MidmTile { MM_NONE, MM_SPLIT16, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
+enum MidmTile { MM_NONE, MM_SPLIT16, MM_SPLIT32x32, MM_SPLIT32, MM_SPLIT64, MM_64, MM_128x64, MM_64x128, MM_128 };
 
 MidmTile midm_tile_of(int mode, const GemmParams& p) {
     const int64_t n = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
@@ -639,11 +639,16 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
     // it, and with a hundred row blocks and more.  Shared 64 x 64 / split 64 x 32, us: 1024 x 256 at 300 rows 4.3 / 3.8, 264 x 512 at 700 5.7 / 4.7,
     // 512 x 384 at 1000 4.7 / 4.1, fp32 rows 6.2 / 4.8, 64 x 512 at 3000 5.2 / 4.6, at 8000 6.1 / 6.4; gated columns 512 x 128 at 96 rows 3.0 / 3.4,
     // 1024 x 320 at 128 4.1 / 4.2, 256 x 512 at 300 4.4 / 3.9, 132 x 512 at 700 4.6 / 4.4, at 1500 4.9 / 5.5.
-    // Few columns (routers, gates, small latents): a workgroup takes in some 50 GB/s whatever it does, so 32 rows x 16 columns split over eight waves
-    // come before the larger tiles.  64 x 32 over four waves / this, us: 100 rows of 64 x 2048 6.6 / 4.1, x 256 3.5 / 2.9, 211 of 64 x 4096 11.1 /
-    // 6.8, 2000 of 64 x 2048 7.4 / 5.6, 300 of 376 x 2048 7.5 / 5.0, 33 of 376 x 8192 16.3 / 9.5, 8000 of 16 x 512 4.7 / 3.2.  From 384 columns
-    // on a projection may be queries, keys and values, whose fused form sums over four waves: there both keep that order.
-    if (!gemm_paired(mode) && p.N < 384 && p.K >= 256 && fits(32, 16)) return MM_SPLIT16;
+    // A workgroup takes in some 50 GB/s of weights that no cache holds, whatever it does, so tiles of 32 rows whose K is split over eight waves come
+    // first, as few columns as one round of the chip allows.  Others / these, us, cold weights.  16 columns, formerly 64 x 32 over four waves:
+    // 100 rows of 64 x 2048 6.6 / 4.1, x 256 3.5 / 2.9, 211 of 64 x 4096 11.1 / 6.8, 2000 of 64 x 2048 7.4 / 5.6, 33 of 376 x 8192 16.3 / 9.5, 128 of
+    // 1024 x 2048 8.9 / 6.2, 64 of 2048 x 2048 10.2 / 7.1, 33 of 2048 x 4096 14.4 / 8.9, 64 of 1024 x 6144 22.7 / 13.0, 100 of 640 x 512 4.6 / 3.8.  32
+    // columns: 128 of 2048 x 2048 9.9 / 8.2, x 4096 15.9 / 12.4, 48 of 3072 x 768 6.1 / 5.3, 96 of 2048 x 512 4.7 / 4.4, 70 of 2048 x 8192 22.6 / 18.2, gated
+    // 100 of 1024 x 2048 9.3 / 7.4.  (48 columns: 128 of 2304 x 2048 9.95 / 9.5 in a row of its own, but 9.8 / 9.9 inside a step, 100 of 3072 x 768
+    // 6.4 / 7.6: not taken.)
+    // (The same chunks by wave and the same order of the eight sums in all of them and in the QKV epilogue's tile.)
+    if (!gemm_paired(mode) && p.K >= (p.N < 384 ? 256 : 512) && fits(32, 16)) return MM_SPLIT16;
+    if (p.K >= 512 && fits(32, 32)) return MM_SPLIT32x32;
     if (fits(64, 32) && (gemm_paired(mode) ? p.K >= (p.R <= 1000 ? 384 : 576) : p.K > 512 || p.R <= 4096)) return MM_SPLIT32;
     if (fits(64, 64)) return p.K >= 8192 ? MM_SPLIT64 : MM_64;
     if (p.R <= 64) return fits(64, 128) ? MM_64x128 : MM_NONE;
@@ -655,8 +660,12 @@ template <int MODE>
 int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
     switch (tile) {
         case MM_SPLIT16:
+            if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);   // (half a head)
             if constexpr (!gemm_paired(MODE)) return launch_midm_cfg<MODE, 2, 1, 8, 2>(p, st);
             break;
+        case MM_SPLIT32x32:
+            if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);
+            return launch_midm_cfg<MODE, 2, 2, 8, 2>(p, st);
         case MM_SPLIT32:   // (half a head in the QKV epilogue; the sums are the same in both tiles)
             if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
             [[fallthrough]];

@@ -96,6 +96,32 @@ def test_gated(ops, M, I, K):
     close(y, act.cpu().double() @ d.double().T, "down")
 
 
+# 32 rows over eight waves: 16 columns (one round of the chip exactly, waves without a chunk at the least K) and 32 (exactly one round), one tile more
+@pytest.mark.parametrize("M,N,K", [(33, 2048, 512), (64, 2044, 576), (97, 996, 1088), (33, 2052, 512), (128, 2048, 2048), (100, 1900, 576), (128, 2052, 512)])
+def test_split_tiles_of_32_rows(ops, M, N, K):
+    x, w, b = rnd(M, K + 8, seed=31)[:, :K], rnd(N, K, seed=32, scale=K ** -0.5), rnd(N, seed=33)
+    xd = torch.empty(M, K + 8, dtype=BF, device="cuda")[:, :K]
+    xd.copy_(x)
+    out = torch.full((M + 2, N), 7.0, dtype=BF, device="cuda")
+    ref = x.double() @ w.double().T
+    close(ops.linear_act(xd, w.cuda(), b.cuda(), out=out[1: M + 1]), ref + b.double(), "bias")
+    assert torch.all(out[0] == 7) and torch.all(out[-1] == 7)
+    bound = 2.0 ** -23 * (x.double().abs() @ w.double().abs().T) * 8
+    assert ((ops.linear_act(xd, w.cuda(), out_f32=True).cpu().double() - ref).abs() <= bound + 1e-7).all()
+
+
+@pytest.mark.parametrize("T,nh,nkv,K", [(96, 4, 1, 512), (100, 12, 2, 512), (128, 16, 2, 576), (97, 14, 1, 1088)])
+def test_split_tiles_of_32_rows_with_rope_store(ops, T, nh, nkv, K):
+    """The fused QKV projection takes half a head per workgroup where the projection by itself takes 16 or 32 columns: bit for bit the same."""
+    N = (nh + 2 * nkv) * 128
+    x, w, b = rnd(T, K, seed=41).cuda(), rnd(N, K, seed=42, scale=K ** -0.5).cuda(), rnd(N, seed=43).cuda()
+    pos = torch.randint(0, 512, (T,), generator=torch.Generator().manual_seed(44)).cuda()
+    cs = O.build_cos_sin_cache(64, 512, 10000.0).reshape(512, 64).contiguous().cuda()
+    q0, k0, v0 = ops.qkv_split_norm_rope_store(ops.gemm_bf16(x, w, b), nh, nkv, 128, pos, cs, 64, None, None, 1e-5, None, None, None, True)
+    q1, k1, v1 = ops.gemm_qkv_rope_store(x, w, b, nh, nkv, 128, pos, cs, 64, None, None, None, True)
+    assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0, v1)
+
+
 @pytest.mark.parametrize("T,E,k,H,I,shared", [(33, 3, 2, 192, 100, True), (97, 5, 3, 576, 72, False), (211, 8, 2, 128, 264, True), (64, 1, 1, 64, 40, False)])
 def test_experts(ops, T, E, k, H, I, shared):
     """Groups of 24 to 95 rows on average, ragged ones among them (an expert without rows, one with more than a block of 64)."""
