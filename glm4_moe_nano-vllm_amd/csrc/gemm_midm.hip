@@ -239,7 +239,9 @@ __device__ __forceinline__ void midm_body(const GemmParams& p, char* smem, int m
             return;
         }
     }
-    gemm_row_epilogue<MODE, RT, MPW>(p, sum, 0, m0 + first, mcnt - first, ncol0, c, g4);
+    // (behind the waves' tiles: nobody else's)
+    f32x4_t* own = reinterpret_cast<f32x4_t*>(smem) + (NW * MT + wid * MPW) * RT * 64 + lane;
+    gemm_row_epilogue<MODE, RT, MPW, true>(p, sum, 0, m0 + first, mcnt - first, ncol0, c, g4, own);
 }
 
 // row block and column tile of this workgroup
@@ -257,7 +259,7 @@ __device__ __forceinline__ void midm_tile(int mblocks, int interleaved, int& m, 
 
 template <int MODE, int MT, int RT, int NW, int NST>
 constexpr int midm_lds() {
-    constexpr int ring = NW * NST * (MT + RT) * 2048, red = NW * MT * RT * 1024;
+    constexpr int MPW = MT < NW ? 1 : MT / NW, ring = NW * NST * (MT + RT) * 2048, red = (NW * MT + (MT < NW ? MT : NW) * MPW) * RT * 1024;
     return ring > red ? ring : red;
 }
 
@@ -488,6 +490,7 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
     constexpr int NW = WM * WN, WR = 16 * RT * WN, XR = 16 * MT * WM;   // weight rows and activation rows of a stage
     constexpr int STAGE = (WR + XR) * MM_ROWB, D = (WR + XR) / 8 / NW, DW = WR / 8 / NW;
     constexpr int HALF = 8 * RT;               // paired modes: gate rows of a wave's columns, then as many up rows
+    static_assert(NST * STAGE >= NW * RT * MT * 1024, "gemm_activate's pieces");
     static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && NST >= 2, "whole DMA instructions per wave");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -561,6 +564,7 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
                 acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f1.w[rt]), __builtin_bit_cast(bf16x8_t, f1.x[mt]), acc[rt][mt], 0, 0, 0);
         slot = slot + 1 == NST ? 0 : slot + 1;
     }
+    if (MODE == GEMM_PLAIN && p.act.kind != GLM_ACT_NONE) __syncthreads();   // the ring is read: gemm_activate's pieces lie in it
     const int first = 16 * MT * wm;
     if (first >= mcnt) return;
     if constexpr (MODE == GEMM_PLAIN) {
@@ -570,7 +574,8 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
         }
     }
     // (slab s of the partial sums: rows s R ..)
-    gemm_row_epilogue<MODE, RT, MT>(p, acc, 0, slice * (int)p.R + m0 + first, mcnt - first, ncol0 + wn * (gemm_paired(MODE) ? HALF : 16 * RT), c, g4);
+    gemm_row_epilogue<MODE, RT, MT, true>(p, acc, 0, slice * (int)p.R + m0 + first, mcnt - first, ncol0 + wn * (gemm_paired(MODE) ? HALF : 16 * RT), c, g4,
+                                     reinterpret_cast<f32x4_t*>(smem) + wid * RT * MT * 64 + lane);
 }
 
 template <int WM, int WN, int MT, int RT, int NST>
