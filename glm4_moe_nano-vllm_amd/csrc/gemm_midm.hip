@@ -515,13 +515,18 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
         vo[i] = ((unsigned)src * (unsigned)(isw ? p.ldw : p.ldx) + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
     }
     const int n = K / MM_KC;
+    // Weights that only this row block reads leave the caches to the activations (nt).  Kept / past them, us, each in a process of its own, cold weights: 128
+    // rows of 32768 x 2048 32.0 / 30.4, 64 of 14336 x 4096 31.0 / 29.1; steps: 64 GLM sequences over fp8 experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With
+    // two row blocks and more, and in the split tiles, single projections gained as much and steps lost it again (a prompt of 211 1.886 / 1.904 ms).
+    const bool nt = p.R <= XR;
     auto issue = [&](int j, int slot) {
         const int soff = j * MM_ROWB;
 #pragma unroll
         for (int i = 0; i < D; ++i) {
             const bool isw = i < DW;
             char* dst = smem + slot * STAGE + (isw ? 0 : WR * MM_ROWB) + ((isw ? i : i - DW) * NW + wid) * 1024;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? wrs : xrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 0);
+            if (isw && nt) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 2);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? wrs : xrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 0);
         }
     };
     f32x4_t acc[RT][MT];
