@@ -39,6 +39,7 @@ namespace {
 
 constexpr int LM_BN = 256;    // weight rows per tile (MFMA row axis); 4 waves x 64 rows
 constexpr int LM_BAND_ROWS = 4;  // row blocks per L2 supertile band
+constexpr int LM_CUT_K = 512;    // shortest reduction whose last tiles are cut
 constexpr int LM_SLOT = 32768;   // CfgR: bytes of a ring slot, one operand tile
 
 // Tile configurations (the kernel is written once over these):
@@ -93,6 +94,10 @@ using LmCfgR = LmCfg<256, 64, 2, true>;
 using LmCfgR8 = LmCfg<256, 64, 2, true, true>;  // fp8 weight operand (its tiles fill half a slot)
 using LmCfgA8 = LmCfg<128, 64, 3, false, true>;
 using LmCfgC88 = LmCfg<256, 128, 2, false, false, true>;  // fp8 x fp8 on the block-scaled MFMA: two 64-KiB buffers, the rest of the LDS holds scales
+
+// configurations whose last tiles may be cut (the 128-row one's ring fits into theirs)
+template <int MODE, class C>
+__host__ __device__ constexpr bool lm_cuts() { return C::RING && !C::W8 && MODE != GEMM_SLICES; }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
@@ -212,13 +217,13 @@ __device__ __forceinline__ void lm_locate_lanes(const int32_t* __restrict__ offs
 // the SCALAR offset, fragment reads use one base register per k-step plus immediate offsets, 16-byte stores (the packed results of two
 // neighbouring 16-column tiles are exchanged between the lane rows).  Needs K % BK == 0, x and W spans < 2 GiB, N % 8 == 0.  The other
 // form covers everything else.
-template <int MODE, class C, bool LEAN, bool WSCALE>
-__global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND) {
+// CUT: tiles of 256 rows from `first` on, each in two of 128.
+template <int MODE, class C, bool LEAN, bool WSCALE, bool CUT>
+__device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, int n_tiles, int total_tiles, int LM_BAND, int first) {
     constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP;  // may store fp32 rows (p.yf)
     constexpr bool BIAS = MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP;
     constexpr bool GROUPED = MODE == GEMM_GATEUP || MODE == GEMM_DOWN;
     static_assert(LEAN || (!C::RING && !C::W8 && !C::A8), "the plain form has the plain ring");
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wid & 3, wm = wid >> 2;
@@ -248,9 +253,22 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
         while (pos0 + ti * pstep < chunk_len) {
             if ((ti & 63) == 0) {
                 const int bid = chunk_base + pos0 + (ti + lane) * pstep;
-                const int band = bid / (LM_BAND * n_tiles), rem = bid % (LM_BAND * n_tiles);
-                lm_locate_lanes(p.offs, p.G, p.R, C::BM, band * LM_BAND + rem % LM_BAND, lane, tab_g, tab_m0, tab_cn);
-                tab_cn |= (rem / LM_BAND) << 9;  // up to 256 rows, up to 2^22 column tiles (checked by the host)
+                if (CUT || (MODE != GEMM_SLICES && p.offs == nullptr)) {   // one group: every position is a tile
+                    int t = CUT ? first + (bid >> 1) : bid, row, ntile_;
+                    const int blk = CUT ? 256 : C::BM, nb = (int)((p.R + blk - 1) / blk), band = t / (LM_BAND * n_tiles), b0 = band * LM_BAND;
+                    const int high = max(1, min(LM_BAND, nb - b0));       // row blocks of the band
+                    t -= b0 * n_tiles;
+                    row = (b0 + t % high) * blk + (CUT ? (bid & 1) * 128 : 0);
+                    ntile_ = t / high;
+                    const int64_t left = p.R - row;
+                    tab_g = bid < total_tiles && left > 0 ? 0 : -1;
+                    tab_m0 = row;
+                    tab_cn = (int)(left < C::BM ? left : (int64_t)C::BM) | ntile_ << 9;
+                } else {
+                    const int band = bid / (LM_BAND * n_tiles), rem = bid % (LM_BAND * n_tiles);
+                    lm_locate_lanes(p.offs, p.G, p.R, C::BM, band * LM_BAND + rem % LM_BAND, lane, tab_g, tab_m0, tab_cn);
+                    tab_cn |= (rem / LM_BAND) << 9;  // up to 256 rows, up to 2^22 column tiles (checked by the host)
+                }
             }
             const int at = ti & 63;
             ++ti;
@@ -1031,6 +1049,19 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
     }
 }
 
+// Tiles are equal and every CU takes its share of them, so what does not fill a round costs one: the tiles behind whole rounds, if they are half a round at
+// most, are cut in two, half a tile for every CU, on the 128-row configuration and its ring (0.7 of a tile's time).  One kind of tile / this, us: 11137 rows of
+// 2048 x 2048 (1.4 rounds) 83.7 / 74.9, of 3072 x 2048 (2.1) 129 / 117, of 6144 x 2048 (4.1) 220 / 209, gated 4096 x 2048 (5.5) 266 / 262, 15074 of 2304 x 2048 (2.1)
+// 128 / 118, x 512 46.6 / 42.4, 4500 of 4096 x 4096 154 / 132; where nothing is cut (15074 of 2048 x 2048, 1.8) 92.8 / 93.1.
+template <int MODE, class C, bool LEAN, bool WSCALE>
+__global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND, int tail) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    largem_tiles<MODE, C, LEAN, WSCALE, false>(p, smem, n_tiles, total_tiles, LM_BAND, 0);
+    if constexpr (lm_cuts<MODE, C>()) {
+        if (tail > 0) largem_tiles<MODE, LmCfgA, true, WSCALE, true>(p, smem, n_tiles, 2 * tail, LM_BAND, total_tiles);
+    }
+}
+
 // option largem_variant: -1 by shape, LM_VAR_LEAN the same, any other number the plain form
 constexpr int LM_VAR_LEAN = 86787;
 
@@ -1042,7 +1073,8 @@ int launch_largem_cfg(const GemmParams& p, hipStream_t st) {
     // (a band higher than the rows' blocks would be mostly positions without a tile: 74 tiles of one block took two passes of 256
     // workgroups)
     const int LM_BAND = p.offs ? LM_BAND_ROWS : (int)(combos < LM_BAND_ROWS ? combos : (int64_t)LM_BAND_ROWS);
-    const int64_t total = (combos + LM_BAND - 1) / LM_BAND * LM_BAND * n_tiles;
+    const bool dense = p.offs == nullptr && MODE != GEMM_SLICES;
+    int64_t total = dense ? combos * n_tiles : (combos + LM_BAND - 1) / LM_BAND * LM_BAND * n_tiles;
     if (total <= 0) return GLM_OK;
     GLM_CHECK_ARG(total < (1ll << 30) && n_tiles < (1 << 22), GLM_ERR_UNSUPPORTED, "gemm_largem: grid too large");
     // the per-row scale of fp8-expanded weights is its own instantiation: as a run-time test it sat inside the epilogue's
@@ -1068,7 +1100,13 @@ int launch_largem_cfg(const GemmParams& p, hipStream_t st) {
     if (nwg < 8) nwg = 8;
     const int64_t need = (total + 7) / 8 * 8;
     if (nwg > need) nwg = need;
-    hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(512), LDS_BYTES, st, p, n_tiles, (int)total, LM_BAND);
+    int64_t tail = 0;
+    if (lm_cuts<MODE, C>() && dense && total > nwg && p.K >= LM_CUT_K) {
+        tail = total % nwg;
+        if (2 * tail > nwg) tail = 0;
+        total -= tail;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(512), LDS_BYTES, st, p, n_tiles, (int)total, LM_BAND, (int)tail);
     GLM_CHECK_LAUNCH("gemm_largem");
     return GLM_OK;
 }

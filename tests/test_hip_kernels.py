@@ -1096,6 +1096,41 @@ def test_gemm_large_m_several_tiles_per_workgroup(ops, K, counts):
     assert_close_bf16(got[0][rows].cpu(), a_ref, 3, 0.06, atol=1e-3, what=f"act K={K} group {e}")
 
 
+@pytest.mark.parametrize("M,N,K", [(8518, 2056, 512), (8448, 2048, 576), (33000, 520, 512), (8705, 2048, 512)])
+def test_gemm_large_m_last_round_in_halves(ops, M, N, K):
+    """More tiles than CUs and at most half a round behind whole ones: those go in halves.  Row blocks that end in the first half and at its end, columns that
+    end inside a tile; bit for bit against the plain form."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn(2 * N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    b = torch.randn(N, device="cuda", generator=g).to(BF)
+    got = []
+    for v in (0, -1):
+        with largem_variant(v):
+            out = torch.full((M + 1, N), 7.0, device="cuda", dtype=BF)
+            ops.linear_act(x, w[:N], b, out=out[:M])
+            got.append((out, ops.linear_act(x, w[:N], act=(ops.ACT_GATE, 264.0, 0.0)), ops.linear_act(x, w[:N], out_f32=True),
+                        ops.gated_glu(x, w[: 2 * (N // 2)], 2.0), ops.grouped_gemm_gateup_silu(x, w.unsqueeze(0), None, None, M)))
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
+    assert bool((got[1][0][-1] == 7).all())
+
+
+@pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (16700, 4, 2, 512)])
+def test_qkv_gemm_with_rope_store_last_round_in_halves(ops, T, nh, nkv, K):
+    """The fused QKV projection with its last tiles in halves == the projection, also cut, and the split / rotary kernel, bit for bit."""
+    N = (nh + 2 * nkv) * 128
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    b = torch.randn(N, device="cuda", generator=g).to(BF)
+    pos = torch.randint(0, 512, (T,), device="cuda", generator=g)
+    cs = dev(O.build_cos_sin_cache(64, 512, 10000.0).reshape(512, 64).contiguous())
+    q0, k0, v0 = ops.qkv_split_norm_rope_store(ops.gemm_bf16(x, w, b), nh, nkv, 128, pos, cs, 64, None, None, 1e-5, None, None, None, True)
+    q1, k1, v1 = ops.gemm_qkv_rope_store(x, w, b, nh, nkv, 128, pos, cs, 64, None, None, None, True)
+    assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0, v1)
+
+
 @pytest.mark.parametrize("last", [1, 63, 64, 65, 128, 129, 192, 193])
 def test_gemm_large_m_last_rows_of_a_group(ops, last):
     """Row blocks of 256 of which 64, 128 or 192 rows exist, or one more or less: waves without rows leave their products out.  Bit for bit against
