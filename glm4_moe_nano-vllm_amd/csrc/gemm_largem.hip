@@ -253,7 +253,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         while (pos0 + ti * pstep < chunk_len) {
             if ((ti & 63) == 0) {
                 const int bid = chunk_base + pos0 + (ti + lane) * pstep;
-                if (CUT || (MODE != GEMM_SLICES && p.offs == nullptr)) {   // one group: every position is a tile
+                if (CUT || (MODE != GEMM_SLICES && p.offs == nullptr)) {   // one group: no position without a tile in front of the last
                     int t = CUT ? first + (bid >> 1) : bid, row, ntile_;
                     const int blk = CUT ? 256 : C::BM, nb = (int)((p.R + blk - 1) / blk), band = t / (LM_BAND * n_tiles), b0 = band * LM_BAND;
                     const int high = max(1, min(LM_BAND, nb - b0));       // row blocks of the band
@@ -261,7 +261,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                     row = (b0 + t % high) * blk + (CUT ? (bid & 1) * 128 : 0);
                     ntile_ = t / high;
                     const int64_t left = p.R - row;
-                    tab_g = bid < total_tiles && left > 0 ? 0 : -1;
+                    tab_g = bid < total_tiles && left > 0 && ntile_ < n_tiles ? 0 : -1;
                     tab_m0 = row;
                     tab_cn = (int)(left < C::BM ? left : (int64_t)C::BM) | ntile_ << 9;
                 } else {
@@ -1052,7 +1052,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
 // Tiles are equal and every CU takes its share of them, so what does not fill a round costs one: the tiles behind whole rounds, if they are half a round at
 // most, are cut in two, half a tile for every CU, on the 128-row configuration and its ring (0.7 of a tile's time).  One kind of tile / this, us: 11137 rows of
 // 2048 x 2048 (1.4 rounds) 83.7 / 74.9, of 3072 x 2048 (2.1) 129 / 117, of 6144 x 2048 (4.1) 220 / 209, gated 4096 x 2048 (5.5) 266 / 262, 15074 of 2304 x 2048 (2.1)
-// 128 / 118, x 512 46.6 / 42.4, 4500 of 4096 x 4096 154 / 132; where nothing is cut (15074 of 2048 x 2048, 1.8) 92.8 / 93.1.
+// 128 / 118, x 512 46.6 / 42.4, 4500 of 4096 x 4096 154 / 132; a forward pass of 9000 rows 5.07 / 4.84 ms, one of 15074 rows with few such launches the same.
 template <int MODE, class C, bool LEAN, bool WSCALE>
 __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, int n_tiles, int total_tiles, int LM_BAND, int tail) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1074,7 +1074,7 @@ int launch_largem_cfg(const GemmParams& p, hipStream_t st) {
     // workgroups)
     const int LM_BAND = p.offs ? LM_BAND_ROWS : (int)(combos < LM_BAND_ROWS ? combos : (int64_t)LM_BAND_ROWS);
     const bool dense = p.offs == nullptr && MODE != GEMM_SLICES;
-    int64_t total = dense ? combos * n_tiles : (combos + LM_BAND - 1) / LM_BAND * LM_BAND * n_tiles;
+    int64_t total = (combos + LM_BAND - 1) / LM_BAND * LM_BAND * n_tiles;
     if (total <= 0) return GLM_OK;
     GLM_CHECK_ARG(total < (1ll << 30) && n_tiles < (1 << 22), GLM_ERR_UNSUPPORTED, "gemm_largem: grid too large");
     // the per-row scale of fp8-expanded weights is its own instantiation: as a run-time test it sat inside the epilogue's
@@ -1101,11 +1101,15 @@ int launch_largem_cfg(const GemmParams& p, hipStream_t st) {
     const int64_t need = (total + 7) / 8 * 8;
     if (nwg > need) nwg = need;
     int64_t tail = 0;
-    if (lm_cuts<MODE, C>() && dense && total > nwg && p.K >= LM_CUT_K) {
-        tail = total % nwg;
+    if (lm_cuts<MODE, C>() && dense && combos * n_tiles > nwg && p.K >= LM_CUT_K) {
+        tail = combos * n_tiles % nwg;
         if (2 * tail > nwg) tail = 0;
-        total -= tail;
+        if (tail > 0) total = combos * n_tiles - tail;
     }
+    // Positions without a tile keep every XCD's share of the list at whole bands (4 row blocks by 8 column tiles at a time, one copy in its L2), so they stay
+    // where leaving them out saves no round.  With / without them inside a forward pass of 15074 rows, us: 2048 x 2048 (1.8 rounds of tiles, 2 of positions)
+    // 95.4 / 100, fp32 logits 184 / 194; where they are a round, 15074 of 14336 x 4096 (12.9 and 13.1): a pass of such layers 31.2 / 30.9 ms.
+    if (dense && tail == 0 && (combos * n_tiles + nwg - 1) / nwg < (total + nwg - 1) / nwg) total = combos * n_tiles;
     hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(512), LDS_BYTES, st, p, n_tiles, (int)total, LM_BAND, (int)tail);
     GLM_CHECK_LAUNCH("gemm_largem");
     return GLM_OK;

@@ -1116,6 +1116,22 @@ def test_gemm_large_m_last_round_in_halves(ops, M, N, K):
     assert bool((got[1][0][-1] == 7).all())
 
 
+@pytest.mark.parametrize("M,N", [(15074, 2048), (8704, 3072), (8248, 7944), (8448, 7936), (512, 32768), (300, 40000)])
+def test_gemm_large_m_tile_lists(ops, M, N):
+    """Lists of more than one round whose last band has fewer row blocks, with the positions behind it (no round more) and without them (a round more),
+    and bands of fewer blocks than usual; bit for bit against the plain form."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, 128, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, 128, device="cuda", generator=g) * 128 ** -0.5).to(BF)
+    got = []
+    for v in (0, -1):
+        with largem_variant(v):
+            out = torch.full((M + 1, N), 7.0, device="cuda", dtype=BF)
+            ops.linear_act(x, w, out=out[:M])
+            got.append(out)
+    assert torch.equal(*got) and bool((got[1][-1] == 7).all())
+
+
 @pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (16700, 4, 2, 512)])
 def test_qkv_gemm_with_rope_store_last_round_in_halves(ops, T, nh, nkv, K):
     """The fused QKV projection with its last tiles in halves == the projection, also cut, and the split / rotary kernel, bit for bit."""
