@@ -17,7 +17,7 @@
 //     operand panels are shared through that XCD's L2.
 //
 // What bounds it: power.  With zeros as operands the same launches run 1.25 to 1.35 times as fast (16384 x 8192 x 8192: 1930 TFLOP/s
-// against 1440), so what counts is both cycles and switching.  Cycles: the ring of the 256-row tiles (CfgR) holds FIVE 32-KiB operand
+// against 1440; 1955 against 1526 with the present epilogue), so what counts is both cycles and switching.  Cycles: the ring of the 256-row tiles (CfgR) holds FIVE 32-KiB operand
 // tiles (W and X of two K tiles and the next W) in all 160 KiB of LDS, in the order they are needed; an operand's slot is refilled as
 // soon as its own last fragment read has retired, so a piece has one to one and a half K tiles to arrive (two 64-KiB buffers: half to
 // one, which a loaded memory side does not make), and a phase is 32 MFMAs between two barriers instead of 16 (fp8 x fp8: 16 of four
@@ -28,9 +28,10 @@
 //   ... 32 per phase                   1371                  1326                   1282                   1253                 1340
 //   ring of five, 32 per phase         1407                  1329                   1315                   1245                 1344
 //   ... alternating direction          1439                  1333                   1350                   1257                 1362
+//   ... decisions and stores by wave   1560                  1467                   1456                   1372                 1501   (another card)
 // (Also measured: one barrier per K tile and fragments read a quarter of a tile ahead into 96 registers, 1187 to 1266; wave
 // priority in the MFMA interval, equal; K slices of the fragments outermost or tiles of the other operand outermost, equal; 2, 3, 6
-// or 8 row blocks per band, up to 7 % slower.)  A tile's stores cost 5 % (K = 8192) to 9 % (K = 2048): all CUs reach them together.
+// or 8 row blocks per band, up to 7 % slower.)  A tile's stores cost 2 % (K = 8192) to 6 % (K = 2048): all CUs reach them together.
 #include "gemm_internal.h"
 #include <type_traits>
 
@@ -917,19 +918,23 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 if (mt == 0) start_next();
             }
         } else if constexpr (LEAN) {
-            // Decisions (bias, scale, kind of column) once per wave and not per element, and stores through a buffer of the tile's own rows and columns: what lies
-            // behind them is dropped by the bounds check, so every store is issued and its address is one addition.  Between a tile's loops the matrix pipe
+            // Decisions (bias, scale, kind of column) once per wave and not per element, and stores through buffers of 16 of the tile's own rows and its columns: what lies
+            // behind them is dropped by the bounds check, so every store is issued, with one offset for all of a tile's rows.  Between a tile's loops the matrix pipe
             // stands still: the instructions here are what counts.  15074 rows, us, with a test and a 64-bit address per element or row / this: 6144 x
             // 2048 with a bias 329 / 285, xIELU 314 / 298, 4096 x 2048 half of them gates 207 / 188, 8192 x 2048 of SiLU and gates 411 / 377, 10240 x
             // 2048 of three kinds 507 / 467, plain 6144 x 2048 283 / 281; down of 8 of 64 experts, 4096 x 1408, 1258 / 1238.
             constexpr unsigned BEYOND = 0x80000000u;
             const bool f32 = F32ROWS && (MODE != GEMM_ACT || p.yf != nullptr);   // (the others have no bf16 form here)
-            const unsigned es = f32 ? 4u : 2u, pitch = (unsigned)p.ldy * es;   // (256 rows are below 2 GiB: launch_largem)
-            const int64_t first = ((MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0) + m0_c) * p.ldy + ncol_w;
+            const unsigned es = f32 ? 4u : 2u, pitch = (unsigned)p.ldy * es;   // (16 rows are below 2 GiB: launch_largem)
+            const int64_t first = ((MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0) + m0_c + wm * (C::BM / 2)) * p.ldy + ncol_w;
             char* ybase = f32 ? reinterpret_cast<char*>(p.yf + first) : reinterpret_cast<char*>(p.y + first);
-            const unsigned bytes = ncol_w < p.N ? (unsigned)(mcnt_c - 1) * pitch + (unsigned)(p.N - ncol_w) * es : 0u;
-            const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(ybase, 0, bytes, 0x00020000);
-            const unsigned lrow = (unsigned)(wm * (C::BM / 2) + c) * pitch;
+            const int left = ncol_w < p.N ? mcnt_c - wm * (C::BM / 2) : 0;
+            auto rows16 = [&](int mt) __attribute__((always_inline)) {
+                const int rows = min(left - 16 * mt, 16);
+                return __builtin_amdgcn_make_buffer_rsrc(ybase + (int64_t)mt * 16 * pitch, 0, rows > 0 ? (unsigned)(rows - 1) * pitch + (unsigned)(p.N - ncol_w) * es : 0u,
+                                                         0x00020000);
+            };
+            const unsigned lrow = (unsigned)c * pitch;
             // stores f of every element
             auto finish = [&](auto&& f) __attribute__((always_inline)) {
                 if constexpr (LATE_FILL) start_next();   // (its loads of scales are back: pinned above)
@@ -937,13 +942,14 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                     if (f32) {   // four columns per store
 #pragma unroll
                         for (int mt = 0; mt < C::MT; ++mt) {
+                            const __amdgpu_buffer_rsrc_t yrs = rows16(mt);
 #pragma unroll
                             for (int t = 0; t < NOUT; ++t) {
                                 const int n = 16 * t + 4 * g4;
                                 f32x4_t o;
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) o[r] = f(t, mt, r);
-                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, (ncol_w + n < p.N ? lrow + n * 4 : BEYOND) + 16 * mt * pitch, 0, 0);
+                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, ncol_w + n < p.N ? lrow + n * 4 : BEYOND, 0, 0);
                             }
                             __builtin_amdgcn_sched_barrier(0);
                         }
@@ -954,12 +960,13 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 // starting at column 8 * (g4 >> 1)
 #pragma unroll
                 for (int mt = 0; mt < C::MT; ++mt) {
+                    const __amdgpu_buffer_rsrc_t yrs = rows16(mt);
 #pragma unroll
                     for (int t = 0; t < NOUT; t += 2) {
                         const int n = 16 * (t + (g4 & 1)) + 8 * (g4 >> 1);
                         const u32x2_t a = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 0), f(t, mt, 1)), pack2bf(f(t + 1, mt, 0), f(t + 1, mt, 1)), false, false);
                         const u32x2_t b = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 2), f(t, mt, 3)), pack2bf(f(t + 1, mt, 2), f(t + 1, mt, 3)), false, false);
-                        __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{a[0], b[0], a[1], b[1]}, yrs, (ncol_w + n < p.N ? lrow + n * 2 : BEYOND) + 16 * mt * pitch, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{a[0], b[0], a[1], b[1]}, yrs, ncol_w + n < p.N ? lrow + n * 2 : BEYOND, 0, 0);
                     }
                     __builtin_amdgcn_sched_barrier(0);   // (the other rows' values would take registers that are not there)
                 }
@@ -1136,7 +1143,7 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int var = glm_option(GLM_OPT_LARGEM_VARIANT);
     const int64_t wrows = gemm_paired(MODE) ? 2 * (int64_t)p.N : (int64_t)p.N;
     const bool lean_ok = p.K % 64 == 0 && p.R * p.ldx * 2 < (1ll << 31) && wrows * p.ldw * 2 < (1ll << 31) &&
-                         p.N % 8 == 0 && p.ldy % 8 == 0 && p.ldy < (1 << 21) && glm_aligned16(p.y);
+                         p.N % 8 == 0 && p.ldy % 8 == 0 && p.ldy < (1 << 25) && glm_aligned16(p.y);
     if (p.w_fp8) {
         // fp8 weight operand: the lean form only;
         // what they do not cover (a K tail, offsets past 2^31) goes back to the caller, which expands the stack instead
@@ -1174,7 +1181,7 @@ int glm_launch_gemm_largem_a8(int mode, const GemmParams& p, hipStream_t st) {
                     p.R * p.ldx < (1ll << 31) && wrows * p.ldw < (1ll << 31) && glm_aligned16(p.x) && glm_aligned16(p.w) &&
                     (mode == GEMM_GATEUP ? (p.xscale != nullptr && p.ybscale != nullptr && p.ldy % 4 == 0 && (((uintptr_t)p.y) & 3) == 0 &&
                                             p.N % 32 == 0 && p.N <= 2048)
-                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && p.ldy < (1 << 21) && glm_aligned16(p.y)));
+                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && p.ldy < (1 << 25) && glm_aligned16(p.y)));
     if (!ok) {
         glm_set_error("gemm_largem(fp8 x fp8): shape not covered (mode %d R=%ld G=%d N=%d K=%d)", mode, (long)p.R, p.G, p.N, p.K);
         return GLM_ERR_UNSUPPORTED;

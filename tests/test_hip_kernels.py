@@ -1132,6 +1132,19 @@ def test_gemm_large_m_tile_lists(ops, M, N):
     assert torch.equal(*got) and bool((got[1][-1] == 7).all())
 
 
+@pytest.mark.parametrize("pitch", [1 << 21, (1 << 23) + 8])
+def test_gemm_large_m_wide_pitch(ops, pitch):
+    """Output rows so far apart that a tile's do not fit into 2 GiB; bit for bit against rows side by side, nothing behind a row's columns."""
+    M, N, K = 700, 8200, 192
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(M, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    out = torch.empty(M * pitch, device="cuda", dtype=BF).view(M, pitch)
+    out[:, N] = 7
+    ops.linear_act(x, w, out=out[:, :N])
+    assert torch.equal(out[:, :N], ops.linear_act(x, w)) and bool((out[:, N] == 7).all())
+
+
 @pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (16700, 4, 2, 512)])
 def test_qkv_gemm_with_rope_store_last_round_in_halves(ops, T, nh, nkv, K):
     """The fused QKV projection with its last tiles in halves == the projection, also cut, and the split / rotary kernel, bit for bit."""
