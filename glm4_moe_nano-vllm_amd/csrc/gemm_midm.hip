@@ -484,7 +484,7 @@ int launch_midm_experts(const GemmParams& p, hipStream_t st) {
 // rows m0 .. m0 + mcnt - 1, columns from ncol0, tile shared by the workgroup: WM x WN waves of MT x RT 16-row tiles each.  Every wave brings
 // its share of a stage (one 64-wide K chunk of all rows); the counted wait is for its own share, the barrier behind it for the others', and
 // it also says that every wave has the stage before in registers: its slot takes the chunk NST - 1 ahead.
-template <int MODE, int WM, int WN, int MT, int RT, int NST>
+template <int MODE, int WM, int WN, int MT, int RT, int NST, bool NT>
 __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem, int m0, int mcnt, int ncol0, int slice) {
     static_assert(RT == 2, "the QKV epilogue takes the two columns that turn together from one lane");
     constexpr int NW = WM * WN, WR = 16 * RT * WN, XR = 16 * MT * WM;   // weight rows and activation rows of a stage
@@ -515,17 +515,13 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
         vo[i] = ((unsigned)src * (unsigned)(isw ? p.ldw : p.ldx) + (pc ^ ((row >> 1) & 7)) * 8) * 2u;
     }
     const int n = K / MM_KC;
-    // Weights that only this row block reads leave the caches to the activations (nt).  Kept / past them, us, each in a process of its own, cold weights: 128
-    // rows of 32768 x 2048 32.0 / 30.4, 64 of 14336 x 4096 31.0 / 29.1; steps: 64 GLM sequences over fp8 experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With
-    // two row blocks and more, and in the split tiles, single projections gained as much and steps lost it again (a prompt of 211 1.886 / 1.904 ms).
-    const bool nt = p.R <= XR;
     auto issue = [&](int j, int slot) {
         const int soff = j * MM_ROWB;
 #pragma unroll
         for (int i = 0; i < D; ++i) {
             const bool isw = i < DW;
             char* dst = smem + slot * STAGE + (isw ? 0 : WR * MM_ROWB) + ((isw ? i : i - DW) * NW + wid) * 1024;
-            if (isw && nt) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 2);
+            if (isw && NT) __builtin_amdgcn_raw_ptr_buffer_load_lds(wrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 2);
             else __builtin_amdgcn_raw_ptr_buffer_load_lds(isw ? wrs : xrs, (mm_lds_void*)dst, 16, vo[i], soff, 0, 0);
         }
     };
@@ -586,14 +582,14 @@ __device__ __forceinline__ void midm_shared_body(const GemmParams& p, char* smem
 template <int WM, int WN, int MT, int RT, int NST>
 constexpr int midm_shared_lds() { return NST * (16 * RT * WN + 16 * MT * WM) * MM_ROWB; }
 
-template <int MODE, int WM, int WN, int MT, int RT, int NST>
+template <int MODE, int WM, int WN, int MT, int RT, int NST, bool NT>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_midm_shared_kernel(const GemmParams p, int mblocks, int interleaved) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int COLS = (gemm_paired(MODE) ? 8 : 16) * RT * WN, ROWS = 16 * MT * WM;
     int m, ntile;
     midm_tile(mblocks, interleaved, m, ntile);
     if (ntile * COLS >= p.N) return;
-    midm_shared_body<MODE, WM, WN, MT, RT, NST>(p, smem, m * ROWS, min(ROWS, (int)p.R - m * ROWS), ntile * COLS, blockIdx.z);
+    midm_shared_body<MODE, WM, WN, MT, RT, NST, NT>(p, smem, m * ROWS, min(ROWS, (int)p.R - m * ROWS), ntile * COLS, blockIdx.z);
 }
 
 template <int MODE, int MT, int RT, int NW, int NST>
@@ -627,7 +623,12 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
     const bool dealt = nt >= 64;
     const int64_t gx = dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8;
     GLM_CHECK_ARG(gx < (1 << 30), GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
-    auto kern = gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST>;
+    // Weights that only one row block reads go past the caches, which they leave to the activations (nt).  Kept / past them, us, weights not in the caches:
+    // 128 rows of 32768 x 2048 33.1 / 31.5, gated 30.7 / 28.8, 64 of 14336 x 4096 29.6 / 27.7, 41 of 8928 x 576 6.5 / 6.0; steps: 64 GLM sequences over fp8
+    // experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With two row blocks and more, and in the split tiles, single projections gained as much and
+    // steps lost it again (a prompt of 211 1.886 / 1.904 ms).  A kernel of its own: chosen inside the loop, for every DMA instruction, it cost all others 1 to
+    // 5 % (gate|up 965 of 456 x 6912 32.9 / 31.3, 300 of 1024 x 2048 12.1 / 11.7, plain 300 of 2048 x 2048 12.6 / 12.4).
+    auto kern = mblocks == 1 ? gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST, true> : gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST, false>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
     hipLaunchKernelGGL(kern, dim3((unsigned)gx, 1, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(WM * WN * 64), LDS, st, p, (int)mblocks, (int)dealt);
     GLM_CHECK_LAUNCH("gemm_midm");

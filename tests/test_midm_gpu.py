@@ -404,3 +404,15 @@ def test_few_columns_row_block_by_row_block(M, N, K, f32):
             assert torch.equal(out[r: r + n, :N], hip_ops.linear_act(x[r: r + n], w, out_f32=f32)), r
     want = x.cpu().double() @ w.cpu().double().T
     assert (out[:M, :N].cpu().double() - want).abs().max() / want.abs().max() < (K * 2.0 ** -24 if f32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("K,N,rows", [(320, 12288, (64, 128, 256)), (576, 8192, (128, 256)), (192, 24576, (64, 128))])
+def test_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
+    """Shared tiles whose weights go past the caches (all rows in one block) and the others of the same columns: every sum in the order of K, so a row
+    is bit for bit the same whatever stands behind it."""
+    x, w = rnd(max(rows), K, seed=61).cuda(), rnd(N, K, seed=62, scale=K ** -0.5).cuda()
+    got = [(ops.linear_act(x[:M], w), ops.gated_glu(x[:M], w, 2.0), ops.grouped_gemm_gateup_silu(x[:M], w.unsqueeze(0), None, None, M)) for M in rows]
+    close(got[-1][0], x.cpu().double() @ w.cpu().double().T, "plain")
+    for y in got[:-1]:
+        for a, b in zip(y, got[-1]):
+            assert torch.equal(a, b[: a.shape[0]])
