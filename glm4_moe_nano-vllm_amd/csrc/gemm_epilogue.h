@@ -1,43 +1,66 @@
 // gemm_epilogue.h — what the kernels for few rows (gemm_smallm.hip, gemm_midm.hip) do with a finished tile.
 #pragma once
 #include "gemm_internal.h"
+#include <type_traits>
 
-// p.act on every element of a finished tile.  What is inlined is chosen for the tile, not per element: a kernel that runs once in a step fetches its
-// instructions from far away, and with every kind of activation behind every element 128 x 128 tiles had 60 KB of code, of which even
-// rows without any jumped over all (32768 fp32 columns x 2048 at 128 rows inside a step of Dafolorn 49.6 us, by itself time after time 37.6).  own: 16 bytes
-// of LDS per lane and 16-byte piece (the next RT * MT - 1 pieces 1024 bytes apart), in which the long forms are a loop (LOOP).
+// p.act on every element of a finished tile.  What is inlined is chosen for the tile, not per element: a kernel that runs once in a step fetches its instructions
+// from far away, and with every kind of activation behind every element 128 x 128 tiles had 60 KB of code, of which even rows without any jumped over all.
+// A kind known at compile time also leaves no branch inside: the tests of glm_act_cols were one per element.  The long forms leave 16-row pieces without a row
+// out, and where LDS is free (LOOP) they are a loop over the pieces there; own: 16 bytes per lane and piece (the next RT * MT - 1 pieces 1024 bytes apart).
+// Every kind behind every element / chosen for the tile with the kinds' tests inside and all pieces / this, us: fp32 rows 300 x 2048 x 2048 with a soft cap
+// 14.5 / 15.4 / 13.0, with gates 14.1 / 15.3 / 12.7, 128 x 32768 x 2048 capped 38.4 / 37.6 / 34.1, the same behind 64 MiB of other traffic 35.0 / 27.9 / 26.1; bf16
+// rows with gates 13.2 / 13.3 / 11.3, 1000 x 2048 x 2048 20.4 / 19.2 / 16.6; streaming kernel, 40 x 2048 x 2056 capped 22.1 / 24.7 / 20.1, gates 20.5 / 19.5 / 18.0,
+// 7 x 9728 x 2048 capped 17.3 / 17.6 / 16.4.
 template <bool LOOP, int RT, int MT>
-__device__ __forceinline__ void gemm_activate(const GemmParams& p, f32x4_t (&acc)[RT][MT], int ncol0, int g4, f32x4_t* own) {
-    auto each = [&](auto&& f) __attribute__((always_inline)) {
+__device__ __forceinline__ void gemm_activate(const GemmParams& p, f32x4_t (&acc)[RT][MT], int mcnt, int ncol0, int g4, f32x4_t* own) {
+    auto each = [&](auto&& f, int rows) __attribute__((always_inline)) {   // (16 x 16 pieces of `rows` rows)
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                if (16 * mt >= rows) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[rt][mt][r] = f(acc[rt][mt][r], ncol0 + 16 * rt + 4 * g4 + r);
+            }
+    };
+    auto looped = [&](auto&& f) __attribute__((always_inline)) {
+        if constexpr (!LOOP) each(f, mcnt);
+        else {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[rt][mt][r] = f(acc[rt][mt][r], ncol0 + 16 * rt + 4 * g4 + r);
-    };
-    const bool f32 = p.yf != nullptr;
-    if (!f32 && p.act.kind == GLM_ACT_XIELU) each([&](float a, int) { return glm_xielu_fast(p.act.a, p.act.b, a); });
-    else if (!f32 && p.act.kind >= GLM_ACT_GATE) each([&](float a, int n) { return glm_act_cols(p.act, a, n); });
-    else if constexpr (!LOOP) each([&](float a, int n) { return f32 ? glm_act_precise(p.act, a, n) : glm_act_fast(p.act, a, n); });
-    else {
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) own[(rt * MT + mt) * 64] = acc[rt][mt];
+                for (int rt = 0; rt < RT; ++rt) own[(mt * RT + rt) * 64] = acc[rt][mt];
+            const int last = min((mcnt + 15) >> 4, MT) * RT - 1;
+            f32x4_t v = own[0];
 #pragma unroll 1
-        for (int i = 0; i < RT * MT; ++i) {
-            f32x4_t v = own[i * 64];
-            const int n = ncol0 + 16 * (i / MT) + 4 * g4;
+            for (int i = 0; i <= last; ++i) {
+                const f32x4_t next = own[min(i + 1, last) * 64];   // (its round trip runs under this piece)
+                const int n = ncol0 + 16 * (i % RT) + 4 * g4;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = f32 ? glm_act_precise(p.act, v[r], n + r) : glm_act_fast(p.act, v[r], n + r);
-            own[i * 64] = v;
+                for (int r = 0; r < 4; ++r) v[r] = f(v[r], n + r);
+                own[i * 64] = v;
+                v = next;
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt][mt] = own[(mt * RT + rt) * 64];
         }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = own[(rt * MT + mt) * 64];
-    }
+    };
+    const GlmAct t = p.act;
+    const bool f32 = p.yf != nullptr;
+    auto precise = [&](auto kind) __attribute__((always_inline)) { looped([&](float a, int n) { return glm_act_precise(GlmAct{decltype(kind)::value, t.a, t.b}, a, n); }); };
+    auto cols = [&](auto kind) __attribute__((always_inline)) { each([&](float a, int n) { return glm_act_cols(GlmAct{decltype(kind)::value, t.a, t.b}, a, n); }, 16 * MT); };
+    using std::integral_constant;
+    if (!f32 && t.kind == GLM_ACT_XIELU) each([&](float a, int) { return glm_xielu_fast(t.a, t.b, a); }, 16 * MT);
+    else if (!f32 && t.kind == GLM_ACT_SILU_GATE) cols(integral_constant<int, GLM_ACT_SILU_GATE>{});
+    else if (!f32 && t.kind == GLM_ACT_RELU2_GATE) cols(integral_constant<int, GLM_ACT_RELU2_GATE>{});
+    else if (!f32 && t.kind == GLM_ACT_GATE) cols(integral_constant<int, GLM_ACT_GATE>{});
+    else if (t.kind == GLM_ACT_SOFTCAP) precise(integral_constant<int, GLM_ACT_SOFTCAP>{});
+    else if (t.kind == GLM_ACT_XIELU) precise(integral_constant<int, GLM_ACT_XIELU>{});
+    else if (t.kind == GLM_ACT_SILU_GATE) precise(integral_constant<int, GLM_ACT_SILU_GATE>{});
+    else if (t.kind == GLM_ACT_RELU2_GATE) precise(integral_constant<int, GLM_ACT_RELU2_GATE>{});
+    else if (t.kind == GLM_ACT_GATE) precise(integral_constant<int, GLM_ACT_GATE>{});
 }
 
 // Lane (c,g4) holds, per (rt, mt), columns n..n+3 of token
@@ -74,7 +97,7 @@ __device__ __forceinline__ void gemm_row_epilogue(const GemmParams& p, f32x4_t (
                 }
             }
         }
-        if (p.act.kind != GLM_ACT_NONE) gemm_activate<LOOP>(p, acc, ncol0, g4, own);
+        if (p.act.kind != GLM_ACT_NONE) gemm_activate<LOOP>(p, acc, mcnt, ncol0, g4, own);
         if (p.yf != nullptr) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {

@@ -416,3 +416,39 @@ def test_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
     for y in got[:-1]:
         for a, b in zip(y, got[-1]):
             assert torch.equal(a, b[: a.shape[0]])
+
+
+def act64(kind, a, b, z, ops):
+    n = torch.arange(z.shape[1])
+    if kind == ops.ACT_SOFTCAP:
+        return N_.soft_cap(z, a)
+    if kind == ops.ACT_XIELU:
+        return torch.where(z > 0, a * z * z + 0.5 * z, b * (torch.expm1(z) - z) + 0.5 * z)
+    s = torch.sigmoid(z)
+    if kind == ops.ACT_RELU2_GATE:
+        return torch.where(n >= b, s, torch.where(n < a, torch.relu(z) ** 2, z))
+    return torch.where(n >= a, s, z * s if kind == ops.ACT_SILU_GATE else z)
+
+
+# rows that end in each 16-row piece of a tile, columns that end inside one: shared and split tiles, then the streaming kernels (few rows, K off the 64-wide chunks)
+@pytest.mark.parametrize("M,N,K", [(65, 8200, 128), (81, 8200, 128), (97, 16424, 64), (128, 20000, 64), (113, 520, 576), (49, 40, 320), (300, 4104, 192),
+                                   (2, 520, 512), (16, 4104, 768), (17, 9736, 512), (33, 520, 200), (49, 40, 72), (95, 136, 200), (200, 72, 264)])
+def test_every_activation(ops, M, N, K):
+    """Every kind, fp32 and bf16 rows.  fp32: of the sums that the same call without an activation stores, off by the functions' own error (a few ulp of the
+    terms; xIELU's cancel: 2^-20 of the largest).  bf16: one rounding of that value."""
+    x, w = rnd(M, K, seed=71).cuda(), rnd(N, K, seed=72, scale=K ** -0.5).cuda()
+    x[M // 2, 0], x[M - 1, :2] = float("inf"), float("inf")       # infinite sums, and NaN where both signs meet
+    z = ops.linear_act(x, w, out_f32=True).cpu().double()
+    assert torch.isinf(z).any() and torch.isnan(z).any()
+    for kind, a, b in ((ops.ACT_SOFTCAP, 3.0, 0.0), (ops.ACT_XIELU, 0.8, 0.7), (ops.ACT_GATE, N // 2, 0.0), (ops.ACT_SILU_GATE, N // 2, 0.0), (ops.ACT_SILU_GATE, N, 0.0),
+                       (ops.ACT_RELU2_GATE, N // 2, N // 2 + 24)):
+        ref, what = act64(kind, a, b, z, ops), f"kind {kind}"
+        fine = torch.isfinite(z) & torch.isfinite(ref)
+        y = ops.linear_act(x, w, act=(kind, float(a), float(b)), out_f32=True).cpu().double()
+        assert ((y - ref).abs()[fine] <= 2.0 ** -20 * (1 + ref.abs() + z.abs())[fine]).all(), what
+        y16 = ops.linear_act(x, w, act=(kind, float(a), float(b))).cpu()
+        assert_close_bf16(y16.masked_fill(~fine, 0), ref.to(BF).masked_fill(~fine, 0), 1, 0.05, atol=2 ** -9, what=what)
+        if kind in (ops.ACT_SOFTCAP, ops.ACT_GATE):   # of infinite sums: the cap, or gates of 0 and 1 (passed ones as they are)
+            inf = torch.isinf(z)
+            assert torch.equal(y[inf], ref[inf]) and torch.equal(y16.double()[inf], ref[inf])
+            assert torch.isnan(y[torch.isnan(z) & torch.isnan(ref)]).all()
