@@ -15,17 +15,18 @@ enum GemmMode : int {
     GEMM_PLAIN = 0,   // y[r,n] = bf16(acc + bias[n])                              (a5, a10)
     GEMM_GATEUP = 1,  // act[r,i] = bf16(bf16(silu(bf16(g))) * bf16(u)), W rows gate|up  (a13)
     GEMM_DOWN = 2,    // y[r,n] = bf16(bf16(acc) * scale[r]) for groups < n_scaled    (a12/a13)
-    // gemm_largem only.  GEMM_PLAIN followed by p.act and / or fp32 output rows (p.yf), and its common case without anything left
-    // to decide in the epilogue: their own instantiations, so that the plain kernel's epilogue stays as it is.  (The decode
-    // bodies take p.act / p.yf in GEMM_PLAIN.)
+    // gemm_largem only.  GEMM_PLAIN followed by p.act and / or fp32 output rows (p.yf): the launch picks one of the modes below.  Each is an
+    // instantiation of its own with nothing but its activation in the epilogue.  All in one, chosen per element at run time, made that
+    // as long as the loop: 2048 x 4096 into fp32 rows at 15074 rows 293 -> 212 us (bf16 rows 200).
+    // (The decode bodies take p.act / p.yf in GEMM_PLAIN.)
     GEMM_ACT = 3,
     GEMM_XIELU = 4,  // xIELU, bf16 rows
     GEMM_COLS = 6,   // per-column activation (glm_act_cols), bf16 rows
-    // Fp32 rows with nothing behind the bias (a loop's entry, logits), and logits through a soft cap: every activation inlined per element
-    // and chosen at run time made GEMM_ACT's epilogue as long as its loop.  2048 x 4096 at 15074 rows 293 -> 212 us (bf16 rows 200); on these
-    // tiles 32768 x 2048 at 128 rows 85 -> 43, with the cap 93 -> 50 (since then a round of gemm_midm.hip's: 43 and 48, weights not in the caches).
-    GEMM_F32 = 8,
-    GEMM_CAP = 9,
+    GEMM_F32 = 8,    // fp32 rows with nothing behind the bias (a loop's entry, logits)
+    GEMM_CAP = 9,    // fp32 rows through a soft cap
+    GEMM_XIELU32 = 10,
+    GEMM_COLS32 = 11,
+    GEMM_CAP16 = 12,
     GEMM_SLICES = 7, // G slices of K side by side, K the length of one: fp32 partial sums, slab s of R rows at yf + s R ldy
     GEMM_GLU = 5,    // GEMM_GATEUP's layout (W rows gate|up) with the clamped gated unit of p.act instead of SiLU; fp32 up to the store
 };

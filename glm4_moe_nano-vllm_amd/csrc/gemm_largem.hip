@@ -100,6 +100,10 @@ using LmCfgC88 = LmCfg<256, 128, 2, false, false, true>;  // fp8 x fp8 on the bl
 template <int MODE, class C>
 __host__ __device__ constexpr bool lm_cuts() { return C::RING && !C::W8 && MODE != GEMM_SLICES; }
 
+// single projections of one matrix, with a bias or not
+template <int MODE>
+__host__ __device__ constexpr bool lm_single() { return MODE != GEMM_GATEUP && MODE != GEMM_DOWN && MODE != GEMM_GLU && MODE != GEMM_SLICES; }
+
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
@@ -221,8 +225,8 @@ __device__ __forceinline__ void lm_locate_lanes(const int32_t* __restrict__ offs
 // CUT: tiles of 256 rows from `first` on, each in two of 128.
 template <int MODE, class C, bool LEAN, bool WSCALE, bool CUT>
 __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, int n_tiles, int total_tiles, int LM_BAND, int first) {
-    constexpr bool F32ROWS = MODE == GEMM_ACT || MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP;  // may store fp32 rows (p.yf)
-    constexpr bool BIAS = MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP;
+    constexpr bool F32 = MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP || MODE == GEMM_XIELU32 || MODE == GEMM_COLS32;  // stores fp32 rows (p.yf)
+    constexpr bool BIAS = lm_single<MODE>();
     constexpr bool GROUPED = MODE == GEMM_GATEUP || MODE == GEMM_DOWN;
     static_assert(LEAN || (!C::RING && !C::W8 && !C::A8), "the plain form has the plain ring");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -471,13 +475,12 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
     // Store instructions a wave issues behind the ring fill of the next tile, where their number is known: the waits that open a tile
     // leave that many in flight (vmcnt counts in issue order).  -1: not known, wait for everything.
     constexpr int LM_NOUT = gemm_paired(MODE) ? 2 : 4;
-    constexpr int STORES = C::MT * LM_NOUT / 2, STORES_F32 = C::MT * 4;
+    constexpr int STORES = C::MT * (F32 ? 4 : LM_NOUT / 2);
     int pending_stores = 0;
     // leave `pending_stores` stores and L later DMA instructions in flight
     auto wait_behind_stores = [&](auto lc) {
         constexpr int L = decltype(lc)::value;
         if (LEAN && pending_stores == STORES) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(STORES + L) : "memory");
-        else if (LEAN && F32ROWS && pending_stores == STORES_F32) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(STORES_F32 + L) : "memory");
         else if (pending_stores == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(L) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
@@ -787,6 +790,22 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         constexpr int NOUT = gemm_paired(MODE) ? 2 : 4;  // 16-column output tiles per wave
         const int ncol_w = gemm_paired(MODE) ? ntile_c * 128 + wn * 32 : ntile_c * LM_BN + wn * 64;
         const bool scaled = MODE == GEMM_DOWN && grp_c < p.n_scaled;
+        // the mode's activation on an element of column tile t; kind: p.act.kind where it is one of several with long code (GEMM_COLS32, with_kind)
+        auto act = [&](float a, int t, int r, auto kind) __attribute__((always_inline)) {
+            const int n = ncol_w + 16 * t + 4 * g4 + r;
+            if constexpr (MODE == GEMM_XIELU) return glm_xielu_fast(p.act.a, p.act.b, a);
+            else if constexpr (MODE == GEMM_XIELU32) return glm_act_precise(GlmAct{GLM_ACT_XIELU, p.act.a, p.act.b}, a, n);
+            else if constexpr (MODE == GEMM_CAP || MODE == GEMM_CAP16) return p.act.a * tanhf(a / p.act.a);
+            else if constexpr (MODE == GEMM_COLS) return glm_act_cols(p.act, a, n);
+            else if constexpr (MODE == GEMM_COLS32) return glm_act_precise(GlmAct{decltype(kind)::value, p.act.a, p.act.b}, a, n);
+            else return a;
+        };
+        auto with_kind = [&](auto&& f) __attribute__((always_inline)) {
+            if constexpr (MODE != GEMM_COLS32) f(std::integral_constant<int, GLM_ACT_NONE>{});
+            else if (p.act.kind == GLM_ACT_SILU_GATE) f(std::integral_constant<int, GLM_ACT_SILU_GATE>{});
+            else if (p.act.kind == GLM_ACT_RELU2_GATE) f(std::integral_constant<int, GLM_ACT_RELU2_GATE>{});
+            else f(std::integral_constant<int, GLM_ACT_GATE>{});
+        };
         bool qkv_epi = false;
         if constexpr (MODE == GEMM_PLAIN && LEAN && !WSCALE) qkv_epi = p.qkv_q != nullptr;
         if (qkv_epi) {
@@ -924,10 +943,10 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             // 2048 with a bias 329 / 285, xIELU 314 / 298, 4096 x 2048 half of them gates 207 / 188, 8192 x 2048 of SiLU and gates 411 / 377, 10240 x
             // 2048 of three kinds 507 / 467, plain 6144 x 2048 283 / 281; down of 8 of 64 experts, 4096 x 1408, 1258 / 1238.
             constexpr unsigned BEYOND = 0x80000000u;
-            const bool f32 = F32ROWS && (MODE != GEMM_ACT || p.yf != nullptr);   // (the others have no bf16 form here)
-            const unsigned es = f32 ? 4u : 2u, pitch = (unsigned)p.ldy * es;   // (16 rows are below 2 GiB: launch_largem)
+            constexpr unsigned es = F32 ? 4u : 2u;
+            const unsigned pitch = (unsigned)p.ldy * es;   // (16 rows are below 2 GiB: launch_largem)
             const int64_t first = ((MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0) + m0_c + wm * (C::BM / 2)) * p.ldy + ncol_w;
-            char* ybase = f32 ? reinterpret_cast<char*>(p.yf + first) : reinterpret_cast<char*>(p.y + first);
+            char* ybase = F32 ? reinterpret_cast<char*>(p.yf + first) : reinterpret_cast<char*>(p.y + first);
             const int left = ncol_w < p.N ? mcnt_c - wm * (C::BM / 2) : 0;
             auto rows16 = [&](int mt) __attribute__((always_inline)) {
                 const int rows = min(left - 16 * mt, 16);
@@ -938,23 +957,21 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             // stores f of every element
             auto finish = [&](auto&& f) __attribute__((always_inline)) {
                 if constexpr (LATE_FILL) start_next();   // (its loads of scales are back: pinned above)
-                if constexpr (F32ROWS) {
-                    if (f32) {   // four columns per store
+                if constexpr (F32) {   // four columns per store
 #pragma unroll
-                        for (int mt = 0; mt < C::MT; ++mt) {
-                            const __amdgpu_buffer_rsrc_t yrs = rows16(mt);
+                    for (int mt = 0; mt < C::MT; ++mt) {
+                        const __amdgpu_buffer_rsrc_t yrs = rows16(mt);
 #pragma unroll
-                            for (int t = 0; t < NOUT; ++t) {
-                                const int n = 16 * t + 4 * g4;
-                                f32x4_t o;
+                        for (int t = 0; t < NOUT; ++t) {
+                            const int n = 16 * t + 4 * g4;
+                            f32x4_t o;
 #pragma unroll
-                                for (int r = 0; r < 4; ++r) o[r] = f(t, mt, r);
-                                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, ncol_w + n < p.N ? lrow + n * 4 : BEYOND, 0, 0);
-                            }
-                            __builtin_amdgcn_sched_barrier(0);
+                            for (int r = 0; r < 4; ++r) o[r] = f(t, mt, r);
+                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, ncol_w + n < p.N ? lrow + n * 4 : BEYOND, 0, 0);
                         }
-                        return;
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                    return;
                 }
                 // tiles (t, t+1): after the swaps lane row g4 holds 8 consecutive columns of tile t + (g4 & 1),
                 // starting at column 8 * (g4 >> 1)
@@ -981,14 +998,6 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 if (scaled) finish([&](int t, int mt, int r) { return rbf(sum(t, mt, r)) * e_row[mt]; });
                 else finish(sum);
             } else {
-                auto act = [&](float a, int t, int r) {
-                    const int n = ncol_w + 16 * t + 4 * g4 + r;
-                    if constexpr (MODE == GEMM_XIELU) return glm_xielu_fast(p.act.a, p.act.b, a);
-                    else if constexpr (MODE == GEMM_CAP) return p.act.a * tanhf(a / p.act.a);
-                    else if constexpr (MODE == GEMM_COLS) return glm_act_cols(p.act, a, n);
-                    else if constexpr (MODE == GEMM_ACT) return f32 ? glm_act_precise(p.act, a, n) : glm_act_fast(p.act, a, n);
-                    else return a;
-                };
                 bool plain = !BIAS || p.bias == nullptr;
                 if (plain) {
                     if constexpr (MODE == GEMM_COLS) {   // (a wave's 64 columns are of one kind nearly always)
@@ -999,16 +1008,19 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         else if (relu2 ? ncol_w >= ca && n1 <= cb : !silu && n1 <= ca) finish(sum);
                         else if (ncol_w >= (relu2 ? cb : ca)) finish([&](int t, int mt, int r) { return sigmoid(acc[t][mt][r]); });
                         else if (silu && n1 <= ca) finish([&](int t, int mt, int r) { return acc[t][mt][r] * sigmoid(acc[t][mt][r]); });
-                        else finish([&](int t, int mt, int r) { return act(acc[t][mt][r], t, r); });
+                        else finish([&](int t, int mt, int r) { return glm_act_cols(p.act, acc[t][mt][r], ncol_w + 16 * t + 4 * g4 + r); });
                     } else {
-                        finish([&](int t, int mt, int r) { return act(acc[t][mt][r], t, r); });
+                        with_kind([&](auto kind) __attribute__((always_inline)) { finish([&](int t, int mt, int r) { return act(acc[t][mt][r], t, r, kind); }); });
                     }
                 } else if constexpr (BIAS) {
-                    finish([&](int t, int mt, int r) { return act(acc[t][mt][r] + (r & 1 ? bfhi(e_bias[t][r >> 1]) : bflo(e_bias[t][r >> 1])), t, r); });
+                    with_kind([&](auto kind) __attribute__((always_inline)) {
+                        finish([&](int t, int mt, int r) { return act(acc[t][mt][r] + (r & 1 ? bfhi(e_bias[t][r >> 1]) : bflo(e_bias[t][r >> 1])), t, r, kind); });
+                    });
                 }
             }
-            if (!LATE_FILL) stored = f32 ? STORES_F32 : STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
+            if (!LATE_FILL) stored = STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
         } else {
+        with_kind([&](auto kind) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < C::MT; ++mt) {
             const int row = wm * (C::BM / 2) + 16 * mt + c;
@@ -1034,22 +1046,17 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         if constexpr (WSCALE) a *= p.wscale[(int64_t)grp_c * p.wscale_gstride + min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)];
                         if (BIAS && p.bias) a += bf2f(p.bias[min(ncol_w + 16 * t + 4 * g4 + r, p.N - 1)]);
                         if (scaled) a = rbf(a) * sc;
-                        if (MODE == GEMM_XIELU) a = glm_xielu_fast(p.act.a, p.act.b, a);
-                        if (MODE == GEMM_CAP) a = p.act.a * tanhf(a / p.act.a);
-                        if (MODE == GEMM_COLS) a = glm_act_cols(p.act, a, ncol_w + 16 * t + 4 * g4 + r);
-                        if (MODE == GEMM_ACT) a = p.yf != nullptr ? glm_act_precise(p.act, a, ncol_w + 16 * t + 4 * g4 + r) : glm_act_fast(p.act, a, ncol_w + 16 * t + 4 * g4 + r);
-                        o[r] = a;
+                        o[r] = act(a, t, r, kind);
                     }
                 }
                 const int n = ncol_w + 16 * t + 4 * g4;
-                if (F32ROWS && p.yf != nullptr) {  // fp32 rows: four columns per store
+                if constexpr (F32) {  // fp32 rows: four columns per store
                     const int64_t slab = MODE == GEMM_SLICES ? (int64_t)grp_c * p.R : 0;
                     if (row_ok && n < p.N) *reinterpret_cast<f32x4_t*>(p.yf + (slab + m0_c + row) * p.ldy + n) = f32x4_t{o[0], o[1], o[2], o[3]};
-                    continue;
-                }
-                if (row_ok && n < p.N) *reinterpret_cast<u32x2_t*>(yrow + n) = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
+                } else if (row_ok && n < p.N) *reinterpret_cast<u32x2_t*>(yrow + n) = u32x2_t{pack2bf(o[0], o[1]), pack2bf(o[2], o[3])};
             }
         }
+        });
         }
         pending_stores = stored;
         if (!more) break;
@@ -1138,7 +1145,7 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int64_t cb = (p.R + 127) / 128, bd = cb < LM_BAND_ROWS ? cb : (int64_t)LM_BAND_ROWS;
     const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
                            (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
-    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !((MODE == GEMM_PLAIN || MODE == GEMM_ACT || MODE == GEMM_XIELU || MODE == GEMM_COLS || MODE == GEMM_F32 || MODE == GEMM_CAP) && p.offs == nullptr && p.N <= 128));
+    const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !(lm_single<MODE>() && p.offs == nullptr && p.N <= 128));
     // the lean form addresses x, the group's weights and a tile's rows of y through 32-bit buffer offsets and has no K tail path
     const int var = glm_option(GLM_OPT_LARGEM_VARIANT);
     const int64_t wrows = gemm_paired(MODE) ? 2 * (int64_t)p.N : (int64_t)p.N;
@@ -1218,12 +1225,19 @@ int glm_launch_gemm_largem(int mode, const GemmParams& p, hipStream_t st) {
     if (mode == GEMM_GATEUP) return launch_largem<GEMM_GATEUP>(p, st);
     if (mode == GEMM_DOWN) return launch_largem<GEMM_DOWN>(p, st);
 #endif  // GLM_EXPERTS
-    if (mode == GEMM_ACT && p.yf == nullptr && p.act.kind >= GLM_ACT_GATE) return launch_largem<GEMM_COLS>(p, st);
-    if (mode == GEMM_ACT && p.yf == nullptr && p.act.kind == GLM_ACT_XIELU) return launch_largem<GEMM_XIELU>(p, st);
-    if (mode == GEMM_ACT && p.yf != nullptr && p.act.kind == GLM_ACT_NONE) return launch_largem<GEMM_F32>(p, st);
-    if (mode == GEMM_ACT && p.yf != nullptr && p.act.kind == GLM_ACT_SOFTCAP) return launch_largem<GEMM_CAP>(p, st);
+    if (mode == GEMM_ACT && p.yf != nullptr) switch (p.act.kind) {
+        case GLM_ACT_NONE: return launch_largem<GEMM_F32>(p, st);
+        case GLM_ACT_SOFTCAP: return launch_largem<GEMM_CAP>(p, st);
+        case GLM_ACT_XIELU: return launch_largem<GEMM_XIELU32>(p, st);
+        default: return launch_largem<GEMM_COLS32>(p, st);
+    }
+    if (mode == GEMM_ACT) switch (p.act.kind) {
+        case GLM_ACT_NONE: return launch_largem<GEMM_PLAIN>(p, st);
+        case GLM_ACT_SOFTCAP: return launch_largem<GEMM_CAP16>(p, st);
+        case GLM_ACT_XIELU: return launch_largem<GEMM_XIELU>(p, st);
+        default: return launch_largem<GEMM_COLS>(p, st);
+    }
     if (mode == GEMM_SLICES) return launch_largem<GEMM_SLICES>(p, st);
-    if (mode == GEMM_ACT) return launch_largem<GEMM_ACT>(p, st);
     if (mode == GEMM_GLU) return launch_largem<GEMM_GLU>(p, st);
     return launch_largem<GEMM_PLAIN>(p, st);
 }

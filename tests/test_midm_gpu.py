@@ -430,9 +430,11 @@ def act64(kind, a, b, z, ops):
     return torch.where(n >= a, s, z * s if kind == ops.ACT_SILU_GATE else z)
 
 
-# rows that end in each 16-row piece of a tile, columns that end inside one: shared and split tiles, then the streaming kernels (few rows, K off the 64-wide chunks)
+# rows that end in each 16-row piece of a tile, columns that end inside one: shared and split tiles, then the streaming kernels (few rows, K off the 64-wide chunks),
+# then the tiled kernel: 256-row blocks in the lean and in the plain form, 128-row blocks in the plain form, several rounds of few rows
 @pytest.mark.parametrize("M,N,K", [(65, 8200, 128), (81, 8200, 128), (97, 16424, 64), (128, 20000, 64), (113, 520, 576), (49, 40, 320), (300, 4104, 192),
-                                   (2, 520, 512), (16, 4104, 768), (17, 9736, 512), (33, 520, 200), (49, 40, 72), (95, 136, 200), (200, 72, 264)])
+                                   (2, 520, 512), (16, 4104, 768), (17, 9736, 512), (33, 520, 200), (49, 40, 72), (95, 136, 200), (200, 72, 264),
+                                   (8500, 1032, 64), (8500, 1036, 64), (1300, 2052, 72), (1030, 15368, 64)])
 def test_every_activation(ops, M, N, K):
     """Every kind, fp32 and bf16 rows.  fp32: of the sums that the same call without an activation stores, off by the functions' own error (a few ulp of the
     terms; xIELU's cancel: 2^-20 of the largest).  bf16: one rounding of that value."""
