@@ -17,7 +17,10 @@ enum GemmMode : int {
     GEMM_DOWN = 2,    // y[r,n] = bf16(bf16(acc) * scale[r]) for groups < n_scaled    (a12/a13)
     // gemm_largem only.  GEMM_PLAIN followed by p.act and / or fp32 output rows (p.yf): the launch picks one of the modes below.  Each is an
     // instantiation of its own with nothing but its activation in the epilogue.  All in one, chosen per element at run time, made that
-    // as long as the loop: 2048 x 4096 into fp32 rows at 15074 rows 293 -> 212 us (bf16 rows 200).
+    // as long as the loop: 2048 x 4096 into fp32 rows at 15074 rows 293 -> 212 us (bf16 rows 200).  Gates, xIELU into fp32 rows and a soft cap into bf16 rows, us, all
+    // in one with every element deciding / all in one with two forms per wave / this: 4100 x 2048 x 2048 gates 86 / 68 / 53, xIELU 90 / 72 / 50, cap 86 / 62 /
+    // 51; 2044 columns (the plain form, whose accumulators had gone to scratch) 93 / 104 / 63, 96 / 110 / 62, 93 / 99 / 61; 12000 x 6148 x 2056 556 / 730 /
+    // 408, 572 / 758 / 408, 500 / 649 / 369.
     // (The decode bodies take p.act / p.yf in GEMM_PLAIN.)
     GEMM_ACT = 3,
     GEMM_XIELU = 4,  // xIELU, bf16 rows
