@@ -42,13 +42,14 @@ constexpr int LM_BN = 256;    // weight rows per tile (MFMA row axis); 4 waves x
 constexpr int LM_BAND_ROWS = 4;  // row blocks per L2 supertile band
 constexpr int LM_CUT_K = 512;    // shortest reduction whose last tiles are cut
 constexpr int LM_SLOT = 32768;   // CfgR: bytes of a ring slot, one operand tile
+constexpr int64_t LM_WIDE = 1 << 25;   // output pitch from which 16 fp32 rows do not fit into a buffer
 
 // Tile configurations (the kernel is written once over these):
 //   CfgR 256(n) x 256(m) x 64(k), five 32-KiB slots of one operand tile each, two phases of 32 MFMAs per K tile
 //   CfgA 256(n) x 128(m) x 64(k), 3-stage ring, wave tile 64x64  (16 LDS reads + 6 DMA per 32 MFMA)
 //   CfgB 256(n) x 256(m) x 32(k), 4-stage ring, wave tile 64x128 (12 LDS reads + 4 DMA per 32 MFMA): only where K is no whole
 //        number of 64 or an operand spans 2 GiB (the plain form)
-template <int BM_, int BK_, int NSTAGE_, bool RING_ = false, bool W8_ = false, bool A8_ = false>
+template <int BM_, int BK_, int NSTAGE_, bool RING_ = false, bool W8_ = false, bool A8_ = false, bool WIDE_ = false>
 struct LmCfg {
     static constexpr int BM = BM_, BK = BK_, NSTAGE = NSTAGE_;
     static constexpr bool RING = RING_;
@@ -63,6 +64,7 @@ struct LmCfg {
     // value) between its ds_read and the MFMA, and the per-row dequantisation scale multiplies the fp32 accumulator in the
     // epilogue (WSCALE) — the arithmetic of the expansion pass + bf16 kernel it replaces, bit for bit.
     static constexpr bool W8 = W8_;
+    static constexpr bool WIDE = WIDE_;            // output rows too far apart for buffers of 16 (fp8 weights: they have no plain form)
     static constexpr int RB = A8 ? BK : BK * 2;    // bytes per ACTIVATION tile row (and per weight tile row unless W8)
     static constexpr int CPR = RB / 16;            // 16-B chunks per row
     static constexpr int RPI = 1024 / RB;          // rows per DMA instruction
@@ -95,6 +97,8 @@ using LmCfgR = LmCfg<256, 64, 2, true>;
 using LmCfgR8 = LmCfg<256, 64, 2, true, true>;  // fp8 weight operand (its tiles fill half a slot)
 using LmCfgA8 = LmCfg<128, 64, 3, false, true>;
 using LmCfgC88 = LmCfg<256, 128, 2, false, false, true>;  // fp8 x fp8 on the block-scaled MFMA: two 64-KiB buffers, the rest of the LDS holds scales
+using LmCfgA8Wide = LmCfg<128, 64, 3, false, true, false, true>;
+using LmCfgC88Wide = LmCfg<256, 128, 2, false, false, true, true>;
 
 // configurations whose last tiles may be cut (the 128-row one's ring fits into theirs)
 template <int MODE, class C>
@@ -983,7 +987,10 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         const int n = 16 * (t + (g4 & 1)) + 8 * (g4 >> 1);
                         const u32x2_t a = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 0), f(t, mt, 1)), pack2bf(f(t + 1, mt, 0), f(t + 1, mt, 1)), false, false);
                         const u32x2_t b = __builtin_amdgcn_permlane16_swap(pack2bf(f(t, mt, 2), f(t, mt, 3)), pack2bf(f(t + 1, mt, 2), f(t + 1, mt, 3)), false, false);
-                        __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{a[0], b[0], a[1], b[1]}, yrs, ncol_w + n < p.N ? lrow + n * 2 : BEYOND, 0, 0);
+                        const u32x4_t o = {a[0], b[0], a[1], b[1]};
+                        if constexpr (C::WIDE) {
+                            if (16 * mt + c < left && ncol_w + n < p.N) *reinterpret_cast<u32x4_t*>(p.y + first + (16 * mt + c) * p.ldy + n) = o;
+                        } else __builtin_amdgcn_raw_buffer_store_b128(o, yrs, ncol_w + n < p.N ? lrow + n * 2 : BEYOND, 0, 0);
                     }
                     __builtin_amdgcn_sched_barrier(0);   // (the other rows' values would take registers that are not there)
                 }
@@ -1018,7 +1025,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                     });
                 }
             }
-            if (!LATE_FILL) stored = STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
+            if (!LATE_FILL && !C::WIDE) stored = STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
         } else {
         with_kind([&](auto kind) __attribute__((always_inline)) {
 #pragma unroll
@@ -1150,11 +1157,12 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int var = glm_option(GLM_OPT_LARGEM_VARIANT);
     const int64_t wrows = gemm_paired(MODE) ? 2 * (int64_t)p.N : (int64_t)p.N;
     const bool lean_ok = p.K % 64 == 0 && p.R * p.ldx * 2 < (1ll << 31) && wrows * p.ldw * 2 < (1ll << 31) &&
-                         p.N % 8 == 0 && p.ldy % 8 == 0 && p.ldy < (1 << 25) && glm_aligned16(p.y);
+                         p.N % 8 == 0 && p.ldy % 8 == 0 && glm_aligned16(p.y);
+    const bool wide = p.ldy >= LM_WIDE;
     if (p.w_fp8) {
         // fp8 weight operand: the lean form only;
         // what they do not cover (a K tail, offsets past 2^31) goes back to the caller, which expands the stack instead
-        if (!lean_ok || p.K % 64 != 0 || p.wscale == nullptr || p.ldw % 16 != 0 || p.w_gstride % 16 != 0) {
+        if (!lean_ok || (wide && MODE != GEMM_DOWN) || p.wscale == nullptr || p.ldw % 16 != 0 || p.w_gstride % 16 != 0) {
             glm_set_error("gemm_largem(fp8 weights): shape not covered (K=%d N=%d ldw=%ld)", p.K, p.N, (long)p.ldw);
             return GLM_ERR_UNSUPPORTED;
         }
@@ -1162,11 +1170,14 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
             glm_set_error("gemm_largem(fp8 weights): only the grouped expert projections are quantised");
             return GLM_ERR_UNSUPPORTED;
         } else {
+            if (wide) {
+                if constexpr (MODE == GEMM_DOWN) return launch_largem_cfg<MODE, LmCfgA8Wide, true>(p, st);
+            }
             if (use_b) return launch_largem_cfg<MODE, LmCfgR8, true>(p, st);
             return launch_largem_cfg<MODE, LmCfgA8, true>(p, st);
         }
     }
-    const bool lean = lean_ok && (var < 0 || var == LM_VAR_LEAN);
+    const bool lean = lean_ok && !wide && (var < 0 || var == LM_VAR_LEAN);
     if (p.qkv_q != nullptr && (!lean || p.wscale != nullptr)) {  // 16-byte-store form, bf16 weights only
         glm_set_error("gemm_largem(qkv epilogue): the plain form has no such epilogue");
         return GLM_ERR_UNSUPPORTED;
@@ -1188,12 +1199,13 @@ int glm_launch_gemm_largem_a8(int mode, const GemmParams& p, hipStream_t st) {
                     p.R * p.ldx < (1ll << 31) && wrows * p.ldw < (1ll << 31) && glm_aligned16(p.x) && glm_aligned16(p.w) &&
                     (mode == GEMM_GATEUP ? (p.xscale != nullptr && p.ybscale != nullptr && p.ldy % 4 == 0 && (((uintptr_t)p.y) & 3) == 0 &&
                                             p.N % 32 == 0 && p.N <= 2048)
-                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && p.ldy < (1 << 25) && glm_aligned16(p.y)));
+                                         : (p.xbscale != nullptr && glm_aligned16(p.xbscale) && p.K <= 2048 && p.ldy % 8 == 0 && glm_aligned16(p.y)));
     if (!ok) {
         glm_set_error("gemm_largem(fp8 x fp8): shape not covered (mode %d R=%ld G=%d N=%d K=%d)", mode, (long)p.R, p.G, p.N, p.K);
         return GLM_ERR_UNSUPPORTED;
     }
     if (mode == GEMM_GATEUP) return launch_largem_cfg<GEMM_GATEUP, LmCfgC88, true>(p, st);
+    if (p.ldy >= LM_WIDE) return launch_largem_cfg<GEMM_DOWN, LmCfgC88Wide, true>(p, st);
     return launch_largem_cfg<GEMM_DOWN, LmCfgC88, true>(p, st);
 }
 

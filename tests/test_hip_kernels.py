@@ -1132,17 +1132,52 @@ def test_gemm_large_m_tile_lists(ops, M, N):
     assert torch.equal(*got) and bool((got[1][-1] == 7).all())
 
 
-@pytest.mark.parametrize("pitch", [1 << 21, (1 << 23) + 8])
-def test_gemm_large_m_wide_pitch(ops, pitch):
-    """Output rows so far apart that a tile's do not fit into 2 GiB; bit for bit against rows side by side, nothing behind a row's columns."""
-    M, N, K = 700, 8200, 192
+@pytest.mark.parametrize("pitch,f32", [(1 << 21, False), ((1 << 25) - 8, False), ((1 << 25) - 8, True), (1 << 25, False), (1 << 25, True)])
+def test_gemm_large_m_wide_pitch(ops, pitch, f32):
+    """Output rows up to 64 MiB (bf16) or 128 MiB (fp32) apart, the most that 16 rows of a store buffer may span, and one step more, where the plain form takes
+    over; bit for bit against rows side by side, nothing behind a row's columns and in the rows around."""
+    M, N, K = 131, 328, 192      # (both halves of a row block)
     g = torch.Generator(device="cuda").manual_seed(3)
     x = torch.randn(M, K, device="cuda", generator=g).to(BF)
     w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
-    out = torch.empty(M * pitch, device="cuda", dtype=BF).view(M, pitch)
-    out[:, N] = 7
-    ops.linear_act(x, w, out=out[:, :N])
-    assert torch.equal(out[:, :N], ops.linear_act(x, w)) and bool((out[:, N] == 7).all())
+    buf = torch.empty((M + 2) * pitch, device="cuda", dtype=torch.float32 if f32 else BF).view(M + 2, pitch)
+    buf[:, N] = 7
+    buf[0, :N], buf[-1, :N] = 7, 7
+    for cfg in (1, 2):
+        with ops.option("largem_cfg", cfg):
+            buf[1:-1, :N] = 0
+            ops.linear_act(x, w, out_f32=f32, out=buf[1:-1, :N])
+            assert torch.equal(buf[1:-1, :N], ops.linear_act(x, w, out_f32=f32))
+        assert bool((buf[:, N] == 7).all()) and bool((buf[0, :N] == 7).all()) and bool((buf[-1, :N] == 7).all())
+
+
+@pytest.mark.parametrize("pitch", [(1 << 25) - 8, 1 << 25, (1 << 25) + 264])
+def test_fp8_expert_down_wide_pitch(ops, pitch):
+    """Down projections of fp8 weights, fp8 or bf16 rows, have no plain form: output rows 64 MiB and more apart are stored through addresses.  Bit for
+    bit against rows side by side."""
+    R, H, I, G = 400, 264, 256, 2
+    g = torch.Generator(device="cuda").manual_seed(5)
+    offs = torch.tensor([0, 193, R], dtype=torch.int32, device="cuda")
+    e4m3 = lambda t: t.to(torch.float8_e4m3fn).view(torch.uint8)
+    w2, ws = e4m3(torch.randn(G, H, I, device="cuda", generator=g)), torch.rand(G, H, device="cuda", generator=g) + 0.5
+    act, act8 = torch.randn(R, I, device="cuda", generator=g).to(BF), e4m3(torch.randn(R, I, device="cuda", generator=g))
+    bs = torch.randint(122, 130, (R, 64), device="cuda", generator=g, dtype=torch.uint8)
+    scale = (torch.rand(R, device="cuda", generator=g) + 0.1).to(BF)
+    lib, p, st = ops.load_library(), ops._p, ops._stream()
+    buf = torch.empty((R + 2) * pitch, device="cuda", dtype=BF).view(R + 2, pitch)
+    buf[:, H] = 7
+    buf[0, :H], buf[-1, :H] = 7, 7
+    for what, ref, call in (
+            ("fp8 x fp8", ops.grouped_gemm_down_fp8a8(act8, bs, w2, ws, offs, scale, G - 1), lambda y: lib.glm_grouped_gemm_down_fp8a8(
+                p(act8), I, p(bs), p(w2), w2.stride(0), I, p(ws), H, p(offs), p(scale), G - 1, p(y), pitch, R, H, I, G, st)),
+            ("fp8 weights", ops.grouped_gemm_down_fp8w(act, w2, ws, offs, scale, G - 1), lambda y: lib.glm_grouped_gemm_down_fp8w(
+                p(act), p(w2), w2.stride(0), I, p(ws), H, p(offs), p(scale), G - 1, p(y), pitch, R, H, I, G, None, 0, st))):
+        assert ref is not None and float(ref.float().abs().sum()) > 0
+        y = buf[1:-1, :H]
+        y.zero_()
+        assert call(y) == 0, what
+        assert torch.equal(y, ref), what
+        assert bool((buf[:, H] == 7).all()) and bool((buf[0, :H] == 7).all()) and bool((buf[-1, :H] == 7).all()), what
 
 
 @pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (16700, 4, 2, 512)])
