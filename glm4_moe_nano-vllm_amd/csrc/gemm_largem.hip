@@ -730,6 +730,12 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         if (wid < 4) __builtin_amdgcn_s_barrier();  // match the other group's extra barrier
         }
 
+        // The epilogue of the fp8 x fp8 gate|up kernel LOADS (weight-row scales, token scales) and vector-memory results return in issue
+        // order — behind the ring fill they cost a whole fill latency per tile (epilogue 23.5k cycles against 6.0k for bf16).
+        // There the next tile's fill is issued once the first 16-row block of the epilogue has its loads back, i.e. behind them and
+        // in front of the bulk of the stores, which lie on both sides of it: the next tile waits for everything.
+        // (The scale vectors as LDS-DMA pieces of the ring fill: no gain.)
+        constexpr bool LATE_FILL = C::A8 && gemm_paired(MODE);
         // What the epilogue reads of the finished tile's rows and columns: requested in front of the ring fill (waiting for a load issued behind the
         // fill would drain the fill first).
         float e_row[C::MT], e_col[4][4];
@@ -745,7 +751,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             }
             // column of the wave's first output column, or gate column, of tile t
             auto col = [&](int t, int r) { return gemm_paired(MODE) ? ntile_c * 128 + wn * 32 + 16 * (t & 1) + 4 * g4 + r : ntile_c * LM_BN + wn * 64 + 16 * t + 4 * g4 + r; };
-            if constexpr (WSCALE && !(C::A8 && gemm_paired(MODE))) {
+            if constexpr (WSCALE && !LATE_FILL) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -763,17 +769,12 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         }
         // ---- next tile: every wave is past its last LDS read, so the ring can be refilled right away ----
         const bool more = find_tile();
-        // The epilogue of the fp8 x fp8 kernels LOADS (weight-row scales, token scales) and vector-memory results return in issue
-        // order — behind the ring fill they cost a whole fill latency per tile (epilogue 23.5k cycles against 6.0k for bf16).
-        // There the next tile's fill is issued once the first 16-row block of the epilogue has its loads back, i.e. behind them and
-        // in front of the bulk of the stores.  (The scale vectors as LDS-DMA pieces of the ring fill: no gain.)
-        constexpr bool LATE_FILL = C::A8;
         if (more) setup_sources();   // (its own loads — the gathered source rows — go out here, behind the epilogue's)
         if constexpr (LEAN && MODE == GEMM_DOWN) {
 #pragma unroll
             for (int mt = 0; mt < C::MT; ++mt) asm volatile("" : "+v"(e_row[mt]));  // the loads stay above the fill
         }
-        if constexpr (LEAN && WSCALE && !(C::A8 && gemm_paired(MODE))) {
+        if constexpr (LEAN && WSCALE && !LATE_FILL) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(e_col[i >> 2][i & 3]));
         }
@@ -877,7 +878,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                     }
                 }
             }
-        } else if constexpr (C::A8 && gemm_paired(MODE)) {
+        } else if constexpr (LATE_FILL) {
             // ---- fp8 x fp8 gate|up: the accumulator x weight-row scale x token scale is the bf16 GEMM's value up to the
             // fp8 roundings of its inputs; same rounding points behind it (mlp.py:49-53: bf16 gate_up, bf16 silu, bf16
             // product).  The product is then quantised for the down projection's fp8 operand in MX form, decided locally:
@@ -960,7 +961,6 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             const unsigned lrow = (unsigned)c * pitch;
             // stores f of every element
             auto finish = [&](auto&& f) __attribute__((always_inline)) {
-                if constexpr (LATE_FILL) start_next();   // (its loads of scales are back: pinned above)
                 if constexpr (F32) {   // four columns per store
 #pragma unroll
                     for (int mt = 0; mt < C::MT; ++mt) {
@@ -1025,7 +1025,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                     });
                 }
             }
-            if (!LATE_FILL && !C::WIDE) stored = STORES;   // (the fp8 x fp8 kernels, whose stores lie on both sides of the fill, wait for everything)
+            if constexpr (!C::WIDE) stored = STORES;
         } else {
         with_kind([&](auto kind) __attribute__((always_inline)) {
 #pragma unroll
