@@ -30,6 +30,9 @@ enum GemmMode : int {
     GEMM_XIELU32 = 10,
     GEMM_COLS32 = 11,
     GEMM_CAP16 = 12,
+    // GEMM_PLAIN with the split / rotary / cache-store epilogue (p.qkv_q).  In one kernel with the bias and plain epilogues of both walks 122 scalars
+    // and 3 vector registers were spilled (28 and 55 scalars now); 15074 x 6144 x 2048, us, kernel with all / this: 308.0 / 305.9 .. 313.5 / 311.2.
+    GEMM_QKV = 13,
     GEMM_SLICES = 7, // G slices of K side by side, K the length of one: fp32 partial sums, slab s of R rows at yf + s R ldy
     GEMM_GLU = 5,    // GEMM_GATEUP's layout (W rows gate|up) with the clamped gated unit of p.act instead of SiLU; fp32 up to the store
 };

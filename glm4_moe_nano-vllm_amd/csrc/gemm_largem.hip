@@ -230,7 +230,7 @@ __device__ __forceinline__ void lm_locate_lanes(const int32_t* __restrict__ offs
 template <int MODE, class C, bool LEAN, bool WSCALE, bool CUT>
 __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, int n_tiles, int total_tiles, int LM_BAND, int first) {
     constexpr bool F32 = MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP || MODE == GEMM_XIELU32 || MODE == GEMM_COLS32;  // stores fp32 rows (p.yf)
-    constexpr bool BIAS = lm_single<MODE>();
+    constexpr bool BIAS = lm_single<MODE>() && MODE != GEMM_QKV;   // (in the common epilogue)
     constexpr bool GROUPED = MODE == GEMM_GATEUP || MODE == GEMM_DOWN;
     static_assert(LEAN || (!C::RING && !C::W8 && !C::A8), "the plain form has the plain ring");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -759,7 +759,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         e_col[t][r] = p.wscale[(int64_t)grp_c * p.wscale_gstride + (gemm_paired(MODE) && t > 1 ? p.N : 0) + min(col(t, r), p.N - 1)];
             }
             if constexpr (BIAS) {
-                if (p.bias != nullptr && (MODE != GEMM_PLAIN || p.qkv_q == nullptr)) {
+                if (p.bias != nullptr) {
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -811,9 +811,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             else if (p.act.kind == GLM_ACT_RELU2_GATE) f(std::integral_constant<int, GLM_ACT_RELU2_GATE>{});
             else f(std::integral_constant<int, GLM_ACT_GATE>{});
         };
-        bool qkv_epi = false;
-        if constexpr (MODE == GEMM_PLAIN && LEAN && !WSCALE) qkv_epi = p.qkv_q != nullptr;
-        if (qkv_epi) {
+        if constexpr (MODE == GEMM_QKV) {
             // ---- QKV epilogue: bias, bf16 rounding (the packed qkv value of the reference, linear.py:75), rotary on the
             // first 64 dims of every q / k head, split, cache scatter.  A wave's 64 columns are one half of one head (ncol_w
             // is a multiple of 64): the rotary half pairs column i with i + 32 = accumulator tiles t and t + 2 in the SAME
@@ -1178,12 +1176,11 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
         }
     }
     const bool lean = lean_ok && !wide && (var < 0 || var == LM_VAR_LEAN);
-    if (p.qkv_q != nullptr && (!lean || p.wscale != nullptr)) {  // 16-byte-store form, bf16 weights only
+    if (lean) return use_b ? launch_largem_cfg<MODE, LmCfgR, true>(p, st) : launch_largem_cfg<MODE, LmCfgA, true>(p, st);
+    if constexpr (MODE == GEMM_QKV) {  // 16-byte-store form only
         glm_set_error("gemm_largem(qkv epilogue): the plain form has no such epilogue");
         return GLM_ERR_UNSUPPORTED;
-    }
-    if (lean) return use_b ? launch_largem_cfg<MODE, LmCfgR, true>(p, st) : launch_largem_cfg<MODE, LmCfgA, true>(p, st);
-    return use_b ? launch_largem_cfg<MODE, LmCfgB, false>(p, st) : launch_largem_cfg<MODE, LmCfgA, false>(p, st);
+    } else return use_b ? launch_largem_cfg<MODE, LmCfgB, false>(p, st) : launch_largem_cfg<MODE, LmCfgA, false>(p, st);
 }
 
 }  // namespace
@@ -1223,7 +1220,7 @@ int glm_launch_gemm_largem_qkv(const GemmParams& p, hipStream_t st) {
     q.y = p.qkv_q;  // never stored through; keeps the generic alignment checks meaningful
     q.ldy = p.N;
     if (glm_midm_takes(GEMM_PLAIN, q)) return glm_launch_gemm_midm(GEMM_PLAIN, q, st);  // where glm_gemm_bf16 goes there, bit-identical to it
-    return launch_largem<GEMM_PLAIN>(q, st);
+    return launch_largem<GEMM_QKV>(q, st);
 }
 #endif  // !GLM_DENSE_ONLY
 
