@@ -614,7 +614,7 @@ int launch_midm_cfg(const GemmParams& p, hipStream_t st) {
     return GLM_OK;
 }
 
-template <int MODE, int WM, int WN, int MT, int RT, int NST>
+template <int MODE, int WM, int WN, int MT, int RT, int NST, bool NT>
 int launch_midm_shared(const GemmParams& p, hipStream_t st) {
     constexpr int LDS = midm_shared_lds<WM, WN, MT, RT, NST>();
     static_assert(LDS <= 160 * 1024, "the ring must fit the CU's LDS");
@@ -623,12 +623,7 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
     const bool dealt = nt >= 64;
     const int64_t gx = dealt ? (int64_t)(nt + 7) / 8 * 8 * mblocks : (nt * mblocks + 7) / 8 * 8;
     GLM_CHECK_ARG(gx < (1 << 30), GLM_ERR_UNSUPPORTED, "gemm_midm: grid too large");
-    // Weights that only one row block reads go past the caches, which they leave to the activations (nt).  Kept / past them, us, weights not in the caches:
-    // 128 rows of 32768 x 2048 33.1 / 31.5, gated 30.7 / 28.8, 64 of 14336 x 4096 29.6 / 27.7, 41 of 8928 x 576 6.5 / 6.0; steps: 64 GLM sequences over fp8
-    // experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With two row blocks and more, and in the split tiles, single projections gained as much and
-    // steps lost it again (a prompt of 211 1.886 / 1.904 ms).  A kernel of its own: chosen inside the loop, for every DMA instruction, it cost all others 1 to
-    // 5 % (gate|up 965 of 456 x 6912 32.9 / 31.3, 300 of 1024 x 2048 12.1 / 11.7, plain 300 of 2048 x 2048 12.6 / 12.4).
-    auto kern = mblocks == 1 ? gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST, true> : gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST, false>;
+    auto kern = gemm_midm_shared_kernel<MODE, WM, WN, MT, RT, NST, NT>;
     if (LDS > 64 * 1024) GLM_SET_MAX_LDS(kern, LDS, "gemm_midm");
     hipLaunchKernelGGL(kern, dim3((unsigned)gx, 1, (unsigned)(p.ksplit > 1 ? p.ksplit : 1)), dim3(WM * WN * 64), LDS, st, p, (int)mblocks, (int)dealt);
     GLM_CHECK_LAUNCH("gemm_midm");
@@ -667,24 +662,30 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
     return fits(128, 128) ? MM_128 : MM_NONE;
 }
 
+// Weights that only one row block reads go past the caches, which they leave to the activations (nt).  Kept / past them, us, weights not in the caches:
+// 128 rows of 32768 x 2048 33.1 / 31.5, gated 30.7 / 28.8, 64 of 14336 x 4096 29.6 / 27.7, 41 of 8928 x 576 6.5 / 6.0; steps: 64 GLM sequences over fp8
+// experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With two row blocks and more, and in the split tiles, single projections gained as much and
+// steps lost it again (a prompt of 211 1.886 / 1.904 ms).  A kernel of its own: chosen inside the loop, for every DMA instruction, it cost all others 1 to
+// 5 % (gate|up 965 of 456 x 6912 32.9 / 31.3, 300 of 1024 x 2048 12.1 / 11.7, plain 300 of 2048 x 2048 12.6 / 12.4).
 template <int MODE>
 int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
+    if constexpr (MODE == GEMM_PLAIN) {   // half a head in the QKV epilogue of 32 rows; the sums are the same in all three
+        if (p.qkv_q != nullptr && (tile == MM_SPLIT16 || tile == MM_SPLIT32x32)) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);
+    }
     switch (tile) {
         case MM_SPLIT16:
-            if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);   // (half a head)
             if constexpr (!gemm_paired(MODE)) return launch_midm_cfg<MODE, 2, 1, 8, 2>(p, st);
             break;
-        case MM_SPLIT32x32:
-            if (MODE == GEMM_PLAIN && p.qkv_q != nullptr) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);
-            return launch_midm_cfg<MODE, 2, 2, 8, 2>(p, st);
+        case MM_SPLIT32x32: return launch_midm_cfg<MODE, 2, 2, 8, 2>(p, st);
         case MM_SPLIT32:   // (half a head in the QKV epilogue; the sums are the same in both tiles)
             if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
             [[fallthrough]];
         case MM_SPLIT64: return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);
-        case MM_64: return launch_midm_shared<MODE, 2, 2, 2, 2, 4>(p, st);
-        case MM_128x64: return launch_midm_shared<MODE, 2, 2, 4, 2, 3>(p, st);
-        case MM_64x128: return launch_midm_shared<MODE, 2, 4, 2, 2, 3>(p, st);
-        case MM_128: return launch_midm_shared<MODE, 2, 4, 4, 2, 4>(p, st);
+        // (true: nt, see above; no more than 64 rows take MM_64x128)
+        case MM_64: return p.R <= 64 ? launch_midm_shared<MODE, 2, 2, 2, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 2, 2, 2, 4, false>(p, st);
+        case MM_128x64: return p.R <= 128 ? launch_midm_shared<MODE, 2, 2, 4, 2, 3, true>(p, st) : launch_midm_shared<MODE, 2, 2, 4, 2, 3, false>(p, st);
+        case MM_64x128: return launch_midm_shared<MODE, 2, 4, 2, 2, 3, true>(p, st);
+        case MM_128: return p.R <= 128 ? launch_midm_shared<MODE, 2, 4, 4, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 4, 4, 2, 4, false>(p, st);
         default: break;
     }
     GLM_CHECK_ARG(false, GLM_ERR_UNSUPPORTED, "gemm_midm: no tile for %ld rows, N=%d", (long)p.R, p.N);
