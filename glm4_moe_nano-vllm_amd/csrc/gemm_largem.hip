@@ -1144,12 +1144,13 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
     const int64_t avg_rows = (p.R_hint > 0 ? p.R_hint : p.R) / (p.G > 0 && MODE != GEMM_SLICES ? p.G : 1);
     // ... and a projection onto <= 128 columns (the router logits at prefill: N = E = 64) is one column tile however the rows
     // are cut, so its parallelism is its row-block count: 128-row blocks (75.8 -> 55.1 us at T = 16384)
-    // ... and so is every single projection whose 128-row tiles are at most one round of the chip (with the band's rounding, as
-    // launch_largem_cfg counts): a K step costs two thirds (14336 x 4096 at 400 rows 86 / 59 us, 4096 x 12288 at 1200 rows 234 / 153; beyond a
-    // round 9728 x 2048 at 800 rows 48 / 60; what is a round of 128 x 128 tiles does not come here, gemm_midm.hip)
-    const int64_t cb = (p.R + 127) / 128, bd = cb < LM_BAND_ROWS ? cb : (int64_t)LM_BAND_ROWS;
+    // ... and so is every single projection whose 128-row tiles are at most one round of the chip (the tiles themselves: launch_largem_cfg leaves out
+    // positions without one where they would be a second round): a K step costs two thirds.  256-row / 128-row tiles, us: 14336 x 4096 at 400 rows 86 /
+    // 59, 4096 x 12288 at 1200 234 / 153, 6144 x 2048 at 1100 (216 tiles, 288 positions) 43.3 / 32.8, 12288 x 4096 at 600 74.4 / 65.1, 10240 x 4096 at 700
+    // 75.2 / 61.0, 3072 x 2048 at 2600 41.0 / 32.6; beyond a round 6144 x 2048 at 1281 43.7 / 53.0, 9728 x 2048 at 800 48 / 60.  (What is a round of 128 x
+    // 128 tiles does not come here, gemm_midm.hip.)
     const bool one_round = p.offs == nullptr && MODE != GEMM_SLICES && p.wscale == nullptr && !p.w_fp8 &&
-                           (cb + bd - 1) / bd * bd * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
+                           (p.R + 127) / 128 * ((p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256)) <= 256;
     const bool use_b = ch == 2 || (ch == 0 && avg_rows >= 192 && !one_round && !(lm_single<MODE>() && p.offs == nullptr && p.N <= 128));
     // the lean form addresses x, the group's weights and a tile's rows of y through 32-bit buffer offsets and has no K tail path
     const int var = glm_option(GLM_OPT_LARGEM_VARIANT);

@@ -1132,6 +1132,37 @@ def test_gemm_large_m_tile_lists(ops, M, N):
     assert torch.equal(*got) and bool((got[1][-1] == 7).all())
 
 
+@pytest.mark.parametrize("M,N", [(1100, 6144), (1280, 6144), (640, 12288), (2688, 3072), (520, 13000)])
+def test_gemm_large_m_one_round_of_128_rows(ops, M, N):
+    """128-row tiles that are one round of the chip, whose last band has positions beyond it: they are the ones taken (less time than 256-row tiles by far
+    more than any two runs differ), bit for bit like the plain form."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, 2048, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, 2048, device="cuda", generator=g) * 2048 ** -0.5).to(BF)
+
+    def us():   # replays of a graph: no host work between the launches
+        graph, best = torch.cuda.CUDAGraph(), 1e9
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                ops.linear_act(x, w)
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    got = ops.linear_act(x, w)
+    with largem_variant(0):
+        assert torch.equal(got, ops.linear_act(x, w))
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        taken = us()
+        with ops.option("largem_cfg", 2):
+            assert taken < 0.95 * us()
+
+
 @pytest.mark.parametrize("pitch,f32", [(1 << 21, False), ((1 << 25) - 8, False), ((1 << 25) - 8, True), (1 << 25, False), (1 << 25, True)])
 def test_gemm_large_m_wide_pitch(ops, pitch, f32):
     """Output rows up to 64 MiB (bf16) or 128 MiB (fp32) apart, the most that 16 rows of a store buffer may span, and one step more, where the plain form takes
