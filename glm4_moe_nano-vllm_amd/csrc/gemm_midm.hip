@@ -632,7 +632,7 @@ int launch_midm_shared(const GemmParams& p, hipStream_t st) {
 
 // The tile of a dense projection: the first of these with a workgroup per CU at most.  More and smaller workgroups put more of the chip to
 // work and have more bytes on their way; a larger tile pulls fewer, and two rounds of one cost more than one round of the next.  Split, 64 x 64,
-// 128 x 64, 128 x 128 (64 rows: 64 x 128), us, cold operands, * the one taken: 4096 x 4096 at 64 rows 16.5* / 21.2 / - / 30, at 211 24.5 / 20.5* /
+// 128 x 64, 128 x 128 (64 rows: 64 x 128), us, cold operands, * the one taken: 4096 x 4096 at 64 rows 16.5 / 21.2 / - / 30 (32 x 32, a round of which comes first, 13.5*), at 211 24.5 / 20.5* /
 // 30.0 / 36.2, at 512 47 / - / 31.8* / 40.2; 14336 x 4096 at 64 36.7 / 27.6* / - / 37.5, at 128 56 / 42.6 / 37.7* / 46.3, at 211 77 / 61.5 / 52 /
 // 43.0*; 2048 x 2048 at 1000 rows - / 16.9 / 17.2* / 19.8 (512 tiles of 64 x 64), at 2000 - / 35.2 / 25.9 / 23.7*; 32768 x 2048 at 64 42 / 30.1 / - / 27.6*.
 // A long K favours split waves at 64 x 64 too, which read each staged byte once: 4096 x 12288 at 211 rows 50 (shared 58), K = 8192 36 (40).
@@ -702,10 +702,11 @@ int launch_midm(const GemmParams& p, hipStream_t st) {
 }
 
 // K slices of a projection whose tiles are a quarter of the chip at most, and the tile for them: as many as bring a workgroup to every CU.  A
-// smaller tile with at least four slices goes before a larger one with more (fewer partial sums for the same workgroups).  One pass / slices, us:
-// 4096 x 12288 at 64 rows 45 / 23 (4 of 64 x 64), at 128 43 / 31 (4 of 128 x 64; 8 of 128 x 128 27), at 211 56 / 37 (4 of 128 x 128; the tiled
-// kernel's 16 38); 2048 x 8192 at 64 26 / 10, at 128 25 / 13 (the tiled kernel's 16 19), at 400 41 / 25 (28).  K = 2048: 8.1 / 6.7, which the
-// consumer's wider reads take back.
+// smaller tile with at least four slices goes before a larger one with more (fewer partial sums for the same workgroups).  With the norm that
+// adds them up, one pass / slices, us: 4096 x 12288 at 64 rows 38.8 / 28.3 (4 of 64 x 64), at 128 45.6 / 34.6 (4 of 128 x 64), at 211 52.9 / 43.2 (4 of 128 x
+// 128); 2048 x 8192 at 33 17.2 / 13.5, at 64 19.4 / 14.5, at 128 23.1 / 18.9, at 400 35.4 / 28.9; 2048 x 4096 at 33 11.8 / 10.3, at 64 12.8 / 11.3, at 128 15.0 /
+// 14.7, at 211 16.6 / 16.3; 4096 x 4096 at 64 17.2 / 15.4; least of all 1024 x 4096 at 128 12.0 / 12.2.  K = 2048: 7.1 / 6.7 without the norm, whose wider
+// reads take that back.
 int midm_slices(int64_t M, int N, int K, MidmTile* tile) {
     if (M <= 32 || K % 64 != 0 || K < 4096 || N % 4 != 0) return 1;
     if (M < 96 && (int64_t)N * K >= 1ll << 29) return 1;   // up to 95 rows slices have no other kernel, and this one's offsets (of padded rows) are 32-bit
@@ -750,21 +751,18 @@ bool glm_midm_takes(int mode, const GemmParams& p) {
     // (a loop of the tiled kernel that is asked for keeps its shapes)
     if (p.R >= 96 && (glm_option(GLM_OPT_LARGEM_VARIANT) >= 0 || glm_option(GLM_OPT_LARGEM_CFG) != 0)) return false;
     // Feed-forwards below 96 rows: the streaming kernel has configurations for them with a workgroup per 16 act columns or 32 columns and block of
-    // 32 rows, which cover the chip where these tiles of 64 rows leave half of it idle, or where K is a few chunks.  Streaming / here, us, cold
-    // operands: gate|up (K x columns of at least 4M) 1024 x 4096 at 48 rows 12.8 / 14.1, 2048 x 4096 at 64 13.7 / 16.8, 768 x 12288 at 64
-    // 32 / 41, but 768 x 4096 at 64 13.0 / 11.3, 2304 x 4096 at 64 23 / 18, 2048 x 8192 at 33 32 / 26; short ones 1536 x 512 at 48 4.4 / 4.8, 1024 x 1024 at 33 5.5 / 5.7,
-    // but 512 x 512 4.3 / 4.0, 2304 x 512 at 64 5.8 / 5.0.  Down (split over its waves from K = 4096 on) 1024 x 4096 at 48 8.3 / 10.5, 2048 x 6144
-    // at 64 12.8 / 23.1, 2048 x 12288 at 33 24.8 / 34.8, but 3072 x 4096 at 48 14.9 / 15.2, 2048 x 3072 at 64 17.2 / 9.7, 2048 x 4096 at 65
-    // 14.2 / 12.9; 2048 x 256 at 64 3.3 / 3.7, 4096 x 384 at 33 4.3 / 4.8, 2048 x 448 at 95 4.2 / 4.4, but 2048 x 512 5.3 / 4.7, 6144 x 384 at 64
-    // 5.4 / 5.0.
+    // 32 rows.  It is ahead where K is a few chunks, half of these tiles' time being the ends then, and in long down projections of four 16-row
+    // pieces, whose activations it brings in once for all columns of a workgroup.  Streaming / here, us, weights not in the caches: gate|up 1024 x 384 at 48 4.3 / 4.7,
+    // 1536 x 512 4.66 / 4.74, 2048 x 512 4.5 / 4.8, 1536 x 768 5.1 / 5.2, but 1024 x 896 5.8 / 5.2, 1024 x 1024 at 33 5.8 / 5.3, 1024 x 4096 at 48 13.0 /
+    // 11.2, at 64 13.1 / 12.3, 2048 x 2048 at 48 8.2 / 8.0, at 64 8.4 / 8.5, 768 x 12288 at 64 32.8 / 29.3, 2048 x 16384 at 41 74 / 48.  Down 2048 x 256 at 64
+    // 3.5 / 3.8, 4096 x 384 at 33 4.6 / 4.8, 2048 x 448 at 48 4.6 / 4.8, but 2048 x 512 at 64 5.3 / 4.7; 1024 x 4096 at 40 8.7 / 7.9, at 48 8.4 / 8.4, at 52
+    // 8.3 / 8.7, at 64 8.9 / 9.4; 2048 x 6144 at 48 12.7 / 12.3, at 52 12.3 / 12.2, at 56 12.2 / 12.6, at 64 12.6 / 13.3; 2048 x 12288 at 48 24.4 / 21.3, at
+    // 52 22.7 / 21.4, at 56 22.3 / 22.2, at 64 22.1 / 23.5, but 2304 x 5120 at 56 18.6 / 14.6, 64 x 4096 at 64 8.9 / 8.6, 2048 x 3072 at 64 17.2 / 9.7.
     if (p.R < 96 && mode != GEMM_PLAIN) {
         const int64_t n = (p.R + 31) / 32 * p.N;
         if (mode == GEMM_DOWN) {
-            if (p.K < 512 ? n <= 8192 : p.K >= 4096 && p.R <= 64 && p.N <= 2560 && p.R * p.N <= 131072) return false;
-        } else {
-            if (p.K > 320 && p.K <= 1024 && p.N >= 1024 && n <= 4096) return false;
-            if (p.R <= 64 && p.N <= 2048 && (int64_t)p.N * p.K >= 4 << 20 && (p.R > 40 || p.K < 8192)) return false;
-        }
+            if (p.K < 512 ? n <= 8192 : p.K >= 4096 && p.R > 48 && p.R <= 64 && p.N >= 128 && p.N <= 2048) return false;
+        } else if (p.K > 320 && p.K <= 768 && p.N >= 1024 && n <= 4096) return false;
     }
     const int64_t wrows = gemm_paired(mode) ? 2 * (int64_t)p.N : (int64_t)p.N;
     if (p.R * p.ldx * 2 >= (1ll << 31) || wrows * p.ldw * 2 >= (1ll << 31)) return false;   // 32-bit offsets
