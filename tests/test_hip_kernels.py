@@ -1096,24 +1096,60 @@ def test_gemm_large_m_several_tiles_per_workgroup(ops, K, counts):
     assert_close_bf16(got[0][rows].cpu(), a_ref, 3, 0.06, atol=1e-3, what=f"act K={K} group {e}")
 
 
-@pytest.mark.parametrize("M,N,K", [(8518, 2056, 512), (8448, 2048, 576), (33000, 520, 512), (8705, 2048, 512)])
+def assert_cut(rows, column_tiles):
+    """The tiles of 256 rows behind whole rounds of the chip are half a round at most, and there are some: the launch cuts them in two."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    tiles = -(-rows // 256) * column_tiles
+    assert tiles > cus and 0 < 2 * (tiles % cus) <= cus
+
+
+# the last row block: 70 rows, whole, exactly the first half, into the second half, one row
+LAST_BLOCKS = [8518, 8448, 8576, 8648, 8705]
+
+
+@pytest.mark.parametrize("M", LAST_BLOCKS)
+@pytest.mark.parametrize("N,K", [(2064, 512), (2048, 576)])
 def test_gemm_large_m_last_round_in_halves(ops, M, N, K):
-    """More tiles than CUs and at most half a round behind whole ones: those go in halves.  Row blocks that end in the first half and at its end, columns that
-    end inside a tile; bit for bit against the plain form."""
+    """More tiles than CUs and at most half a round behind whole ones: those go in halves.  Row blocks that end inside either half and at their ends, columns
+    that end inside a tile; bit for bit against the plain form."""
     g = torch.Generator(device="cuda").manual_seed(K)
     x = torch.randn(M, K, device="cuda", generator=g).to(BF)
     w = (torch.randn(2 * N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
     b = torch.randn(N, device="cuda", generator=g).to(BF)
+    for tiles in (-(-N // 256), -(-(N // 2) // 128), -(-N // 128)):   # single, N / 2 gated columns, N gated columns
+        assert_cut(M, tiles)
     got = []
     for v in (0, -1):
         with largem_variant(v):
             out = torch.full((M + 1, N), 7.0, device="cuda", dtype=BF)
             ops.linear_act(x, w[:N], b, out=out[:M])
             got.append((out, ops.linear_act(x, w[:N], act=(ops.ACT_GATE, 264.0, 0.0)), ops.linear_act(x, w[:N], out_f32=True),
-                        ops.gated_glu(x, w[: 2 * (N // 2)], 2.0), ops.grouped_gemm_gateup_silu(x, w.unsqueeze(0), None, None, M)))
+                        ops.linear_act(x, w[:N], act=(ops.ACT_SILU_GATE, 264.0, 0.0), out_f32=True),
+                        ops.gated_glu(x, w[:N], 2.0), ops.grouped_gemm_gateup_silu(x, w.unsqueeze(0), None, None, M)))
     for a, c in zip(*got):
         assert torch.equal(a, c)
     assert bool((got[1][0][-1] == 7).all())
+
+
+@pytest.mark.parametrize("M", LAST_BLOCKS)
+def test_expanded_fp8_weights_last_round_in_halves(ops, M):
+    """One expert whose fp8 weights are expanded, row scales on the accumulators: its last tiles go in halves too."""
+    I, H = 2064, 512
+    assert_cut(M, -(-I // 128))
+    assert_cut(M, -(-I // 256))
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, act = (torch.randn(M, H, device="cuda", generator=g).to(BF) for _ in range(2))
+    q13, s13 = ops.quantize_fp8_rowwise(torch.randn(1, 2 * I, H, device="cuda", generator=g) * H ** -0.5)
+    q2, s2 = ops.quantize_fp8_rowwise(torch.randn(1, I, H, device="cuda", generator=g) * H ** -0.5)
+    scale = (torch.rand(M, device="cuda", generator=g) + 0.1).to(BF)
+    got = []
+    with ops.option("fp8w_native", 0):
+        for v in (0, -1):
+            with largem_variant(v):
+                got.append((ops.grouped_gemm_gateup_silu_fp8w(x, q13, s13, None, None, M), ops.grouped_gemm_down_fp8w(act, q2, s2, None, scale, 1),
+                            ops.grouped_gemm_down_fp8w(act, q2, s2, None, None, 0)))
+    for a, c in zip(*got):
+        assert torch.equal(a, c)
 
 
 @pytest.mark.parametrize("M,N", [(15074, 2048), (8704, 3072), (8248, 7944), (8448, 7936), (512, 32768), (300, 40000)])
@@ -1211,10 +1247,11 @@ def test_fp8_expert_down_wide_pitch(ops, pitch):
         assert bool((buf[:, H] == 7).all()) and bool((buf[0, :H] == 7).all()) and bool((buf[-1, :H] == 7).all()), what
 
 
-@pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (16700, 4, 2, 512)])
+@pytest.mark.parametrize("T,nh,nkv,K", [(8518, 12, 2, 512), (8576, 12, 2, 512), (8648, 12, 2, 576), (8705, 12, 2, 512), (16700, 4, 2, 512)])
 def test_qkv_gemm_with_rope_store_last_round_in_halves(ops, T, nh, nkv, K):
     """The fused QKV projection with its last tiles in halves == the projection, also cut, and the split / rotary kernel, bit for bit."""
     N = (nh + 2 * nkv) * 128
+    assert_cut(T, N // 256)
     g = torch.Generator(device="cuda").manual_seed(T)
     x = torch.randn(T, K, device="cuda", generator=g).to(BF)
     w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
