@@ -16,19 +16,21 @@
 //     ordered in bands of 4 row blocks x all n-tiles (n-tile major): the workgroups co-resident on an XCD form a supertile whose
 //     operand panels are shared through that XCD's L2.
 //
-// What bounds it: power.  With zeros as operands the same launches run 1.25 to 1.35 times as fast (16384 x 8192 x 8192: 1930 TFLOP/s
-// against 1440; 1955 against 1526 with the present epilogue), so what counts is both cycles and switching.  Cycles: the ring of the 256-row tiles (CfgR) holds FIVE 32-KiB operand
+// What bounds it: power, in the products for the most part, and the traffic that feeds them.  On normal values the products alone, from registers, reach 2070
+// TFLOP/s, this kernel without its DMA 1813, with operands in L2 1629, as it is 1526 (16384 x 8192 x 8192); on zeros it runs 1.25 to 1.35 times as
+// fast, so what counts is both cycles and switching.  Cycles: the ring of the 256-row tiles (CfgR) holds FIVE 32-KiB operand
 // tiles (W and X of two K tiles and the next W) in all 160 KiB of LDS, in the order they are needed; an operand's slot is refilled as
 // soon as its own last fragment read has retired, so a piece has one to one and a half K tiles to arrive (two 64-KiB buffers: half to
 // one, which a loaded memory side does not make), and a phase is 32 MFMAs between two barriers instead of 16 (fp8 x fp8: 16 of four
 // times the work).  Switching: consecutive MFMAs share one operand (rows of tiles in alternating direction).  Both together, TFLOP/s
-// on normal values, one process, all bit-identical:
+// on normal values, all bit-identical, four steps in one process and the last again with the next in one on another card:
 //                               16384 x 8192 x 8192   15074 x 14336 x 4096   15074 x 4096 x 12288   15074 x 6144 x 2048   x 2048 x 6144
 //   two buffers, 16 per phase          1363                  1264                   1247                   1204                 1311
 //   ... 32 per phase                   1371                  1326                   1282                   1253                 1340
 //   ring of five, 32 per phase         1407                  1329                   1315                   1245                 1344
 //   ... alternating direction          1439                  1333                   1350                   1257                 1362
-//   ... decisions and stores by wave   1560                  1467                   1456                   1372                 1501   (another card)
+//   the same, the other card           1537                  1425                   1440                   1310                 1449
+//   ... decisions and stores by wave   1546                  1496                   1447                   1322                 1462
 // (Also measured: one barrier per K tile and fragments read a quarter of a tile ahead into 96 registers, 1187 to 1266; wave
 // priority in the MFMA interval, equal; K slices of the fragments outermost or tiles of the other operand outermost, equal; 2, 3, 6
 // or 8 row blocks per band, up to 7 % slower.)  A tile's stores cost 2 % (K = 8192) to 6 % (K = 2048): all CUs reach them together.
