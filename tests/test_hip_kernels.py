@@ -1199,6 +1199,25 @@ def test_gemm_large_m_one_round_of_128_rows(ops, M, N):
             assert taken < 0.95 * us()
 
 
+@pytest.mark.parametrize("M,N,K", [(1083, 40, 552), (1404, 148, 1032), (664, 1172, 1640), (9000, 2052, 200), (8500, 1036, 64)])
+def test_gemm_large_m_plain_form_bias(ops, M, N, K):
+    """The plain form (K or columns that the other does not take) with a bias: the fp32 sum that the same call without one stores, plus the bias, one rounding.
+    Bit for bit, over several tiles per workgroup and columns that end inside a tile; nothing behind a row's columns."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    b = torch.randn(N, device="cuda", generator=g).to(BF)
+    b[::7] = 300
+    want = ops.linear_act(x, w, out_f32=True) + b.float()
+    for f32 in (False, True):
+        out = torch.full((M + 1, N + 4), 7.0, device="cuda", dtype=torch.float32 if f32 else BF)
+        ops.linear_act(x, w, b, out_f32=f32, out=out[:M, :N])
+        assert torch.equal(out[:M, :N], want if f32 else want.to(BF))
+        assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+    cap = ops.linear_act(x, w, b, act=(ops.ACT_SOFTCAP, 2.0, 0.0), out_f32=True)
+    assert ((cap.double() - 2 * torch.tanh(want.double() / 2)).abs() <= 2.0 ** -20).all()
+
+
 @pytest.mark.parametrize("pitch,f32", [(1 << 21, False), ((1 << 25) - 8, False), ((1 << 25) - 8, True), (1 << 25, False), (1 << 25, True)])
 def test_gemm_large_m_wide_pitch(ops, pitch, f32):
     """Output rows up to 64 MiB (bf16) or 128 MiB (fp32) apart, the most that 16 rows of a store buffer may span, and one step more, where the plain form takes
