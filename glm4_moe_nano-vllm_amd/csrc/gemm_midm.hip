@@ -662,16 +662,21 @@ MidmTile midm_tile_of(int mode, const GemmParams& p) {
     return fits(128, 128) ? MM_128 : MM_NONE;
 }
 
-// Weights that only one row block reads go past the caches, which they leave to the activations (nt).  Kept / past them, us, weights not in the caches:
-// 128 rows of 32768 x 2048 33.1 / 31.5, gated 30.7 / 28.8, 64 of 14336 x 4096 29.6 / 27.7, 41 of 8928 x 576 6.5 / 6.0; steps: 64 GLM sequences over fp8
-// experts 2156 / 2139, 100 Gulozen ones 1123 / 1116.  With two row blocks and more, and in the split tiles, single projections gained as much and
-// steps lost it again (a prompt of 211 1.886 / 1.904 ms).  A kernel of its own: chosen inside the loop, for every DMA instruction, it cost all others 1 to
-// 5 % (gate|up 965 of 456 x 6912 32.9 / 31.3, 300 of 1024 x 2048 12.1 / 11.7, plain 300 of 2048 x 2048 12.6 / 12.4).
+// Weights that only one row block reads go past the caches, which they leave to the activations (nt), from 64 MiB on.  Kept / past them, us, weights not in
+// the caches: 128 rows of 32768 x 2048 33.1 / 31.5, 64 of 14336 x 4096 32.0 / 29.4, gated 49.9 / 47.2; steps: 64 GLM sequences over fp8 experts 2149 / 2131, 128
+// Dafolorn ones 469.7 / 462.0, 100 Gulozen ones 1146 / 1142.  Weights that are still in the 256 MiB behind the L2 from the last time are read from HBM
+// all the same (64 of 14336 x 4096 21.8 / 29.1, 128 of 12288 x 2048, gated, 14.7 / 17.2), so a layer whose matrices may all lie there is spared: what
+// matrices below the line gain by themselves (41 of 8928 x 576 6.5 / 6.0) steps do not show (Dafolorn with it on those too 465.7, Gulozen 1147).  With two row blocks and more, and in the split tiles,
+// single projections gained as much and steps lost it again (a prompt of 211 1.886 / 1.904 ms).  A kernel of its own: chosen inside the loop, for every DMA
+// instruction, it cost all others 1 to 5 % (gate|up 965 of 456 x 6912 32.9 / 31.3, 300 of 1024 x 2048 12.1 / 11.7, plain 300 of 2048 x 2048 12.6 / 12.4).
+constexpr int64_t MM_NT_BYTES = 64 << 20;
+
 template <int MODE>
 int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
     if constexpr (MODE == GEMM_PLAIN) {   // half a head in the QKV epilogue of 32 rows; the sums are the same in all three
         if (p.qkv_q != nullptr && (tile == MM_SPLIT16 || tile == MM_SPLIT32x32)) return launch_midm_cfg<MODE, 2, 4, 8, 1>(p, st);
     }
+    const bool nt = (gemm_paired(MODE) ? 2 : 1) * (int64_t)p.N * p.ldw * 2 >= MM_NT_BYTES;
     switch (tile) {
         case MM_SPLIT16:
             if constexpr (!gemm_paired(MODE)) return launch_midm_cfg<MODE, 2, 1, 8, 2>(p, st);
@@ -681,11 +686,10 @@ int launch_midm_tile(MidmTile tile, const GemmParams& p, hipStream_t st) {
             if (MODE != GEMM_PLAIN || p.qkv_q == nullptr) return launch_midm_cfg<MODE, 4, 2, 4, 2>(p, st);
             [[fallthrough]];
         case MM_SPLIT64: return launch_midm_cfg<MODE, 4, 4, 4, 2>(p, st);
-        // (true: nt, see above; no more than 64 rows take MM_64x128)
-        case MM_64: return p.R <= 64 ? launch_midm_shared<MODE, 2, 2, 2, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 2, 2, 2, 4, false>(p, st);
-        case MM_128x64: return p.R <= 128 ? launch_midm_shared<MODE, 2, 2, 4, 2, 3, true>(p, st) : launch_midm_shared<MODE, 2, 2, 4, 2, 3, false>(p, st);
-        case MM_64x128: return launch_midm_shared<MODE, 2, 4, 2, 2, 3, true>(p, st);
-        case MM_128: return p.R <= 128 ? launch_midm_shared<MODE, 2, 4, 4, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 4, 4, 2, 4, false>(p, st);
+        case MM_64: return nt && p.R <= 64 ? launch_midm_shared<MODE, 2, 2, 2, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 2, 2, 2, 4, false>(p, st);
+        case MM_128x64: return nt && p.R <= 128 ? launch_midm_shared<MODE, 2, 2, 4, 2, 3, true>(p, st) : launch_midm_shared<MODE, 2, 2, 4, 2, 3, false>(p, st);
+        case MM_64x128: return nt && p.R <= 64 ? launch_midm_shared<MODE, 2, 4, 2, 2, 3, true>(p, st) : launch_midm_shared<MODE, 2, 4, 2, 2, 3, false>(p, st);
+        case MM_128: return nt && p.R <= 128 ? launch_midm_shared<MODE, 2, 4, 4, 2, 4, true>(p, st) : launch_midm_shared<MODE, 2, 4, 4, 2, 4, false>(p, st);
         default: break;
     }
     GLM_CHECK_ARG(false, GLM_ERR_UNSUPPORTED, "gemm_midm: no tile for %ld rows, N=%d", (long)p.R, p.N);

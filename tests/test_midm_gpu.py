@@ -407,8 +407,8 @@ def test_few_columns_row_block_by_row_block(M, N, K, f32):
 
 
 @pytest.mark.parametrize("K,N,rows", [(320, 12288, (64, 128, 256)), (576, 8192, (128, 256)), (192, 24576, (64, 128))])
-def test_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
-    """Shared tiles whose weights go past the caches (all rows in one block) and the others of the same columns: every sum in the order of K, so a row
+def test_shared_tiles_of_one_row_block(ops, K, N, rows):
+    """Shared tiles with all rows in one block and the others of the same columns: every sum in the order of K, so a row
     is bit for bit the same whatever stands behind it."""
     x, w = rnd(max(rows), K, seed=61).cuda(), rnd(N, K, seed=62, scale=K ** -0.5).cuda()
     got = [(ops.linear_act(x[:M], w), ops.gated_glu(x[:M], w, 2.0), ops.grouped_gemm_gateup_silu(x[:M], w.unsqueeze(0), None, None, M)) for M in rows]
@@ -416,6 +416,19 @@ def test_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
     for y in got[:-1]:
         for a, b in zip(y, got[-1]):
             assert torch.equal(a, b[: a.shape[0]])
+
+
+@pytest.mark.parametrize("K,N,rows", [(2048, 16384, (41, 64, 100, 128)), (1088, 32768, (64, 128))])
+def test_large_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
+    """64 MiB of weights and more, which go past the caches where one block holds all rows, in every shared tile: bit for bit the same columns of fewer weights."""
+    x, w = rnd(max(rows), K, seed=63).cuda(), rnd(N, K, seed=64, scale=K ** -0.5).cuda()
+    n = N // 4 * 3               # (below the line, and still no round of the tiles whose K is split over the waves)
+    few = torch.cat([w[: n // 2], w[N // 2: N // 2 + n // 2]])
+    for M in rows:
+        for _ in range(2):   # (the second time they are where the first left them)
+            assert torch.equal(ops.linear_act(x[:M], w)[:, :n], ops.linear_act(x[:M], w[:n]))
+            assert torch.equal(ops.gated_glu(x[:M], w, 2.0)[:, : n // 2], ops.gated_glu(x[:M], few, 2.0))
+    close(ops.linear_act(x, w)[:, -64:], x.cpu().double() @ w[-64:].cpu().double().T, "plain")
 
 
 def act64(kind, a, b, z, ops):
