@@ -431,6 +431,25 @@ def test_large_weights_of_one_row_block_past_the_caches(ops, K, N, rows):
     close(ops.linear_act(x, w)[:, -64:], x.cpu().double() @ w[-64:].cpu().double().T, "plain")
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 2720, 512), (96, 2692, 576), (190, 2640, 1088), (330, 5300, 192), (161, 4168, 128), (350, 1352, 512)])
+def test_column_tiles_whose_last_turn_is_not_every_xcds(ops, M, N, K):
+    """A round of tiles that is more than one where every XCD counts as many column tiles as the first: they go in runs.  Every row and column, single and gated."""
+    x, w, s = rnd(M, K, seed=81).cuda(), rnd(2 * N, K, seed=82, scale=K ** -0.5).cuda(), rnd(M, seed=83).cuda()
+    z = x.cpu().double() @ w.cpu().double().T
+    out = torch.full((M + 1, N + 4), 7.0, device="cuda", dtype=BF)
+    ops.linear_act(x, w[:N], out=out[:M, :N])
+    close(out[:M, :N].cpu(), z[:, :N], "plain")
+    assert bool((out[M] == 7).all()) and bool((out[:, N:] == 7).all())
+    close(ops.linear_act(x, w[:N], out_f32=True).cpu(), z[:, :N], "fp32")
+    for n in (N, N // 8 * 4):
+        g, u = z[:, :n], z[:, n: 2 * n]
+        got = ops.grouped_gemm_gateup_silu(x, w[: 2 * n].unsqueeze(0), None, None, M).cpu()
+        ref = (torch.nn.functional.silu(g.to(BF).double()).to(BF).double() * u.to(BF).double()).to(BF)
+        assert_close_bf16(got, ref, SILU[0], SILU[1], atol=SILU[2], what=f"gate|up {n}")
+    got = ops.grouped_gemm_down(x, w[:N].unsqueeze(0), None, s, 1).cpu()
+    assert_close_bf16(got, (z[:, :N].to(BF).double() * s.cpu().double()[:, None]).to(BF), 2, 0.05, atol=2 ** -8, what="down")
+
+
 def act64(kind, a, b, z, ops):
     n = torch.arange(z.shape[1])
     if kind == ops.ACT_SOFTCAP:
