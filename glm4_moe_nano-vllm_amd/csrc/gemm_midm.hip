@@ -714,10 +714,10 @@ int launch_midm(const GemmParams& p, hipStream_t st) {
 
 // K slices of a projection whose tiles are a quarter of the chip at most, and the tile for them: as many as bring a workgroup to every CU.  A
 // smaller tile with at least four slices goes before a larger one with more (fewer partial sums for the same workgroups).  With the norm that
-// adds them up, one pass / slices, us: 4096 x 12288 at 64 rows 38.8 / 28.3 (4 of 64 x 64), at 128 45.6 / 34.6 (4 of 128 x 64), at 211 52.9 / 43.2 (4 of 128 x
-// 128); 2048 x 8192 at 33 17.2 / 13.5, at 64 19.4 / 14.5, at 128 23.1 / 18.9, at 400 35.4 / 28.9; 2048 x 4096 at 33 11.8 / 10.3, at 64 12.8 / 11.3, at 128 15.0 /
-// 14.7, at 211 16.6 / 16.3; 4096 x 4096 at 64 17.2 / 15.4; least of all 1024 x 4096 at 128 12.0 / 12.2.  K = 2048: 7.1 / 6.7 without the norm, whose wider
-// reads take that back.
+// adds them up, one pass / slices, us, cold weights: 4096 x 12288 at 64 rows 36.9 / 27.5 (4 of 64 x 64), at 128 46.1 / 35.3 (4 of 128 x 64), at 211 54.5 / 43.5 (4 of
+// 128 x 128); 2048 x 8192 at 33 17.5 / 13.6, at 64 19.1 / 14.7, at 128 22.3 / 17.5, at 400 33.8 / 29.5; 2048 x 4096 at 33 11.5 / 11.0, at 64 12.6 / 11.8, at 211 16.7 /
+// 16.2; 4096 x 4096 at 64 17.8 / 16.1; 1024 x 4096 at 64 12.0 / 10.4; least of all K = 4096 at 128 rows: 2048 columns 14.7 / 15.2, 1024 12.1 / 12.7.  K = 2048: 7.1 /
+// 6.7 without the norm, whose wider reads take that back.
 int midm_slices(int64_t M, int N, int K, MidmTile* tile) {
     if (M <= 32 || K % 64 != 0 || K < 4096 || N % 4 != 0) return 1;
     if (M < 96 && (int64_t)N * K >= 1ll << 29) return 1;   // up to 95 rows slices have no other kernel, and this one's offsets (of padded rows) are 32-bit
