@@ -1152,6 +1152,39 @@ def test_expanded_fp8_weights_last_round_in_halves(ops, M):
         assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("counts", [[256 * 5 + 1, 0, 256 * 9 + 128, 300, 256 * 12 + 129, 1, 1000, 256, 0, 90],     # 40 row blocks: 320 tiles, 64 in halves
+                                    [200] * 33, [129] * 40 + [4] * 7, [1] * 20 + [256 * 14]])
+def test_gemm_large_m_groups_last_round_in_halves(ops, counts):
+    """Groups whose last tiles go in halves, and lists whose row blocks are far fewer than rows and groups could make: bit for bit against the plain form, which cuts
+    nothing, and every row against products in 32 bits.  Rows behind the last group stay as they were."""
+    K, I, N2, spare = 512, 1024, 2048, 700
+    E, R, T = len(counts), sum(counts), 400
+    tiles = sum(-(-c // 256) for c in counts) * 8
+    cus = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    assert tiles > cus and 0 < 2 * (tiles % cus) <= cus or tiles <= cus
+    g = torch.Generator(device="cuda").manual_seed(E)
+    offs = dev(torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32))
+    tok = torch.randint(0, T, (R + spare,), device="cuda", generator=g, dtype=torch.int32)
+    x, act = torch.randn(T, K, device="cuda", generator=g).to(BF), torch.randn(R, K, device="cuda", generator=g).to(BF)
+    w13, w2 = (torch.randn(E, n, K, device="cuda", generator=g).mul_(K ** -0.5).to(BF) for n in (2 * I, N2))
+    scale = (torch.rand(R, device="cuda", generator=g) + 0.1).to(BF)
+    got = []
+    for v in (0, -1):
+        with largem_variant(v), ops.option("largem_cfg", 2):
+            got.append((ops.grouped_gemm_gateup_silu(x, w13, offs, tok, R + spare)[:R], ops.grouped_gemm_down(act, w2, offs, scale, E - 1)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    lo = 0
+    for e, n in enumerate(counts):
+        rows = slice(lo, lo + n)
+        lo += n
+        gate, up = (x[tok[rows].long()].float() @ w13[e].float().T).chunk(2, -1)
+        y = act[rows].float() @ w2[e].float().T * (scale[rows, None].float() if e < E - 1 else 1.0)
+        # a rounding to bf16 (7 bits behind the first) is up to 2^-8 of the value.  silu(g) u: of up, of silu(g), of the product, and of g, which silu enlarges by its condition number
+        # g silu'(g) / silu(g) = 1 + g sigmoid(-g) <= 1 + |g|.  Down: of the sum and of its product with the scale.  Sums of 512 products of fp32 in another order: some 1e-6.
+        for a, b, r in ((got[1][0][rows], torch.nn.functional.silu(gate) * up, 4 + gate.abs()), (got[1][1][rows], y, 2)):
+            assert bool(((a.float() - b).abs() <= 1.01 * r * 2.0 ** -8 * b.abs() + 2e-5).all())
+
+
 @pytest.mark.parametrize("M,N", [(15074, 2048), (8704, 3072), (8248, 7944), (8448, 7936), (512, 32768), (300, 40000)])
 def test_gemm_large_m_tile_lists(ops, M, N):
     """Lists of more than one round whose last band has fewer row blocks, with the positions behind it (no round more) and without them (a round more),
