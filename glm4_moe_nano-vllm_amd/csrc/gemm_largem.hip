@@ -44,6 +44,8 @@ constexpr int LM_BN = 256;    // weight rows per tile (MFMA row axis); 4 waves x
 constexpr int LM_BAND_ROWS = 4;  // row blocks per L2 supertile band
 constexpr int LM_CUT_K = 512;    // shortest reduction whose last tiles are cut
 constexpr int LM_SLOT = 32768;   // CfgR: bytes of a ring slot, one operand tile
+constexpr int LM_THROUGH_K = 2048;   // longest reduction whose output is written through the L2
+constexpr int LM_SC1 = 16;           // cache policy bit of a store: device scope
 constexpr int64_t LM_WIDE = 1 << 25;   // output pitch from which 16 fp32 rows do not fit into a buffer
 
 // Tile configurations (the kernel is written once over these):
@@ -982,6 +984,16 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                                                          0x00020000);
             };
             const unsigned lrow = (unsigned)c * pitch;
+            // Of short reductions (much output for its time) whole cache lines are written through the L2: what stays dirty there is written out when a tile of operands needs
+            // the place and, 32 MiB of it, at the launch's end.  Kept dirty / through, us, in a step: 15074 x 4096 x 256 52.2 / 47.4, x 2048 x 2048 98.0 / 95.4,
+            // x 6144 x 2048 (xIELU) 320 / 315, 11137 x 4096 x 2048 gated 279 / 274, and attention behind such a launch 582 / 570, 173 / 170.  K of 4096 and more loses
+            // 0 to 1 %, experts 2 to 3 %, and rows that start inside a line 12 % (15074 x 9232 x 2048 419 / 470).  By itself, 2000 to 15074 rows of 2048 to 10240 columns:
+            // K of 256 and 512 1.00 to 1.18 times as fast (3700 x 2048 x 512 12.8 / 10.8), of 2048 0.99 to 1.06.
+            const bool through = !GROUPED && K <= LM_THROUGH_K && ((pitch | (unsigned)(F32 ? (uintptr_t)p.yf : (uintptr_t)p.y)) & 127u) == 0;
+            auto put = [&](const u32x4_t v, const __amdgpu_buffer_rsrc_t yrs, unsigned at) __attribute__((always_inline)) {
+                if (through) __builtin_amdgcn_raw_buffer_store_b128(v, yrs, at, 0, LM_SC1);
+                else __builtin_amdgcn_raw_buffer_store_b128(v, yrs, at, 0, 0);
+            };
             // stores f of every element
             auto finish = [&](auto&& f) __attribute__((always_inline)) {
                 if constexpr (F32) {   // four columns per store
@@ -994,7 +1006,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                             f32x4_t o;
 #pragma unroll
                             for (int r = 0; r < 4; ++r) o[r] = f(t, mt, r);
-                            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), yrs, ncol_w + n < p.N ? lrow + n * 4 : BEYOND, 0, 0);
+                            put(__builtin_bit_cast(u32x4_t, o), yrs, ncol_w + n < p.N ? lrow + n * 4 : BEYOND);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
@@ -1013,7 +1025,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         const u32x4_t o = {a[0], b[0], a[1], b[1]};
                         if constexpr (C::WIDE) {
                             if (16 * mt + c < left && ncol_w + n < p.N) *reinterpret_cast<u32x4_t*>(p.y + first + (16 * mt + c) * p.ldy + n) = o;
-                        } else __builtin_amdgcn_raw_buffer_store_b128(o, yrs, ncol_w + n < p.N ? lrow + n * 2 : BEYOND, 0, 0);
+                        } else put(o, yrs, ncol_w + n < p.N ? lrow + n * 2 : BEYOND);
                     }
                     __builtin_amdgcn_sched_barrier(0);   // (the other rows' values would take registers that are not there)
                 }
