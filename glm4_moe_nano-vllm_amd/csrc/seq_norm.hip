@@ -50,13 +50,17 @@ struct SeqNormArgs {
 
 constexpr int SN_NT = 256;
 
-__device__ __forceinline__ f32x4_t sn_load_y(const SeqNormArgs& a, int64_t row, int col) {
+// y, or the first slab of it
+__device__ __forceinline__ f32x4_t sn_load_y1(const SeqNormArgs& a, int64_t row, int col) {
     if (!a.y_f32) {
         const u32x2_t u = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const bf16_t*>(a.y) + row * a.ldy + col);
         return f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
     }
+    return *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.y) + row * a.ldy + col);
+}
+__device__ __forceinline__ f32x4_t sn_load_y(const SeqNormArgs& a, int64_t row, int col) {
+    f32x4_t v = sn_load_y1(a, row, col);
     const float* p = reinterpret_cast<const float*>(a.y) + row * a.ldy + col;
-    f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
     for (int s = 1; s < a.n_slabs; ++s) v += *reinterpret_cast<const f32x4_t*>(p + s * a.slab_stride);
     return v;
 }
@@ -247,55 +251,86 @@ __device__ __forceinline__ void sn_st8(void* base, int64_t off, int f32, const R
 }
 __device__ __forceinline__ float sn_sumsq8(const Row8& v) { return sn_sumsq(v.a) + sn_sumsq(v.b); }
 
-template <int TAPS, int NT>
+// Tables that no launch changes while it reads them: through the scalar cache, so that a row's bookkeeping waits for no vector load or store
+__device__ __forceinline__ int sn_table(const int32_t* p, int64_t i) { return reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p))[i]; }
+// `bytes` of a row; nothing if there is no such buffer
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sn_row(const void* base, int64_t off, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base) + off), 0, base ? bytes : 0, 0x00020000);
+}
+__device__ __forceinline__ void sn_put8f(__amdgpu_buffer_rsrc_t rs, int at, const Row8& v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v.a), rs, at, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v.b), rs, at, 16, 0);
+}
+__device__ __forceinline__ u32x4_t sn_pack8(const Row8& v) {
+    return u32x4_t{pack2bf(v.a[0], v.a[1]), pack2bf(v.a[2], v.a[3]), pack2bf(v.b[0], v.b[1]), pack2bf(v.b[2], v.b[3])};
+}
+__device__ __forceinline__ Row8 sn_unpack8(const u32x4_t& u) {
+    return {f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])}, f32x4_t{bflo(u[2]), bfhi(u[2]), bflo(u[3]), bfhi(u[3])}};
+}
+
+// sn_load_y with four slabs in flight
+__device__ __forceinline__ f32x4_t sn_load_slabs(const SeqNormArgs& a, int64_t row, int col) {
+    f32x4_t v = sn_load_y1(a, row, col);
+    const float* p = reinterpret_cast<const float*>(a.y) + row * a.ldy + col;
+    for (int s = 1; s < a.n_slabs; s += 4) {
+        f32x4_t t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] = *reinterpret_cast<const f32x4_t*>(p + min(s + j, a.n_slabs - 1) * a.slab_stride);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (s + j < a.n_slabs) v += t[j];
+    }
+    return v;
+}
+
+// ANY: y or the activations may be fp32 (y in slabs: then it is summed up where it is requested)
+template <int TAPS, int NT, bool ANY>
 __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm_stream_kernel(const SeqNormArgs a, int tr) {
     constexpr int HALO = TAPS - 1, NW = NT / 64;
     __shared__ float s_red[2][2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int c = tid * 8;
+    const int c = tid * 8, cl = min(c, a.wp - 8);   // cl: what a thread behind the row's end reads instead
     const bool on = c < a.wp;
     const int64_t r0 = (int64_t)blockIdx.x * tr, r1 = min(r0 + tr, a.T);
     const float inv_w = 1.0f / (float)a.width;
-    int s = 0, qs = 0, qe = 0;
+    int s = 0, qs = 0, qe = 0, sin = 0, so = 0;
+    auto sequence = [&](int64_t r) {
+        s = sn_table(a.seq_of, r);
+        qs = sn_table(a.q_start, s);
+        qe = sn_table(a.q_start, s + 1);
+        sin = (int)min(max((int64_t)sn_table(a.state_in, s), (int64_t)0), a.n_state - 1);
+        so = sn_table(a.state_out, s);
+    };
     int64_t lo = r0;
     if constexpr (TAPS > 1) {
-        s = a.seq_of[r0];
-        qs = a.q_start[s];
-        qe = a.q_start[s + 1];
+        sequence(r0);
         lo = max(r0 - HALO, (int64_t)qs);
     }
     const Row8 zero = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     Row8 gq = zero, gp = zero, hist[TAPS];
     u32x4_t w[TAPS];  // eight taps packed
-    if (on) {
-        if (a.y) gq = sn_ld8f(a.g_post + c);
-        if (a.g_pre) gp = sn_ld8f(a.g_pre + c);
-        if constexpr (TAPS > 1) {
+    if (a.y) gq = sn_ld8f(a.g_post + cl);
+    if (a.g_pre) gp = sn_ld8f(a.g_pre + cl);
+    if constexpr (TAPS > 1) {
 #pragma unroll
-            for (int j = 0; j < TAPS; ++j) w[j] = *reinterpret_cast<const u32x4_t*>(a.conv_w + (int64_t)j * a.wp + c);
-        }
-    }
-    if (TAPS > 1 && !on) {
-#pragma unroll
-        for (int j = 0; j < TAPS; ++j) w[j] = u32x4_t{0, 0, 0, 0};
+        for (int j = 0; j < TAPS; ++j) w[j] = *reinterpret_cast<const u32x4_t*>(a.conv_w + (int64_t)j * a.wp + cl);
     }
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) hist[j] = zero;
     auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
-    auto load_row = [&](int64_t r, Row8& x, Row8& y) {
-        if (!on) return;
-        const int64_t row = a.row_index ? a.row_index[r] : r;
-        x = sn_ld8f(a.x_in + row * a.ldx + c);
-        if (!a.y) return;
-        if (!a.y_f32) {
-            const u32x4_t u = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const bf16_t*>(a.y) + row * a.ldy + c);
-            y.a = f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
-            y.b = f32x4_t{bflo(u[2]), bfhi(u[2]), bflo(u[3]), bfhi(u[3])};
-        } else {
-            y.a = sn_load_y(a, row, c);
-            y.b = sn_load_y(a, row, c + 4);
-        }
+    auto source = [&](int64_t r) -> int64_t { return a.row_index ? sn_table(a.row_index, r) : r; };
+    using Y = typename std::conditional<ANY, Row8, u32x4_t>::type;
+    auto load_x = [&](int64_t r) { return sn_ld8f(a.x_in + source(r) * a.ldx + cl); };
+    auto load_y = [&](int64_t r) -> Y {
+        const int64_t row = source(r);
+        if constexpr (ANY) return {sn_load_slabs(a, row, cl), sn_load_slabs(a, row, cl + 4)};
+        else return *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const bf16_t*>(a.y) + row * a.ldy + cl);
     };
+    auto value = [](const Y& y) -> Row8 {
+        if constexpr (ANY) return y;
+        else return sn_unpack8(y);
+    };
+    auto sumsq = [&](const Row8& v) { return on ? sn_sumsq8(v) : 0.f; };
     // sums over the workgroup of two values per thread
     auto reduce2 = [&](float u, float v, int par, float& su, float& sv) {
         u = sn_wave_sum(u);
@@ -312,38 +347,61 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
             sv += s_red[par][1][i];
         }
     };
-    Row8 x = zero, y = zero, xn = zero, yn = zero;
-    load_row(lo, x, y);
+    // A row's x and the next row's y are there when its turn comes; the next x and the y behind it are requested first thing.  Every store of a turn is
+    // issued whatever the launch has (buffers that there are not: of no length), and y stays as it was read until it is used, so that a turn waits for the loads of the
+    // one before and not for its stores.  (It read sequence tables and state rows' numbers for every
+    // row, unpacked y where it read it and stored under tests, and so waited for everything it had just asked for.)  In a step, us, that / this: four taps, y and x out, 15074
+    // rows of 2048 86 / 70, 7180 40 / 35, 5000 of 4096 56 / 51; eight slabs, 700 of 2048 56 / 48; without y 57 / 44; without taps 50 / 46.  Non-temporal stores of x 74,
+    // written through 106 (a lane's two halves go in two stores).
+    Row8 x = load_x(lo);
+    Y y{}, y1{};
     float ry = 0.f, su, sv;
     int par = 0;
     if (a.y) {
-        reduce2(sn_sumsq8(y), 0.f, par, su, sv);
+        y = load_y(lo);
+        if (!ANY && lo + 1 < r1) y1 = load_y(lo + 1);
+        reduce2(sumsq(value(y)), 0.f, par, su, sv);
         ry = 1.0f / sqrtf(su * inv_w + a.eps);
         par ^= 1;
     }
+    // (what was requested so far is waited for here: a wait in the loop counts what is behind a load on every way to it)
+    asm volatile("" : "+v"(x.a), "+v"(x.b), "+v"(gq.a), "+v"(gq.b), "+v"(gp.a), "+v"(gp.b));
+    if constexpr (!ANY) asm volatile("" : "+v"(y), "+v"(y1));
+    const bool f32 = ANY && a.act_f32;
+    const int rowb = a.wp * 4, actb = a.wp * (f32 ? 4 : 2);
+    auto put = [&](void* base, int64_t ld, int64_t r, bool mine, const Row8& v) __attribute__((always_inline)) {   // activations
+        const __amdgpu_buffer_rsrc_t rs = sn_row(base, r * ld * (f32 ? 4 : 2), mine ? actb : 0);
+        if (f32) sn_put8f(rs, c * 4, v);
+        else __builtin_amdgcn_raw_buffer_store_b128(sn_pack8(v), rs, c * 2, 0, 0);
+    };
     for (int64_t r = lo; r < r1; ++r) {
-        const bool more = r + 1 < r1;
         if constexpr (TAPS > 1) {  // opaque: unpacked outside the loop the taps would take twice the registers
 #pragma unroll
             for (int j = 0; j < TAPS; ++j) asm volatile("" : "+v"(w[j]));
         }
-        if (more) load_row(r + 1, xn, yn);
+        Row8 xn = zero;
+        Y y2{};
+        if (r + 1 < r1) xn = load_x(r + 1);
+        if constexpr (ANY) {
+            if (a.y && r + 1 < r1) y1 = load_y(r + 1);
+        } else if (a.y && r + 2 < r1) y2 = load_y(r + 2);
         if (a.y) {
+            const Row8 v = value(y);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                x.a[i] = x.a[i] + y.a[i] * ry * gq.a[i];
-                x.b[i] = x.b[i] + y.b[i] * ry * gq.b[i];
+                x.a[i] = x.a[i] + v.a[i] * ry * gq.a[i];
+                x.b[i] = x.b[i] + v.b[i] * ry * gq.b[i];
             }
         }
-        if (r >= r0 && on) {
-            if (a.x_out) sn_st8f(a.x_out + r * a.ldx + c, x);
-            if (a.x_cast) sn_st8(a.x_cast, r * a.ldc + c, a.act_f32, x);
-        }
-        reduce2(sn_sumsq8(x), more ? sn_sumsq8(yn) : 0.f, par, su, sv);
+        const bool mine = TAPS == 1 || r >= r0;
+        sn_put8f(sn_row(a.x_out, r * a.ldx * 4, mine ? rowb : 0), c * 4, x);
+        put(a.x_cast, a.ldc, r, mine, x);
+        reduce2(sumsq(x), a.y && r + 1 < r1 ? sumsq(value(y1)) : 0.f, par, su, sv);
         par ^= 1;
+        Row8 o = zero;
         if (a.g_pre) {
             const float rx = 1.0f / sqrtf(su * inv_w + a.eps);
-            Row8 h, o;
+            Row8 h;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 h.a[i] = x.a[i] * rx * gp.a[i];
@@ -351,19 +409,16 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
             }
             o = h;
             if constexpr (TAPS > 1) {
-                if (r == qe) {  // the next sequence's portion begins
-                    s = a.seq_of[r];
-                    qs = a.q_start[s];
-                    qe = a.q_start[s + 1];
-                }
-                const int64_t sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
+                if (r == qe) sequence(r);  // the next sequence's portion begins
                 if (r == qs) {
-                    const int p = a.pos[r];
+                    const int p = sn_table(a.pos, r);
 #pragma unroll
                     for (int k = 1; k < TAPS; ++k) {
                         hist[k - 1] = zero;
-                        if (on && p - k >= 0) hist[k - 1] = sn_ld8f(a.state + (sin * HALO + (HALO - k)) * a.wp + c);
+                        if (on && p - k >= 0) hist[k - 1] = sn_ld8f(a.state + ((int64_t)sin * HALO + (HALO - k)) * a.wp + c);
                     }
+#pragma unroll
+                    for (int k = 1; k < TAPS; ++k) asm volatile("" : "+v"(hist[k - 1].a), "+v"(hist[k - 1].b));   // (waited for here, not in every turn)
                 }
                 Row8 acc = zero;
 #pragma unroll
@@ -378,23 +433,23 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
                     o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
                     o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
                 }
-                const int64_t so = a.state_out[s];
                 const int e = qe - 1 - (int)r;  // tokens of the portion behind this one
-                if (r >= r0 && e < HALO && on && so >= 0 && so < a.n_state && a.pos[r] >= 0) {
-                    sn_st8f(a.state + (so * HALO + (HALO - 1 - e)) * a.wp + c, h);
+                if (mine && e < HALO && so >= 0 && so < a.n_state && sn_table(a.pos, r) >= 0 && on) {
+                    sn_st8f(a.state + ((int64_t)so * HALO + (HALO - 1 - e)) * a.wp + c, h);
                     if (e == 0)  // a portion shorter than the history: the older inputs move up
                         for (int i = 0; i < HALO - (qe - qs); ++i)
-                            sn_st8f(a.state + (so * HALO + i) * a.wp + c, sn_ld8f(a.state + (sin * HALO + i + (qe - qs)) * a.wp + c));
+                            sn_st8f(a.state + ((int64_t)so * HALO + i) * a.wp + c, sn_ld8f(a.state + ((int64_t)sin * HALO + i + (qe - qs)) * a.wp + c));
                 }
 #pragma unroll
                 for (int k = HALO; k >= 2; --k) hist[k - 1] = hist[k - 2];
                 hist[0] = h;
             }
-            if (r >= r0 && on) sn_st8(a.h, r * a.ldh + c, a.act_f32, o);
         }
+        put(a.h, a.ldh, r, mine, o);
         if (a.y) ry = 1.0f / sqrtf(sv * inv_w + a.eps);
         x = xn;
-        y = yn;
+        y = y1;
+        if constexpr (!ANY) y1 = y2;
     }
 }
 
@@ -580,7 +635,8 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
     // stay one to a workgroup, re-reading the halo, as long as those are no more than four waves a SIMD (2048 workgroups of 64 threads: two), and
     // longer runs are cut for as many.  Four taps, us, runs of eight rows and more for 512 workgroups / this: 1024 columns at 800 rows 19.4 / 10.4, at 2048 20.6 / 15.9, at 8000
     // 46 / 33; 2048 at 600 rows 21.5 / 12.5, at 1024 21.9 / 16.0 (1025: 21.8, runs of eight), at 6000 45 / 40, at 15074 108 / 98 (without taps
-    // 95 / 83; 2048 workgroups 78 where 1024 took 75).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
+    // 95 / 83; 2048 workgroups 78 where 1024 took 75; with loads a turn ahead
+    // 512, 768, 1024 and 2048 workgroups 72.1, 70.5, 70.5 and 76.3).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
     if constexpr (NT < 1024 || TAPS == 1) {  // (1024 threads do not have the registers for rows, taps and history at once)
         // With taps: portions of one row, up to three quarters of the CUs.  Longer ones take the stream kernel, which knows where a portion begins before it
@@ -596,7 +652,9 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
     }
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;
-    hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT>), dim3((unsigned)((a.T + tr - 1) / tr)), dim3(NT), 0, st, a, tr);
+    const dim3 grid((unsigned)((a.T + tr - 1) / tr));
+    if (a.act_f32 || (a.y && a.y_f32)) hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, true>), grid, dim3(NT), 0, st, a, tr);
+    else hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, false>), grid, dim3(NT), 0, st, a, tr);
     GLM_CHECK_LAUNCH("glm_seq_norm");
     return GLM_OK;
 }

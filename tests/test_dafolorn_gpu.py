@@ -150,6 +150,36 @@ def test_seq_norm_is_one_launch_whatever_the_portions(width, taps, lens, monkeyp
             assert all(torch.equal(a, b) for a, b in zip(got[0], other))
 
 
+@pytest.mark.parametrize("width,taps", [(64, 1), (72, 2), (520, 3), (1032, 4), (2048, 4), (4104, 4), (2056, 6), (4096, 8), (8192, 1)])
+@pytest.mark.parametrize("lens", [[700, 1, 41, 2, 9, 600, 3, 1500], [4100]])
+def test_seq_norm_stream_of_bf16(width, taps, lens):
+    """Runs of rows with activations in bf16 (loads a row ahead, stores through buffers) against the form for fp32 rows: the same bits, h and the cast row rounded.  Rows of
+    the cast start anywhere and what is around them stays; a launch without y, without h, without a cast and one of gathered rows."""
+    from nanovllm import hip_ops
+    wp, T, S = hip_ops.round8(width), sum(lens), len(lens)
+    pos = i32([(40 if s % 3 == 1 else 0) + p for s, n in enumerate(lens) for p in range(n)])
+    meta = types.SimpleNamespace(pos=pos, seq_of=i32([s for s, n in enumerate(lens) for _ in range(n)]), q_start=i32([sum(lens[:s]) for s in range(S + 1)]),
+                                 state_in=i32(list(range(S))), state_out=i32([S + s if s % 5 != 4 else -1 for s in range(S)]))
+    torch.manual_seed(width)
+    x, gain, gp = torch.randn(T, wp, device="cuda"), torch.randn(wp, device="cuda"), torch.randn(wp, device="cuda")
+    y = torch.randn(T, wp, device="cuda").bfloat16()
+    state = torch.randn(2 * S, max(taps - 1, 1), wp, device="cuda")
+    conv = (torch.randn(taps, wp, device="cuda").bfloat16(), state) if taps > 1 else None
+    index = torch.randperm(T, device="cuda", dtype=torch.int32)
+    for yv, g, shift, rows in [(y, gain, 0, None), (y, gain, 1, None), (y, gain, 4, None), (y, None, 8, None), (None, gain, None, None)] + ([(y, gain, None, index)] if taps == 1 else []):
+        got = []
+        for dtype in (torch.float32, torch.bfloat16):
+            kept = state.clone()
+            cast = torch.full((T, wp + 16), 7.0, device="cuda", dtype=dtype) if shift is not None else None
+            xo, h = hip_ops.seq_norm(x, width, 1e-5, y=yv, g_post=gp, g_pre=g, conv=(conv[0], kept) if conv and g is not None else None, meta=meta, rows=rows, act_dtype=dtype,
+                                     x_cast=cast[:, shift: shift + wp] if cast is not None else None)
+            got.append([xo, kept] + ([] if h is None else [h.bfloat16()]) + ([] if cast is None else [cast.bfloat16()]))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+        if shift is not None:
+            c = got[1][-1]
+            assert bool((c[:, :shift] == 7).all()) and bool((c[:, shift + wp:] == 7).all()) and torch.equal(c[:, shift: shift + wp], got[1][0].bfloat16())
+
+
 @pytest.mark.parametrize("n", [1, 3, 5, 6, 9, 16])
 @pytest.mark.parametrize("T,width", [(1, 64), (7, 2048), (512, 520), (513, 520)])
 def test_seq_norm_adds_slabs_in_their_order(n, T, width):
