@@ -15,6 +15,7 @@
 // because the workgroup that writes a portion's last h is not the one that reads the previous portion's.  A token's h is the
 // same arithmetic whether it was computed in this step or kept from an earlier one.
 #include "common.h"
+#include <type_traits>
 
 namespace {
 
@@ -50,40 +51,49 @@ __device__ __forceinline__ f32x4_t st_load4(const void* base, int64_t off, int f
     const u32x2_t u = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const bf16_t*>(base) + off);
     return f32x4_t{bflo(u[0]), bfhi(u[0]), bflo(u[1]), bfhi(u[1])};
 }
-__device__ __forceinline__ void st_store4(void* base, int64_t off, int f32, const f32x4_t& v) {
-    if (f32) *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(base) + off) = v;
-    else *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(base) + off) = u32x2_t{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
-}
 __device__ __forceinline__ float st_sumsq(const f32x4_t& v) { return v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3]; }
 
-// S streams, NV vectors of four columns per thread, NT threads: wp <= 4 NV NT
-template <int S, int NV, int NT>
+// Tables that no launch changes while it reads them: through the scalar cache, so that a row's bookkeeping waits for no vector load or store
+__device__ __forceinline__ int st_table(const int32_t* p, int64_t i) { return reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p))[i]; }
+// `bytes` of a row; nothing if there is no such buffer
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t st_row(const void* base, int64_t off, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base) + off), 0, base ? bytes : 0, 0x00020000);
+}
+
+// S streams, NV vectors of four columns per thread, NT threads: wp <= 4 NV NT.  ANY: y or h may be fp32
+template <int S, int NV, int NT, bool ANY>
 __global__ __launch_bounds__(NT) void stream_norm_kernel(const StreamNormArgs a, int tr) {
-    constexpr int NW = NT / 64;
+    constexpr int NW = NT / 64, NTEMP = 2;   // NTEMP: cache policy bit of a store, not to be kept
     __shared__ float s_red[2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     const int64_t r0 = (int64_t)blockIdx.x * tr, r1 = min(r0 + tr, a.T);
     const float inv_w = 1.0f / (float)a.width;
-    const bool shifted = a.shift != nullptr;
-    int s = 0, qs = 0, qe = 0;
+    const bool shifted = a.shift != nullptr, y_f32 = ANY && a.y_f32, h_f32 = ANY && a.h_f32;
+    int s = 0, qs = 0, qe = 0, sin = 0, so = 0;
+    auto sequence = [&](int64_t r) {
+        s = st_table(a.seq_of, r);
+        qs = st_table(a.q_start, s);
+        qe = st_table(a.q_start, s + 1);
+        sin = (int)min(max((int64_t)st_table(a.state_in, s), (int64_t)0), a.n_state - 1);
+        so = st_table(a.state_out, s);
+    };
     int64_t lo = r0;
     if (shifted) {
-        s = a.seq_of[r0];
-        qs = a.q_start[s];
-        qe = a.q_start[s + 1];
+        sequence(r0);
         if (r0 > qs) lo = r0 - 1;
     }
-    // vector j of this thread: columns 4 (tid + j NT) .. + 3
-    int col[NV];
+    // vector j of this thread: columns 4 (tid + j NT) .. + 3; at: what a thread behind the row's end reads instead
+    int col[NV], at[NV];
     bool on[NV];
     f32x4_t ys[NV], sh[NV], hist[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         col[j] = 4 * (tid + j * NT);
         on[j] = col[j] < a.wp;
-        ys[j] = (on[j] && a.y) ? *reinterpret_cast<const f32x4_t*>(a.y_scale + col[j]) : zero;
-        sh[j] = (on[j] && shifted) ? *reinterpret_cast<const f32x4_t*>(a.shift + col[j]) : zero;
+        at[j] = min(col[j], a.wp - 4);
+        ys[j] = a.y ? *reinterpret_cast<const f32x4_t*>(a.y_scale + at[j]) : zero;
+        sh[j] = shifted ? *reinterpret_cast<const f32x4_t*>(a.shift + at[j]) : zero;
         hist[j] = zero;
     }
     float mix[S][S], wo[S], wi[S];
@@ -94,27 +104,50 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const StreamNormArgs a,
 #pragma unroll
         for (int t = 0; t < S; ++t) mix[f][t] = a.y ? a.mix_out[f * S + t] : 0.f;
     }
-    auto load_row = [&](int64_t r, f32x4_t (&x)[S][NV], f32x4_t (&y)[NV]) {
-        const int64_t row = a.row_index ? a.row_index[r] : r;
+    using Y = typename std::conditional<ANY, f32x4_t, u32x2_t>::type;   // y as it was read
+    auto load_row = [&](int64_t r, f32x4_t (&x)[S][NV], Y (&y)[NV]) __attribute__((always_inline)) {
+        const int64_t row = a.row_index ? st_table(a.row_index, r) : r;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-            if (!on[j]) continue;
 #pragma unroll
-            for (int t = 0; t < S; ++t) x[t][j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(a.x_in + row * a.ldx + t * a.sx + col[j]));
-            if (a.y) y[j] = st_load4(a.y, row * a.ldy + col[j], a.y_f32);
+            for (int t = 0; t < S; ++t) x[t][j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(a.x_in + row * a.ldx + t * a.sx + at[j]));
+        }
+        if (a.y) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                if constexpr (ANY) y[j] = st_load4(a.y, row * a.ldy + at[j], y_f32);
+                else y[j] = *reinterpret_cast<const u32x2_t*>(reinterpret_cast<const bf16_t*>(a.y) + row * a.ldy + at[j]);
+            }
         }
     };
-    f32x4_t x[S][NV], y[NV], xn[S][NV], yn[NV];
+    auto value = [](const Y& y, int i) -> float {
+        if constexpr (ANY) return y[i];
+        else return i & 1 ? bfhi(y[i >> 1]) : bflo(y[i >> 1]);
+    };
+    f32x4_t x[S][NV], xn[S][NV];
+    Y y[NV], yn[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-        y[j] = yn[j] = zero;
+        y[j] = yn[j] = Y{};
 #pragma unroll
         for (int t = 0; t < S; ++t) x[t][j] = xn[t][j] = zero;
     }
     load_row(lo, x, y);
+    // Every store of a turn is issued whatever the launch has (buffers that there are not: of no length), and y stays as it was read until it is used, so that a turn waits
+    // for the loads of the one before it and not for its stores.  (It unpacked y where it read it, read the sequence tables for every row and stored under tests, and so waited
+    // for everything it had just asked for.)  In a step, two streams, us, that / this: 11137 rows of 2048 102 / 80 with a token shift, 84 / 75 without, without y 53 / 37;
+    // 5500 61 / 41, 44 / 36; 4600 of 4096 77 / 68, 70 / 64; 700 of 2048 11.9 / 10.3.
+    // (What was requested so far is waited for here: a wait in the loop counts what is behind a load on every way to it.)
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        asm volatile("" : "+v"(y[j]), "+v"(ys[j]), "+v"(sh[j]));
+#pragma unroll
+        for (int t = 0; t < S; ++t) asm volatile("" : "+v"(x[t][j]));
+    }
     int par = 0;
     for (int64_t r = lo; r < r1; ++r) {
         if (r + 1 < r1) load_row(r + 1, xn, yn);
+        const bool mine = r >= r0;
         float sq = 0.f;
         f32x4_t u[NV];
 #pragma unroll
@@ -125,7 +158,7 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const StreamNormArgs a,
                 for (int t = 0; t < S; ++t) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float acc = wo[t] * (ys[j][i] * y[j][i]);
+                        float acc = wo[t] * (ys[j][i] * value(y[j], i));
 #pragma unroll
                         for (int f = 0; f < S; ++f) acc = fmaf(mix[f][t], x[f][j][i], acc);
                         v[t][i] = acc;
@@ -134,17 +167,20 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const StreamNormArgs a,
 #pragma unroll
                 for (int t = 0; t < S; ++t) x[t][j] = v[t];
             }
-            if (a.x_out && r >= r0 && on[j]) {
-#pragma unroll
-                for (int t = 0; t < S; ++t) __builtin_nontemporal_store(x[t][j], reinterpret_cast<f32x4_t*>(a.x_out + (r * S + t) * a.wp + col[j]));
-            }
             u[j] = zero;
 #pragma unroll
             for (int t = 0; t < S; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) u[j][i] = fmaf(wi[t], x[t][j][i], u[j][i]);
-            sq += st_sumsq(u[j]);
+            sq += on[j] ? st_sumsq(u[j]) : 0.f;
         }
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+            const __amdgpu_buffer_rsrc_t rs = st_row(a.x_out, (r * S + t) * a.wp * 4, mine ? a.wp * 4 : 0);
+#pragma unroll
+            for (int j = 0; j < NV; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, x[t][j]), rs, col[j] * 4, 0, NTEMP);
+        }
+        f32x4_t o[NV];
         if (a.h) {
             sq = wave_sum(sq);
             if constexpr (NW > 1) {
@@ -156,36 +192,39 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const StreamNormArgs a,
                 par ^= 1;
             }
             const float rms = sqrtf(sq * inv_w + a.eps), f = a.gain / rms;
-            int64_t so = -1;
-            bool first = false;
-            int64_t sin = 0;
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[j][i] = u[j][i] * f;
             if (shifted) {
-                if (r == qe) {  // the next sequence's portion begins
-                    s = a.seq_of[r];
-                    qs = a.q_start[s];
-                    qe = a.q_start[s + 1];
+                if (r == qe) sequence(r);  // the next sequence's portion begins
+                if (r == qs) {
+                    // first token of its sequence: whatever the state row holds is not its
+                    const bool fresh = st_table(a.pos, r) <= 0;
+#pragma unroll
+                    for (int j = 0; j < NV; ++j) hist[j] = fresh ? zero : *reinterpret_cast<const f32x4_t*>(a.state + (int64_t)sin * a.wp + at[j]);
+#pragma unroll
+                    for (int j = 0; j < NV; ++j) asm volatile("" : "+v"(hist[j]));   // (waited for here, not in every turn)
                 }
-                first = r == qs;
-                sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
-                if (r == qe - 1 && r >= r0 && a.pos[r] >= 0) so = a.state_out[s];
-                if (so >= a.n_state) so = -1;
-            }
-            const bool fresh = first && a.pos[r] <= 0;  // first token of its sequence: whatever the state row holds is not its
+                const bool keep = mine && r == qe - 1 && so >= 0 && so < a.n_state && st_table(a.pos, r) >= 0;
 #pragma unroll
-            for (int j = 0; j < NV; ++j) {
-                f32x4_t o;
+                for (int j = 0; j < NV; ++j) {
+                    const f32x4_t hv = o[j];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) o[i] = u[j][i] * f;
-                if (shifted && on[j]) {
-                    const f32x4_t hv = o;
-                    if (first) hist[j] = fresh ? zero : *reinterpret_cast<const f32x4_t*>(a.state + sin * a.wp + col[j]);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) o[i] = fmaf(hist[j][i] - hv[i], sh[j][i], hv[i]);
+                    for (int i = 0; i < 4; ++i) o[j][i] = fmaf(hist[j][i] - hv[i], sh[j][i], hv[i]);
                     hist[j] = hv;
-                    if (so >= 0) *reinterpret_cast<f32x4_t*>(a.state + so * a.wp + col[j]) = hv;
+                    if (keep && on[j]) *reinterpret_cast<f32x4_t*>(a.state + (int64_t)so * a.wp + col[j]) = hv;
                 }
-                if (r >= r0 && on[j]) st_store4(a.h, r * a.ldh + col[j], a.h_f32, o);
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NV; ++j) o[j] = zero;
+        }
+        const __amdgpu_buffer_rsrc_t rs = st_row(a.h, r * a.ldh * (h_f32 ? 4 : 2), mine ? a.wp * (h_f32 ? 4 : 2) : 0);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            if (h_f32) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o[j]), rs, col[j] * 4, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{pack2bf(o[j][0], o[j][1]), pack2bf(o[j][2], o[j][3])}, rs, col[j] * 2, 0, 0);
         }
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
@@ -265,7 +304,9 @@ int launch_stream(const StreamNormArgs& a, hipStream_t st) {
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);   // four waves on every SIMD
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;
-    hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT>), dim3((unsigned)((a.T + tr - 1) / tr)), dim3(NT), 0, st, a, tr);
+    const dim3 grid((unsigned)((a.T + tr - 1) / tr));
+    if ((a.y && a.y_f32) || (a.h && a.h_f32)) hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT, true>), grid, dim3(NT), 0, st, a, tr);
+    else hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT, false>), grid, dim3(NT), 0, st, a, tr);
     GLM_CHECK_LAUNCH("glm_stream_norm");
     return GLM_OK;
 }

@@ -137,6 +137,31 @@ def test_stream_norm(width, S, y_kind):
             assert torch.allclose(o[s], outs[0][s][: o[s].shape[0]], rtol=1e-6, atol=2e-6)
 
 
+@pytest.mark.parametrize("width,S", [(64, 1), (520, 2), (2048, 2), (2056, 3), (4096, 2), (72, 4), (1024, 6), (4104, 8)])
+@pytest.mark.parametrize("lens", [[1, 30, 2, 1], [700, 1, 41, 2, 9, 600, 3, 1500], [4100]])
+def test_stream_norm_of_bf16(width, S, lens):
+    """Runs of rows with activations in bf16 (loads a row ahead, stores through buffers) against the form for fp32 rows: the same bits, h rounded.  With the token shift and
+    without, broadcast streams, no y, no h, gathered rows."""
+    from nanovllm import hip_ops
+    wp, T, n = hip_ops.round8(width), sum(lens), len(lens)
+    pos = i32([(40 if s % 3 == 1 else 0) + p for s, c in enumerate(lens) for p in range(c)])
+    meta = types.SimpleNamespace(pos=pos, seq_of=i32([s for s, c in enumerate(lens) for _ in range(c)]), q_start=i32([sum(lens[:s]) for s in range(n + 1)]),
+                                 state_in=i32(list(range(n))), state_out=i32([n + s if s % 5 != 4 else -1 for s in range(n)]))
+    torch.manual_seed(width)
+    r = lambda *d: torch.randn(*d, device="cuda")  # noqa: E731
+    x, row, y, state, wi = r(T, S, wp), r(T, wp), r(T, wp).bfloat16(), r(2 * n, wp), r(S)
+    out, shift, index = dict(y=y, y_scale=r(wp), mix_out=r(S * (S + 1))), r(wp), torch.randperm(T, device="cuda", dtype=torch.int32)
+    for xs, kw in [(x, dict(out, w_in=wi, shift=shift)), (x, dict(out, w_in=wi)), (x, dict(out)), (row, dict(w_in=wi, shift=shift)), (row, dict(out, w_in=wi, shift=shift)),
+                   (x, dict(out, w_in=wi, rows=index))]:
+        got = []
+        for dtype in (torch.float32, torch.bfloat16):
+            kept = state.clone()
+            kw_ = dict(kw, y=kw["y"].to(dtype)) if "y" in kw else kw     # (fp32 copies of the same values: the other form also where there is no h)
+            xo, h = hip_ops.stream_norm(xs, S, width, 1e-5, gain=1.5, state=kept, meta=meta, act_dtype=dtype, **kw_)
+            got.append([xo, kept] + ([] if h is None else [h.bfloat16()]))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 def _paged(rows, G, bs, n_blocks, perm):
     """[T, G, d] of several sequences scattered over the blocks `perm`; unused memory is NaN."""
     cache = torch.full((n_blocks, G, bs, rows[0].shape[2]), float("nan"))
