@@ -313,69 +313,115 @@ __global__ __launch_bounds__(1024) void depth_norm_kernel(const DepthArgs a) {
     dn_st<VEC>(a.h, r * a.ldh + c, a.act_f32, h, nc);
 }
 
-// h = x + conv(x) and the state, eight columns per thread down a run of rows, the next row's load in flight
-template <int TAPS>
+// Tables that no launch changes while it reads them: through the scalar cache, so that a row's bookkeeping waits for no vector load or store
+__device__ __forceinline__ int dn_table(const int32_t* p, int64_t i) { return reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(p))[i]; }
+__device__ __forceinline__ void dn_put(void* base, int64_t off, int bytes, int at, const u32x4_t& v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(base) + off, 0, bytes, 0x00020000), at, 0, 0);
+}
+
+// h = x + conv(x) and the state, eight columns per thread down a run of rows, UN rows at a time, the next ones' loads in flight: what a turn needs of memory was requested
+// a turn ago, rows stay as they were read until they are used, and every store is issued (of no length behind the run's end), so that no turn waits for what it has just
+// asked for or stored.  (Padding columns masked
+// where they were read and the state row's number read for every row, as it was / this, us in a step, four taps, runs of 16 rows: 15074 rows of 2048 41.3 / 38.3, 5000 of 4096
+// 35 / 25.6, 700 of 2048 16.8 / 10.3, 40 single rows and 5400 of prompts 74 / 42.)
+template <int TAPS, bool F32>
 __global__ __launch_bounds__(256) void depth_conv_kernel(const DepthArgs a, const float* __restrict__ xs, int tr) {
-    constexpr int HALO = TAPS - 1;
+    constexpr int HALO = TAPS - 1, UN = TAPS <= 4 ? 2 : 1;
     const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
     if (c >= a.wp) return;
     const int nc = min(8, a.width - c);   // (the padding columns of x are not written by anyone)
     const int64_t r0 = (int64_t)blockIdx.x * tr, r1 = min(r0 + tr, a.T);
-    auto load = [&](const float* p) {
-        Col8 v = dn_ldf<true>(p, 8);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v.v[i] = i < nc ? v.v[i] : 0.f;
-        return v;
+    struct Raw {
+        f32x4_t a, b;
     };
-    Col8 w[TAPS], hist[TAPS];
+    auto raw = [&](const float* p) -> Raw { return {*reinterpret_cast<const f32x4_t*>(p), *reinterpret_cast<const f32x4_t*>(p + 4)}; };
+    auto masked = [&](const Raw& v) {
+        Col8 o;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o.v[i] = i < nc ? (i < 4 ? v.a[i & 3] : v.b[i & 3]) : 0.f;
+        return o;
+    };
+    u32x4_t w[TAPS];   // eight taps packed
+    Col8 hist[TAPS];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
-        w[j] = dn_ldh<true>(a.conv_w + (int64_t)j * a.wp + c, 8);
+        w[j] = *reinterpret_cast<const u32x4_t*>(a.conv_w + (int64_t)j * a.wp + c);
         hist[j] = dn_zero();
     }
-    int s = a.seq_of[r0], qs = a.q_start[s], qe = a.q_start[s + 1];
-    int64_t sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
-    auto history = [&](int64_t r) {   // inputs of the tokens in front of row r
-        const int p = a.pos[r];
+    auto tap = [](const u32x4_t& p, int i) { return (i & 1) ? bfhi(p[i >> 1]) : bflo(p[i >> 1]); };
+    int s = 0, qs = 0, qe = 0, so = 0;
+    int64_t sin = 0;
+    auto sequence = [&](int64_t r) {   // and the inputs of the tokens in front of row r
+        s = dn_table(a.seq_of, r);
+        qs = dn_table(a.q_start, s);
+        qe = dn_table(a.q_start, s + 1);
+        sin = min(max((int64_t)dn_table(a.state_in, s), (int64_t)0), a.n_state - 1);
+        so = dn_table(a.state_out, s);
+        const int p = dn_table(a.pos, r);
+        Raw t[TAPS];
 #pragma unroll
         for (int k = 1; k < TAPS; ++k) {
-            hist[k - 1] = dn_zero();
+            t[k - 1] = Raw{};
             if (p - k < 0) continue;
-            if (r - k >= qs) hist[k - 1] = load(xs + (r - k) * a.ld + c);
-            else hist[k - 1] = load(a.state + (sin * HALO + (HALO - (qs - (r - k)))) * a.wp + c);
+            if (r - k >= qs) t[k - 1] = raw(xs + (r - k) * a.ld + c);
+            else t[k - 1] = raw(a.state + (sin * HALO + (HALO - (qs - (r - k)))) * a.wp + c);
+        }
+#pragma unroll
+        for (int k = 1; k < TAPS; ++k) {
+            asm volatile("" : "+v"(t[k - 1].a), "+v"(t[k - 1].b));   // (waited for here, not in every turn)
+            hist[k - 1] = masked(t[k - 1]);
         }
     };
-    history(r0);
-    Col8 x = load(xs + r0 * a.ld + c), xn = dn_zero();
-    for (int64_t r = r0; r < r1; ++r) {
-        if (r + 1 < r1) xn = load(xs + (r + 1) * a.ld + c);
-        if (r == qe) {  // the next sequence's portion begins
-            s = a.seq_of[r];
-            qs = a.q_start[s];
-            qe = a.q_start[s + 1];
-            sin = min(max((int64_t)a.state_in[s], (int64_t)0), a.n_state - 1);
-            history(r);
+    Raw x[UN], xn[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+        x[u] = xn[u] = Raw{};
+        if (r0 + u < r1) x[u] = raw(xs + (r0 + u) * a.ld + c);
+    }
+    sequence(r0);
+#pragma unroll
+    for (int u = 0; u < UN; ++u) asm volatile("" : "+v"(x[u].a), "+v"(x[u].b));
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) asm volatile("" : "+v"(w[j]));
+    const int rowb = a.wp * (F32 ? 4 : 2);
+    for (int64_t r = r0; r < r1; r += UN) {
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) asm volatile("" : "+v"(w[j]));  // opaque: unpacked outside the loop the taps would take twice the registers
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+            if (r + UN + u < r1) xn[u] = raw(xs + (r + UN + u) * a.ld + c);
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const int64_t row = r + u;
+            const bool there = row < r1;
+            if (there && row == qe) sequence(row);  // the next sequence's portion begins
+            const Col8 xv = masked(x[u]);
+            Col8 acc = dn_zero(), h;
+#pragma unroll
+            for (int k = HALO; k >= 1; --k)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc.v[i] = acc.v[i] + tap(w[TAPS - 1 - k], i) * hist[k - 1].v[i];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) h.v[i] = xv.v[i] + (acc.v[i] + tap(w[TAPS - 1], i) * xv.v[i]);
+            if constexpr (F32) {
+                dn_put(a.h, row * a.ldh * 4, there ? rowb : 0, c * 4, __builtin_bit_cast(u32x4_t, f32x4_t{h.v[0], h.v[1], h.v[2], h.v[3]}));
+                dn_put(a.h, row * a.ldh * 4, there ? rowb : 0, c * 4 + 16, __builtin_bit_cast(u32x4_t, f32x4_t{h.v[4], h.v[5], h.v[6], h.v[7]}));
+            } else {
+                dn_put(a.h, row * a.ldh * 2, there ? rowb : 0, c * 2, u32x4_t{pack2bf(h.v[0], h.v[1]), pack2bf(h.v[2], h.v[3]), pack2bf(h.v[4], h.v[5]), pack2bf(h.v[6], h.v[7])});
+            }
+            const int e = qe - 1 - (int)row;  // tokens of the portion behind this one
+            if (there && e < HALO && so >= 0 && so < a.n_state && dn_table(a.pos, row) >= 0) {
+                dn_stf<true>(a.state + ((int64_t)so * HALO + (HALO - 1 - e)) * a.wp + c, xv, 8);
+                if (e == 0)  // a portion shorter than the history: the older inputs move up
+                    for (int i = 0; i < HALO - (qe - qs); ++i)
+                        dn_stf<true>(a.state + ((int64_t)so * HALO + i) * a.wp + c, dn_ldf<true>(a.state + (sin * HALO + i + (qe - qs)) * a.wp + c, 8), 8);
+            }
+#pragma unroll
+            for (int k = HALO; k >= 2; --k) hist[k - 1] = hist[k - 2];
+            hist[0] = xv;
         }
-        Col8 acc = dn_zero(), h;
 #pragma unroll
-        for (int k = HALO; k >= 1; --k)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc.v[i] = acc.v[i] + w[TAPS - 1 - k].v[i] * hist[k - 1].v[i];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) h.v[i] = x.v[i] + (acc.v[i] + w[TAPS - 1].v[i] * x.v[i]);
-        dn_st<true>(a.h, r * a.ldh + c, a.act_f32, h, 8);
-        const int64_t so = a.state_out[s];
-        const int e = qe - 1 - (int)r;  // tokens of the portion behind this one
-        if (e < HALO && so >= 0 && so < a.n_state && a.pos[r] >= 0) {
-            dn_stf<true>(a.state + (so * HALO + (HALO - 1 - e)) * a.wp + c, x, 8);
-            if (e == 0)  // a portion shorter than the history: the older inputs move up
-                for (int i = 0; i < HALO - (qe - qs); ++i)
-                    dn_stf<true>(a.state + (so * HALO + i) * a.wp + c, dn_ldf<true>(a.state + (sin * HALO + i + (qe - qs)) * a.wp + c, 8), 8);
-        }
-#pragma unroll
-        for (int k = HALO; k >= 2; --k) hist[k - 1] = hist[k - 2];
-        hist[0] = x;
-        x = xn;
+        for (int u = 0; u < UN; ++u) x[u] = xn[u];
     }
 }
 
@@ -383,10 +429,14 @@ constexpr int64_t DN_SPLIT_ROWS = 512;   // rows from which norm and convolution
 
 template <int TAPS>
 int launch_depth_conv(const DepthArgs& a, const float* xs, hipStream_t st) {
-    // 16 rows per workgroup: four workgroups to a CU (15074 rows of 2048: 57 -> 40 us; 32 rows left two, 8 read too many rows twice: 43).  With the
-    // norm ahead of it, 32 / 16 rows, us: 1000 rows of 1024 32 / 21, of 4096 44 / 31; 4096 rows of 2048 52 / 40, 15074 rows of 4096 206 / 209
-    const int tr = 16;
-    hipLaunchKernelGGL(depth_conv_kernel<TAPS>, dim3((unsigned)((a.T + tr - 1) / tr), (unsigned)((a.wp + 2047) / 2048)), dim3(256), 0, st, a, xs, tr);
+    // Runs of four rows and more for 1024 workgroups, of 16 at most: portions that begin inside a run wait for their state one after the other, and shorter runs read more
+    // rows twice.  16 rows / 512 workgroups / this / 2048, us: 15074 rows of 2048 38.3 / 38.3 / 38.3 / 41.3, 5000 of 4096 25.6 / 25.8 / 25.3 / 26.4, 700 of 2048 10.3 / 6.2 / 6.2 /
+    // 6.3, 40 single rows and 5400 of prompts 41.8 / 31.6 / 24.4 / 20.0, 60 and 5800 44.7 / 36.9 / 25.4 / 22.0.
+    const int64_t per = (a.T * ((a.wp + 2047) / 2048) + 1023) / 1024;
+    const int tr = (int)(per < 4 ? 4 : per > 16 ? 16 : (per + 1) / 2 * 2);
+    const dim3 grid((unsigned)((a.T + tr - 1) / tr), (unsigned)((a.wp + 2047) / 2048));
+    if (a.act_f32) hipLaunchKernelGGL((depth_conv_kernel<TAPS, true>), grid, dim3(256), 0, st, a, xs, tr);
+    else hipLaunchKernelGGL((depth_conv_kernel<TAPS, false>), grid, dim3(256), 0, st, a, xs, tr);
     GLM_CHECK_LAUNCH("glm_depth_norm(convolution)");
     return GLM_OK;
 }

@@ -146,6 +146,38 @@ def test_depth_norm(dtype, width, groups, taps, depth):
         assert torch.allclose(h[:, :width].cpu().double(), O.norm_groups(xn[pick], gain.double(), groups, eps), atol=2 * tol, rtol=tol), kind
 
 
+@pytest.mark.parametrize("width,taps", [(72, 4), (76, 3), (64, 2), (1032, 6), (4104, 4)])
+@pytest.mark.parametrize("lens", [[3000, 1, 1, 1, 6000, 2, 900], [5, 1, 700, 3, 1, 1, 2]])
+def test_convolution_down_runs(width, taps, lens):
+    """Runs of rows of several lengths, portions that begin and end inside them: against the same sum in 64 bits, the state row by row, and rows in bf16 as those in fp32, rounded."""
+    from nanovllm import hip_ops
+    wp, tp, T, S = hip_ops.round8(width), hip_ops.depth_norm_taps(taps), sum(lens), len(lens)
+    starts = [0 if s % 2 else 40 for s in range(S)]
+    meta, order = batch_meta(lens, starts)
+    x, old = torch.randn(T, width, generator=g(1)), torch.randn(S, tp - 1, width, generator=g(2))
+    cw = torch.zeros(tp, wp)
+    cw[tp - taps:, :width] = (torch.randn(width, taps, generator=g(3)) * 0.5).to(torch.bfloat16).float().T
+    state = torch.full((2 * S, tp - 1, wp), float("nan"), device="cuda")
+    for s, row in enumerate(order[:S]):
+        state[row] = padc(old[s], wp).cuda()
+    xp = torch.full((T, wp), float("nan"))      # (padding columns are nobody's)
+    xp[:, :width] = x
+    got = []
+    for dt in (torch.float32, torch.bfloat16):
+        kept = state.clone()
+        h = hip_ops.depth_norm(dev(xp), width, 1, 1e-3, conv=(dev(cw, torch.bfloat16), kept), meta=meta, act_dtype=dt)[1]
+        got.append((h.bfloat16(), kept[:, :, :width], h))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1].nan_to_num(7.0), got[1][1].nan_to_num(7.0))
+    at, h = 0, got[0][2].cpu().double()
+    assert bool((h[:, width:] == 0).all())
+    for s, (n, start) in enumerate(zip(lens, starts)):
+        z = torch.cat([old[s] if start else torch.zeros(tp - 1, width), x[at: at + n]]).double()
+        want = z[tp - 1:] + sum(z[j: j + n] * cw[j, :width].double() for j in range(tp))
+        assert torch.allclose(h[at: at + n, :width], want, atol=2e-5, rtol=2e-5), s
+        assert torch.equal(got[0][1][order[S + s]].cpu(), z[-(tp - 1):].float()) or start == 0 and n < tp - 1
+        at += n
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,ff,E,top", [(76, 20, 5, 2), (136, 72, 9, 1), (64, 8, 70, 6), (72, 24, 300, 8), (40, 44, 3, 3), (256, 512, 64, 4)])
 def test_experts(dtype, width, ff, E, top):
