@@ -637,6 +637,7 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
     // 46 / 33; 2048 at 600 rows 21.5 / 12.5, at 1024 21.9 / 16.0 (1025: 21.8, runs of eight), at 6000 45 / 40, at 15074 108 / 98 (without taps
     // 95 / 83; 2048 workgroups 78 where 1024 took 75; with loads a turn ahead
     // 512, 768, 1024 and 2048 workgroups 72.1, 70.5, 70.5 and 76.3).  Wider rows, of 512 and 1024 threads, have four and eight waves a SIMD with 512 workgroups.
+    // Runs of eight rows at least / of four (two: equal but for slabs), us: 40 single rows and 5400 of prompts 35 / 31, without y 26.9 / 22.0, 3000 rows 22.7 / 20.4, 1200 19 / 16.
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);
     if constexpr (NT < 1024 || TAPS == 1) {  // (1024 threads do not have the registers for rows, taps and history at once)
         // With taps: portions of one row, up to three quarters of the CUs.  Longer ones take the stream kernel, which knows where a portion begins before it
@@ -651,7 +652,7 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
         }
     }
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
-    if (tr > 1) tr = tr < 8 ? 8 : tr > 32 ? 32 : tr;
+    if (tr > 1) tr = tr < 4 ? 4 : tr > 32 ? 32 : tr;
     const dim3 grid((unsigned)((a.T + tr - 1) / tr));
     if (a.act_f32 || (a.y && a.y_f32)) hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, true>), grid, dim3(NT), 0, st, a, tr);
     else hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, false>), grid, dim3(NT), 0, st, a, tr);
