@@ -50,6 +50,7 @@ constexpr int64_t LM_WIDE = 1 << 25;   // output pitch from which 16 fp32 rows d
 
 // Tile configurations (the kernel is written once over these):
 //   CfgR 256(n) x 256(m) x 64(k), five 32-KiB slots of one operand tile each, two phases of 32 MFMAs per K tile
+//   CfgR192 the same with 192(m): phases of 24 MFMAs
 //   CfgA 256(n) x 128(m) x 64(k), 3-stage ring, wave tile 64x64  (16 LDS reads + 6 DMA per 32 MFMA)
 //   CfgB 256(n) x 256(m) x 32(k), 4-stage ring, wave tile 64x128 (12 LDS reads + 4 DMA per 32 MFMA): only where K is no whole
 //        number of 64 or an operand spans 2 GiB (the plain form)
@@ -81,6 +82,7 @@ struct LmCfg {
     static constexpr int DPW = W_DMA + X_DMA;
     static constexpr int KS = A8 ? 2 : BK / 32;    // MFMA k-steps per tile (A8: the two 16-byte halves of ONE K = 128 operand)
     static constexpr int MT = BM / 2 / 16;         // 16-token MFMA tiles per wave (2 waves along m)
+    static constexpr int XH = MT / 2;              // of these in each of a K tile's two phases (ring)
     static constexpr int WT = LM_BN * WRB;         // weight tile bytes
     static constexpr int XT = BM * RB;
     static constexpr int STAGE = WT + XT;
@@ -98,6 +100,7 @@ struct LmCfg {
 using LmCfgA = LmCfg<128, 64, 3>;
 using LmCfgB = LmCfg<256, 32, 4>;
 using LmCfgR = LmCfg<256, 64, 2, true>;
+using LmCfgR192 = LmCfg<192, 64, 2, true>;
 using LmCfgR8 = LmCfg<256, 64, 2, true, true>;  // fp8 weight operand (its tiles fill half a slot)
 using LmCfgA8 = LmCfg<128, 64, 3, false, true>;
 using LmCfgC88 = LmCfg<256, 128, 2, false, false, true>;  // fp8 x fp8 on the block-scaled MFMA: two 64-KiB buffers, the rest of the LDS holds scales
@@ -106,7 +109,7 @@ using LmCfgC88Wide = LmCfg<256, 128, 2, false, false, true, true>;
 
 // configurations whose last tiles may be cut (the 128-row one's ring fits into theirs)
 template <int MODE, class C>
-__host__ __device__ constexpr bool lm_cuts() { return C::RING && !C::W8 && MODE != GEMM_SLICES; }
+__host__ __device__ constexpr bool lm_cuts() { return C::RING && C::BM == 256 && !C::W8 && MODE != GEMM_SLICES; }
 
 // single projections of one matrix, with a bias or not
 template <int MODE>
@@ -524,7 +527,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
 #pragma unroll
             for (int j = 0; j < C::MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         using I0 = std::integral_constant<int, 0>;
-        using I4 = std::integral_constant<int, 4>;
+        using IH = std::integral_constant<int, C::XH>;
 
         if constexpr (C::RING) {
             if (nk > 1) wait_behind_stores(std::integral_constant<int, C::DPW>{});  // K tile 1 stays in flight
@@ -550,7 +553,8 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         // Between tiles: the last fragment read retires before the last barrier but one, and every wave passes the barrier after the
         // loop before it refills the ring.
         if (wid >= 4) __builtin_amdgcn_s_barrier();   // the stagger
-        u32x4_t fw[8], fx[8];  // [k-step][W tile 0-3], [k-step][X tile of the current half]
+        constexpr int XH = C::XH;
+        u32x4_t fw[8], fx[2 * XH];  // [k-step][W tile 0-3], [k-step][X tile of the current half]
         int sxw[8] = {127, 127, 127, 127, 127, 127, 127, 127};  // A8: per X tile, the E8M0 scale bytes of four K tiles (127 = 2^0:
                                                                  // gate|up, whose activation scale is per token)
         int ksh = 0;                                             // 8 * (K tile & 3): the byte of the current K tile
@@ -586,9 +590,9 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             static_for<C::KS>([&](auto ksc) {
                 constexpr int ks = decltype(ksc)::value;
                 const unsigned ax = fbx[ks] + so;
-                static_for<4>([&](auto jc) {
+                static_for<XH>([&](auto jc) {
                     constexpr int j = decltype(jc)::value;
-                    lds_read_b128_o<16 * (mt0 + j) * C::RB>(fx[ks * 4 + j], ax);
+                    lds_read_b128_o<16 * (mt0 + j) * C::RB>(fx[ks * XH + j], ax);
                 });
             });
         };
@@ -610,7 +614,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 }
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) pin(fx[i]);
+            for (int i = 0; i < 2 * XH; ++i) pin(fx[i]);
         };
         // W tiles 0-3 x X tiles m0 .. m0+3, every MFMA sharing an operand with the one before it
         auto mfmas = [&](auto m0c) {
@@ -628,11 +632,11 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                         XBS ? (int)((unsigned)sxw[mt0 + j] >> ksh) : 127);
                 });
             } else {
-                static_for<C::KS * 16>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value, ks = i / 16;
-                    constexpr int t = ks & 1 ? 3 - i / 4 % 4 : i / 4 % 4, j = i / 4 & 1 ? 3 - i % 4 : i % 4;
+                static_for<C::KS * 4 * XH>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value, ks = i / (4 * XH);
+                    constexpr int t = ks & 1 ? 3 - i / XH % 4 : i / XH % 4, j = i / XH & 1 ? XH - 1 - i % XH : i % XH;
                     acc[t][mt0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fw[ks * 4 + t]),
-                                                                              __builtin_bit_cast(bf16x8_t, fx[ks * 4 + j]), acc[t][mt0 + j], 0, 0, 0);
+                                                                              __builtin_bit_cast(bf16x8_t, fx[ks * XH + j]), acc[t][mt0 + j], 0, 0, 0);
                 });
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -667,7 +671,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 if (rows_a) mfmas(I0{});
                 __builtin_amdgcn_s_barrier();
                 // ---- phase B
-                rd_x(ox, I4{});
+                rd_x(ox, IH{});
                 __builtin_amdgcn_sched_barrier(0);
                 if (has2) {
                     if constexpr (C::RING) stage_x(ow, kt + 2);
@@ -679,7 +683,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
                 else if (C::RING && kt == 0) wait_behind_stores(std::integral_constant<int, YOUNGER>{});  // (K tile 1 was issued in front of them)
                 else asm volatile("s_waitcnt vmcnt(%0)" ::"i"(YOUNGER) : "memory");
                 close_load();
-                if (rows_b) mfmas(I4{});
+                if (rows_b) mfmas(IH{});
                 __builtin_amdgcn_s_barrier();
                 if constexpr (C::RING) {
                     of = ox;
@@ -692,7 +696,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         // gate|up, down of 64 experts, 6 of 1024 x 2048 at 6000 tokens 337 / 308, 200 / 186, 8 of 1408 x 4096 at 4096 800 / 774, 445 / 431, at 15074
         // 2181 / 2184, 1258 / 1222.  (The rows dealt anew to both waves along m: 10 to 40 registers spilled, whole tiles 2 to 5 % slower.)
         // A projection without groups has one such block per column tile: there the second loop costs more than it gives (0.3 to 1 %).
-        if (!GROUPED || mcnt_c > 192) k_tiles(std::true_type{}, std::true_type{});
+        if (!GROUPED || C::BM != 256 || mcnt_c > 192) k_tiles(std::true_type{}, std::true_type{});
         else if constexpr (GROUPED) k_tiles(mcnt_c > wm * 128, mcnt_c > wm * 128 + 64);
         if (wid < 4) __builtin_amdgcn_s_barrier();  // match the other group's extra barrier
         } else {
@@ -1228,6 +1232,13 @@ int launch_largem(const GemmParams& p, hipStream_t st) {
         }
     }
     const bool lean = lean_ok && !wide && (var < 0 || var == LM_VAR_LEAN);
+    // One round of 192-row tiles where 256-row ones would leave CUs without work and 128-row ones would be two rounds.  256 / 192, us: 4200 rows of 2048 x 2048 38.4 /
+    // 34.0, x 8192 134 / 120, 4780 38.6 / 36.5, 141 / 132, 6100 42.0 / 39.5, 153 / 145, 3000 of 3072 x 2048 39.1 / 34.6, of 4096 x 4096 81.8 / 76.6, 1300 of 6144 x 2048
+    // 42.3 / 36.0, gated 4096 x 2048 50.4 / 40.7.  Where they are two rounds for one or two with a cut tail, a tile's K step costing seven eighths, 0.95 to 1.1 of the time.
+    if constexpr (lm_single<MODE>() || MODE == GEMM_GLU) {
+        const int64_t cols = (p.N + (gemm_paired(MODE) ? 127 : 255)) / (gemm_paired(MODE) ? 128 : 256);
+        if (lean && use_b && ch == 0 && p.offs == nullptr && (p.R + 191) / 192 * cols <= 256) return launch_largem_cfg<MODE, LmCfgR192, true>(p, st);
+    }
     if (lean) return use_b ? launch_largem_cfg<MODE, LmCfgR, true>(p, st) : launch_largem_cfg<MODE, LmCfgA, true>(p, st);
     if constexpr (MODE == GEMM_QKV) {  // 16-byte-store form only
         glm_set_error("gemm_largem(qkv epilogue): the plain form has no such epilogue");

@@ -1131,6 +1131,28 @@ def test_gemm_large_m_last_round_in_halves(ops, M, N, K):
     assert bool((got[1][0][-1] == 7).all())
 
 
+@pytest.mark.parametrize("M", [3600, 4609, 4704, 4705, 4800, 5376])
+@pytest.mark.parametrize("N,K", [(2064, 64), (2064, 128), (2304, 576)])
+def test_gemm_large_m_one_round_of_192_rows(ops, M, N, K):
+    """192-row tiles that are one round of the chip where 128-row ones are two: last row blocks of every third of a wave's rows and one row more, columns that end inside a
+    tile; every epilogue a projection without experts has, bit for bit against the plain form, in buffers that stay as they were around it."""
+    assert -(-M // 128) * 9 > 256 >= -(-M // 192) * 9
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    b = torch.randn(N, device="cuda", generator=g).to(BF)
+    got = []
+    for v in (0, -1):
+        with largem_variant(v):
+            out, f32 = torch.full((M + 2, N), 7.0, device="cuda", dtype=BF), torch.full((M + 2, N), 7.0, device="cuda")
+            ops.linear_act(x, w, b, out=out[1: M + 1])
+            ops.linear_act(x, w, out_f32=True, out=f32[1: M + 1])
+            got.append([out, f32, ops.gated_glu(x, w, 2.0)] + [ops.linear_act(x, w, act=a, out_f32=f) for f in (False, True) for a in (
+                (ops.ACT_XIELU, 0.8, 0.7), (ops.ACT_SOFTCAP, 3.0, 0.0), (ops.ACT_GATE, 264.0, 0.0), (ops.ACT_SILU_GATE, 264.0, 0.0), (ops.ACT_RELU2_GATE, 264.0, 520.0))])
+    assert all(torch.equal(a, c) for a, c in zip(*got))
+    assert all(bool((t[0] == 7).all()) and bool((t[-1] == 7).all()) for t in got[1][:2])
+
+
 @pytest.mark.parametrize("M", LAST_BLOCKS)
 def test_expanded_fp8_weights_last_round_in_halves(ops, M):
     """One expert whose fp8 weights are expanded, row scales on the accumulators: its last tiles go in halves too."""
@@ -1313,6 +1335,28 @@ def test_qkv_gemm_with_rope_store_last_round_in_halves(ops, T, nh, nkv, K):
     q0, k0, v0 = ops.qkv_split_norm_rope_store(ops.gemm_bf16(x, w, b), nh, nkv, 128, pos, cs, 64, None, None, 1e-5, None, None, None, True)
     q1, k1, v1 = ops.gemm_qkv_rope_store(x, w, b, nh, nkv, 128, pos, cs, 64, None, None, None, True)
     assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0, v1)
+
+
+@pytest.mark.parametrize("T", [3300, 4609, 4704, 4800])
+def test_qkv_gemm_with_rope_store_one_round_of_192_rows(ops, T):
+    """The fused QKV projection on 192-row tiles == the projection on them and the split / rotary kernel, bit for bit, and the projection == its plain form."""
+    nh, nkv, K, bs = 16, 2, 192, 64
+    assert -(-T // 128) * 10 > 256 >= -(-T // 192) * 10
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, K, device="cuda", generator=g).to(BF)
+    w = (torch.randn((nh + 2 * nkv) * 128, K, device="cuda", generator=g) * K ** -0.5).to(BF)
+    b = torch.randn(w.shape[0], device="cuda", generator=g).to(BF)
+    pos = torch.randint(0, 512, (T,), device="cuda", generator=g)
+    slots = torch.randperm(-(-T // bs) * bs, device="cuda", generator=g)[:T].to(torch.int32)
+    slots[::7] = -1
+    cs = dev(O.build_cos_sin_cache(64, 512, 10000.0).reshape(512, 64).contiguous())
+    y = ops.gemm_bf16(x, w, b)
+    with largem_variant(0):
+        assert torch.equal(y, ops.gemm_bf16(x, w, b))
+    kv = [[torch.full((-(-T // bs), bs, nkv, 128), 7.0, device="cuda", dtype=BF) for _ in range(2)] for _ in range(2)]
+    want = ops.qkv_split_norm_rope_store(y, nh, nkv, 128, pos, cs, 64, None, None, 1e-5, *kv[0], slots, True)
+    got = ops.gemm_qkv_rope_store(x, w, b, nh, nkv, 128, pos, cs, 64, *kv[1], slots, True)
+    assert all(torch.equal(a, c) for a, c in zip(want, got)) and all(torch.equal(a, c) for a, c in zip(*kv))
 
 
 @pytest.mark.parametrize("last", [1, 63, 64, 65, 128, 129, 192, 193])
