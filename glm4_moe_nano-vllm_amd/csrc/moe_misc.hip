@@ -553,86 +553,103 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// Bucketing at prefill sizes (T k >= ALIGN_PAR_MIN_PAIRS): the single-workgroup kernel above walks 131072 pairs in 128
-// serial rounds (200 us at T = 16384).  Three launches over chunks of ALIGN_CHUNK pairs instead:
-//   count:   chunk c histograms its pairs in LDS and reserves, per expert, a range inside the expert's group with ONE
-//            global add per (chunk, expert): base[c][e] = atomicAdd(total[e], hist[e])  (total[] zeroed by the host side)
-//   offsets: exclusive scan of total[] -> expert_offsets (one wave)
-//   scatter: chunk c redoes its LDS ranking from expert_offsets[e] + base[c][e] and writes the rows.
-// Rows of one expert end up in arrival order of the chunks' adds — as with the LDS atomics of the small kernel the order
-// inside a group is not specified (no consumer depends on it: pair_pos carries the permutation).
-constexpr int ALIGN_CHUNK = 8192;  // pairs per workgroup (8 per thread)
+// Bucketing of many pairs: the single-workgroup kernel above walks 131072 of them in 128 serial rounds (200 us at T = 16384).  Two launches over chunks of
+// ALIGN_CHUNK pairs instead:
+//   count:   chunk c's pairs per expert, counted in LDS -> counts[c][e]
+//   scatter: chunk c adds up all chunks' counts (E per chunk, from the caches), which gives the experts' places and its own places in them, ranks
+//            its pairs once more in LDS and writes the rows; chunk 0 writes expert_offsets.
+// (Totals reserved by atomics in a zeroed array and scanned by a launch of their own, four launches over chunks of 8192 / this, us: 64 experts 6000 pairs 13.1 / 6.4,
+// 33000 16.3 / 7.0, 131072 16.9 / 8.0, 256 experts 33000 14.9 / 8.7, 131072 15.2 / 11.5.)
+// Rows of one expert are in the order of the chunks, inside a chunk in that of its LDS atomics (not specified: pair_pos carries the permutation).
+constexpr int ALIGN_CHUNK = 2048;  // pairs per workgroup (two per thread)
 
-__global__ __launch_bounds__(1024) void moe_align_count_kernel(const int64_t* __restrict__ topk_idx, int64_t P, int E,
-                                                               int32_t* __restrict__ total, int32_t* __restrict__ base) {
+__global__ __launch_bounds__(1024) void moe_align_count_kernel(const int64_t* __restrict__ topk_idx, int64_t P, int E, int32_t* __restrict__ counts) {
     __shared__ int hist[ALIGN_MAX_G];
     const int tid = threadIdx.x;
-    for (int e = tid; e < E; e += 1024) hist[e] = 0;
-    __syncthreads();
     const int64_t p0 = (int64_t)blockIdx.x * ALIGN_CHUNK;
+    int64_t e[ALIGN_CHUNK / 1024];
 #pragma unroll
-    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) {
-        const int64_t p = p0 + i * 1024 + tid;
-        if (p < P) {
-            const int64_t e = topk_idx[p];
-            if (e >= 0 && e < E) atomicAdd(&hist[(int)e], 1);
-        }
-    }
+    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) e[i] = p0 + i * 1024 + tid < P ? topk_idx[p0 + i * 1024 + tid] : -1;
+    for (int g = tid; g < E; g += 1024) hist[g] = 0;
     __syncthreads();
-    for (int e = tid; e < E; e += 1024) {
-        const int c = hist[e];
-        base[(int64_t)blockIdx.x * E + e] = c ? atomicAdd(&total[e], c) : 0;
-    }
-}
-
-__global__ __launch_bounds__(64) void moe_align_offsets_kernel(const int32_t* __restrict__ total, int E, int64_t T,
-                                                               int with_shared, int32_t* __restrict__ expert_offsets) {
-    const int lane = threadIdx.x;
-    int run = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-        const int e = e0 + lane;
-        const int c = e < E ? total[e] : 0;
-        const int incl = wave_scan_incl(c);
-        if (e < E) expert_offsets[e] = run + incl - c;
-        run += __builtin_amdgcn_readlane(incl, 63);
-    }
-    if (lane == 0) {
-        expert_offsets[E] = run;
-        if (with_shared) expert_offsets[E + 1] = run + (int)T;
-    }
+#pragma unroll
+    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i)
+        if (e[i] >= 0 && e[i] < E) atomicAdd(&hist[(int)e[i]], 1);
+    __syncthreads();
+    for (int g = tid; g < E; g += 1024) counts[(int64_t)blockIdx.x * E + g] = hist[g];
 }
 
 __global__ __launch_bounds__(1024) void moe_align_scatter_kernel(
-    const int64_t* __restrict__ topk_idx, const bf16_t* __restrict__ topk_w, const int32_t* __restrict__ expert_offsets,
-    const int32_t* __restrict__ base, int32_t* __restrict__ sorted_token, bf16_t* __restrict__ sorted_scale,
-    int32_t* __restrict__ pair_pos, int64_t T, int k, int E, int with_shared) {
-    __shared__ int cur[ALIGN_MAX_G];
-    const int tid = threadIdx.x;
-    const int64_t P = T * k;
-    for (int e = tid; e < E; e += 1024) cur[e] = expert_offsets[e] + base[(int64_t)blockIdx.x * E + e];
-    __syncthreads();
-    const int64_t p0 = (int64_t)blockIdx.x * ALIGN_CHUNK;
+    const int64_t* __restrict__ topk_idx, const bf16_t* __restrict__ topk_w, const int32_t* __restrict__ counts, int32_t* __restrict__ expert_offsets,
+    int32_t* __restrict__ sorted_token, bf16_t* __restrict__ sorted_scale, int32_t* __restrict__ pair_pos, int64_t T, int k, int E, int with_shared) {
+    __shared__ int cur[ALIGN_MAX_G], all[ALIGN_MAX_G], s_run;
+    const int tid = threadIdx.x, chunks = gridDim.x, me = blockIdx.x;
+    const int64_t P = T * k, p0 = (int64_t)me * ALIGN_CHUNK;
+    int64_t ex[ALIGN_CHUNK / 1024];
+    bf16_t wt[ALIGN_CHUNK / 1024];
 #pragma unroll
     for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) {
         const int64_t p = p0 + i * 1024 + tid;
-        if (p < P) {
-            const int64_t e = topk_idx[p];
-            if (e >= 0 && e < E) {
-                const int pos = atomicAdd(&cur[(int)e], 1);
-                sorted_token[pos] = (int32_t)(p / k);
-                if (sorted_scale) sorted_scale[pos] = topk_w[p];
-                pair_pos[p] = pos;
-            } else {
-                pair_pos[p] = -1;
+        ex[i] = p < P ? topk_idx[p] : -1;
+        wt[i] = p < P && sorted_scale ? topk_w[p] : (bf16_t)0;
+    }
+    for (int e = tid; e < E; e += 1024) cur[e] = all[e] = 0;
+    __syncthreads();
+    // a wave adds up every 16th chunk for 64 experts at a time
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = e0 + (tid & 63);
+        int sum = 0, before = 0;
+        if (e < E) {
+#pragma unroll 8
+            for (int c = tid >> 6; c < chunks; c += 16) {
+                const int n = counts[(int64_t)c * E + e];
+                sum += n;
+                before += c < me ? n : 0;
+            }
+            if (sum) atomicAdd(&all[e], sum);
+            if (before) atomicAdd(&cur[e], before);
+        }
+    }
+    __syncthreads();
+    if (tid < 64) {  // exclusive scan of the counts, 64 experts at a time
+        int run = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + tid;
+            const int c = e < E ? all[e] : 0;
+            const int incl = wave_scan_incl(c);
+            if (e < E) {
+                cur[e] += run + incl - c;
+                if (me == 0) expert_offsets[e] = run + incl - c;
+            }
+            run += __builtin_amdgcn_readlane(incl, 63);
+        }
+        if (tid == 0) {
+            s_run = run;
+            if (me == 0) {
+                expert_offsets[E] = run;
+                if (with_shared) expert_offsets[E + 1] = run + (int)T;
             }
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) {
+        const int64_t p = p0 + i * 1024 + tid;
+        if (p >= P) continue;
+        if (ex[i] >= 0 && ex[i] < E) {
+            const int pos = atomicAdd(&cur[(int)ex[i]], 1);
+            sorted_token[pos] = (int32_t)(p / k);
+            if (sorted_scale) sorted_scale[pos] = wt[i];
+            pair_pos[p] = pos;
+        } else {
+            pair_pos[p] = -1;
+        }
+    }
     if (with_shared) {  // the shared group's rows of this chunk's token range
-        const int sbase = expert_offsets[E];
-        const int64_t t0 = (int64_t)blockIdx.x * ALIGN_CHUNK;  // chunks outnumber ceil(T / ALIGN_CHUNK): k >= 1
+        const int64_t t0 = (int64_t)me * ALIGN_CHUNK;  // chunks outnumber ceil(T / ALIGN_CHUNK): k >= 1
         for (int64_t t = t0 + tid; t < min(T, t0 + ALIGN_CHUNK); t += 1024) {
-            sorted_token[sbase + t] = (int32_t)t;
-            sorted_scale[sbase + t] = 0x3F80;  // bf16 1.0
+            sorted_token[s_run + t] = (int32_t)t;
+            sorted_scale[s_run + t] = 0x3F80;  // bf16 1.0
         }
     }
 }
@@ -1055,12 +1072,11 @@ extern "C" int glm_moe_align(const int64_t* topk_idx, const void* topk_w, int32_
 
 extern "C" size_t glm_moe_align_workspace_bytes(int64_t T, int k, int E) {
     const int64_t P = (T > 0 ? T : 0) * (int64_t)(k > 0 ? k : 0);
-    const int64_t chunks = (P + ALIGN_CHUNK - 1) / ALIGN_CHUNK;
-    return (size_t)(E > 0 ? E : 0) * sizeof(int32_t) * (size_t)(1 + chunks);
+    const int64_t chunks = P > 0 ? (P + ALIGN_CHUNK - 1) / ALIGN_CHUNK : 1;
+    return (size_t)(E > 0 ? E : 0) * sizeof(int32_t) * (size_t)chunks;
 }
 
-// glm_moe_align over many workgroups (prefill sizes).  workspace: glm_moe_align_workspace_bytes(T, k, E), its first E
-// words (the per-expert totals) ZERO on entry — the caller clears them (hipMemsetAsync / a zeroed tensor) per call.
+// glm_moe_align over many workgroups.  workspace: glm_moe_align_workspace_bytes(T, k, E), whatever it holds on entry.
 extern "C" int glm_moe_align_parallel(const int64_t* topk_idx, const void* topk_w, int32_t* expert_offsets,
                                       int32_t* sorted_token, void* sorted_scale, int32_t* pair_pos, int64_t T, int k,
                                       int E, int with_shared, int32_t* workspace, size_t workspace_bytes,
@@ -1073,16 +1089,11 @@ extern "C" int glm_moe_align_parallel(const int64_t* topk_idx, const void* topk_
     GLM_CHECK_ARG(workspace_bytes >= glm_moe_align_workspace_bytes(T, k, E), GLM_ERR_WORKSPACE,
                   "glm_moe_align_parallel: workspace %zu < %zu bytes", workspace_bytes, glm_moe_align_workspace_bytes(T, k, E));
     const int64_t P = T * k;
-    const unsigned chunks = (unsigned)((P + ALIGN_CHUNK - 1) / ALIGN_CHUNK);
+    const unsigned chunks = P > 0 ? (unsigned)((P + ALIGN_CHUNK - 1) / ALIGN_CHUNK) : 1;   // (of no pairs one that writes the offsets)
     hipStream_t st = glm_s(stream);
-    int32_t* total = workspace;
-    int32_t* base = workspace + E;
-    if (chunks > 0)
-        hipLaunchKernelGGL(moe_align_count_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, P, E, total, base);
-    hipLaunchKernelGGL(moe_align_offsets_kernel, dim3(1), dim3(64), 0, st, total, E, T, with_shared, expert_offsets);
-    if (chunks > 0)
-        hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, (const bf16_t*)topk_w,
-                           expert_offsets, base, sorted_token, (bf16_t*)sorted_scale, pair_pos, T, k, E, with_shared);
+    hipLaunchKernelGGL(moe_align_count_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, P, E, workspace);
+    hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, (const bf16_t*)topk_w, workspace, expert_offsets, sorted_token,
+                       (bf16_t*)sorted_scale, pair_pos, T, k, E, with_shared);
     GLM_CHECK_LAUNCH("glm_moe_align_parallel");
     return GLM_OK;
 }

@@ -789,7 +789,9 @@ def add_rmsnorm_router_topk(x, residual: torch.Tensor, norm_weight: torch.Tensor
     return y.view(residual.shape), ro.view(residual.shape), idx, w
 
 
-ALIGN_PARALLEL_MIN_PAIRS = 16384  # from here on the one-workgroup bucketing kernel is the slower one (200 us at 131072 pairs)
+# from here on the one-workgroup bucketing kernel is the slower one; one / many, us: 64 experts 4096 pairs 6.4 / 6.3, 6000 8.7 / 6.4, without weights 4.6 / 5.2, 6.0 / 5.3,
+# 256 experts 6000 7.0 / 7.3, 8192 8.9 / 7.3
+ALIGN_PARALLEL_MIN_PAIRS = 5120
 
 
 def moe_align(topk_idx: torch.Tensor, topk_w: torch.Tensor | None, E: int, with_shared: bool):
@@ -802,9 +804,9 @@ def moe_align(topk_idx: torch.Tensor, topk_w: torch.Tensor | None, E: int, with_
     tok = torch.empty(R, dtype=torch.int32, device=dev)
     scale = torch.empty(R, dtype=torch.bfloat16, device=dev) if topk_w is not None else None
     pos = torch.empty(T * k, dtype=torch.int32, device=dev)
-    if T * k >= ALIGN_PARALLEL_MIN_PAIRS:  # prefill sizes: count / offsets / scatter over many workgroups
+    if T * k >= ALIGN_PARALLEL_MIN_PAIRS:  # prefill sizes: count / scatter over many workgroups
         lib = load_library()
-        ws = torch.zeros(lib.glm_moe_align_workspace_bytes(T, k, E) // 4, dtype=torch.int32, device=dev)
+        ws = torch.empty(lib.glm_moe_align_workspace_bytes(T, k, E) // 4, dtype=torch.int32, device=dev)
         _check(lib.glm_moe_align_parallel(_p(topk_idx), _p(topk_w), _p(offs), _p(tok), _p(scale), _p(pos), T, k, E,
                                           1 if with_shared else 0, _p(ws), ws.numel() * 4, _stream()),
                "glm_moe_align_parallel")

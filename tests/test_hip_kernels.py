@@ -537,6 +537,28 @@ def test_moe_align_parallel(ops, T, k, E, shared):
         assert int(offs[E + 1]) == P + T and tok[P:].tolist() == list(range(T)) and bool((scale[P:].float() == 1.0).all())
 
 
+@pytest.mark.parametrize("T,k,E,shared", [(5120, 1, 1000, False), (1025, 5, 64, True), (3072, 2, 63, True), (6145, 1, 65, True), (700, 8, 256, False), (20000, 3, 200, True)])
+def test_moe_align_parallel_chunks(ops, T, k, E, shared):
+    """Chunks that are whole, end by one pair or hold one pair, experts that fill several passes, pairs without an expert, a workspace of whatever values."""
+    assert T * k >= ops.ALIGN_PARALLEL_MIN_PAIRS
+    g = torch.Generator().manual_seed(T)
+    idx = torch.randint(0, E, (T, k), generator=g) if k == 1 else torch.rand(T, E, generator=g).topk(k, -1).indices
+    idx[::97, 0] = -1
+    w = (torch.rand(T, k, generator=g) + 0.1).to(BF)
+    junk = torch.full((1 << 20,), -77, dtype=torch.int32, device="cuda")
+    del junk     # (what the workspace may be made of)
+    offs, tok, scale, pos = [a.cpu() for a in ops.moe_align(dev(idx), dev(w), E, shared)]
+    flat, ok = idx.flatten(), idx.flatten() >= 0
+    n = int(ok.sum())
+    assert torch.equal(offs[: E + 1].long(), torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(flat[ok], minlength=E).cumsum(0)]))
+    assert bool((pos[~ok] == -1).all()) and sorted(pos[ok].tolist()) == list(range(n))
+    p = pos[ok].long()
+    assert torch.equal(torch.bucketize(p, offs[1: E + 1].long(), right=True), flat[ok])
+    assert torch.equal(tok[p].long(), (torch.arange(T * k) // k)[ok]) and torch.equal(scale[p], w.flatten()[ok])
+    if shared:
+        assert int(offs[E + 1]) == n + T and tok[n: n + T].tolist() == list(range(T)) and bool((scale[n: n + T].float() == 1.0).all())
+
+
 def test_moe_align(ops):
     T, k, E = 37, 4, 16
     g = torch.Generator().manual_seed(41)
