@@ -164,10 +164,6 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
             if (k < dm) S.qf[t][i] = *reinterpret_cast<const u32x4_t*>(qp + k);
         }
     }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < KQ; ++i) asm volatile("" : "+v"(S.qf[t][i]));
     const unsigned base = lds_addr(smem);
     // Sources of the DMA pieces: piece i of a wave holds 64 / CPR rows from 16 w + i 64 / CPR on, and the chunk permutation repeats after eight
     // rows: offsets of the pieces of eight rows, from two bases.  Tiles whose rows are all there, without padding columns, take addresses (a few per cent
@@ -216,12 +212,18 @@ __global__ __launch_bounds__(256, (DK + DV) <= 256 ? 2 : 1) void group_attn_pref
     // before it asks again)
     const int blk0 = ga_uniform(block_of(0)), blk1 = ga_uniform(block_of(1));
     int blk = -1;
-    attn_tiles<DK, DV, F, KDMA + VDMA>(S, base, n, jlo, g, sc, F == GA_SOFTMAX && a.slope != nullptr, [&](int it, auto startc) {
+    auto bring = [&](int it, auto startc) __attribute__((always_inline)) {
         if constexpr (decltype(startc)::value == 0) issue(0, blk0);
         else if constexpr (decltype(startc)::value == 1) issue(1, blk1);
         else issue(it, ga_uniform(blk));
         if constexpr (decltype(startc)::value != 0) blk = block_of(it + 1);
-    });
+    };
+    bring(0, std::integral_constant<int, 0>{});   // in front of the wait for the queries
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < KQ; ++i) asm volatile("" : "+v"(S.qf[t][i]));
+    attn_tiles<DK, DV, F, KDMA + VDMA>(S, base, n, jlo, g, sc, F == GA_SOFTMAX && a.slope != nullptr, bring);
     if constexpr (TWO) {
         // both maps of a row are in the same lane: their difference and its norm over the head's columns (padding columns are zeros)
         const float i0 = 1.0f / S.mass(0), i1 = a.lam / S.mass(1);

@@ -60,47 +60,6 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
     const int qlast = min(qo + 127, nq - 1);
     const int jlo = max(0, hist + qo - a.window + 1), jhi = hist + qlast;
     const int n = (jhi - jlo + 64) >> 6;
-    // The walk hides keys and takes maxima in front of the scale, which has to be positive there: the queries take its sign, and are zeros where it is zero.
-    const unsigned sign = a.scale < 0.f ? 0x80008000u : 0u, keep = a.scale == 0.f ? 0u : ~0u;
-    const float scale = a.scale == 0.f ? 1.f : fabsf(a.scale);
-    // this wave's rows: tile t holds rows qo + 64 t + 16 w + c (the two half-dead tiles of the causal edge cost all waves the same)
-    SL S;
-    S.init(lane);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int r0 = qo + 64 * t + 16 * w, r = r0 + c;
-        const bool some = r0 < nq;
-        const int a0 = hist + r0, a1 = hist + min(r0 + 15, nq - 1);
-        S.rp[t] = r < nq ? hist + r : -1;      // key index of the row itself
-        S.rlo[t] = S.rp[t] - a.window + 1;
-        S.any_lo[t] = some ? a0 - a.window + 1 : 1 << 30;
-        S.any_hi[t] = some ? a1 : -1;
-        S.full_lo[t] = some ? a1 - a.window + 1 : 1 << 30;
-        S.full_hi[t] = some ? a0 : -1;
-        const bf16_t* qp = a.q + (int64_t)(qs + min(r, nq - 1)) * a.ldq + (int64_t)h * a.dk;
-#pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            const int k = 32 * i + 8 * g;
-            S.qf[t][i] = u32x4_t{0, 0, 0, 0};
-            if (k < a.dk) S.qf[t][i] = *reinterpret_cast<const u32x4_t*>(qp + k);
-            if (k >= a.dkn && k < a.dk) {  // rotated here: a lane holds whole pairs
-                const float* cs = a.cs + (int64_t)(qs + min(r, nq - 1)) * (a.dk - a.dkn) + (k - a.dkn);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float u = bflo(S.qf[t][i][j]), v = bfhi(S.qf[t][i][j]), co = cs[2 * j], si = cs[2 * j + 1];
-                    S.qf[t][i][j] = pack2bf(u * co - v * si, v * co + u * si);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < KS; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) S.qf[t][i][j] = (S.qf[t][i][j] & keep) ^ sign;
-            asm volatile("" : "+v"(S.qf[t][i]));
-        }
     const unsigned base = lds_addr(smem);
     const bf16_t* kbase = a.k + (int64_t)(ks0 + jlo) * a.ldkv + (int64_t)h * a.dkn;
     const bf16_t* rbase = a.kr ? a.kr + (int64_t)(ks0 + jlo) * a.ldr : kbase;
@@ -174,6 +133,48 @@ __global__ __launch_bounds__(256, (DK + DV) <= 320 ? 2 : 1) void window_attn_ker
                 lds_dma16(attn_rows(vb + (int64_t)(i / VPER) * 8 * kvb, left - 8 * (i / VPER), kvb), voff[i % VPER], st + KTILE + (w * VDMA + i) * 1024);
         }
     };
+    issue(0, std::integral_constant<int, 0>{});   // in front of everything that waits for the queries
+    // The walk hides keys and takes maxima in front of the scale, which has to be positive there: the queries take its sign, and are zeros where it is zero.
+    const unsigned sign = a.scale < 0.f ? 0x80008000u : 0u, keep = a.scale == 0.f ? 0u : ~0u;
+    const float scale = a.scale == 0.f ? 1.f : fabsf(a.scale);
+    // this wave's rows: tile t holds rows qo + 64 t + 16 w + c (the two half-dead tiles of the causal edge cost all waves the same)
+    SL S;
+    S.init(lane);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int r0 = qo + 64 * t + 16 * w, r = r0 + c;
+        const bool some = r0 < nq;
+        const int a0 = hist + r0, a1 = hist + min(r0 + 15, nq - 1);
+        S.rp[t] = r < nq ? hist + r : -1;      // key index of the row itself
+        S.rlo[t] = S.rp[t] - a.window + 1;
+        S.any_lo[t] = some ? a0 - a.window + 1 : 1 << 30;
+        S.any_hi[t] = some ? a1 : -1;
+        S.full_lo[t] = some ? a1 - a.window + 1 : 1 << 30;
+        S.full_hi[t] = some ? a0 : -1;
+        const bf16_t* qp = a.q + (int64_t)(qs + min(r, nq - 1)) * a.ldq + (int64_t)h * a.dk;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int k = 32 * i + 8 * g;
+            S.qf[t][i] = u32x4_t{0, 0, 0, 0};
+            if (k < a.dk) S.qf[t][i] = *reinterpret_cast<const u32x4_t*>(qp + k);
+            if (k >= a.dkn && k < a.dk) {  // rotated here: a lane holds whole pairs
+                const float* cs = a.cs + (int64_t)(qs + min(r, nq - 1)) * (a.dk - a.dkn) + (k - a.dkn);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float u = bflo(S.qf[t][i][j]), v = bfhi(S.qf[t][i][j]), co = cs[2 * j], si = cs[2 * j + 1];
+                    S.qf[t][i][j] = pack2bf(u * co - v * si, v * co + u * si);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) S.qf[t][i][j] = (S.qf[t][i][j] & keep) ^ sign;
+            asm volatile("" : "+v"(S.qf[t][i]));
+        }
     attn_tiles<DK, DV, GA_SOFTMAX, KDMA + VDMA>(S, base, n, jlo, g, scale * GA_LOG2E, false, issue);
     const float sk = a.sink[h] * GA_LOG2E;
 #pragma unroll
