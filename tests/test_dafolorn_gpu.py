@@ -370,6 +370,30 @@ def test_window_attn_prefill(H, dk, dv, window):
             assert (got[qs[s]: qs[s + 1], h] - ref).abs().max() < 4e-2, (s, h)
 
 
+@pytest.mark.parametrize("H,dk,dv", [(2, 128, 128), (3, 24, 40), (2, 192, 128), (1, 256, 256), (2, 72, 104)])
+def test_window_attn_prefill_gate(H, dk, dv):
+    """Rows behind whole tiles and heads narrower than theirs, gates in rows of a pitch of their own."""
+    from nanovllm import hip_ops
+    lens, window = [129, 1, 64, 273], 90
+    qs = [0, 129, 130, 194, 467]
+    T = qs[-1]
+    q, k, v = (torch.randn(T, H * d, generator=g(i)).to(torch.bfloat16) for i, d in ((1, dk), (2, dk), (3, dv)))
+    sink, kv = dev(torch.randn(H, generator=g(4))), torch.cat([k, v], 1).cuda()
+    wide = torch.randn(T, H * dv + 12, generator=g(5)).to(torch.bfloat16)
+    gate = dev(wide)[:, 4: 4 + H * dv]
+    tiles = [(s, o) for s, n in enumerate(lens) for o in range(0, n, 128)]
+    got = []
+    for gt in (None, gate):
+        out = torch.full((T, H * dv + 4), float("nan"), dtype=torch.bfloat16, device="cuda")
+        hip_ops.window_attn_prefill(dev(q), kv[:, : H * dk], kv[:, H * dk:], out[:, : H * dv], i32(qs), i32(qs), i32([t[0] for t in tiles]), i32([t[1] for t in tiles]), H, dk, dv,
+                                    window, dk ** -0.5, sink, gate=gt)
+        assert out[:, H * dv:].isnan().all()
+        got.append(out[:, : H * dv].cpu().double())
+    # the same sums in 32 bits, rounded to bf16 once in front of the factor (here) and once behind it: 2 ** -8 of the value each, at most
+    ref = got[0] * wide[:, 4: 4 + H * dv].double()
+    assert ((got[1] - ref).abs() <= 2 ** -7 * ref.abs() + 1e-30).all()
+
+
 @pytest.mark.parametrize("H,dk,dv", [(2, 128, 128), (3, 24, 40), (2, 192, 128), (1, 256, 256)])
 @pytest.mark.parametrize("scale", [-0.3, 0.0, -0.0, -1e-40, 1e-40])
 def test_window_attn_prefill_any_scale(H, dk, dv, scale):
