@@ -167,14 +167,21 @@ __device__ __forceinline__ float dn_part_rms(const DepthArgs& a, const Col8& v, 
     }
     return 1.0f / sqrtf(q / (float)a.gs + a.eps);
 }
-// x_out and x_next of one row (the row of x_in, y and the depths), the loads together
+struct DepthRow {   // of one row: x_in, the first four depths
+    Col8 x, e0[4];
+};
 template <bool VEC>
-__device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, int nc, int lane, int wid, float (*s_red)[16], int& par, Col8& x, Col8& xn) {
-    x = dn_ldf<VEC>(a.x_in + row * a.ld + c, nc);
+__device__ __forceinline__ void dn_fetch(const DepthArgs& a, int64_t row, int c, int nc, DepthRow& f) {
+    f.x = dn_ldf<VEC>(a.x_in + row * a.ld + c, nc);
     const float* d = a.depth ? a.depth + row * a.ld + c : nullptr;
-    Col8 e0[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) e0[u] = a.depth && u < a.n_depth ? dn_ldf<VEC>(d + u * a.depth_stride, nc) : dn_zero();
+    for (int u = 0; u < 4; ++u) f.e0[u] = a.depth && u < a.n_depth ? dn_ldf<VEC>(d + u * a.depth_stride, nc) : dn_zero();
+}
+// x_out and x_next of one row (f of x_in, y and the depths), the loads together
+template <bool VEC>
+__device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, int nc, int lane, int wid, float (*s_red)[16], int& par, const DepthRow& f, Col8& x, Col8& xn) {
+    x = f.x;
+    const float* d = a.depth ? a.depth + row * a.ld + c : nullptr;
     if (a.y) {
         Col8 y = dn_zero();
         if (!a.pair_pos) {
@@ -220,7 +227,7 @@ __device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, i
     for (int u = 0; u < 4; ++u)
         if (u < a.n_depth) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) avg.v[i] = fmaf(a.coef[u], e0[u].v[i], avg.v[i]);
+            for (int i = 0; i < 8; ++i) avg.v[i] = fmaf(a.coef[u], f.e0[u].v[i], avg.v[i]);
         }
     for (int j = 4; j < a.n_depth; j += 4) {
         Col8 e[4];
@@ -239,16 +246,26 @@ __device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, i
 }
 
 // One row per workgroup.  TAPS > 1: with the convolution, for which the TAPS-1 rows in front are computed as well, as far as they are of
-// this step.
-template <int TAPS, bool VEC>
-__global__ __launch_bounds__(1024) void depth_norm_kernel(const DepthArgs a) {
+// this step.  What bounds it with few rows is a chain of trips to memory.  Up to 512 threads and four taps (NT, with registers for it) the row, the depths and the taps are requested
+// in front of the sequence's tables, not behind them and not behind the stores: behind k = 6 experts and one to three depths, four taps, in a step, us: 100 rows of 2048 10.8 / 9.2, 9 rows
+// 10.2 / 8.8, 60 rows of 4096 13.3 / 10.5, without experts 7.8 / 6.3, 300 rows of two prompts, each with the three in front of it, 19.2 / 18.5.
+template <int TAPS, bool VEC, int NT>
+__global__ __launch_bounds__(NT) void depth_norm_kernel(const DepthArgs a) {
     constexpr int HALO = TAPS - 1;
+    constexpr bool EARLY = NT <= 512;
     __shared__ float s_red[2][16];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     int c, nc, par = 0;
     dn_columns(a, lane, wid, c, nc);
     const int64_t r = blockIdx.x;
     Col8 x, xn, hist[TAPS];
+    DepthRow f;
+    u32x4_t wk[TAPS];
+    if constexpr (EARLY) {
+        dn_fetch<VEC>(a, r, c, nc, f);   // (the convolution's rows are not gathered)
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) wk[k] = *reinterpret_cast<const u32x4_t*>(a.conv_w + (int64_t)k * a.wp + c);
+    }
     int s = 0, qs = 0, qe = 0;
     int64_t sin = 0, lo = r;
     if constexpr (TAPS > 1) {
@@ -262,13 +279,17 @@ __global__ __launch_bounds__(1024) void depth_norm_kernel(const DepthArgs a) {
         for (int k = 1; k < TAPS; ++k)  // what lies in front of the portion
             hist[k - 1] = dn_ldf<VEC>(a.state + (sin * HALO + (r - k < qs ? HALO - (qs - (r - k)) : 0)) * a.wp + c, p - k >= 0 && r - k < qs ? nc : 0);
         for (int64_t q = lo; q < r; ++q) {
-            dn_row<VEC>(a, q, c, nc, lane, wid, s_red, par, x, xn);
+            DepthRow e;
+            dn_fetch<VEC>(a, q, c, nc, e);
+            dn_row<VEC>(a, q, c, nc, lane, wid, s_red, par, e, x, xn);
 #pragma unroll
             for (int k = 1; k < TAPS; ++k)
                 if (r - q == k) hist[k - 1] = xn;
         }
     }
-    dn_row<VEC>(a, a.row_index ? (int64_t)a.row_index[r] : r, c, nc, lane, wid, s_red, par, x, xn);
+    const int64_t row = TAPS == 1 && a.row_index ? (int64_t)a.row_index[r] : r;
+    if constexpr (!EARLY) dn_fetch<VEC>(a, row, c, nc, f);
+    dn_row<VEC>(a, row, c, nc, lane, wid, s_red, par, f, x, xn);
     if (a.x_out) dn_stf<VEC>(a.x_out + r * a.ld + c, x, nc);
     if (a.x_cast) dn_st<VEC>(a.x_cast, r * a.ldc + c, a.act_f32, x, nc);
     if (a.depth && a.x_next) dn_stf<VEC>(a.x_next + r * a.ld + c, xn, nc);
@@ -295,7 +316,16 @@ __global__ __launch_bounds__(1024) void depth_norm_kernel(const DepthArgs a) {
         Col8 acc = dn_zero();
 #pragma unroll
         for (int k = HALO; k >= 0; --k) {
-            const Col8 w = dn_ldh<VEC>(a.conv_w + (int64_t)(TAPS - 1 - k) * a.wp + c, nc);
+            Col8 w;
+            if constexpr (EARLY) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    w.v[2 * i] = bflo(wk[TAPS - 1 - k][i]);
+                    w.v[2 * i + 1] = bfhi(wk[TAPS - 1 - k][i]);
+                }
+            } else {
+                w = dn_ldh<VEC>(a.conv_w + (int64_t)(TAPS - 1 - k) * a.wp + c, nc);
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc.v[i] = acc.v[i] + w.v[i] * (k ? hist[k ? k - 1 : 0].v[i] : xn.v[i]);
         }
@@ -455,8 +485,15 @@ int launch_depth_norm(const DepthArgs& a, int nt, bool vec, hipStream_t st) {
             return launch_depth_conv<TAPS>(a, xs, st);
         }
     }
-    if (vec) hipLaunchKernelGGL((depth_norm_kernel<TAPS, true>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
-    else hipLaunchKernelGGL((depth_norm_kernel<TAPS, false>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
+    if constexpr (TAPS > 1 && TAPS <= 4) {
+        if (vec && nt <= 512) {
+            hipLaunchKernelGGL((depth_norm_kernel<TAPS, true, 512>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
+            GLM_CHECK_LAUNCH("glm_depth_norm");
+            return GLM_OK;
+        }
+    }
+    if (vec) hipLaunchKernelGGL((depth_norm_kernel<TAPS, true, 1024>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
+    else hipLaunchKernelGGL((depth_norm_kernel<TAPS, false, 1024>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
     GLM_CHECK_LAUNCH("glm_depth_norm");
     return GLM_OK;
 }

@@ -146,6 +146,13 @@ def test_depth_norm(dtype, width, groups, taps, depth):
         assert torch.allclose(h[:, :width].cpu().double(), O.norm_groups(xn[pick], gain.double(), groups, eps), atol=2 * tol, rtol=tol), kind
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 2), (4608, 1, 4, 3), (512, 1, 4, 5), (8, 1, 4, 1)])
+def test_depth_norm_512_threads(dtype, width, groups, taps, depth):
+    """Four taps in 512 threads, in more, in one wave and in one lane."""
+    test_depth_norm(dtype, width, groups, taps, depth)
+
+
 @pytest.mark.parametrize("width,taps", [(72, 4), (76, 3), (64, 2), (1032, 6), (4104, 4)])
 @pytest.mark.parametrize("lens", [[3000, 1, 1, 1, 6000, 2, 900], [5, 1, 700, 3, 1, 1, 2]])
 def test_convolution_down_runs(width, taps, lens):
