@@ -15,7 +15,7 @@
 // state rows, which are double-buffered: a step reads row set state_in and writes row set state_out.  Everything is fp32 up to the store
 // of h, the same arithmetic for a token of this step as for one whose row was kept.
 //
-// Steps of many rows take two launches, norm and average (every row for itself) and depth_conv: re-reading x_next costs four bytes a
+// Steps of many rows, and prompts of some hundred, take two launches, norm and average (every row for itself) and depth_conv: re-reading x_next costs four bytes a
 // column; with runs of sixteen rows, recomputing the TAPS-1 in front cost a fifth of rows that are k experts and several depths
 // wide.
 #include "common.h"
@@ -248,7 +248,7 @@ __device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, i
 // One row per workgroup.  TAPS > 1: with the convolution, for which the TAPS-1 rows in front are computed as well, as far as they are of
 // this step.  What bounds it with few rows is a chain of trips to memory.  Up to 512 threads and four taps (NT, with registers for it) the row, the depths and the taps are requested
 // in front of the sequence's tables, not behind them and not behind the stores: behind k = 6 experts and one to three depths, four taps, in a step, us: 100 rows of 2048 10.8 / 9.2, 9 rows
-// 10.2 / 8.8, 60 rows of 4096 13.3 / 10.5, without experts 7.8 / 6.3, 300 rows of two prompts, each with the three in front of it, 19.2 / 18.5.
+// 10.2 / 8.8, 60 rows of 4096 13.3 / 10.5, without experts 7.8 / 6.3.
 template <int TAPS, bool VEC, int NT>
 __global__ __launch_bounds__(NT) void depth_norm_kernel(const DepthArgs a) {
     constexpr int HALO = TAPS - 1;
@@ -456,6 +456,10 @@ __global__ __launch_bounds__(256) void depth_conv_kernel(const DepthArgs a, cons
 }
 
 constexpr int64_t DN_SPLIT_ROWS = 512;   // rows from which norm and convolution are launches of their own
+// and rows beyond one per sequence: a row in the middle of a portion computes the TAPS-1 in front of it as well, one after the other.  One launch / two, whole steps of four layers, us: two
+// prompts of 150 and 131 1004 / 982, one of 500 1239 / 1209, 90 rows and 300 of prompts (4096 columns) 2850 / 2808; below, the host's launches take longer than the kernels: one prompt of
+// 20 881 / 896, of 40 869 / 878, of 135 912 / 921, 60 rows and 40 of a prompt 944 / 950.
+constexpr int64_t DN_SPLIT_EXTRA = 256;
 
 template <int TAPS>
 int launch_depth_conv(const DepthArgs& a, const float* xs, hipStream_t st) {
@@ -472,14 +476,15 @@ int launch_depth_conv(const DepthArgs& a, const float* xs, hipStream_t st) {
 }
 
 template <int TAPS>
-int launch_depth_norm(const DepthArgs& a, int nt, bool vec, hipStream_t st) {
+int launch_depth_norm(const DepthArgs& a, int64_t seqs, int nt, bool vec, hipStream_t st) {
     if constexpr (TAPS > 1) {
         const float* xs = a.depth ? a.x_next : a.y ? a.x_out : a.x_in;
-        if (a.T > DN_SPLIT_ROWS && xs) {
+        const bool whole = glm_aligned16(xs) && glm_aligned16(a.h) && glm_aligned16(a.conv_w) && glm_aligned16(a.state);
+        if (xs && (a.T > DN_SPLIT_ROWS || (a.T >= seqs + DN_SPLIT_EXTRA && whole))) {
             if (a.y || a.depth || a.x_cast || a.x_out) {
                 DepthArgs b = a;
                 b.h = nullptr;
-                const int rc = launch_depth_norm<1>(b, nt, vec, st);
+                const int rc = launch_depth_norm<1>(b, seqs, nt, vec, st);
                 if (rc != GLM_OK) return rc;
             }
             return launch_depth_conv<TAPS>(a, xs, st);
@@ -511,6 +516,15 @@ extern "C" int glm_depth_norm(const float* x_in, const int32_t* row_index, int64
                               const float* g_pre, const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of, const int32_t* q_start,
                               const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32, int64_t T, int width, int wp, int groups, float eps,
                               glm_stream_t stream) {
+    return glm_depth_norm_portions(x_in, row_index, ld, y, ldy, pair_pos, pair_w, k, n_rows, g_post, x_out, x_cast, ldc, depth, depth_stride, n_depth, coef, x_next, g_pre, conv_w, taps, state,
+                                   n_state, pos, seq_of, q_start, state_in, state_out, h, ldh, act_f32, T, T, width, wp, groups, eps, stream);
+}
+
+extern "C" int glm_depth_norm_portions(const float* x_in, const int32_t* row_index, int64_t ld, const void* y, int64_t ldy, const int32_t* pair_pos, const float* pair_w, int k, int64_t n_rows,
+                              const float* g_post, float* x_out, void* x_cast, int64_t ldc, const float* depth, int64_t depth_stride, int n_depth, const float* coef, float* x_next,
+                              const float* g_pre, const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of, const int32_t* q_start,
+                              const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32, int64_t T, int64_t seqs, int width, int wp, int groups, float eps,
+                              glm_stream_t stream) {
     GLM_CHECK_ARG(x_in && T >= 0 && width > 0 && wp >= width && wp % 8 == 0 && wp - width < 8 && ld >= wp && ld % 4 == 0 && groups > 0 && width % groups == 0, GLM_ERR_INVALID,
                   "glm_depth_norm: bad shape T=%ld width=%d wp=%d groups=%d ld=%ld", (long)T, width, wp, groups, (long)ld);
     GLM_CHECK_ARG(!y || (g_post && ldy >= wp && ldy % 8 == 0), GLM_ERR_INVALID, "glm_depth_norm: bad sublayer output (ldy=%ld)", (long)ldy);
@@ -540,13 +554,13 @@ extern "C" int glm_depth_norm(const float* x_in, const int32_t* row_index, int64
     const int nt = waves * 64;
     hipStream_t st = glm_s(stream);
     switch (taps) {
-        case 1: return launch_depth_norm<1>(a, nt, vec, st);
-        case 2: return launch_depth_norm<2>(a, nt, vec, st);
-        case 3: return launch_depth_norm<3>(a, nt, vec, st);
-        case 4: return launch_depth_norm<4>(a, nt, vec, st);
-        case 6: return launch_depth_norm<6>(a, nt, vec, st);
-        case 8: return launch_depth_norm<8>(a, nt, vec, st);
-        case 16: return launch_depth_norm<16>(a, nt, vec, st);
-        default: return launch_depth_norm<32>(a, nt, vec, st);
+        case 1: return launch_depth_norm<1>(a, seqs, nt, vec, st);
+        case 2: return launch_depth_norm<2>(a, seqs, nt, vec, st);
+        case 3: return launch_depth_norm<3>(a, seqs, nt, vec, st);
+        case 4: return launch_depth_norm<4>(a, seqs, nt, vec, st);
+        case 6: return launch_depth_norm<6>(a, seqs, nt, vec, st);
+        case 8: return launch_depth_norm<8>(a, seqs, nt, vec, st);
+        case 16: return launch_depth_norm<16>(a, seqs, nt, vec, st);
+        default: return launch_depth_norm<32>(a, seqs, nt, vec, st);
     }
 }

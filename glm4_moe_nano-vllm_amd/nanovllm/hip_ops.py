@@ -208,6 +208,9 @@ _SIGNATURES = {
     "glm_depth_norm": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p,
         c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p,
         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_int, c_int, c_float, c_void_p]),
+    "glm_depth_norm_portions": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int64, c_void_p, c_void_p,
+        c_void_p, c_int64, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_void_p,
+        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int64, c_int64, c_int, c_int, c_int, c_float, c_void_p]),
     "glm_router_softmax": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "glm_router_softmax_align": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
         c_void_p]),
@@ -2058,9 +2061,10 @@ def depth_norm(x: torch.Tensor, width: int, groups: int, eps: float, y=None, g_p
         assert st.shape[1:] == (taps - 1, wp) and rows is None
         args = (meta.pos, meta.seq_of, meta.q_start, meta.state_in, meta.state_out)
         assert meta.pos.numel() == meta.seq_of.numel() == T
-    _check(load_library().glm_depth_norm(
+    seqs = meta.q_start.numel() - 1 if conv is not None else T
+    _check(load_library().glm_depth_norm_portions(
         _p(x), _p(rows), wp, yp, ldy, pos_p, w_p, k, n_rows, _p(g_post) if y is not None else None, _p(x_out), _p(x_cast), wp, dp, stride, n_depth, cp, _p(x_next), _p(g_pre),
-        _p(cw), taps, _p(st), n_state, *(_p(a) for a in args), _p(h), wp, f32, T, width, wp, groups, eps, _stream()), "glm_depth_norm")
+        _p(cw), taps, _p(st), n_state, *(_p(a) for a in args), _p(h), wp, f32, T, seqs, width, wp, groups, eps, _stream()), "glm_depth_norm")
     return x_cast, h
 
 

@@ -658,7 +658,8 @@ int glm_row_norm_gate(const void* o, int64_t ldo, int o_f32, const void* gate, i
  * of `groups` equal parts by its own root mean square), x_next = sum_j coef[j] depth_j + coef[n_depth] x_out (depth_j at depth + j
  * depth_stride), and h = x_next + conv(x_next) or, with g_pre, norm(x_next) g_pre.  y: rows of the sublayer, or with pair_pos [T, k] the
  * experts' rows, weighed by pair_w in fp32.  All fp32 rows have pitch ld; every part is optional; taps as glm_depth_norm_taps; rows of a
- * step and state rows [n_state][taps-1][wp] as for glm_seq_norm; row_index gathers rows of x_in, y and the depths (no convolution).   */
+ * step and state rows [n_state][taps-1][wp] as for glm_seq_norm; row_index gathers rows of x_in, y and the depths (no convolution).
+ * _portions: the same, told how many sequences the T rows belong to (which decides about the launches, not about results).   */
 int glm_depth_norm_taps(int taps);
 int glm_depth_norm(const float* x_in, const int32_t* row_index, int64_t ld, const void* y, int64_t ldy, const int32_t* pair_pos,
                    const float* pair_w, int k, int64_t n_rows, const float* g_post, float* x_out, void* x_cast, int64_t ldc,
@@ -666,6 +667,12 @@ int glm_depth_norm(const float* x_in, const int32_t* row_index, int64_t ld, cons
                    const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of,
                    const int32_t* q_start, const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32,
                    int64_t T, int width, int wp, int groups, float eps, glm_stream_t stream);
+int glm_depth_norm_portions(const float* x_in, const int32_t* row_index, int64_t ld, const void* y, int64_t ldy, const int32_t* pair_pos,
+                   const float* pair_w, int k, int64_t n_rows, const float* g_post, float* x_out, void* x_cast, int64_t ldc,
+                   const float* depth, int64_t depth_stride, int n_depth, const float* coef, float* x_next, const float* g_pre,
+                   const void* conv_w, int taps, float* state, int64_t n_state, const int32_t* pos, const int32_t* seq_of,
+                   const int32_t* q_start, const int32_t* state_in, const int32_t* state_out, void* h, int64_t ldh, int act_f32,
+                   int64_t T, int64_t seqs, int width, int wp, int groups, float eps, glm_stream_t stream);
 
 /* Softmax router: the k largest of softmax(logits) over E experts, fp32 weights, not renormalised; descending.  _align: and the bucketing
  * of glm_moe_align (no shared group, no scales) in one launch, for few tokens (T k <= 1024, E <= 256).  combine_weighted: out[t] = sum_j w[t,j] y[pair_pos[t,j]]. */

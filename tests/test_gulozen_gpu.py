@@ -147,6 +147,28 @@ def test_depth_norm(dtype, width, groups, taps, depth):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,groups,taps,depth", [(76, 4, 3, 0), (1032, 1, 4, 1), (2048, 4, 4, 3), (200, 5, 6, 5), (72, 72, 17, 1), (24, 3, 32, 2), (4104, 3, 2, 2)])
+@pytest.mark.parametrize("lens,starts", [([257], [0]), ([1] * 9 + [2, 256], [5] * 9 + [0, 3]), ([3, 170, 1, 150], [0, 40, 7, 1]), ([512], [2])])
+def test_depth_norm_launches(dtype, width, groups, taps, depth, lens, starts):
+    """Norm and convolution in a launch each (256 rows and more beyond one per sequence) and in one: the same bits, in every row and in the state."""
+    from nanovllm import hip_ops
+    wp, tp, T, S, dt = hip_ops.round8(width), hip_ops.depth_norm_taps(taps), sum(lens), len(lens), DT[dtype]
+    meta, _ = batch_meta(lens, starts, 3)
+    many = types.SimpleNamespace(**{**vars(meta), "q_start": torch.cat([meta.q_start, meta.q_start[-1:].expand(T)])})   # empty portions behind: one launch
+    x, y, gain = dev(padc(torch.randn(T, width, generator=g(1)), wp)), dev(padc(torch.randn(T, width, generator=g(2)).to(dt), wp)), dev(padc(torch.rand(width, generator=g(3)), wp))
+    planes, coef = dev(padc(torch.randn(max(depth, 1), T, width, generator=g(4)), wp)), dev(torch.randn(depth + 1, generator=g(5)))
+    cw, st = dev(padc(torch.randn(tp, width, generator=g(6)).to(torch.bfloat16), wp)), padc(torch.randn(2 * S, tp - 1, width, generator=g(7)), wp)
+    got = []
+    for m in (meta, many):
+        state, x_out, x_next = st.cuda().clone(), torch.zeros(T, wp, device="cuda"), torch.zeros(T, wp, device="cuda")
+        cast, h = hip_ops.depth_norm(x, width, groups, 1e-5, y=y, g_post=gain, x_out=x_out, cast=True, depth=(planes[:depth], coef) if depth else None, x_next=x_next if depth else None,
+                                     conv=(cw, state), meta=m, act_dtype=dt)
+        got.append((h, cast, x_out, x_next, state))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 2), (4608, 1, 4, 3), (512, 1, 4, 5), (8, 1, 4, 1)])
 def test_depth_norm_512_threads(dtype, width, groups, taps, depth):
     """Four taps in 512 threads, in more, in one wave and in one lane."""
