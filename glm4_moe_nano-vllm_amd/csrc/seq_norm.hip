@@ -283,15 +283,21 @@ __device__ __forceinline__ f32x4_t sn_load_slabs(const SeqNormArgs& a, int64_t r
     return v;
 }
 
-// ANY: y or the activations may be fp32 (y in slabs: then it is summed up where it is requested)
-template <int TAPS, int NT, bool ANY>
+// ANY: y or the activations may be fp32 (y in slabs: then it is summed up where it is requested).
+// FORM: SN_RUNS, as described at the loop.  SN_ONE: one row per workgroup, behind the TAPS-1 in front of it: nothing waits behind its stores, so those are under tests, and the rows in front
+// have neither stores nor a convolution.  SN_TESTS: the same for runs shorter than 16 rows with six and eight taps, of which a third and more are rows in front.  Stores issued
+// whatever there is / this, us, prompts: four taps 64 rows of 4096 9.6 / 7.5, 300 14.7 / 11.6, 1024 of 2048 16.4 / 14.1, without y 11.9 / 8.9, 2000 of 1024
+// 16.8 / 14.0; eight taps 300 of 2048 18.8 / 13.5, 2000 of them in runs of four 26.4 / 21.5; six taps 1024 of 4096 21.8 / 18.7.  Runs of 16 rows, eight taps 116 / 124.
+constexpr int SN_ONE = 0, SN_TESTS = 1, SN_RUNS = 2;
+template <int TAPS, int NT, bool ANY, int FORM>
 __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm_stream_kernel(const SeqNormArgs a, int tr) {
     constexpr int HALO = TAPS - 1, NW = NT / 64;
+    constexpr bool RUN = FORM != SN_ONE, ALL = FORM == SN_RUNS;
     __shared__ float s_red[2][2][NW];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int c = tid * 8, cl = min(c, a.wp - 8);   // cl: what a thread behind the row's end reads instead
     const bool on = c < a.wp;
-    const int64_t r0 = (int64_t)blockIdx.x * tr, r1 = min(r0 + tr, a.T);
+    const int64_t r0 = (int64_t)blockIdx.x * tr, r1 = RUN ? min(r0 + tr, a.T) : r0 + 1;
     const float inv_w = 1.0f / (float)a.width;
     int s = 0, qs = 0, qe = 0, sin = 0, so = 0;
     auto sequence = [&](int64_t r) {
@@ -370,10 +376,25 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
     const bool f32 = ANY && a.act_f32;
     const int rowb = a.wp * 4, actb = a.wp * (f32 ? 4 : 2);
     auto put = [&](void* base, int64_t ld, int64_t r, bool mine, const Row8& v) __attribute__((always_inline)) {   // activations
+        if (!ALL && !(mine && base)) return;
         const __amdgpu_buffer_rsrc_t rs = sn_row(base, r * ld * (f32 ? 4 : 2), mine ? actb : 0);
         if (f32) sn_put8f(rs, c * 4, v);
         else __builtin_amdgcn_raw_buffer_store_b128(sn_pack8(v), rs, c * 2, 0, 0);
     };
+    // of a portion's first row r, out of the state (waited for here, not in every turn)
+    auto history = [&](int64_t r) __attribute__((always_inline)) {
+        const int p = sn_table(a.pos, r);
+#pragma unroll
+        for (int k = 1; k < TAPS; ++k) {
+            hist[k - 1] = zero;
+            if (on && p - k >= 0) hist[k - 1] = sn_ld8f(a.state + ((int64_t)sin * HALO + (HALO - k)) * a.wp + c);
+        }
+#pragma unroll
+        for (int k = 1; k < TAPS; ++k) asm volatile("" : "+v"(hist[k - 1].a), "+v"(hist[k - 1].b));
+    };
+    if constexpr (TAPS > 1 && !RUN) {
+        if (a.g_pre && lo == qs) history(lo);
+    }
     for (int64_t r = lo; r < r1; ++r) {
         if constexpr (TAPS > 1) {  // opaque: unpacked outside the loop the taps would take twice the registers
 #pragma unroll
@@ -394,7 +415,7 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
             }
         }
         const bool mine = TAPS == 1 || r >= r0;
-        sn_put8f(sn_row(a.x_out, r * a.ldx * 4, mine ? rowb : 0), c * 4, x);
+        if (ALL || (mine && a.x_out)) sn_put8f(sn_row(a.x_out, r * a.ldx * 4, mine ? rowb : 0), c * 4, x);
         put(a.x_cast, a.ldc, r, mine, x);
         reduce2(sumsq(x), a.y && r + 1 < r1 ? sumsq(value(y1)) : 0.f, par, su, sv);
         par ^= 1;
@@ -409,36 +430,31 @@ __global__ __launch_bounds__(NT, (TAPS <= 4 && NT <= 512 ? 4 : 1)) void seq_norm
             }
             o = h;
             if constexpr (TAPS > 1) {
-                if (r == qe) sequence(r);  // the next sequence's portion begins
-                if (r == qs) {
-                    const int p = sn_table(a.pos, r);
-#pragma unroll
-                    for (int k = 1; k < TAPS; ++k) {
-                        hist[k - 1] = zero;
-                        if (on && p - k >= 0) hist[k - 1] = sn_ld8f(a.state + ((int64_t)sin * HALO + (HALO - k)) * a.wp + c);
-                    }
-#pragma unroll
-                    for (int k = 1; k < TAPS; ++k) asm volatile("" : "+v"(hist[k - 1].a), "+v"(hist[k - 1].b));   // (waited for here, not in every turn)
+                if constexpr (RUN) {
+                    if (r == qe) sequence(r);  // the next sequence's portion begins
+                    if (r == qs) history(r);
                 }
-                Row8 acc = zero;
+                if (ALL || mine) {
+                    Row8 acc = zero;
 #pragma unroll
-                for (int k = HALO; k >= 1; --k)
+                    for (int k = HALO; k >= 1; --k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * hist[k - 1].a[i];
+                            acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * hist[k - 1].b[i];
+                        }
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        acc.a[i] = acc.a[i] + tap(w[TAPS - 1 - k], i) * hist[k - 1].a[i];
-                        acc.b[i] = acc.b[i] + tap(w[TAPS - 1 - k], 4 + i) * hist[k - 1].b[i];
+                        o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
+                        o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
                     }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    o.a[i] = h.a[i] + (acc.a[i] + tap(w[TAPS - 1], i) * h.a[i]);
-                    o.b[i] = h.b[i] + (acc.b[i] + tap(w[TAPS - 1], 4 + i) * h.b[i]);
-                }
-                const int e = qe - 1 - (int)r;  // tokens of the portion behind this one
-                if (mine && e < HALO && so >= 0 && so < a.n_state && sn_table(a.pos, r) >= 0 && on) {
-                    sn_st8f(a.state + ((int64_t)so * HALO + (HALO - 1 - e)) * a.wp + c, h);
-                    if (e == 0)  // a portion shorter than the history: the older inputs move up
-                        for (int i = 0; i < HALO - (qe - qs); ++i)
-                            sn_st8f(a.state + ((int64_t)so * HALO + i) * a.wp + c, sn_ld8f(a.state + ((int64_t)sin * HALO + i + (qe - qs)) * a.wp + c));
+                    const int e = qe - 1 - (int)r;  // tokens of the portion behind this one
+                    if (mine && e < HALO && so >= 0 && so < a.n_state && sn_table(a.pos, r) >= 0 && on) {
+                        sn_st8f(a.state + ((int64_t)so * HALO + (HALO - 1 - e)) * a.wp + c, h);
+                        if (e == 0)  // a portion shorter than the history: the older inputs move up
+                            for (int i = 0; i < HALO - (qe - qs); ++i)
+                                sn_st8f(a.state + ((int64_t)so * HALO + i) * a.wp + c, sn_ld8f(a.state + ((int64_t)sin * HALO + i + (qe - qs)) * a.wp + c));
+                    }
                 }
 #pragma unroll
                 for (int k = HALO; k >= 2; --k) hist[k - 1] = hist[k - 2];
@@ -651,11 +667,18 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
             return GLM_OK;
         }
     }
+    const bool any = a.act_f32 || (a.y && a.y_f32);
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
     if (tr > 1) tr = tr < 4 ? 4 : tr > 32 ? 32 : tr;
     const dim3 grid((unsigned)((a.T + tr - 1) / tr));
-    if (a.act_f32 || (a.y && a.y_f32)) hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, true>), grid, dim3(NT), 0, st, a, tr);
-    else hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, false>), grid, dim3(NT), 0, st, a, tr);
+    auto launch = [&](auto formc) {
+        constexpr int FORM = decltype(formc)::value;
+        if (any) hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, true, FORM>), grid, dim3(NT), 0, st, a, tr);
+        else hipLaunchKernelGGL((seq_norm_stream_kernel<TAPS, NT, false, FORM>), grid, dim3(NT), 0, st, a, tr);
+    };
+    if (tr == 1) launch(std::integral_constant<int, SN_ONE>{});
+    else if (TAPS > 4 && tr < 16) launch(std::integral_constant<int, (TAPS > 4 ? SN_TESTS : SN_RUNS)>{});
+    else launch(std::integral_constant<int, SN_RUNS>{});
     GLM_CHECK_LAUNCH("glm_seq_norm");
     return GLM_OK;
 }

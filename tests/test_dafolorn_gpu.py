@@ -180,6 +180,39 @@ def test_seq_norm_stream_of_bf16(width, taps, lens):
             assert bool((c[:, :shift] == 7).all()) and bool((c[:, shift + wp:] == 7).all()) and torch.equal(c[:, shift: shift + wp], got[1][0].bfloat16())
 
 
+@pytest.mark.parametrize("width,taps", [(64, 1), (72, 2), (520, 3), (1032, 4), (2048, 4), (4104, 4), (200, 6), (2056, 6), (2048, 8), (4096, 8), (8192, 1)])
+@pytest.mark.parametrize("more", [600, 9000])
+def test_seq_norm_rows_alone_and_in_runs(width, taps, more):
+    """Rows of a step of 300, each in a workgroup of its own, and the same rows in a longer step, in runs: the same bits in whatever the launch has, and in the state.
+    Slabs in every number from one to nine."""
+    from nanovllm import hip_ops
+    wp, lens = hip_ops.round8(width), [3, 170, 1, 126]
+    T, S = sum(lens), 5
+    torch.manual_seed(width + taps)
+    x, gain, gp = (torch.randn(*d, device="cuda") for d in ((T + more, wp), (wp,), (wp,)))
+    x[:, width:] = 0
+    state = torch.randn(2 * S, max(taps - 1, 1), wp, device="cuda")
+    conv_w = torch.randn(taps, wp, device="cuda").bfloat16()
+    y, slabs = torch.randn(T + more, wp, device="cuda"), torch.randn(9, T + more, wp, device="cuda") if more == 600 else None
+    kinds = [(None, torch.bfloat16), (y.bfloat16(), torch.bfloat16), (y.bfloat16(), torch.float32), (y, torch.float32)] + [(n, torch.bfloat16) for n in range(1, 10) if more == 600]
+    for kind, dtype in kinds:
+        for cast, keep, norm in ((True, True, True), (False, False, True), (True, False, False), (False, True, True)):
+            if not norm and taps > 1:
+                continue
+            got = []
+            for ls in (lens, lens + [more]):
+                n, meta_s = sum(ls), len(ls)
+                meta = types.SimpleNamespace(pos=i32([(40 if s % 3 == 1 else 0) + p for s, c in enumerate(ls) for p in range(c)]), seq_of=i32([s for s, c in enumerate(ls) for _ in range(c)]),
+                                             q_start=i32([sum(ls[:s]) for s in range(meta_s + 1)]), state_in=i32(list(range(meta_s))), state_out=i32([S + s for s in range(meta_s)]))
+                kept, xc = state.clone(), torch.zeros(n, wp, device="cuda", dtype=dtype) if cast else None
+                yk = hip_ops.PartialSum(slabs[:kind, :n].contiguous()) if isinstance(kind, int) else None if kind is None else kind[:n].contiguous()
+                xo, h = hip_ops.seq_norm(x[:n].contiguous(), width, 1e-5, y=yk, g_post=gp, g_pre=gain if norm else None, conv=(conv_w, kept) if taps > 1 else None, meta=meta, act_dtype=dtype,
+                                         x_cast=xc, keep_x=keep)
+                got.append([None if t is None else t[:T] for t in (xo, h, xc)] + [kept[: S + 4]])
+            for a, b in zip(*got):
+                assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), (dtype, cast, keep)
+
+
 @pytest.mark.parametrize("n", [1, 3, 5, 6, 9, 16])
 @pytest.mark.parametrize("T,width", [(1, 64), (7, 2048), (512, 520), (513, 520)])
 def test_seq_norm_adds_slabs_in_their_order(n, T, width):
