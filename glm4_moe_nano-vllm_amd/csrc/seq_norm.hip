@@ -647,6 +647,25 @@ __global__ __launch_bounds__(NT) void seq_norm_row_kernel(const SeqNormArgs a) {
     finish(x, y, a.y ? rms(reduce(sn_sumsq8(y))) : 0.f, hist);
 }
 
+// Rows of a run: `rows`, but four at least, or eight at least
+//   - where runs of four are more workgroups than there is room for at once, and take more turns than runs of eight.  Runs of four / eight, us: 2000 rows of 4096, six taps 40.3 / 30.8, 1200 of
+//     8192, four taps 44.8 / 35.4; beside that the shorter ones: 2000 of 2048, four taps, 17.3 / 18.2, 1024 of 4096, six taps 22.3 / 28.3;
+//   - where y (or h) is fp32 and there are enough workgroups to be bound by memory: the rows in front are read again.  Four taps, 2048 columns: eight slabs, 2100 rows 60.9 / 48.0, 3000 96.7 / 62.9,
+//     four 2100 36.0 / 34.3, 4000 53.0 / 47.4, two 3000 30.1 / 29.8, 4000 37.7 / 34.4, one 4000 28.4 / 26.8; fewer rows are a chain: six slabs, 1200 29.7 / 35.4, 1600 34.6 / 37.6.  Of
+//     512 threads a CU has one workgroup or two, and their turns decide as well: six slabs, 1200 rows of 4096 53.3 / 47.8, 2100 84.4 / 97.5.
+template <int TAPS, int NT>
+int seq_norm_run(int64_t T, int rows, bool any, int slabs) {
+    constexpr int HALO = TAPS - 1, WAVES = TAPS <= 4 ? 16 : 12, WGW = NT / 64;   // waves of a CU that the registers are there for
+    const int four = rows < 4 ? 4 : rows > 32 ? 32 : rows;
+    if (four >= 8) return four;
+    auto wgs = [&](int n) { return (T + n - 1) / n; };
+    auto turns = [&](int n, int64_t at_once) { return (wgs(n) + at_once - 1) / at_once * (n + HALO); };
+    const int64_t fit = 256 * ((TAPS == 8 && any ? 8 : WAVES) / WGW);
+    if (turns(8, fit) < turns(four, fit)) return 8;
+    if (any && wgs(8) * WGW >= (slabs >= 4 ? 1000 : 1900) && (NT < 512 || turns(8, 256) < turns(four, 256))) return 8;
+    return four;
+}
+
 template <int TAPS, int NT>
 int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) {
     // decode: seq_norm_row_kernel; else runs of rows long enough to spread the halo and the register setup, short enough
@@ -672,7 +691,7 @@ int launch_seq_norm_stream(const SeqNormArgs& a, int64_t n_seq, hipStream_t st) 
     }
     const bool any = a.act_f32 || (a.y && a.y_f32);
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
-    if (tr > 1) tr = tr < 4 ? 4 : tr > 32 ? 32 : tr;
+    if (tr > 1) tr = seq_norm_run<TAPS, NT>(a.T, tr, any, a.y && a.y_f32 ? a.n_slabs : 1);
     const dim3 grid((unsigned)((a.T + tr - 1) / tr));
     auto launch = [&](auto formc) {
         constexpr int FORM = decltype(formc)::value;
