@@ -304,9 +304,17 @@ int launch_stream(const StreamNormArgs& a, hipStream_t st) {
     constexpr int WGS = NT >= 512 ? 512 : 4096 / (NT / 64) > 2048 ? 2048 : 4096 / (NT / 64);   // four waves on every SIMD
     // (of eight rows at least / of four, two streams of 2048, us: 40 single rows and 5400 of prompts 40.7 / 37.2, 36.6 / 33.3 without a shift, 3000 rows 25.9 / 23.6, 24.1 / 20.9)
     int tr = a.T <= 512 ? 1 : (int)((a.T + WGS - 1) / WGS);
-    if (tr > 1) tr = tr < 4 ? 4 : tr > 32 ? 32 : tr;
+    const bool any = (a.y && a.y_f32) || (a.h && a.h_f32);
+    if (tr > 1) {
+        tr = tr < 4 ? 4 : tr > 32 ? 32 : tr;
+        // Runs of eight rows at least where those of four are more workgroups than there is room for at once (registers: four waves on a SIMD, three with eight streams) and take as many turns,
+        // us, four / eight: eight streams of 4096, 1200 rows 96.8 / 82.1 with a shift, 83.9 / 73.4, 3000 166 / 155, 145 / 142.
+        const int64_t fit = 256 * ((S == 8 && (NT <= 256 || (NT == 512 && any)) ? 12 : 16) / (NT / 64));
+        auto turns = [&](int n) { return ((a.T + n - 1) / n + fit - 1) / fit * (n + (a.shift ? 1 : 0)); };
+        if (tr < 8 && turns(8) <= turns(tr)) tr = 8;
+    }
     const dim3 grid((unsigned)((a.T + tr - 1) / tr));
-    if ((a.y && a.y_f32) || (a.h && a.h_f32)) hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT, true>), grid, dim3(NT), 0, st, a, tr);
+    if (any) hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT, true>), grid, dim3(NT), 0, st, a, tr);
     else hipLaunchKernelGGL((stream_norm_kernel<S, NV, NT, false>), grid, dim3(NT), 0, st, a, tr);
     GLM_CHECK_LAUNCH("glm_stream_norm");
     return GLM_OK;

@@ -137,6 +137,35 @@ def test_stream_norm(width, S, y_kind):
             assert torch.allclose(o[s], outs[0][s][: o[s].shape[0]], rtol=1e-6, atol=2e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width,S", [(64, 1), (520, 2), (2048, 3), (1032, 4), (2048, 6), (200, 8), (1024, 8), (2048, 8), (4096, 8), (4096, 1), (8192, 2)])
+@pytest.mark.parametrize("more", [300, 600, 2700])
+def test_stream_norm_rows_alone_and_in_runs(width, S, more, dtype):
+    """Rows of a step of 300, each in a workgroup of its own, and the same rows in a longer step, in runs: the same bits in whatever the launch has, and in the state."""
+    from nanovllm import hip_ops
+    wp, lens = hip_ops.round8(width), [3, 170, 1, 126]
+    T, N = sum(lens), 5
+    torch.manual_seed(width + S)
+    r = lambda *d: torch.randn(*d, device="cuda")  # noqa: E731
+    x, y, state, wi, ys, mix, sh = r(T + more, S, wp), r(T + more, wp).to(dtype), r(2 * N, wp), r(S), r(wp), r(S * (S + 1)), r(wp)
+    for with_y, shift, norm in ((True, True, True), (True, False, True), (False, True, True), (False, False, True), (True, False, False)):
+        got = []
+        for ls in (lens, lens + [more]):
+            n, c = sum(ls), len(ls)
+            meta = types.SimpleNamespace(pos=i32([(40 if s % 3 == 1 else 0) + p for s, k in enumerate(ls) for p in range(k)]), seq_of=i32([s for s, k in enumerate(ls) for _ in range(k)]),
+                                         q_start=i32([sum(ls[:s]) for s in range(c + 1)]), state_in=i32(list(range(c))), state_out=i32([N + s for s in range(c)]))
+            kept = state.clone()
+            kw = dict(y=y[:n], y_scale=ys, mix_out=mix) if with_y else {}
+            if norm:
+                kw["w_in"] = wi
+            if shift:
+                kw.update(shift=sh, state=kept, meta=meta)
+            xo, h = hip_ops.stream_norm(x[:n], S, width, 1e-5, gain=1.5, act_dtype=dtype, **kw)
+            got.append([None if t is None else t[:T] for t in (xo, h)] + [kept[: N + 4]])
+        for a, b in zip(*got):
+            assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), (with_y, shift, norm)
+
+
 @pytest.mark.parametrize("width,S", [(64, 1), (520, 2), (2048, 2), (2056, 3), (4096, 2), (72, 4), (1024, 6), (4104, 8)])
 @pytest.mark.parametrize("lens", [[1, 30, 2, 1], [700, 1, 41, 2, 9, 600, 3, 1500], [4100]])
 def test_stream_norm_of_bf16(width, S, lens):
