@@ -246,7 +246,7 @@ __device__ __forceinline__ void dn_row(const DepthArgs& a, int64_t row, int c, i
 }
 
 // One row per workgroup.  TAPS > 1: with the convolution, for which the TAPS-1 rows in front are computed as well, as far as they are of
-// this step.  What bounds it with few rows is a chain of trips to memory.  Up to 512 threads and four taps (NT, with registers for it) the row, the depths and the taps are requested
+// this step.  What bounds it with few rows is a chain of trips to memory.  Up to 512 threads, four taps and one round of the chip (NT, with registers for it) the row, the depths and the taps are requested
 // in front of the sequence's tables, not behind them and not behind the stores: behind k = 6 experts and one to three depths, four taps, in a step, us: 100 rows of 2048 10.8 / 9.2, 9 rows
 // 10.2 / 8.8, 60 rows of 4096 13.3 / 10.5, without experts 7.8 / 6.3.
 template <int TAPS, bool VEC, int NT>
@@ -491,7 +491,9 @@ int launch_depth_norm(const DepthArgs& a, int64_t seqs, int nt, bool vec, hipStr
         }
     }
     if constexpr (TAPS > 1 && TAPS <= 4) {
-        if (vec && nt <= 512) {
+        // (a CU has room for eight waves of it: as long as the rows are one round.  Beyond / the form for 1024 threads, us, single rows: 257 of 3072 columns 11.5 / 9.5, 300 of 4096 14.8 / 12.9, behind
+        // experts 17.6 / 15.9; 512 of 2048, still one round, 9.2 / 10.3)
+        if (vec && nt <= 512 && a.T * (nt / 64) <= 8 * 256) {
             hipLaunchKernelGGL((depth_norm_kernel<TAPS, true, 512>), dim3((unsigned)a.T), dim3(nt), 0, st, a);
             GLM_CHECK_LAUNCH("glm_depth_norm");
             return GLM_OK;

@@ -169,6 +169,34 @@ def test_depth_norm_launches(dtype, width, groups, taps, depth, lens, starts):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 3), (3072, 1, 4, 0), (4096, 1, 2, 5), (2048, 2, 3, 1), (512, 1, 4, 5), (4608, 3, 4, 1)])
+def test_depth_norm_rows_of_a_round_and_beyond(dtype, width, groups, taps, depth):
+    """Single rows, more of them than there is room for at once, and the same rows in launches of 128: the same bits behind a sublayer, experts and nothing."""
+    from nanovllm import hip_ops
+    T, part, dt, k = 512, 128, DT[dtype], 3
+    meta, _ = batch_meta([1] * T, [s % 6 for s in range(T)], 4)
+    x, y, rows, gain = dev(torch.randn(T, width, generator=g(1))), dev(torch.randn(T, width, generator=g(2)), dt), dev(torch.randn(T * k, width, generator=g(3)), dt), dev(torch.rand(width, generator=g(4)))
+    pair = torch.randperm(T * k, generator=g(5)).view(T, k)
+    pair[::7, 1] = -1
+    pair, w = pair.to(torch.int32).cuda(), dev(torch.rand(T, k, generator=g(6)))
+    planes, coef = dev(torch.randn(max(depth, 1), T, width, generator=g(7))), dev(torch.randn(depth + 1, generator=g(8)))
+    cw, st = dev(torch.randn(taps, width, generator=g(9)), torch.bfloat16), dev(torch.randn(2 * T, taps - 1, width, generator=g(10)))
+    for kind in ("rows", "experts", "none"):
+        got = []
+        for n in (T, part):
+            state, outs = st.clone(), []
+            for a in range(0, T, n):
+                m = types.SimpleNamespace(pos=meta.pos[a: a + n], seq_of=meta.seq_of[:n], q_start=meta.q_start[: n + 1], state_in=meta.state_in[a: a + n], state_out=meta.state_out[a: a + n])
+                yk = {"rows": y[a: a + n], "experts": hip_ops.ExpertRows(rows, pair[a: a + n].reshape(-1), w[a: a + n]), "none": None}[kind]
+                xo, xn = (torch.zeros(n, width, device="cuda") for _ in range(2))
+                cast, h = hip_ops.depth_norm(x[a: a + n], width, groups, 1e-5, y=yk, g_post=gain, x_out=xo, cast=True, depth=(planes[:depth, a: a + n], coef) if depth else None,
+                                             x_next=xn if depth else None, conv=(cw, state), meta=m, act_dtype=dt)
+                outs.append((cast, h, xo, xn))
+            got.append([torch.cat(t) for t in zip(*outs)] + [state])
+        assert all(torch.equal(a, b) for a, b in zip(*got)), kind
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 2), (4608, 1, 4, 3), (512, 1, 4, 5), (8, 1, 4, 1)])
 def test_depth_norm_512_threads(dtype, width, groups, taps, depth):
     """Four taps in 512 threads, in more, in one wave and in one lane."""
