@@ -459,6 +459,11 @@ constexpr int64_t DN_SPLIT_ROWS = 512;   // rows from which norm and convolution
 // and rows beyond one per sequence: a row in the middle of a portion computes the TAPS-1 in front of it as well, one after the other.  One launch / two, whole steps of four layers, us: two
 // prompts of 150 and 131 1004 / 982, one of 500 1239 / 1209, 90 rows and 300 of prompts (4096 columns) 2850 / 2808; below, the host's launches take longer than the kernels: one prompt of
 // 20 881 / 896, of 40 869 / 878, of 135 912 / 921, 60 rows and 40 of a prompt 944 / 950.
+// The rows in front (their number times what one costs: one that is only read 1, a norm 2, with one depth 3, with more of them or with experts' rows 5) have to be worth the other launch, in
+// which portions of one row wait for their states one after the other: 8, and 5 for rows of more than 256 threads.  One / two launches, us, 400 rows of four prompts, then of forty single rows
+// and prompts: 2048 columns, four taps, a norm 9.9 / 9.9, 10.1 / 12.3, nothing in front 5.8 / 7.1, 6.0 / 9.9, one depth 14.5 / 10.7, 14.1 / 13.2, six experts 17.7 / 10.9, 17.5 / 13.5; two
+// taps, a norm 7.1 / 8.8, 7.2 / 9.5, experts 10.0 / 9.6, 9.6 / 10.5; six taps, nothing 9.3 / 8.3, 10.1 / 13.2, a norm 19.7 / 11.2, 20.0 / 15.9; 4096 columns, four taps, a norm 16.9 / 13.0,
+// 16.5 / 16.4, nothing 8.7 / 7.7, 9.0 / 10.8; two taps, experts, 512 rows 18.6 / 15.5, 18.3 / 16.6.
 constexpr int64_t DN_SPLIT_EXTRA = 256;
 
 template <int TAPS>
@@ -480,7 +485,8 @@ int launch_depth_norm(const DepthArgs& a, int64_t seqs, int nt, bool vec, hipStr
     if constexpr (TAPS > 1) {
         const float* xs = a.depth ? a.x_next : a.y ? a.x_out : a.x_in;
         const bool whole = glm_aligned16(xs) && glm_aligned16(a.h) && glm_aligned16(a.conv_w) && glm_aligned16(a.state);
-        if (xs && (a.T > DN_SPLIT_ROWS || (a.T >= seqs + DN_SPLIT_EXTRA && whole))) {
+        const int again = (TAPS - 1) * (!a.y ? 1 : a.pair_pos || (a.depth && a.n_depth > 1) ? 5 : a.depth && a.n_depth ? 3 : 2);
+        if (xs && (a.T > DN_SPLIT_ROWS || (a.T >= seqs + DN_SPLIT_EXTRA && whole && again >= (nt > 256 ? 5 : 8)))) {
             if (a.y || a.depth || a.x_cast || a.x_out) {
                 DepthArgs b = a;
                 b.h = nullptr;

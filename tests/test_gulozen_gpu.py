@@ -169,6 +169,33 @@ def test_depth_norm_launches(dtype, width, groups, taps, depth, lens, starts):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width,groups,taps,depth", [(72, 3, 4, 0), (2048, 4, 4, 1), (520, 1, 3, 2), (2056, 1, 2, 0), (4096, 4, 6, 0), (4104, 3, 2, 3), (200, 5, 9, 1)])
+@pytest.mark.parametrize("lens,starts", [([257], [0]), ([1] * 9 + [2, 256], [5] * 9 + [0, 3]), ([3, 170, 1, 150], [0, 40, 7, 1]), ([512], [2])])
+def test_depth_norm_launches_behind_experts(dtype, width, groups, taps, depth, lens, starts):
+    """As above, behind experts' rows and behind nothing, with more portions than rows (one launch); states that start in the middle of 16 bytes: one launch of some hundred rows as well."""
+    from nanovllm import hip_ops
+    wp, tp, T, S, dt, k = hip_ops.round8(width), hip_ops.depth_norm_taps(taps), sum(lens), len(lens), DT[dtype], 3
+    meta, _ = batch_meta(lens, starts, 3)
+    many = types.SimpleNamespace(**{**vars(meta), "q_start": torch.cat([meta.q_start, meta.q_start[-1:].expand(T)])})
+    x, rows, gain = dev(padc(torch.randn(T, width, generator=g(1)), wp)), dev(padc(torch.randn(T * k, width, generator=g(2)).to(dt), wp)), dev(padc(torch.rand(width, generator=g(3)), wp))
+    pair, w = torch.randperm(T * k, generator=g(4)).view(T, k), dev(torch.rand(T, k, generator=g(5)))
+    pair[::7, 1] = -1
+    planes, coef = dev(padc(torch.randn(max(depth, 1), T, width, generator=g(6)), wp)), dev(torch.randn(depth + 1, generator=g(7)))
+    cw, st = dev(padc(torch.randn(tp, width, generator=g(8)).to(torch.bfloat16), wp)), padc(torch.randn(2 * S, tp - 1, width, generator=g(9)), wp).cuda()
+    for experts in (True, False):
+        got = []
+        for m, shift in ((meta, 0), (many, 0), (meta, 1)):
+            state = torch.zeros(st.numel() + shift, device="cuda")[shift:].view(st.shape).copy_(st)
+            x_out, x_next = torch.zeros(T, wp, device="cuda"), torch.zeros(T, wp, device="cuda")
+            y = hip_ops.ExpertRows(rows, i32(pair.reshape(-1)), w) if experts else None
+            cast, h = hip_ops.depth_norm(x, width, groups, 1e-5, y=y, g_post=gain, x_out=x_out if experts else None, cast=True, depth=(planes[:depth], coef) if depth else None,
+                                         x_next=x_next if depth else None, conv=(cw, state), meta=m, act_dtype=dt)
+            got.append((h, cast, x_out, x_next, state))
+        for other in got[1:]:
+            assert all(torch.equal(a, b) for a, b in zip(got[0], other)), experts
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 3), (3072, 1, 4, 0), (4096, 1, 2, 5), (2048, 2, 3, 1), (512, 1, 4, 5), (4608, 3, 4, 1)])
 def test_depth_norm_rows_of_a_round_and_beyond(dtype, width, groups, taps, depth):
     """Single rows, more of them than there is room for at once, and the same rows in launches of 128: the same bits behind a sublayer, experts and nothing."""
