@@ -7,6 +7,7 @@
 #include "common.h"
 #include "fused_rows.h"
 #include <string.h>
+#include <type_traits>
 
 namespace {
 
@@ -554,58 +555,94 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(
 
 // ------------------------------------------------------------------------------------------
 // Bucketing of many pairs: the single-workgroup kernel above walks 131072 of them in 128 serial rounds (200 us at T = 16384).  Two launches over chunks of
-// ALIGN_CHUNK pairs instead:
+// align_blocks() blocks of ALIGN_BLOCK pairs instead:
 //   count:   chunk c's pairs per expert, counted in LDS -> counts[c][e]
 //   scatter: chunk c adds up all chunks' counts (E per chunk, from the caches), which gives the experts' places and its own places in them, ranks
 //            its pairs once more in LDS and writes the rows; chunk 0 writes expert_offsets.
 // (Totals reserved by atomics in a zeroed array and scanned by a launch of their own, four launches over chunks of 8192 / this, us: 64 experts 6000 pairs 13.1 / 6.4,
-// 33000 16.3 / 7.0, 131072 16.9 / 8.0, 256 experts 33000 14.9 / 8.7, 131072 15.2 / 11.5.)
+// 33000 16.1 / 7.1, 131072 16.8 / 7.5, 1 M 22.8 / 15.0, 4 M 51 / 40, 256 experts 33000 14.7 / 8.7, 131072 15.2 / 8.9, 4 M 43 / 34, 1000 experts 131072 19.9 / 17.9, 4 M 64 / 62.)
 // Rows of one expert are in the order of the chunks, inside a chunk in that of its LDS atomics (not specified: pair_pos carries the permutation).
-constexpr int ALIGN_CHUNK = 2048;  // pairs per workgroup (two per thread)
+constexpr int ALIGN_BLOCK = 2048;  // pairs that a workgroup reads at once (two per thread)
 
-__global__ __launch_bounds__(1024) void moe_align_count_kernel(const int64_t* __restrict__ topk_idx, int64_t P, int E, int32_t* __restrict__ counts) {
+// Blocks of a chunk: as many as leave a chunk per CU, or half of that where the counts to add up are many.  Chunks of one block / this, us: 256 experts 1 M pairs 23.6 / 16.0, 4 M 180 / 34, 64
+// experts 1 M 17.1 / 15.0, 4 M 77 / 40, 1000 experts 1 M 72 / 26.6, 4 M 796 / 62.
+int align_blocks(int64_t P, int E) {
+    const int64_t all = (P + ALIGN_BLOCK - 1) / ALIGN_BLOCK;
+    int n = 1;
+    while (all > (int64_t)n * (E > 256 ? 128 : 256)) n *= 2;
+    return n;
+}
+int64_t align_chunks(int64_t P, int blocks) {
+    const int64_t chunk = (int64_t)blocks * ALIGN_BLOCK;
+    return P > 0 ? (P + chunk - 1) / chunk : 1;   // (of no pairs one that writes the offsets)
+}
+
+__global__ __launch_bounds__(1024) void moe_align_count_kernel(const int64_t* __restrict__ topk_idx, int64_t P, int E, int blocks, int32_t* __restrict__ counts) {
     __shared__ int hist[ALIGN_MAX_G];
     const int tid = threadIdx.x;
-    const int64_t p0 = (int64_t)blockIdx.x * ALIGN_CHUNK;
-    int64_t e[ALIGN_CHUNK / 1024];
+    int64_t p0 = (int64_t)blockIdx.x * blocks * ALIGN_BLOCK;
+    int64_t e[ALIGN_BLOCK / 1024];
+    auto fetch = [&]() {
 #pragma unroll
-    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) e[i] = p0 + i * 1024 + tid < P ? topk_idx[p0 + i * 1024 + tid] : -1;
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i) e[i] = p0 + i * 1024 + tid < P ? topk_idx[p0 + i * 1024 + tid] : -1;
+    };
+    fetch();
     for (int g = tid; g < E; g += 1024) hist[g] = 0;
     __syncthreads();
+    for (int b = 0; b < blocks; ++b) {
+        int64_t was[ALIGN_BLOCK / 1024];
 #pragma unroll
-    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i)
-        if (e[i] >= 0 && e[i] < E) atomicAdd(&hist[(int)e[i]], 1);
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i) was[i] = e[i];
+        p0 += ALIGN_BLOCK;
+        if (b + 1 < blocks) fetch();
+#pragma unroll
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i)
+            if (was[i] >= 0 && was[i] < E) atomicAdd(&hist[(int)was[i]], 1);
+    }
     __syncthreads();
     for (int g = tid; g < E; g += 1024) counts[(int64_t)blockIdx.x * E + g] = hist[g];
 }
 
 __global__ __launch_bounds__(1024) void moe_align_scatter_kernel(
     const int64_t* __restrict__ topk_idx, const bf16_t* __restrict__ topk_w, const int32_t* __restrict__ counts, int32_t* __restrict__ expert_offsets,
-    int32_t* __restrict__ sorted_token, bf16_t* __restrict__ sorted_scale, int32_t* __restrict__ pair_pos, int64_t T, int k, int E, int with_shared) {
+    int32_t* __restrict__ sorted_token, bf16_t* __restrict__ sorted_scale, int32_t* __restrict__ pair_pos, int64_t T, int k, int E, int blocks, int with_shared) {
     __shared__ int cur[ALIGN_MAX_G], all[ALIGN_MAX_G], s_run;
     const int tid = threadIdx.x, chunks = gridDim.x, me = blockIdx.x;
-    const int64_t P = T * k, p0 = (int64_t)me * ALIGN_CHUNK;
-    int64_t ex[ALIGN_CHUNK / 1024];
-    bf16_t wt[ALIGN_CHUNK / 1024];
+    const int64_t P = T * k, chunk = (int64_t)blocks * ALIGN_BLOCK;
+    int64_t p0 = me * chunk;
+    int64_t ex[ALIGN_BLOCK / 1024];
+    bf16_t wt[ALIGN_BLOCK / 1024];
+    auto fetch = [&]() {
 #pragma unroll
-    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) {
-        const int64_t p = p0 + i * 1024 + tid;
-        ex[i] = p < P ? topk_idx[p] : -1;
-        wt[i] = p < P && sorted_scale ? topk_w[p] : (bf16_t)0;
-    }
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i) {
+            const int64_t p = p0 + i * 1024 + tid;
+            ex[i] = p < P ? topk_idx[p] : -1;
+            wt[i] = p < P && sorted_scale ? topk_w[p] : (bf16_t)0;
+        }
+    };
+    fetch();
     for (int e = tid; e < E; e += 1024) cur[e] = all[e] = 0;
     __syncthreads();
-    // a wave adds up every 16th chunk for 64 experts at a time
+    // a wave adds up every 16th chunk for 64 experts at a time, eight of them requested together, of what is left four (one by one: 1000 experts 131072 pairs 29 us, so 18)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int e0 = 0; e0 < E; e0 += 64) {
         const int e = e0 + (tid & 63);
         int sum = 0, before = 0;
         if (e < E) {
-#pragma unroll 8
-            for (int c = tid >> 6; c < chunks; c += 16) {
-                const int n = counts[(int64_t)c * E + e];
-                sum += n;
-                before += c < me ? n : 0;
-            }
+            auto add = [&](int c0, auto countc) __attribute__((always_inline)) {
+                constexpr int N = decltype(countc)::value;
+                int n[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) n[j] = counts[(int64_t)min(c0 + 16 * j, chunks - 1) * E + e];
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    sum += c0 + 16 * j < chunks ? n[j] : 0;
+                    before += c0 + 16 * j < me ? n[j] : 0;
+                }
+            };
+            int c = wave;
+            for (; c + 112 < chunks; c += 128) add(c, std::integral_constant<int, 8>{});
+            for (; c < chunks; c += 64) add(c, std::integral_constant<int, 4>{});
             if (sum) atomicAdd(&all[e], sum);
             if (before) atomicAdd(&cur[e], before);
         }
@@ -632,22 +669,34 @@ __global__ __launch_bounds__(1024) void moe_align_scatter_kernel(
         }
     }
     __syncthreads();
+    for (int b = 0; b < blocks; ++b) {
+        const int64_t q0 = p0 + tid;
+        int64_t e[ALIGN_BLOCK / 1024];
+        bf16_t w[ALIGN_BLOCK / 1024];
 #pragma unroll
-    for (int i = 0; i < ALIGN_CHUNK / 1024; ++i) {
-        const int64_t p = p0 + i * 1024 + tid;
-        if (p >= P) continue;
-        if (ex[i] >= 0 && ex[i] < E) {
-            const int pos = atomicAdd(&cur[(int)ex[i]], 1);
-            sorted_token[pos] = (int32_t)(p / k);
-            if (sorted_scale) sorted_scale[pos] = wt[i];
-            pair_pos[p] = pos;
-        } else {
-            pair_pos[p] = -1;
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i) {
+            e[i] = ex[i];
+            w[i] = wt[i];
+        }
+        p0 += ALIGN_BLOCK;
+        if (b + 1 < blocks) fetch();
+#pragma unroll
+        for (int i = 0; i < ALIGN_BLOCK / 1024; ++i) {
+            const int64_t p = q0 + i * 1024;
+            if (p >= P) continue;
+            if (e[i] >= 0 && e[i] < E) {
+                const int pos = atomicAdd(&cur[(int)e[i]], 1);
+                sorted_token[pos] = (int32_t)(p / k);
+                if (sorted_scale) sorted_scale[pos] = w[i];
+                pair_pos[p] = pos;
+            } else {
+                pair_pos[p] = -1;
+            }
         }
     }
     if (with_shared) {  // the shared group's rows of this chunk's token range
-        const int64_t t0 = (int64_t)me * ALIGN_CHUNK;  // chunks outnumber ceil(T / ALIGN_CHUNK): k >= 1
-        for (int64_t t = t0 + tid; t < min(T, t0 + ALIGN_CHUNK); t += 1024) {
+        const int64_t t0 = (int64_t)me * chunk;  // chunks outnumber ceil(T / chunk): k >= 1
+        for (int64_t t = t0 + tid; t < min(T, t0 + chunk); t += 1024) {
             sorted_token[s_run + t] = (int32_t)t;
             sorted_scale[s_run + t] = 0x3F80;  // bf16 1.0
         }
@@ -1072,8 +1121,7 @@ extern "C" int glm_moe_align(const int64_t* topk_idx, const void* topk_w, int32_
 
 extern "C" size_t glm_moe_align_workspace_bytes(int64_t T, int k, int E) {
     const int64_t P = (T > 0 ? T : 0) * (int64_t)(k > 0 ? k : 0);
-    const int64_t chunks = P > 0 ? (P + ALIGN_CHUNK - 1) / ALIGN_CHUNK : 1;
-    return (size_t)(E > 0 ? E : 0) * sizeof(int32_t) * (size_t)chunks;
+    return (size_t)(E > 0 ? E : 0) * sizeof(int32_t) * (size_t)align_chunks(P, align_blocks(P, E));
 }
 
 // glm_moe_align over many workgroups.  workspace: glm_moe_align_workspace_bytes(T, k, E), whatever it holds on entry.
@@ -1089,11 +1137,12 @@ extern "C" int glm_moe_align_parallel(const int64_t* topk_idx, const void* topk_
     GLM_CHECK_ARG(workspace_bytes >= glm_moe_align_workspace_bytes(T, k, E), GLM_ERR_WORKSPACE,
                   "glm_moe_align_parallel: workspace %zu < %zu bytes", workspace_bytes, glm_moe_align_workspace_bytes(T, k, E));
     const int64_t P = T * k;
-    const unsigned chunks = P > 0 ? (unsigned)((P + ALIGN_CHUNK - 1) / ALIGN_CHUNK) : 1;   // (of no pairs one that writes the offsets)
+    const int blocks = align_blocks(P, E);
+    const unsigned chunks = (unsigned)align_chunks(P, blocks);
     hipStream_t st = glm_s(stream);
-    hipLaunchKernelGGL(moe_align_count_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, P, E, workspace);
+    hipLaunchKernelGGL(moe_align_count_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, P, E, blocks, workspace);
     hipLaunchKernelGGL(moe_align_scatter_kernel, dim3(chunks), dim3(1024), 0, st, topk_idx, (const bf16_t*)topk_w, workspace, expert_offsets, sorted_token,
-                       (bf16_t*)sorted_scale, pair_pos, T, k, E, with_shared);
+                       (bf16_t*)sorted_scale, pair_pos, T, k, E, blocks, with_shared);
     GLM_CHECK_LAUNCH("glm_moe_align_parallel");
     return GLM_OK;
 }

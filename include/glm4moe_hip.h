@@ -179,7 +179,7 @@ int glm_moe_align(const int64_t* topk_idx, const void* topk_w,
                   glm_stream_t stream);
 
 /* The same bucketing over many workgroups, for prefill sizes (the kernel above is ONE workgroup: 200 us at T = 16384,
- *     k = 8): count and scatter launches over chunks of 2048 pairs.  workspace: glm_moe_align_workspace_bytes(),
+ *     k = 8): count and scatter launches over chunks of 2048 pairs and more.  workspace: glm_moe_align_workspace_bytes(),
  *     int32, whatever it holds on entry.  Same contract for the outputs; the order of the rows inside a group is
  *     unspecified in both.                                                                                     */
 size_t glm_moe_align_workspace_bytes(int64_t T, int k, int E);

@@ -516,8 +516,8 @@ def _check_align(offs, tok, scale, pos, idx, w, E, shared):
 
 @pytest.mark.parametrize("T,k,E,shared", [(4096, 8, 64, True), (2100, 8, 128, False), (16384, 1, 4, True), (9000, 2, 16, True)])
 def test_moe_align_parallel(ops, T, k, E, shared):
-    """Prefill-size bucketing (count / offsets / scatter over chunks of 8192 pairs): moe_align's contract, incl. an expert
-    nobody picked, a ragged last chunk and the shared group."""
+    """Bucketing of many pairs (count / scatter over chunks of 2048 pairs): moe_align's contract, incl. an expert nobody
+    picked, a ragged last chunk and the shared group."""
     assert T * k >= ops.ALIGN_PARALLEL_MIN_PAIRS
     g = torch.Generator().manual_seed(T + k + E)
     pool = max(k, E - 1)  # expert E-1 is never selected
@@ -537,16 +537,46 @@ def test_moe_align_parallel(ops, T, k, E, shared):
         assert int(offs[E + 1]) == P + T and tok[P:].tolist() == list(range(T)) and bool((scale[P:].float() == 1.0).all())
 
 
+@pytest.mark.parametrize("P,k,E,shared", [(1, 1, 1, False), (2048, 1, 1000, False), (2049, 1, 1023, False), (2040, 8, 64, True), (33 * 2048 + 2, 2, 256, True), (16 * 2048, 8, 257, False),
+                                          (131072, 8, 1000, False), (256 * 2048, 8, 64, True), (256 * 2048 + 8, 8, 64, True), (128 * 2048 + 1, 1, 300, False), (515 * 2048, 4, 130, True), (1030 * 2048 + 5, 5, 65, False)])
+def test_moe_align_parallel_workspace(ops, P, k, E, shared):
+    """Chunks of one block, two, four and more, with whatever the workspace holds: the same offsets and groups as from a workspace of zeros; nothing behind its end is written."""
+    T, lib, guard = P // k, ops.load_library(), 64
+    P, G = T * k, E + int(shared)
+    g = torch.Generator(device="cuda").manual_seed(P + E)
+    idx = torch.randint(0, E, (T, k), device="cuda", generator=g)
+    idx[::97, 0] = -1
+    w = torch.rand(T, k, device="cuda", generator=g).to(BF)
+    words = lib.glm_moe_align_workspace_bytes(T, k, E) // 4
+    ok, order = (idx >= 0).flatten(), torch.arange(P, device="cuda")
+    n = int(ok.sum())
+    R = P + T * int(shared)
+    for fill in (0, -77, 2 ** 31 - 1, 0x55555555):
+        ws = torch.full((words + guard,), fill, dtype=torch.int32, device="cuda")
+        ws[words:] = 123
+        offs, tok, pos = (torch.full((c + guard,), -5, dtype=torch.int32, device="cuda") for c in (G + 1, R, P))
+        scale = torch.full((R + guard,), -5.0, dtype=BF, device="cuda")
+        ops._check(lib.glm_moe_align_parallel(ops._p(idx), ops._p(w), ops._p(offs), ops._p(tok), ops._p(scale), ops._p(pos), T, k, E, int(shared), ops._p(ws), words * 4, ops._stream()), "align")
+        assert bool((ws[words:] == 123).all()) and all(bool((t[-guard:] == -5).all()) for t in (offs, tok, scale, pos))
+        counts = torch.bincount(idx.flatten()[ok], minlength=E)
+        assert torch.equal(offs[1: E + 1].long(), counts.cumsum(0)) and int(offs[0]) == 0
+        p = pos[:P].long()
+        assert bool((p[~ok] == -1).all()) and torch.equal(p[ok].sort().values, order[:n])
+        assert torch.equal(torch.bucketize(p[ok], offs[1: E + 1].long(), right=True), idx.flatten()[ok])
+        assert torch.equal(tok[p[ok]].long(), (order // k)[ok]) and torch.equal(scale[p[ok]], w.flatten()[ok])
+        if shared:
+            assert int(offs[E + 1]) == n + T and torch.equal(tok[n: n + T].long(), order[:T]) and bool((scale[n: n + T] == 1).all())
+    assert lib.glm_moe_align_parallel(ops._p(idx), ops._p(w), ops._p(offs), ops._p(tok), ops._p(scale), ops._p(pos), T, k, E, int(shared), ops._p(ws), words * 4 - 4, ops._stream()) != 0
+
+
 @pytest.mark.parametrize("T,k,E,shared", [(5120, 1, 1000, False), (1025, 5, 64, True), (3072, 2, 63, True), (6145, 1, 65, True), (700, 8, 256, False), (20000, 3, 200, True)])
 def test_moe_align_parallel_chunks(ops, T, k, E, shared):
-    """Chunks that are whole, end by one pair or hold one pair, experts that fill several passes, pairs without an expert, a workspace of whatever values."""
+    """Chunks that are whole, end by one pair or hold one pair, experts that fill several passes, pairs without an expert."""
     assert T * k >= ops.ALIGN_PARALLEL_MIN_PAIRS
     g = torch.Generator().manual_seed(T)
     idx = torch.randint(0, E, (T, k), generator=g) if k == 1 else torch.rand(T, E, generator=g).topk(k, -1).indices
     idx[::97, 0] = -1
     w = (torch.rand(T, k, generator=g) + 0.1).to(BF)
-    junk = torch.full((1 << 20,), -77, dtype=torch.int32, device="cuda")
-    del junk     # (what the workspace may be made of)
     offs, tok, scale, pos = [a.cpu() for a in ops.moe_align(dev(idx), dev(w), E, shared)]
     flat, ok = idx.flatten(), idx.flatten() >= 0
     n = int(ok.sum())
