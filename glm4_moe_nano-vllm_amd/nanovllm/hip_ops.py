@@ -792,9 +792,14 @@ def add_rmsnorm_router_topk(x, residual: torch.Tensor, norm_weight: torch.Tensor
     return y.view(residual.shape), ro.view(residual.shape), idx, w
 
 
-# from here on the one-workgroup bucketing kernel is the slower one; one / many, us: 64 experts 4096 pairs 6.4 / 6.3, 6000 8.7 / 6.4, without weights 4.6 / 5.2, 6.0 / 5.3,
-# 256 experts 6000 7.0 / 7.3, 8192 8.9 / 7.3
 ALIGN_PARALLEL_MIN_PAIRS = 5120
+
+
+def align_parallel_pairs(E: int, weights: bool) -> int:
+    """Pairs from which on the one-workgroup bucketing kernel is the slower one: every workgroup of the other adds up counts of all experts.  One / many, us, without
+    weights: 8 experts 5120 pairs 4.8 / 5.5, 7000 5.9 / 5.5, 64 5120 5.2 / 5.6, 6000 6.0 / 5.7, 256 6000 7.0 / 7.5, 7000 7.8 / 7.6, 512 8192 9.4 / 10.3, 9216 10.3 / 10.4, 1000 12288 13.9 / 15.5,
+    14336 15.8 / 15.5; with them: 64 4096 6.3 / 6.2, 256 5120 8.7 / 8.4, 512 6000 10.6 / 10.8, 7000 12.2 / 11.3, 1000 8192 14.8 / 16.0, 9216 16.4 / 16.5."""
+    return max(ALIGN_PARALLEL_MIN_PAIRS, 3500 + 11 * E // 2) if weights else max(ALIGN_PARALLEL_MIN_PAIRS + 640, 4500 + 9 * E)
 
 
 def moe_align(topk_idx: torch.Tensor, topk_w: torch.Tensor | None, E: int, with_shared: bool):
@@ -807,7 +812,7 @@ def moe_align(topk_idx: torch.Tensor, topk_w: torch.Tensor | None, E: int, with_
     tok = torch.empty(R, dtype=torch.int32, device=dev)
     scale = torch.empty(R, dtype=torch.bfloat16, device=dev) if topk_w is not None else None
     pos = torch.empty(T * k, dtype=torch.int32, device=dev)
-    if T * k >= ALIGN_PARALLEL_MIN_PAIRS:  # prefill sizes: count / scatter over many workgroups
+    if T * k >= align_parallel_pairs(E, topk_w is not None):  # prefill sizes: count / scatter over many workgroups
         lib = load_library()
         ws = torch.empty(lib.glm_moe_align_workspace_bytes(T, k, E) // 4, dtype=torch.int32, device=dev)
         _check(lib.glm_moe_align_parallel(_p(topk_idx), _p(topk_w), _p(offs), _p(tok), _p(scale), _p(pos), T, k, E,

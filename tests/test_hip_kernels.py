@@ -518,7 +518,7 @@ def _check_align(offs, tok, scale, pos, idx, w, E, shared):
 def test_moe_align_parallel(ops, T, k, E, shared):
     """Bucketing of many pairs (count / scatter over chunks of 2048 pairs): moe_align's contract, incl. an expert nobody
     picked, a ragged last chunk and the shared group."""
-    assert T * k >= ops.ALIGN_PARALLEL_MIN_PAIRS
+    assert T * k >= ops.align_parallel_pairs(E, True)
     g = torch.Generator().manual_seed(T + k + E)
     pool = max(k, E - 1)  # expert E-1 is never selected
     idx = torch.stack([torch.randperm(pool, generator=g)[:k].sort()[0] for _ in range(T)]).to(torch.int64)
@@ -569,10 +569,10 @@ def test_moe_align_parallel_workspace(ops, P, k, E, shared):
     assert lib.glm_moe_align_parallel(ops._p(idx), ops._p(w), ops._p(offs), ops._p(tok), ops._p(scale), ops._p(pos), T, k, E, int(shared), ops._p(ws), words * 4 - 4, ops._stream()) != 0
 
 
-@pytest.mark.parametrize("T,k,E,shared", [(5120, 1, 1000, False), (1025, 5, 64, True), (3072, 2, 63, True), (6145, 1, 65, True), (700, 8, 256, False), (20000, 3, 200, True)])
+@pytest.mark.parametrize("T,k,E,shared", [(10240, 1, 1000, False), (1025, 5, 64, True), (3072, 2, 63, True), (6145, 1, 65, True), (700, 8, 256, False), (20000, 3, 200, True)])
 def test_moe_align_parallel_chunks(ops, T, k, E, shared):
     """Chunks that are whole, end by one pair or hold one pair, experts that fill several passes, pairs without an expert."""
-    assert T * k >= ops.ALIGN_PARALLEL_MIN_PAIRS
+    assert T * k >= ops.align_parallel_pairs(E, True)
     g = torch.Generator().manual_seed(T)
     idx = torch.randint(0, E, (T, k), generator=g) if k == 1 else torch.rand(T, E, generator=g).topk(k, -1).indices
     idx[::97, 0] = -1
@@ -587,6 +587,27 @@ def test_moe_align_parallel_chunks(ops, T, k, E, shared):
     assert torch.equal(tok[p].long(), (torch.arange(T * k) // k)[ok]) and torch.equal(scale[p], w.flatten()[ok])
     if shared:
         assert int(offs[E + 1]) == n + T and tok[n: n + T].tolist() == list(range(T)) and bool((scale[n: n + T].float() == 1.0).all())
+
+
+@pytest.mark.parametrize("E", [1, 8, 64, 257, 1000])
+@pytest.mark.parametrize("weights", [False, True])
+def test_moe_align_on_both_sides_of_the_line(ops, E, weights, monkeypatch):
+    """One pair before the line the bucketing takes one workgroup, from it on many; the same offsets and groups on both sides."""
+    lib, P, seen = ops.load_library(), ops.align_parallel_pairs(E, weights), []
+
+    class Library:
+        def __getattr__(self, name):
+            if name in ("glm_moe_align", "glm_moe_align_parallel"):
+                seen.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(ops, "load_library", Library)
+    for n in (P - 1, P):
+        idx = torch.randint(0, E, (n, 1), device="cuda", generator=torch.Generator(device="cuda").manual_seed(E))
+        offs, tok, scale, pos = ops.moe_align(idx, torch.rand(n, 1, device="cuda").to(BF) if weights else None, E, weights)
+        assert torch.equal(offs[1: E + 1].long(), torch.bincount(idx.flatten(), minlength=E).cumsum(0)) and (scale is None) == (not weights)
+        assert torch.equal(torch.bucketize(pos.long(), offs[1: E + 1].long(), right=True), idx.flatten()) and torch.equal(tok[pos.long()].long(), torch.arange(n, device="cuda"))
+    assert seen == ["glm_moe_align", "glm_moe_align_parallel"]
 
 
 def test_moe_align(ops):
