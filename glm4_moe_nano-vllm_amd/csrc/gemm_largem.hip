@@ -990,9 +990,13 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             const unsigned lrow = (unsigned)c * pitch;
             // Of short reductions (much output for its time) whole cache lines are written through the L2: what stays dirty there is written out when a tile of operands needs
             // the place and, 32 MiB of it, at the launch's end.  Kept dirty / through, us, in a step: 15074 x 4096 x 256 52.2 / 47.4, x 2048 x 2048 98.0 / 95.4,
-            // x 6144 x 2048 (xIELU) 320 / 315, 11137 x 4096 x 2048 gated 279 / 274, and attention behind such a launch 582 / 570, 173 / 170.  K of 4096 and more loses
-            // 0 to 1 %, experts 2 to 3 %, and rows that start inside a line 12 % (15074 x 9232 x 2048 419 / 470).  By itself, 2000 to 15074 rows of 2048 to 10240 columns:
-            // K of 256 and 512 1.00 to 1.18 times as fast (3700 x 2048 x 512 12.8 / 10.8), of 2048 0.99 to 1.06.
+            // x 6144 x 2048 (xIELU) 320 / 315, 11137 x 4096 x 2048 gated 279 / 274, and attention behind such a launch 582 / 570, 173 / 170.  Experts lose 2 to 3 %, rows that start inside
+            // a line 12 % (15074 x 9232 x 2048 419 / 470).  By itself, times of kept dirty, up to a round of tiles: K of 256 to 1024 0.83 to 0.95 (3756 x 2048 x 512 13.4 / 11.4), of several
+            // rounds 0.90 to 0.98, of 2048 0.98 to 1.0; rows of 16 KiB (8192 columns) 0.94 to 1.07, 1.00 in the mean (3756 x 8192 x 512 34.4 / 36.1; such a launch inside a step of width 4096,
+            // 36 rows and four prompts of 930, 48 / 50, the step 4430 / 4460), outputs of more than 256 MiB 1.0 to 1.2.
+            // The line: whole steps of 2048 columns gain 1 to 2.5 % by it on three cards of four, 0 to -1 % on the fourth, nearly all of it from K = 2048.  Beyond it K of 2560 and 3072 take 0.95 to
+            // 1.0 of the time by themselves (4200 x 2048 x 3072 51.4 / 49.2, 15074 x 6144 x 3072 403 / 402), 4096 and 6144 0.97 to 1.02, but steps with those get nothing: eleven of 15 kinds 0.1 to
+            // 0.7 % slower, one 1 % faster.
             const bool through = !GROUPED && K <= LM_THROUGH_K && ((pitch | (unsigned)(F32 ? (uintptr_t)p.yf : (uintptr_t)p.y)) & 127u) == 0;
             auto put = [&](const u32x4_t v, const __amdgpu_buffer_rsrc_t yrs, unsigned at) __attribute__((always_inline)) {
                 if (through) __builtin_amdgcn_raw_buffer_store_b128(v, yrs, at, 0, LM_SC1);
