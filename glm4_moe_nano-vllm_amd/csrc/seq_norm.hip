@@ -257,9 +257,12 @@ __device__ __forceinline__ int sn_table(const int32_t* p, int64_t i) { return re
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t sn_row(const void* base, int64_t off, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(base) + off), 0, base ? bytes : 0, 0x00020000);
 }
+// (The second half is 16 bytes of the vector offset and not a scalar one: that is taken off the length before the offset is compared with it, and a buffer of no length has none to take off.
+// Opaque: kept over the loop, the sum would take a register of its own.)
 __device__ __forceinline__ void sn_put8f(__amdgpu_buffer_rsrc_t rs, int at, const Row8& v) {
+    asm volatile("" : "+v"(at));
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v.a), rs, at, 0, 0);
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v.b), rs, at, 16, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v.b), rs, at + 16, 0, 0);
 }
 __device__ __forceinline__ u32x4_t sn_pack8(const Row8& v) {
     return u32x4_t{pack2bf(v.a[0], v.a[1]), pack2bf(v.a[2], v.a[3]), pack2bf(v.b[0], v.b[1]), pack2bf(v.b[2], v.b[3])};

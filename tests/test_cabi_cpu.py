@@ -134,6 +134,19 @@ def test_no_asm_takes_maxima_of_mfma_results():
             assert "v_max3_f32" not in open(os.path.join(csrc, f)).read(), f
 
 
+def test_buffer_stores_have_no_scalar_offset():
+    """Stores go into buffers of no length where there is nothing to store.  A scalar offset is taken off the length before the vector offset is compared with it:
+    off a length of zero there is nothing to take."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "glm4_moe_nano-vllm_amd", "csrc")
+    seen = 0
+    for f in sorted(os.listdir(csrc)):
+        for line in open(os.path.join(csrc, f)):
+            for call in re.findall(r"__builtin_amdgcn_raw_buffer_store_b\d+\((.*?)\);", line):
+                seen += 1
+                assert call.split(",")[-2].strip() == "0", (f, call)
+    assert seen > 5
+
+
 def test_asm_mfma_statements_have_no_compiler_placed_hazards():
     """csrc/prefill_attn64.hip issues its MFMAs from inline asm, which the compiler's hazard recogniser cannot see: a register
     copy it places right in front of one (VALU write of SrcC) or right behind one (VALU read of the result) silently corrupts
