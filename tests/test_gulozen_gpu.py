@@ -86,13 +86,13 @@ def batch_meta(lens, starts, seed=0):
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,groups,taps,depth", [(76, 4, 3, 0), (64, 8, 2, 3), (1032, 1, 4, 1), (200, 5, 6, 5), (2048, 2, 3, 9), (4104, 3, 2, 2), (136, 1, 1, 4), (72, 72, 17, 1), (24, 3, 32, 2)])
-def test_depth_norm(dtype, width, groups, taps, depth):
-    """Closing norm, average over depth, convolution and its state in one launch, over portions whose history lies in the step, in the state
-    or in front of the sequence; experts' rows instead of a sublayer's; the norm in front of the head on gathered rows."""
+def test_depth_norm(dtype, width, groups, taps, depth, longest=700):
+    """Closing norm, average over depth, convolution and its state, over portions whose history lies in the step, in the state or in front of the sequence (steps of
+    some 750 rows: in two launches); experts' rows instead of a sublayer's; the norm in front of the head on gathered rows."""
     from nanovllm import hip_ops
     from nanovllm.layers.depth_norm import CausalTaps
     dt, wp, eps = DT[dtype], hip_ops.round8(width), 1e-3
-    lens, starts = [1, 2, 40, 1, 700, taps, 5], [9, 0, 1, 0, 30, 3, 40]
+    lens, starts = [1, 2, 40, 1, longest, taps, 5], [9, 0, 1, 0, 30, 3, 40]
     T = sum(lens)
     meta, order = batch_meta(lens, starts)
     conv = CausalTaps(width, taps)
@@ -224,9 +224,10 @@ def test_depth_norm_rows_of_a_round_and_beyond(dtype, width, groups, taps, depth
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 2), (4608, 1, 4, 3), (512, 1, 4, 5), (8, 1, 4, 1)])
+@pytest.mark.parametrize("width,groups,taps,depth", [(4096, 4, 4, 2), (4096, 4, 3, 5), (4608, 1, 4, 3), (512, 1, 4, 5), (2048, 4, 2, 6), (8, 1, 4, 1)])
 def test_depth_norm_512_threads(dtype, width, groups, taps, depth):
-    """Four taps in 512 threads, in more, in one wave and in one lane."""
+    """Two to four taps in 512 threads, in more, in four waves, in one wave and in one lane: some 140 rows, which are one launch, and some 750."""
+    test_depth_norm(dtype, width, groups, taps, depth, longest=90)
     test_depth_norm(dtype, width, groups, taps, depth)
 
 
