@@ -466,13 +466,30 @@ constexpr int64_t DN_SPLIT_ROWS = 512;   // rows from which norm and convolution
 // 16.5 / 16.4, nothing 8.7 / 7.7, 9.0 / 10.8; two taps, experts, 512 rows 18.6 / 15.5, 18.3 / 16.6.
 constexpr int64_t DN_SPLIT_EXTRA = 256;
 
+// Rows of a run.  Four and more for 1024 workgroups, 16 at most: portions that begin inside a run wait for their state one after the other, and shorter runs read more
+// rows twice.  16 rows / 512 workgroups / this / 2048, us: 15074 rows of 2048 38.3 / 38.3 / 38.3 / 41.3, 5000 of 4096 25.6 / 25.8 / 25.3 / 26.4, 700 of 2048 10.3 / 6.2 / 6.2 /
+// 6.3, 40 single rows and 5400 of prompts 41.8 / 31.6 / 24.4 / 20.0, 60 and 5800 44.7 / 36.9 / 25.4 / 22.0.
+// Longer ones with more than four taps, where a run of four begins with five to 31 rows of its own, for some long portions (single rows would wait in them):
+//   - six and eight taps, for as many threads with columns as 512 workgroups of 2048 columns have.  The rule above / this, us: six taps, 3000 rows of 2048 13.0 / 11.6, of 4096
+//     19.3 / 16.8, 5000 of 2048 17.6 / 14.7; eight, 3000 of 4096 23.3 / 19.5, 4000 of 2048 19.0 / 15.6, 7000 24.9 / 20.8; of 1024 columns both are the same to 4 %
+//   - 16 and 32, for one workgroup per CU (its registers), whose rounds take as long as the run and two or three rows more: 16 taps, 1200 rows of 1024 18.2 / 13.4, 3000 of 2048
+//     37.5 / 28.0 (runs of 16 32.0), 32 taps, 1500 of 2048 51.0 / 38.4, 4000 of 4096 167 / 144
 template <int TAPS>
-int launch_depth_conv(const DepthArgs& a, const float* xs, hipStream_t st) {
-    // Runs of four rows and more for 1024 workgroups, of 16 at most: portions that begin inside a run wait for their state one after the other, and shorter runs read more
-    // rows twice.  16 rows / 512 workgroups / this / 2048, us: 15074 rows of 2048 38.3 / 38.3 / 38.3 / 41.3, 5000 of 4096 25.6 / 25.8 / 25.3 / 26.4, 700 of 2048 10.3 / 6.2 / 6.2 /
-    // 6.3, 40 single rows and 5400 of prompts 41.8 / 31.6 / 24.4 / 20.0, 60 and 5800 44.7 / 36.9 / 25.4 / 22.0.
-    const int64_t per = (a.T * ((a.wp + 2047) / 2048) + 1023) / 1024;
-    const int tr = (int)(per < 4 ? 4 : per > 16 ? 16 : (per + 1) / 2 * 2);
+int depth_conv_run(int64_t T, int wp, int64_t seqs) {
+    const int64_t cols = (wp + 2047) / 2048;
+    auto even = [](int64_t per) { return (int)(per < 4 ? 4 : per > 16 ? 16 : (per + 1) / 2 * 2); };
+    if (TAPS <= 4 || seqs > 8 || T < 128 * seqs) return even((T * cols + 1023) / 1024);
+    if (TAPS <= 8) return even((T * wp + (1 << 20) - 1) >> 20);
+    int best = 4;
+    auto time = [&](int n) { return ((T + n - 1) / n * cols + 255) / 256 * (2 * n + 5); };
+    for (int n = 6; n <= 16; n += 2)
+        if (time(n) < time(best)) best = n;
+    return best;
+}
+
+template <int TAPS>
+int launch_depth_conv(const DepthArgs& a, int64_t seqs, const float* xs, hipStream_t st) {
+    const int tr = depth_conv_run<TAPS>(a.T, a.wp, seqs);
     const dim3 grid((unsigned)((a.T + tr - 1) / tr), (unsigned)((a.wp + 2047) / 2048));
     if (a.act_f32) hipLaunchKernelGGL((depth_conv_kernel<TAPS, true>), grid, dim3(256), 0, st, a, xs, tr);
     else hipLaunchKernelGGL((depth_conv_kernel<TAPS, false>), grid, dim3(256), 0, st, a, xs, tr);
@@ -493,7 +510,7 @@ int launch_depth_norm(const DepthArgs& a, int64_t seqs, int nt, bool vec, hipStr
                 const int rc = launch_depth_norm<1>(b, seqs, nt, vec, st);
                 if (rc != GLM_OK) return rc;
             }
-            return launch_depth_conv<TAPS>(a, xs, st);
+            return launch_depth_conv<TAPS>(a, seqs, xs, st);
         }
     }
     if constexpr (TAPS > 1 && TAPS <= 4) {

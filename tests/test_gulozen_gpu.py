@@ -263,6 +263,13 @@ def test_convolution_down_runs(width, taps, lens):
         at += n
 
 
+@pytest.mark.parametrize("width,taps", [(2048, 6), (4096, 6), (2056, 8), (72, 16), (1024, 16), (4104, 16), (520, 32), (2048, 32)])
+@pytest.mark.parametrize("lens", [[530], [1500, 1100], [128, 3001, 700, 2000], [1279, 1], [300] * 8])
+def test_convolution_of_long_portions(width, taps, lens):
+    """More than four taps down runs of four to 16 rows."""
+    test_convolution_down_runs(width, taps, lens)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width,ff,E,top", [(76, 20, 5, 2), (136, 72, 9, 1), (64, 8, 70, 6), (72, 24, 300, 8), (40, 44, 3, 3), (256, 512, 64, 4)])
 def test_experts(dtype, width, ff, E, top):
