@@ -242,7 +242,7 @@ __device__ __forceinline__ void lm_locate_lanes(const int32_t* __restrict__ offs
 // the SCALAR offset, fragment reads use one base register per k-step plus immediate offsets, 16-byte stores (the packed results of two
 // neighbouring 16-column tiles are exchanged between the lane rows).  Needs K % BK == 0, x and W spans < 2 GiB, N % 8 == 0.  The other
 // form covers everything else.
-// blocks: row blocks there are (CUT: of 256 rows).  CUT: tiles of 256 rows from `first` on, each in two of 128.
+// blocks: row blocks there are, or more than the list has (CUT: of 256 rows).  CUT: tiles of 256 rows from `first` on, each in two of 128.
 template <int MODE, class C, bool LEAN, bool WSCALE, bool CUT>
 __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, int n_tiles, int total_tiles, int LM_BAND, int blocks, int first) {
     constexpr bool F32 = MODE == GEMM_SLICES || MODE == GEMM_F32 || MODE == GEMM_CAP || MODE == GEMM_XIELU32 || MODE == GEMM_COLS32;  // stores fp32 rows (p.yf)
@@ -278,7 +278,7 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
         while (pos0 + ti * pstep < chunk_len) {
             if ((ti & 63) == 0) {
                 const int bid = chunk_base + pos0 + (ti + lane) * pstep;
-                if constexpr (MODE != GEMM_SLICES) {   // no position without a tile in front of the last one
+                if constexpr (MODE != GEMM_SLICES) {
                     const int half = CUT ? bid & 1 : 0;
                     int t = CUT ? first + (bid >> 1) : bid;
                     const int band = t / (LM_BAND * n_tiles), b0 = band * LM_BAND;
@@ -1125,8 +1125,11 @@ __global__ __launch_bounds__(512) void gemm_largem_kernel(const GemmParams p, in
     // without a tile were all in the last XCD's share, so that the others took up to two rounds more.  List of the most / of what there is, us: gate|up, down of 64
     // experts, 6 of 1024 x 2048 at 2400 tokens 192 / 153, 117 / 96, at 6000 314 / 293, 188 / 176, at 15074 646 / 604, 404 / 377; 8 of 1408 x 4096 at 2400 600 /
     // 564, 341 / 318, at 4096 842 / 756, 489 / 438, at 15074 2387 / 2379, 1355 / 1328.  (Without halves behind whole rounds: 0 to 3 % slower.)
+    // A list of the most that is one round stays: a workgroup has one position at most, and counting would put a trip to memory in front of it.
     if constexpr (MODE == GEMM_GATEUP || MODE == GEMM_DOWN) {
-        if (p.offs != nullptr) {
+        if (p.offs != nullptr && total_tiles <= (int)gridDim.x) {
+            blocks = 1 << 30;
+        } else if (p.offs != nullptr) {
             blocks = lm_row_blocks(p.offs, p.G, C::BM, threadIdx.x & 63);
             total_tiles = blocks * n_tiles;
             const int wgs = gridDim.x, rest = total_tiles % wgs;

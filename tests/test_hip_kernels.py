@@ -1280,6 +1280,12 @@ def test_gemm_large_m_groups_last_round_in_halves(ops, counts):
             assert bool(((a.float() - b).abs() <= 1.01 * r * 2.0 ** -8 * b.abs() + 2e-5).all())
 
 
+@pytest.mark.parametrize("counts", [[600, 0, 257, 1000, 1], [300], [681] * 7 + [677], [681] * 7 + [933], [0] * 20 + [2048], [0] * 23 + [2500, 0], [256] * 12 + [0] * 5])
+def test_gemm_large_m_groups_list_of_one_round(ops, counts):
+    """Lists of as many row blocks as rows and groups could make, up to a round of the chip and a row block more (from there on: of those that there are)."""
+    test_gemm_large_m_groups_last_round_in_halves(ops, counts)
+
+
 @pytest.mark.parametrize("M,N", [(15074, 2048), (8704, 3072), (8248, 7944), (8448, 7936), (512, 32768), (300, 40000)])
 def test_gemm_large_m_tile_lists(ops, M, N):
     """Lists of more than one round whose last band has fewer row blocks, with the positions behind it (no round more) and without them (a round more),
