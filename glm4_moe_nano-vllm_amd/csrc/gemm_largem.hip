@@ -45,6 +45,7 @@ constexpr int LM_BAND_ROWS = 4;  // row blocks per L2 supertile band
 constexpr int LM_CUT_K = 512;    // shortest reduction whose last tiles are cut
 constexpr int LM_SLOT = 32768;   // CfgR: bytes of a ring slot, one operand tile
 constexpr int LM_THROUGH_K = 2048;   // longest reduction whose output is written through the L2
+constexpr int64_t LM_THROUGH_BF16 = 400 << 20, LM_THROUGH_F32 = 240 << 20;   // bytes of it, at most
 constexpr int LM_SC1 = 16;           // cache policy bit of a store: device scope
 constexpr int64_t LM_WIDE = 1 << 25;   // output pitch from which 16 fp32 rows do not fit into a buffer
 
@@ -993,11 +994,14 @@ __device__ __forceinline__ void largem_tiles(const GemmParams& p, char* smem, in
             // x 6144 x 2048 (xIELU) 320 / 315, 11137 x 4096 x 2048 gated 279 / 274, and attention behind such a launch 582 / 570, 173 / 170.  Experts lose 2 to 3 %, rows that start inside
             // a line 12 % (15074 x 9232 x 2048 419 / 470).  By itself, times of kept dirty, up to a round of tiles: K of 256 to 1024 0.83 to 0.95 (3756 x 2048 x 512 13.4 / 11.4), of several
             // rounds 0.90 to 0.98, of 2048 0.98 to 1.0; rows of 16 KiB (8192 columns) 0.94 to 1.07, 1.00 in the mean (3756 x 8192 x 512 34.4 / 36.1; such a launch inside a step of width 4096,
-            // 36 rows and four prompts of 930, 48 / 50, the step 4430 / 4460), outputs of more than 256 MiB 1.0 to 1.2.
+            // 36 rows and four prompts of 930, 48 / 50, the step 4430 / 4460).  With weights that come from memory, as in a step, and more than some 40 G multiply-adds 1.00 to 1.08, but steps with
+            // such launches written through take 0.990 to 0.997 of the time (Dafolorn, Napadra, Gulozen, Loselix 2k, prompts of 15074 rows).
+            // Not the largest outputs, which no cache holds.  bf16 of 256 to 400 MiB 1.00 to 1.03 by themselves, but a step with six launches of 324 MiB (15074 x 11264 x 2048) 0.987 to 0.995; beyond
+            // 1.02 to 1.3 (16198 x 18688 x 1536 707 / 782, 10212 x 31872 x 128 188 / 246), fp32 beyond 240 MiB 1.04 to 1.22 (13055 x 15872 x 384 248 / 303, 11943 x 23040 x 2048 929 / 1067).
             // The line: whole steps of 2048 columns gain 1 to 2.5 % by it on three cards of four, 0 to -1 % on the fourth, nearly all of it from K = 2048.  Beyond it K of 2560 and 3072 take 0.95 to
             // 1.0 of the time by themselves (4200 x 2048 x 3072 51.4 / 49.2, 15074 x 6144 x 3072 403 / 402), 4096 and 6144 0.97 to 1.02, but steps with those get nothing: eleven of 15 kinds 0.1 to
             // 0.7 % slower, one 1 % faster.
-            const bool through = !GROUPED && K <= LM_THROUGH_K && ((pitch | (unsigned)(F32 ? (uintptr_t)p.yf : (uintptr_t)p.y)) & 127u) == 0;
+            const bool through = !GROUPED && K <= LM_THROUGH_K && p.R * p.ldy * (F32 ? 4 : 2) <= (F32 ? LM_THROUGH_F32 : LM_THROUGH_BF16) && ((pitch | (unsigned)(F32 ? (uintptr_t)p.yf : (uintptr_t)p.y)) & 127u) == 0;
             auto put = [&](const u32x4_t v, const __amdgpu_buffer_rsrc_t yrs, unsigned at) __attribute__((always_inline)) {
                 if (through) __builtin_amdgcn_raw_buffer_store_b128(v, yrs, at, 0, LM_SC1);
                 else __builtin_amdgcn_raw_buffer_store_b128(v, yrs, at, 0, 0);

@@ -1286,6 +1286,21 @@ def test_gemm_large_m_groups_list_of_one_round(ops, counts):
     test_gemm_large_m_groups_last_round_in_halves(ops, counts)
 
 
+@pytest.mark.parametrize("M,N,f32", [(16384, 12800, False), (16384, 12808, False), (16385, 12800, False), (16384, 3840, True), (16384, 3904, True), (16000, 3936, True)])
+def test_gemm_large_m_largest_output_through_the_l2(ops, M, N, f32):
+    """Outputs of as many bytes as are written through the L2, and of more, whole lines and not, bit for bit against the plain form."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, 64, device="cuda", generator=g).to(BF)
+    w = (torch.randn(N, 64, device="cuda", generator=g) * 64 ** -0.5).to(BF)
+    got = []
+    for v in (0, -1):
+        with largem_variant(v):
+            out = torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.float32 if f32 else BF)
+            ops.linear_act(x, w, out_f32=f32, out=out[:M])
+            got.append(out)
+    assert torch.equal(*got) and bool((got[1][-1] == 7).all())
+
+
 @pytest.mark.parametrize("M,N", [(15074, 2048), (8704, 3072), (8248, 7944), (8448, 7936), (512, 32768), (300, 40000)])
 def test_gemm_large_m_tile_lists(ops, M, N):
     """Lists of more than one round whose last band has fewer row blocks, with the positions behind it (no round more) and without them (a round more),
